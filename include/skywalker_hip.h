@@ -16,9 +16,9 @@
  *     (sky_graph_set_option).  Every graph works on the null stream, like the reference's entry functions.
  *   - "device pointer" arguments are HIP device addresses on the current device
  *     (from sky_device_malloc, or any other allocator of the same process).
- *   - `seconds` outputs report the kernel region only (launch to completion,
- *     measured with HIP events on the stream the kernels run on), like the
- *     gettimeofday bracket of the reference (src/util.cu:35-44).
+ *   - `seconds` outputs report the kernel region only (start of the first kernel to the end of the last,
+ *     by the device's constant-rate clock), like the gettimeofday bracket of the reference
+ *     (src/util.cu:35-44).
  *   - unreached output slots are never written; callers that want a sentinel
  *     pre-fill with sky_device_fill_u32.
  */

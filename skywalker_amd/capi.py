@@ -47,6 +47,15 @@ def lib():
         L = C.CDLL(LIB_PATH)
         L.sky_last_error.restype = C.c_char_p
         L.sky_version.restype = C.c_char_p
+        # argument types of the calls that programs repeat: ctypes then converts plain numbers by itself, which costs
+        # half of what wrapping each of them here does
+        p, u32, u64, f32 = C.c_void_p, C.c_uint32, C.c_uint64, C.c_float
+        walk_out = [p, p, p, p]
+        L.sky_alias_build_all.argtypes = [p, p]
+        L.sky_alias_build_from_weights.argtypes = [p, p, p]
+        L.sky_walk_offline.argtypes = [p, p, u32, u32, f32, u64] + walk_out
+        L.sky_walk_online.argtypes = [p, C.c_int, f32, f32, p, u32, u32, f32, u64] + walk_out
+        L.sky_sample_offline.argtypes = L.sky_sample_online.argtypes = [p, p, u32, p, u32, u64] + walk_out
         _lib = L
     return _lib
 
@@ -136,6 +145,9 @@ class Graph:
         V, E, md = C.c_uint32(0), C.c_uint32(0), C.c_uint32(0)
         _ck(lib().sky_graph_info(self.h, C.byref(V), C.byref(E), C.byref(md)))
         self.V, self.E, self.max_degree = V.value, E.value, md.value
+        # where calls on this graph leave their counts and times
+        self._sampled, self._sec = C.c_uint64(0), C.c_double(0)
+        self._sampled_ref, self._sec_ref = C.byref(self._sampled), C.byref(self._sec)
 
     @classmethod
     def upload(cls, xadj, adjncy, adjwgt):
@@ -179,15 +191,13 @@ class Graph:
 
     def build_tables(self):
         """ConstructTable: returns the kernel-region seconds."""
-        sec = C.c_double(0)
-        _ck(lib().sky_alias_build_all(self.h, C.byref(sec)))
-        return sec.value
+        _ck(lib().sky_alias_build_all(self.h, self._sec_ref))
+        return self._sec.value
 
     def build_tables_from_weights(self, weights):
         """Tables from a caller's device array of E floats (a DeviceArray) instead of the graph's own weights."""
-        sec = C.c_double(0)
-        _ck(lib().sky_alias_build_from_weights(self.h, weights.ptr, C.byref(sec)))
-        return sec.value
+        _ck(lib().sky_alias_build_from_weights(self.h, weights.ptr, self._sec_ref))
+        return self._sec.value
 
     def build_profile(self):
         names = (C.c_char_p * 64)()
@@ -222,10 +232,8 @@ class Graph:
             lengths = DeviceArray(N, np.uint32, fill=0)
         else:
             paths, lengths = out
-        sampled, sec = C.c_uint64(0), C.c_double(0)
-        _ck(fn(self.h, *pre, seeds_d.ptr, C.c_uint32(N), C.c_uint32(length), C.c_float(stop_prob), C.c_uint64(seed),
-               paths.ptr, lengths.ptr, C.byref(sampled), C.byref(sec)))
-        return paths, lengths, sampled.value, sec.value
+        _ck(fn(self.h, *pre, seeds_d.ptr, N, length, stop_prob, seed, paths.ptr, lengths.ptr, self._sampled_ref, self._sec_ref))
+        return paths, lengths, self._sampled.value, self._sec.value
 
     def walk_offline(self, seeds, length, stop_prob, seed, out=None):
         """OfflineWalk: returns (paths DeviceArray, lengths DeviceArray, sampled, seconds)."""
@@ -245,23 +253,21 @@ class Graph:
 
     def walk_online(self, bias_kind, p, q, seeds, length, stop_prob, seed, out=None):
         """OnlineWalkShMem."""
-        return self._walk(lib().sky_walk_online, (C.c_int(bias_kind), C.c_float(p), C.c_float(q)), seeds, length,
+        return self._walk(lib().sky_walk_online, (bias_kind, p, q), seeds, length,
                           stop_prob, seed, out)
 
     def _sample(self, fn, seeds, fanout, seed, out=None):
         seeds_d = seeds if isinstance(seeds, DeviceArray) else DeviceArray.from_host(np.asarray(seeds, np.uint32))
         N = seeds_d.count
-        fan = np.asarray(fanout, np.uint32)
-        lps, slen = sample_layout(fan)
+        fan = (C.c_uint32 * len(fanout))(*[int(k) for k in fanout])
         if out is None:
+            lps, slen = sample_layout(fanout)
             data = DeviceArray(N * lps, np.uint32, fill=FILL)
             sl = DeviceArray(N * slen, np.uint32, fill=0)
         else:
             data, sl = out
-        sampled, sec = C.c_uint64(0), C.c_double(0)
-        _ck(fn(self.h, seeds_d.ptr, C.c_uint32(N), _p(fan), C.c_uint32(len(fan)), C.c_uint64(seed), data.ptr, sl.ptr,
-               C.byref(sampled), C.byref(sec)))
-        return data, sl, sampled.value, sec.value
+        _ck(fn(self.h, seeds_d.ptr, N, fan, len(fan), seed, data.ptr, sl.ptr, self._sampled_ref, self._sec_ref))
+        return data, sl, self._sampled.value, self._sec.value
 
     def sample_offline(self, seeds, fanout, seed, out=None):
         """OfflineSample."""

@@ -268,6 +268,12 @@ __global__ __launch_bounds__(256) void build_group_kernel(const RowRef* __restri
   }
 }
 
+__global__ __launch_bounds__(128) void build_begin_kernel(uint32_t* __restrict__ counters, uint32_t words,
+                                                          CallDevice* call) {
+  call_stamp(call);
+  for (uint32_t i = threadIdx.x; i < words; i += 128u) counters[i] = 0;
+}
+
 // ---------------------------------------------------------------- binning
 // `src` lists the vertices to bin (n of them); a null src means vertices 0..n-1.  Block b of the
 // count and scatter kernels owns the items [b * per_block, (b + 1) * per_block): the count kernel
@@ -1206,8 +1212,6 @@ void free_build_scratch(sky_graph* g) {
   g->build_scratch = nullptr;
 }
 
-EventTimer::EventTimer(sky_graph* g) : stream(g->stream), pooled(g->ev), npooled(2) {}
-
 int pool_get(sky_graph* g, int slot, size_t bytes, void** out) {
   sky_graph::PoolBuf& b = g->pool[slot];
   if (b.cap < bytes) {
@@ -1225,10 +1229,6 @@ void pool_release(sky_graph* g) {
     if (b.p) (void)hipFree(b.p);
     b.p = nullptr;
     b.cap = 0;
-  }
-  for (hipEvent_t& e : g->ev) {
-    if (e) (void)hipEventDestroy(e);
-    e = nullptr;
   }
   for (hipStream_t& s : g->side) {
     if (s) (void)hipStreamDestroy(s);
@@ -1323,12 +1323,7 @@ struct StreamSwap {
 
 int EventTimer::mark(const char* name, uint64_t e) {
   hipEvent_t x;
-  if (ev.size() < npooled) {
-    if (!pooled[ev.size()]) SKY_HIP(hipEventCreate(&pooled[ev.size()]));
-    x = pooled[ev.size()];
-  } else {
-    SKY_HIP(hipEventCreate(&x));
-  }
+  SKY_HIP(hipEventCreate(&x));
   SKY_HIP(hipEventRecord(x, stream));
   ev.push_back(x);
   names.push_back(name);
@@ -1338,11 +1333,11 @@ int EventTimer::mark(const char* name, uint64_t e) {
 int EventTimer::finish(std::vector<sky_graph::ProfileEntry>* profile, double* seconds) {
   SKY_HIP(hipStreamSynchronize(stream));
   SKY_HIP(hipGetLastError());
-  if (profile) profile->clear();
+  profile->clear();
   for (size_t i = 1; i < ev.size(); ++i) {
     float ms = 0;
     SKY_HIP(hipEventElapsedTime(&ms, ev[i - 1], ev[i]));
-    if (profile) profile->push_back({names[i], ms, edges[i]});
+    profile->push_back({names[i], ms, edges[i]});
   }
   float total_ms = 0;
   if (ev.size() >= 2) SKY_HIP(hipEventElapsedTime(&total_ms, ev.front(), ev.back()));
@@ -1350,7 +1345,7 @@ int EventTimer::finish(std::vector<sky_graph::ProfileEntry>* profile, double* se
   return SKY_OK;
 }
 EventTimer::~EventTimer() {
-  for (size_t i = npooled; i < ev.size(); ++i) (void)hipEventDestroy(ev[i]);
+  for (hipEvent_t e : ev) (void)hipEventDestroy(e);
 }
 
 int ensure_table_storage(sky_graph* g) {
@@ -1383,7 +1378,7 @@ int prepare_build_scratch(sky_graph* g, uint32_t max_rows) {
 
 // Builds the rows listed in `src` (device array of n vertex ids; null = vertices 0..n-1).
 // prepare_build_scratch(n) and ensure_table_storage must have been called.
-int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm) {
+int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, CallDevice* call) {
   hipStream_t st = g->stream;
   g->has_walk_index = false;  // the table entries it was made from are about to change
   BuildScratch& sc = scratch_of(g);
@@ -1407,13 +1402,14 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm) {
     hipLaunchKernelGGL(small_rows_kernel, dim3((n + per_wave - 1) / per_wave), dim3(64), 0, s, g->xadj, g->adjwgt, src, n,
                        per_wave, g->table, g->valid);
   };
+  // clears the counters of the binning pass and notes when the call began
+  hipLaunchKernelGGL(build_begin_kernel, dim3(1), dim3(128), 0, st, sc.counters, (uint32_t)(COUNTER_BYTES / 4), call);
   if (n > 0) {
     if (small_in_place && !tm) {
       hipStream_t side;
       SKY_TRY(fan.branch(sky_graph::SIDE_STREAMS - 1, &side));
       launch_small(side);
     }
-    SKY_HIP(hipMemsetAsync(sc.counters, 0, COUNTER_BYTES, st));
     // at most BIN_BLOCKS blocks, each a multiple of one scatter step
     const uint32_t step = 256u * BIN_ITEMS;
     const uint32_t per_block = ((n + BIN_BLOCKS - 1) / BIN_BLOCKS + step - 1) / step * step;
@@ -1776,15 +1772,20 @@ int build_rows_dev(sky_graph* g, const uint32_t* src, const uint32_t* n_dev, uin
 int build_all_tables(sky_graph* g, double* seconds) {
   SKY_TRY(ensure_table_storage(g));
   SKY_TRY(prepare_build_scratch(g, g->V));
-  EventTimer tm(g);
-  SKY_TRY(tm.mark("start", 0));
   if (option(g, OPT_BUILD_PROFILE)) {
+    EventTimer tm(g->stream);
+    SKY_TRY(tm.mark("start", 0));
     SKY_TRY(build_rows(g, nullptr, g->V, &tm));
-  } else {  // one bracket around the whole build: no event between the kernels
-    SKY_TRY(build_rows(g, nullptr, g->V, nullptr));
-    SKY_TRY(tm.mark("build", g->E));
+    SKY_TRY(tm.finish(&g->build_profile, seconds));
+  } else {  // no event between the kernels
+    CallDevice* call = nullptr;
+    double sec = 0;
+    SKY_TRY(call_begin(g, &call));
+    SKY_TRY(build_rows(g, nullptr, g->V, nullptr, call));
+    SKY_TRY(call_end(g, nullptr, &sec));
+    g->build_profile.assign(1, {"build", (float)(sec * 1e3), g->E});
+    if (seconds) *seconds = sec;
   }
-  SKY_TRY(tm.finish(&g->build_profile, seconds));
   g->has_tables = true;
   return SKY_OK;
 }

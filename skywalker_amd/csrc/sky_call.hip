@@ -1,0 +1,164 @@
+// End of a call: results and completion through pinned host words (sky_call.h).
+#include <chrono>
+#include <mutex>
+#include <vector>
+
+#include "sky_graph.h"
+
+namespace sky {
+
+// One workgroup: adds up `counts` if there are any, reports.
+__global__ __launch_bounds__(1024) void call_end_kernel(CallDevice* call, CallHost* host, unsigned long long seq,
+                                                        const uint32_t* __restrict__ counts, uint32_t n) {
+  __shared__ unsigned long long s_w[16];
+  unsigned long long t = 0;
+  if (n) {
+    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) t += counts[i];
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
+    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = t;
+    __syncthreads();
+    t = 0;
+    for (uint32_t w = 0; w < blockDim.x / 64; ++w) t += s_w[w];
+  }
+  if (threadIdx.x == 0) call_report(call, host, seq, call->sampled + t);
+}
+
+__global__ __launch_bounds__(256) void sum_counts_kernel(const uint32_t* __restrict__ x, uint64_t n, CallDevice* call) {
+  __shared__ unsigned long long s_w[4];
+  unsigned long long t = 0;
+  for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256u) t += x[i];
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
+  if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = t;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const unsigned long long b = s_w[0] + s_w[1] + s_w[2] + s_w[3];
+    if (b) atomicAdd(&call->sampled, b);
+  }
+}
+
+// The call words of all graphs: chunks of 64, per device, handed out one to a graph for its lifetime.  A chunk none of
+// whose words is in use goes back to the runtime when another one has free words.
+namespace {
+constexpr int CHUNK = 64;
+struct Chunk {
+  int device = 0, used = 0, khz = 0;
+  CallDevice* dev = nullptr;
+  CallHost* host = nullptr;
+  bool taken[CHUNK] = {false};
+};
+std::mutex g_mutex;
+std::vector<Chunk*> g_chunks;
+
+void free_chunk(Chunk* c) {
+  if (c->dev) (void)hipFree(c->dev);
+  if (c->host) (void)hipHostFree(c->host);
+  delete c;
+}
+int take_words(sky_graph* g) {
+  std::lock_guard<std::mutex> lock(g_mutex);
+  Chunk* use = nullptr;
+  for (Chunk* c : g_chunks)
+    if (c->device == g->device && c->used < CHUNK) use = c;
+  if (!use) {
+    Chunk* c = new Chunk();
+    c->device = g->device;
+    auto body = [&]() -> int {
+      SKY_HIP(hipDeviceGetAttribute(&c->khz, hipDeviceAttributeWallClockRate, g->device));
+      if (c->khz <= 0) return fail(SKY_ERR_HIP, "the device reports no wall clock rate");
+      SKY_HIP(hipMalloc((void**)&c->dev, CHUNK * sizeof(CallDevice)));
+      SKY_HIP(hipMemset(c->dev, 0, CHUNK * sizeof(CallDevice)));
+      SKY_HIP(hipHostMalloc((void**)&c->host, CHUNK * sizeof(CallHost), hipHostMallocCoherent | hipHostMallocPortable));
+      return SKY_OK;
+    };
+    const int rc = body();
+    if (rc != SKY_OK) {
+      free_chunk(c);
+      return rc;
+    }
+    for (int k = 0; k < CHUNK; ++k) c->host[k] = CallHost{};
+    g_chunks.push_back(c);
+    use = c;
+  }
+  int k = 0;
+  while (use->taken[k]) ++k;
+  use->taken[k] = true;
+  ++use->used;
+  g->call_dev = use->dev + k;
+  g->call_host = use->host + k;
+  g->call_khz = use->khz;
+  g->call_seq = use->host[k].seq;
+  return SKY_OK;
+}
+}  // namespace
+
+void call_release(sky_graph* g) {
+  if (!g->call_host) return;
+  std::lock_guard<std::mutex> lock(g_mutex);
+  for (size_t i = 0; i < g_chunks.size(); ++i) {
+    Chunk* c = g_chunks[i];
+    if (g->call_host < c->host || g->call_host >= c->host + CHUNK) continue;
+    const size_t k = (size_t)(g->call_host - c->host);
+    if (g->call_dirty) (void)hipMemset(c->dev + k, 0, sizeof(CallDevice));
+    c->taken[k] = false;
+    --c->used;
+    bool other = false;
+    for (Chunk* o : g_chunks) other = other || (o != c && o->device == c->device && o->used < CHUNK);
+    if (c->used == 0 && other) {
+      g_chunks.erase(g_chunks.begin() + (long)i);
+      free_chunk(c);
+    }
+    break;
+  }
+  g->call_dev = nullptr;
+  g->call_host = nullptr;
+}
+
+int call_begin(sky_graph* g, CallDevice** call) {
+  if (!g->call_host) SKY_TRY(take_words(g));
+  if (g->call_dirty) SKY_HIP(hipMemsetAsync(g->call_dev, 0, sizeof(CallDevice), g->stream));
+  g->call_dirty = true;  // until it has ended well
+  *call = g->call_dev;
+  return SKY_OK;
+}
+
+// Up to this many counts are added up by the end kernel itself; more get a grid of their own.
+constexpr uint64_t END_COUNTS = 32768;
+// The host polls this long before it hands the wait to the runtime: a call that takes longer does not notice the
+// five microseconds, and one whose kernels fault ends with the runtime's error instead of polling for ever.
+constexpr auto POLL_FOR = std::chrono::microseconds(3000);
+
+int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
+  hipStream_t st = g->stream;
+  if (n > END_COUNTS) {
+    hipLaunchKernelGGL(sum_counts_kernel, dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 1024)), dim3(256), 0, st, counts,
+                       n, g->call_dev);
+    n = 0;
+  }
+  const unsigned long long seq = ++g->call_seq;
+  hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, st, g->call_dev, g->call_host, seq, counts,
+                     (uint32_t)n);
+  SKY_HIP(hipGetLastError());
+  auto ended = [&] { return __atomic_load_n(&g->call_host->seq, __ATOMIC_ACQUIRE) == seq; };
+  bool done = ended();
+  if (!done) {
+    const auto t0 = std::chrono::steady_clock::now();
+    do {
+      for (int k = 0; k < 64 && !done; ++k) {
+        __builtin_ia32_pause();
+        done = ended();
+      }
+    } while (!done && std::chrono::steady_clock::now() - t0 < POLL_FOR);
+  }
+  if (!done) {
+    SKY_HIP(hipStreamSynchronize(st));
+    if (!ended()) return fail(SKY_ERR_HIP, "the call's end was not reported");
+  }
+  g->call_dirty = false;
+  if (sampled) *sampled = g->call_host->sampled;
+  if (seconds) *seconds = (double)g->call_host->ticks / ((double)g->call_khz * 1e3);
+  return SKY_OK;
+}
+
+}  // namespace sky

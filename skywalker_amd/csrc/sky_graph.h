@@ -2,6 +2,7 @@
 #pragma once
 #include <vector>
 
+#include "sky_call.h"
 #include "sky_common.h"
 
 // The tuning knobs of sky_set_option / sky_graph_set_option.  A graph reads a knob through option(g, ...): its own
@@ -56,15 +57,20 @@ struct sky_graph {
   };
   std::vector<ProfileEntry> build_profile;
 
-  // Device buffers that calls on this graph reuse instead of allocating each time (they only grow), and the two
-  // events that bracket a call's kernel region.
-  enum PoolSlot { POOL_COUNTERS = 0, POOL_BITMAP, POOL_LIST, POOL_SLOTS };
+  // How a call on this graph reports its end (sky_call.h).
+  sky::CallDevice* call_dev = nullptr;
+  sky::CallHost* call_host = nullptr;
+  unsigned long long call_seq = 0;
+  int call_khz = 0;
+  bool call_dirty = false;  // a call has begun and not ended well: its device words may not be zero
+
+  // Device buffers that calls on this graph reuse instead of allocating each time (they only grow).
+  enum PoolSlot { POOL_BITMAP = 0, POOL_LIST, POOL_SLOTS };
   struct PoolBuf {
     void* p = nullptr;
     size_t cap = 0;
   };
   PoolBuf pool[POOL_SLOTS];
-  hipEvent_t ev[2] = {nullptr, nullptr};
   // Pinned host words into which the device reports, step by step, how many walkers of an online walk still walk;
   // the host reads them without waiting (they lag behind the enqueued steps) to stop enqueuing once none does.
   uint32_t* live_report = nullptr;
@@ -125,13 +131,10 @@ struct EventTimer {
   std::vector<hipEvent_t> ev;
   std::vector<const char*> names;
   std::vector<uint64_t> edges;
-  hipEvent_t* pooled = nullptr;  // events that exist already are used first and are not destroyed
-  size_t npooled = 0;
   explicit EventTimer(hipStream_t s) : stream(s) {}
-  EventTimer(sky_graph* g);  // on the graph's stream, with the graph's two events for the first two marks
   ~EventTimer();
   int mark(const char* name, uint64_t edges);
-  // synchronises, then fills `profile` (may be null) and the time from first to last mark
+  // synchronises, then fills `profile` and the time from first to last mark
   int finish(std::vector<sky_graph::ProfileEntry>* profile, double* seconds);
 };
 
@@ -140,7 +143,7 @@ int pool_get(sky_graph* g, int slot, size_t bytes, void** out);
 void pool_release(sky_graph* g);
 int ensure_table_storage(sky_graph* g);
 int prepare_build_scratch(sky_graph* g, uint32_t max_rows);
-int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm);
+int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, CallDevice* call = nullptr);
 int build_all_tables(sky_graph* g, double* seconds);
 // rows of more than 4093 entries: tile-parallel path, and how many tiles per row it accepts
 constexpr uint32_t TILED_TILE = 1024;  // slots per tile of the tile-parallel path

@@ -15,7 +15,8 @@ namespace sky {
 
 __global__ __launch_bounds__(256) void walk_init_kernel(const uint32_t* __restrict__ seeds, uint32_t N, uint32_t len,
                                                         uint32_t V, uint32_t* __restrict__ paths,
-                                                        uint32_t* __restrict__ lengths) {
+                                                        uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
+  call_stamp(call);
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
   if (i >= N) return;
   const uint32_t v = seeds[i];
@@ -81,15 +82,6 @@ __global__ __launch_bounds__(256) void walk_step_kernel(const uint32_t* __restri
   path[s + 1] = adjncy[off + cand];
 }
 
-__global__ __launch_bounds__(256) void sum_lengths_kernel(const uint32_t* __restrict__ lengths, uint32_t N,
-                                                          unsigned long long* __restrict__ out) {
-  unsigned long long t = 0;
-  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < N; i += gridDim.x * 256u) t += lengths[i];
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
-  if ((threadIdx.x & 63) == 0 && t) atomicAdd(out, t);
-}
-
 int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, uint32_t N, uint32_t len,
                          float stop_prob, uint64_t seed, uint32_t* paths, uint32_t* lengths, uint64_t* sampled,
                          double* seconds);
@@ -126,7 +118,7 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
     return SKY_OK;
   }
   hipStream_t st = g->stream;
-  unsigned long long* d_sampled = nullptr;
+  CallDevice* call = nullptr;
   uint32_t *bitmap = nullptr, *list = nullptr, *d_cnt = nullptr;
   const uint32_t words = (g->V + 31) / 32;
   // Without a row too long for the streaming kernel, no step waits for the device: the size of a step's list stays
@@ -148,17 +140,14 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
       for (uint32_t s = 0; s < len; ++s) g->live_report[s] = 0xFFFFFFFFu;  // "not reported yet"
     }
     SKY_TRY(prepare_build_scratch(g, std::min(N, g->V)));
-    SKY_TRY(pool_get(g, sky_graph::POOL_COUNTERS, 64, (void**)&d_sampled));
-    d_cnt = reinterpret_cast<uint32_t*>(d_sampled + 1);
+    SKY_TRY(call_begin(g, &call));
+    d_cnt = call->count;
     SKY_TRY(pool_get(g, sky_graph::POOL_BITMAP, (size_t)words * 4, (void**)&bitmap));
     SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)std::min(N, g->V) * 4, (void**)&list));
-    SKY_HIP(hipMemsetAsync(d_sampled, 0, 8, st));
-    EventTimer tm(g);
-    SKY_TRY(tm.mark("start", 0));
     const uint32_t blocks = (N + 255) / 256;
     if (N) {
       SKY_HIP(hipMemsetAsync(bitmap, 0, (size_t)words * 4, st));
-      hipLaunchKernelGGL(walk_init_kernel, dim3(blocks), dim3(256), 0, st, seeds, N, len, g->V, paths, lengths);
+      hipLaunchKernelGGL(walk_init_kernel, dim3(blocks), dim3(256), 0, st, seeds, N, len, g->V, paths, lengths, call);
       for (uint32_t s = 0; s < len; ++s) {
         SKY_HIP(hipMemsetAsync(d_cnt, 0, 8, st));
         hipLaunchKernelGGL(walk_collect_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, N, len, s, stop_prob, seed,
@@ -179,15 +168,8 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
         hipLaunchKernelGGL(walk_step_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, g->adjncy, g->table, N,
                            len, s, seed, paths, lengths);
       }
-      hipLaunchKernelGGL(sum_lengths_kernel, dim3(std::min<uint32_t>(blocks, 1024)), dim3(256), 0, st, lengths, N,
-                         d_sampled);
     }
-    SKY_TRY(tm.mark("walk", 0));
-    SKY_TRY(tm.finish(nullptr, seconds));
-    unsigned long long h = 0;
-    SKY_HIP(hipMemcpy(&h, d_sampled, 8, hipMemcpyDeviceToHost));
-    if (sampled) *sampled = h;
-    return SKY_OK;
+    return call_end(g, sampled, seconds, lengths, N);
   };
   return body();
 }
@@ -251,29 +233,15 @@ int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, 
                          float stop_prob, uint64_t seed, uint32_t* paths, uint32_t* lengths, uint64_t* sampled,
                          double* seconds) {
   hipStream_t st = g->stream;
-  unsigned long long* d_sampled = nullptr;
-  auto body = [&]() -> int {
-    SKY_TRY(pool_get(g, sky_graph::POOL_COUNTERS, 64, (void**)&d_sampled));
-    SKY_HIP(hipMemsetAsync(d_sampled, 0, 8, st));
-    EventTimer tm(g);
-    SKY_TRY(tm.mark("start", 0));
-    if (N) {
-      const uint32_t blocks = (N + 255) / 256;
-      hipLaunchKernelGGL(walk_init_kernel, dim3(blocks), dim3(256), 0, st, seeds, N, len, g->V, paths, lengths);
-      for (uint32_t s = 0; s < len; ++s)
-        hipLaunchKernelGGL(n2v_step_kernel, dim3(N), dim3(N2V_T), 0, st, g->xadj, g->adjncy, g->adjwgt, len, s, p, q,
-                           stop_prob, seed, paths, lengths);
-      hipLaunchKernelGGL(sum_lengths_kernel, dim3(std::min<uint32_t>(blocks, 1024)), dim3(256), 0, st, lengths, N,
-                         d_sampled);
-    }
-    SKY_TRY(tm.mark("walk", 0));
-    SKY_TRY(tm.finish(nullptr, seconds));
-    unsigned long long h = 0;
-    SKY_HIP(hipMemcpy(&h, d_sampled, 8, hipMemcpyDeviceToHost));
-    if (sampled) *sampled = h;
-    return SKY_OK;
-  };
-  return body();
+  CallDevice* call = nullptr;
+  SKY_TRY(call_begin(g, &call));
+  if (N) {
+    hipLaunchKernelGGL(walk_init_kernel, dim3((N + 255) / 256), dim3(256), 0, st, seeds, N, len, g->V, paths, lengths, call);
+    for (uint32_t s = 0; s < len; ++s)
+      hipLaunchKernelGGL(n2v_step_kernel, dim3(N), dim3(N2V_T), 0, st, g->xadj, g->adjncy, g->adjwgt, len, s, p, q, stop_prob,
+                         seed, paths, lengths);
+  }
+  return call_end(g, sampled, seconds, lengths, N);
 }
 
 }  // namespace sky

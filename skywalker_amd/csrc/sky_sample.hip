@@ -131,23 +131,6 @@ __global__ __launch_bounds__(DISTINCT_T) void sample_hop_distinct_kernel(
   sl[si * g.slen + g.loff + s] = cnt;
 }
 
-// Sampled edges of the call = sum of sample_lengths (as the reference counts them, src/main.cu:378-394): one pass
-// at the end, one atomic per workgroup; a counter bumped by every wavefront of every hop is a hot spot.
-__global__ __launch_bounds__(256) void sum_u32_kernel(const uint32_t* __restrict__ x, uint64_t n,
-                                                      unsigned long long* __restrict__ out) {
-  __shared__ unsigned long long s_w[4];
-  unsigned long long t = 0;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256u) t += x[i];
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
-  if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = t;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned long long b = s_w[0] + s_w[1] + s_w[2] + s_w[3];
-    if (b) atomicAdd(out, b);
-  }
-}
-
 // Collects the distinct vertices of the filled slots of hop h whose table has not been built
 // during this call: first setter of the vertex's bit appends it.  One counter update per workgroup of 1024
 // lanes: every append of a launch goes through one word, and a word serves its atomics one after another
@@ -211,12 +194,17 @@ __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint3
   }
 }
 
+// Start of a call: start vertices in place, counts of children and (online) the bitmap of built rows cleared.
 __global__ __launch_bounds__(256) void sample_init_kernel(const uint32_t* __restrict__ seeds, uint32_t N, uint64_t lps,
-                                                          uint32_t* __restrict__ data) {
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i < N) data[(uint64_t)i * lps] = seeds[i];
+                                                          uint32_t* __restrict__ data, uint32_t* __restrict__ sl,
+                                                          uint64_t nsl, uint32_t* __restrict__ bitmap, uint32_t words,
+                                                          CallDevice* __restrict__ call) {
+  call_stamp(call);
+  const uint64_t i0 = (uint64_t)blockIdx.x * 256u + threadIdx.x, step = (uint64_t)gridDim.x * 256u;
+  for (uint64_t i = i0; i < nsl; i += step) sl[i] = 0;
+  for (uint64_t i = i0; i < words; i += step) bitmap[i] = 0;
+  for (uint64_t i = i0; i < N; i += step) data[i * lps] = seeds[i];
 }
-
 
 // One call of the k-hop sampler, taken apart hop by hop: begin (outputs cleared, start vertices in place), then for
 // every hop frontier (online: the distinct parents whose rows are not built yet), build (online: their rows) and
@@ -232,12 +220,11 @@ struct SampleSession {
   std::vector<uint32_t> fanout;
   std::vector<uint64_t> width, off, loff;
   uint64_t lps = 0, slen = 0;
-  unsigned long long* d_sampled = nullptr;
+  CallDevice* call = nullptr;
   uint32_t *bitmap = nullptr, *list = nullptr, *d_count = nullptr;
   uint32_t frontier_upper = 0;   // most rows the last frontier can hold
   uint32_t frontier_count = 0;   // its size, when the host has read it (dev_sized false)
-  EventTimer tm;
-  explicit SampleSession(sky_graph* g_) : g(g_), tm(g_) {}
+  explicit SampleSession(sky_graph* g_) : g(g_) {}
 
   HopGeom geom(uint32_t h) const {
     HopGeom hg;
@@ -291,10 +278,6 @@ struct SampleSession {
     }
     if ((uint64_t)N * lps > (1ull << 40)) return fail(SKY_ERR_LIMIT, "sample: output too large");
     const uint32_t words = (g->V + 31) / 32;
-    SKY_TRY(pool_get(g, sky_graph::POOL_COUNTERS, 64, (void**)&d_sampled));
-    d_count = reinterpret_cast<uint32_t*>(d_sampled + 1);
-    SKY_HIP(hipMemsetAsync(d_sampled, 0, 8, st));
-    if (N && slen) SKY_HIP(hipMemsetAsync(sample_lengths, 0, (size_t)N * slen * 4, st));
     if (online) {
       SKY_TRY(ensure_table_storage(g));
       if (dev_sized) SKY_TRY(ensure_class_census(g));  // once per graph
@@ -302,9 +285,11 @@ struct SampleSession {
       SKY_TRY(pool_get(g, sky_graph::POOL_BITMAP, (size_t)words * 4, (void**)&bitmap));
       SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)g->V * 4, (void**)&list));
     }
-    SKY_TRY(tm.mark("start", 0));
-    if (online) SKY_HIP(hipMemsetAsync(bitmap, 0, (size_t)words * 4, st));
-    if (N) hipLaunchKernelGGL(sample_init_kernel, dim3((N + 255) / 256), dim3(256), 0, st, seeds, N, lps, data);
+    SKY_TRY(call_begin(g, &call));
+    d_count = call->count;
+    const uint64_t items = std::max<uint64_t>(std::max<uint64_t>((uint64_t)N * slen, online ? words : 0u), 1u);
+    hipLaunchKernelGGL(sample_init_kernel, dim3((uint32_t)std::min<uint64_t>((items + 255) / 256, 2048)), dim3(256), 0, st, seeds,
+                       N, lps, data, sample_lengths, (uint64_t)N * slen, bitmap, online ? words : 0u, call);
     return SKY_OK;
   }
 
@@ -358,18 +343,7 @@ struct SampleSession {
   }
 
   int end(uint64_t* sampled, double* seconds) {
-    hipStream_t st = g->stream;
-    if (N && slen) {
-      const uint64_t n = (uint64_t)N * slen;
-      hipLaunchKernelGGL(sum_u32_kernel, dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 1024)), dim3(256), 0, st,
-                         sample_lengths, n, d_sampled);
-    }
-    SKY_TRY(tm.mark("sample", 0));
-    SKY_TRY(tm.finish(nullptr, seconds));
-    unsigned long long hcount = 0;
-    SKY_HIP(hipMemcpy(&hcount, d_sampled, 8, hipMemcpyDeviceToHost));
-    if (sampled) *sampled = hcount;
-    return SKY_OK;
+    return call_end(g, sampled, seconds, sample_lengths, (uint64_t)N * slen);
   }
 };
 

@@ -61,8 +61,9 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
     const WalkEntry* __restrict__ index, const uint32_t* __restrict__ seeds, const uint32_t* __restrict__ live,
     const uint32_t* __restrict__ n_live_dev, uint32_t n_live, uint32_t V, uint32_t len, uint32_t s_begin,
     uint32_t s_end, float stop_prob, uint64_t seed, uint32_t* __restrict__ paths, uint32_t* __restrict__ lengths,
-    uint32_t* __restrict__ next_live, uint32_t* __restrict__ n_next, unsigned long long* __restrict__ sampled,
+    uint32_t* __restrict__ next_live, uint32_t* __restrict__ n_next, CallDevice* __restrict__ call,
     unsigned long long* __restrict__ block_partials) {
+  if (s_begin == 0) call_stamp(call);
   __shared__ unsigned long long s_part[WALK_BLOCK / 64];
   const uint32_t t = blockIdx.x * WALK_BLOCK + threadIdx.x;
   if (n_live_dev) n_live = min(n_live, *n_live_dev);  // the list's length is only known on the device
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
       block_partials[blockIdx.x] = b;
     }
   } else if ((threadIdx.x & 63) == 0 && tot) {
-    atomicAdd(sampled, tot);
+    atomicAdd(&call->sampled, tot);
   }
 }
 
@@ -155,23 +156,23 @@ template <bool INDEXED>
 static void launch_walk(sky_graph* g, const uint32_t* seeds, const uint32_t* live, const uint32_t* n_live_dev,
                         uint32_t n_live, uint32_t len, uint32_t s_begin, uint32_t s_end, float stop_prob, uint64_t seed,
                         uint32_t* paths, uint32_t* lengths, uint32_t* next_live, uint32_t* n_next,
-                        unsigned long long* sampled, unsigned long long* partials) {
+                        CallDevice* call, unsigned long long* partials) {
   const dim3 grid((n_live + WALK_BLOCK - 1) / WALK_BLOCK), block(WALK_BLOCK);
   if (walk_reads_once(g))
     hipLaunchKernelGGL((walk_offline_kernel<INDEXED, true>), grid, block, 0, g->stream, g->xadj, g->adjncy, g->table,
                        INDEXED ? g->walk_index : nullptr, seeds, live, n_live_dev, n_live, g->V, len, s_begin, s_end, stop_prob,
-                       seed, paths, lengths, next_live, n_next, sampled, partials);
+                       seed, paths, lengths, next_live, n_next, call, partials);
   else
     hipLaunchKernelGGL((walk_offline_kernel<INDEXED, false>), grid, block, 0, g->stream, g->xadj, g->adjncy, g->table,
                        INDEXED ? g->walk_index : nullptr, seeds, live, n_live_dev, n_live, g->V, len, s_begin, s_end, stop_prob,
-                       seed, paths, lengths, next_live, n_next, sampled, partials);
+                       seed, paths, lengths, next_live, n_next, call, partials);
 }
 
 int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, float stop_prob, uint64_t seed,
                  uint32_t* paths, uint32_t* lengths, uint64_t* sampled, double* seconds) {
   hipStream_t st = g->stream;
-  unsigned long long* d_sampled = nullptr;
-  SKY_TRY(pool_get(g, sky_graph::POOL_COUNTERS, 64, (void**)&d_sampled));
+  CallDevice* call = nullptr;
+  SKY_TRY(call_begin(g, &call));
   const uint32_t every = (uint32_t)option(g, OPT_WALK_COMPACT_EVERY);
   const bool segmented = every > 0 && every < len && N > 0;
   const uint32_t nseg = segmented ? (len + every - 1) / every : 1;
@@ -181,16 +182,13 @@ int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, 
     SKY_TRY(pool_get(g, sky_graph::POOL_BITMAP, (size_t)(nseg + 1) * 4, (void**)&counts));
     SKY_HIP(hipMemsetAsync(counts, 0, (size_t)(nseg + 1) * 4, st));
   }
-  SKY_HIP(hipMemsetAsync(d_sampled, 0, 8, st));
-  EventTimer tm(g);
-  SKY_TRY(tm.mark("start", 0));
   auto run = [&](auto... a) {
     if (g->has_walk_index) launch_walk<true>(g, a...);
     else launch_walk<false>(g, a...);
   };
   if (N && !segmented) {
     run(seeds, (const uint32_t*)nullptr, (const uint32_t*)nullptr, N, len, 0u, len, stop_prob, seed, paths, lengths,
-        (uint32_t*)nullptr, (uint32_t*)nullptr, d_sampled, (unsigned long long*)nullptr);
+        (uint32_t*)nullptr, (uint32_t*)nullptr, call, (unsigned long long*)nullptr);
   } else if (N) {
     for (uint32_t k = 0; k < nseg; ++k) {
       const uint32_t s0 = k * every, s1 = std::min(len, s0 + every);
@@ -198,15 +196,10 @@ int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, 
       uint32_t* out = s1 < len ? lists + (size_t)(k & 1) * N : nullptr;
       // the survivors of segment k - 1 are counted in counts[k]; the grid covers all N, blocks past the count leave
       run(seeds, in, k ? counts + k : (const uint32_t*)nullptr, N, len, s0, s1, stop_prob, seed, paths, lengths, out,
-          counts + k + 1, d_sampled, (unsigned long long*)nullptr);
+          counts + k + 1, call, (unsigned long long*)nullptr);
     }
   }
-  SKY_TRY(tm.mark("walk", 0));
-  SKY_TRY(tm.finish(nullptr, seconds));
-  unsigned long long h = 0;
-  SKY_HIP(hipMemcpy(&h, d_sampled, 8, hipMemcpyDeviceToHost));
-  if (sampled) *sampled = h;
-  return SKY_OK;
+  return call_end(g, sampled, seconds);
 }
 
 // ---------------------------------------------------------------- walk index
@@ -217,7 +210,9 @@ constexpr uint32_t IDX_TILE = 1024;
 constexpr uint32_t IDX_ROWS = 4096;  // row offsets of a tile kept in LDS; tiles that span more rows search xadj itself
 
 __global__ __launch_bounds__(256) void index_tile_rows_kernel(const uint32_t* __restrict__ xadj, uint32_t V,
-                                                              uint32_t* __restrict__ row_of_tile) {
+                                                              uint32_t* __restrict__ row_of_tile,
+                                                              CallDevice* __restrict__ call) {
+  call_stamp(call);
   const uint32_t v = blockIdx.x * 256u + threadIdx.x;
   if (v >= V) return;
   const uint32_t lo = xadj[v], hi = xadj[v + 1];
@@ -269,13 +264,12 @@ int build_walk_index(sky_graph* g, double* seconds) {
   const uint32_t ntiles = (g->E + IDX_TILE - 1) / IDX_TILE;
   uint32_t* row_of_tile = nullptr;
   SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)ntiles * 4, (void**)&row_of_tile));
-  EventTimer tm(g);
-  SKY_TRY(tm.mark("start", 0));
-  hipLaunchKernelGGL(index_tile_rows_kernel, dim3((g->V + 255) / 256), dim3(256), 0, st, g->xadj, g->V, row_of_tile);
+  CallDevice* call = nullptr;
+  SKY_TRY(call_begin(g, &call));
+  hipLaunchKernelGGL(index_tile_rows_kernel, dim3((g->V + 255) / 256), dim3(256), 0, st, g->xadj, g->V, row_of_tile, call);
   hipLaunchKernelGGL(index_fill_kernel, dim3(ntiles), dim3(256), 0, st, g->xadj, g->adjncy, g->table, row_of_tile,
                      ntiles, g->V, g->E, g->walk_index);
-  SKY_TRY(tm.mark("index", 0));
-  SKY_TRY(tm.finish(nullptr, seconds));
+  SKY_TRY(call_end(g, nullptr, seconds));
   g->has_walk_index = true;
   return SKY_OK;
 }
@@ -366,7 +360,8 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_kernel(
     const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
     const AliasEntry* __restrict__ table, const uint32_t* __restrict__ seeds, uint32_t N, uint32_t V, uint32_t len,
     float fp, float fq, float fmax, float stop_prob, uint64_t seed, bool once, uint32_t* __restrict__ paths,
-    uint32_t* __restrict__ lengths, unsigned long long* __restrict__ sampled) {
+    uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
+  call_stamp(call);
   const uint32_t i = blockIdx.x * WALK_BLOCK + threadIdx.x;
   uint32_t s = 0;
   if (i < N) {
@@ -406,7 +401,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_kernel(
   unsigned long long t = s;
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
-  if ((threadIdx.x & 63) == 0 && t) atomicAdd(sampled, t);
+  if ((threadIdx.x & 63) == 0 && t) atomicAdd(&call->sampled, t);
 }
 
 // The same walk with 8 lanes per walker, for batches too small to fill the GPU with one walker per lane (a
@@ -449,7 +444,8 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
     const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
     const AliasEntry* __restrict__ table, const uint32_t* __restrict__ seeds, uint32_t N, uint32_t V, uint32_t len,
     float fp, float fq, float fmax, float stop_prob, uint64_t seed, bool once, uint32_t* __restrict__ paths,
-    uint32_t* __restrict__ lengths, unsigned long long* __restrict__ sampled) {
+    uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
+  call_stamp(call);
   const uint32_t i = (blockIdx.x * WALK_BLOCK + threadIdx.x) / N2V_G;
   const bool first = (threadIdx.x & (N2V_G - 1)) == 0;  // the lane that writes for the group
   uint32_t s = 0;
@@ -491,7 +487,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
   unsigned long long t = first ? s : 0u;
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
-  if ((threadIdx.x & 63) == 0 && t) atomicAdd(sampled, t);
+  if ((threadIdx.x & 63) == 0 && t) atomicAdd(&call->sampled, t);
 }
 
 int walk_node2vec_reject(sky_graph* g, float p, float q, const uint32_t* seeds, uint32_t N, uint32_t len,
@@ -502,32 +498,19 @@ int walk_node2vec_reject(sky_graph* g, float p, float q, const uint32_t* seeds, 
   if (!g->has_tables) SKY_TRY(build_all_tables(g, &build_sec));  // first-order tables, built on demand
   const float fp = 1.0f / p, fq = 1.0f / q;
   const float fmax = fmaxf(1.0f, fmaxf(fp, fq));
-  unsigned long long* d_sampled = nullptr;
-  auto body = [&]() -> int {
-    SKY_TRY(pool_get(g, sky_graph::POOL_COUNTERS, 64, (void**)&d_sampled));
-    SKY_HIP(hipMemsetAsync(d_sampled, 0, 8, st));
-    EventTimer tm(g);
-    SKY_TRY(tm.mark("start", 0));
-    if (N && N <= N2V_GROUP_MAX_WALKERS)
-      hipLaunchKernelGGL(walk_n2v_reject_group_kernel,
-                         dim3((uint32_t)(((uint64_t)N * N2V_G + WALK_BLOCK - 1) / WALK_BLOCK)), dim3(WALK_BLOCK), 0, st,
-                         g->xadj, g->adjncy, g->table, seeds, N, g->V, len, fp, fq, fmax, stop_prob, seed, walk_reads_once(g), paths,
-                         lengths, d_sampled);
-    else if (N)
-      hipLaunchKernelGGL(walk_n2v_reject_kernel, dim3((N + WALK_BLOCK - 1) / WALK_BLOCK), dim3(WALK_BLOCK), 0, st,
-                         g->xadj, g->adjncy, g->table, seeds, N, g->V, len, fp, fq, fmax, stop_prob, seed, walk_reads_once(g), paths,
-                         lengths, d_sampled);
-    SKY_TRY(tm.mark("walk", 0));
-    double sec = 0;
-    SKY_TRY(tm.finish(nullptr, &sec));
-    SKY_HIP(hipGetLastError());
-    unsigned long long h = 0;
-    SKY_HIP(hipMemcpy(&h, d_sampled, 8, hipMemcpyDeviceToHost));
-    if (sampled) *sampled = h;
-    if (seconds) *seconds = sec + build_sec;
-    return SKY_OK;
-  };
-  return body();
+  CallDevice* call = nullptr;
+  SKY_TRY(call_begin(g, &call));
+  if (N && N <= N2V_GROUP_MAX_WALKERS)
+    hipLaunchKernelGGL(walk_n2v_reject_group_kernel, dim3((uint32_t)(((uint64_t)N * N2V_G + WALK_BLOCK - 1) / WALK_BLOCK)),
+                       dim3(WALK_BLOCK), 0, st, g->xadj, g->adjncy, g->table, seeds, N, g->V, len, fp, fq, fmax, stop_prob, seed,
+                       walk_reads_once(g), paths, lengths, call);
+  else if (N)
+    hipLaunchKernelGGL(walk_n2v_reject_kernel, dim3((N + WALK_BLOCK - 1) / WALK_BLOCK), dim3(WALK_BLOCK), 0, st, g->xadj,
+                       g->adjncy, g->table, seeds, N, g->V, len, fp, fq, fmax, stop_prob, seed, walk_reads_once(g), paths,
+                       lengths, call);
+  SKY_TRY(call_end(g, sampled, seconds));
+  if (seconds) *seconds += build_sec;
+  return SKY_OK;
 }
 
 }  // namespace sky

@@ -178,13 +178,13 @@ int main(int argc, char* argv[]) {
   const float ms = time * 1000, tp = sampled / time / 1000000;
   const bool show_table = !FLAGS_ol && FLAGS_bias;
   if (FLAGS_csv) {
-    if (show_table) printf("%0.2f,\t", table_time);
-    printf("%0.2f,\t", ms);
+    if (show_table) printf("%0.4f,\t", table_time);
+    printf("%0.4f,\t", ms);
     printf("%0.2f,\n", tp);
   } else {
-    if (show_table) printf("%0.2f\t", table_time);
+    if (show_table) printf("%0.4f\t", table_time);
     printf("\n");
-    printf("%0.2f\t", ms);
+    printf("%0.4f\t", ms);
     printf("\n");
     printf("%0.2f\t", tp);
     printf("\n");
