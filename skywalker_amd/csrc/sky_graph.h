@@ -65,7 +65,7 @@ struct sky_graph {
   bool call_dirty = false;  // a call has begun and not ended well: its device words may not be zero
 
   // Device buffers that calls on this graph reuse instead of allocating each time (they only grow).
-  enum PoolSlot { POOL_BITMAP = 0, POOL_LIST, POOL_SLOTS };
+  enum PoolSlot { POOL_BITMAP = 0, POOL_LIST, POOL_TOTALS, POOL_SLOTS };
   struct PoolBuf {
     void* p = nullptr;
     size_t cap = 0;

@@ -7,8 +7,9 @@
 // slots s*fanout[h+1].. of hop h+1; sample_lengths holds one count per parent slot of every hop
 // but the last.  A parent of degree deg with fanout k contributes all its neighbours when
 // k >= deg, else k alias draws with replacement; draw i of slot s uses
-// Philox(seed; seed index, s*k + i, h, DOM_SAMPLE).  One lane per (seed, slot, draw), one launch
-// per hop: no device-side queues, and the result does not depend on scheduling.
+// Philox(seed; seed index, s*k + i, h, DOM_SAMPLE).  One workgroup per start vertex takes it through all
+// hops (or through one, when the rows of the next hop are built in between): no device-side queues, and the
+// result does not depend on scheduling.
 //
 // Online mode builds the table of every distinct frontier vertex, once, through the same
 // kernels as the offline build (into the graph's table storage), then samples the hop.
@@ -33,57 +34,109 @@ __device__ __forceinline__ bool slot_filled(const HopGeom& g, const uint32_t* sl
   return sl[si * g.slen + g.loff_prev + s32 / g.fan_h] > s32 % g.fan_h;
 }
 
-// One lane per (seed, slot, draw).  `narrow` (N * width * k below 2^32, the usual case) keeps the index
-// arithmetic in 32 bits: three 64-bit divisions per lane cost more than the draw itself.
-__global__ __launch_bounds__(256) void sample_hop_kernel(const uint32_t* __restrict__ xadj,
-                                                         const uint32_t* __restrict__ adjncy,
-                                                         const AliasEntry* __restrict__ table,
-                                                         const int8_t* __restrict__ valid, uint64_t total,
-                                                         uint32_t V, HopGeom g, uint64_t seed, bool narrow,
-                                                         uint32_t* __restrict__ data,
-                                                         uint32_t* __restrict__ sl) {
-  const uint64_t tid = (uint64_t)blockIdx.x * 256u + threadIdx.x;
-  if (tid < total) {
-    uint64_t si, s;
-    uint32_t i;
-    if (narrow) {
-      const uint32_t t32 = (uint32_t)tid, width = (uint32_t)g.width;
-      const uint32_t parent = t32 / g.k;
-      i = t32 - parent * g.k;
-      const uint32_t si32 = parent / width;
-      si = si32;
-      s = parent - si32 * width;
-    } else {
-      const uint64_t per_seed = g.width * g.k;
-      const uint64_t rem = tid % per_seed;
-      si = tid / per_seed;
-      s = rem / g.k;
-      i = (uint32_t)(rem % g.k);
-    }
-    if (slot_filled(g, sl, si, s)) {
-      const uint32_t v = data[si * g.lps + g.off + s];
-      uint32_t o = 0, deg = 0;
-      if (v < V && valid[v]) {  // a seed that does not exist, or a row without weight, has no children
-        o = xadj[v];
-        deg = xadj[v + 1] - o;
+constexpr uint32_t SAMPLE_HOPS = 7;  // sky_sample_layout takes at most 8 levels
+struct SampleArgs {
+  const uint32_t *xadj, *adjncy;
+  const AliasEntry* table;
+  const int8_t* valid;
+  const uint32_t* seeds;  // read at hop 0, whose slots this kernel then writes; null: they are in place
+  uint32_t *data, *sl;
+  uint32_t* totals;  // children of a start vertex over all hops so far (null: not wanted)
+  uint32_t V, h0, h1;  // hops [h0, h1)
+  uint32_t parts;      // workgroups per start vertex (1 unless h1 == h0 + 1)
+  uint32_t lanes;      // lanes per start vertex (a power of two; 64 when parts > 1)
+  uint64_t first, N;   // start vertices [first, N)
+  CallDevice* call;    // stamped by the call's first kernel (null: another kernel was)
+  uint64_t seed;
+  HopGeom hop[SAMPLE_HOPS];
+};
+
+// The parent in slot s of hop g.h, V when the slot is not filled.
+__device__ __forceinline__ uint32_t parent_of(const SampleArgs& a, const HopGeom& g, uint64_t si, uint32_t s) {
+  if (g.h == 0 && a.seeds) return a.seeds[si];
+  return slot_filled(g, a.sl, si, s) ? a.data[si * g.lps + g.off + s] : 0xFFFFFFFFu;
+}
+
+// Children with replacement: one lane per (slot, draw), U of them at a time so that their chains of four dependent
+// loads overlap.  What bounds a hop is that chain, not its bytes; a wavefront for itself is the cheapest unit that
+// waits for it: no barrier between hops, and the hops of one start vertex follow one another without the rest of the
+// batch (one launch per hop over all slots, filled or not, took 117 us for the 40,000 x 25 x 10 batch on the scale-22
+// graph, most of its 10 M lanes idle).
+constexpr int SAMPLE_T = 64, SAMPLE_U = 4;
+__global__ __launch_bounds__(SAMPLE_T) void sample_draw_kernel(SampleArgs a) {
+  constexpr int U = SAMPLE_U;
+  if (a.h0 == 0) call_stamp(a.call);
+  // start vertices with few draws share the wavefront, a.lanes lanes each
+  const uint32_t T = a.lanes, tid = threadIdx.x & (T - 1), part = blockIdx.x % a.parts;
+  const uint64_t si = a.first + (uint64_t)(blockIdx.x / a.parts) * (SAMPLE_T / T) + threadIdx.x / T;
+  const bool own = si < a.N;
+  uint32_t mine = 0;
+  for (uint32_t h = a.h0; h < a.h1; ++h) {
+    const HopGeom& g = a.hop[h];
+    const uint64_t total = g.width * g.k;  // at most 2^32
+    if (h == 0 && a.seeds && part == 0 && tid == 0 && own) a.data[si * g.lps] = a.seeds[si];
+    for (uint64_t j0 = (uint64_t)part * (T * U); j0 < total; j0 += (uint64_t)a.parts * (T * U)) {
+      uint32_t s[U], i[U], v[U], o[U], deg[U], cand[U], child[U];
+      bool in[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint64_t j = j0 + u * T + tid;
+        in[u] = own && j < total;
+        s[u] = (uint32_t)j / g.k;
+        i[u] = (uint32_t)j - s[u] * g.k;
+        v[u] = in[u] ? parent_of(a, g, si, s[u]) : 0xFFFFFFFFu;
       }
-      if (deg != 0) {
-        uint32_t* out = data + si * g.lps + g.off_next + s * g.k;
-        uint32_t cnt;
-        if (g.k >= deg) {
-          cnt = deg;
-          if (i < deg) out[i] = adjncy[o + i];
-        } else {
-          cnt = g.k;
-          const u32x4 r = philox(seed, (uint32_t)si, (uint32_t)(s * g.k + i), g.h, DOM_SAMPLE);
-          const uint32_t col = __umulhi(r.x, deg);
-          const AliasEntry e = table[o + col];
-          const uint32_t cand = u24(r.y) < e.prob ? col : e.alias;
-          out[i] = adjncy[o + cand];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        o[u] = deg[u] = 0;
+        if (v[u] < a.V) {
+          o[u] = a.xadj[v[u]];
+          deg[u] = a.xadj[v[u] + 1] - o[u];
         }
-        if (i == 0) sl[si * g.slen + g.loff + s] = cnt;
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        // a row without weight has no children: its entries say so where one is drawn, its flag where all are copied
+        cand[u] = SKY_INVALID;
+        if (deg[u] > g.k) {
+          const u32x4 r = philox(a.seed, (uint32_t)si, s[u] * g.k + i[u], g.h, DOM_SAMPLE);
+          const uint32_t col = __umulhi(r.x, deg[u]);
+          const AliasEntry e = a.table[o[u] + col];
+          cand[u] = u24(r.y) < e.prob ? col : e.alias;
+        } else if (deg[u]) {
+          if (!a.valid[v[u]]) deg[u] = 0;
+          if (i[u] < deg[u]) cand[u] = i[u];
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        child[u] = 0;
+        if (cand[u] != SKY_INVALID) child[u] = a.adjncy[o[u] + cand[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (!in[u]) continue;
+        if (cand[u] != SKY_INVALID) a.data[si * g.lps + g.off_next + (uint64_t)s[u] * g.k + i[u]] = child[u];
+        if (i[u] == 0) {
+          const uint32_t cnt = cand[u] != SKY_INVALID ? min(deg[u], g.k) : 0u;
+          a.sl[si * g.slen + g.loff + s[u]] = cnt;
+          mine += cnt;
+        }
       }
     }
+    if (h + 1 < a.h1) {  // the next hop reads what this wavefront has just written
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+  }
+  if (a.totals) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      const uint32_t o = (uint32_t)__shfl_xor((int)mine, m, 64);
+      if ((uint32_t)m < T) mine += o;
+    }
+    if (tid == 0 && own) a.totals[si] = (a.h0 ? a.totals[si] : 0u) + mine;
   }
 }
 
@@ -92,43 +145,102 @@ __global__ __launch_bounds__(256) void sample_hop_kernel(const uint32_t* __restr
 // dropped, a parent may end with fewer than k children), made sequential so that the result does not depend on
 // scheduling: draw i of slot s tries Philox(seed; seed index, s*k + i, h + 256 t, DOM_SAMPLE) for t = 0..10 and
 // keeps the first candidate slot that no earlier draw of this parent kept; the children are written densely in
-// the order of i.  One lane per (seed, slot); the slots it has kept so far sit in LDS, one column per lane.
-constexpr int DISTINCT_T = 128;          // threads per workgroup
+// the order of i.
+// A group of G lanes (the power of two that holds k) shares a parent, one draw per lane.  All draws take their first
+// candidate at once.  Let f be the first draw whose candidate equals that of an earlier one: the draws before it are
+// final, and every draw from f on whose candidate one of those has kept goes on to its next try, again all at once,
+// until no two candidates are equal.  The sequential rule comes out of this exactly, in as many rounds of dependent
+// loads as candidates collide in a row, where one lane per parent took one per try: hop 1 of a 1024-seed batch with
+// fanout 25 197 -> 17 us.
 constexpr uint32_t DISTINCT_MAX_K = 64;  // largest fanout of this rule
 constexpr uint32_t DISTINCT_ROUNDS = 11;
-__global__ __launch_bounds__(DISTINCT_T) void sample_hop_distinct_kernel(
-    const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy, const AliasEntry* __restrict__ table,
-    const int8_t* __restrict__ valid, uint64_t total, uint32_t V, HopGeom g, uint64_t seed,
-    uint32_t* __restrict__ data, uint32_t* __restrict__ sl) {
-  __shared__ uint32_t s_taken[DISTINCT_MAX_K][DISTINCT_T];
-  const uint64_t tid = (uint64_t)blockIdx.x * DISTINCT_T + threadIdx.x;
-  if (tid >= total) return;
-  const uint64_t si = tid / g.width, s = tid % g.width;
-  if (!slot_filled(g, sl, si, s)) return;
-  const uint32_t v = data[si * g.lps + g.off + s];
-  if (v >= V || !valid[v]) return;
-  const uint32_t o = xadj[v], deg = xadj[v + 1] - o;
-  if (deg == 0) return;
-  uint32_t* out = data + si * g.lps + g.off_next + s * g.k;
-  uint32_t cnt = 0;
-  if (g.k >= deg) {
-    for (; cnt < deg; ++cnt) out[cnt] = adjncy[o + cnt];
-  } else {
-    for (uint32_t i = 0; i < g.k; ++i)
-      for (uint32_t t = 0; t < DISTINCT_ROUNDS; ++t) {
-        const u32x4 r = philox(seed, (uint32_t)si, (uint32_t)(s * g.k + i), g.h + 256u * t, DOM_SAMPLE);
-        const uint32_t col = __umulhi(r.x, deg);
-        const AliasEntry e = table[o + col];
-        const uint32_t cand = u24(r.y) < e.prob ? col : e.alias;
-        bool seen = false;
-        for (uint32_t j = 0; j < cnt; ++j) seen = seen || s_taken[j][threadIdx.x] == cand;
-        if (seen) continue;
-        s_taken[cnt][threadIdx.x] = cand;
-        out[cnt++] = adjncy[o + cand];
-        break;
+__device__ __forceinline__ uint32_t distinct_lanes(uint32_t k) { return k <= 4 ? 4u : k == 64u ? 64u : 1u << (32 - __clz((int)(k - 1))); }
+
+// T = 256 spreads the parents of one start vertex over four wavefronts, for batches of a few start vertices.
+template <int T>
+__global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
+  __shared__ __align__(16) uint32_t s_c[T];
+  __shared__ uint32_t s_n[T / 64];
+  if (a.h0 == 0) call_stamp(a.call);
+  const uint64_t si = a.first + blockIdx.x / a.parts;
+  const uint32_t part = blockIdx.x % a.parts, tid = threadIdx.x, lane = tid & 63;
+  uint32_t mine = 0;
+  for (uint32_t h = a.h0; h < a.h1; ++h) {
+    const HopGeom& g = a.hop[h];
+    const uint32_t k = g.k, G = distinct_lanes(k), i = tid & (G - 1), gbase = tid - i;
+    const unsigned long long gm = G == 64 ? ~0ull : ((1ull << G) - 1ull);
+    auto group_mask = [&](bool p) { return (__ballot(p) >> (lane & ~(G - 1))) & gm; };
+    if (h == 0 && a.seeds && part == 0 && tid == 0) a.data[si * g.lps] = a.seeds[si];
+    const uint32_t groups = T / G;
+    for (uint64_t s0 = (uint64_t)part * groups; s0 < g.width; s0 += (uint64_t)a.parts * groups) {
+      const uint64_t slot = s0 + tid / G;
+      const uint32_t s = (uint32_t)slot;
+      const bool in = slot < g.width;
+      const uint32_t v = in ? parent_of(a, g, si, s) : 0xFFFFFFFFu;
+      uint32_t o = 0, deg = 0;
+      if (v < a.V && a.valid[v]) {
+        o = a.xadj[v];
+        deg = a.xadj[v + 1] - o;
       }
+      uint32_t cand = 0, child = 0, t = 0;
+      bool live = i < min(deg, k);  // a draw that keeps something, as far as is known
+      auto take = [&] {
+        const u32x4 r = philox(a.seed, (uint32_t)si, s * k + i, g.h + 256u * t, DOM_SAMPLE);
+        const uint32_t col = __umulhi(r.x, deg);
+        const AliasEntry e = a.table[o + col];
+        cand = u24(r.y) < e.prob ? col : e.alias;
+        child = a.adjncy[o + cand];
+      };
+      if (live) {
+        if (deg > k) take();
+        else child = a.adjncy[o + (cand = i)];  // all neighbours
+      }
+      for (;;) {
+        s_c[tid] = cand;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        unsigned long long same = 0;  // earlier draws of the group with this draw's candidate
+        for (uint32_t j = 0; j < k; j += 4) {
+          const uint4 c = *reinterpret_cast<const uint4*>(s_c + gbase + j);
+          const uint32_t m = (c.x == cand ? 1u : 0u) | (c.y == cand ? 2u : 0u) | (c.z == cand ? 4u : 0u) | (c.w == cand ? 8u : 0u);
+          same |= (unsigned long long)m << j;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the next round's candidates stay behind these reads
+        __builtin_amdgcn_wave_barrier();
+        const unsigned long long alive = group_mask(live);
+        same &= alive & ((1ull << i) - 1ull);
+        const unsigned long long bad = group_mask(live && same != 0);
+        if (!__any(bad != 0)) break;
+        if (bad) {
+          const uint32_t f = (uint32_t)__ffsll((long long)bad) - 1;
+          if (live && i >= f && (same & ((1ull << f) - 1ull))) {  // a final draw holds the candidate
+            if (++t == DISTINCT_ROUNDS) live = false;
+            else take();
+          }
+        }
+      }
+      const unsigned long long kept = group_mask(live);
+      if (live) a.data[si * g.lps + g.off_next + slot * k + (uint32_t)__popcll(kept & ((1ull << i) - 1ull))] = child;
+      if (in && i == 0) {
+        a.sl[si * g.slen + g.loff + s] = (uint32_t)__popcll(kept);
+        mine += (uint32_t)__popcll(kept);
+      }
+    }
+    if (h + 1 < a.h1) __syncthreads();  // the next hop reads what this workgroup has just written
   }
-  sl[si * g.slen + g.loff + s] = cnt;
+  if (a.totals) {
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) mine += (uint32_t)__shfl_xor((int)mine, m, 64);
+    if (lane == 0) s_n[tid >> 6] = mine;
+    __syncthreads();
+    if (tid == 0) {
+      mine = a.h0 ? a.totals[si] : 0u;
+#pragma unroll
+      for (int w = 0; w < T / 64; ++w) mine += s_n[w];
+      a.totals[si] = mine;
+    }
+  }
 }
 
 // Collects the distinct vertices of the filled slots of hop h whose table has not been built
@@ -138,7 +250,7 @@ __global__ __launch_bounds__(DISTINCT_T) void sample_hop_distinct_kernel(
 constexpr int COLLECT_T = 1024;
 __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint32_t* __restrict__ data,
                                                                      const uint32_t* __restrict__ sl, uint64_t total,
-                                                                     uint32_t V, HopGeom g, uint32_t* __restrict__ bitmap,
+                                                                     uint32_t V, HopGeom g, uint32_t* bitmap,
                                                                      uint32_t* __restrict__ list,
                                                                      uint32_t* __restrict__ count) {
   __shared__ uint32_t s_n[COLLECT_T / 64];
@@ -162,20 +274,12 @@ __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint3
       live = v < V;
     }
   }
-  // The draws of a hop land on a few well-connected vertices again and again: the lanes of the wavefront that hold
-  // the same vertex send one atomic between them (the lanes take turns by distinct vertex, at most 64 short rounds).
-  {
-    unsigned long long todo = __ballot(live);
-    while (todo) {
-      const int first = __ffsll((long long)todo) - 1;
-      const uint32_t v0 = (uint32_t)__shfl((int)v, first, 64);
-      const unsigned long long same = __ballot(live && v == v0);
-      if (lane == first) {
-        const uint32_t bit = 1u << (v & 31);
-        fresh = !(atomicOr(&bitmap[v >> 5], bit) & bit);
-      }
-      todo &= ~same;
-    }
+  // The draws of a hop land on a few well-connected vertices again and again.  A bit that reads as set needs no
+  // atomic (bits are never cleared during a call; one that another XCD has set a moment ago may still read as clear,
+  // and then the atomic decides): 94 -> 23 us for a million slots of which a quarter is filled.
+  if (live) {
+    const uint32_t bit = 1u << (v & 31);
+    if (!(bitmap[v >> 5] & bit)) fresh = !(atomicOr(&bitmap[v >> 5], bit) & bit);
   }
   const unsigned long long m = __ballot(fresh);
   if (lane == 0) s_n[wave] = (uint32_t)__popcll(m);
@@ -194,14 +298,12 @@ __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint3
   }
 }
 
-// Start of a call: start vertices in place, counts of children and (online) the bitmap of built rows cleared.
+// Start of an online call: start vertices in place, the bitmap of built rows cleared.
 __global__ __launch_bounds__(256) void sample_init_kernel(const uint32_t* __restrict__ seeds, uint32_t N, uint64_t lps,
-                                                          uint32_t* __restrict__ data, uint32_t* __restrict__ sl,
-                                                          uint64_t nsl, uint32_t* __restrict__ bitmap, uint32_t words,
-                                                          CallDevice* __restrict__ call) {
+                                                          uint32_t* __restrict__ data, uint32_t* __restrict__ bitmap,
+                                                          uint32_t words, CallDevice* __restrict__ call) {
   call_stamp(call);
   const uint64_t i0 = (uint64_t)blockIdx.x * 256u + threadIdx.x, step = (uint64_t)gridDim.x * 256u;
-  for (uint64_t i = i0; i < nsl; i += step) sl[i] = 0;
   for (uint64_t i = i0; i < words; i += step) bitmap[i] = 0;
   for (uint64_t i = i0; i < N; i += step) data[i * lps] = seeds[i];
 }
@@ -222,6 +324,7 @@ struct SampleSession {
   uint64_t lps = 0, slen = 0;
   CallDevice* call = nullptr;
   uint32_t *bitmap = nullptr, *list = nullptr, *d_count = nullptr;
+  uint32_t* totals = nullptr;    // children of each start vertex, when the kernels add them up
   uint32_t frontier_upper = 0;   // most rows the last frontier can hold
   uint32_t frontier_count = 0;   // its size, when the host has read it (dev_sized false)
   explicit SampleSession(sky_graph* g_) : g(g_) {}
@@ -287,9 +390,10 @@ struct SampleSession {
     }
     SKY_TRY(call_begin(g, &call));
     d_count = call->count;
-    const uint64_t items = std::max<uint64_t>(std::max<uint64_t>((uint64_t)N * slen, online ? words : 0u), 1u);
-    hipLaunchKernelGGL(sample_init_kernel, dim3((uint32_t)std::min<uint64_t>((items + 255) / 256, 2048)), dim3(256), 0, st, seeds,
-                       N, lps, data, sample_lengths, (uint64_t)N * slen, bitmap, online ? words : 0u, call);
+    if (N && one_workgroup()) SKY_TRY(pool_get(g, sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
+    if (online)
+      hipLaunchKernelGGL(sample_init_kernel, dim3(std::min((std::max(N, words) + 255) / 256, 2048u)), dim3(256), 0, st, seeds, N,
+                         lps, data, bitmap, words, call);
     return SKY_OK;
   }
 
@@ -324,25 +428,58 @@ struct SampleSession {
     return rc;
   }
 
-  int draw(uint32_t h) {
+  // Passes a wavefront (distinct children: a workgroup of 256) would need for one start vertex at hop h.
+  uint64_t passes(uint32_t h) const {
+    const uint64_t per_pass = distinct ? (fanout[h + 1] <= 16 ? 16u : fanout[h + 1] <= 32 ? 8u : 4u) : (uint64_t)SAMPLE_T * SAMPLE_U;
+    const uint64_t items = distinct ? width[h] : width[h] * fanout[h + 1];
+    return (items + per_pass - 1) / per_pass;
+  }
+  // A workgroup takes its start vertex through every hop when the widest of them keeps it busy for a few passes only, or
+  // when there are start vertices enough to fill the GPU anyway (8,192 wavefronts); otherwise several workgroups
+  // share a start vertex, hop by hop.
+  bool one_workgroup() const { return passes(hops - 2) <= 8 || N >= 8192; }
+
+  int draw(uint32_t h0, uint32_t h1) {
     if (!N) return SKY_OK;
     hipStream_t st = g->stream;
-    const HopGeom hg = geom(h);
-    const uint64_t total = (uint64_t)N * hg.width * hg.k;
-    if (total > 0xFFFFFFFFull * 256ull) return fail(SKY_ERR_LIMIT, "sample: hop too large for one launch");
-    if (distinct) {
-      const uint64_t slots = (uint64_t)N * hg.width;
-      hipLaunchKernelGGL(sample_hop_distinct_kernel, dim3((uint32_t)((slots + DISTINCT_T - 1) / DISTINCT_T)),
-                         dim3(DISTINCT_T), 0, st, g->xadj, g->adjncy, g->table, g->valid, slots, g->V, hg, seed, data,
-                         sample_lengths);
-      return SKY_OK;
+    SampleArgs a = {};
+    a.xadj = g->xadj;
+    a.adjncy = g->adjncy;
+    a.table = g->table;
+    a.valid = g->valid;
+    a.seeds = online ? nullptr : seeds;
+    a.call = online ? nullptr : call;
+    a.data = data;
+    a.sl = sample_lengths;
+    a.totals = totals;
+    a.V = g->V;
+    a.h0 = h0;
+    a.h1 = h1;
+    a.N = N;
+    a.seed = seed;
+    for (uint32_t h = h0; h < h1; ++h) a.hop[h] = geom(h);
+    const uint64_t parts = totals ? 1 : std::min<uint64_t>(passes(h0), 65536);
+    a.parts = (uint32_t)parts;
+    a.lanes = 64;
+    if (totals && !distinct) {
+      const uint64_t draws = width[h1 - 1] * fanout[h1];
+      while (a.lanes > 1 && draws <= a.lanes / 2) a.lanes /= 2;
     }
-    hipLaunchKernelGGL(sample_hop_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, st, g->xadj, g->adjncy,
-                       g->table, g->valid, total, g->V, hg, seed, total <= 0xFFFFFFFFull, data, sample_lengths);
+    // T = 64 as soon as that fills the GPU with wavefronts
+    const uint32_t T = distinct && (N < 4096 || parts > 1) ? 256 : 64, per_block = distinct ? 1 : SAMPLE_T / a.lanes;
+    const uint64_t most = 0xFFFFFFFFull / T / parts * per_block;  // start vertices of one launch (below 2^32 threads)
+    for (a.first = 0; a.first < N; a.first += most) {
+      const dim3 grid((uint32_t)((std::min<uint64_t>(most, N - a.first) + per_block - 1) / per_block * parts));
+      if (!distinct) hipLaunchKernelGGL(sample_draw_kernel, grid, dim3(SAMPLE_T), 0, st, a);
+      else if (T == 64) hipLaunchKernelGGL(sample_distinct_kernel<64>, grid, dim3(64), 0, st, a);
+      else hipLaunchKernelGGL(sample_distinct_kernel<256>, grid, dim3(256), 0, st, a);
+      a.call = nullptr;
+    }
     return SKY_OK;
   }
 
   int end(uint64_t* sampled, double* seconds) {
+    if (totals) return call_end(g, sampled, seconds, totals, N);
     return call_end(g, sampled, seconds, sample_lengths, (uint64_t)N * slen);
   }
 };
@@ -351,10 +488,14 @@ int sample_khop(sky_graph* g, bool online, const uint32_t* seeds, uint32_t N, co
                 uint64_t seed, uint32_t* data, uint32_t* sample_lengths, uint64_t* sampled, double* seconds) {
   SampleSession s(g);
   SKY_TRY(s.begin(online, seeds, N, fanout, hops, seed, data, sample_lengths));
+  if (!s.online && s.totals) {
+    SKY_TRY(s.draw(0, hops - 1));
+    return s.end(sampled, seconds);
+  }
   for (uint32_t h = 0; h + 1 < hops; ++h) {
     SKY_TRY(s.frontier(h));
     SKY_TRY(s.build(nullptr));
-    SKY_TRY(s.draw(h));
+    SKY_TRY(s.draw(h, h + 1));
   }
   return s.end(sampled, seconds);
 }
@@ -383,7 +524,7 @@ int sample_session_frontier(SampleSession* s, uint32_t hop, const uint32_t** lis
 int sample_session_hop(SampleSession* s, uint32_t hop, const float* weights) {
   if (hop + 1 >= s->hops) return fail(SKY_ERR_ARG, "sky_sample_session_hop: no such hop");
   SKY_TRY(s->build(weights));
-  return s->draw(hop);
+  return s->draw(hop, hop + 1);
 }
 int sample_session_end(SampleSession* s, uint64_t* sampled, double* seconds) {
   const int rc = s->end(sampled, seconds);
