@@ -24,248 +24,28 @@
 // 64 to 512 threads per vertex with the row's prefix arrays in LDS (rows up to 4093 entries),
 // and the tile-parallel path of sky_build_tiled.hip for longer rows.
 #include <algorithm>
-#include <functional>
-#include <utility>
 #include <vector>
 
-#include "sky_build_common.h"
+#include "sky_build_fused.h"
+#include "sky_build_rows.h"
 #include "sky_graph.h"
 
 namespace sky {
 
-__host__ __device__ __forceinline__ int degree_class(uint32_t d) {
-  if (d == 0) return CLS_EMPTY;
-  if (d <= 2) return CLS_TINY;
-  // rows of the group kernels start at any slot (their vector loads and stores only need 4-byte alignment)
-  if (d <= 8) return CLS_G2;
-  if (d <= 16) return CLS_G4;
-  if (d <= 32) return CLS_G8;
-  if (d <= 64) return CLS_G16;
-  if (d <= 128) return CLS_G32;
-  if (d <= 160) return CLS_G32S;
-  if (d <= 192) return CLS_G32X;
-  if (d <= 253) return CLS_LDS_W1;
-  // These kernels are bound by instruction issue: a row pays for the slots of its class, not for its entries.  The
-  // two classes whose rows differ most in length (by a factor of two) are halved: 6 instead of 8 slots per thread
-  // for their shorter rows.
-  if (d <= 381) return CLS_LDS_W6;
-  if (d <= 509) return CLS_LDS_W2;
-  if (d <= 765) return CLS_MW2_6;
-  const uint32_t nw = (d + 3 + 511) / 512;  // wavefronts of 512 slots that hold the row from any 16-byte phase
-  // The arrays of a longer row (14 bytes of LDS per slot) would leave room for one workgroup per CU only: such a row
-  // keeps its heavies alone in LDS, and its entries in registers as long as 512 threads can hold them (1024 threads
-  // for rows of up to 16381 entries, one workgroup per CU, ran at 1.7 TB/s where the streaming kernel reaches 1.95).
-  if (nw <= MERGE_MAX_NW) return CLS_MW2 + (int)nw - 2;
-  if (d <= HOLD_MAX_DEG) return CLS_HOLD;
-  if (d > STREAM_MAX_DEG) return CLS_HUGE;
-  if (d > 65533u) return CLS_STREAM_WIDE;
-  return d > 24576u ? CLS_STREAM : CLS_STREAM_LAST;
-}
-
-// Vectors that are only 4-byte aligned: global loads and stores of 8 and 16 bytes need no more on gfx950.
-typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef float float2u __attribute__((ext_vector_type(2), aligned(4)));
-typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(4)));
-
-// ---------------------------------------------------------------- 2..32 lanes per row
-// G lanes share one row of at most PER * G slots; every lane holds PER consecutive weights, so a
-// wavefront carries 64 / G rows and the per-row steps that do not depend on the row length (exact
-// sum, ledger, scans) are paid once per 64 / G rows.  Prefix sums run over the group by DPP; SL and
-// SH of every slot go to a per-group LDS strip padded to PER * G slots (slots outside the row add
-// nothing), which each entry then searches once with a fixed number of probes; the heavies' slots,
-// compacted by rank, give "next heavy" and "last heavy".  The rank rides in bits 52..63 of the SH scan.
-// Every lane of the wavefront must call this together (DPP); a group without a row passes d = 0.
-// s_pre: [2 * BLOCK * PER] u64 ([0, BLK): SL of every slot of the block; [BLK, 2 * BLK): SH), s_hs: [BLOCK * PER]
-// (per group: row-local slot of its h-th heavy).  Returns false for a row whose weights sum to zero.
-constexpr uint64_t GROUP_CNT = 1ull << 52;
-
-template <int G, int PER, int BLOCK = 256>
-__device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const float* __restrict__ wgt,
-                                                AliasEntry* __restrict__ table, uint64_t* __restrict__ s_pre,
-                                                uint8_t* __restrict__ s_hs, uint32_t tid = threadIdx.x) {
-  static_assert(PER >= 4 && PER <= 6, "a lane loads one float4 (and one float), or three float2");
-  constexpr uint32_t SLOTS = PER * G;
-  constexpr uint32_t HB = PER == 4 ? SLOTS : PER == 5 ? SLOTS / 5 * 4 : SLOTS / 3 * 2;  // largest power of two <= SLOTS
-  static_assert((HB & (HB - 1)) == 0 && HB <= SLOTS && 2 * HB > SLOTS && SLOTS <= 256, "G is a power of two");
-  constexpr uint32_t BLK = BLOCK * PER;                      // slots of one block's strips (BLOCK threads)
-  const int gl = tid & (G - 1);
-  const int lane = tid & 63;
-  const uint32_t gbase = (uint32_t)PER * (tid - gl);  // first LDS slot of the group
-  const uint32_t pos = (uint32_t)PER * gl;
-
-  float xs[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) xs[k] = 0.0f;
-  if (PER == 4 || PER == 5) {
-    if (pos < d) {
-      const float4u x = *reinterpret_cast<const float4u*>(wgt + off + pos);
-      xs[0] = x.x; xs[1] = x.y; xs[2] = x.z; xs[3] = x.w;
-    }
-  } else {
-#pragma unroll
-    for (int h = 0; h < PER / 2; ++h)
-      if (pos + 2 * h < d) {
-        const float2u x = *reinterpret_cast<const float2u*>(wgt + off + pos + 2 * h);
-        xs[2 * h] = x.x;
-        xs[2 * h + 1] = x.y;
-      }
-  }
-  if (PER % 2 == 1 && pos + PER - 1 < d) xs[PER - 1] = wgt[off + pos + PER - 1];
-  double wd[PER];
-  uint32_t live = 0;
-  // the sum of the row as a plain fp64 sum where that is exact (plain_sum_is_exact); a wavefront in which some
-  // group's is not falls back to the three-limb sum for all of its groups
-  double Sd = 0.0;
-  uint32_t mn = 0xFFFFFFFFu;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const bool in = pos + k < d;
-    if (in) live |= 1u << k;
-    const float cw = masked_weight(xs[k], in);
-    wd[k] = (double)cw;
-    Sd += wd[k];
-    mn = min(mn, __float_as_uint(cw) - 1u);
-  }
-  Sd = group_sum_f64<G>(Sd);
-  mn = group_min_u32<G>(mn);
-  const bool plain = plain_sum_is_exact(Sd, mn);
-  if (__any(!plain)) {
-    WSum3 S{0.0, 0.0, 0.0};
-#pragma unroll
-    for (int k = 0; k < PER; ++k) wsum3_add(S, wd[k]);
-    S = group_sum_wsum3<G>(S);
-    if (!plain) Sd = S.top + S.mid + S.low != 0.0 ? wsum3_to_double(S) : 0.0;
-  }
-  const bool row_ok = Sd != 0.0;
-  Ledger L = make_ledger_small(d, Sd);
-  if (!row_ok) L.scale = 0.0;
-  const double neg_fs = -L.fs;
-
-  uint64_t dl[PER], sl[PER], sh[PER];
-  float op[PER];
-  uint32_t heavy = 0;
-  uint64_t ra = 0, rb = 0;
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const Entry e = classify_small_fma(wd[k], L, neg_fs);
-    dl[k] = (e.heavy || !((live >> k) & 1)) ? 0 : e.amount;
-    ra += dl[k];
-    rb += e.heavy ? (e.amount | GROUP_CNT) : 0;
-    sl[k] = ra;
-    sh[k] = rb;
-    op[k] = (float)e.p;
-    if (e.heavy) heavy |= 1u << k;
-  }
-  const uint64_t ia = group_scan_u64<G>(ra), ib = group_scan_u64<G>(rb);
-  const uint32_t nh = (uint32_t)(shfl_u64(ib, (lane - gl) + G - 1) >> 52);
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    sl[k] += ia - ra;
-    sh[k] += ib - rb;
-    s_pre[gbase + pos + k] = sl[k];
-    s_pre[BLK + gbase + pos + k] = sh[k] & (GROUP_CNT - 1);
-    if ((heavy >> k) & 1) s_hs[gbase + (uint32_t)(sh[k] >> 52) - 1] = (uint8_t)(pos + k);
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-  // light: first slot with SH > SL - D.  heavy: first slot with SL >= SH, i.e. SL > SH - 1.
-  // The first probe narrows the answer to a window of HB slots that ends inside the strip.
-  uint32_t arr[PER], at[PER];
-  uint64_t key[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const bool hv = (heavy >> k) & 1;
-    arr[k] = gbase + (hv ? 0u : BLK);
-    key[k] = hv ? (sh[k] & (GROUP_CNT - 1)) - 1 : sl[k] - dl[k];
-    at[k] = HB == SLOTS ? 0u : (s_pre[arr[k] + HB - 1] <= key[k] ? SLOTS - HB : 0u);
-  }
-#pragma unroll
-  for (uint32_t step = HB / 2; step >= 1; step >>= 1) {
-    uint64_t v[PER];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) v[k] = s_pre[arr[k] + at[k] + step - 1];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) at[k] += v[k] <= key[k] ? step : 0u;
-  }
-  uint32_t oa[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const uint64_t v = s_pre[arr[k] + at[k]];
-    const bool found = v > key[k];
-    const uint32_t self = pos + k;
-    if (!((heavy >> k) & 1)) {
-      oa[k] = found ? at[k] : (nh ? (uint32_t)s_hs[gbase + nh - 1] : self);
-    } else {
-      const uint32_t hc = (uint32_t)(sh[k] >> 52);
-      if (hc < nh && found) {
-        op[k] = residual_prob(L.one + key[k] + 1 - v, L);
-        oa[k] = s_hs[gbase + hc];
-      } else {
-        op[k] = 1.0f;
-        oa[k] = self;
-      }
-    }
-    if (!row_ok) {
-      op[k] = 0.0f;
-      oa[k] = SKY_INVALID;
-    }
-  }
-  // the next row of this group reuses the strips: its writes must stay behind these reads
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-#pragma unroll
-  for (int h = 0; h < PER / 2; ++h) {
-    const uint32_t m = (live >> (2 * h)) & 3u;
-    AliasEntry* t = table + off + pos + 2 * h;
-    if (m == 3u) {
-      uint4u o;
-      o.x = __float_as_uint(op[2 * h]); o.y = oa[2 * h]; o.z = __float_as_uint(op[2 * h + 1]); o.w = oa[2 * h + 1];
-      *reinterpret_cast<uint4u*>(t) = o;
-    } else if (m == 1u) {
-      t[0] = AliasEntry{op[2 * h], oa[2 * h]};
-    }
-  }
-  if (PER % 2 == 1 && ((live >> (PER - 1)) & 1)) table[off + pos + PER - 1] = AliasEntry{op[PER - 1], oa[PER - 1]};
-  return row_ok || d == 0;
-}
-
-// Where a class kernel finds its rows.  A build whose class sizes the host knows passes the class's segment of the
-// row list and its length, and launches exactly the workgroups the rows need (dev null).  A build whose sizes only
-// the device knows (the rows of a frontier that the host never waits for) passes the whole list and the counter
-// block of the binning pass: the class's rows start after those of the classes before it, and a grid of fixed
-// size strides over them.
-__device__ __forceinline__ void class_segment(const uint32_t* __restrict__ dev, int cls, int ncls, uint32_t& start,
-                                              uint32_t& count) {
-  if (!dev) return;
-  uint32_t st = 0;
-  for (int c = 0; c < cls; ++c) st += dev[c];
-  uint32_t n = 0;
-  for (int c = cls; c < cls + ncls; ++c) n += dev[c];
-  start = st;
-  count = n;
-}
-
-template <int G, int PER, bool DEV = false>
+// Class kernels: `vlist` is the class's segment of the row list, `count` its length.  Every row's builder writes its flag
+// (1, or 0 for a row without weight): a build may follow one that found other weights.
+template <int G, int PER>
 __global__ __launch_bounds__(256) void build_group_kernel(const RowRef* __restrict__ vlist, uint32_t count,
-                                                          const uint32_t* __restrict__ dev, int cls,
                                                           const float* __restrict__ wgt,
                                                           AliasEntry* __restrict__ table,
                                                           int8_t* __restrict__ valid) {
   __shared__ uint64_t s_pre[2 * 256 * PER];
   __shared__ uint8_t s_hs[256 * PER];
-  uint32_t start = 0;
-  if (DEV) class_segment(dev, cls, 1, start, count);
-  constexpr uint32_t ROWS = 256 / G;  // rows per workgroup and round
-  // DEV false: one round per workgroup, and the loop is none
-  for (uint32_t b = blockIdx.x; DEV ? b * ROWS < count : b == blockIdx.x; b += DEV ? gridDim.x : 1u) {
-    const uint32_t grp = b * ROWS + threadIdx.x / G;
-    RowRef rr{0, 0, 0, 0};
-    if (grp < count) rr = vlist[start + grp];
-    const bool ok = group_build_row<G, PER>(rr.off, rr.d, wgt, table, s_pre, s_hs);
-    if ((threadIdx.x & (G - 1)) == 0 && !ok) valid[rr.v] = 0;  // the binning pass has set it
-  }
+  const uint32_t grp = blockIdx.x * (256 / G) + threadIdx.x / G;
+  RowRef rr{0, 0, 0, 0};
+  if (grp < count) rr = vlist[grp];
+  const bool ok = group_build_row<G, PER>(rr.off, rr.d, wgt, table, s_pre, s_hs);
+  if ((threadIdx.x & (G - 1)) == 0 && grp < count) valid[rr.v] = ok ? 1 : 0;
 }
 
 __global__ __launch_bounds__(128) void build_begin_kernel(uint32_t* __restrict__ counters, uint32_t words,
@@ -282,11 +62,15 @@ __global__ __launch_bounds__(128) void build_begin_kernel(uint32_t* __restrict__
 // cursors it keeps in LDS, so no global atomic is involved and the lists come out grouped by block.
 constexpr int BIN_BLOCKS = 4096;  // most blocks a binning pass uses
 constexpr int BIN_ITEMS = 4;      // vertices per thread and step
+// at most BIN_BLOCKS blocks, each a multiple of one scatter step
+static uint32_t bin_per_block(uint32_t n) {
+  const uint32_t step = 256u * BIN_ITEMS;
+  return ((n + BIN_BLOCKS - 1) / BIN_BLOCKS + step - 1) / step * step;
+}
 
 __global__ __launch_bounds__(256) void bin_count_kernel(const uint32_t* __restrict__ xadj,
                                                         const uint32_t* __restrict__ src, uint32_t n,
-                                                        const uint32_t* __restrict__ n_dev,
-                                                        uint32_t per_block, int listed_from,
+                                                        uint32_t per_block,
                                                         uint32_t* __restrict__ blk_cnt,
                                                         unsigned long long* __restrict__ class_edges) {
   __shared__ uint32_t s_cnt[CLS_COUNT];
@@ -296,7 +80,6 @@ __global__ __launch_bounds__(256) void bin_count_kernel(const uint32_t* __restri
     s_edges[threadIdx.x] = 0;
   }
   __syncthreads();
-  if (n_dev) n = min(n, *n_dev);  // the host passed an upper bound
   const uint32_t lo = blockIdx.x * per_block, hi = min(n, lo + per_block);
   uint32_t tiny_edges = 0;  // rows of 1..2 entries, the commonest kind of a power-law graph, stay out of the LDS atomics
   // four vertices per thread and step: their loads are in flight together (one at a time, the loop waits a
@@ -316,7 +99,7 @@ __global__ __launch_bounds__(256) void bin_count_kernel(const uint32_t* __restri
     for (int k = 0; k < BIN_ITEMS; ++k) {
       const int c = degree_class(d[k]);
       if (c >= CLS_G2) {
-        if (c >= listed_from) atomicAdd(&s_cnt[c], 1u);  // classes below get no list: small_rows_kernel builds them
+        atomicAdd(&s_cnt[c], 1u);
         atomicAdd(&s_edges[c], (unsigned long long)d[k]);
       } else {
         tiny_edges += d[k];  // 0 for an empty row
@@ -360,36 +143,6 @@ __global__ __launch_bounds__(256) void bin_offsets_kernel(uint32_t* __restrict__
   if (tid == 0) counts[c] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
 }
 
-// A row of one or two entries in closed form.
-__device__ __forceinline__ bool tiny_row(uint32_t off, uint32_t d, const float* __restrict__ wgt,
-                                         AliasEntry* __restrict__ table) {
-  // a weight adds to the exact sum iff it is at least 2^-64
-  constexpr float UNIT = 5.421010862427522170037e-20f;  // 2^-64
-  const float w0 = clamp_weight(wgt[off]);
-  if (d == 1) {
-    const bool ok = w0 >= UNIT;
-    table[off] = AliasEntry{ok ? 1.0f : 0.0f, ok ? 0u : SKY_INVALID};
-    return ok;
-  }
-  const float w1 = clamp_weight(wgt[off + 1]);
-  const bool ok = w0 >= UNIT || w1 >= UNIT;
-  AliasEntry a{0.0f, SKY_INVALID}, b{0.0f, SKY_INVALID};
-  if (ok) {
-    WSum3 S{0.0, 0.0, 0.0};
-    wsum3_add(S, (double)w0);
-    wsum3_add(S, (double)w1);
-    const Ledger L = make_ledger_small(2, wsum3_to_double(S));
-    const Entry e0 = classify_small((double)w0, true, L), e1 = classify_small((double)w1, true, L);
-    // a lone heavy is the last heavy: it keeps its bucket and tops up the light
-    a = AliasEntry{e0.heavy ? 1.0f : (float)e0.p, (!e0.heavy && e1.heavy) ? 1u : 0u};
-    b = AliasEntry{e1.heavy ? 1.0f : (float)e1.p, (!e1.heavy && e0.heavy) ? 0u : 1u};
-  }
-  uint4u o;
-  o.x = __float_as_uint(a.prob); o.y = a.alias; o.z = __float_as_uint(b.prob); o.w = b.alias;
-  *reinterpret_cast<uint4u*>(table + off) = o;
-  return ok;
-}
-
 // Writes each row of class >= CLS_G2 into its class segment of vlist, and finishes
 // the classes that need no cooperation: deg 0 (valid = 0) and deg 1..2 (closed form).  The rows of one
 // or two entries that a wavefront meets in a step go to a list of its own in LDS first and are then
@@ -398,7 +151,6 @@ __device__ __forceinline__ bool tiny_row(uint32_t off, uint32_t d, const float* 
 __global__ __launch_bounds__(256) void bin_scatter_kernel(const uint32_t* __restrict__ xadj,
                                                           const float* __restrict__ wgt,
                                                           const uint32_t* __restrict__ src, uint32_t n,
-                                                          const uint32_t* __restrict__ n_dev,
                                                           uint32_t per_block, int listed_from,
                                                           const uint32_t* __restrict__ counts,
                                                           const uint32_t* __restrict__ blk_off,
@@ -410,12 +162,11 @@ __global__ __launch_bounds__(256) void bin_scatter_kernel(const uint32_t* __rest
   __shared__ uint8_t s_tiny_d[4][64 * BIN_ITEMS];
   if (threadIdx.x < CLS_COUNT) {  // the class lists lie back to back in class order
     uint32_t start = 0;
-    for (uint32_t c = 0; c < threadIdx.x; ++c) start += counts[c];
+    for (uint32_t c = (uint32_t)listed_from; c < threadIdx.x; ++c) start += counts[c];  // classes below have no list
     s_cur[threadIdx.x] = start + blk_off[blockIdx.x * CLS_COUNT + threadIdx.x];
   }
   __syncthreads();
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (n_dev) n = min(n, *n_dev);
   const uint32_t lo = blockIdx.x * per_block, hi = min(n, lo + per_block);
   for (uint32_t chunk = lo; chunk < hi; chunk += 256u * BIN_ITEMS) {
     uint32_t nt = 0;  // wave-uniform: rows in this wavefront's list
@@ -457,127 +208,13 @@ __global__ __launch_bounds__(256) void bin_scatter_kernel(const uint32_t* __rest
 }
 
 // ---------------------------------------------------------------- rows of at most 32 entries, where they lie
-// One wavefront walks a contiguous range of vertices, 64 at a time, and builds every row of 1..32 entries it
-// meets: the rows of a class queue up in LDS until they fill the wavefront (64 rows of 1..2 entries, 32 of 3..8 with
-// 2 lanes each, 16 of 9..16 with 4, 8 of 17..32 with 8) and are then built by the same code as in the class kernels.
-// Neighbouring rows of different classes share their cache lines, and here the same wavefront touches them within a
-// few steps; no row list is written or read for these classes.  Also sets valid[] of the vertices it owns (rows of
-// 0..32 entries).  Workgroups are single wavefronts: nothing in here waits for another wavefront.
-// Queue capacities (128, 96, 80, 72): less than one batch left over plus the 64 vertices of a step
-// (64 + 63, 64 + 31, 64 + 15, 64 + 7), rounded up.  A queue entry is the row's offset and, in 16 bits, its degree (6 bits) above the vertex's position in
-// the wavefront's range (10 bits): the vertex id itself is only needed for a row without weight, whose flag is
-// cleared.  6.5 KB of LDS per wavefront, so that six of them fit every SIMD (the kernel's registers allow six).
-constexpr uint32_t SMALL_RANGE = 1024;  // most vertices per wavefront
-constexpr uint32_t SMALL_QBASE[4] = {0, 128, 224, 304};
-constexpr uint32_t SMALL_QTOTAL = 376;
 __global__ __launch_bounds__(64) void small_rows_kernel(const uint32_t* __restrict__ xadj,
                                                         const float* __restrict__ wgt,
                                                         const uint32_t* __restrict__ src, uint32_t n,
                                                         uint32_t per_wave, AliasEntry* __restrict__ table,
                                                         int8_t* __restrict__ valid) {
-  __shared__ uint64_t s_pre[2 * 64 * 4];
-  __shared__ uint8_t s_hs[64 * 4];
-  __shared__ uint32_t q_off[SMALL_QTOTAL];
-  __shared__ uint16_t q_it[SMALL_QTOTAL];
-  const uint32_t lane = threadIdx.x;
-  const uint32_t lo = blockIdx.x * per_wave, hi = min(n, lo + per_wave);
-  uint32_t cnt[4] = {0, 0, 0, 0};  // wave-uniform queue lengths: rows of 1..2, 3..8, 9..16, 17..32 entries
-
-  // the last `rows` entries of queue q, one per group of G lanes; d = 0 for a group without a row.  `t` is the lane
-  // number behind an empty asm statement: it keeps what depends on the lane number inside one batch (hoisted
-  // out of the loop for all four row sizes at once, those values double the registers of the kernel).
-  auto take = [&](int q, uint32_t rows, uint32_t G, uint32_t& t, uint32_t& off, uint32_t& it, uint32_t& d) {
-    t = lane;
-    asm volatile("" : "+v"(t));
-    const uint32_t r = t / G;
-    off = it = d = 0;
-    if (r < rows) {
-      const uint32_t k = SMALL_QBASE[q] + cnt[q] - rows + r;
-      off = q_off[k];
-      const uint32_t x = q_it[k];
-      it = x & (SMALL_RANGE - 1);
-      d = x >> 10;
-    }
-  };
-  auto clear_valid = [&](uint32_t it) {  // a row whose weights sum to zero (rare)
-    const uint32_t item = lo + it;
-    valid[src ? src[item] : item] = 0;
-  };
-  auto build_tiny = [&](uint32_t rows) {
-    uint32_t t, off, it, d;
-    take(0, rows, 1, t, off, it, d);
-    if (d && !tiny_row(off, d, wgt, table)) clear_valid(it);
-    cnt[0] -= rows;
-  };
-  auto build_g2 = [&](uint32_t rows) {
-    uint32_t t, off, it, d;
-    take(1, rows, 2, t, off, it, d);
-    const bool ok = group_build_row<2, 4, 64>(off, d, wgt, table, s_pre, s_hs, t);
-    if ((t & 1) == 0 && !ok) clear_valid(it);
-    cnt[1] -= rows;
-  };
-  auto build_g4 = [&](uint32_t rows) {
-    uint32_t t, off, it, d;
-    take(2, rows, 4, t, off, it, d);
-    const bool ok = group_build_row<4, 4, 64>(off, d, wgt, table, s_pre, s_hs, t);
-    if ((t & 3) == 0 && !ok) clear_valid(it);
-    cnt[2] -= rows;
-  };
-  auto build_g8 = [&](uint32_t rows) {
-    uint32_t t, off, it, d;
-    take(3, rows, 8, t, off, it, d);
-    const bool ok = group_build_row<8, 4, 64>(off, d, wgt, table, s_pre, s_hs, t);
-    if ((t & 7) == 0 && !ok) clear_valid(it);
-    cnt[3] -= rows;
-  };
-
-  // the row offsets of step i + 1 are requested before the batches of step i are built
-  auto fetch = [&](uint32_t base, uint32_t& v, uint32_t& off, uint32_t& end) {
-    const uint32_t item = base + lane;
-    v = 0xFFFFFFFFu;
-    off = end = 0;
-    if (item < hi) {
-      v = src ? src[item] : item;
-      off = xadj[v];
-      end = xadj[v + 1];
-    }
-  };
-  uint32_t nv, noff, nend;
-  fetch(lo, nv, noff, nend);
-  for (uint32_t base = lo; base < hi; base += 64u) {
-    const uint32_t v = nv, off = noff, d = nend - noff;
-    if (base + 64u < hi) fetch(base + 64u, nv, noff, nend);
-    int q = -1;
-    if (v != 0xFFFFFFFFu && d <= 32u) {
-      valid[v] = d != 0;  // a row without weight clears it when it is built
-      q = d == 0 ? -1 : d <= 2 ? 0 : d <= 8 ? 1 : d <= 16 ? 2 : 3;
-    }
-    const uint32_t packed = (d << 10) | (base - lo + lane);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const unsigned long long m = __ballot(q == c);
-      if (q == c) {
-        const uint32_t p = SMALL_QBASE[c] + cnt[c] + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-        q_off[p] = off;
-        q_it[p] = (uint16_t)packed;
-      }
-      cnt[c] += (uint32_t)__popcll(m);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    while (cnt[0] >= 64u) build_tiny(64);
-    while (cnt[1] >= 32u) build_g2(32);
-    while (cnt[2] >= 16u) build_g4(16);
-    while (cnt[3] >= 8u) build_g8(8);
-    // the next step's queue entries stay behind this step's reads of the queues
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  }
-  if (cnt[0]) build_tiny(cnt[0]);
-  if (cnt[1]) build_g2(cnt[1]);
-  if (cnt[2]) build_g4(cnt[2]);
-  if (cnt[3]) build_g8(cnt[3]);
+  __shared__ uint64_t smem[(SMALL_LDS_BYTES + 7) / 8];
+  small_rows_range(blockIdx.x * per_wave, xadj, wgt, src, n, per_wave, table, valid, smem);
 }
 
 // ---------------------------------------------------------------- one row per workgroup, prefix arrays in LDS
@@ -781,252 +418,17 @@ __global__ __launch_bounds__(ROWT) void build_lds_kernel(const RowRef* __restric
   }
 }
 
-// ---------------------------------------------------------------- one row per workgroup, pairing by merge
-// Same table as build_lds_kernel, reached without a binary search per entry.  Lights and heavies
-// are compacted by rank into one LDS array (inclusive SL of the lights from the front, inclusive
-// SH of the heavies from the back, a sentinel after each).  In the order of the merged sequence,
-// ties heavy first,
-//   the alias of light r is the heavy rank reached when light r - 1 is taken (rank 0 for r = 0),
-//   the light that finishes heavy h is the light rank reached when heavy h is taken,
-// so each thread finds where its share of PER merged elements starts (one diagonal search) and
-// walks it.  The heavy count rides in bits 52..63 of the SH scan: a row of at most 4093 entries
-// keeps its sums below 2^52.
-constexpr uint64_t MERGE_CNT = 1ull << 52;
-constexpr uint32_t MERGE_SELF = 0x80000000u;  // "prob 1, alias self" in the per-heavy result word
-
-template <int ROWT, int PER, int MINW = 4, int DEV = 0>  // DEV 1: segment from the device, one row per workgroup; 2: striding grid
-__global__ __launch_bounds__(ROWT, MINW) void build_merge_kernel(const RowRef* __restrict__ vlist, uint32_t count,
-                                                           const uint32_t* __restrict__ dev, int cls,
-                                                           const float* __restrict__ wgt,
+// ---------------------------------------------------------------- one row per workgroup, pairing by merge (merge_row)
+// MINW: wavefronts per SIMD the registers must leave room for; 3 where LDS (50 KB for 256 threads of 14 slots) allows no
+// more anyway.
+template <int ROWT, int PER, int MINW = 4>
+__global__ __launch_bounds__(ROWT, MINW) void build_merge_kernel(const RowRef* __restrict__ vlist, const float* __restrict__ wgt,
                                                            AliasEntry* __restrict__ table, int8_t* __restrict__ valid) {
-  // PER consecutive slots per thread, counted from the row's 16-byte aligned start; a thread moves them as
-  // quads when PER is a multiple of 4, as pairs otherwise (its first slot is then only 8-byte aligned)
-  constexpr int VEC = PER % 4 == 0 ? 4 : 2;
-  static_assert(PER % VEC == 0 && PER <= 16, "whole vectors, and `live` has one bit per slot");
-  constexpr int CAP = ROWT * PER;
-  constexpr int NW = ROWT / 64;
-  constexpr uint32_t TOP = CAP + 1;  // heavy h lives at index TOP - h of the value array and of the result array
-  constexpr bool PACKED = CAP <= 4096;  // the heavy count rides in the SH scan; larger rows scan it separately
-  static_assert(CAP <= 8192, "sums and shifts below assume rows of fewer than 2^13 entries");
   extern __shared__ uint64_t smem[];
-  uint64_t* s_v = smem;                                             // [CAP + 2]
-  uint32_t* s_res = reinterpret_cast<uint32_t*>(smem + CAP + 2);  // [CAP + 2]
-  uint16_t* s_hs = reinterpret_cast<uint16_t*>(s_res + CAP + 2);   // [CAP + 2] row-local slot of heavy h
-  __shared__ WSum3 s_wsum[NW];
-  __shared__ double s_fsum[NW];
-  __shared__ uint32_t s_mn[NW];
-  __shared__ uint64_t s_ex[3 * NW];
-
-  uint32_t start = 0;
-  if (DEV) class_segment(dev, cls, 1, start, count);
-  if (DEV == 1 && blockIdx.x >= count) return;
-  // DEV 0 and 1: one row per workgroup, and the loop is none
-  for (uint32_t row = blockIdx.x; DEV == 2 ? row < count : row == blockIdx.x; row += DEV == 2 ? gridDim.x : 1u) {
-  if (DEV == 2 && row != blockIdx.x) __syncthreads();  // the arrays in LDS are about to be rewritten
-  const RowRef rr = vlist[start + row];
-  const uint32_t v = rr.v, off = rr.off, d = rr.d;
-  const uint32_t base = off & ~3u, lead = off - base, span = lead + d;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const uint32_t pos0 = (uint32_t)PER * (uint32_t)tid;
-  const bool wave_on = (uint32_t)(PER * 64 * wave) < span;
-
-  double wd[PER];
-  uint32_t live = 0;  // bit j: slot pos0 + j belongs to the row
-  // the sum of the row as a plain fp64 sum where that is exact (plain_sum_is_exact), else as three limbs
-  double rsum = 0.0;
-  uint32_t mn = 0xFFFFFFFFu;
-  if (wave_on) {
-#pragma unroll
-    for (int t = 0; t < PER / VEC; ++t) {
-      const uint32_t pos = pos0 + (uint32_t)(VEC * t);
-      float xs[4] = {0.f, 0.f, 0.f, 0.f};
-      if (pos < span) {
-        if constexpr (VEC == 4) {
-          const float4 x = *reinterpret_cast<const float4*>(wgt + base + pos);
-          xs[0] = x.x; xs[1] = x.y; xs[2] = x.z; xs[3] = x.w;
-        } else {
-          const float2 x = *reinterpret_cast<const float2*>(wgt + base + pos);
-          xs[0] = x.x; xs[1] = x.y;
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) {
-        const uint32_t idx = pos + k;
-        const bool in = idx - lead < d;  // one unsigned compare: slots before the row wrap around
-        if (in) live |= 1u << (t * VEC + k);
-        const float cw = masked_weight(xs[k], in);
-        wd[t * VEC + k] = (double)cw;
-        rsum += wd[t * VEC + k];
-        mn = min(mn, __float_as_uint(cw) - 1u);
-      }
-    }
-    rsum = group_sum_f64<64>(rsum);
-    mn = wave_min_u32(mn);
-  } else {
-#pragma unroll
-    for (int j = 0; j < PER; ++j) wd[j] = 0.0;
-  }
-  if (NW > 1) {
-    if (lane == 0) {
-      s_fsum[wave] = rsum;
-      s_mn[wave] = mn;
-    }
-    __syncthreads();
-    rsum = s_fsum[0];
-    mn = s_mn[0];
-#pragma unroll
-    for (int i = 1; i < NW; ++i) {
-      rsum += s_fsum[i];
-      mn = min(mn, s_mn[i]);
-    }
-  }
-  if (!plain_sum_is_exact(rsum, (uint32_t)__builtin_amdgcn_readfirstlane((int)mn))) {  // uniform over the workgroup
-    WSum3 sum{0.0, 0.0, 0.0};
-    if (wave_on) {
-#pragma unroll
-      for (int j = 0; j < PER; ++j) wsum3_add(sum, wd[j]);
-      sum = group_sum_wsum3<64>(sum);
-    }
-    if (NW > 1) {
-      if (lane == 0) s_wsum[wave] = sum;
-      __syncthreads();
-      sum = s_wsum[0];
-#pragma unroll
-      for (int i = 1; i < NW; ++i) {
-        sum.top += s_wsum[i].top;
-        sum.mid += s_wsum[i].mid;
-        sum.low += s_wsum[i].low;
-      }
-    }
-    rsum = sum.top + sum.mid + sum.low != 0.0 ? wsum3_to_double(sum) : 0.0;
-  }
-  if (rsum == 0.0) {
-#pragma unroll
-    for (int j = 0; j < PER; ++j)
-      if ((live >> j) & 1) table[base + pos0 + j] = AliasEntry{0.0f, SKY_INVALID};
-    if (tid == 0) valid[v] = 0;
-    continue;
-  }
-  const Ledger L = make_ledger_small(d, rsum);
-  const double neg_fs = -L.fs;
-
-  float op[PER];
-  uint32_t hcnt[PER];  // heavies up to and including this slot
-  uint32_t heavy = 0;
-  uint32_t nh, nl;
-  {
-    uint64_t dl[PER], dh[PER], sl[PER], sh[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const bool in = (live >> j) & 1;
-      const Entry e = PACKED ? classify_small_fma(wd[j], L, neg_fs) : classify_fast(wd[j], in, L);
-      dl[j] = (e.heavy || !in) ? 0 : e.amount;
-      dh[j] = e.heavy ? (PACKED ? (e.amount | MERGE_CNT) : e.amount) : 0;
-      op[j] = (float)e.p;
-      if (e.heavy) heavy |= 1u << j;
-    }
-    uint64_t total_l, total_h;
-    uint32_t ex_c = 0;
-    if constexpr (PACKED) {
-      block_scan2_flat<ROWT, PER>(dl, dh, s_ex, sl, sh, total_l, total_h, wave_on);
-      nh = (uint32_t)(total_h >> 52);
-    } else {
-      block_scan2c_flat<ROWT, PER>(dl, dh, (uint32_t)__popc(heavy), s_ex, sl, sh, ex_c, total_l, total_h, nh, wave_on);
-    }
-    nl = d - nh;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const uint32_t hc = PACKED ? (uint32_t)(sh[j] >> 52) : ex_c + (uint32_t)__popc(heavy & ((2u << j) - 1));
-      hcnt[j] = hc;
-      if (!((live >> j) & 1)) continue;
-      const uint32_t li = pos0 + j - lead;
-      const bool hv = (heavy >> j) & 1;
-      s_v[hv ? TOP + 1 - hc : li - hc] = hv ? (PACKED ? (sh[j] & (MERGE_CNT - 1)) : sh[j]) : sl[j];
-      if (hv) s_hs[hc - 1] = (uint16_t)li;
-    }
-  }
-  if (tid == 0) {
-    s_v[nl] = ~0ull;
-    s_v[TOP - nh] = ~0ull;
-  }
-  __syncthreads();
-
-  if (nh) {
-    if (tid == 0) s_res[0] = s_hs[0];  // the first light starts in the first heavy
-    // merged positions [k0, k0 + PER) belong to this thread; a lights and k0 - a heavies come before them
-    const uint32_t k0 = pos0;
-    if (k0 < d) {
-      uint32_t lo = k0 > nh ? k0 - nh : 0u, hi = min(k0, nl);
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        if (s_v[mid - 1] < s_v[TOP - (k0 - mid)]) lo = mid; else hi = mid - 1;
-      }
-      uint32_t a = lo, b = k0 - lo;
-      const uint32_t steps = min((uint32_t)PER, d - k0);
-      uint64_t va = s_v[a], vb = s_v[TOP - b];  // heads of the two sequences: only the one taken is read again
-#pragma unroll
-      for (int s = 0; s < PER; ++s) {
-        if ((uint32_t)s < steps) {
-          if (vb <= va) {
-            s_res[TOP - b] = a;
-            ++b;
-            vb = s_v[TOP - b];
-          } else {
-            ++a;
-            if (a < nl) s_res[a] = s_hs[min(b, nh - 1)];
-            va = s_v[a];
-          }
-        }
-      }
-    }
-    __syncthreads();
-    // heavies, densely by rank: residual probability from the light that finishes them
-    for (uint32_t h = tid; h < nh; h += ROWT) {
-      const uint32_t r = s_res[TOP - h];
-      uint32_t out = MERGE_SELF;
-      if (h + 1 < nh && r < nl) out = __float_as_uint(residual_prob(L.one + s_v[TOP - h] - s_v[r], L));
-      s_res[TOP - h] = out;
-    }
-    __syncthreads();
-  }
-
-  if (pos0 < span) {
-    uint32_t oa[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const uint32_t li = pos0 + j - lead;
-      const uint32_t hc = hcnt[j];
-      oa[j] = li;
-      if (nh && ((live >> j) & 1)) {
-        if ((heavy >> j) & 1) {
-          const uint32_t x = s_res[TOP - (hc - 1)];
-          op[j] = x == MERGE_SELF ? 1.0f : __uint_as_float(x);
-          if (x != MERGE_SELF) oa[j] = s_hs[hc];
-        } else {
-          oa[j] = s_res[li - hc];
-        }
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < PER / VEC; ++t) {
-      const uint32_t pos = pos0 + (uint32_t)(VEC * t);
-      if (pos >= lead && pos + VEC <= span) {
-        if constexpr (VEC == 4) {
-          const float p4[4] = {op[4 * t], op[4 * t + 1], op[4 * t + 2], op[4 * t + 3]};
-          const uint32_t a4[4] = {oa[4 * t], oa[4 * t + 1], oa[4 * t + 2], oa[4 * t + 3]};
-          store_entries4(table + base + pos, p4, a4);
-        } else {
-          *reinterpret_cast<uint4*>(table + base + pos) =
-              make_uint4(__float_as_uint(op[2 * t]), oa[2 * t], __float_as_uint(op[2 * t + 1]), oa[2 * t + 1]);
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k)
-          if ((live >> (t * VEC + k)) & 1) table[base + pos + k] = AliasEntry{op[VEC * t + k], oa[VEC * t + k]};
-      }
-    }
-  }
-  }  // rows of this workgroup
+  __shared__ uint64_t s_aux[8 * (ROWT / 64)];
+  const RowRef rr = vlist[blockIdx.x];
+  const bool ok = merge_row<ROWT, PER>(rr, smem, s_aux, wgt, table);
+  if (threadIdx.x == 0) valid[rr.v] = ok ? 1 : 0;
 }
 
 // ---------------------------------------------------------------- rows beyond LDS: global scratch
@@ -1367,10 +769,8 @@ int prepare_build_scratch(sky_graph* g, uint32_t max_rows) {
   if (!sc.blk_cnt) SKY_HIP(hipMalloc((void**)&sc.blk_cnt, (size_t)BIN_BLOCKS * CLS_COUNT * 4));
   if (!g_lds_enabled) {
     SKY_TRY(enable_big_lds(build_lds_kernel<512, 2>, 512 * 4 * 2 * 16));
-    SKY_TRY(enable_big_lds(build_merge_kernel<512, 10>, (512 * 10 + 2) * 14));
-    SKY_TRY(enable_big_lds(build_merge_kernel<768, 6>, (768 * 6 + 2) * 14));
-    SKY_TRY(enable_big_lds((build_merge_kernel<512, 10, 4, 1>), (512 * 10 + 2) * 14));
-    SKY_TRY(enable_big_lds((build_merge_kernel<768, 6, 4, 1>), (768 * 6 + 2) * 14));
+    SKY_TRY(enable_big_lds(build_merge_kernel<512, 10>, (int)merge_lds_bytes(512, 10)));
+    SKY_TRY(enable_big_lds(build_merge_kernel<768, 6>, (int)merge_lds_bytes(768, 6)));
     g_lds_enabled = true;
   }
   return SKY_OK;
@@ -1402,6 +802,12 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     hipLaunchKernelGGL(small_rows_kernel, dim3((n + per_wave - 1) / per_wave), dim3(64), 0, s, g->xadj, g->adjwgt, src, n,
                        per_wave, g->table, g->valid);
   };
+  // A build of all vertices that leaves the short rows where they lie takes the lists of the others from the graph's
+  // plan: they depend on the row offsets alone, and binning 67 M vertices again took 0.35 ms.
+  const bool all_rows = src == nullptr && n == g->V;
+  const bool planned = all_rows && small_in_place && n > 0;
+  if (planned) SKY_TRY(ensure_plan(g));
+  RowRef* vlist = planned ? g->plan->rows : sc.vlist;
   // clears the counters of the binning pass and notes when the call began
   hipLaunchKernelGGL(build_begin_kernel, dim3(1), dim3(128), 0, st, sc.counters, (uint32_t)(COUNTER_BYTES / 4), call);
   if (n > 0) {
@@ -1410,38 +816,23 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
       SKY_TRY(fan.branch(sky_graph::SIDE_STREAMS - 1, &side));
       launch_small(side);
     }
-    // at most BIN_BLOCKS blocks, each a multiple of one scatter step
-    const uint32_t step = 256u * BIN_ITEMS;
-    const uint32_t per_block = ((n + BIN_BLOCKS - 1) / BIN_BLOCKS + step - 1) / step * step;
-    const uint32_t blocks = (n + per_block - 1) / per_block;
-    hipLaunchKernelGGL(bin_count_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, src, n, (const uint32_t*)nullptr,
-                       per_block, listed_from, sc.blk_cnt,
-                       reinterpret_cast<unsigned long long*>(sc.counters + 2 * CLS_COUNT));
-    hipLaunchKernelGGL(bin_offsets_kernel, dim3(CLS_COUNT), dim3(256), 0, st, sc.blk_cnt, blocks, sc.counters);
-    hipLaunchKernelGGL(bin_scatter_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, g->adjwgt, src, n,
-                       (const uint32_t*)nullptr, per_block, listed_from, sc.counters, sc.blk_cnt, sc.vlist, g->table,
-                       g->valid);
-    // The class sizes decide the launches that follow.  Those of all vertices depend on xadj alone and are kept
-    // with the graph after the first time; any other list of rows is waited for.
-    const bool all_rows = src == nullptr && n == g->V;
-    if (all_rows && g->bin_known && g->bin_listed_from == listed_from) {
+    if (planned) {
       for (int c = 0; c < CLS_COUNT; ++c) {
         host.counts[c] = g->bin_counts[c];
         host.edges[c] = g->bin_edges[c];
       }
     } else {
+      // The class sizes decide the launches that follow.
+      const uint32_t per_block = bin_per_block(n), blocks = (n + per_block - 1) / per_block;
+      hipLaunchKernelGGL(bin_count_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, src, n, per_block, sc.blk_cnt,
+                         reinterpret_cast<unsigned long long*>(sc.counters + 2 * CLS_COUNT));
+      hipLaunchKernelGGL(bin_offsets_kernel, dim3(CLS_COUNT), dim3(256), 0, st, sc.blk_cnt, blocks, sc.counters);
+      hipLaunchKernelGGL(bin_scatter_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, g->adjwgt, src, n, per_block, listed_from,
+                         sc.counters, sc.blk_cnt, sc.vlist, g->table, g->valid);
       SKY_HIP(hipMemcpyAsync(&host, sc.counters, COUNTER_BYTES, hipMemcpyDeviceToHost, st));
       SKY_HIP(hipStreamSynchronize(st));
-      if (all_rows) {
-        for (int c = 0; c < CLS_COUNT; ++c) {
-          g->bin_counts[c] = host.counts[c];
-          g->bin_edges[c] = host.edges[c];
-        }
-        g->bin_known = true;
-        g->bin_listed_from = listed_from;
-      }
     }
-    for (int c = 0; c < CLS_COUNT; ++c) counts[c] = host.counts[c];
+    for (int c = listed_from; c < CLS_COUNT; ++c) counts[c] = host.counts[c];
     uint32_t acc = 0;
     for (int c = 0; c < CLS_COUNT; ++c) {
       starts[c] = acc;
@@ -1454,7 +845,6 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     launch_small(st);
     SKY_TRY(tm->mark("small", small_edges));
   }
-  RowRef* const vlist = sc.vlist;
   uint64_t call_edges = 0;
   for (int c = 0; c < CLS_COUNT; ++c) call_edges += host.edges[c];
   if (!tm && option(g, OPT_BUILD_STREAMS) && call_edges >= FAN_MIN_EDGES && call_edges < FAN_MAX_EDGES) SKY_TRY(fan.start());
@@ -1464,7 +854,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     if (cnt) {
       const uint32_t per_block = 256 / G;
       hipLaunchKernelGGL(kernel, dim3((cnt + per_block - 1) / per_block), dim3(256), 0, fan.next(host.edges[cls]), vlist + starts[cls],
-                         cnt, (const uint32_t*)nullptr, 0, g->adjwgt, g->table, g->valid);
+                         cnt, g->adjwgt, g->table, g->valid);
     }
     return (tm && cnt) ? tm->mark(name, host.edges[cls]) : SKY_OK;  // no bracket for an empty class
   };
@@ -1490,7 +880,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   if (row_merge && counts[CLS_HOLD]) {
     {
       StreamSwap sw(g, fan.next(2 * host.edges[CLS_HOLD]));
-      SKY_TRY(build_rows_hold(g, vlist + starts[CLS_HOLD], counts[CLS_HOLD], nullptr, 0));
+      SKY_TRY(build_rows_hold(g, vlist + starts[CLS_HOLD], counts[CLS_HOLD]));
     }
     if (tm) SKY_TRY(tm->mark("hold", host.edges[CLS_HOLD]));
   }
@@ -1506,9 +896,9 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   auto mrg = [&](int cls, auto kernel, int rowt, int per, const char* name) -> int {
     const uint32_t cnt = counts[cls];
     if (cnt) {
-      const size_t bytes = ((size_t)rowt * per + 2) * 14;
-      hipLaunchKernelGGL(kernel, dim3(cnt), dim3(rowt), bytes, fan.next(host.edges[cls]), vlist + starts[cls], cnt,
-                         (const uint32_t*)nullptr, 0, g->adjwgt, g->table, g->valid);
+      const size_t bytes = merge_lds_bytes(rowt, per);
+      hipLaunchKernelGGL(kernel, dim3(cnt), dim3(rowt), bytes, fan.next(host.edges[cls]), vlist + starts[cls],
+                         g->adjwgt, g->table, g->valid);
     }
     return (tm && cnt) ? tm->mark(name, host.edges[cls]) : SKY_OK;  // no bracket for an empty class
   };
@@ -1529,7 +919,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     SKY_MW(4);
     SKY_TRY(mrg(CLS_MW2 + 3, build_merge_kernel<256, 10>, 256, 10, mw_name[3]));
     SKY_TRY(mrg(CLS_MW2 + 4, build_merge_kernel<512, 6>, 512, 6, mw_name[4]));
-    SKY_TRY(mrg(CLS_MW2 + 5, build_merge_kernel<256, 14>, 256, 14, mw_name[5]));
+    SKY_TRY(mrg(CLS_MW2 + 5, (build_merge_kernel<256, 14, 3>), 256, 14, mw_name[5]));
     SKY_MW(8);
     SKY_TRY(mrg(CLS_MW2 + 7, build_merge_kernel<768, 6>, 768, 6, mw_name[7]));
     SKY_TRY(mrg(CLS_MW2 + 8, build_merge_kernel<512, 10>, 512, 10, mw_name[8]));
@@ -1612,165 +1002,60 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   return fan.join();
 }
 
-// ---------------------------------------------------------------- builds that never wait for the device
-// The rows of a frontier: how many there are, and how many fall into each degree class, is known on the device
-// only.  The binning kernels take the length of the list from a device word, every class kernel finds its segment
-// of the row list through the counter block (class_segment) and strides over it with a grid of fixed size.  Which
-// classes can hold a row at all depends on the graph alone: a census of all vertices, taken once per graph, lets
-// the host skip the launches of the classes the graph does not populate.
-// Most workgroups of a launch, by workgroup size: enough to fill every CU several times over (a class that
-// turns out small leaves most of them with nothing to do, which costs microseconds).
-constexpr uint32_t DEV_GRID_STREAM = 512;
-constexpr uint32_t dev_grid_cap(int threads) { return threads <= 64 ? 16384u : threads <= 256 ? 8192u : 2048u; }
-
-bool build_rows_dev_possible(const sky_graph* g) { return option(g, OPT_ROW_MERGE) != 0 && tiled_max_tiles(g) == (1u << 22); }
-
-int ensure_class_census(sky_graph* g) {
-  if (g->bin_known || g->V == 0) return SKY_OK;
+int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start) {
   hipStream_t st = g->stream;
-  SKY_TRY(prepare_build_scratch(g, 1));
+  SKY_TRY(ensure_table_storage(g));
+  SKY_TRY(prepare_build_scratch(g, 0));
   BuildScratch& sc = scratch_of(g);
   struct {
     uint32_t counts[2 * CLS_COUNT];
     unsigned long long edges[CLS_COUNT];
   } host = {};
-  const uint32_t n = g->V, step = 256u * BIN_ITEMS;
-  const uint32_t per_block = ((n + BIN_BLOCKS - 1) / BIN_BLOCKS + step - 1) / step * step;
-  const uint32_t blocks = (n + per_block - 1) / per_block;
-  SKY_HIP(hipMemsetAsync(sc.counters, 0, COUNTER_BYTES, st));
-  hipLaunchKernelGGL(bin_count_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, (const uint32_t*)nullptr, n,
-                     (const uint32_t*)nullptr, per_block, (int)CLS_G2, sc.blk_cnt,
-                     reinterpret_cast<unsigned long long*>(sc.counters + 2 * CLS_COUNT));
-  hipLaunchKernelGGL(bin_offsets_kernel, dim3(CLS_COUNT), dim3(256), 0, st, sc.blk_cnt, blocks, sc.counters);
-  SKY_HIP(hipMemcpyAsync(&host, sc.counters, COUNTER_BYTES, hipMemcpyDeviceToHost, st));
-  SKY_HIP(hipStreamSynchronize(st));
+  const uint32_t n = g->V, per_block = bin_per_block(n), blocks = n ? (n + per_block - 1) / per_block : 0;
+  if (n) {
+    hipLaunchKernelGGL(build_begin_kernel, dim3(1), dim3(128), 0, st, sc.counters, (uint32_t)(COUNTER_BYTES / 4),
+                       (CallDevice*)nullptr);
+    hipLaunchKernelGGL(bin_count_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, (const uint32_t*)nullptr, n, per_block,
+                       sc.blk_cnt, reinterpret_cast<unsigned long long*>(sc.counters + 2 * CLS_COUNT));
+    hipLaunchKernelGGL(bin_offsets_kernel, dim3(CLS_COUNT), dim3(256), 0, st, sc.blk_cnt, blocks, sc.counters);
+    SKY_HIP(hipMemcpyAsync(&host, sc.counters, COUNTER_BYTES, hipMemcpyDeviceToHost, st));
+    SKY_HIP(hipStreamSynchronize(st));
+  }
+  size_t listed = 0;
   for (int c = 0; c < CLS_COUNT; ++c) {
     g->bin_counts[c] = host.counts[c];
     g->bin_edges[c] = host.edges[c];
+    start[c] = (uint32_t)listed;
+    if (c >= listed_from) listed += host.counts[c];
   }
-  g->bin_known = true;
-  g->bin_listed_from = CLS_G2;
-  return SKY_OK;
-}
-
-int build_rows_dev(sky_graph* g, const uint32_t* src, const uint32_t* n_dev, uint32_t n_upper) {
-  if (n_upper == 0) return SKY_OK;
-  if (!build_rows_dev_possible(g) || !g->bin_known)
-    return fail(SKY_ERR_STATE, "build_rows_dev: needs the class census and rows the streaming kernel takes");
-  hipStream_t st = g->stream;
-  g->has_walk_index = false;
-  BuildScratch& sc = scratch_of(g);
-  const uint32_t step = 256u * BIN_ITEMS;
-  const uint32_t per_block = ((n_upper + BIN_BLOCKS - 1) / BIN_BLOCKS + step - 1) / step * step;
-  const uint32_t blocks = (n_upper + per_block - 1) / per_block;
-  SKY_HIP(hipMemsetAsync(sc.counters, 0, COUNTER_BYTES, st));
-  hipLaunchKernelGGL(bin_count_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, src, n_upper, n_dev, per_block,
-                     (int)CLS_G2, sc.blk_cnt, reinterpret_cast<unsigned long long*>(sc.counters + 2 * CLS_COUNT));
-  hipLaunchKernelGGL(bin_offsets_kernel, dim3(CLS_COUNT), dim3(256), 0, st, sc.blk_cnt, blocks, sc.counters);
-  hipLaunchKernelGGL(bin_scatter_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, g->adjwgt, src, n_upper, n_dev,
-                     per_block, (int)CLS_G2, sc.counters, sc.blk_cnt, sc.vlist, g->table, g->valid);
-  // a class of the graph holds bin_counts[c] rows at most (bin_edges tells whether it holds any: the counts of the
-  // census leave out the classes that a large full build does not list)
-  auto rows_of = [&](int cls) -> uint32_t {
-    if (g->bin_edges[cls] == 0) return 0;
-    const uint32_t in_graph = g->bin_listed_from <= cls ? g->bin_counts[cls] : n_upper;
-    return std::min(n_upper, std::max(1u, in_graph));
-  };
-  const uint32_t* const dev = sc.counters;
-  const RowRef* const vlist = sc.vlist;
-  // the class kernels are independent of one another: they go out in turn over the graph's stream and its side streams
-  StreamFan fan(g, st);
-  if (option(g, OPT_BUILD_STREAMS) && n_upper >= 4096) SKY_TRY(fan.start());
-  // Rows of 8190 entries and more first, because theirs is the longest chain of launches.  The classes STREAM,
-  // STREAM_LAST, STREAM_WIDE, HUGE lie back to back.  What the graph holds of them decides, as in a build of all
-  // rows, which go to the streaming kernel (one workgroup per row) and which are built tile by tile by the whole
-  // GPU: the two longest classes always are (a frontier holds a few such rows at most, and one workgroup would need
-  // a millisecond for one), the other two when the graph has too few of their rows to fill the GPU with one
-  // workgroup each.
-  static_assert(CLS_STREAM_LAST == CLS_STREAM + 1 && CLS_STREAM_WIDE == CLS_STREAM + 2 && CLS_HUGE == CLS_STREAM + 3,
-                "the lists of the long rows lie back to back");
-  const bool narrow_tiled = g->bin_edges[CLS_STREAM] + g->bin_edges[CLS_STREAM_LAST] <= (uint64_t)option(g, OPT_STREAM_MIN_EDGES);
-  const uint32_t stream_rows = narrow_tiled ? 0 : rows_of(CLS_STREAM) + rows_of(CLS_STREAM_LAST);
-  const int t_first = narrow_tiled ? CLS_STREAM : CLS_STREAM_WIDE;
-  uint32_t tiled_rows = 0;
-  uint64_t tiled_edges = 0;
-  for (int c = t_first; c <= CLS_HUGE; ++c) {
-    tiled_rows += rows_of(c);
-    tiled_edges += g->bin_edges[c];
-  }
-  // A stream is chosen by the work it already carries; the work of a class is what the graph holds of it (a
-  // frontier mirrors the graph), weighted for the kernels of the long rows, which are slow beside the others.
-  if (tiled_rows) {
-    StreamSwap sw(g, fan.next(2 * tiled_edges));
-    SKY_TRY(build_rows_tiled_dev(g, vlist, dev, t_first, CLS_HUGE - t_first + 1, tiled_rows, tiled_edges));
-  }
-  // the streaming kernel fills the LDS of every CU it reaches: the tile-parallel path, whose first kernels are small,
-  // is enqueued before it
-  if (stream_rows) {
-    StreamSwap sw(g, fan.next(3 * (g->bin_edges[CLS_STREAM] + g->bin_edges[CLS_STREAM_LAST])));
-    SKY_TRY(build_rows_stream_dev(g, vlist, dev, 2, std::min(DEV_GRID_STREAM, stream_rows)));
-  }
-  auto grp = [&](int cls, auto kernel, int G) {
-    const uint32_t rows = rows_of(cls);
-    if (!rows) return;
-    const uint32_t per = 256 / G;
-    hipLaunchKernelGGL(kernel, dim3(std::min(dev_grid_cap(256), (rows + per - 1) / per)), dim3(256), 0,
-                       fan.next(g->bin_edges[cls]), vlist, 0u, dev, cls, g->adjwgt, g->table, g->valid);
-  };
-  auto mrg = [&](int cls, auto kernel, int rowt, int per) {
-    const uint32_t rows = rows_of(cls);
-    if (!rows) return;
-    const size_t bytes = ((size_t)rowt * per + 2) * 14;
-    // one wavefront per row: a striding grid; larger workgroups: one per row the class can hold (the code of a
-    // loop over rows costs these kernels registers they do not have)
-    hipLaunchKernelGGL(kernel, dim3(rowt <= 64 ? std::min(dev_grid_cap(rowt), rows) : rows), dim3(rowt), bytes,
-                       fan.next(g->bin_edges[cls]), vlist, 0u, dev, cls, g->adjwgt, g->table, g->valid);
-  };
-  // The class kernels go out in the order of the classes' sizes in the graph, the largest first: a frontier mirrors
-  // the graph, and the streams should not end on a long kernel that started last.
-  std::vector<std::pair<unsigned long long, std::function<void()>>> queue;
-#define SKY_Q(CLS, CALL) queue.emplace_back(g->bin_edges[CLS], [&] { CALL; })
-  SKY_Q(CLS_G2, grp(CLS_G2, (build_group_kernel<2, 4, true>), 2));
-  SKY_Q(CLS_G4, grp(CLS_G4, (build_group_kernel<4, 4, true>), 4));
-  SKY_Q(CLS_G8, grp(CLS_G8, (build_group_kernel<8, 4, true>), 8));
-  SKY_Q(CLS_G16, grp(CLS_G16, (build_group_kernel<16, 4, true>), 16));
-  SKY_Q(CLS_G32, grp(CLS_G32, (build_group_kernel<32, 4, true>), 32));
-  SKY_Q(CLS_G32S, grp(CLS_G32S, (build_group_kernel<32, 5, true>), 32));
-  SKY_Q(CLS_G32X, grp(CLS_G32X, (build_group_kernel<32, 6, true>), 32));
-  SKY_Q(CLS_LDS_W1, mrg(CLS_LDS_W1, (build_merge_kernel<64, 4, 4, 2>), 64, 4));
-  SKY_Q(CLS_LDS_W6, mrg(CLS_LDS_W6, (build_merge_kernel<64, 6, 4, 2>), 64, 6));
-  SKY_Q(CLS_LDS_W2, mrg(CLS_LDS_W2, (build_merge_kernel<64, 8, 4, 2>), 64, 8));
-  SKY_Q(CLS_MW2_6, mrg(CLS_MW2_6, (build_merge_kernel<128, 6, 4, 1>), 128, 6));
-#define SKY_MW(NW) SKY_Q(CLS_MW2 + NW - 2, mrg(CLS_MW2 + NW - 2, (build_merge_kernel<64 * NW, 8, 4, 1>), 64 * NW, 8))
-  SKY_MW(2);
-  SKY_Q(CLS_MW2 + 1, mrg(CLS_MW2 + 1, (build_merge_kernel<256, 6, 4, 1>), 256, 6));
-  SKY_MW(4);
-  SKY_Q(CLS_MW2 + 3, mrg(CLS_MW2 + 3, (build_merge_kernel<256, 10, 4, 1>), 256, 10));
-  SKY_Q(CLS_MW2 + 4, mrg(CLS_MW2 + 4, (build_merge_kernel<512, 6, 4, 1>), 512, 6));
-  SKY_Q(CLS_MW2 + 5, mrg(CLS_MW2 + 5, (build_merge_kernel<256, 14, 4, 1>), 256, 14));
-  SKY_MW(8);
-  SKY_Q(CLS_MW2 + 7, mrg(CLS_MW2 + 7, (build_merge_kernel<768, 6, 4, 1>), 768, 6));
-  SKY_Q(CLS_MW2 + 8, mrg(CLS_MW2 + 8, (build_merge_kernel<512, 10, 4, 1>), 512, 10));
-#undef SKY_MW
-  auto hold = [&](int cls) -> int {
-    const uint32_t rows = rows_of(cls);
-    if (!rows) return SKY_OK;
-    StreamSwap sw(g, fan.next(2 * g->bin_edges[cls]));
-    return build_rows_hold(g, vlist, rows, dev, cls);
-  };
-  int hold_rc = SKY_OK;
-  SKY_Q(CLS_HOLD, { const int rc = hold(CLS_HOLD); if (rc != SKY_OK) hold_rc = rc; });
-#undef SKY_Q
-  std::stable_sort(queue.begin(), queue.end(), [](const auto& a, const auto& b) { return a.first > b.first; });
-  for (auto& q : queue) q.second();
-  SKY_TRY(fan.join());
-  if (hold_rc != SKY_OK) return hold_rc;
+  SKY_HIP(hipMalloc((void**)rows, listed * sizeof(RowRef) + 16));
+  if (listed)
+    hipLaunchKernelGGL(bin_scatter_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, g->adjwgt, (const uint32_t*)nullptr, n, per_block,
+                       listed_from, sc.counters, sc.blk_cnt, *rows, g->table, g->valid);
   SKY_HIP(hipGetLastError());
   return SKY_OK;
 }
 
+// Largest build that goes out in the four launches of sky_build_fused.hip.
+constexpr uint64_t FUSED_MAX_ENTRIES = 1ull << 27;
+
 int build_all_tables(sky_graph* g, double* seconds) {
   SKY_TRY(ensure_table_storage(g));
+  // Knobs that name kernels of their own, and per-kernel timing, want the class kernels.
+  const bool fused = fused_possible(g) && !option(g, OPT_BUILD_PROFILE) && option(g, OPT_SMALL_IN_PLACE) < 0 &&
+                     option(g, OPT_BUILD_STREAMS) != 0 && g->E <= (getenv("FUSED_MAX") ? atoll(getenv("FUSED_MAX")) : FUSED_MAX_ENTRIES) && g->V;
+  if (fused) {
+    SKY_TRY(ensure_plan(g));
+    CallDevice* call = nullptr;
+    double sec = 0;
+    SKY_TRY(call_begin(g, &call));
+    SKY_TRY(build_all_fused(g, call));
+    SKY_TRY(call_end(g, nullptr, &sec));
+    g->build_profile.assign(1, {"build", (float)(sec * 1e3), g->E});
+    if (seconds) *seconds = sec;
+    g->has_tables = true;
+    return SKY_OK;
+  }
   SKY_TRY(prepare_build_scratch(g, g->V));
   if (option(g, OPT_BUILD_PROFILE)) {
     EventTimer tm(g->stream);

@@ -1,0 +1,726 @@
+// Builds whose launches, not their entries, would bound them: everything from a graph of a thousand edges up to FUSED_MAX_ENTRIES, and
+// the rows of a frontier.
+//
+// The class kernels of sky_build.hip give every degree class a launch of its own.  That is right where a class fills
+// the GPU for a millisecond; a build of 17 M entries spent 220 us on 27 launches of 5 to 25 us each, 2.4 us apart on
+// the host and each with a tail of its own, and spreading them over four streams costs 30 us for the fork and the
+// join alone.  Here one launch takes all classes whose rows need the same number of threads, and the passes of the
+// rows that are built tile by tile, which depend on one another, ride along in the same four launches:
+//
+//   fused_wave_kernel    64 threads    rows of up to 509 entries         tile sums
+//   fused_pair_kernel    128 threads   rows of 510..1021                 row sums -> ledger, tile totals
+//   fused_wide_kernel    512 threads   rows of 2558 and more             scan over a row's tiles
+//   fused_block_kernel   256 threads   rows of 1022..2557                entries of the tiles
+//
+// A launch whose classes are empty is left out.  Every row builder is the one the class kernels call, so the
+// tables are the same bits.  The lists of rows by class and the geometry of the tiles depend on the row offsets alone:
+// they are made by the first build of a graph and kept with it.
+#include <algorithm>
+#include <cstddef>
+#include <type_traits>
+
+#include "sky_build_fused.h"
+#include "sky_build_long.h"
+#include "sky_build_rows.h"
+#include "sky_build_tile.h"
+
+namespace sky {
+
+// What a unit of a launch's work is.
+enum Section : uint32_t {
+  SEC_SWEEP,  // 64 threads: a range of vertices, all their rows of at most 32 entries
+  SEC_TINY,   //             64 listed rows of 1..2 entries
+  SEC_G2, SEC_G4, SEC_G8, SEC_G16, SEC_G32, SEC_G32S, SEC_G32X, SEC_W1, SEC_W6, SEC_W2,
+  SEC_SUM,    //             the sum of a tile
+  SEC_P6, SEC_P8,                              // 128 threads
+  SEC_TOTALS,                                  //             two tiles
+  SEC_STREAM, SEC_B6, SEC_B8, SEC_B10,  // 512 threads
+  SEC_SCAN,                                    //             a row's tiles
+  SEC_M6, SEC_M8, SEC_M10,                     // 256 threads
+  SEC_EMIT                                     //             a tile
+};
+struct SectionRef {
+  uint32_t kind;
+  uint32_t units;    // host-sized: units of this section; device-sized: not used
+  uint32_t per;      // rows per unit
+  uint32_t start;    // first row in the list
+  int cls0, ncls;    // device-sized: classes whose rows lie back to back from `start` on
+  uint32_t stride;   // device-sized: distance between the segments of consecutive classes
+};
+constexpr int MAX_SECTIONS = 14;
+struct FusedArgs {
+  const RowRef* list;
+  const uint32_t* counts;  // device-sized: rows of every class (null: host-sized)
+  const uint32_t* xadj;
+  const float* wgt;
+  AliasEntry* table;
+  int8_t* valid;
+  uint32_t V, per_wave;  // SEC_SWEEP
+  // rows built tile by tile
+  TiledRow* trows;
+  const TileGeom* geom;
+  u128* tsum;
+  TileTotals* ttot;
+  uint64_t *BL, *BH;
+  uint32_t* nfh;
+  uint4* ranges;
+  const uint32_t* bitmap;  // frontier: bit set for every vertex whose row has been asked for (null: every row is built)
+  uint32_t epoch;          // frontier: number of the call, to tell rows built earlier in it
+  uint32_t tile0, trow0;  // first tile and row of those this build makes tile by tile
+  bool ledgers_done;
+  CallDevice* call;  // the call's first launch notes when it began
+  uint32_t nsec;
+  uint32_t first[MAX_SECTIONS];  // host-sized: first unit of every section, 2^32 - 1 past the last
+  SectionRef sec[MAX_SECTIONS];
+};
+
+// The section and the unit inside it that unit u of the launch is; false past the end.  Host-sized launches have
+// one workgroup per unit and the sections' first units in their arguments; device-sized ones find out how many units
+// each section has, section i in lane i of every wavefront, once per workgroup.
+template <bool DEV>
+struct UnitFinder;
+template <>
+struct UnitFinder<false> {
+  __device__ __forceinline__ explicit UnitFinder(const FusedArgs&) {}
+  __device__ __forceinline__ bool find(const FusedArgs& a, uint32_t u, SectionRef& s, uint32_t& unit, uint32_t& rows) const {
+    uint32_t k = 0, first = 0;
+#pragma unroll
+    for (int i = 1; i < MAX_SECTIONS; ++i)
+      if (u >= a.first[i]) {
+        k = i;
+        first = a.first[i];
+      }
+    s = a.sec[k];
+    unit = u - first;
+    rows = 0;
+    return true;
+  }
+};
+template <>
+struct UnitFinder<true> {
+  uint32_t incl, rows_of;
+  __device__ __forceinline__ explicit UnitFinder(const FusedArgs& a) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t n = 0;
+    rows_of = 0;
+    if (lane < a.nsec) {
+      const SectionRef s = a.sec[lane];
+      n = s.units;
+      if (s.cls0 >= 0) {
+        for (int c = 0; c < s.ncls; ++c) rows_of += a.counts[s.cls0 + c];
+        n = (rows_of + s.per - 1) / s.per;
+      }
+    }
+    incl = group_scan_u32<16>(n);
+  }
+  __device__ __forceinline__ bool find(const FusedArgs& a, uint32_t u, SectionRef& s, uint32_t& unit, uint32_t& rows) const {
+    const unsigned long long m = __ballot(u < incl) & ((1ull << MAX_SECTIONS) - 1ull);
+    if (!m) return false;
+    const int k = __ffsll((long long)m) - 1;
+    s = a.sec[k];
+    unit = u - (k ? (uint32_t)__builtin_amdgcn_readlane((int)incl, k - 1) : 0u);
+    rows = (uint32_t)__builtin_amdgcn_readlane((int)rows_of, k);
+    return true;
+  }
+};
+// Row `i` of a section (host-sized: `rows` holds none, the section's last unit may be partly empty).
+template <bool DEV>
+__device__ __forceinline__ bool row_at(const FusedArgs& a, const SectionRef& s, uint32_t i, uint32_t rows, RowRef& rr) {
+  rr = RowRef{0, 0, 0, 0};
+  if (!DEV) {
+    if (i >= s.stride) return false;  // host-sized: stride holds the number of rows
+    rr = a.list[s.start + i];
+    return true;
+  }
+  if (i >= rows) return false;
+  uint32_t at = s.start;
+  for (int c = 0; c + 1 < s.ncls; ++c) {
+    const uint32_t n = a.counts[s.cls0 + c];
+    if (i < n) break;
+    i -= n;
+    at += s.stride;
+  }
+  rr = a.list[at + i];
+  return true;
+}
+
+__device__ __forceinline__ bool tile_active(const FusedArgs& a, const TiledRow& r) {
+  return !a.bitmap || (((a.bitmap[r.v >> 5] >> (r.v & 31)) & 1u) && r.done != a.epoch);
+}
+
+// The exact sum of tile `tile` by a wavefront: 16 slots per lane.
+__device__ __forceinline__ void tile_sum_wave(const FusedArgs& a, uint32_t tile) {
+  const uint32_t lane = threadIdx.x & 63;
+  const TileGeom tg = a.geom[tile];
+  if (tg.span == 0) return;  // there are fewer tiles than their bound
+  const TiledRow* row = a.trows + tg.row;
+  if (a.bitmap) {
+    const bool active = tile_active(a, *row);
+    if (tg.T == 0 && lane == 0) a.trows[tg.row].active = active ? 1u : 0u;
+    if (!active) return;
+  }
+  float4 x[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t pos = tg.T * TILE + 256u * k + 4u * lane;
+    x[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (pos < tg.span) x[k] = *reinterpret_cast<const float4*>(a.wgt + tg.base + pos);
+  }
+  WSum3 sum{0.0, 0.0, 0.0};  // exact: a tile adds at most 1024 limbs below 2^32 + 1
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float xs[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t idx = tg.T * TILE + 256u * k + 4u * lane + j;
+      wsum3_add(sum, (double)masked_weight(xs[j], idx - tg.lead < tg.span - tg.lead));
+    }
+  }
+  sum = group_sum_wsum3<64>(sum);
+  if (lane == 0) a.tsum[tile] = wsum3_to_u128(sum);
+}
+
+// Row sum -> ledger, and the totals of one tile, by a wavefront.  Every tile of a row adds up its row's tile sums, which
+// spares a launch in between; where a row has so many that this would take long (LEDGER_TILES) there is that launch.
+__device__ __forceinline__ void tile_totals_wave(const FusedArgs& a, uint32_t tile) {
+  const uint32_t lane = threadIdx.x & 63;
+  const TileGeom tg = a.geom[tile];
+  if (tg.span == 0) return;
+  TiledRow* row = a.trows + tg.row;
+  if (a.bitmap && !row->active) return;
+  float4 x[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t pos = tg.T * TILE + 256u * k + 4u * lane;
+    x[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (pos < tg.span) x[k] = *reinterpret_cast<const float4*>(a.wgt + tg.base + pos);
+  }
+  bool ok;
+  Ledger L = {0.0, 0.0, 0.0, 0};
+  if (a.ledgers_done) {
+    ok = row->ok;
+    L = row_ledger(*row);
+  } else {
+    u128 sum{0, 0};
+    const uint32_t t0 = row->tile0, nt = row->ntiles;
+    for (uint32_t t = lane; t < nt; t += 64) sum = add128(sum, a.tsum[t0 + t]);
+    sum = group_sum_u128<64>(sum);
+    ok = (sum.lo | sum.hi) != 0;
+    if (ok) L = make_ledger(row->d, sum);
+    if (tg.T == 0 && lane == 0) {
+      row->ok = ok;
+      row->scale = L.scale;
+      row->fs = L.fs;
+      row->inv_fs = L.inv_fs;
+      row->one = L.one;
+    }
+  }
+  if (!ok) return;
+  uint64_t sd = 0, su = 0;
+  uint32_t fh = NONE32, lh = 0;  // lh holds idx + 1 so that 0 means none
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float xs[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t idx = tg.T * TILE + 256u * k + 4u * lane + j;
+      const bool in = idx - tg.lead < tg.span - tg.lead;
+      const Entry e = classify_fast((double)masked_weight(xs[j], in), in, L);
+      if (!in) continue;
+      if (e.heavy) {
+        su += e.amount;
+        fh = min(fh, idx);
+        lh = max(lh, idx + 1);
+      } else {
+        sd += e.amount;
+      }
+    }
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    sd += shfl_xor_u64(sd, m);
+    su += shfl_xor_u64(su, m);
+    fh = min(fh, (uint32_t)__shfl_xor((int)fh, m, 64));
+    lh = max(lh, (uint32_t)__shfl_xor((int)lh, m, 64));
+  }
+  if (lane == 0) a.ttot[tile] = TileTotals{sd, su, fh, lh ? lh - 1 : NONE32};
+}
+
+template <bool DEV, int G, int PER>
+__device__ __forceinline__ void group_unit(const FusedArgs& a, const SectionRef& s, uint32_t unit, uint32_t rows,
+                                           uint64_t* smem) {
+  uint32_t t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // what depends on the lane number stays inside this unit's code
+  RowRef rr;
+  const bool have = row_at<DEV>(a, s, unit * (64 / G) + t / G, rows, rr);
+  const bool ok = group_build_row<G, PER, 64>(rr.off, rr.d, a.wgt, a.table, smem,
+                                              reinterpret_cast<uint8_t*>(smem + 2 * 64 * PER), t);
+  if (have && (t & (G - 1)) == 0) a.valid[rr.v] = ok ? 1 : 0;
+}
+template <bool DEV, int ROWT, int PER>
+__device__ __forceinline__ void merge_unit(const FusedArgs& a, const SectionRef& s, uint32_t unit, uint32_t rows,
+                                           uint64_t* smem, uint64_t* s_aux) {
+  RowRef rr;
+  if (!row_at<DEV>(a, s, unit, rows, rr)) return;
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));  // see group_unit
+  const bool ok = merge_row<ROWT, PER>(rr, smem, s_aux, a.wgt, a.table, t);
+  if (threadIdx.x == 0) a.valid[rr.v] = ok ? 1 : 0;
+}
+
+constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
+constexpr size_t WAVE_LDS = cmax(cmax(SMALL_LDS_BYTES, 2 * 64 * 6 * 8 + 64 * 6), merge_lds_bytes(64, 8));
+
+template <bool DEV>
+__global__ __launch_bounds__(64) void fused_wave_kernel(FusedArgs a) {
+  __shared__ uint64_t smem[(WAVE_LDS + 7) / 8];
+  __shared__ uint64_t s_aux[8];
+  call_stamp(a.call);
+  const UnitFinder<DEV> units(a);
+  for (uint32_t u = blockIdx.x;; u += gridDim.x) {
+    SectionRef s;
+    uint32_t unit = 0, rows = 0;
+    if (!units.find(a, u, s, unit, rows)) return;
+    switch (s.kind) {
+      case SEC_SWEEP:
+        if constexpr (!DEV)
+          small_rows_range(unit * a.per_wave, a.xadj, a.wgt, nullptr, a.V, a.per_wave, a.table, a.valid, smem);
+        break;
+      case SEC_TINY:
+        if constexpr (DEV) {
+          RowRef rr;
+          if (row_at<DEV>(a, s, unit * 64 + threadIdx.x, rows, rr)) a.valid[rr.v] = tiny_row(rr.off, rr.d, a.wgt, a.table) ? 1 : 0;
+        }
+        break;
+      case SEC_G2: if constexpr (DEV) group_unit<DEV, 2, 4>(a, s, unit, rows, smem); break;
+      case SEC_G4: if constexpr (DEV) group_unit<DEV, 4, 4>(a, s, unit, rows, smem); break;
+      case SEC_G8: if constexpr (DEV) group_unit<DEV, 8, 4>(a, s, unit, rows, smem); break;
+      case SEC_G16: group_unit<DEV, 16, 4>(a, s, unit, rows, smem); break;
+      case SEC_G32: group_unit<DEV, 32, 4>(a, s, unit, rows, smem); break;
+      case SEC_G32S: group_unit<DEV, 32, 5>(a, s, unit, rows, smem); break;
+      case SEC_G32X: group_unit<DEV, 32, 6>(a, s, unit, rows, smem); break;
+      case SEC_W1: merge_unit<DEV, 64, 4>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_W6: merge_unit<DEV, 64, 6>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_W2: merge_unit<DEV, 64, 8>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_SUM: tile_sum_wave(a, a.tile0 + unit); break;
+      default: break;
+    }
+    if (!DEV) return;
+    __syncthreads();  // the next unit rewrites the arrays in LDS
+  }
+}
+
+template <bool DEV>
+__global__ __launch_bounds__(128) void fused_pair_kernel(FusedArgs a) {
+  __shared__ uint64_t smem[(merge_lds_bytes(128, 8) + 7) / 8];
+  __shared__ uint64_t s_aux[16];
+  const UnitFinder<DEV> units(a);
+  for (uint32_t u = blockIdx.x;; u += gridDim.x) {
+    SectionRef s;
+    uint32_t unit = 0, rows = 0;
+    if (!units.find(a, u, s, unit, rows)) return;
+    switch (s.kind) {
+      case SEC_P6: merge_unit<DEV, 128, 6>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_P8: merge_unit<DEV, 128, 8>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_TOTALS: {
+        const uint32_t t = unit * 2 + (threadIdx.x >> 6);
+        if (t < s.stride) tile_totals_wave(a, a.tile0 + t);
+        break;
+      }
+      default: break;
+    }
+    if (!DEV) return;
+    __syncthreads();
+  }
+}
+
+constexpr size_t WIDE_LDS = sizeof(StreamLds);  // two workgroups of it fill a CU
+static_assert(WIDE_LDS % 8 == 0 && merge_lds_bytes(512, 10) + 512 <= WIDE_LDS, "everything fits the same LDS");
+template <bool DEV>
+__global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
+  __shared__ __align__(16) uint64_t smem[(WIDE_LDS + 7) / 8];
+  // the wavefronts' sums of merge_row, past the end of their arrays
+  uint64_t* const s_aux = smem + (WIDE_LDS - 512) / 8;
+  const UnitFinder<DEV> units(a);
+  for (uint32_t u = blockIdx.x;; u += gridDim.x) {
+    SectionRef s;
+    uint32_t unit = 0, rows = 0;
+    if (!units.find(a, u, s, unit, rows)) return;
+    switch (s.kind) {
+      case SEC_STREAM: {
+        RowRef rr;
+        if (row_at<DEV>(a, s, unit, rows, rr)) {
+          const bool ok = stream_row(rr, *reinterpret_cast<StreamLds*>(smem), a.wgt, a.table);
+          if (threadIdx.x == 0) a.valid[rr.v] = ok ? 1 : 0;
+        }
+        break;
+      }
+      case SEC_B6: merge_unit<DEV, 512, 6>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_B8: merge_unit<DEV, 512, 8>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_B10: merge_unit<DEV, 512, 10>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_SCAN: {
+        const uint32_t r = a.trow0 + unit;
+        if (a.bitmap && !a.trows[r].active) break;
+        if (a.trows[r].ntiles && a.trows[r].ok)
+          tile_scan_row<512>(a.trows, r, a.ttot, a.BL, a.BH, a.nfh, a.ranges, *reinterpret_cast<TileScanLds<512>*>(smem));
+        if (threadIdx.x == 0) a.trows[r].done = a.epoch;
+        break;
+      }
+      default: break;
+    }
+    if (!DEV) return;
+    __syncthreads();
+  }
+}
+
+template <bool DEV>
+__global__ __launch_bounds__(256) void fused_block_kernel(FusedArgs a) {
+  __shared__ __align__(16) uint64_t smem[(cmax(merge_lds_bytes(256, 10), sizeof(TileEmitLds)) + 7) / 8];
+  __shared__ uint64_t s_aux[32];
+  const UnitFinder<DEV> units(a);
+  for (uint32_t u = blockIdx.x;; u += gridDim.x) {
+    SectionRef s;
+    uint32_t unit = 0, rows = 0;
+    if (!units.find(a, u, s, unit, rows)) return;
+    switch (s.kind) {
+      case SEC_M6: merge_unit<DEV, 256, 6>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_M8: merge_unit<DEV, 256, 8>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_M10: merge_unit<DEV, 256, 10>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_EMIT: {
+        const uint32_t tile = a.tile0 + unit;
+        const TileGeom tg = a.geom[tile];
+        if (tg.span == 0 || (a.bitmap && !a.trows[tg.row].active)) break;
+        tile_emit(tg, tile, a.trows, a.wgt, a.BL, a.BH, a.nfh, a.ranges, a.table, a.valid,
+                  *reinterpret_cast<TileEmitLds*>(smem));
+        break;
+      }
+      default: break;
+    }
+    if (!DEV) return;
+    __syncthreads();
+  }
+}
+// ---------------------------------------------------------------- plan of a graph
+// Geometry of the rows that are built tile by tile, in list order: one workgroup, once per graph.
+__global__ __launch_bounds__(1024) void plan_rows_kernel(const RowRef* __restrict__ list, uint32_t n, TiledRow* __restrict__ rows) {
+  __shared__ uint32_t s_w[16];
+  const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  uint32_t carry = 0;
+  for (uint32_t c = 0; c < n; c += 1024u) {
+    const uint32_t r = c + tid;
+    uint32_t nt = 0;
+    RowRef rr{0, 0, 0, 0};
+    if (r < n) {
+      rr = list[r];
+      nt = ((rr.off & 3u) + rr.d + TILE - 1) / TILE;
+    }
+    const uint32_t inc = group_scan_u32<64>(nt);
+    if (lane == 63) s_w[wave] = inc;
+    __syncthreads();
+    uint32_t before = carry, total = 0;
+    for (uint32_t w = 0; w < 16; ++w) {
+      if (w == wave) before += total;
+      total += s_w[w];
+    }
+    if (r < n) {
+      TiledRow& o = rows[r];
+      o.v = rr.v;
+      o.off = rr.off;
+      o.d = rr.d;
+      o.base = rr.off & ~3u;
+      o.lead = rr.off & 3u;
+      o.span = o.lead + rr.d;
+      o.ntiles = nt;
+      o.tile0 = before + inc - nt;
+      o.bofs = o.tile0 + r;  // every row owns ntiles + 1 prefix slots
+      o.active = o.done = 0;
+    }
+    carry += total;
+    __syncthreads();
+  }
+}
+__global__ __launch_bounds__(256) void plan_tiles_kernel(const TiledRow* __restrict__ rows, TileGeom* __restrict__ geom) {
+  const TiledRow& row = rows[blockIdx.x];
+  for (uint32_t t = threadIdx.x; t < row.ntiles; t += 256)
+    geom[row.tile0 + t] = TileGeom{blockIdx.x, t, row.base, row.lead, row.span, {0, 0, 0}};
+}
+__global__ __launch_bounds__(64) void fused_ledger_kernel(TiledRow* __restrict__ rows, uint32_t row0, const u128* __restrict__ tsum,
+                                                          bool frontier) {
+  TiledRow& row = rows[row0 + blockIdx.x];
+  if (row.ntiles == 0 || (frontier && !row.active)) return;
+  u128 sum{0, 0};
+  for (uint32_t t = threadIdx.x; t < row.ntiles; t += 64) sum = add128(sum, tsum[row.tile0 + t]);
+  sum = group_sum_u128<64>(sum);
+  if (threadIdx.x == 0) {
+    const bool ok = (sum.lo | sum.hi) != 0;
+    row.ok = ok;
+    if (ok) {
+      const Ledger L = make_ledger(row.d, sum);
+      row.scale = L.scale;
+      row.fs = L.fs;
+      row.inv_fs = L.inv_fs;
+      row.one = L.one;
+    }
+  }
+}
+
+namespace {
+// Rows of more tiles than this get their ledger from a launch of its own: 2048 tiles add up 2048 x 2048 sums of 16
+// bytes, 67 MB out of L2, when every tile does it.
+constexpr uint32_t LEDGER_TILES = 2048;
+
+// Frontiers of at most this many rows make the rows of 8190..65533 entries tile by tile.
+constexpr uint32_t SMALL_FRONTIER = 65536;
+
+int alloc(void** p, size_t bytes) {
+  SKY_HIP(hipMalloc(p, bytes + 16));
+  return SKY_OK;
+}
+}  // namespace
+
+void free_plan(sky_graph* g) {
+  if (!g->plan) return;
+  void* ptrs[] = {g->plan->rows, g->plan->trows, g->plan->tiles, g->plan->front};
+  for (void* p : ptrs)
+    if (p) (void)hipFree(p);
+  delete g->plan;
+  g->plan = nullptr;
+}
+
+int ensure_plan(sky_graph* g) {
+  const long long narrow_limit = option(g, OPT_STREAM_MIN_EDGES);
+  if (g->plan && g->plan->narrow_limit == narrow_limit) return SKY_OK;
+  free_plan(g);
+  hipStream_t st = g->stream;
+  g->plan = new BuildPlan();
+  BuildPlan& p = *g->plan;
+  auto body = [&]() -> int {
+    SKY_TRY(bin_all_rows(g, CLS_G16, &p.rows, p.start));
+    p.listed = 0;
+    for (int c = CLS_G16; c < CLS_COUNT; ++c) p.listed += g->bin_counts[c];
+    p.narrow_limit = narrow_limit;
+    // Rows of 8190..65533 entries are streamed, one workgroup each, by builds that hold enough of them to fill the GPU that
+    // way; other builds, and those of small frontiers, make them tile by tile, for which they need geometry.  A graph
+    // with very many of them does without: 65536 tiles that a frontier may have to pass over take 20 us a launch.
+    const uint64_t narrow = g->bin_edges[CLS_STREAM] + g->bin_edges[CLS_STREAM_LAST];
+    p.t_all = (long long)narrow <= narrow_limit ? CLS_STREAM : CLS_STREAM_WIDE;
+    p.t_first = p.t_all == CLS_STREAM || narrow <= 65536ull * TILE ? CLS_STREAM : CLS_STREAM_WIDE;
+    uint64_t edges = 0;
+    for (int c = p.t_first; c <= CLS_HUGE; ++c) {
+      p.n_trows += g->bin_counts[c];
+      edges += g->bin_edges[c];
+    }
+    if (!p.n_trows) return SKY_OK;
+    const uint64_t bound = edges / TILE + 2ull * p.n_trows;
+    if (bound >= (1ull << 31)) return fail(SKY_ERR_LIMIT, "the number of tiles has no usable bound");
+    p.n_tiles = (uint32_t)bound;
+    SKY_TRY(alloc((void**)&p.trows, (size_t)p.n_trows * sizeof(TiledRow)));
+    const size_t nb = (size_t)p.n_tiles + p.n_trows;
+    // one allocation for everything that has one entry per tile
+    const size_t bytes = (size_t)p.n_tiles * (sizeof(TileGeom) + sizeof(u128) + sizeof(uint4) + sizeof(TileTotals) + 4) + nb * 16;
+    char* at = nullptr;
+    SKY_TRY(alloc((void**)&at, bytes));
+    p.tiles = at;
+    auto take = [&](auto& ptr, size_t n) {
+      ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(at);
+      at += n * sizeof(*ptr);
+    };
+    take(p.geom, p.n_tiles);
+    take(p.tsum, p.n_tiles);
+    take(p.ranges, p.n_tiles);
+    take(p.ttot, p.n_tiles);
+    take(p.BL, nb);
+    take(p.BH, nb);
+    take(p.nfh, p.n_tiles);
+    SKY_HIP(hipMemsetAsync(p.geom, 0, (size_t)p.n_tiles * sizeof(TileGeom), st));  // span 0: no such tile
+    hipLaunchKernelGGL(plan_rows_kernel, dim3(1), dim3(1024), 0, st, p.rows + p.start[p.t_first], p.n_trows, p.trows);
+    hipLaunchKernelGGL(plan_tiles_kernel, dim3(p.n_trows), dim3(256), 0, st, p.trows, p.geom);
+    SKY_HIP(hipGetLastError());
+    if (p.t_first != p.t_all) {  // the rows that every build makes tile by tile come after the others
+      p.wide_row = g->bin_counts[CLS_STREAM] + g->bin_counts[CLS_STREAM_LAST];
+      if (p.wide_row < p.n_trows) {
+        SKY_HIP(hipMemcpyAsync(&p.wide_tile, &p.trows[p.wide_row].tile0, 4, hipMemcpyDeviceToHost, st));
+        SKY_HIP(hipStreamSynchronize(st));
+      } else {
+        p.wide_tile = p.n_tiles;
+      }
+    }
+    return SKY_OK;
+  };
+  const int rc = body();
+  if (rc != SKY_OK) free_plan(g);
+  return rc;
+}
+
+namespace {
+struct Launch {
+  FusedArgs a;
+  uint64_t units = 0;
+  uint32_t threads;
+  Launch(const FusedArgs& base, uint32_t t) : a(base), threads(t) {
+    a.nsec = 0;
+    for (uint32_t& f : a.first) f = 0xFFFFFFFFu;
+  }
+  // host-sized: `rows` rows from `start` on
+  void add(Section k, uint32_t rows, uint32_t per, uint32_t start) {
+    if (!rows) return;
+    a.first[a.nsec] = (uint32_t)units;
+    a.sec[a.nsec++] = SectionRef{k, (rows + per - 1) / per, per, start, -1, 0, rows};
+    units += (rows + per - 1) / per;
+  }
+  // device-sized: at most `upper` rows in the segments of the classes cls .. cls + ncls - 1
+  void add_dev(Section k, uint32_t upper, uint32_t per, uint32_t start, int cls, int ncls, uint32_t stride) {
+    if (!upper) return;
+    a.sec[a.nsec++] = SectionRef{k, 0, per, start, cls, ncls, stride};
+    units += (upper + per - 1) / per;
+  }
+};
+
+FusedArgs common_args(sky_graph* g, int tiled_from) {
+  const BuildPlan& p = *g->plan;
+  FusedArgs a = {};
+  a.xadj = g->xadj;
+  a.wgt = g->adjwgt;
+  a.table = g->table;
+  a.valid = g->valid;
+  a.V = g->V;
+  a.trows = p.trows;
+  a.geom = p.geom;
+  a.tsum = p.tsum;
+  a.ttot = p.ttot;
+  a.BL = p.BL;
+  a.BH = p.BH;
+  a.nfh = p.nfh;
+  a.ranges = p.ranges;
+  a.trow0 = tiled_from == p.t_first ? 0u : p.wide_row;
+  a.tile0 = tiled_from == p.t_first ? 0u : p.wide_tile;
+  a.ledgers_done = p.n_trows > a.trow0 && ((uint64_t)g->max_degree + 3 + TILE - 1) / TILE > LEDGER_TILES;
+  return a;
+}
+
+// The four launches, in order on the graph's stream.
+template <bool DEV>
+int launch_all(sky_graph* g, Launch& wave, Launch& pair, Launch& wide, Launch& block) {
+  hipStream_t st = g->stream;
+  // Device-sized launches know a bound of their units only: as many workgroups as the GPU holds at a time stride
+  // over what there is.
+  auto grid = [&](const Launch& l, uint32_t cap) { return dim3((uint32_t)(DEV ? std::min<uint64_t>(l.units, cap) : l.units)); };
+  if (wave.units) hipLaunchKernelGGL((fused_wave_kernel<DEV>), grid(wave, 5120), dim3(64), 0, st, wave.a);
+  if (wave.a.ledgers_done) hipLaunchKernelGGL(fused_ledger_kernel, dim3(g->plan->n_trows - wave.a.trow0), dim3(64), 0, st, g->plan->trows, wave.a.trow0,
+                                              g->plan->tsum, DEV);
+  if (pair.units) hipLaunchKernelGGL((fused_pair_kernel<DEV>), grid(pair, 2560), dim3(128), 0, st, pair.a);
+  if (wide.units) hipLaunchKernelGGL((fused_wide_kernel<DEV>), grid(wide, 512), dim3(512), 0, st, wide.a);
+  if (block.units) hipLaunchKernelGGL((fused_block_kernel<DEV>), grid(block, 1024), dim3(256), 0, st, block.a);
+  SKY_HIP(hipGetLastError());
+  return SKY_OK;
+}
+}  // namespace
+
+bool fused_possible(const sky_graph* g) { return option(g, OPT_ROW_MERGE) != 0 && tiled_max_tiles(g) == (1u << 22); }
+
+int build_all_fused(sky_graph* g, CallDevice* call) {
+  g->has_walk_index = false;
+  const BuildPlan& p = *g->plan;
+  FusedArgs base = common_args(g, p.t_all);
+  const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
+  base.list = p.rows;
+  base.call = call;  // the sweep over the vertices is never empty
+  // at least 64 vertices a wavefront, 1024 at most, and enough wavefronts for every SIMD in between
+  base.per_wave = std::max(64u, std::min(SMALL_RANGE, g->V / 8192u / 64u * 64u));
+  Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
+  auto rows = [&](int c) { return g->bin_counts[c]; };
+  wave.add(SEC_SUM, n_tiles, 1, 0);
+  wave.add(SEC_W2, rows(CLS_LDS_W2), 1, p.start[CLS_LDS_W2]);
+  wave.add(SEC_SWEEP, g->V, base.per_wave, 0);
+  wave.add(SEC_W6, rows(CLS_LDS_W6), 1, p.start[CLS_LDS_W6]);
+  wave.add(SEC_W1, rows(CLS_LDS_W1), 1, p.start[CLS_LDS_W1]);
+  wave.add(SEC_G32X, rows(CLS_G32X), 2, p.start[CLS_G32X]);
+  wave.add(SEC_G32S, rows(CLS_G32S), 2, p.start[CLS_G32S]);
+  wave.add(SEC_G32, rows(CLS_G32), 2, p.start[CLS_G32]);
+  wave.add(SEC_G16, rows(CLS_G16), 4, p.start[CLS_G16]);
+  pair.add(SEC_TOTALS, n_tiles, 2, 0);
+  pair.add(SEC_P8, rows(CLS_MW2), 1, p.start[CLS_MW2]);
+  pair.add(SEC_P6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
+  wide.add(SEC_SCAN, n_trows, 1, 0);
+  if (p.t_all != CLS_STREAM) wide.add(SEC_STREAM, rows(CLS_STREAM) + rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM]);
+  wide.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);  // hold_row beside the others would spill 190 registers
+  wide.add(SEC_B10, rows(CLS_MW2 + 7) + rows(CLS_MW2 + 8), 1, p.start[CLS_MW2 + 7]);
+  wide.add(SEC_B8, rows(CLS_MW2 + 5) + rows(CLS_MW2 + 6), 1, p.start[CLS_MW2 + 5]);
+  wide.add(SEC_B6, rows(CLS_MW2 + 4), 1, p.start[CLS_MW2 + 4]);
+  block.add(SEC_EMIT, n_tiles, 1, 0);
+  block.add(SEC_M10, rows(CLS_MW2 + 3), 1, p.start[CLS_MW2 + 3]);
+  block.add(SEC_M8, rows(CLS_MW2 + 2), 1, p.start[CLS_MW2 + 2]);
+  block.add(SEC_M6, rows(CLS_MW2 + 1), 1, p.start[CLS_MW2 + 1]);
+  return launch_all<false>(g, wave, pair, wide, block);
+}
+
+// ---------------------------------------------------------------- rows of a frontier
+int frontier_lists(sky_graph* g, uint32_t n_upper, FrontierLists* f) {
+  SKY_TRY(ensure_plan(g));
+  BuildPlan& p = *g->plan;
+  // A workgroup needs 125 us to stream a row of 65,000 entries, which is as long as everything else that the build of a
+  // small frontier does; the rows of a large one keep all workgroups streaming, and that is cheaper by the entry.
+  f->tiled_from = n_upper <= SMALL_FRONTIER ? p.t_first : p.t_all;
+  uint64_t at = 0;
+  for (int c = 0; c < CLS_COUNT; ++c) {
+    f->start[c] = (uint32_t)at;
+    const bool tiled = c >= f->tiled_from && c <= CLS_HUGE;
+    const uint64_t in_graph = c == CLS_TINY ? g->bin_edges[c] : g->bin_counts[c];  // a tiny row has an entry at least
+    p.front_cap[c] = c == CLS_EMPTY || tiled ? 0u : (uint32_t)std::min<uint64_t>(n_upper, in_graph);
+    at += p.front_cap[c];
+  }
+  if (p.front_rows < at) {
+    if (p.front) SKY_HIP(hipFree(p.front));
+    p.front = nullptr;
+    p.front_rows = 0;
+    SKY_TRY(alloc((void**)&p.front, at * sizeof(RowRef)));
+    p.front_rows = at;
+  }
+  f->list = p.front;
+  return SKY_OK;
+}
+
+int build_frontier(sky_graph* g, const FrontierLists& f, const uint32_t* counts, const uint32_t* bitmap, uint32_t epoch) {
+  g->has_walk_index = false;
+  const BuildPlan& p = *g->plan;
+  FusedArgs base = common_args(g, f.tiled_from);
+  const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
+  base.list = f.list;
+  base.counts = counts;
+  base.bitmap = bitmap;
+  base.epoch = epoch;
+  Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
+  auto add = [&](Launch& l, Section k, uint32_t per, int cls, int ncls = 1) {
+    uint32_t upper = 0;
+    for (int c = 0; c < ncls; ++c) upper += p.front_cap[cls + c];
+    l.add_dev(k, upper, per, f.start[cls], cls, ncls, ncls > 1 ? f.start[cls + 1] - f.start[cls] : 0u);
+  };
+  wave.add(SEC_SUM, n_tiles, 1, 0);
+  add(wave, SEC_W2, 1, CLS_LDS_W2);
+  add(wave, SEC_W6, 1, CLS_LDS_W6);
+  add(wave, SEC_W1, 1, CLS_LDS_W1);
+  add(wave, SEC_G32X, 2, CLS_G32X);
+  add(wave, SEC_G32S, 2, CLS_G32S);
+  add(wave, SEC_G32, 2, CLS_G32);
+  add(wave, SEC_G16, 4, CLS_G16);
+  add(wave, SEC_G8, 8, CLS_G8);
+  add(wave, SEC_G4, 16, CLS_G4);
+  add(wave, SEC_G2, 32, CLS_G2);
+  add(wave, SEC_TINY, 64, CLS_TINY);
+  pair.add(SEC_TOTALS, n_tiles, 2, 0);
+  add(pair, SEC_P8, 1, CLS_MW2);
+  add(pair, SEC_P6, 1, CLS_MW2_6);
+  wide.add(SEC_SCAN, n_trows, 1, 0);
+  if (f.tiled_from != CLS_STREAM) add(wide, SEC_STREAM, 1, CLS_STREAM, 2);
+  add(wide, SEC_STREAM, 1, CLS_HOLD);
+  add(wide, SEC_B10, 1, CLS_MW2 + 7, 2);
+  add(wide, SEC_B8, 1, CLS_MW2 + 5, 2);
+  add(wide, SEC_B6, 1, CLS_MW2 + 4);
+  block.add(SEC_EMIT, n_tiles, 1, 0);
+  add(block, SEC_M10, 1, CLS_MW2 + 3);
+  add(block, SEC_M8, 1, CLS_MW2 + 2);
+  add(block, SEC_M6, 1, CLS_MW2 + 1);
+  return launch_all<true>(g, wave, pair, wide, block);
+}
+
+}  // namespace sky

@@ -239,6 +239,7 @@ int sky_graph_free(sky_graph* g) {
     if (p) (void)hipFree(p);
   pool_release(g);
   call_release(g);
+  free_plan(g);
   free_build_scratch(g);
   free_tiled_scratch(g);
   if (g->live_report) (void)hipHostFree(g->live_report);

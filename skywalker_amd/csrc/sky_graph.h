@@ -23,12 +23,17 @@ enum SkyOpt : int {
   OPT_COUNT
 };
 
+namespace sky {
+struct BuildPlan;
+}
 struct sky_graph {
   uint32_t V = 0, E = 0, max_degree = 0;
   long long opt_value[OPT_COUNT] = {0};
   bool opt_own[OPT_COUNT] = {false};  // the graph has a value of its own for the knob
   // scratch memory of the table builds on this graph (allocated on first use, reused by every later build, freed
   // with the graph): row lists and counters of the binning pass, and the arrays of the tile-parallel path
+  sky::BuildPlan* plan = nullptr;  // sky_build_fused.h
+  uint32_t frontier_epoch = 0;     // calls that have built frontiers
   void* build_scratch = nullptr;
   void* tiled_scratch = nullptr;
   int device = 0;  // the device that was current when the graph was created: its arrays live there
@@ -65,7 +70,7 @@ struct sky_graph {
   bool call_dirty = false;  // a call has begun and not ended well: its device words may not be zero
 
   // Device buffers that calls on this graph reuse instead of allocating each time (they only grow).
-  enum PoolSlot { POOL_BITMAP = 0, POOL_LIST, POOL_TOTALS, POOL_SLOTS };
+  enum PoolSlot { POOL_BITMAP = 0, POOL_LIST, POOL_TOTALS, POOL_FRONT, POOL_SLOTS };
   struct PoolBuf {
     void* p = nullptr;
     size_t cap = 0;
@@ -82,10 +87,7 @@ struct sky_graph {
   hipEvent_t fork_ev = nullptr;
   hipEvent_t join_ev[SIDE_STREAMS] = {nullptr, nullptr, nullptr};
 
-  // Class sizes of the last binning of all vertices.  They depend on xadj alone, which never changes, so a
-  // later build of all vertices sizes its launches from them without waiting for the device.
-  bool bin_known = false;
-  int bin_listed_from = 0;  // first class that the binning pass behind these sizes gave a list
+  // Class sizes of all vertices (of the classes from CLS_G2 on; entries also of CLS_TINY), valid once there is a plan.
   uint32_t bin_counts[32] = {0};
   unsigned long long bin_edges[32] = {0};
 };
@@ -119,6 +121,38 @@ enum BuildClass : int {
   CLS_COUNT = 30
 };
 
+constexpr int MERGE_MAX_NW = 10;  // rows of at most 512 * 10 - 3 = 5117 entries pair by merge in LDS
+constexpr uint32_t HOLD_MAX_DEG = 8189;  // 512 threads x 16 slots hold such a row from any 16-byte phase
+constexpr uint32_t STREAM_MAX_DEG = 524287;  // longest row of the streaming classes (one workgroup takes 1.5 ms for it)
+__host__ __device__ __forceinline__ int degree_class(uint32_t d) {
+  if (d == 0) return CLS_EMPTY;
+  if (d <= 2) return CLS_TINY;
+  // rows of the group kernels start at any slot (their vector loads and stores only need 4-byte alignment)
+  if (d <= 8) return CLS_G2;
+  if (d <= 16) return CLS_G4;
+  if (d <= 32) return CLS_G8;
+  if (d <= 64) return CLS_G16;
+  if (d <= 128) return CLS_G32;
+  if (d <= 160) return CLS_G32S;
+  if (d <= 192) return CLS_G32X;
+  if (d <= 253) return CLS_LDS_W1;
+  // These kernels are bound by instruction issue: a row pays for the slots of its class, not for its entries.  The
+  // two classes whose rows differ most in length (by a factor of two) are halved: 6 instead of 8 slots per thread
+  // for their shorter rows.
+  if (d <= 381) return CLS_LDS_W6;
+  if (d <= 509) return CLS_LDS_W2;
+  if (d <= 765) return CLS_MW2_6;
+  const uint32_t nw = (d + 3 + 511) / 512;  // wavefronts of 512 slots that hold the row from any 16-byte phase
+  // The arrays of a longer row (14 bytes of LDS per slot) would leave room for one workgroup per CU only: such a row
+  // keeps its heavies alone in LDS, and its entries in registers as long as 512 threads can hold them (1024 threads
+  // for rows of up to 16381 entries, one workgroup per CU, ran at 1.7 TB/s where the streaming kernel reaches 1.95).
+  if (nw <= MERGE_MAX_NW) return CLS_MW2 + (int)nw - 2;
+  if (d <= HOLD_MAX_DEG) return CLS_HOLD;
+  if (d > STREAM_MAX_DEG) return CLS_HUGE;
+  if (d > 65533u) return CLS_STREAM_WIDE;
+  return d > 24576u ? CLS_STREAM : CLS_STREAM_LAST;
+}
+
 // One listed row of a degree class: the build kernels read where the row lies from the list itself
 // instead of chasing xadj[v] after the list entry (one dependent global load less at every row start).
 struct RowRef {
@@ -149,26 +183,18 @@ int build_all_tables(sky_graph* g, double* seconds);
 constexpr uint32_t TILED_TILE = 1024;  // slots per tile of the tile-parallel path
 int build_rows_tiled(sky_graph* g, const RowRef* rows_list, uint32_t n, uint32_t* skipped, EventTimer* tm,
                      uint64_t edges);
-int build_rows_tiled_dev(sky_graph* g, const RowRef* vlist, const uint32_t* dev, int cls, int ncls, uint32_t n_upper,
-                         uint64_t edges_upper);
-constexpr int MERGE_MAX_NW = 10;  // rows of at most 512 * 10 - 3 = 5117 entries pair by merge in LDS
-constexpr uint32_t HOLD_MAX_DEG = 8189;  // 512 threads x 16 slots hold such a row from any 16-byte phase
-constexpr uint32_t STREAM_MAX_DEG = 524287;  // longest row of the streaming classes (one workgroup takes 1.5 ms for it)
 int build_rows_stream(sky_graph* g, const RowRef* first_list, uint32_t n_first, const RowRef* rows_list, uint32_t n);
-int build_rows_stream_dev(sky_graph* g, const RowRef* vlist, const uint32_t* dev, int ncls, uint32_t grid);
-int build_rows_hold(sky_graph* g, const RowRef* rows, uint32_t n, const uint32_t* dev, int cls);
-// Builds the rows listed in src[0 .. *n_dev) (n_dev: a device word the host never reads; n_upper: what it cannot
-// exceed) without waiting for the device at any point.  Needs the graph's class census and a longest row the
-// streaming kernel takes (build_rows_dev_possible).
-bool build_rows_dev_possible(const sky_graph* g);
-int ensure_class_census(sky_graph* g);
-int build_rows_dev(sky_graph* g, const uint32_t* src, const uint32_t* n_dev, uint32_t n_upper);
+int build_rows_hold(sky_graph* g, const RowRef* rows, uint32_t n);
 int build_walk_index(sky_graph* g, double* seconds);
 uint32_t tiled_max_tiles(const sky_graph* g);
 // process-wide values of the knobs (sky_capi.hip) and the accessor every use goes through
 extern long long g_option_value[OPT_COUNT];
 inline long long option(const sky_graph* g, SkyOpt o) { return g && g->opt_own[o] ? g->opt_value[o] : g_option_value[o]; }
 void free_build_scratch(sky_graph* g);
+void free_plan(sky_graph* g);
+// Bins all vertices: the graph's class sizes, and the rows of the classes from `listed_from` on in a list of their own
+// (*rows, allocated here; class c starts at start[c]).
+int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start);
 void free_tiled_scratch(sky_graph* g);
 int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, float stop_prob, uint64_t seed,
                  uint32_t* paths, uint32_t* lengths, uint64_t* sampled, double* seconds);

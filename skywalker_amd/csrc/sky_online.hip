@@ -8,6 +8,7 @@
 //
 // node2vec: the weights of a step depend on the walker's previous vertex
 // (src/api/bias_node2vec.cu:15-27), so each (walker, step) builds its own table.
+#include "sky_build_fused.h"
 #include "sky_graph.h"
 #include "sky_step_draw.h"
 
@@ -15,71 +16,81 @@ namespace sky {
 
 __global__ __launch_bounds__(256) void walk_init_kernel(const uint32_t* __restrict__ seeds, uint32_t N, uint32_t len,
                                                         uint32_t V, uint32_t* __restrict__ paths,
-                                                        uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
+                                                        uint32_t* __restrict__ lengths, CallDevice* __restrict__ call,
+                                                        uint32_t* __restrict__ bitmap, uint32_t words,
+                                                        uint32_t* __restrict__ counts, uint32_t ncounts) {
   call_stamp(call);
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i >= N) return;
-  const uint32_t v = seeds[i];
-  paths[(size_t)i * (len + 1)] = v;
-  // "still walking"; a walker that stops at step s stores s < len.  A start vertex that does not exist
-  // is recorded and never left.
-  lengths[i] = v < V ? len : 0u;
+  const uint32_t i0 = blockIdx.x * 256u + threadIdx.x, step = gridDim.x * 256u;
+  for (uint32_t i = i0; i < words; i += step) bitmap[i] = 0;
+  for (uint32_t i = i0; i < ncounts; i += step) counts[i] = 0;
+  for (uint32_t i = i0; i < N; i += step) {
+    const uint32_t v = seeds[i];
+    paths[(size_t)i * (len + 1)] = v;
+    // "still walking"; a walker that stops at step s stores s < len.  A start vertex that does not exist
+    // is recorded and never left.
+    lengths[i] = v < V ? len : 0u;
+  }
 }
+constexpr uint32_t WALK_INIT_BLOCKS = 2048;
 
-// Stop test and dead-end test of step s; collects the vertices whose table is still missing.
-// counters[0] = new vertices appended to list, counters[1] = walkers that will draw.
-__global__ __launch_bounds__(256) void walk_collect_kernel(const uint32_t* __restrict__ xadj, uint32_t N, uint32_t len,
-                                                           uint32_t s, float stop_prob, uint64_t seed,
-                                                           const uint32_t* __restrict__ paths,
-                                                           uint32_t* __restrict__ lengths,
-                                                           uint32_t* __restrict__ bitmap, uint32_t* __restrict__ list,
-                                                           uint32_t* __restrict__ counters) {
+// The draw of step s - 1 (the rows it needs have just been built) and, for the walkers that go on, the stop and dead-end
+// tests of step s: the vertices whose table is still missing are appended to the segments of the degree
+// classes, or, without segments (list not null), to a plain list.  counts[s * FRONTIER_WORDS ...] are the rows appended
+// per class (or, in word 0, to the list), and in the last word the walkers that will draw.
+constexpr uint32_t LIVE_WORD = FRONTIER_WORDS - 1;
+static_assert((int)LIVE_WORD >= (int)CLS_COUNT, "no class counts in the word of the live walkers");
+__global__ __launch_bounds__(256) void walk_advance_kernel(const uint32_t* __restrict__ xadj,
+                                                           const uint32_t* __restrict__ adjncy,
+                                                           const AliasEntry* __restrict__ table, int8_t* __restrict__ valid,
+                                                           uint32_t N, uint32_t len, uint32_t s, float stop_prob, uint64_t seed,
+                                                           uint32_t* __restrict__ paths, uint32_t* __restrict__ lengths,
+                                                           uint32_t* bitmap, FrontierLists f, uint32_t* __restrict__ list,
+                                                           uint32_t* __restrict__ all_counts, uint32_t* __restrict__ report) {
+  __shared__ uint32_t s_cnt[CLS_COUNT], s_base[CLS_COUNT];
+  __shared__ uint32_t s_n[256 / 64 + 1];
   const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  uint32_t* const counts = all_counts + (size_t)s * FRONTIER_WORDS;
+  // how many walkers drew in the step before, for the host
+  if (report && s && blockIdx.x == 0 && threadIdx.x == 0)
+    __hip_atomic_store(report + s - 1, all_counts[(size_t)(s - 1) * FRONTIER_WORDS + LIVE_WORD], __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
   bool draws = false, fresh = false;
   uint32_t v = 0;
   if (i < N && lengths[i] == len) {
-    const u32x4 r = philox(seed, i, s, 0, DOM_WALK);
-    v = paths[(size_t)i * (len + 1) + s];
-    if ((stop_prob > 0.0f && u24(r.z) < stop_prob) || xadj[v + 1] == xadj[v]) {
-      lengths[i] = s;
-    } else {
-      draws = true;
-      const uint32_t bit = 1u << (v & 31);
-      fresh = !(atomicOr(&bitmap[v >> 5], bit) & bit);
+    uint32_t* path = paths + (size_t)i * (len + 1);
+    bool walking = true;
+    v = path[s ? s - 1 : 0];
+    if (s) {
+      const u32x4 r = philox(seed, i, s - 1, 0, DOM_WALK);
+      const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
+      const uint32_t col = __umulhi(r.x, deg);
+      const AliasEntry e = table[off + col];
+      const uint32_t cand = u24(r.y) < e.prob ? col : e.alias;
+      if (cand == SKY_INVALID) {
+        lengths[i] = s - 1;
+        walking = false;
+      } else {
+        v = adjncy[off + cand];
+        path[s] = v;
+      }
+    }
+    if (walking && s < len) {
+      const u32x4 r = philox(seed, i, s, 0, DOM_WALK);
+      if ((stop_prob > 0.0f && u24(r.z) < stop_prob) || xadj[v + 1] == xadj[v]) {
+        lengths[i] = s;
+      } else {
+        draws = true;
+        const uint32_t bit = 1u << (v & 31);
+        if (!(bitmap[v >> 5] & bit)) fresh = !(atomicOr(&bitmap[v >> 5], bit) & bit);
+      }
     }
   }
-  // one counter update per wavefront and counter
-  const int lane = threadIdx.x & 63;
-  const unsigned long long md = __ballot(draws), mf = __ballot(fresh);
-  if (md && lane == __ffsll((long long)md) - 1) atomicAdd(&counters[1], (uint32_t)__popcll(md));
-  if (mf) {
-    const int first = __ffsll((long long)mf) - 1;
-    uint32_t base = 0;
-    if (lane == first) base = atomicAdd(&counters[0], (uint32_t)__popcll(mf));
-    base = (uint32_t)__shfl((int)base, first, 64);
-    if (fresh) list[base + (uint32_t)__popcll(mf & ((1ull << lane) - 1ull))] = v;
-  }
-}
-
-__global__ __launch_bounds__(256) void walk_step_kernel(const uint32_t* __restrict__ xadj,
-                                                        const uint32_t* __restrict__ adjncy,
-                                                        const AliasEntry* __restrict__ table, uint32_t N, uint32_t len,
-                                                        uint32_t s, uint64_t seed, uint32_t* __restrict__ paths,
-                                                        uint32_t* __restrict__ lengths) {
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  if (i >= N || lengths[i] != len) return;
-  const u32x4 r = philox(seed, i, s, 0, DOM_WALK);
-  uint32_t* path = paths + (size_t)i * (len + 1);
-  const uint32_t v = path[s];
-  const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
-  const uint32_t col = __umulhi(r.x, deg);
-  const AliasEntry e = table[off + col];
-  const uint32_t cand = u24(r.y) < e.prob ? col : e.alias;
-  if (cand == SKY_INVALID) {
-    lengths[i] = s;
-    return;
-  }
-  path[s + 1] = adjncy[off + cand];
+  if (s == len) return;
+  if (!__syncthreads_or(draws)) return;
+  const unsigned long long md = __ballot(draws);
+  if (md && (threadIdx.x & 63) == (uint32_t)__ffsll((long long)md) - 1) atomicAdd(&counts[LIVE_WORD], (uint32_t)__popcll(md));
+  if (list) append_list(fresh, v, list, counts, s_n);
+  else append_rows(fresh, v, xadj, valid, f, counts, s_cnt, s_base);
 }
 
 int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, uint32_t N, uint32_t len,
@@ -119,59 +130,58 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
   }
   hipStream_t st = g->stream;
   CallDevice* call = nullptr;
-  uint32_t *bitmap = nullptr, *list = nullptr, *d_cnt = nullptr;
+  uint32_t *bitmap = nullptr, *list = nullptr, *counts = nullptr;
   const uint32_t words = (g->V + 31) / 32;
-  // Without a row too long for the streaming kernel, no step waits for the device: the size of a step's list stays
-  // there (build_rows_dev), and whether any walker still walks comes back through pinned host words that the host
-  // reads as they arrive, some steps behind what it has enqueued; the steps enqueued past the last walker's end find
-  // nothing to do.
-  const bool dev_sized = build_rows_dev_possible(g) && option(g, OPT_ONLINE_DEVICE_SIZED) != 0;
-  auto body = [&]() -> int {
-    SKY_TRY(ensure_table_storage(g));
-    if (dev_sized) {
-      SKY_TRY(ensure_class_census(g));
-      if (g->live_report_cap < len) {
-        if (g->live_report) SKY_HIP(hipHostFree(g->live_report));
-        g->live_report = nullptr;
-        g->live_report_cap = 0;
-        SKY_HIP(hipHostMalloc((void**)&g->live_report, (size_t)len * 4, hipHostMallocDefault));
-        g->live_report_cap = len;
-      }
-      for (uint32_t s = 0; s < len; ++s) g->live_report[s] = 0xFFFFFFFFu;  // "not reported yet"
+  // Normally no step waits for the device: the rows of a step's list stay there (build_frontier), and whether any
+  // walker still walks comes back through pinned host words that the host reads as they arrive, some steps behind
+  // what it has enqueued; the steps enqueued past the last walker's end find nothing to do.
+  const bool dev_sized = fused_possible(g) && option(g, OPT_ONLINE_DEVICE_SIZED) != 0;
+  FrontierLists front;
+  SKY_TRY(ensure_table_storage(g));
+  const uint32_t upper = std::min(N, g->V);
+  if (dev_sized) {
+    SKY_TRY(frontier_lists(g, upper, &front));
+    if (g->live_report_cap < len) {
+      if (g->live_report) SKY_HIP(hipHostFree(g->live_report));
+      g->live_report = nullptr;
+      g->live_report_cap = 0;
+      SKY_HIP(hipHostMalloc((void**)&g->live_report, (size_t)len * 4, hipHostMallocCoherent));
+      g->live_report_cap = len;
     }
-    SKY_TRY(prepare_build_scratch(g, std::min(N, g->V)));
-    SKY_TRY(call_begin(g, &call));
-    d_cnt = call->count;
-    SKY_TRY(pool_get(g, sky_graph::POOL_BITMAP, (size_t)words * 4, (void**)&bitmap));
-    SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)std::min(N, g->V) * 4, (void**)&list));
-    const uint32_t blocks = (N + 255) / 256;
-    if (N) {
-      SKY_HIP(hipMemsetAsync(bitmap, 0, (size_t)words * 4, st));
-      hipLaunchKernelGGL(walk_init_kernel, dim3(blocks), dim3(256), 0, st, seeds, N, len, g->V, paths, lengths, call);
-      for (uint32_t s = 0; s < len; ++s) {
-        SKY_HIP(hipMemsetAsync(d_cnt, 0, 8, st));
-        hipLaunchKernelGGL(walk_collect_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, N, len, s, stop_prob, seed,
-                           paths, lengths, bitmap, list, d_cnt);
-        if (dev_sized) {
-          SKY_HIP(hipMemcpyAsync(&g->live_report[s], d_cnt + 1, 4, hipMemcpyDeviceToHost, st));
-          bool ended = false;
-          for (uint32_t k = 0; k < s && !ended; ++k) ended = *(volatile uint32_t*)&g->live_report[k] == 0;
-          if (ended) break;  // a step that has run found no walker left
-          SKY_TRY(build_rows_dev(g, list, d_cnt, std::min(N, g->V)));
-        } else {
-          uint32_t cnt[2] = {0, 0};
-          SKY_HIP(hipMemcpyAsync(cnt, d_cnt, 8, hipMemcpyDeviceToHost, st));
-          SKY_HIP(hipStreamSynchronize(st));
-          if (cnt[1] == 0) break;  // every walker has stopped
-          SKY_TRY(build_rows(g, list, cnt[0], nullptr));
-        }
-        hipLaunchKernelGGL(walk_step_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, g->adjncy, g->table, N,
-                           len, s, seed, paths, lengths);
+    for (uint32_t s = 0; s < len; ++s) g->live_report[s] = 0xFFFFFFFFu;  // "not reported yet"
+    ++g->frontier_epoch;
+  } else {
+    SKY_TRY(prepare_build_scratch(g, upper));
+    SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)upper * 4, (void**)&list));
+  }
+  const uint64_t ncounts = ((uint64_t)len + 1) * FRONTIER_WORDS;
+  if (ncounts > 0xFFFFFFFFull) return fail(SKY_ERR_LIMIT, "walk: too many steps");
+  SKY_TRY(pool_get(g, sky_graph::POOL_BITMAP, (size_t)words * 4, (void**)&bitmap));
+  SKY_TRY(pool_get(g, sky_graph::POOL_FRONT, (size_t)ncounts * 4, (void**)&counts));
+  SKY_TRY(call_begin(g, &call));
+  if (N) {
+    const uint32_t blocks = (uint32_t)(((uint64_t)N + 255) / 256);
+    hipLaunchKernelGGL(walk_init_kernel, dim3(std::min(std::max(blocks, (words + 255) / 256), WALK_INIT_BLOCKS)), dim3(256), 0, st,
+                       seeds, N, len, g->V, paths, lengths, call, bitmap, words, counts, (uint32_t)ncounts);
+    for (uint32_t s = 0; s <= len; ++s) {
+      hipLaunchKernelGGL(walk_advance_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, g->adjncy, g->table, g->valid, N, len, s,
+                         stop_prob, seed, paths, lengths, bitmap, front, list, counts, dev_sized ? g->live_report : nullptr);
+      if (s == len) break;
+      if (dev_sized) {
+        bool ended = false;
+        for (uint32_t k = 0; k < s && !ended; ++k) ended = *(volatile uint32_t*)&g->live_report[k] == 0;
+        if (ended) break;  // a step that has run found no walker left
+        SKY_TRY(build_frontier(g, front, counts + (size_t)s * FRONTIER_WORDS, bitmap, g->frontier_epoch));
+      } else {
+        uint32_t cnt[FRONTIER_WORDS] = {0};
+        SKY_HIP(hipMemcpyAsync(cnt, counts + (size_t)s * FRONTIER_WORDS, sizeof(cnt), hipMemcpyDeviceToHost, st));
+        SKY_HIP(hipStreamSynchronize(st));
+        if (cnt[LIVE_WORD] == 0) break;  // every walker has stopped
+        SKY_TRY(build_rows(g, list, cnt[0], nullptr));
       }
     }
-    return call_end(g, sampled, seconds, lengths, N);
-  };
-  return body();
+  }
+  return call_end(g, sampled, seconds, lengths, N);
 }
 
 // ---------------------------------------------------------------- node2vec
@@ -236,7 +246,8 @@ int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, 
   CallDevice* call = nullptr;
   SKY_TRY(call_begin(g, &call));
   if (N) {
-    hipLaunchKernelGGL(walk_init_kernel, dim3((N + 255) / 256), dim3(256), 0, st, seeds, N, len, g->V, paths, lengths, call);
+    hipLaunchKernelGGL(walk_init_kernel, dim3(std::min((uint32_t)(((uint64_t)N + 255) / 256), WALK_INIT_BLOCKS)), dim3(256), 0, st,
+                       seeds, N, len, g->V, paths, lengths, call, (uint32_t*)nullptr, 0u, (uint32_t*)nullptr, 0u);
     for (uint32_t s = 0; s < len; ++s)
       hipLaunchKernelGGL(n2v_step_kernel, dim3(N), dim3(N2V_T), 0, st, g->xadj, g->adjncy, g->adjwgt, len, s, p, q, stop_prob,
                          seed, paths, lengths);

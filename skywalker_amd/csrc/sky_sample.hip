@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <vector>
 
+#include "sky_build_fused.h"
 #include "sky_graph.h"
 
 namespace sky {
@@ -244,19 +245,21 @@ __global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
 }
 
 // Collects the distinct vertices of the filled slots of hop h whose table has not been built
-// during this call: first setter of the vertex's bit appends it.  One counter update per workgroup of 1024
-// lanes: every append of a launch goes through one word, and a word serves its atomics one after another
-// (one update per wavefront made this kernel as long as the build it feeds).
+// during this call: the first setter of the vertex's bit appends it, to the segments of the degree classes (sky_build_fused.h), to
+// a plain list, or to both (a null pointer leaves one out).  One update per workgroup of 1024 lanes and counter: a word
+// serves its atomics one after another.
 constexpr int COLLECT_T = 1024;
 __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint32_t* __restrict__ data,
                                                                      const uint32_t* __restrict__ sl, uint64_t total,
                                                                      uint32_t V, HopGeom g, uint32_t* bitmap,
+                                                                     const uint32_t* __restrict__ xadj,
+                                                                     int8_t* __restrict__ valid, FrontierLists f,
+                                                                     uint32_t* __restrict__ counts,
                                                                      uint32_t* __restrict__ list,
                                                                      uint32_t* __restrict__ count) {
-  __shared__ uint32_t s_n[COLLECT_T / 64];
-  __shared__ uint32_t s_base;
+  __shared__ uint32_t s_cnt[CLS_COUNT], s_base[CLS_COUNT];
+  __shared__ uint32_t s_n[COLLECT_T / 64 + 1];
   const uint64_t tid = (uint64_t)blockIdx.x * COLLECT_T + threadIdx.x;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   bool fresh = false, live = false;
   uint32_t v = 0;
   if (tid < total) {
@@ -275,34 +278,24 @@ __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint3
     }
   }
   // The draws of a hop land on a few well-connected vertices again and again.  A bit that reads as set needs no
-  // atomic (bits are never cleared during a call; one that another XCD has set a moment ago may still read as clear,
-  // and then the atomic decides): 94 -> 23 us for a million slots of which a quarter is filled.
+  // atomic: bits are never cleared during a call, and one that another XCD has just set and that still reads as clear
+  // is decided by the atomic.
   if (live) {
     const uint32_t bit = 1u << (v & 31);
     if (!(bitmap[v >> 5] & bit)) fresh = !(atomicOr(&bitmap[v >> 5], bit) & bit);
   }
-  const unsigned long long m = __ballot(fresh);
-  if (lane == 0) s_n[wave] = (uint32_t)__popcll(m);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t n = 0;
-#pragma unroll
-    for (int w = 0; w < COLLECT_T / 64; ++w) n += s_n[w];
-    s_base = n ? atomicAdd(count, n) : 0u;
-  }
-  __syncthreads();
-  if (fresh) {
-    uint32_t base = s_base;
-    for (int w = 0; w < wave; ++w) base += s_n[w];
-    list[base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = v;
-  }
+  if (counts) append_rows(fresh, v, xadj, valid, f, counts, s_cnt, s_base);
+  if (list) append_list(fresh, v, list, count, s_n);
 }
 
 // Start of an online call: start vertices in place, the bitmap of built rows cleared.
 __global__ __launch_bounds__(256) void sample_init_kernel(const uint32_t* __restrict__ seeds, uint32_t N, uint64_t lps,
                                                           uint32_t* __restrict__ data, uint32_t* __restrict__ bitmap,
-                                                          uint32_t words, CallDevice* __restrict__ call) {
+                                                          uint32_t words, uint32_t* __restrict__ counts, uint32_t ncounts,
+                                                          CallDevice* __restrict__ call) {
   call_stamp(call);
+  if (blockIdx.x == 0)
+    for (uint32_t i = threadIdx.x; i < ncounts; i += 256u) counts[i] = 0;
   const uint64_t i0 = (uint64_t)blockIdx.x * 256u + threadIdx.x, step = (uint64_t)gridDim.x * 256u;
   for (uint64_t i = i0; i < words; i += step) bitmap[i] = 0;
   for (uint64_t i = i0; i < N; i += step) data[i * lps] = seeds[i];
@@ -324,6 +317,9 @@ struct SampleSession {
   uint64_t lps = 0, slen = 0;
   CallDevice* call = nullptr;
   uint32_t *bitmap = nullptr, *list = nullptr, *d_count = nullptr;
+  uint32_t* front_counts = nullptr;  // FRONTIER_WORDS device words per hop: rows of every degree class (dev_sized)
+  FrontierLists front;
+  bool want_list = false;        // the caller is to see the frontier as a list of vertices
   uint32_t* totals = nullptr;    // children of each start vertex, when the kernels add them up
   uint32_t frontier_upper = 0;   // most rows the last frontier can hold
   uint32_t frontier_count = 0;   // its size, when the host has read it (dev_sized false)
@@ -364,7 +360,7 @@ struct SampleSession {
     if (g->has_tables) online = false;  // every row is already there: nothing to build on the way
     // Without the option the host reads the size of every frontier and sizes the launches of its build exactly;
     // with it (the default) nothing inside the call waits for the device.
-    dev_sized = online && build_rows_dev_possible(g) && option(g, OPT_ONLINE_DEVICE_SIZED) != 0;
+    dev_sized = online && fused_possible(g) && option(g, OPT_ONLINE_DEVICE_SIZED) != 0;
     width.assign(hops, 0);
     off.assign(hops, 0);
     loff.assign(hops, 0);
@@ -383,17 +379,22 @@ struct SampleSession {
     const uint32_t words = (g->V + 31) / 32;
     if (online) {
       SKY_TRY(ensure_table_storage(g));
-      if (dev_sized) SKY_TRY(ensure_class_census(g));  // once per graph
-      SKY_TRY(prepare_build_scratch(g, g->V));
+      if (dev_sized) {
+        SKY_TRY(ensure_plan(g));
+        SKY_TRY(pool_get(g, sky_graph::POOL_FRONT, (size_t)(hops - 1) * FRONTIER_WORDS * 4, (void**)&front_counts));
+        ++g->frontier_epoch;
+      } else {
+        SKY_TRY(prepare_build_scratch(g, g->V));
+      }
       SKY_TRY(pool_get(g, sky_graph::POOL_BITMAP, (size_t)words * 4, (void**)&bitmap));
-      SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)g->V * 4, (void**)&list));
+      if (want_list || !dev_sized) SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)g->V * 4, (void**)&list));
     }
     SKY_TRY(call_begin(g, &call));
     d_count = call->count;
     if (N && one_workgroup()) SKY_TRY(pool_get(g, sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
     if (online)
       hipLaunchKernelGGL(sample_init_kernel, dim3(std::min((std::max(N, words) + 255) / 256, 2048u)), dim3(256), 0, st, seeds, N,
-                         lps, data, bitmap, words, call);
+                         lps, data, bitmap, words, front_counts, dev_sized ? (hops - 1) * FRONTIER_WORDS : 0u, call);
     return SKY_OK;
   }
 
@@ -405,10 +406,12 @@ struct SampleSession {
     hipStream_t st = g->stream;
     const HopGeom hg = geom(h);
     const uint64_t slots = (uint64_t)N * hg.width;
-    SKY_HIP(hipMemsetAsync(d_count, 0, 4, st));
-    hipLaunchKernelGGL(frontier_collect_kernel, dim3((uint32_t)((slots + COLLECT_T - 1) / COLLECT_T)), dim3(COLLECT_T), 0,
-                       st, data, sample_lengths, slots, g->V, hg, bitmap, list, d_count);
     frontier_upper = (uint32_t)std::min<uint64_t>(slots, g->V);
+    d_count = call->count + h;
+    if (dev_sized) SKY_TRY(frontier_lists(g, frontier_upper, &front));
+    hipLaunchKernelGGL(frontier_collect_kernel, dim3((uint32_t)((slots + COLLECT_T - 1) / COLLECT_T)), dim3(COLLECT_T), 0, st,
+                       data, sample_lengths, slots, g->V, hg, bitmap, g->xadj, g->valid, front,
+                       dev_sized ? front_counts + h * FRONTIER_WORDS : nullptr, list, d_count);
     if (!dev_sized) {
       SKY_HIP(hipMemcpyAsync(&frontier_count, d_count, 4, hipMemcpyDeviceToHost, st));
       SKY_HIP(hipStreamSynchronize(st));
@@ -419,11 +422,12 @@ struct SampleSession {
   // Online: the rows of the last frontier, from `weights` (null: the graph's own).  The length of the list stays
   // on the device where it can: the kernels of the build find it there, and the host goes on to enqueue the hop
   // without waiting (the reference's sampler never leaves the device either, src/online_sample_new.cu:191-270).
-  int build(const float* weights) {
+  int build(uint32_t h, const float* weights) {
     if (!online || !N || !frontier_upper) return SKY_OK;
     float* const own = g->adjwgt;
     if (weights) g->adjwgt = const_cast<float*>(weights);  // the build only reads it
-    const int rc = dev_sized ? build_rows_dev(g, list, d_count, frontier_upper) : build_rows(g, list, frontier_count, nullptr);
+    const int rc = dev_sized ? build_frontier(g, front, front_counts + h * FRONTIER_WORDS, bitmap, g->frontier_epoch)
+                             : build_rows(g, list, frontier_count, nullptr);
     g->adjwgt = own;
     return rc;
   }
@@ -494,7 +498,7 @@ int sample_khop(sky_graph* g, bool online, const uint32_t* seeds, uint32_t N, co
   }
   for (uint32_t h = 0; h + 1 < hops; ++h) {
     SKY_TRY(s.frontier(h));
-    SKY_TRY(s.build(nullptr));
+    SKY_TRY(s.build(h, nullptr));
     SKY_TRY(s.draw(h, h + 1));
   }
   return s.end(sampled, seconds);
@@ -504,6 +508,7 @@ int sample_khop(sky_graph* g, bool online, const uint32_t* seeds, uint32_t N, co
 int sample_session_begin(sky_graph* g, const uint32_t* seeds, uint32_t N, const uint32_t* fanout, uint32_t hops,
                          uint64_t seed, uint32_t* data, uint32_t* sample_lengths, SampleSession** out) {
   SampleSession* s = new SampleSession(g);
+  s->want_list = true;
   const int rc = s->begin(true, seeds, N, fanout, hops, seed, data, sample_lengths);
   if (rc != SKY_OK) {
     delete s;
@@ -523,7 +528,7 @@ int sample_session_frontier(SampleSession* s, uint32_t hop, const uint32_t** lis
 }
 int sample_session_hop(SampleSession* s, uint32_t hop, const float* weights) {
   if (hop + 1 >= s->hops) return fail(SKY_ERR_ARG, "sky_sample_session_hop: no such hop");
-  SKY_TRY(s->build(weights));
+  SKY_TRY(s->build(hop, weights));
   return s->draw(hop, hop + 1);
 }
 int sample_session_end(SampleSession* s, uint64_t* sampled, double* seconds) {
