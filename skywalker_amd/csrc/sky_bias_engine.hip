@@ -109,6 +109,8 @@ __global__ __launch_bounds__(sky::N2V_T) void bias_step_kernel(View g, uint32_t 
                                                                uint32_t* __restrict__ paths,
                                                                uint32_t* __restrict__ lengths,
                                                                sky_walker_state* __restrict__ states) {
+  __shared__ sky::DrawLds<sky::N2V_T> lds;
+  __shared__ float s_w[sky::FN_CACHE];
   if (live && blockIdx.x >= *n_live) return;
   const uint32_t i = live ? live[blockIdx.x] : blockIdx.x;
   const int tid = threadIdx.x;
@@ -121,17 +123,19 @@ __global__ __launch_bounds__(sky::N2V_T) void bias_step_kernel(View g, uint32_t 
     if (tid == 0) lengths[i] = s;
     return;
   }
-  OperatorRow row;
-  row.view = sky_row_view{g.xadj, g.adjncy, g.adjwgt, g.V, v, off, d};
-  row.st = states + i;
-  row.nbr = g.adjncy + off;
-  const uint32_t cand = sky::step_draw_slot(row, d, r);
+  sky::FunctionRow<OperatorRow> row;
+  row.fn.view = sky_row_view{g.xadj, g.adjncy, g.adjwgt, g.V, v, off, d};
+  row.fn.st = states + i;
+  row.fn.nbr = g.adjncy + off;
+  row.d = d;
+  row.cache = s_w;
+  const uint32_t cand = sky::draw_slot<sky::N2V_T>(row, d, r, lds);
   __syncthreads();  // every lane has read the state before it moves on
   if (tid == 0) {
     if (cand == sky::NONE_SLOT) {
       lengths[i] = s;
     } else {
-      path[s + 1] = row.nbr[cand];
+      path[s + 1] = row.fn.nbr[cand];
       sky_walker_state st = states[i];
       st.last = v;
       st.has_last = 1;

@@ -47,6 +47,8 @@ bool fused_possible(const sky_graph* g);
 int ensure_plan(sky_graph* g);
 // All rows; needs the plan and vertices.
 int build_all_fused(sky_graph* g, CallDevice* call);
+// The rows of at least min_degree entries alone (a class boundary of 33 or more); needs the plan.  `call` is stamped.
+int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call);
 // Segments for a frontier of at most n_upper rows.
 int frontier_lists(sky_graph* g, uint32_t n_upper, FrontierLists* f);
 // Builds the rows in the segments (counts: their lengths, on the device) and those of the tiled classes whose bit is set

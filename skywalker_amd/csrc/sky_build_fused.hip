@@ -314,6 +314,7 @@ template <bool DEV>
 __global__ __launch_bounds__(128) void fused_pair_kernel(FusedArgs a) {
   __shared__ uint64_t smem[(merge_lds_bytes(128, 8) + 7) / 8];
   __shared__ uint64_t s_aux[16];
+  call_stamp(a.call);
   const UnitFinder<DEV> units(a);
   for (uint32_t u = blockIdx.x;; u += gridDim.x) {
     SectionRef s;
@@ -341,6 +342,7 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[(WIDE_LDS + 7) / 8];
   // the wavefronts' sums of merge_row, past the end of their arrays
   uint64_t* const s_aux = smem + (WIDE_LDS - 512) / 8;
+  call_stamp(a.call);
   const UnitFinder<DEV> units(a);
   for (uint32_t u = blockIdx.x;; u += gridDim.x) {
     SectionRef s;
@@ -377,6 +379,7 @@ template <bool DEV>
 __global__ __launch_bounds__(256) void fused_block_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[(cmax(merge_lds_bytes(256, 10), sizeof(TileEmitLds)) + 7) / 8];
   __shared__ uint64_t s_aux[32];
+  call_stamp(a.call);
   const UnitFinder<DEV> units(a);
   for (uint32_t u = blockIdx.x;; u += gridDim.x) {
     SectionRef s;
@@ -600,8 +603,15 @@ FusedArgs common_args(sky_graph* g, int tiled_from) {
 
 // The four launches, in order on the graph's stream.
 template <bool DEV>
-int launch_all(sky_graph* g, Launch& wave, Launch& pair, Launch& wide, Launch& block) {
+int launch_all(sky_graph* g, Launch& wave, Launch& pair, Launch& wide, Launch& block, CallDevice* call) {
   hipStream_t st = g->stream;
+  // the first launch that has anything to do is the call's first
+  Launch* const order[4] = {&wave, &pair, &wide, &block};
+  for (Launch* l : order)
+    if (l->units) {
+      l->a.call = call;
+      break;
+    }
   // Device-sized launches know a bound of their units only: as many workgroups as the GPU holds at a time stride
   // over what there is.
   auto grid = [&](const Launch& l, uint32_t cap) { return dim3((uint32_t)(DEV ? std::min<uint64_t>(l.units, cap) : l.units)); };
@@ -618,20 +628,19 @@ int launch_all(sky_graph* g, Launch& wave, Launch& pair, Launch& wide, Launch& b
 
 bool fused_possible(const sky_graph* g) { return option(g, OPT_ROW_MERGE) != 0 && tiled_max_tiles(g) == (1u << 22); }
 
-int build_all_fused(sky_graph* g, CallDevice* call) {
+static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call) {
   g->has_walk_index = false;
   const BuildPlan& p = *g->plan;
   FusedArgs base = common_args(g, p.t_all);
   const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
   base.list = p.rows;
-  base.call = call;  // the sweep over the vertices is never empty
   // at least 64 vertices a wavefront, 1024 at most, and enough wavefronts for every SIMD in between
   base.per_wave = std::max(64u, std::min(SMALL_RANGE, g->V / 8192u / 64u * 64u));
   Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
-  auto rows = [&](int c) { return g->bin_counts[c]; };
+  auto rows = [&](int c) { return class_min_degree(c) >= min_degree ? g->bin_counts[c] : 0u; };
   wave.add(SEC_SUM, n_tiles, 1, 0);
   wave.add(SEC_W2, rows(CLS_LDS_W2), 1, p.start[CLS_LDS_W2]);
-  wave.add(SEC_SWEEP, g->V, base.per_wave, 0);
+  if (min_degree == 0) wave.add(SEC_SWEEP, g->V, base.per_wave, 0);
   wave.add(SEC_W6, rows(CLS_LDS_W6), 1, p.start[CLS_LDS_W6]);
   wave.add(SEC_W1, rows(CLS_LDS_W1), 1, p.start[CLS_LDS_W1]);
   wave.add(SEC_G32X, rows(CLS_G32X), 2, p.start[CLS_G32X]);
@@ -644,15 +653,19 @@ int build_all_fused(sky_graph* g, CallDevice* call) {
   wide.add(SEC_SCAN, n_trows, 1, 0);
   if (p.t_all != CLS_STREAM) wide.add(SEC_STREAM, rows(CLS_STREAM) + rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM]);
   wide.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);  // hold_row beside the others would spill 190 registers
-  wide.add(SEC_B10, rows(CLS_MW2 + 7) + rows(CLS_MW2 + 8), 1, p.start[CLS_MW2 + 7]);
-  wide.add(SEC_B8, rows(CLS_MW2 + 5) + rows(CLS_MW2 + 6), 1, p.start[CLS_MW2 + 5]);
+  // two classes whose lists lie back to back; min_degree may leave out the first
+  auto add_two = [&](Section k, int c) { wide.add(k, rows(c) + rows(c + 1), 1, p.start[rows(c) ? c : c + 1]); };
+  add_two(SEC_B10, CLS_MW2 + 7);
+  add_two(SEC_B8, CLS_MW2 + 5);
   wide.add(SEC_B6, rows(CLS_MW2 + 4), 1, p.start[CLS_MW2 + 4]);
   block.add(SEC_EMIT, n_tiles, 1, 0);
   block.add(SEC_M10, rows(CLS_MW2 + 3), 1, p.start[CLS_MW2 + 3]);
   block.add(SEC_M8, rows(CLS_MW2 + 2), 1, p.start[CLS_MW2 + 2]);
   block.add(SEC_M6, rows(CLS_MW2 + 1), 1, p.start[CLS_MW2 + 1]);
-  return launch_all<false>(g, wave, pair, wide, block);
+  return launch_all<false>(g, wave, pair, wide, block, call);
 }
+int build_all_fused(sky_graph* g, CallDevice* call) { return build_host_sized(g, 0, call); }
+int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call) { return build_host_sized(g, min_degree, call); }
 
 // ---------------------------------------------------------------- rows of a frontier
 int frontier_lists(sky_graph* g, uint32_t n_upper, FrontierLists* f) {
@@ -720,7 +733,7 @@ int build_frontier(sky_graph* g, const FrontierLists& f, const uint32_t* counts,
   add(block, SEC_M10, 1, CLS_MW2 + 3);
   add(block, SEC_M8, 1, CLS_MW2 + 2);
   add(block, SEC_M6, 1, CLS_MW2 + 1);
-  return launch_all<true>(g, wave, pair, wide, block);
+  return launch_all<true>(g, wave, pair, wide, block, nullptr);
 }
 
 }  // namespace sky

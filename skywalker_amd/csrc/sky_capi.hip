@@ -242,7 +242,6 @@ int sky_graph_free(sky_graph* g) {
   free_plan(g);
   free_build_scratch(g);
   free_tiled_scratch(g);
-  if (g->live_report) (void)hipHostFree(g->live_report);
   delete g;
   return SKY_OK;
 }

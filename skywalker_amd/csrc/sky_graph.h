@@ -76,10 +76,6 @@ struct sky_graph {
     size_t cap = 0;
   };
   PoolBuf pool[POOL_SLOTS];
-  // Pinned host words into which the device reports, step by step, how many walkers of an online walk still walk;
-  // the host reads them without waiting (they lag behind the enqueued steps) to stop enqueuing once none does.
-  uint32_t* live_report = nullptr;
-  size_t live_report_cap = 0;
   // Side streams (default priority) over which a small build spreads its class kernels, the event they wait for
   // and the events the graph's stream waits for afterwards; created on first use.
   static constexpr int SIDE_STREAMS = 3;
@@ -151,6 +147,32 @@ __host__ __device__ __forceinline__ int degree_class(uint32_t d) {
   if (d > STREAM_MAX_DEG) return CLS_HUGE;
   if (d > 65533u) return CLS_STREAM_WIDE;
   return d > 24576u ? CLS_STREAM : CLS_STREAM_LAST;
+}
+
+// Shortest row of a class.
+inline uint32_t class_min_degree(int c) {
+  switch (c) {
+    case CLS_EMPTY: return 0;
+    case CLS_TINY: return 1;
+    case CLS_G2: return 3;
+    case CLS_G4: return 9;
+    case CLS_G8: return 17;
+    case CLS_G16: return 33;
+    case CLS_G32: return 65;
+    case CLS_G32S: return 129;
+    case CLS_G32X: return 161;
+    case CLS_LDS_W1: return 193;
+    case CLS_LDS_W6: return 254;
+    case CLS_LDS_W2: return 382;
+    case CLS_MW2_6: return 510;
+    case CLS_MW2: return 766;
+    case CLS_HOLD: return 512u * MERGE_MAX_NW - 2;
+    case CLS_STREAM_LAST: return HOLD_MAX_DEG + 1;
+    case CLS_STREAM: return 24577;
+    case CLS_STREAM_WIDE: return 65534;
+    case CLS_HUGE: return STREAM_MAX_DEG + 1;
+    default: return c > CLS_MW2 && c <= CLS_MW2 + MERGE_MAX_NW - 2 ? 512u * (uint32_t)(c - CLS_MW2 + 1) - 2 : 0;
+  }
 }
 
 // One listed row of a degree class: the build kernels read where the row lies from the list itself

@@ -1,114 +1,119 @@
-// Walks that build the alias table of the current vertex on the fly (replaces OnlineWalkKernel /
+// Walks on a graph without tables (replaces OnlineWalkKernel /
 // OnlineWalkShMem / OnlineWalkGMem of src/online_walk.cu:82-166,245-327 and online_walk_gmem.cu).
 //
-// Static bias (DeepWalk, PPR): the table of a vertex does not depend on the walker, so each
-// step builds, once, the tables of the distinct vertices the live walkers stand on that were
-// not built earlier in the call, through the kernels of the offline build, and then advances
-// every walker by one draw.  The draws, and so the paths, are those of the offline walk.
+// Static bias (DeepWalk, PPR): the rows that the walk is expected to draw from often get their tables, by the kernels of
+// the offline build; from any other row the one entry that the draw reads is evaluated from the weights.  One
+// kernel then takes every walker through its whole walk.  The draws, and so the paths, are those of the offline walk.
 //
 // node2vec: the weights of a step depend on the walker's previous vertex
-// (src/api/bias_node2vec.cu:15-27), so each (walker, step) builds its own table.
+// (src/api/bias_node2vec.cu:15-27), so each (walker, step) has a table of its own, of which one entry is evaluated.
 #include "sky_build_fused.h"
 #include "sky_graph.h"
 #include "sky_step_draw.h"
 
 namespace sky {
 
-__global__ __launch_bounds__(256) void walk_init_kernel(const uint32_t* __restrict__ seeds, uint32_t N, uint32_t len,
-                                                        uint32_t V, uint32_t* __restrict__ paths,
-                                                        uint32_t* __restrict__ lengths, CallDevice* __restrict__ call,
-                                                        uint32_t* __restrict__ bitmap, uint32_t words,
-                                                        uint32_t* __restrict__ counts, uint32_t ncounts) {
-  call_stamp(call);
-  const uint32_t i0 = blockIdx.x * 256u + threadIdx.x, step = gridDim.x * 256u;
-  for (uint32_t i = i0; i < words; i += step) bitmap[i] = 0;
-  for (uint32_t i = i0; i < ncounts; i += step) counts[i] = 0;
-  for (uint32_t i = i0; i < N; i += step) {
-    const uint32_t v = seeds[i];
-    paths[(size_t)i * (len + 1)] = v;
-    // "still walking"; a walker that stops at step s stores s < len.  A start vertex that does not exist
-    // is recorded and never left.
-    lengths[i] = v < V ? len : 0u;
-  }
-}
-constexpr uint32_t WALK_INIT_BLOCKS = 2048;
-
-// The draw of step s - 1 (the rows it needs have just been built) and, for the walkers that go on, the stop and dead-end
-// tests of step s: the vertices whose table is still missing are appended to the segments of the degree
-// classes, or, without segments (list not null), to a plain list.  counts[s * FRONTIER_WORDS ...] are the rows appended
-// per class (or, in word 0, to the list), and in the last word the walkers that will draw.
-constexpr uint32_t LIVE_WORD = FRONTIER_WORDS - 1;
-static_assert((int)LIVE_WORD >= (int)CLS_COUNT, "no class counts in the word of the live walkers");
-__global__ __launch_bounds__(256) void walk_advance_kernel(const uint32_t* __restrict__ xadj,
-                                                           const uint32_t* __restrict__ adjncy,
-                                                           const AliasEntry* __restrict__ table, int8_t* __restrict__ valid,
-                                                           uint32_t N, uint32_t len, uint32_t s, float stop_prob, uint64_t seed,
-                                                           uint32_t* __restrict__ paths, uint32_t* __restrict__ lengths,
-                                                           uint32_t* bitmap, FrontierLists f, uint32_t* __restrict__ list,
-                                                           uint32_t* __restrict__ all_counts, uint32_t* __restrict__ report) {
-  __shared__ uint32_t s_cnt[CLS_COUNT], s_base[CLS_COUNT];
-  __shared__ uint32_t s_n[256 / 64 + 1];
-  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
-  uint32_t* const counts = all_counts + (size_t)s * FRONTIER_WORDS;
-  // how many walkers drew in the step before, for the host
-  if (report && s && blockIdx.x == 0 && threadIdx.x == 0)
-    __hip_atomic_store(report + s - 1, all_counts[(size_t)(s - 1) * FRONTIER_WORDS + LIVE_WORD], __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_SYSTEM);
-  bool draws = false, fresh = false;
-  uint32_t v = 0;
-  if (i < N && lengths[i] == len) {
-    uint32_t* path = paths + (size_t)i * (len + 1);
-    bool walking = true;
-    v = path[s ? s - 1 : 0];
-    if (s) {
-      const u32x4 r = philox(seed, i, s - 1, 0, DOM_WALK);
-      const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
-      const uint32_t col = __umulhi(r.x, deg);
-      const AliasEntry e = table[off + col];
-      const uint32_t cand = u24(r.y) < e.prob ? col : e.alias;
-      if (cand == SKY_INVALID) {
-        lengths[i] = s - 1;
-        walking = false;
-      } else {
-        v = adjncy[off + cand];
-        path[s] = v;
-      }
-    }
-    if (walking && s < len) {
-      const u32x4 r = philox(seed, i, s, 0, DOM_WALK);
-      if ((stop_prob > 0.0f && u24(r.z) < stop_prob) || xadj[v + 1] == xadj[v]) {
-        lengths[i] = s;
-      } else {
-        draws = true;
-        const uint32_t bit = 1u << (v & 31);
-        if (!(bitmap[v >> 5] & bit)) fresh = !(atomicOr(&bitmap[v >> 5], bit) & bit);
-      }
-    }
-  }
-  if (s == len) return;
-  if (!__syncthreads_or(draws)) return;
-  const unsigned long long md = __ballot(draws);
-  if (md && (threadIdx.x & 63) == (uint32_t)__ffsll((long long)md) - 1) atomicAdd(&counts[LIVE_WORD], (uint32_t)__popcll(md));
-  if (list) append_list(fresh, v, list, counts, s_n);
-  else append_rows(fresh, v, xadj, valid, f, counts, s_cnt, s_base);
-}
-
 int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, uint32_t N, uint32_t len,
                          float stop_prob, uint64_t seed, uint32_t* paths, uint32_t* lengths, uint64_t* sampled,
                          double* seconds);
 
-// Option online_full_build: -1: decide by the estimate below; 0: always build lazily, step by step; 1: always build
-// every row first.
+// Vectors that are only 4-byte aligned: global loads of 16 bytes need no more on gfx950.
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// Estimated milliseconds of the two ways to serve a static-bias online walk.  A lazy round costs a
-// host round trip and a handful of small launches (about 1/8 ms measured), and the rounds together
-// build at most min(N * len, V) rows; the full build runs at about 1.3e8 edges per millisecond.
-static bool online_prefers_full_build(const sky_graph* g, uint32_t N, uint32_t len) {
+// ---------------------------------------------------------------- static bias
+// The graph's own weights of a row (the weight array has 16 spare bytes, so four slots can be read from any).
+struct PlainRow {
+  static constexpr int U = 4;
+  const float* w;
+  uint32_t d;
+  __device__ __forceinline__ void first(uint32_t k, float (&x)[4]) const {
+    x[0] = x[1] = x[2] = x[3] = 0.0f;
+    if (k < d) {
+      const float4u q = *reinterpret_cast<const float4u*>(w + k);
+      x[0] = clamp_weight(q.x);
+      x[1] = masked_weight(q.y, k + 1 < d);
+      x[2] = masked_weight(q.z, k + 2 < d);
+      x[3] = masked_weight(q.w, k + 3 < d);
+    }
+  }
+  __device__ __forceinline__ void again(uint32_t k, float (&x)[4]) const { first(k, x); }
+};
+
+// A walker per workgroup of T threads, for the whole walk.  Rows of table_from entries and more have tables; from the
+// others the draw is evaluated directly.
+template <int T>
+__global__ __launch_bounds__(T) void walk_direct_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
+                                                        const float* __restrict__ wgt, const AliasEntry* __restrict__ table,
+                                                        uint32_t table_from, const uint32_t* __restrict__ seeds, uint32_t first,
+                                                        uint32_t V, uint32_t len, float stop_prob, uint64_t seed,
+                                                        uint32_t* __restrict__ paths, uint32_t* __restrict__ lengths,
+                                                        CallDevice* __restrict__ call) {
+  __shared__ DrawLds<T> lds;
+  call_stamp(call);
+  const uint32_t i = first + blockIdx.x;
+  uint32_t* const path = paths + (size_t)i * (len + 1);
+  uint32_t v = seeds[i], s = 0;
+  if (threadIdx.x == 0) path[0] = v;
+  for (; s < len && v < V; ++s) {
+    const u32x4 r = philox(seed, i, s, 0, DOM_WALK);
+    if (stop_prob > 0.0f && u24(r.z) < stop_prob) break;
+    const uint32_t off = xadj[v], d = xadj[v + 1] - off;
+    if (d == 0) break;
+    uint32_t cand;
+    if (d >= table_from) {
+      const uint32_t col = __umulhi(r.x, d);
+      const AliasEntry e = table[off + col];
+      cand = u24(r.y) < e.prob ? col : e.alias;
+      static_assert(NONE_SLOT == SKY_INVALID, "a row without weight ends the walk either way");
+    } else {
+      PlainRow row{wgt + off, d};
+      cand = draw_slot<T>(row, d, r, lds);
+    }
+    if (cand == NONE_SLOT) break;
+    v = adjncy[off + cand];
+    if (threadIdx.x == 0) path[s + 1] = v;
+  }
+  if (threadIdx.x == 0) lengths[i] = s;
+}
+
+// How to serve a static-bias walk on a graph without tables.  Every row drawn from costs either its table (about
+// BUILD_PS a entry, once) or two sweeps over its weights (about DRAW_PS a entry, each time).  A step leads to a row
+// with a probability that grows with its length, so a row of d entries is drawn from about N * len * d / E times, and
+// its table pays from the length on at which N * len * d / E * DRAW_PS exceeds BUILD_PS.  Measured on one MI355X.
+constexpr double BUILD_PS = 8.0, DRAW_PS = 2.5;
+constexpr double BUILD_US = 40.0, STEP_US = 4.0;  // launches of a build; the chain of loads and scans of a step
+
+struct OnlinePlan {
+  bool full;            // every row, then the offline walk
+  uint32_t table_from;  // else: the rows of at least so many entries
+};
+static int online_plan(sky_graph* g, uint32_t N, uint32_t len, OnlinePlan* o) {
   const long long mode = option(g, OPT_ONLINE_FULL_BUILD);
-  if (mode >= 0) return mode != 0;
-  const double all_ms = (double)g->E / 1.3e8;
-  const double visited = std::min(1.0, (double)N * len / std::max(1u, g->V));
-  return 0.4 + all_ms < 0.125 * len + visited * all_ms;
+  *o = OnlinePlan{mode > 0, 0xFFFFFFFFu};
+  if (mode > 0) return SKY_OK;
+  SKY_TRY(ensure_plan(g));
+  const double E = std::max(1u, g->E), draws = (double)N * len;
+  const double from = BUILD_PS / DRAW_PS * E / std::max(1.0, draws);
+  // the shortest class whose rows are all that long; the classes below G16 (33 entries) are not built apart from the rest
+  double built = 0, direct = 0;
+  bool any = false;
+  for (int c = CLS_TINY; c < CLS_COUNT; ++c) {
+    const double entries = (double)g->bin_edges[c], lo = class_min_degree(c);
+    if (entries == 0) continue;
+    const double mean = c == CLS_TINY ? 1.5 : entries / std::max(1u, g->bin_counts[c]);
+    if (c >= CLS_G16 && lo >= from) {
+      built += entries;
+      o->table_from = std::min(o->table_from, class_min_degree(c));
+      any = true;
+    } else {
+      direct += draws * entries / E * mean;
+    }
+  }
+  const double hybrid_us = (any ? BUILD_US : 0.0) + (built * BUILD_PS + direct * DRAW_PS) * 1e-6 + STEP_US * len;
+  const double full_us = BUILD_US + E * BUILD_PS * 1e-6 + 1.2 * len;
+  o->full = mode < 0 && full_us < hybrid_us;
+  return SKY_OK;
 }
 
 int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* seeds, uint32_t N, uint32_t len,
@@ -118,11 +123,14 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
     return walk_node2vec_reject(g, p, q, seeds, N, len, stop_prob, seed, paths, lengths, sampled, seconds);
   if (bias_kind == SKY_BIAS_NODE2VEC)
     return walk_online_node2vec(g, p, q, seeds, N, len, stop_prob, seed, paths, lengths, sampled, seconds);
-  // Tables that already exist are used as they are.  Otherwise one build of every row, then the
-  // offline kernel, is taken when it is expected to cost less than len rounds of lazy builds, each
-  // of which waits for the host; the paths are the same either way.
+  // Tables that already exist are used as they are.  Otherwise the rows that the walk will draw from often get theirs, all
+  // of them when that is most of what it meets; the paths are the same either way.
   double build_sec = 0;
-  if (!g->has_tables && N && len && online_prefers_full_build(g, N, len)) SKY_TRY(build_all_tables(g, &build_sec));
+  OnlinePlan how{false, 0xFFFFFFFFu};
+  if (!g->has_tables && N && len) {
+    SKY_TRY(online_plan(g, N, len, &how));
+    if (how.full) SKY_TRY(build_all_tables(g, &build_sec));
+  }
   if (g->has_tables) {
     SKY_TRY(walk_offline(g, seeds, N, len, stop_prob, seed, paths, lengths, sampled, seconds));
     if (seconds) *seconds += build_sec;
@@ -130,113 +138,224 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
   }
   hipStream_t st = g->stream;
   CallDevice* call = nullptr;
-  uint32_t *bitmap = nullptr, *list = nullptr, *counts = nullptr;
-  const uint32_t words = (g->V + 31) / 32;
-  // Normally no step waits for the device: the rows of a step's list stay there (build_frontier), and whether any
-  // walker still walks comes back through pinned host words that the host reads as they arrive, some steps behind
-  // what it has enqueued; the steps enqueued past the last walker's end find nothing to do.
-  const bool dev_sized = fused_possible(g) && option(g, OPT_ONLINE_DEVICE_SIZED) != 0;
-  FrontierLists front;
-  SKY_TRY(ensure_table_storage(g));
-  const uint32_t upper = std::min(N, g->V);
-  if (dev_sized) {
-    SKY_TRY(frontier_lists(g, upper, &front));
-    if (g->live_report_cap < len) {
-      if (g->live_report) SKY_HIP(hipHostFree(g->live_report));
-      g->live_report = nullptr;
-      g->live_report_cap = 0;
-      SKY_HIP(hipHostMalloc((void**)&g->live_report, (size_t)len * 4, hipHostMallocCoherent));
-      g->live_report_cap = len;
-    }
-    for (uint32_t s = 0; s < len; ++s) g->live_report[s] = 0xFFFFFFFFu;  // "not reported yet"
-    ++g->frontier_epoch;
-  } else {
-    SKY_TRY(prepare_build_scratch(g, upper));
-    SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)upper * 4, (void**)&list));
-  }
-  const uint64_t ncounts = ((uint64_t)len + 1) * FRONTIER_WORDS;
-  if (ncounts > 0xFFFFFFFFull) return fail(SKY_ERR_LIMIT, "walk: too many steps");
-  SKY_TRY(pool_get(g, sky_graph::POOL_BITMAP, (size_t)words * 4, (void**)&bitmap));
-  SKY_TRY(pool_get(g, sky_graph::POOL_FRONT, (size_t)ncounts * 4, (void**)&counts));
   SKY_TRY(call_begin(g, &call));
+  if (how.table_from != 0xFFFFFFFFu) {
+    SKY_TRY(build_rows_from(g, how.table_from, call));
+    call = nullptr;  // the build's first kernel is the call's
+  }
   if (N) {
-    const uint32_t blocks = (uint32_t)(((uint64_t)N + 255) / 256);
-    hipLaunchKernelGGL(walk_init_kernel, dim3(std::min(std::max(blocks, (words + 255) / 256), WALK_INIT_BLOCKS)), dim3(256), 0, st,
-                       seeds, N, len, g->V, paths, lengths, call, bitmap, words, counts, (uint32_t)ncounts);
-    for (uint32_t s = 0; s <= len; ++s) {
-      hipLaunchKernelGGL(walk_advance_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, g->adjncy, g->table, g->valid, N, len, s,
-                         stop_prob, seed, paths, lengths, bitmap, front, list, counts, dev_sized ? g->live_report : nullptr);
-      if (s == len) break;
-      if (dev_sized) {
-        bool ended = false;
-        for (uint32_t k = 0; k < s && !ended; ++k) ended = *(volatile uint32_t*)&g->live_report[k] == 0;
-        if (ended) break;  // a step that has run found no walker left
-        SKY_TRY(build_frontier(g, front, counts + (size_t)s * FRONTIER_WORDS, bitmap, g->frontier_epoch));
-      } else {
-        uint32_t cnt[FRONTIER_WORDS] = {0};
-        SKY_HIP(hipMemcpyAsync(cnt, counts + (size_t)s * FRONTIER_WORDS, sizeof(cnt), hipMemcpyDeviceToHost, st));
-        SKY_HIP(hipStreamSynchronize(st));
-        if (cnt[LIVE_WORD] == 0) break;  // every walker has stopped
-        SKY_TRY(build_rows(g, list, cnt[0], nullptr));
-      }
+    // Few walkers leave most of the GPU idle: a larger workgroup then takes its walker through a long row faster.
+    constexpr uint32_t FEW = 1024;
+    const uint32_t most = N <= FEW ? 0xFFFFFFFFu / 256 : 0xFFFFFFFFu / 64;  // walkers of one launch: below 2^32 threads
+    for (uint32_t f = 0; f < N; f += std::min(most, N - f)) {
+      const dim3 grid(std::min(most, N - f));
+      if (N <= FEW)
+        hipLaunchKernelGGL(walk_direct_kernel<256>, grid, dim3(256), 0, st, g->xadj, g->adjncy, g->adjwgt, g->table, how.table_from,
+                           seeds, f, g->V, len, stop_prob, seed, paths, lengths, call);
+      else
+        hipLaunchKernelGGL(walk_direct_kernel<64>, grid, dim3(64), 0, st, g->xadj, g->adjncy, g->adjwgt, g->table, how.table_from,
+                           seeds, f, g->V, len, stop_prob, seed, paths, lengths, call);
+      call = nullptr;
     }
   }
   return call_end(g, sampled, seconds, lengths, N);
 }
 
 // ---------------------------------------------------------------- node2vec
-// One workgroup per (walker, step) evaluates the one entry of the step's second-order table that the draw
-// reads (step_draw_slot of sky_step_draw.h).
+// One walker per workgroup of T threads, for the whole walk; every step evaluates the one entry of its second-order
+// table that the draw reads (draw_slot).  The weights of a step need, for every neighbour of the current vertex,
+// whether it is a neighbour of the previous one too.  Both rows are sorted, so each wavefront moves through its part of
+// the current row and, beside it, through the previous row a window of WIN ids at a time that it keeps in LDS: the ids of
+// 256 slots are searched there together.  (A binary search per neighbour in the row in memory, 15 to 17 dependent loads,
+// in every pass, and a launch per step that waited for its slowest walker: 480 us a step for 2,000 walkers on the scale-18
+// graph, 1.1 M entries.)  What the search found stays in LDS, two bits per slot, for the passes that follow.
+constexpr uint32_t N2V_WIN = 1024;       // ids of the previous row in LDS, per wavefront
+constexpr uint32_t N2V_CODES = 65536;    // slots of a row whose result is kept
+constexpr uint32_t N2V_SPARSE = 32;      // previous row longer than the current one by this factor: searched in memory
+
+// number of ids of row[lo .. n) that lie below key, plus lo; a wavefront probes 64 places at a time
+__device__ __forceinline__ uint32_t wave_lower_bound(const uint32_t* __restrict__ row, uint32_t lo, uint32_t n, uint32_t key) {
+  const uint32_t lane = threadIdx.x & 63;
+  uint32_t len = n - lo;
+  while (len > 64u) {
+    const uint32_t step = len / 65u + 1u, end = lo + len, p = lo + (lane + 1) * step - 1;
+    const uint32_t c = (uint32_t)__popcll(__ballot(p < end && row[p] < key));
+    lo += c * step;
+    len = min(step, end - lo);
+  }
+  return lo + (uint32_t)__popcll(__ballot(lane < len && row[lo + lane] < key));
+}
+
 struct N2vRow {
+  static constexpr int U = 1;
   const float* w;
   const uint32_t* nbr;
   const uint32_t* prow;
-  uint32_t pdeg, prev;
+  uint32_t d, pdeg, prev;
   bool has_prev;
   float p, q;
+  uint32_t* win;   // [N2V_WIN], this wavefront's own
+  uint8_t* codes;  // [N2V_CODES / 4]: per slot 0 neighbour of both, 1 the previous vertex, 2 neither
+  uint32_t wpos, wlen;  // window: ids wpos .. wpos + wlen of the previous row
+
   // weight of the edge in slot k after the second-order factor (src/api/bias_node2vec.cu:15-27)
-  __device__ __forceinline__ float operator()(uint32_t k) const {
-    float x = w[k];
-    if (has_prev) {
-      const uint32_t t = nbr[k];
-      if (t == prev) x = __fdiv_rn(x, p);
-      else if (!row_contains(prow, pdeg, t)) x = __fdiv_rn(x, q);
-    }
+  __device__ __forceinline__ float weigh(float x, uint32_t code) const {
+    if (code == 1u) x = __fdiv_rn(x, p);
+    else if (code == 2u) x = __fdiv_rn(x, q);
     return clamp_weight(x);
+  }
+  __device__ __forceinline__ void load_window(uint32_t from) {
+    const uint32_t lane = threadIdx.x & 63;
+    wpos = from;
+    wlen = min(N2V_WIN, pdeg - from);
+    uint4u x[N2V_WIN / 256];
+#pragma unroll
+    for (int j = 0; j < (int)(N2V_WIN / 256); ++j) {
+      const uint32_t k = 256u * j + 4u * lane;
+      x[j] = uint4u{0, 0, 0, 0};
+      if (k < wlen) x[j] = *reinterpret_cast<const uint4u*>(prow + from + k);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // searches of the window before are done
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int j = 0; j < (int)(N2V_WIN / 256); ++j) {
+      const uint32_t k = 256u * j + 4u * lane;
+      win[k] = k < wlen ? x[j].x : 0xFFFFFFFFu;  // no vertex has this id
+      win[k + 1] = k + 1 < wlen ? x[j].y : 0xFFFFFFFFu;
+      win[k + 2] = k + 2 < wlen ? x[j].z : 0xFFFFFFFFu;
+      win[k + 3] = k + 3 < wlen ? x[j].w : 0xFFFFFFFFu;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  // codes of the four slots k .. (two bits each); all lanes of the wavefront together, 4 slots per lane in slot order
+  __device__ __forceinline__ uint32_t find(uint32_t k, const uint32_t (&t)[4]) {
+    uint32_t code = 0;
+    if (pdeg > N2V_SPARSE * d) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (k + j < d) code |= (t[j] == prev ? 1u : row_contains(prow, pdeg, t[j]) ? 0u : 2u) << (2 * j);
+      return code;
+    }
+    // ids of the wavefront's first and last slot (lane 0 is always inside the row)
+    const uint32_t lane = threadIdx.x & 63, kw = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)t[0]);
+    const uint32_t last_slot = min(255u, d - 1 - kw), lj = last_slot & 3u;
+    const uint32_t mine = lj == 0 ? t[0] : lj == 1 ? t[1] : lj == 2 ? t[2] : t[3];
+    const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)(last_slot >> 2));
+    (void)lane;
+    bool hit[4] = {false, false, false, false};
+    if (wlen == 0 || win[wlen - 1] < first) {  // the window lies wholly below these slots
+      const uint32_t from = wpos + wlen;
+      if (from < pdeg) {
+        // a short way is one more window; a long one is searched
+        const uint32_t at = prow[min(from + N2V_WIN, pdeg) - 1] >= first ? from : wave_lower_bound(prow, from, pdeg, first);
+        if (at < pdeg) load_window(at);
+        else { wpos = pdeg; wlen = 0; }
+      }
+    }
+    while (wlen) {
+      uint32_t steps = 1u;
+      while (steps < wlen) steps *= 2;  // wlen <= steps <= N2V_WIN; the places past wlen hold the largest id
+      uint32_t at[4] = {0, 0, 0, 0};
+      for (uint32_t h = steps / 2; h; h /= 2) {
+        uint32_t x[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[j] = win[at[j] + h - 1];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) at[j] += x[j] < t[j] ? h : 0u;
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) hit[j] = hit[j] || win[at[j]] == t[j];
+      if (win[wlen - 1] >= last || wpos + wlen >= pdeg) break;
+      load_window(wpos + wlen);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if (k + j < d) code |= (t[j] == prev ? 1u : hit[j] ? 0u : 2u) << (2 * j);
+    return code;
+  }
+  __device__ __forceinline__ void first(uint32_t k, float (&x)[4]) {
+    uint32_t t[4] = {0, 0, 0, 0};
+    x[0] = x[1] = x[2] = x[3] = 0.0f;
+    if (k < d) {
+      const float4u a = *reinterpret_cast<const float4u*>(w + k);
+      x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
+      if (has_prev) {
+        const uint4u b = *reinterpret_cast<const uint4u*>(nbr + k);
+        t[0] = b.x; t[1] = b.y; t[2] = b.z; t[3] = b.w;
+      }
+    }
+    uint32_t code = 0;
+    if (has_prev) {
+      code = find(k, t);
+      if (d <= N2V_CODES && k < d) codes[k >> 2] = (uint8_t)code;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = k + j < d ? weigh(x[j], (code >> (2 * j)) & 3u) : 0.0f;
+  }
+  __device__ __forceinline__ void again(uint32_t k, float (&x)[4]) const {
+    x[0] = x[1] = x[2] = x[3] = 0.0f;
+    if (k >= d) return;
+    const float4u a = *reinterpret_cast<const float4u*>(w + k);
+    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
+    uint32_t code = 0;
+    if (has_prev) {
+      if (d <= N2V_CODES) {
+        code = codes[k >> 2];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (k + j < d) code |= (nbr[k + j] == prev ? 1u : row_contains(prow, pdeg, nbr[k + j]) ? 0u : 2u) << (2 * j);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = k + j < d ? weigh(x[j], (code >> (2 * j)) & 3u) : 0.0f;
   }
 };
 
-__global__ __launch_bounds__(N2V_T) void n2v_step_kernel(const uint32_t* __restrict__ xadj,
-                                                         const uint32_t* __restrict__ adjncy,
-                                                         const float* __restrict__ wgt, uint32_t len, uint32_t s,
-                                                         float p, float q, float stop_prob, uint64_t seed,
-                                                         uint32_t* __restrict__ paths,
-                                                         uint32_t* __restrict__ lengths) {
-  const uint32_t i = blockIdx.x;
-  const int tid = threadIdx.x;
-  if (lengths[i] != len) return;  // stopped at an earlier step
-  const u32x4 r = philox(seed, i, s, 0, DOM_WALK);
-  uint32_t* path = paths + (size_t)i * (len + 1);
-  const uint32_t v = path[s];
-  const uint32_t off = xadj[v], d = xadj[v + 1] - off;
-  if ((stop_prob > 0.0f && u24(r.z) < stop_prob) || d == 0) {
-    if (tid == 0) lengths[i] = s;
-    return;
+template <int T>
+__global__ __launch_bounds__(T) void walk_n2v_table_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
+                                                           const float* __restrict__ wgt, const uint32_t* __restrict__ seeds,
+                                                           uint32_t first, uint32_t V, uint32_t len, float p, float q,
+                                                           float stop_prob, uint64_t seed, uint32_t* __restrict__ paths,
+                                                           uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
+  __shared__ DrawLds<T> lds;
+  __shared__ uint32_t s_win[T / 64][N2V_WIN];
+  __shared__ uint8_t s_codes[N2V_CODES / 4];
+  call_stamp(call);
+  const uint32_t i = first + blockIdx.x;
+  uint32_t* const path = paths + (size_t)i * (len + 1);
+  uint32_t v = seeds[i], s = 0, prev = 0, prev_off = 0, prev_deg = 0;
+  if (threadIdx.x == 0) path[0] = v;
+  for (; s < len && v < V; ++s) {
+    const u32x4 r = philox(seed, i, s, 0, DOM_WALK);
+    if (stop_prob > 0.0f && u24(r.z) < stop_prob) break;
+    const uint32_t off = xadj[v], d = xadj[v + 1] - off;
+    if (d == 0) break;
+    N2vRow row;
+    row.w = wgt + off;
+    row.nbr = adjncy + off;
+    row.prow = adjncy + prev_off;
+    row.d = d;
+    row.pdeg = prev_deg;
+    row.prev = prev;
+    row.has_prev = s > 0;
+    row.p = p;
+    row.q = q;
+    row.win = s_win[threadIdx.x >> 6];
+    row.codes = s_codes;
+    row.wpos = row.wlen = 0;
+    const uint32_t cand = draw_slot<T>(row, d, r, lds);
+    if (cand == NONE_SLOT) break;
+    prev = v;
+    prev_off = off;
+    prev_deg = d;
+    v = row.nbr[cand];
+    if (threadIdx.x == 0) path[s + 1] = v;
   }
-  N2vRow row;
-  row.w = wgt + off;
-  row.nbr = adjncy + off;
-  row.has_prev = s > 0;
-  row.prev = s > 0 ? path[s - 1] : 0;
-  row.prow = adjncy + xadj[row.prev];
-  row.pdeg = xadj[row.prev + 1] - xadj[row.prev];
-  row.p = p;
-  row.q = q;
-  const uint32_t cand = step_draw_slot(row, d, r);
-  if (tid == 0) {
-    if (cand == NONE_SLOT) lengths[i] = s;
-    else path[s + 1] = row.nbr[cand];
-  }
+  if (threadIdx.x == 0) lengths[i] = s;
 }
 
 int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, uint32_t N, uint32_t len,
@@ -245,12 +364,18 @@ int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, 
   hipStream_t st = g->stream;
   CallDevice* call = nullptr;
   SKY_TRY(call_begin(g, &call));
-  if (N) {
-    hipLaunchKernelGGL(walk_init_kernel, dim3(std::min((uint32_t)(((uint64_t)N + 255) / 256), WALK_INIT_BLOCKS)), dim3(256), 0, st,
-                       seeds, N, len, g->V, paths, lengths, call, (uint32_t*)nullptr, 0u, (uint32_t*)nullptr, 0u);
-    for (uint32_t s = 0; s < len; ++s)
-      hipLaunchKernelGGL(n2v_step_kernel, dim3(N), dim3(N2V_T), 0, st, g->xadj, g->adjncy, g->adjwgt, len, s, p, q, stop_prob,
-                         seed, paths, lengths);
+  // Four wavefronts per walker (42 KB of LDS, three walkers to a CU); eight while that leaves CUs without one.
+  constexpr uint32_t FEW = 512;
+  const uint32_t most = 0xFFFFFFFFu / 512;  // walkers of one launch: below 2^32 threads
+  for (uint32_t f = 0; f < N; f += std::min(most, N - f)) {
+    const dim3 grid(std::min(most, N - f));
+    if (N <= FEW)
+      hipLaunchKernelGGL(walk_n2v_table_kernel<512>, grid, dim3(512), 0, st, g->xadj, g->adjncy, g->adjwgt, seeds, f, g->V, len, p, q,
+                         stop_prob, seed, paths, lengths, call);
+    else
+      hipLaunchKernelGGL(walk_n2v_table_kernel<256>, grid, dim3(256), 0, st, g->xadj, g->adjncy, g->adjwgt, seeds, f, g->V, len, p, q,
+                         stop_prob, seed, paths, lengths, call);
+    call = nullptr;
   }
   return call_end(g, sampled, seconds, lengths, N);
 }

@@ -1,18 +1,34 @@
-// The draw of one (walker, step) from a table that is never built: only entry `col` of the step's table is ever
-// read, so one workgroup evaluates that entry alone, from the same prefix-sum definition the offline build uses:
+// The draw of one (walker, step) from a table that is never built: only entry `col` of the step's table is ever read, so
+// the threads of a workgroup evaluate that entry alone, from the same prefix-sum definition the offline build uses:
 //   pass 1  exact sum of the row's weights -> ledger, class of entry col
 //           (a light col whose own share accepts the draw needs nothing more)
-//   pass 2  prefix of deficits (or surpluses) up to col
-//   pass 3  first slot whose running prefix crosses it (and the last / next heavy)
-// The result is bit for bit the draw from the fully built table.  The row's weights come from a functor, so the
-// same code serves node2vec's second-order weights and the weights of a bias operator linked in from outside.
+//   pass 2  deficits and surpluses of every chunk of the row; their prefixes over the chunks
+//   then    the one chunk that holds col gives the prefix up to col, and the one chunk in which the other kind's
+//           prefix crosses it gives the slot (and the chunk with the next or last heavy that heavy)
+// The result is bit for bit the draw from the fully built table.  The row's weights come from an object, so the
+// same code serves node2vec's second-order weights, a graph's own weights and those of a bias operator linked in.
+//
+// What bounds it is latency: a walker's step is this chain, one after another.  Two sweeps of the row without a barrier
+// inside and a constant number of steps after them replaced sweeps that synchronised the workgroup six times per 256
+// slots (a row of 35,000 entries: 137 rounds).
 #pragma once
 #include "sky_common.h"
 
 namespace sky {
 
 constexpr int N2V_T = 256;
-constexpr uint32_t N2V_CACHE = 4096;  // second-order weights of rows up to this degree stay in LDS between passes
+constexpr uint32_t NONE_SLOT = 0xFFFFFFFFu;
+constexpr uint32_t DRAW_CHUNK = 256;  // slots a wavefront takes at a time: 4 consecutive ones per lane
+constexpr int DRAW_CHUNKS = 256;      // most chunks of a row; longer rows have longer chunks (a power of two times 256)
+
+template <int T>
+struct DrawLds {
+  uint64_t d[DRAW_CHUNKS], u[DRAW_CHUNKS];  // deficits and surpluses of every chunk, then their inclusive prefixes
+  double fsum[T / 64];
+  u128 sum[T / 64];
+  uint32_t mn[T / 64];
+  uint32_t result;
+};
 
 __device__ __forceinline__ bool row_contains(const uint32_t* __restrict__ row, uint32_t n, uint32_t key) {
   uint32_t lo = 0, len = n;
@@ -30,159 +46,287 @@ __device__ __forceinline__ bool row_contains(const uint32_t* __restrict__ row, u
   return false;
 }
 
-template <class T>
-__device__ __forceinline__ T block_bcast_min(T v, T* s_tmp) {
+// Row-local slot that (walker, step) with random numbers r draws from the row of d >= 1 entries, or NONE_SLOT when
+// their weights sum to zero.  Called by every thread of a workgroup of T.  `row`:
+//   row.first(k, w)   clamped weights of slots k .. k + 3 (k a multiple of 4; zeros past the row).  A wavefront goes
+//                     through its part of the row in slot order, once, all lanes together (k advances by 4 per lane)
+//   row.again(k, w)   the same, afterwards, for any slots and by any wavefront
+//   Row::U            how many chunks' worth of first() may be in flight at once
+template <int T, class Row>
+__device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const u32x4& r, DrawLds<T>& lds) {
+  constexpr int NW = T / 64, U = Row::U;
+  const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  uint32_t csz = DRAW_CHUNK;
+  while ((uint64_t)csz * DRAW_CHUNKS < d) csz *= 2;
+  const uint32_t nc = (uint32_t)(((uint64_t)d + csz - 1) / csz), cpw = (nc + NW - 1) / NW;
+  const uint32_t c0 = wave * cpw, c1 = min(nc, c0 + cpw);
+  __syncthreads();  // the draw before has been read by everyone
+  const uint32_t k0 = c0 < nc ? c0 * csz : d, k1 = c0 < nc ? (c1 == nc ? d : c1 * csz) : d;  // this wavefront's slots
+
+  // pass 1: the sum as a plain fp64 sum where that is exact (plain_sum_is_exact), else in 128 bits
+  double fsum = 0.0;
+  uint32_t mn = 0xFFFFFFFFu;
+  for (uint32_t base = k0; base < k1; base += DRAW_CHUNK * U) {
+    float w[U][4];
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    const T o = (T)shfl_xor_u64((uint64_t)v, m);
-    v = o < v ? o : v;
-  }
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) s_tmp[threadIdx.x >> 6] = v;
-  __syncthreads();
-  T r = s_tmp[0];
-  for (int i = 1; i < N2V_T / 64; ++i) r = s_tmp[i] < r ? s_tmp[i] : r;
-  return r;
-}
-__device__ __forceinline__ uint64_t block_bcast_sum(uint64_t v, uint64_t* s_tmp) {
+    for (int j = 0; j < U; ++j) {
+      w[j][0] = w[j][1] = w[j][2] = w[j][3] = 0.0f;
+      if (base + DRAW_CHUNK * j < k1) row.first(base + DRAW_CHUNK * j + 4 * lane, w[j]);
+    }
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v += shfl_xor_u64(v, m);
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) s_tmp[threadIdx.x >> 6] = v;
-  __syncthreads();
-  uint64_t r = 0;
-  for (int i = 0; i < N2V_T / 64; ++i) r += s_tmp[i];
-  return r;
-}
-
-
-constexpr uint32_t NONE_SLOT = 0xFFFFFFFFu;
-
-// Row-local slot that (walker, step) with random numbers r draws from the row of d >= 1 entries whose clamped
-// weights are row(0..d-1), or NONE_SLOT when they sum to zero.  Called by every thread of a workgroup of N2V_T.
-template <class RowFn>
-__device__ uint32_t step_draw_slot(const RowFn& row, uint32_t d, const u32x4& r) {
-  __shared__ float s_w[N2V_CACHE];
-  __shared__ uint64_t s_tmp[N2V_T / 64];
-  __shared__ u128 s_sum[N2V_T / 64];
-  const int tid = threadIdx.x;
-  const bool cached = d <= N2V_CACHE;
-  auto weight = [&](uint32_t k) -> float { return cached ? s_w[k] : row(k); };
-
-  // pass 1: exact total
-  u128 sum{0, 0};
-  for (uint32_t k = tid; k < d; k += N2V_T) {
-    const float x = row(k);
-    if (cached) s_w[k] = x;
-    sum = add128(sum, weight_fixed(x));
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        fsum += (double)w[j][k];
+        mn = min(mn, __float_as_uint(w[j][k]) - 1u);
+      }
   }
-  sum = group_sum_u128<64>(sum);
-  if ((tid & 63) == 0) s_sum[tid >> 6] = sum;
-  __syncthreads();
-  sum = s_sum[0];
-  for (int k = 1; k < N2V_T / 64; ++k) sum = add128(sum, s_sum[k]);
-  if ((sum.lo | sum.hi) == 0) return NONE_SLOT;
-  const Ledger L = make_ledger(d, sum);
+  fsum = group_sum_f64<64>(fsum);
+  mn = wave_min_u32(mn);
+  if (NW > 1) {
+    if (lane == 0) {
+      lds.fsum[wave] = fsum;
+      lds.mn[wave] = mn;
+    }
+    __syncthreads();
+    fsum = lds.fsum[0];
+    mn = lds.mn[0];
+#pragma unroll
+    for (int i = 1; i < NW; ++i) {
+      fsum += lds.fsum[i];
+      mn = min(mn, lds.mn[i]);
+    }
+  } else {
+    __syncthreads();  // what first() has left in LDS
+  }
+  Ledger L;
+  if (plain_sum_is_exact(fsum, mn)) {
+    if (fsum == 0.0) return NONE_SLOT;
+    L = make_ledger_small(d, fsum);
+    if (d >= (1u << 22)) {
+      const int F = 62 - (31 - __clz((int)d));
+      L.one = 1ull << F;
+      L.fs = (double)L.one;
+      L.inv_fs = 1.0 / L.fs;
+    }
+  } else {
+    u128 sum{0, 0};
+    for (uint32_t base = k0; base < k1; base += DRAW_CHUNK) {
+      float w[4];
+      row.again(base + 4 * lane, w);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) sum = add128(sum, weight_fixed(w[k]));
+    }
+    sum = group_sum_u128<64>(sum);
+    if (NW > 1) {
+      if (lane == 0) lds.sum[wave] = sum;
+      __syncthreads();
+      sum = lds.sum[0];
+#pragma unroll
+      for (int i = 1; i < NW; ++i) sum = add128(sum, lds.sum[i]);
+    }
+    if ((sum.lo | sum.hi) == 0) return NONE_SLOT;
+    L = make_ledger(d, sum);
+  }
   const uint32_t col = __umulhi(r.x, d);
   const float u = u24(r.y);
-  const Entry ec = classify(weight(col), L);
+  Entry ec;
+  {
+    float w[4];
+    row.again(col & ~3u, w);
+    const uint32_t j = col & 3u;
+    ec = classify_fast((double)(j == 0 ? w[0] : j == 1 ? w[1] : j == 2 ? w[2] : w[3]), true, L);
+  }
   if (!ec.heavy && u < (float)ec.p) return col;  // the light keeps the draw: its alias is never read
 
-  // pass 2: prefix up to col of the amounts of col's own kind (exclusive for a light, inclusive for a heavy)
-  uint64_t part = 0;
-  const uint32_t upto = ec.heavy ? col + 1 : col;
-  for (uint32_t k = tid; k < upto; k += N2V_T) {
-    const Entry e = classify(weight(k), L);
-    if (e.heavy == ec.heavy) part += e.amount;
-  }
-  const uint64_t key = block_bcast_sum(part, s_tmp);  // x of a light, y of a heavy
+  // the four slots of this lane in the 256 from `base` on: amounts of the two kinds
+  auto amounts = [&](uint32_t base, uint64_t (&dd)[4], uint64_t (&uu)[4]) {
+    float w[4];
+    row.again(base + 4 * lane, w);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool in = base + 4 * lane + k < d;
+      const Entry e = classify_fast((double)w[k], in, L);
+      dd[k] = in && !e.heavy ? e.amount : 0;
+      uu[k] = e.heavy ? e.amount : 0;
+    }
+  };
 
-  // pass 3: running prefix of the other kind until it crosses the key
-  uint32_t cand;
-  if (!ec.heavy) {
-    // first heavy m with SH(m) > x; the last heavy if none; col itself if the row has no heavy
-    uint64_t carry = 0;
-    uint32_t found = 0xFFFFFFFFu, last_heavy = 0xFFFFFFFFu;
-    for (uint32_t base = 0; base < d && found == 0xFFFFFFFFu; base += N2V_T) {
-      const uint32_t k = base + tid;
-      uint64_t amt = 0;
-      bool heavy = false;
-      if (k < d) {
-        const Entry e = classify(weight(k), L);
-        heavy = e.heavy;
-        amt = heavy ? e.amount : 0;
-      }
-      const uint64_t inc = group_scan_u64<64>(amt);
-      __syncthreads();
-      if ((tid & 63) == 63) s_tmp[tid >> 6] = inc;
-      __syncthreads();
-      uint64_t before = carry, total = 0;
-      for (int wv = 0; wv < N2V_T / 64; ++wv) {
-        if (wv == (tid >> 6)) before += total;
-        total += s_tmp[wv];
-      }
-      const uint32_t hit = (heavy && before + inc > key) ? k : 0xFFFFFFFFu;
-      const uint32_t lh = heavy ? ~k : 0xFFFFFFFFu;  // min of ~k = max of k
-      found = block_bcast_min<uint32_t>(hit, reinterpret_cast<uint32_t*>(s_tmp));
-      const uint32_t lhm = block_bcast_min<uint32_t>(lh, reinterpret_cast<uint32_t*>(s_tmp));
-      if (lhm != 0xFFFFFFFFu) last_heavy = ~lhm;
-      carry += total;
+  // pass 2: totals of the chunks
+  for (uint32_t c = c0; c < c1; ++c) {
+    uint64_t sd = 0, su = 0;
+    const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
+    for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
+      uint64_t dd[4], uu[4];
+      amounts(base, dd, uu);
+      sd += (dd[0] + dd[1]) + (dd[2] + dd[3]);
+      su += (uu[0] + uu[1]) + (uu[2] + uu[3]);
     }
-    cand = found != 0xFFFFFFFFu ? found : (last_heavy != 0xFFFFFFFFu ? last_heavy : col);
-  } else {
-    // next heavy after col (none: col is the last heavy and keeps the draw), then the first light l
-    // with SL(l) >= y: prob = (one + y - SL(l)) / one
-    uint32_t nxt = 0xFFFFFFFFu;
-    for (uint32_t base = col + 1; base < d && nxt == 0xFFFFFFFFu; base += N2V_T) {
-      const uint32_t k = base + tid;
-      uint32_t hit = 0xFFFFFFFFu;
-      if (k < d && classify(weight(k), L).heavy) hit = k;
-      nxt = block_bcast_min<uint32_t>(hit, reinterpret_cast<uint32_t*>(s_tmp));
-    }
-    cand = col;
-    if (nxt != 0xFFFFFFFFu) {
-      uint64_t carry = 0, best = ~0ull;  // best = (index << 0) encoded below
-      uint32_t li = 0xFFFFFFFFu;
-      uint64_t sl_at = 0;
-      for (uint32_t base = 0; base < d && li == 0xFFFFFFFFu; base += N2V_T) {
-        const uint32_t k = base + tid;
-        uint64_t amt = 0;
-        bool light = false;
-        if (k < d) {
-          const Entry e = classify(weight(k), L);
-          light = !e.heavy;
-          amt = light ? e.amount : 0;
-        }
-        const uint64_t inc = group_scan_u64<64>(amt);
-        __syncthreads();
-        if ((tid & 63) == 63) s_tmp[tid >> 6] = inc;
-        __syncthreads();
-        uint64_t before = carry, total = 0;
-        for (int wv = 0; wv < N2V_T / 64; ++wv) {
-          if (wv == (tid >> 6)) before += total;
-          total += s_tmp[wv];
-        }
-        const uint64_t mine = before + inc;
-        const uint32_t hit = (light && mine >= key) ? k : 0xFFFFFFFFu;
-        li = block_bcast_min<uint32_t>(hit, reinterpret_cast<uint32_t*>(s_tmp));
-        if (li != 0xFFFFFFFFu) {
-          // the owner of slot li publishes its prefix
-          __syncthreads();
-          if (k == li) s_tmp[0] = mine;
-          __syncthreads();
-          sl_at = s_tmp[0];
-        }
-        carry += total;
-      }
-      (void)best;
-      if (li != 0xFFFFFFFFu) {
-        const float pr = residual_prob(L.one + key - sl_at, L);
-        cand = u < pr ? col : nxt;
-      }
+    sd = group_scan_u64<64>(sd);
+    su = group_scan_u64<64>(su);
+    if (lane == 63) {
+      lds.d[c] = sd;
+      lds.u[c] = su;
     }
   }
+  __syncthreads();
+
+  if (wave == 0) {
+    {  // prefixes over the chunks: 4 consecutive ones per lane
+      constexpr int PER = DRAW_CHUNKS / 64;
+      uint64_t pd[PER], pu[PER], rd = 0, ru = 0;
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const uint32_t c = lane * PER + j;
+        rd += c < nc ? lds.d[c] : 0;
+        ru += c < nc ? lds.u[c] : 0;
+        pd[j] = rd;
+        pu[j] = ru;
+      }
+      const uint64_t bd = group_scan_u64<64>(rd) - rd, bu = group_scan_u64<64>(ru) - ru;
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        lds.d[lane * PER + j] = bd + pd[j];
+        lds.u[lane * PER + j] = bu + pu[j];
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    // first chunk of the row whose inclusive prefix in p exceeds key, nc if none
+    auto chunk_above = [&](const uint64_t* p, uint64_t key) -> uint32_t {
+#pragma unroll
+      for (int j = 0; j < DRAW_CHUNKS / 64; ++j) {
+        const uint32_t c = 64 * j + lane;
+        const unsigned long long m = __ballot(c < nc && p[c] > key);
+        if (m) return 64 * j + (uint32_t)__ffsll((long long)m) - 1;
+      }
+      return nc;
+    };
+    // first slot of chunk c whose inclusive prefix (of surpluses or deficits) exceeds key, and that prefix
+    auto slot_above = [&](uint32_t c, bool surplus, uint64_t key, uint64_t& at) -> uint32_t {
+      const uint64_t* p = surplus ? lds.u : lds.d;
+      uint64_t before = c ? p[c - 1] : 0;
+      for (uint32_t base = c * csz;; base += DRAW_CHUNK) {
+        uint64_t dd[4], uu[4], run[4];
+        amounts(base, dd, uu);
+        uint64_t t = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          t += surplus ? uu[k] : dd[k];
+          run[k] = t;
+        }
+        const uint64_t inc = group_scan_u64<64>(t), mine = before + inc - t;
+        const unsigned long long m = __ballot(before + inc > key);
+        if (m) {
+          const int l = __ffsll((long long)m) - 1;
+          uint32_t k = 3;
+          uint64_t x = mine + run[3];
+#pragma unroll
+          for (int j = 2; j >= 0; --j)
+            if (mine + run[j] > key) {
+              k = j;
+              x = mine + run[j];
+            }
+          at = shfl_u64(x, l);
+          return (uint32_t)__shfl((int)(base + 4 * lane + k), l, 64);
+        }
+        before += shfl_u64(inc, 63);
+      }
+    };
+    // first (last) heavy slot of [from, end), both inside chunk c; NONE_SLOT if there is none
+    auto heavy_in = [&](uint32_t c, uint32_t from, bool last) -> uint32_t {
+      const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
+      uint32_t got = NONE_SLOT;
+      for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
+        if (base + DRAW_CHUNK <= from) continue;
+        uint64_t dd[4], uu[4];
+        amounts(base, dd, uu);
+        uint32_t mine = NONE_SLOT;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t slot = base + 4 * lane + k;
+          if (uu[k] && slot >= from && (last || mine == NONE_SLOT)) mine = slot;
+        }
+        const unsigned long long m = __ballot(mine != NONE_SLOT);
+        if (m) {
+          const int l = last ? 63 - __clzll((long long)m) : __ffsll((long long)m) - 1;
+          got = (uint32_t)__shfl((int)mine, l, 64);
+          if (!last) break;
+        }
+      }
+      return got;
+    };
+
+    // key: deficits before a light col, surpluses up to and with a heavy col
+    const uint32_t cc = col / csz;
+    uint64_t key = ec.heavy ? (cc ? lds.u[cc - 1] : 0) : (cc ? lds.d[cc - 1] : 0), part = 0;
+    for (uint32_t base = cc * csz; base <= col; base += DRAW_CHUNK) {
+      uint64_t dd[4], uu[4];
+      amounts(base, dd, uu);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t slot = base + 4 * lane + k;
+        part += ec.heavy ? (slot <= col ? uu[k] : 0) : (slot < col ? dd[k] : 0);
+      }
+    }
+    key += shfl_u64(group_scan_u64<64>(part), 63);
+
+    uint32_t cand = col;
+    const uint64_t total_u = lds.u[nc - 1];
+    if (!ec.heavy) {
+      // first heavy whose surplus prefix exceeds the key; the last heavy if there is none; col itself without any heavy
+      const uint32_t cm = chunk_above(lds.u, key);
+      if (cm < nc) {
+        uint64_t at;
+        cand = slot_above(cm, true, key, at);
+      } else if (total_u) {
+        cand = heavy_in(chunk_above(lds.u, total_u - 1), 0, true);
+      }
+    } else {
+      // next heavy after col (none: col is the last heavy and keeps the draw), then the first light l with
+      // SL(l) >= y: prob = (one + y - SL(l)) / one
+      uint32_t nxt = col + 1 < d ? heavy_in(cc, col + 1, false) : NONE_SLOT;
+      if (nxt == NONE_SLOT) {
+        const uint32_t cn = chunk_above(lds.u, lds.u[cc]);
+        if (cn < nc) nxt = heavy_in(cn, 0, false);
+      }
+      const uint32_t cl = nxt != NONE_SLOT ? chunk_above(lds.d, key - 1) : nc;
+      if (cl < nc) {
+        uint64_t sl = 0;
+        (void)slot_above(cl, false, key - 1, sl);
+        cand = u < residual_prob(L.one + key - sl, L) ? col : nxt;
+      }
+    }
+    if (NW == 1) return cand;
+    if (lane == 0) lds.result = cand;
+  }
+  __syncthreads();
+  const uint32_t cand = lds.result;
+  __syncthreads();  // the next draw rewrites what the others still read
   return cand;
 }
 
+// A row whose weights are computed by a function of the slot (row(k): clamped weight of slot k < d): those of a row of up
+// to CAP entries stay in LDS after the first pass, those of a longer one are computed again.
+constexpr uint32_t FN_CACHE = 4096;
+template <class Fn>
+struct FunctionRow {
+  static constexpr int U = 1;
+  Fn fn;
+  uint32_t d;
+  float* cache;  // [FN_CACHE]
+  __device__ __forceinline__ void first(uint32_t k, float (&w)[4]) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      w[j] = k + j < d ? fn(k + j) : 0.0f;
+      if (d <= FN_CACHE && k + j < d) cache[k + j] = w[j];
+    }
+  }
+  __device__ __forceinline__ void again(uint32_t k, float (&w)[4]) const {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = k + j < d ? (d <= FN_CACHE ? cache[k + j] : fn(k + j)) : 0.0f;
+  }
+};
 
 }  // namespace sky
