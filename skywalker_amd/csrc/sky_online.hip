@@ -81,7 +81,11 @@ __global__ __launch_bounds__(T) void walk_direct_kernel(const uint32_t* __restri
 // BUILD_PS a entry, once) or two sweeps over its weights (about DRAW_PS a entry, each time).  A step leads to a row
 // with a probability that grows with its length, so a row of d entries is drawn from about N * len * d / E times, and
 // its table pays from the length on at which N * len * d / E * DRAW_PS exceeds BUILD_PS.  Measured on one MI355X.
-constexpr double BUILD_PS = 8.0, DRAW_PS = 2.5;
+// A few thousand walkers do not fill the GPU: what counts then is how long one walker's draw takes, on four wavefronts, and
+// tables pay from half that length on (R-MAT scale 18 to 24, 10 to 40,000 walkers, 4 to 16 steps: both lie within 10 % of
+// the best of a sweep over the ratio, but for single walkers in long rows).
+constexpr double BUILD_PS = 8.0, DRAW_PS = 2.5, DRAW_FEW_PS = 5.0;
+constexpr uint32_t FEW_WALKERS = 4096;
 constexpr double BUILD_US = 40.0, STEP_US = 4.0;  // launches of a build; the chain of loads and scans of a step
 
 struct OnlinePlan {
@@ -94,7 +98,8 @@ static int online_plan(sky_graph* g, uint32_t N, uint32_t len, OnlinePlan* o) {
   if (mode > 0) return SKY_OK;
   SKY_TRY(ensure_plan(g));
   const double E = std::max(1u, g->E), draws = (double)N * len;
-  const double from = BUILD_PS / DRAW_PS * E / std::max(1.0, draws);
+  const double draw_ps = N <= FEW_WALKERS ? DRAW_FEW_PS : DRAW_PS;
+  const double from = BUILD_PS / draw_ps * E / std::max(1.0, draws);
   // the shortest class whose rows are all that long; the classes below G16 (33 entries) are not built apart from the rest
   double built = 0, direct = 0;
   bool any = false;
@@ -110,7 +115,7 @@ static int online_plan(sky_graph* g, uint32_t N, uint32_t len, OnlinePlan* o) {
       direct += draws * entries / E * mean;
     }
   }
-  const double hybrid_us = (any ? BUILD_US : 0.0) + (built * BUILD_PS + direct * DRAW_PS) * 1e-6 + STEP_US * len;
+  const double hybrid_us = (any ? BUILD_US : 0.0) + (built * BUILD_PS + direct * draw_ps) * 1e-6 + STEP_US * len;
   const double full_us = BUILD_US + E * BUILD_PS * 1e-6 + 1.2 * len;
   o->full = mode < 0 && full_us < hybrid_us;
   return SKY_OK;
@@ -144,17 +149,17 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
     call = nullptr;  // the build's first kernel is the call's
   }
   if (N) {
-    // Few walkers leave most of the GPU idle: a larger workgroup then takes its walker through a long row faster.
-    constexpr uint32_t FEW = 1024;
-    const uint32_t most = N <= FEW ? 0xFFFFFFFFu / 256 : 0xFFFFFFFFu / 64;  // walkers of one launch: below 2^32 threads
+    // the fewer walkers, the larger the workgroup that takes one through a long row
+    const uint32_t T = N <= 256 ? 1024 : N <= FEW_WALKERS ? 256 : 64;
+    const uint32_t most = 0xFFFFFFFFu / T;  // walkers of one launch: below 2^32 threads
     for (uint32_t f = 0; f < N; f += std::min(most, N - f)) {
-      const dim3 grid(std::min(most, N - f));
-      if (N <= FEW)
-        hipLaunchKernelGGL(walk_direct_kernel<256>, grid, dim3(256), 0, st, g->xadj, g->adjncy, g->adjwgt, g->table, how.table_from,
-                           seeds, f, g->V, len, stop_prob, seed, paths, lengths, call);
-      else
-        hipLaunchKernelGGL(walk_direct_kernel<64>, grid, dim3(64), 0, st, g->xadj, g->adjncy, g->adjwgt, g->table, how.table_from,
-                           seeds, f, g->V, len, stop_prob, seed, paths, lengths, call);
+      auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(std::min(most, N - f)), dim3(T), 0, st, g->xadj, g->adjncy, g->adjwgt, g->table,
+                           how.table_from, seeds, f, g->V, len, stop_prob, seed, paths, lengths, call);
+      };
+      if (T == 1024) go(walk_direct_kernel<1024>);
+      else if (T == 256) go(walk_direct_kernel<256>);
+      else go(walk_direct_kernel<64>);
       call = nullptr;
     }
   }
