@@ -1043,7 +1043,7 @@ int build_all_tables(sky_graph* g, double* seconds) {
   SKY_TRY(ensure_table_storage(g));
   // Knobs that name kernels of their own, and per-kernel timing, want the class kernels.
   const bool fused = fused_possible(g) && !option(g, OPT_BUILD_PROFILE) && option(g, OPT_SMALL_IN_PLACE) < 0 &&
-                     option(g, OPT_BUILD_STREAMS) != 0 && g->E <= (getenv("FUSED_MAX") ? atoll(getenv("FUSED_MAX")) : FUSED_MAX_ENTRIES) && g->V;
+                     option(g, OPT_BUILD_STREAMS) != 0 && g->E <= FUSED_MAX_ENTRIES && g->V;
   if (fused) {
     SKY_TRY(ensure_plan(g));
     CallDevice* call = nullptr;

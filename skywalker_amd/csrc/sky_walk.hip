@@ -16,14 +16,15 @@ constexpr int WALK_STAGE = 4;  // steps whose vertices leave together as one 16-
 
 typedef uint32_t path4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// One draw from the row of v.  With the walk index one 16-byte entry holds both possible next vertices (two
-// cache lines per step: xadj and the entry); without it the neighbour id is a third gather.
+// What a step reads first: the bounds of the row of v, eight bytes that need not be aligned to eight.
+typedef uint32_t bounds2u __attribute__((ext_vector_type(2), aligned(4)));
+
+// One draw from the row [off, off + deg) of deg > 0 entries.  With the walk index one 16-byte entry holds both possible
+// next vertices (two cache lines per step: xadj and the entry); without it the neighbour id is a third gather.
 template <bool INDEXED, bool ONCE>
-__device__ __forceinline__ bool walk_draw(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
-                                          const AliasEntry* __restrict__ table, const WalkEntry* __restrict__ index,
-                                          const u32x4& r, uint32_t v, uint32_t& next) {
-  const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
-  if (deg == 0) return false;
+__device__ __forceinline__ bool walk_draw(const uint32_t* __restrict__ adjncy, const AliasEntry* __restrict__ table,
+                                          const WalkEntry* __restrict__ index, const u32x4& r, uint32_t off, uint32_t deg,
+                                          uint32_t& next) {
   const uint32_t col = __umulhi(r.x, deg);
   if (INDEXED) {
     // like the table entry below: read once, so it should not push the row offsets out of L2
@@ -82,6 +83,12 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
     }
     uint32_t s = s_begin;
     walking = v < V;  // a start vertex that does not exist is recorded and never left
+    // The random numbers of a step do not depend on where the walker stands: those of the next step are computed
+    // while the row bounds of this one are on their way (ten rounds, a fifth of a step's time otherwise: 4,096 walkers x
+    // 80 steps on the scale-16 graph 93 -> 85 us, 250,000 PPR walkers with the index 91 -> 74).  Spreading few walkers over
+    // more wavefronts, or requesting the neighbour of col beside the table entry, gained nothing: a step is two or
+    // three loads that miss L2, one after another.
+    u32x4 r = philox(seed, i, s, 0, DOM_WALK);
     while (walking && s < s_end) {
       uint32_t b[WALK_STAGE];
       uint32_t got = 0;
@@ -89,14 +96,21 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
       for (int k = 0; k < WALK_STAGE; ++k) {
         b[k] = 0;
         if (walking && s + got < s_end) {
-          const u32x4 r = philox(seed, i, s + got, 0, DOM_WALK);
-          uint32_t nx = 0;
-          if ((stop_prob > 0.0f && u24(r.z) < stop_prob) || !walk_draw<INDEXED, ONCE>(xadj, adjncy, table, index, r, v, nx)) {
+          if (stop_prob > 0.0f && u24(r.z) < stop_prob) {
             walking = false;
           } else {
-            v = nx;
-            b[k] = nx;
-            got = k + 1;
+            const bounds2u x = *reinterpret_cast<const bounds2u*>(xadj + v);
+            u32x4 rn = philox(seed, i, s + got + 1, 0, DOM_WALK);
+            asm volatile("" : "+v"(rn.x), "+v"(rn.y), "+v"(rn.z));  // here, not where it is used
+            uint32_t nx = 0;
+            if (x.y == x.x || !walk_draw<INDEXED, ONCE>(adjncy, table, index, r, x.x, x.y - x.x, nx)) {
+              walking = false;
+            } else {
+              v = nx;
+              b[k] = nx;
+              got = k + 1;
+            }
+            r = rn;
           }
         }
       }
@@ -345,142 +359,123 @@ int walk_offline_noalloc(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32
 // u24(r_t.w) * fmax < f(candidate), fmax = max(1/p, 1, 1/q); the 65537th candidate is kept whatever
 // it is.  One membership search in the previous vertex's sorted row per trial, instead of one
 // per neighbour of the current vertex.  The reference's unbiased node2vec walker rejects the same way
-// (src/unbiased_walk.cu:14-60).  One walker per lane.
-__device__ __forceinline__ bool row_has(const uint32_t* __restrict__ row, uint32_t n, uint32_t key) {
-  uint32_t lo = 0;
-  while (n > 1) {  // invariant: if key is in the row it is in [lo, lo + n)
-    const uint32_t half = n >> 1;
-    lo = row[lo + half] <= key ? lo + half : lo;
-    n -= half;
-  }
-  return n == 1 && row[lo] == key;
-}
-
-__global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_kernel(
-    const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
-    const AliasEntry* __restrict__ table, const uint32_t* __restrict__ seeds, uint32_t N, uint32_t V, uint32_t len,
-    float fp, float fq, float fmax, float stop_prob, uint64_t seed, bool once, uint32_t* __restrict__ paths,
-    uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
-  call_stamp(call);
-  const uint32_t i = blockIdx.x * WALK_BLOCK + threadIdx.x;
-  uint32_t s = 0;
-  if (i < N) {
-    uint32_t* path = paths + (size_t)i * (len + 1);
-    uint32_t v = seeds[i], prev = 0, prev_off = 0, prev_deg = 0;
-    path[0] = v;
-    for (; s < len && v < V; ++s) {
-      u32x4 r = philox(seed, i, s, 0, DOM_WALK);
-      if (stop_prob > 0.0f && u24(r.z) < stop_prob) break;
-      const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
-      if (deg == 0) break;
-      uint32_t next = 0;
-      bool dead = false;
-      for (uint32_t t = 0;; ++t) {
-        if (t) r = philox(seed, i, s, t, DOM_WALK);
-        const uint32_t col = __umulhi(r.x, deg);
-        const AliasEntry e = once ? load_entry_once(table + off + col) : table[off + col];
-        const uint32_t cand = u24(r.y) < e.prob ? col : e.alias;
-        if (cand == SKY_INVALID) {
-          dead = true;
-          break;
-        }
-        next = adjncy[off + cand];
-        if (s == 0 || t >= 65536u) break;
-        const float f = next == prev ? fp : (row_has(adjncy + prev_off, prev_deg, next) ? 1.0f : fq);
-        if (u24(r.w) * fmax < f) break;
-      }
-      if (dead) break;
-      prev = v;
-      prev_off = off;
-      prev_deg = deg;
-      v = next;
-      path[s + 1] = v;
-    }
-    lengths[i] = s;
-  }
-  unsigned long long t = s;
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
-  if ((threadIdx.x & 63) == 0 && t) atomicAdd(&call->sampled, t);
-}
-
-// The same walk with 8 lanes per walker, for batches too small to fill the GPU with one walker per lane (a
-// batch then lasts as long as its longest walker: steps x the chain of dependent loads of one step).  The lanes
-// of a group hold the walker's state alike and search the previous row together: 8 probes per round narrow
-// the range 9-fold, so a row of 100,000 entries takes 6 dependent loads instead of 17.  Same draws, same paths.
-constexpr int N2V_G = 8;  // a batch of 40,000 walkers x 80 steps on the scale-24 graph, tables built inside: 2.81 ms with one lane per
-                          // walker, 2.35 with 4, 2.25 with 8, 2.45 with 16, 2.59 with 32, 2.68 with 64
-constexpr uint32_t N2V_GROUP_MAX_WALKERS = 1u << 18;
+// (src/unbiased_walk.cu:14-60).
+//
+// G lanes per walker, which hold its state alike and share the work of a step: the random numbers, which cost more
+// instructions than everything else in a trial, are computed for TRIALS trials of STEPS steps at once, one lane each, and
+// all search the previous row together, G probes per round.  Most trials need no search at all: whether the candidate is
+// kept depends on its being a neighbour of the previous vertex only when the drawn number lies between the two cases'
+// limits.  The bounds of the candidate's own row are requested before the search, for the step after.  Leaving the first
+// probe until it is known to be needed, or reading the next step's entry during the search as if the candidate were
+// kept, was slower.
+//
+// A walk lasts as long as its longest chain of dependent loads, so G is the largest whose wavefronts are all resident at
+// once (seven on each of the 1024 SIMDs); once the walkers alone fill the GPU the lanes are worth more as walkers.  80 steps
+// with p = 2, q = 0.5 on a scale-24 graph, in us (the best G for the size, then 8 lanes without the other points above,
+// or one lane above 262,144 walkers): 100 walkers 102 / 175, 10,000 254 / 325, 40,000 401 / 433, 100,000 573 / 900,
+// 1,000,000 (40 steps) 2213 / 2796.
+constexpr uint64_t N2V_LANES = 7ull * 1024 * 64;
+template <int G>
 __device__ __forceinline__ unsigned long long group_ballot(bool p) {
-  const unsigned long long b = __ballot(p) >> (lane_id() & (64u - N2V_G));
-  return N2V_G == 64 ? b : b & ((1ull << (N2V_G & 63)) - 1ull);
+  const unsigned long long b = __ballot(p) >> (lane_id() & (64u - G));
+  return G == 64 ? b : b & ((1ull << (G & 63)) - 1ull);
 }
 // Every lane of the group must call this together with the same row, n and key.
 // The first round's probes depend on the row alone: group_first_probe loads them as soon as the row is known
 // (a step before the key is), and group_row_has takes the value.
+template <int G>
 __device__ __forceinline__ uint32_t group_first_probe(const uint32_t* __restrict__ row, uint32_t n) {
-  const uint32_t gl = lane_id() & (N2V_G - 1);
-  if (n <= (uint32_t)N2V_G) return 0xFFFFFFFFu;
-  const uint32_t p = (gl + 1) * (n / (N2V_G + 1) + 1) - 1;
-  return p < n ? row[p] : 0xFFFFFFFFu;
+  const uint32_t gl = lane_id() & (G - 1);
+  if (n <= (uint32_t)G) return gl < n ? row[gl] : 0xFFFFFFFFu;
+  const uint32_t p = (gl + 1) * (n / (G + 1) + 1) - 1;
+  return p < n ? row[p] : 0xFFFFFFFFu;  // no vertex has this id
 }
+template <int G>
 __device__ __forceinline__ bool group_row_has(const uint32_t* __restrict__ row, uint32_t n, uint32_t key, uint32_t x0) {
-  const uint32_t gl = lane_id() & (N2V_G - 1);
+  const uint32_t gl = lane_id() & (G - 1);
+  if (n <= (uint32_t)G) return group_ballot<G>(x0 == key) != 0;
   uint32_t lo = 0, len = n;  // if the key is in the row it is in [lo, lo + len)
   bool first_round = true;
-  while (len > (uint32_t)N2V_G) {
-    const uint32_t step = len / (N2V_G + 1) + 1, end = lo + len;
+  while (len > (uint32_t)G) {
+    const uint32_t step = len / (G + 1) + 1, end = lo + len;
     const uint32_t p = lo + (gl + 1) * step - 1;           // probe gl: last element of part gl
-    const uint32_t x = first_round ? x0 : (p < end ? row[p] : 0xFFFFFFFFu);  // no vertex has this id
+    const uint32_t x = first_round ? x0 : (p < end ? row[p] : 0xFFFFFFFFu);
     first_round = false;
-    const uint32_t c = (uint32_t)__popcll(group_ballot(x < key));  // parts that lie wholly below the key
+    const uint32_t c = (uint32_t)__popcll(group_ballot<G>(x < key));  // parts that lie wholly below the key
     lo += c * step;
     len = min(step, end - lo);
   }
-  return group_ballot(gl < len && row[lo + gl] == key) != 0;
+  return group_ballot<G>(gl < len && row[lo + gl] == key) != 0;
 }
 
+template <int G>
 __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
     const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
     const AliasEntry* __restrict__ table, const uint32_t* __restrict__ seeds, uint32_t N, uint32_t V, uint32_t len,
     float fp, float fq, float fmax, float stop_prob, uint64_t seed, bool once, uint32_t* __restrict__ paths,
     uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
+  constexpr uint32_t TRIALS = G < 16 ? 2 : G < 32 ? 4 : 8, STEPS = G / TRIALS;
   call_stamp(call);
-  const uint32_t i = (blockIdx.x * WALK_BLOCK + threadIdx.x) / N2V_G;
-  const bool first = (threadIdx.x & (N2V_G - 1)) == 0;  // the lane that writes for the group
+  const uint32_t i = (uint32_t)(((uint64_t)blockIdx.x * WALK_BLOCK + threadIdx.x) / G), gl = threadIdx.x & (G - 1);
+  const int base = (int)(lane_id() & (64u - G));  // first lane of the group
+  const bool first = gl == 0;                     // the lane that writes for the group
   uint32_t s = 0;
   if (i < N) {
     uint32_t* path = paths + (size_t)i * (len + 1);
     uint32_t v = seeds[i], prev = 0, prev_off = 0, prev_deg = 0;
     if (first) path[0] = v;
-    for (; s < len && v < V; ++s) {
-      const uint32_t x0 = group_first_probe(adjncy + prev_off, prev_deg);  // in flight during the loads below
-      u32x4 r = philox(seed, i, s, 0, DOM_WALK);
-      if (stop_prob > 0.0f && u24(r.z) < stop_prob) break;
-      const uint32_t off = xadj[v], deg = xadj[v + 1] - off;
-      if (deg == 0) break;
-      uint32_t next = 0;
-      bool dead = false;
-      for (uint32_t t = 0;; ++t) {
-        if (t) r = philox(seed, i, s, t, DOM_WALK);
-        const uint32_t col = __umulhi(r.x, deg);
-        const AliasEntry e = once ? load_entry_once(table + off + col) : table[off + col];
-        const uint32_t cand = u24(r.y) < e.prob ? col : e.alias;
-        if (cand == SKY_INVALID) {
-          dead = true;
-          break;
+    if (v < V && len) {
+      bounds2u x = *reinterpret_cast<const bounds2u*>(xadj + v);
+      // trial gl % TRIALS of step s0 + gl / TRIALS, where s0 is the last multiple of STEPS
+      u32x4 mine = philox(seed, i, gl / TRIALS, gl % TRIALS, DOM_WALK);
+      const float lo = fminf(1.0f, fq), hi = fmaxf(1.0f, fq);
+      for (;;) {
+        const uint32_t x0 = group_first_probe<G>(adjncy + prev_off, prev_deg);  // in flight during the loads below
+        const uint32_t off = x.x, deg = x.y - x.x;
+        const int from = base + (int)(s % STEPS * TRIALS);
+        if ((stop_prob > 0.0f && u24((uint32_t)__shfl((int)mine.z, from, 64)) < stop_prob) || deg == 0) break;
+        uint32_t next = 0;
+        bool dead = false;
+        u32x4 ahead = mine, more = mine;
+        for (uint32_t t = 0;; ++t) {
+          if (t >= TRIALS && (t - TRIALS) % G == 0) more = philox(seed, i, s, t + gl, DOM_WALK);
+          const bool late = t >= TRIALS;
+          const int lane = late ? base + (int)((t - TRIALS) % G) : from + (int)t;
+          const uint32_t rx = (uint32_t)__shfl((int)(late ? more.x : mine.x), lane, 64);
+          const uint32_t ry = (uint32_t)__shfl((int)(late ? more.y : mine.y), lane, 64);
+          const uint32_t rw = (uint32_t)__shfl((int)(late ? more.w : mine.w), lane, 64);
+          const uint32_t col = __umulhi(rx, deg);
+          const AliasEntry e = once ? load_entry_once(table + off + col) : table[off + col];
+          if (t == 0 && (s + 1) % STEPS == 0) {  // the numbers of the steps ahead, while the entry is on its way
+            ahead = philox(seed, i, s + 1 + gl / TRIALS, gl % TRIALS, DOM_WALK);
+            asm volatile("" : "+v"(ahead.x), "+v"(ahead.y), "+v"(ahead.z), "+v"(ahead.w));
+          }
+          const uint32_t cand = u24(ry) < e.prob ? col : e.alias;
+          if (cand == SKY_INVALID) {
+            dead = true;
+            break;
+          }
+          next = adjncy[off + cand];
+          x = *reinterpret_cast<const bounds2u*>(xadj + next);
+          if (s == 0 || t >= 65536u) break;
+          const float need = u24(rw) * fmax;
+          bool keep;
+          if (next == prev) keep = need < fp;
+          else if (need < lo) keep = true;
+          else if (!(need < hi)) keep = false;
+          else keep = need < (group_row_has<G>(adjncy + prev_off, prev_deg, next, x0) ? 1.0f : fq);
+          if (keep) break;
         }
-        next = adjncy[off + cand];
-        if (s == 0 || t >= 65536u) break;
-        const float f = next == prev ? fp : (group_row_has(adjncy + prev_off, prev_deg, next, x0) ? 1.0f : fq);
-        if (u24(r.w) * fmax < f) break;
+        if (dead) break;
+        mine = ahead;
+        prev = v;
+        prev_off = off;
+        prev_deg = deg;
+        v = next;
+        ++s;
+        if (first) path[s] = v;
+        if (s == len) break;
       }
-      if (dead) break;
-      prev = v;
-      prev_off = off;
-      prev_deg = deg;
-      v = next;
-      if (first) path[s + 1] = v;
     }
     if (first) lengths[i] = s;
   }
@@ -500,14 +495,19 @@ int walk_node2vec_reject(sky_graph* g, float p, float q, const uint32_t* seeds, 
   const float fmax = fmaxf(1.0f, fmaxf(fp, fq));
   CallDevice* call = nullptr;
   SKY_TRY(call_begin(g, &call));
-  if (N && N <= N2V_GROUP_MAX_WALKERS)
-    hipLaunchKernelGGL(walk_n2v_reject_group_kernel, dim3((uint32_t)(((uint64_t)N * N2V_G + WALK_BLOCK - 1) / WALK_BLOCK)),
+  auto run = [&](auto lanes) {
+    constexpr int G = decltype(lanes)::value;
+    hipLaunchKernelGGL(walk_n2v_reject_group_kernel<G>, dim3((uint32_t)(((uint64_t)N * G + WALK_BLOCK - 1) / WALK_BLOCK)),
                        dim3(WALK_BLOCK), 0, st, g->xadj, g->adjncy, g->table, seeds, N, g->V, len, fp, fq, fmax, stop_prob, seed,
                        walk_reads_once(g), paths, lengths, call);
-  else if (N)
-    hipLaunchKernelGGL(walk_n2v_reject_kernel, dim3((N + WALK_BLOCK - 1) / WALK_BLOCK), dim3(WALK_BLOCK), 0, st, g->xadj,
-                       g->adjncy, g->table, seeds, N, g->V, len, fp, fq, fmax, stop_prob, seed, walk_reads_once(g), paths,
-                       lengths, call);
+  };
+  const uint64_t lanes = N ? N2V_LANES / N : 0;  // per walker
+  if (lanes >= 64) run(std::integral_constant<int, 64>{});
+  else if (lanes >= 32) run(std::integral_constant<int, 32>{});
+  else if (lanes >= 16) run(std::integral_constant<int, 16>{});
+  else if (lanes >= 8) run(std::integral_constant<int, 8>{});
+  else if (lanes >= 4) run(std::integral_constant<int, 4>{});
+  else if (N) run(std::integral_constant<int, 2>{});
   SKY_TRY(call_end(g, sampled, seconds));
   if (seconds) *seconds += build_sec;
   return SKY_OK;

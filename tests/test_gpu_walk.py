@@ -223,6 +223,25 @@ def test_node2vec_rejection_one_walker_per_lane_for_large_batches(orc):
     assert np.array_equal(small, opaths[:70000])
 
 
+@pytest.mark.parametrize("walkers", [1, 7168, 7169, 14337, 28673, 57345, 114689])
+def test_node2vec_rejection_group_sizes(orc, walkers):
+    # 64, 64, 32, 16, 8, 4 and 2 lanes per walker; rows around the lengths one and two rounds of probes cover, many trials
+    from skywalker_amd import capi
+    rng = np.random.default_rng(44)
+    degs = [0, 1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 79, 80, 81, 287, 1055, 1056, 4159, 4160, 4161] * 12
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "sparse")
+    seeds = rng.integers(0, len(degs), walkers, dtype=np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    prob, alias, _ = g.tables()
+    for p, q, stop in ((0.25, 4.0, 0.02), (4.0, 0.5, 0.0)):
+        paths, lengths, sampled, _ = g.walk_online(capi.BIAS_NODE2VEC_REJECT, p, q, seeds, 9, stop, 23)
+        want = orc.walk_node2vec_reject(xadj, adjncy, prob, alias, p, q, seeds, 9, stop, 23)
+        assert np.array_equal(paths.to_host((walkers, 10)), want[0]) and np.array_equal(lengths.to_host(), want[1])
+        assert sampled == want[2]
+    g.free()
+
+
 def test_node2vec_rejection_second_step_law(orc):
     # exact second-order law on a small graph, sampled on the device
     from skywalker_amd import capi
