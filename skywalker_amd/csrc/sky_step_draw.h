@@ -206,8 +206,9 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
     // first slot of chunk c whose inclusive prefix (of surpluses or deficits) exceeds key, and that prefix
     auto slot_above = [&](uint32_t c, bool surplus, uint64_t key, uint64_t& at) -> uint32_t {
       const uint64_t* p = surplus ? lds.u : lds.d;
+      const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
       uint64_t before = c ? p[c - 1] : 0;
-      for (uint32_t base = c * csz;; base += DRAW_CHUNK) {
+      for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
         uint64_t dd[4], uu[4], run[4];
         amounts(base, dd, uu);
         uint64_t t = 0;
@@ -233,6 +234,10 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
         }
         before += shfl_u64(inc, 63);
       }
+      // not reached while the weights stay what they were in pass 2; a bias operator that answers differently each
+      // time must not keep the wavefront here
+      at = key + 1;
+      return end - 1;
     };
     // first (last) heavy slot of [from, end), both inside chunk c; NONE_SLOT if there is none
     auto heavy_in = [&](uint32_t c, uint32_t from, bool last) -> uint32_t {
