@@ -411,16 +411,17 @@ __device__ __forceinline__ bool group_row_has(const uint32_t* __restrict__ row, 
 template <int G>
 __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
     const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
-    const AliasEntry* __restrict__ table, const uint32_t* __restrict__ seeds, uint32_t N, uint32_t V, uint32_t len,
+    const AliasEntry* __restrict__ table, const uint32_t* __restrict__ seeds, uint32_t walker0, uint32_t N, uint32_t V, uint32_t len,
     float fp, float fq, float fmax, float stop_prob, uint64_t seed, bool once, uint32_t* __restrict__ paths,
     uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
   constexpr uint32_t TRIALS = G < 16 ? 2 : G < 32 ? 4 : 8, STEPS = G / TRIALS;
-  call_stamp(call);
-  const uint32_t i = (uint32_t)(((uint64_t)blockIdx.x * WALK_BLOCK + threadIdx.x) / G), gl = threadIdx.x & (G - 1);
+  if (walker0 == 0) call_stamp(call);
+  const uint64_t wi = walker0 + ((uint64_t)blockIdx.x * WALK_BLOCK + threadIdx.x) / G;
+  const uint32_t i = (uint32_t)wi, gl = threadIdx.x & (G - 1);
   const int base = (int)(lane_id() & (64u - G));  // first lane of the group
   const bool first = gl == 0;                     // the lane that writes for the group
   uint32_t s = 0;
-  if (i < N) {
+  if (wi < N) {
     uint32_t* path = paths + (size_t)i * (len + 1);
     uint32_t v = seeds[i], prev = 0, prev_off = 0, prev_deg = 0;
     if (first) path[0] = v;
@@ -497,9 +498,13 @@ int walk_node2vec_reject(sky_graph* g, float p, float q, const uint32_t* seeds, 
   SKY_TRY(call_begin(g, &call));
   auto run = [&](auto lanes) {
     constexpr int G = decltype(lanes)::value;
-    hipLaunchKernelGGL(walk_n2v_reject_group_kernel<G>, dim3((uint32_t)(((uint64_t)N * G + WALK_BLOCK - 1) / WALK_BLOCK)),
-                       dim3(WALK_BLOCK), 0, st, g->xadj, g->adjncy, g->table, seeds, N, g->V, len, fp, fq, fmax, stop_prob, seed,
-                       walk_reads_once(g), paths, lengths, call);
+    const uint64_t most = 0x80000000ull / G;  // walkers of one launch: below 2^32 threads
+    for (uint64_t f = 0; f < N; f += most) {
+      const uint64_t threads = std::min<uint64_t>(most, N - f) * G;
+      hipLaunchKernelGGL(walk_n2v_reject_group_kernel<G>, dim3((uint32_t)((threads + WALK_BLOCK - 1) / WALK_BLOCK)),
+                         dim3(WALK_BLOCK), 0, st, g->xadj, g->adjncy, g->table, seeds, (uint32_t)f, N, g->V, len, fp, fq, fmax,
+                         stop_prob, seed, walk_reads_once(g), paths, lengths, call);
+    }
   };
   const uint64_t lanes = N ? N2V_LANES / N : 0;  // per walker
   if (lanes >= 64) run(std::integral_constant<int, 64>{});
