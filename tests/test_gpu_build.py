@@ -385,3 +385,51 @@ def test_device_addresses_of_the_resident_arrays(orc):
     assert np.array_equal(entries[:, 0].view(np.float32), prob) and np.array_equal(entries[:, 1], alias)
     assert np.array_equal(read(pv, len(xadj) - 1, np.int8), valid)
     g.free()
+
+
+def compare_tables(orc, g, xadj, w, label):
+    oprob, oalias, ovalid = orc.alias_build(xadj, w)
+    prob, alias, valid = g.tables()
+    bad = np.flatnonzero((prob.view(np.uint32) != oprob.view(np.uint32)) | (alias != oalias))
+    deg = np.diff(xadj)
+    assert not len(bad), "%s: %d entries differ, first in a row of %d" % (
+        label, len(bad), deg[np.searchsorted(xadj, bad[0], side="right") - 1])
+    assert np.array_equal(valid, ovalid)
+
+
+@pytest.mark.parametrize("stream_min_edges", [0, 4000000])
+@pytest.mark.parametrize("dist", ["lognormal2", "uniform", "equal", "nearequal", "sparse"])
+def test_builds_in_four_launches(orc, dist, stream_min_edges):
+    # the default for up to 2^27 entries: rows of every class, those of 8190..65533 entries streamed or tile by tile; the
+    # second and third build find the row lists of the first, with other weights and with the graph's own again
+    from helpers import weights
+    from skywalker_amd import capi
+    rng = np.random.default_rng(51)
+    degs = EDGE_DEGREES + [24576, 24577, 65533, 65534] + list(rng.integers(0, 300, 700)) + list(rng.integers(300, 9000, 40))
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, dist, V=len(degs) + 70)
+    w2 = weights(len(w), rng, "sparse" if dist == "uniform" else "uniform")
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("stream_min_edges", stream_min_edges)
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, dist)
+    g.build_tables_from_weights(capi.DeviceArray.from_host(np.concatenate([w2, np.zeros(4, np.float32)])))
+    compare_tables(orc, g, xadj, w2, dist + ", other weights")
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, dist + ", again")
+    g.free()
+
+
+@pytest.mark.parametrize("degree", [2048 * 1024 - 3, 2048 * 1024 + 1])
+def test_ledger_of_rows_of_very_many_tiles_in_four_launches(orc, degree):
+    # up to 2048 tiles every tile adds up its row's sums itself, above a launch in between does
+    from helpers import weights
+    from skywalker_amd import capi
+    rng = np.random.default_rng(52)
+    xadj = np.cumsum([0, 3, degree, 0, 700000, 5]).astype(np.uint32)
+    adjncy = rng.integers(0, 5, int(xadj[-1]), dtype=np.uint32)
+    w = weights(len(adjncy), rng, "sparse")
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, "row of %d" % degree)
+    g.free()

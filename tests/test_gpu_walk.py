@@ -357,3 +357,44 @@ def test_walk_index_goes_stale_when_tables_change(orc):
     paths, lengths, sampled, _ = g.walk_offline(seeds, 30, 0.0, 2)
     assert np.array_equal(paths.to_host((3000, 31)), opaths) and sampled == osampled
     g.free()
+
+
+@pytest.mark.parametrize("dist", ["lognormal2", "nearequal", "sparse"])
+@pytest.mark.parametrize("walkers", [1, 256, 257, 4096, 4097])
+def test_online_static_draws_evaluated_from_the_weights(orc, walkers, dist):
+    # workgroups of 1024, 256 and 64 threads; rows around a chunk of 256 slots, and rows of more than 256 chunks; the
+    # fewer draws are expected, the fewer rows get a table
+    from skywalker_amd import capi
+    rng = np.random.default_rng(45)
+    degs = [1, 2, 3, 4, 5, 63, 64, 65, 255, 256, 257, 511, 513, 1023, 1025, 4097, 65535, 65536, 65537, 140001, 0] + \
+        list(rng.integers(1, 400, 60))
+    xadj, adjncy, w = graph_from_degrees(degs, rng, dist)
+    seeds = ((np.arange(walkers) + 19) % len(degs)).astype(np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_full_build", 0)
+    for length, stop in ((1, 0.0), (9, 0.03)):
+        paths, lengths, sampled, _ = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, length, stop, 29)
+        want = orc.walk_online(xadj, adjncy, w, 0, 1.0, 1.0, seeds, length, stop, 29)
+        assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host((walkers, length + 1)), want[0])
+        assert sampled == want[2]
+    g.free()
+
+
+@pytest.mark.parametrize("walkers", [512, 513])
+def test_node2vec_table_rows_beyond_the_window(orc, walkers):
+    # eight and four wavefronts per walker; rows of more than 65,536 entries (membership is searched again instead of kept),
+    # previous rows of many windows of 1024 ids, and of more than 32 times the current row's length
+    from skywalker_amd import capi
+    rng = np.random.default_rng(46)
+    degs = list(rng.integers(0, 300, 1500)) + list(rng.integers(900, 4200, 250)) + [1023, 1024, 1025] * 30 + \
+        list(rng.integers(20000, 65537, 30)) + [65537, 66001, 140003] * 6
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "sparse", V=len(degs) + 3)
+    rows = np.argsort(np.diff(xadj))[-400:]
+    seeds = rng.choice(rows, walkers).astype(np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    paths, lengths, sampled, _ = g.walk_online(capi.BIAS_NODE2VEC, 4.0, 0.25, seeds, 7, 0.0, 31)
+    want = orc.walk_online(xadj, adjncy, w, 1, 4.0, 0.25, seeds, 7, 0.0, 31)
+    assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host((walkers, 8)), want[0])
+    assert sampled == want[2]
+    g.free()
