@@ -234,7 +234,7 @@ def online_bench(args, cfg, capi, g, seeds, name, cus, t_gen, torch):
                   "distinct_rows_built": int(len(distinct)), "distinct_row_edges": int(deg[distinct].sum()),
                   "per_slot_formula": "sum over frontier slots of 8 + 4 d + 8 min(k, d)",
                   "per_slot_bytes": per_slot, "per_slot_frac": per_slot / ksec / HBM_PEAK}
-        kernel = "one batch: frontier_collect_kernel, the build kernels of the frontier rows, sample_hop_kernel (per hop)"
+        kernel = "one batch: frontier_collect_kernel, the fused kernels that build the frontier rows, sample_draw_kernel (per hop)"
     else:
         steps = sampled
         if args.n2v_table:
@@ -248,7 +248,7 @@ def online_bench(args, cfg, capi, g, seeds, name, cus, t_gen, torch):
             dp[:, 0] = 0
             alg_bytes = int(((12 + 8 * dc + 4 * dp) * mask).sum())
             detail = {"formula": "sum over steps of 12 + 8 d + 4 d_prev"}
-            kernel = "n2v_step_kernel (one launch per step)"
+            kernel = "walk_n2v_table_kernel (one launch)"
         else:
             alg_bytes = 12 * g.E + 5 * g.V + 24 * steps
             detail = {"formula": "12 E + 5 V (first-order tables) + 24 per step; the rejection trials' reads "

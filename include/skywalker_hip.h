@@ -247,19 +247,21 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      at most 64, at most 256 hops (SKY_ERR_LIMIT otherwise).
  *      "small_in_place" (default -1): 1 builds the rows of at most 32 entries in one kernel that walks the vertices
  *      in order and needs no row lists (it runs beside the binning pass and the kernels of the long rows); 0 builds
- *      them by degree class like all other rows; -1 takes the former for builds of at least 2^25 rows.  Same tables.
- *      "build_streams" (default 1): a build of 2 M .. 1 G entries without per-kernel timing sends the kernels of
- *      its degree classes out over the graph's stream and three side streams (small builds are bound by one
- *      kernel waiting for the one before); 0 keeps every kernel on the graph's stream.  Same tables.
+ *      them by degree class like all other rows; -1 takes the former for builds of at least 2^25 rows, and in the four
+ *      launches that make all of a build of up to 2^27 entries.  0 or 1 gives such a build its class kernels back.
+ *      Same tables.
+ *      "build_streams" (default 1): builds of up to 2^27 entries without per-kernel timing go out in four launches;
+ *      larger ones of up to 1 G entries (and smaller ones whose other knobs ask for class kernels) send the kernels of
+ *      their degree classes out over the graph's stream and three side streams (small builds are bound by one
+ *      kernel waiting for the one before); 0 keeps every class kernel on the graph's stream.  Same tables.
  *      "build_profile" (default 0): 1 records a HIP event after every kernel of sky_alias_build_all for
  *      sky_last_build_profile (about 3 microseconds each; a small graph pays 20 % of its build for them).
  *      "online_full_build" (default -1): how sky_walk_online serves a static bias on a graph without tables:
  *      0 builds the long rows that the walk is expected to draw from often and evaluates the draws from all others
  *      directly; 1 builds every row first and walks as sky_walk_offline does; -1 takes whichever is estimated to be
  *      faster.  The paths are the same.
- *      "online_device_sized" (default 1): sky_sample_online builds the
- *      rows of a frontier without the host ever learning how many they are: the sizes of
- *      its degree classes stay on the device, every build kernel finds its rows through them, and the call waits for
+ *      "online_device_sized" (default 1): sky_sample_online builds the rows of a frontier without the host ever
+ *      learning how many they are: the sizes of its degree classes stay on the device, every build kernel finds its rows through them, and the call waits for
  *      the device only once, at its end.  0 makes the host read the size of every frontier and size the launches
  *      exactly, which waits twice per hop.  Same results.
  *      "walk_compact_every" (default 0): k > 0 makes sky_walk_offline run k steps per launch and hand the next
