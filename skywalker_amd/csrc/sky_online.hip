@@ -174,7 +174,6 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
 // 256 slots are searched there together.  (A binary search per neighbour in the row in memory, 15 to 17 dependent loads,
 // in every pass, and a launch per step that waited for its slowest walker: 480 us a step for 2,000 walkers on the scale-18
 // graph, 1.1 M entries.)  What the search found stays in LDS, two bits per slot, for the passes that follow.
-constexpr uint32_t N2V_WIN = 1024;       // ids of the previous row in LDS, per wavefront
 constexpr uint32_t N2V_CODES = 65536;    // slots of a row whose result is kept
 constexpr uint32_t N2V_SPARSE = 32;      // previous row longer than the current one by this factor: searched in memory
 
@@ -191,6 +190,8 @@ __device__ __forceinline__ uint32_t wave_lower_bound(const uint32_t* __restrict_
   return lo + (uint32_t)__popcll(__ballot(lane < len && row[lo + lane] < key));
 }
 
+// WIN: ids of the previous row in LDS, per wavefront
+template <uint32_t WIN>
 struct N2vRow {
   static constexpr int U = 1;
   const float* w;
@@ -199,7 +200,7 @@ struct N2vRow {
   uint32_t d, pdeg, prev;
   bool has_prev;
   float p, q;
-  uint32_t* win;   // [N2V_WIN], this wavefront's own
+  uint32_t* win;   // [WIN], this wavefront's own
   uint8_t* codes;  // [N2V_CODES / 4]: per slot 0 neighbour of both, 1 the previous vertex, 2 neither
   uint32_t wpos, wlen;  // window: ids wpos .. wpos + wlen of the previous row
 
@@ -212,10 +213,10 @@ struct N2vRow {
   __device__ __forceinline__ void load_window(uint32_t from) {
     const uint32_t lane = threadIdx.x & 63;
     wpos = from;
-    wlen = min(N2V_WIN, pdeg - from);
-    uint4u x[N2V_WIN / 256];
+    wlen = min(WIN, pdeg - from);
+    uint4u x[WIN / 256];
 #pragma unroll
-    for (int j = 0; j < (int)(N2V_WIN / 256); ++j) {
+    for (int j = 0; j < (int)(WIN / 256); ++j) {
       const uint32_t k = 256u * j + 4u * lane;
       x[j] = uint4u{0, 0, 0, 0};
       if (k < wlen) x[j] = *reinterpret_cast<const uint4u*>(prow + from + k);
@@ -223,7 +224,7 @@ struct N2vRow {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // searches of the window before are done
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
-    for (int j = 0; j < (int)(N2V_WIN / 256); ++j) {
+    for (int j = 0; j < (int)(WIN / 256); ++j) {
       const uint32_t k = 256u * j + 4u * lane;
       win[k] = k < wlen ? x[j].x : 0xFFFFFFFFu;  // no vertex has this id
       win[k + 1] = k + 1 < wlen ? x[j].y : 0xFFFFFFFFu;
@@ -255,14 +256,14 @@ struct N2vRow {
       const uint32_t from = wpos + wlen;
       if (from < pdeg) {
         // a short way is one more window; a long one is searched
-        const uint32_t at = prow[min(from + N2V_WIN, pdeg) - 1] >= first ? from : wave_lower_bound(prow, from, pdeg, first);
+        const uint32_t at = prow[min(from + WIN, pdeg) - 1] >= first ? from : wave_lower_bound(prow, from, pdeg, first);
         if (at < pdeg) load_window(at);
         else { wpos = pdeg; wlen = 0; }
       }
     }
     while (wlen) {
       uint32_t steps = 1u;
-      while (steps < wlen) steps *= 2;  // wlen <= steps <= N2V_WIN; the places past wlen hold the largest id
+      while (steps < wlen) steps *= 2;  // wlen <= steps <= WIN; the places past wlen hold the largest id
       uint32_t at[4] = {0, 0, 0, 0};
       for (uint32_t h = steps / 2; h; h /= 2) {
         uint32_t x[4];
@@ -320,14 +321,14 @@ struct N2vRow {
   }
 };
 
-template <int T>
+template <int T, uint32_t WIN>
 __global__ __launch_bounds__(T) void walk_n2v_table_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
                                                            const float* __restrict__ wgt, const uint32_t* __restrict__ seeds,
                                                            uint32_t first, uint32_t V, uint32_t len, float p, float q,
                                                            float stop_prob, uint64_t seed, uint32_t* __restrict__ paths,
                                                            uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
   __shared__ DrawLds<T> lds;
-  __shared__ uint32_t s_win[T / 64][N2V_WIN];
+  __shared__ uint32_t s_win[T / 64][WIN];
   __shared__ uint8_t s_codes[N2V_CODES / 4];
   call_stamp(call);
   const uint32_t i = first + blockIdx.x;
@@ -339,7 +340,7 @@ __global__ __launch_bounds__(T) void walk_n2v_table_kernel(const uint32_t* __res
     if (stop_prob > 0.0f && u24(r.z) < stop_prob) break;
     const uint32_t off = xadj[v], d = xadj[v + 1] - off;
     if (d == 0) break;
-    N2vRow row;
+    N2vRow<WIN> row;
     row.w = wgt + off;
     row.nbr = adjncy + off;
     row.prow = adjncy + prev_off;
@@ -369,17 +370,21 @@ int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, 
   hipStream_t st = g->stream;
   CallDevice* call = nullptr;
   SKY_TRY(call_begin(g, &call));
-  // Four wavefronts per walker (42 KB of LDS, three walkers to a CU); eight while that leaves CUs without one.
-  constexpr uint32_t FEW = 512;
+  // Four wavefronts per walker, eight while that leaves CUs without one.  A window of 1024 ids per wavefront makes 37 KB
+  // of LDS, four walkers to a CU; more walkers than that get windows of 512, 29 KB, five to a CU, so that fewer of them
+  // wait for a CU (2,000 walkers x 40 steps on the scale-18 graph 872 -> 703 us; 900 walkers on the scale-17 graph 538
+  // with 1024 ids, 555 with 512).  Less LDS still, by fewer slots whose result is kept or smaller windows, was slower.
+  constexpr uint32_t FEW = 512, RESIDENT = 1024;
   const uint32_t most = 0xFFFFFFFFu / 512;  // walkers of one launch: below 2^32 threads
   for (uint32_t f = 0; f < N; f += std::min(most, N - f)) {
     const dim3 grid(std::min(most, N - f));
-    if (N <= FEW)
-      hipLaunchKernelGGL(walk_n2v_table_kernel<512>, grid, dim3(512), 0, st, g->xadj, g->adjncy, g->adjwgt, seeds, f, g->V, len, p, q,
-                         stop_prob, seed, paths, lengths, call);
-    else
-      hipLaunchKernelGGL(walk_n2v_table_kernel<256>, grid, dim3(256), 0, st, g->xadj, g->adjncy, g->adjwgt, seeds, f, g->V, len, p, q,
-                         stop_prob, seed, paths, lengths, call);
+    auto go = [&](auto kernel, uint32_t threads) {
+      hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, st, g->xadj, g->adjncy, g->adjwgt, seeds, f, g->V, len, p, q, stop_prob,
+                         seed, paths, lengths, call);
+    };
+    if (N <= FEW) go(walk_n2v_table_kernel<512, 1024>, 512);
+    else if (N <= RESIDENT) go(walk_n2v_table_kernel<256, 1024>, 256);
+    else go(walk_n2v_table_kernel<256, 512>, 256);
     call = nullptr;
   }
   return call_end(g, sampled, seconds, lengths, N);

@@ -380,10 +380,10 @@ def test_online_static_draws_evaluated_from_the_weights(orc, walkers, dist):
     g.free()
 
 
-@pytest.mark.parametrize("walkers", [512, 513])
+@pytest.mark.parametrize("walkers", [512, 513, 1025])
 def test_node2vec_table_rows_beyond_the_window(orc, walkers):
-    # eight and four wavefronts per walker; rows of more than 65,536 entries (membership is searched again instead of kept),
-    # previous rows of many windows of 1024 ids, and of more than 32 times the current row's length
+    # eight and four wavefronts per walker, windows of 1024 and 512 ids; rows of more than 65,536 entries (membership is searched again instead of kept),
+    # previous rows of many windows, and of more than 32 times the current row's length
     from skywalker_amd import capi
     rng = np.random.default_rng(46)
     degs = list(rng.integers(0, 300, 1500)) + list(rng.integers(900, 4200, 250)) + [1023, 1024, 1025] * 30 + \
