@@ -506,7 +506,15 @@ int ensure_plan(sky_graph* g) {
     // way; other builds, and those of small frontiers, make them tile by tile, for which they need geometry.  A graph
     // with very many of them does without: 65536 tiles that a frontier may have to pass over take 20 us a launch.
     const uint64_t narrow = g->bin_edges[CLS_STREAM] + g->bin_edges[CLS_STREAM_LAST];
-    p.t_all = (long long)narrow <= narrow_limit ? CLS_STREAM : CLS_STREAM_WIDE;
+    // A workgroup takes 2.4 ns an entry for such a row, and the launch lasts at least as long as the longest of them.
+    // The launch of the rows of 2558..65533 entries as a whole takes 6 ps an entry, the tile passes 13 ps (one
+    // MI355X; this tells the faster way for 13 of 13 graphs of 4 to 117 M entries: 40 M entries in rows of 1..300,000
+    // 409 -> 367 us by tiles, R-MAT scale 22 edge factor 28 754 us streamed, 888 by tiles).
+    uint64_t wide = narrow + g->bin_edges[CLS_HOLD];
+    for (int c = CLS_MW2 + 4; c <= CLS_MW2 + MERGE_MAX_NW - 2; ++c) wide += g->bin_edges[c];
+    const uint32_t longest = std::min(g->max_degree, g->bin_counts[CLS_STREAM] ? 65533u : 24576u);
+    const double stream_us = std::max(longest * 2.4e-3, wide * 6e-6), tiles_us = (wide - narrow) * 6e-6 + narrow * 13e-6;
+    p.t_all = (long long)narrow <= narrow_limit || (narrow_limit > 0 && tiles_us < stream_us) ? CLS_STREAM : CLS_STREAM_WIDE;
     p.t_first = p.t_all == CLS_STREAM || narrow <= 65536ull * TILE ? CLS_STREAM : CLS_STREAM_WIDE;
     uint64_t edges = 0;
     for (int c = p.t_first; c <= CLS_HUGE; ++c) {
