@@ -271,8 +271,11 @@ __device__ __forceinline__ void merge_unit(const FusedArgs& a, const SectionRef&
 constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
 constexpr size_t WAVE_LDS = cmax(cmax(SMALL_LDS_BYTES, 2 * 64 * 6 * 8 + 64 * 6), merge_lds_bytes(64, 8));
 
+// The second launch bounds: what LDS lets reside anyway (21 wavefronts, 10 pairs, 4 workgroups of 256 to a CU).  Left alone the
+// device-sized kernels took 109, 104 and 132 registers, one workgroup in five and one in four less (the 134,652 rows of a
+// 40,000-seed batch's second hop on the scale-22 graph: 79, 91 and 133 us, with the bounds 63, 70 and 81).
 template <bool DEV>
-__global__ __launch_bounds__(64) void fused_wave_kernel(FusedArgs a) {
+__global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
   __shared__ uint64_t smem[(WAVE_LDS + 7) / 8];
   __shared__ uint64_t s_aux[8];
   call_stamp(a.call);
@@ -311,7 +314,7 @@ __global__ __launch_bounds__(64) void fused_wave_kernel(FusedArgs a) {
 }
 
 template <bool DEV>
-__global__ __launch_bounds__(128) void fused_pair_kernel(FusedArgs a) {
+__global__ __launch_bounds__(128, 5) void fused_pair_kernel(FusedArgs a) {
   __shared__ uint64_t smem[(merge_lds_bytes(128, 8) + 7) / 8];
   __shared__ uint64_t s_aux[16];
   call_stamp(a.call);
@@ -376,7 +379,7 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
 }
 
 template <bool DEV>
-__global__ __launch_bounds__(256) void fused_block_kernel(FusedArgs a) {
+__global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[(cmax(merge_lds_bytes(256, 10), sizeof(TileEmitLds)) + 7) / 8];
   __shared__ uint64_t s_aux[32];
   call_stamp(a.call);
