@@ -381,6 +381,11 @@ struct SampleSession {
       SKY_TRY(ensure_table_storage(g));
       if (dev_sized) {
         SKY_TRY(ensure_plan(g));
+        // room for the largest hop's rows from the start: growing it at a later hop would free and allocate with that
+        // hop's predecessor running (first call on a graph, 40,000 seeds: 1.80 -> 1.45 ms)
+        uint64_t most = 0;
+        for (uint32_t h = 0; h + 1 < hops; ++h) most = std::max(most, (uint64_t)N * width[h]);
+        SKY_TRY(frontier_lists(g, (uint32_t)std::min<uint64_t>(most, g->V), &front));
         SKY_TRY(pool_get(g, sky_graph::POOL_FRONT, (size_t)(hops - 1) * FRONTIER_WORDS * 4, (void**)&front_counts));
         ++g->frontier_epoch;
       } else {
