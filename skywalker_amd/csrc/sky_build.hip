@@ -1036,14 +1036,19 @@ int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start) 
   return SKY_OK;
 }
 
-// Largest build that goes out in the four launches of sky_build_fused.hip.
-constexpr uint64_t FUSED_MAX_ENTRIES = 1ull << 27;
+// Builds that go out in the four launches of sky_build_fused.hip: up to 2^27 entries, or up to 2^28 in at most 2^23 rows.
+// Above, a class fills the GPU by itself, and short rows beside the others in a kernel of their own are worth
+// more than fewer launches (four launches / by class, us: scale 23 with 31 edges a vertex 1418 / 1534, scale 22 with 50
+// 1151 / 1207; scale 23 with 56 2896 / 2699, scale 24 with 16 1575 / 1585, scale 25 with 15 3096 / 3065).
+constexpr uint64_t FUSED_MAX_ENTRIES = 1ull << 27, FUSED_MAX_ENTRIES_FEW_ROWS = 1ull << 28;
+constexpr uint32_t FUSED_FEW_ROWS = 1u << 23;
 
 int build_all_tables(sky_graph* g, double* seconds) {
   SKY_TRY(ensure_table_storage(g));
   // Knobs that name kernels of their own, and per-kernel timing, want the class kernels.
   const bool fused = fused_possible(g) && !option(g, OPT_BUILD_PROFILE) && option(g, OPT_SMALL_IN_PLACE) < 0 &&
-                     option(g, OPT_BUILD_STREAMS) != 0 && g->E <= FUSED_MAX_ENTRIES && g->V;
+                     option(g, OPT_BUILD_STREAMS) != 0 && g->V &&
+                     g->E <= (g->V <= FUSED_FEW_ROWS ? FUSED_MAX_ENTRIES_FEW_ROWS : FUSED_MAX_ENTRIES);
   if (fused) {
     SKY_TRY(ensure_plan(g));
     CallDevice* call = nullptr;

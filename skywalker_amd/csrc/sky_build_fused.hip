@@ -1,4 +1,4 @@
-// Builds whose launches, not their entries, would bound them: everything from a graph of a thousand edges up to FUSED_MAX_ENTRIES, and
+// Builds whose launches, not their entries, would bound them: from a graph of a thousand edges up to FUSED_MAX_ENTRIES, and
 // the rows of a frontier.
 //
 // The class kernels of sky_build.hip give every degree class a launch of its own.  That is right where a class fills
