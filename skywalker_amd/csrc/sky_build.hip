@@ -776,8 +776,27 @@ int prepare_build_scratch(sky_graph* g, uint32_t max_rows) {
   return SKY_OK;
 }
 
+// Builds that go out in the four launches of sky_build_fused.hip: up to 2^27 entries, or up to 2^28 in at most 2^23 rows.
+// Above, a class fills the GPU by itself, and short rows beside the others in a kernel of their own are worth
+// more than fewer launches (four launches / by class, us: scale 23 with 31 edges a vertex 1418 / 1534, scale 22 with 50
+// 1151 / 1207; scale 23 with 56 2896 / 2699, scale 24 with 16 1575 / 1585, scale 25 with 15 3096 / 3065).
+constexpr uint64_t FUSED_MAX_ENTRIES = 1ull << 27, FUSED_MAX_ENTRIES_FEW_ROWS = 1ull << 28;
+constexpr uint32_t FUSED_FEW_ROWS = 1u << 23;
+
+// Whether a build leaves its rows of at most 32 entries to small_rows_kernel, which builds them where they lie,
+// without lists.  Taken alone it is slower than the class kernels of these rows (1.39 against 1.12 ms on the
+// scale-26 graph), but it depends on no list: on a side stream it runs beside the kernels of the long rows (it waits on
+// memory, they on the vector ALU).  A build of all vertices then needs no binning either: the lists of the longer rows
+// are in the graph's plan.  Every build of all vertices that is too large for four launches gains by that (R-MAT
+// lognormal, by class / in place, us: scale 24 with 16 edges a vertex 1613 / 1535, with 56 5172 / 4888, scale 23 with 40
+// 2069 / 1928, scale 22 with 66 1772 / 1668); a list of vertices has to be binned, and takes it from 2^25 rows on.
+static bool small_rows_in_place(const sky_graph* g, const uint32_t* src, uint32_t n) {
+  const long long sip = option(g, OPT_SMALL_IN_PLACE);
+  return sip < 0 ? n >= (1u << 25) || (src == nullptr && n == g->V && g->E > FUSED_MAX_ENTRIES) : sip != 0;
+}
+
 // Builds the rows listed in `src` (device array of n vertex ids; null = vertices 0..n-1).
-// prepare_build_scratch(n) and ensure_table_storage must have been called.
+// prepare_build_scratch(n) (not needed for a build of all vertices with small_rows_in_place) and ensure_table_storage must have been called.
 int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, CallDevice* call) {
   hipStream_t st = g->stream;
   g->has_walk_index = false;  // the table entries it was made from are about to change
@@ -788,13 +807,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     unsigned long long edges[CLS_COUNT];
   } host = {};
   static_assert(sizeof(host) == COUNTER_BYTES, "counter block layout");
-  // A large build leaves its rows of at most 32 entries to small_rows_kernel, which builds them where they lie,
-  // without lists.  Taken alone it is slower than the class kernels of these rows (1.39 against 1.12 ms on the
-  // scale-26 graph), but it does not depend on the binning pass: on a side stream it runs beside the binning and
-  // the kernels of the long rows (it waits on memory, they on the vector ALU): 10.2 -> 9.95 ms for the whole build.
-  // Smaller builds, whose class kernels already overlap, gain nothing (scale 24: 3 % slower).
-  const long long sip = option(g, OPT_SMALL_IN_PLACE);
-  const bool small_in_place = sip < 0 ? n >= (1u << 25) : sip != 0;
+  const bool small_in_place = small_rows_in_place(g, src, n);
   const int listed_from = small_in_place ? CLS_G16 : CLS_G2;
   StreamFan fan(g, st);
   auto launch_small = [&](hipStream_t s) {
@@ -1036,13 +1049,6 @@ int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start) 
   return SKY_OK;
 }
 
-// Builds that go out in the four launches of sky_build_fused.hip: up to 2^27 entries, or up to 2^28 in at most 2^23 rows.
-// Above, a class fills the GPU by itself, and short rows beside the others in a kernel of their own are worth
-// more than fewer launches (four launches / by class, us: scale 23 with 31 edges a vertex 1418 / 1534, scale 22 with 50
-// 1151 / 1207; scale 23 with 56 2896 / 2699, scale 24 with 16 1575 / 1585, scale 25 with 15 3096 / 3065).
-constexpr uint64_t FUSED_MAX_ENTRIES = 1ull << 27, FUSED_MAX_ENTRIES_FEW_ROWS = 1ull << 28;
-constexpr uint32_t FUSED_FEW_ROWS = 1u << 23;
-
 int build_all_tables(sky_graph* g, double* seconds) {
   SKY_TRY(ensure_table_storage(g));
   // Knobs that name kernels of their own, and per-kernel timing, want the class kernels.
@@ -1061,7 +1067,7 @@ int build_all_tables(sky_graph* g, double* seconds) {
     g->has_tables = true;
     return SKY_OK;
   }
-  SKY_TRY(prepare_build_scratch(g, g->V));
+  SKY_TRY(prepare_build_scratch(g, small_rows_in_place(g, nullptr, g->V) ? 0 : g->V));
   if (option(g, OPT_BUILD_PROFILE)) {
     EventTimer tm(g->stream);
     SKY_TRY(tm.mark("start", 0));
