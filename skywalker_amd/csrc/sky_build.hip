@@ -776,12 +776,11 @@ int prepare_build_scratch(sky_graph* g, uint32_t max_rows) {
   return SKY_OK;
 }
 
-// Builds that go out in the four launches of sky_build_fused.hip: up to 2^27 entries, or up to 2^28 in at most 2^23 rows.
-// Above, a class fills the GPU by itself, and short rows beside the others in a kernel of their own are worth
-// more than fewer launches (four launches / by class, us: scale 23 with 31 edges a vertex 1418 / 1534, scale 22 with 50
-// 1151 / 1207; scale 23 with 56 2896 / 2699, scale 24 with 16 1575 / 1585, scale 25 with 15 3096 / 3065).
-constexpr uint64_t FUSED_MAX_ENTRIES = 1ull << 27, FUSED_MAX_ENTRIES_FEW_ROWS = 1ull << 28;
-constexpr uint32_t FUSED_FEW_ROWS = 1u << 23;
+// Largest build that goes out in the four launches of sky_build_fused.hip.  Above, a class fills the GPU by itself, and short
+// rows beside the others in a kernel of their own are worth more than fewer launches.  (Four launches / by class, us:
+// scale 20 with 120 edges a vertex 799 / 829, scale 23 with 10 585 / 608, scale 24 with 7 868 / 877, scale 22 with 20
+// 588 / 564; scale 22 with 36 911 / 846, scale 24 with 9 1071 / 1045, with 16 1631 / 1534, scale 23 with 31 1433 / 1438.)
+constexpr uint64_t FUSED_MAX_ENTRIES = 1ull << 27;
 
 // Whether a build leaves its rows of at most 32 entries to small_rows_kernel, which builds them where they lie,
 // without lists.  Taken alone it is slower than the class kernels of these rows (1.39 against 1.12 ms on the
@@ -1053,8 +1052,7 @@ int build_all_tables(sky_graph* g, double* seconds) {
   SKY_TRY(ensure_table_storage(g));
   // Knobs that name kernels of their own, and per-kernel timing, want the class kernels.
   const bool fused = fused_possible(g) && !option(g, OPT_BUILD_PROFILE) && option(g, OPT_SMALL_IN_PLACE) < 0 &&
-                     option(g, OPT_BUILD_STREAMS) != 0 && g->V &&
-                     g->E <= (g->V <= FUSED_FEW_ROWS ? FUSED_MAX_ENTRIES_FEW_ROWS : FUSED_MAX_ENTRIES);
+                     option(g, OPT_BUILD_STREAMS) != 0 && g->E <= FUSED_MAX_ENTRIES && g->V;
   if (fused) {
     SKY_TRY(ensure_plan(g));
     CallDevice* call = nullptr;
