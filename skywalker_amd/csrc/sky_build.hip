@@ -644,10 +644,10 @@ void pool_release(sky_graph* g) {
   g->fork_ev = nullptr;
 }
 
-// The class kernels of one build are independent of one another once the binning pass has run.  A small build is
-// bound by launching them one after another (a class of a few hundred rows takes as long as one row), so it sends
-// them out in turn over the graph's stream and three side streams; the graph's stream waits for the others at
-// the end.  Not used when every kernel is timed on its own, nor for builds so large that each kernel fills the GPU.
+// The class kernels of one build are independent of one another once their lists are there.  A build of up to 1 G entries
+// sends them out over the graph's stream and three side streams (a class of few rows takes as long as one row, and
+// the tail of one kernel is filled by another); the graph's stream waits for the others at the end.  Not used when
+// every kernel is timed on its own.
 constexpr uint64_t FAN_MIN_EDGES = 2000000, FAN_MAX_EDGES = 1ull << 30;
 struct StreamFan {
   sky_graph* g;
