@@ -614,16 +614,18 @@ void free_build_scratch(sky_graph* g) {
   g->build_scratch = nullptr;
 }
 
+int buf_grow(sky_graph::PoolBuf* b, size_t bytes) {
+  if (b->cap >= bytes && b->p) return SKY_OK;
+  if (b->p) SKY_HIP(hipFree(b->p));
+  b->p = nullptr;
+  b->cap = 0;
+  SKY_HIP(hipMalloc(&b->p, bytes + 16));
+  b->cap = bytes;
+  return SKY_OK;
+}
 int pool_get(sky_graph* g, int slot, size_t bytes, void** out) {
-  sky_graph::PoolBuf& b = g->pool[slot];
-  if (b.cap < bytes) {
-    if (b.p) SKY_HIP(hipFree(b.p));
-    b.p = nullptr;
-    b.cap = 0;
-    SKY_HIP(hipMalloc(&b.p, bytes + 16));
-    b.cap = bytes;
-  }
-  *out = b.p;
+  SKY_TRY(buf_grow(&g->pool[slot], bytes));
+  *out = g->pool[slot].p;
   return SKY_OK;
 }
 void pool_release(sky_graph* g) {

@@ -486,7 +486,7 @@ int alloc(void** p, size_t bytes) {
 
 void free_plan(sky_graph* g) {
   if (!g->plan) return;
-  void* ptrs[] = {g->plan->rows, g->plan->trows, g->plan->tiles, g->plan->front};
+  void* ptrs[] = {g->plan->rows, g->plan->trows, g->plan->tiles};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete g->plan;
@@ -499,6 +499,7 @@ int ensure_plan(sky_graph* g) {
   free_plan(g);
   hipStream_t st = g->stream;
   g->plan = new BuildPlan();
+  ++g->plan_serial;
   BuildPlan& p = *g->plan;
   auto body = [&]() -> int {
     SKY_TRY(bin_all_rows(g, CLS_G16, &p.rows, p.start));
@@ -679,9 +680,9 @@ int build_all_fused(sky_graph* g, CallDevice* call) { return build_host_sized(g,
 int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call) { return build_host_sized(g, min_degree, call); }
 
 // ---------------------------------------------------------------- rows of a frontier
-int frontier_lists(sky_graph* g, uint32_t n_upper, FrontierLists* f) {
+int frontier_lists(sky_graph* g, uint32_t n_upper, sky_graph::PoolBuf* buf, FrontierLists* f) {
   SKY_TRY(ensure_plan(g));
-  BuildPlan& p = *g->plan;
+  const BuildPlan& p = *g->plan;
   // A workgroup needs 125 us to stream a row of 65,000 entries, which is as long as everything else that the build of a
   // small frontier does; the rows of a large one keep all workgroups streaming, and that is cheaper by the entry.
   f->tiled_from = n_upper <= SMALL_FRONTIER ? p.t_first : p.t_all;
@@ -690,21 +691,18 @@ int frontier_lists(sky_graph* g, uint32_t n_upper, FrontierLists* f) {
     f->start[c] = (uint32_t)at;
     const bool tiled = c >= f->tiled_from && c <= CLS_HUGE;
     const uint64_t in_graph = c == CLS_TINY ? g->bin_edges[c] : g->bin_counts[c];  // a tiny row has an entry at least
-    p.front_cap[c] = c == CLS_EMPTY || tiled ? 0u : (uint32_t)std::min<uint64_t>(n_upper, in_graph);
-    at += p.front_cap[c];
+    f->cap[c] = c == CLS_EMPTY || tiled ? 0u : (uint32_t)std::min<uint64_t>(n_upper, in_graph);
+    at += f->cap[c];
   }
-  if (p.front_rows < at) {
-    if (p.front) SKY_HIP(hipFree(p.front));
-    p.front = nullptr;
-    p.front_rows = 0;
-    SKY_TRY(alloc((void**)&p.front, at * sizeof(RowRef)));
-    p.front_rows = at;
-  }
-  f->list = p.front;
+  f->plan_serial = g->plan_serial;
+  SKY_TRY(buf_grow(buf, at * sizeof(RowRef)));
+  f->list = (RowRef*)buf->p;
   return SKY_OK;
 }
 
 int build_frontier(sky_graph* g, const FrontierLists& f, const uint32_t* counts, const uint32_t* bitmap, uint32_t epoch) {
+  if (!g->plan || f.plan_serial != g->plan_serial)
+    return fail(SKY_ERR_STATE, "a knob that decides how long rows are built was changed between a frontier and its build");
   g->has_walk_index = false;
   const BuildPlan& p = *g->plan;
   FusedArgs base = common_args(g, f.tiled_from);
@@ -716,7 +714,7 @@ int build_frontier(sky_graph* g, const FrontierLists& f, const uint32_t* counts,
   Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
   auto add = [&](Launch& l, Section k, uint32_t per, int cls, int ncls = 1) {
     uint32_t upper = 0;
-    for (int c = 0; c < ncls; ++c) upper += p.front_cap[cls + c];
+    for (int c = 0; c < ncls; ++c) upper += f.cap[cls + c];
     l.add_dev(k, upper, per, f.start[cls], cls, ncls, ncls > 1 ? f.start[cls + 1] - f.start[cls] : 0u);
   };
   wave.add(SEC_SUM, n_tiles, 1, 0);

@@ -33,6 +33,7 @@ struct sky_graph {
   // scratch memory of the table builds on this graph (allocated on first use, reused by every later build, freed
   // with the graph): row lists and counters of the binning pass, and the arrays of the tile-parallel path
   sky::BuildPlan* plan = nullptr;  // sky_build_fused.h
+  uint32_t plan_serial = 0;        // plans made so far
   uint32_t frontier_epoch = 0;     // calls that have built frontiers
   void* build_scratch = nullptr;
   void* tiled_scratch = nullptr;
@@ -70,12 +71,13 @@ struct sky_graph {
   bool call_dirty = false;  // a call has begun and not ended well: its device words may not be zero
 
   // Device buffers that calls on this graph reuse instead of allocating each time (they only grow).
-  enum PoolSlot { POOL_BITMAP = 0, POOL_LIST, POOL_TOTALS, POOL_FRONT, POOL_SLOTS };
+  enum PoolSlot { POOL_WALK_LIST = 0, POOL_WALK_COUNTS, POOL_BITMAP, POOL_LIST, POOL_TOTALS, POOL_FRONT, POOL_SEGMENTS, POOL_SLOTS };
   struct PoolBuf {
     void* p = nullptr;
     size_t cap = 0;
   };
   PoolBuf pool[POOL_SLOTS];
+  bool sampler_busy = false;  // a sampling session holds the slots from POOL_BITMAP on; other calls bring their own
   // Side streams (default priority) over which a small build spreads its class kernels, the event they wait for
   // and the events the graph's stream waits for afterwards; created on first use.
   static constexpr int SIDE_STREAMS = 3;
@@ -196,6 +198,7 @@ struct EventTimer {
 
 // A device buffer of at least `bytes` bytes that belongs to the graph; its contents do not survive a larger request.
 int pool_get(sky_graph* g, int slot, size_t bytes, void** out);
+int buf_grow(sky_graph::PoolBuf* b, size_t bytes);
 void pool_release(sky_graph* g);
 int ensure_table_storage(sky_graph* g);
 int prepare_build_scratch(sky_graph* g, uint32_t max_rows);

@@ -321,9 +321,29 @@ struct SampleSession {
   FrontierLists front;
   bool want_list = false;        // the caller is to see the frontier as a list of vertices
   uint32_t* totals = nullptr;    // children of each start vertex, when the kernels add them up
+  uint32_t epoch = 0;            // this call's number, by which rows made tile by tile tell that it has built them
   uint32_t frontier_upper = 0;   // most rows the last frontier can hold
   uint32_t frontier_count = 0;   // its size, when the host has read it (dev_sized false)
-  explicit SampleSession(sky_graph* g_) : g(g_) {}
+  // A session keeps its buffers while other calls, other sessions among them, use the same graph: the first to come holds
+  // those of the graph, the others have their own.
+  bool holds_pool = false;
+  sky_graph::PoolBuf own[sky_graph::POOL_SLOTS];
+  explicit SampleSession(sky_graph* g_) : g(g_) {
+    holds_pool = !g->sampler_busy;
+    g->sampler_busy = true;
+  }
+  SampleSession(const SampleSession&) = delete;
+  ~SampleSession() {
+    if (holds_pool) g->sampler_busy = false;
+    for (auto& b : own)
+      if (b.p) (void)hipFree(b.p);
+  }
+  sky_graph::PoolBuf* buffer(int slot) { return holds_pool ? &g->pool[slot] : &own[slot]; }
+  int get(int slot, size_t bytes, void** out) {
+    SKY_TRY(buf_grow(buffer(slot), bytes));
+    *out = buffer(slot)->p;
+    return SKY_OK;
+  }
 
   HopGeom geom(uint32_t h) const {
     HopGeom hg;
@@ -385,18 +405,18 @@ struct SampleSession {
         // hop's predecessor running (first call on a graph, 40,000 seeds: 1.80 -> 1.45 ms)
         uint64_t most = 0;
         for (uint32_t h = 0; h + 1 < hops; ++h) most = std::max(most, (uint64_t)N * width[h]);
-        SKY_TRY(frontier_lists(g, (uint32_t)std::min<uint64_t>(most, g->V), &front));
-        SKY_TRY(pool_get(g, sky_graph::POOL_FRONT, (size_t)(hops - 1) * FRONTIER_WORDS * 4, (void**)&front_counts));
-        ++g->frontier_epoch;
+        SKY_TRY(frontier_lists(g, (uint32_t)std::min<uint64_t>(most, g->V), buffer(sky_graph::POOL_SEGMENTS), &front));
+        SKY_TRY(get(sky_graph::POOL_FRONT, (size_t)(hops - 1) * FRONTIER_WORDS * 4, (void**)&front_counts));
+        epoch = ++g->frontier_epoch;
       } else {
         SKY_TRY(prepare_build_scratch(g, g->V));
       }
-      SKY_TRY(pool_get(g, sky_graph::POOL_BITMAP, (size_t)words * 4, (void**)&bitmap));
-      if (want_list || !dev_sized) SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)g->V * 4, (void**)&list));
+      SKY_TRY(get(sky_graph::POOL_BITMAP, (size_t)words * 4, (void**)&bitmap));
+      if (want_list || !dev_sized) SKY_TRY(get(sky_graph::POOL_LIST, (size_t)g->V * 4, (void**)&list));
     }
     SKY_TRY(call_begin(g, &call));
     d_count = call->count;
-    if (N && one_workgroup()) SKY_TRY(pool_get(g, sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
+    if (N && one_workgroup()) SKY_TRY(get(sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
     if (online)
       hipLaunchKernelGGL(sample_init_kernel, dim3(std::min((std::max(N, words) + 255) / 256, 2048u)), dim3(256), 0, st, seeds, N,
                          lps, data, bitmap, words, front_counts, dev_sized ? (hops - 1) * FRONTIER_WORDS : 0u, call);
@@ -413,7 +433,7 @@ struct SampleSession {
     const uint64_t slots = (uint64_t)N * hg.width;
     frontier_upper = (uint32_t)std::min<uint64_t>(slots, g->V);
     d_count = call->count + h;
-    if (dev_sized) SKY_TRY(frontier_lists(g, frontier_upper, &front));
+    if (dev_sized) SKY_TRY(frontier_lists(g, frontier_upper, buffer(sky_graph::POOL_SEGMENTS), &front));
     hipLaunchKernelGGL(frontier_collect_kernel, dim3((uint32_t)((slots + COLLECT_T - 1) / COLLECT_T)), dim3(COLLECT_T), 0, st,
                        data, sample_lengths, slots, g->V, hg, bitmap, g->xadj, g->valid, front,
                        dev_sized ? front_counts + h * FRONTIER_WORDS : nullptr, list, d_count);
@@ -431,7 +451,7 @@ struct SampleSession {
     if (!online || !N || !frontier_upper) return SKY_OK;
     float* const own = g->adjwgt;
     if (weights) g->adjwgt = const_cast<float*>(weights);  // the build only reads it
-    const int rc = dev_sized ? build_frontier(g, front, front_counts + h * FRONTIER_WORDS, bitmap, g->frontier_epoch)
+    const int rc = dev_sized ? build_frontier(g, front, front_counts + h * FRONTIER_WORDS, bitmap, epoch)
                              : build_rows(g, list, frontier_count, nullptr);
     g->adjwgt = own;
     return rc;

@@ -192,8 +192,8 @@ int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, 
   const uint32_t nseg = segmented ? (len + every - 1) / every : 1;
   uint32_t *lists = nullptr, *counts = nullptr;
   if (segmented) {  // two lists of walker numbers used in turn, one survivor count per segment
-    SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)2 * N * 4, (void**)&lists));
-    SKY_TRY(pool_get(g, sky_graph::POOL_BITMAP, (size_t)(nseg + 1) * 4, (void**)&counts));
+    SKY_TRY(pool_get(g, sky_graph::POOL_WALK_LIST, (size_t)2 * N * 4, (void**)&lists));
+    SKY_TRY(pool_get(g, sky_graph::POOL_WALK_COUNTS, (size_t)(nseg + 1) * 4, (void**)&counts));
     SKY_HIP(hipMemsetAsync(counts, 0, (size_t)(nseg + 1) * 4, st));
   }
   auto run = [&](auto... a) {
@@ -277,7 +277,7 @@ int build_walk_index(sky_graph* g, double* seconds) {
   if (g->E == 0) return SKY_OK;
   const uint32_t ntiles = (g->E + IDX_TILE - 1) / IDX_TILE;
   uint32_t* row_of_tile = nullptr;
-  SKY_TRY(pool_get(g, sky_graph::POOL_LIST, (size_t)ntiles * 4, (void**)&row_of_tile));
+  SKY_TRY(pool_get(g, sky_graph::POOL_WALK_LIST, (size_t)ntiles * 4, (void**)&row_of_tile));
   CallDevice* call = nullptr;
   SKY_TRY(call_begin(g, &call));
   hipLaunchKernelGGL(index_tile_rows_kernel, dim3((g->V + 255) / 256), dim3(256), 0, st, g->xadj, g->V, row_of_tile, call);

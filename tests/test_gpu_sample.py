@@ -240,3 +240,45 @@ def test_batches_by_workgroup_and_by_hop(orc, n, fanout, distinct):
         assert np.array_equal(sl.to_host((n, slen)), want[1]) and np.array_equal(data.to_host((n, lps)), want[0])
         assert sampled == want[2]
     g.free()
+
+
+def test_other_calls_between_the_steps_of_a_session(orc):
+    # a larger batch with more hops, and a second session, on the same graph between the steps: buffers of the first
+    # session neither move nor change
+    import ctypes as C
+    from helpers import graph_from_degrees
+    from skywalker_amd import capi
+    rng = np.random.default_rng(79)
+    degs = list(rng.integers(0, 60, 3000)) + [300, 700, 3000, 6000, 9000, 70001] * 3
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal")
+    V = len(xadj) - 1
+    g = capi.Graph.upload(xadj, adjncy, w)
+    L, fan = capi.lib(), np.array([1, 5, 4, 2], np.uint32)
+    lps, slen = capi.sample_layout(fan)
+    sessions = []
+    for n in (40, 900):
+        seeds = rng.integers(0, V, n).astype(np.uint32)
+        seeds_d = capi.DeviceArray.from_host(seeds)
+        data, sl = capi.DeviceArray(n * lps, np.uint32, fill=0xFFFFFFFF), capi.DeviceArray(n * slen, np.uint32, fill=0)
+        sess = C.c_void_p()
+        assert L.sky_sample_session_begin(g.h, seeds_d.ptr, C.c_uint32(n), fan.ctypes.data_as(C.c_void_p), C.c_uint32(len(fan)),
+                                          C.c_uint64(41), data.ptr, sl.ptr, C.byref(sess)) == 0
+        sessions.append((n, seeds, seeds_d, data, sl, sess))
+    big = rng.integers(0, V, 20000).astype(np.uint32)
+    for hop in range(3):
+        for _, _, _, _, _, sess in sessions:
+            lst, cnt, upper = C.c_void_p(), C.c_void_p(), C.c_uint32()
+            assert L.sky_sample_session_frontier(sess, C.c_uint32(hop), C.byref(lst), C.byref(cnt), C.byref(upper)) == 0
+        got = g.sample_online(big[:20000 >> (2 * (2 - hop))], [1, 3, 2, 2, 2], 43)
+        want = orc.sample_online(xadj, adjncy, w, big[:20000 >> (2 * (2 - hop))], [1, 3, 2, 2, 2], 43)
+        assert np.array_equal(got[0].to_host(want[0].shape), want[0]) and got[2] == want[2]
+        for _, _, _, _, _, sess in sessions:
+            assert L.sky_sample_session_hop(sess, C.c_uint32(hop), None) == 0
+    for n, seeds, _, data, sl, sess in sessions:
+        sampled, sec = C.c_uint64(), C.c_double()
+        assert L.sky_sample_session_end(sess, C.byref(sampled), C.byref(sec)) == 0
+        want = orc.sample_online(xadj, adjncy, w, seeds, fan, 41)
+        assert np.array_equal(data.to_host((n, lps)), want[0]) and np.array_equal(sl.to_host((n, slen)), want[1])
+        assert sampled.value == want[2]
+    g.free()
