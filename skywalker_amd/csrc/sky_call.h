@@ -14,7 +14,7 @@ namespace sky {
 struct CallDevice {
   unsigned long long start;    // wall clock of the first kernel
   unsigned long long sampled;  // edges sampled so far
-  uint32_t count[12];          // counters of the call's kernels
+  unsigned long long pad[6];
 };
 // Pinned host words of a call, written by the end kernel.
 struct CallHost {
@@ -23,6 +23,15 @@ struct CallHost {
   unsigned long long pad[5];
 };
 static_assert(sizeof(CallDevice) == 64 && sizeof(CallHost) == 64, "one cache line each");
+// Where a call reports.  A graph has one for the calls that begin and end within one entry point; a call that stays open
+// between entry points (a sampling session) has its own, because other calls on the graph begin and end meanwhile.
+struct CallWords {
+  CallDevice* dev = nullptr;
+  CallHost* host = nullptr;
+  unsigned long long seq = 0;
+  int khz = 0;
+  bool dirty = false;  // a call has begun and not ended well: its device words may not be zero
+};
 
 // The call's first kernel: its first thread notes when it began.
 __device__ __forceinline__ void call_stamp(CallDevice* call) {
@@ -35,16 +44,17 @@ __device__ __forceinline__ void call_report(CallDevice* call, CallHost* host, un
   host->ticks = call->start ? wall_clock64() - call->start : 0;  // 0: the call had nothing to launch
   call->start = 0;
   call->sampled = 0;
-#pragma unroll
-  for (int k = 0; k < 12; ++k) call->count[k] = 0;
   __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// The graph's call words, cleared; a call that ended in an error may have left something in them.
-int call_begin(sky_graph* g, CallDevice** call);
+// The device words of `w` (taken on first use), cleared; a call that ended in an error may have left something in them.
+int call_begin(sky_graph* g, CallWords* w, CallDevice** call);
 // Enqueues the end kernel behind what the call has put on the graph's stream, waits for it and hands out the results.
 // Outputs may be null.  `counts` (n of them, device, may be null) are added to the sampled edges.
+int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);
+// With the graph's own words.
+int call_begin(sky_graph* g, CallDevice** call);
 int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);
-void call_release(sky_graph* g);
+void call_release(CallWords* w);
 
 }  // namespace sky

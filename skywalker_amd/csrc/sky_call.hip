@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256) void sum_counts_kernel(const uint32_t* __restr
   }
 }
 
-// The call words of all graphs: chunks of 64, per device, handed out one to a graph for its lifetime.  A chunk none of
+// The call words of all graphs and sessions: chunks of 64, per device, handed out one to an owner for its lifetime.  A chunk none of
 // whose words is in use goes back to the runtime when another one has free words.
 namespace {
 constexpr int CHUNK = 64;
@@ -56,16 +56,16 @@ void free_chunk(Chunk* c) {
   if (c->host) (void)hipHostFree(c->host);
   delete c;
 }
-int take_words(sky_graph* g) {
+int take_words(int device, CallWords* w) {
   std::lock_guard<std::mutex> lock(g_mutex);
   Chunk* use = nullptr;
   for (Chunk* c : g_chunks)
-    if (c->device == g->device && c->used < CHUNK) use = c;
+    if (c->device == device && c->used < CHUNK) use = c;
   if (!use) {
     Chunk* c = new Chunk();
-    c->device = g->device;
+    c->device = device;
     auto body = [&]() -> int {
-      SKY_HIP(hipDeviceGetAttribute(&c->khz, hipDeviceAttributeWallClockRate, g->device));
+      SKY_HIP(hipDeviceGetAttribute(&c->khz, hipDeviceAttributeWallClockRate, device));
       if (c->khz <= 0) return fail(SKY_ERR_HIP, "the device reports no wall clock rate");
       SKY_HIP(hipMalloc((void**)&c->dev, CHUNK * sizeof(CallDevice)));
       SKY_HIP(hipMemset(c->dev, 0, CHUNK * sizeof(CallDevice)));
@@ -85,22 +85,22 @@ int take_words(sky_graph* g) {
   while (use->taken[k]) ++k;
   use->taken[k] = true;
   ++use->used;
-  g->call_dev = use->dev + k;
-  g->call_host = use->host + k;
-  g->call_khz = use->khz;
-  g->call_seq = use->host[k].seq;
+  w->dev = use->dev + k;
+  w->host = use->host + k;
+  w->khz = use->khz;
+  w->seq = use->host[k].seq;
   return SKY_OK;
 }
 }  // namespace
 
-void call_release(sky_graph* g) {
-  if (!g->call_host) return;
+void call_release(CallWords* w) {
+  if (!w->host) return;
   std::lock_guard<std::mutex> lock(g_mutex);
   for (size_t i = 0; i < g_chunks.size(); ++i) {
     Chunk* c = g_chunks[i];
-    if (g->call_host < c->host || g->call_host >= c->host + CHUNK) continue;
-    const size_t k = (size_t)(g->call_host - c->host);
-    if (g->call_dirty) (void)hipMemset(c->dev + k, 0, sizeof(CallDevice));
+    if (w->host < c->host || w->host >= c->host + CHUNK) continue;
+    const size_t k = (size_t)(w->host - c->host);
+    if (w->dirty) (void)hipMemset(c->dev + k, 0, sizeof(CallDevice));
     c->taken[k] = false;
     --c->used;
     bool other = false;
@@ -111,17 +111,17 @@ void call_release(sky_graph* g) {
     }
     break;
   }
-  g->call_dev = nullptr;
-  g->call_host = nullptr;
+  *w = CallWords{};
 }
 
-int call_begin(sky_graph* g, CallDevice** call) {
-  if (!g->call_host) SKY_TRY(take_words(g));
-  if (g->call_dirty) SKY_HIP(hipMemsetAsync(g->call_dev, 0, sizeof(CallDevice), g->stream));
-  g->call_dirty = true;  // until it has ended well
-  *call = g->call_dev;
+int call_begin(sky_graph* g, CallWords* w, CallDevice** call) {
+  if (!w->host) SKY_TRY(take_words(g->device, w));
+  if (w->dirty) SKY_HIP(hipMemsetAsync(w->dev, 0, sizeof(CallDevice), g->stream));
+  w->dirty = true;  // until it has ended well
+  *call = w->dev;
   return SKY_OK;
 }
+int call_begin(sky_graph* g, CallDevice** call) { return call_begin(g, &g->call, call); }
 
 // Up to this many counts are added up by the end kernel itself; more get a grid of their own.
 constexpr uint64_t END_COUNTS = 32768;
@@ -129,18 +129,18 @@ constexpr uint64_t END_COUNTS = 32768;
 // five microseconds, and one whose kernels fault ends with the runtime's error instead of polling for ever.
 constexpr auto POLL_FOR = std::chrono::microseconds(3000);
 
-int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
+int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
   hipStream_t st = g->stream;
   if (n > END_COUNTS) {
     hipLaunchKernelGGL(sum_counts_kernel, dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 1024)), dim3(256), 0, st, counts,
-                       n, g->call_dev);
+                       n, w->dev);
     n = 0;
   }
-  const unsigned long long seq = ++g->call_seq;
-  hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, st, g->call_dev, g->call_host, seq, counts,
+  const unsigned long long seq = ++w->seq;
+  hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, st, w->dev, w->host, seq, counts,
                      (uint32_t)n);
   SKY_HIP(hipGetLastError());
-  auto ended = [&] { return __atomic_load_n(&g->call_host->seq, __ATOMIC_ACQUIRE) == seq; };
+  auto ended = [&] { return __atomic_load_n(&w->host->seq, __ATOMIC_ACQUIRE) == seq; };
   bool done = ended();
   if (!done) {
     const auto t0 = std::chrono::steady_clock::now();
@@ -155,10 +155,13 @@ int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* c
     SKY_HIP(hipStreamSynchronize(st));
     if (!ended()) return fail(SKY_ERR_HIP, "the call's end was not reported");
   }
-  g->call_dirty = false;
-  if (sampled) *sampled = g->call_host->sampled;
-  if (seconds) *seconds = (double)g->call_host->ticks / ((double)g->call_khz * 1e3);
+  w->dirty = false;
+  if (sampled) *sampled = w->host->sampled;
+  if (seconds) *seconds = (double)w->host->ticks / ((double)w->khz * 1e3);
   return SKY_OK;
+}
+int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
+  return call_end(g, &g->call, sampled, seconds, counts, n);
 }
 
 }  // namespace sky

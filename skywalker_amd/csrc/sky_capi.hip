@@ -238,7 +238,7 @@ int sky_graph_free(sky_graph* g) {
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   pool_release(g);
-  call_release(g);
+  call_release(&g->call);
   free_plan(g);
   free_build_scratch(g);
   free_tiled_scratch(g);

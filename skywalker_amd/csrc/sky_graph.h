@@ -63,12 +63,7 @@ struct sky_graph {
   };
   std::vector<ProfileEntry> build_profile;
 
-  // How a call on this graph reports its end (sky_call.h).
-  sky::CallDevice* call_dev = nullptr;
-  sky::CallHost* call_host = nullptr;
-  unsigned long long call_seq = 0;
-  int call_khz = 0;
-  bool call_dirty = false;  // a call has begun and not ended well: its device words may not be zero
+  sky::CallWords call;  // how a call on this graph reports its end (sky_call.h)
 
   // Device buffers that calls on this graph reuse instead of allocating each time (they only grow).
   enum PoolSlot { POOL_WALK_LIST = 0, POOL_WALK_COUNTS, POOL_BITMAP, POOL_LIST, POOL_TOTALS, POOL_FRONT, POOL_SEGMENTS, POOL_SLOTS };

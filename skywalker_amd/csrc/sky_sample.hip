@@ -288,7 +288,7 @@ __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint3
   if (list) append_list(fresh, v, list, count, s_n);
 }
 
-// Start of an online call: start vertices in place, the bitmap of built rows cleared.
+// Start of an online call: start vertices in place, the bitmap of built rows and the counters cleared.
 __global__ __launch_bounds__(256) void sample_init_kernel(const uint32_t* __restrict__ seeds, uint32_t N, uint64_t lps,
                                                           uint32_t* __restrict__ data, uint32_t* __restrict__ bitmap,
                                                           uint32_t words, uint32_t* __restrict__ counts, uint32_t ncounts,
@@ -316,8 +316,11 @@ struct SampleSession {
   std::vector<uint64_t> width, off, loff;
   uint64_t lps = 0, slen = 0;
   CallDevice* call = nullptr;
+  CallWords own_words;  // of a session whose steps are calls of their own
   uint32_t *bitmap = nullptr, *list = nullptr, *d_count = nullptr;
-  uint32_t* front_counts = nullptr;  // FRONTIER_WORDS device words per hop: rows of every degree class (dev_sized)
+  // Counters of the frontiers, a hop's own each, cleared when the call begins: the length of its list, then FRONTIER_WORDS
+  // with the rows of every degree class (dev_sized).
+  uint32_t *list_counts = nullptr, *front_counts = nullptr;
   FrontierLists front;
   bool want_list = false;        // the caller is to see the frontier as a list of vertices
   uint32_t* totals = nullptr;    // children of each start vertex, when the kernels add them up
@@ -335,10 +338,12 @@ struct SampleSession {
   SampleSession(const SampleSession&) = delete;
   ~SampleSession() {
     if (holds_pool) g->sampler_busy = false;
+    call_release(&own_words);
     for (auto& b : own)
       if (b.p) (void)hipFree(b.p);
   }
   sky_graph::PoolBuf* buffer(int slot) { return holds_pool ? &g->pool[slot] : &own[slot]; }
+  CallWords* words() { return want_list ? &own_words : &g->call; }
   int get(int slot, size_t bytes, void** out) {
     SKY_TRY(buf_grow(buffer(slot), bytes));
     *out = buffer(slot)->p;
@@ -396,7 +401,8 @@ struct SampleSession {
       }
     }
     if ((uint64_t)N * lps > (1ull << 40)) return fail(SKY_ERR_LIMIT, "sample: output too large");
-    const uint32_t words = (g->V + 31) / 32;
+    const uint32_t bits = (g->V + 31) / 32;  // words of the bitmap
+    uint32_t counters = 0;
     if (online) {
       SKY_TRY(ensure_table_storage(g));
       if (dev_sized) {
@@ -406,25 +412,27 @@ struct SampleSession {
         uint64_t most = 0;
         for (uint32_t h = 0; h + 1 < hops; ++h) most = std::max(most, (uint64_t)N * width[h]);
         SKY_TRY(frontier_lists(g, (uint32_t)std::min<uint64_t>(most, g->V), buffer(sky_graph::POOL_SEGMENTS), &front));
-        SKY_TRY(get(sky_graph::POOL_FRONT, (size_t)(hops - 1) * FRONTIER_WORDS * 4, (void**)&front_counts));
         epoch = ++g->frontier_epoch;
       } else {
         SKY_TRY(prepare_build_scratch(g, g->V));
       }
-      SKY_TRY(get(sky_graph::POOL_BITMAP, (size_t)words * 4, (void**)&bitmap));
+      counters = (hops - 1) * (1 + (dev_sized ? FRONTIER_WORDS : 0u));
+      SKY_TRY(get(sky_graph::POOL_FRONT, (size_t)counters * 4, (void**)&list_counts));
+      d_count = list_counts;
+      if (dev_sized) front_counts = list_counts + (hops - 1);
+      SKY_TRY(get(sky_graph::POOL_BITMAP, (size_t)bits * 4, (void**)&bitmap));
       if (want_list || !dev_sized) SKY_TRY(get(sky_graph::POOL_LIST, (size_t)g->V * 4, (void**)&list));
     }
-    SKY_TRY(call_begin(g, &call));
-    d_count = call->count;
+    SKY_TRY(call_begin(g, words(), &call));
     if (N && one_workgroup()) SKY_TRY(get(sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
     if (online)
-      hipLaunchKernelGGL(sample_init_kernel, dim3(std::min((std::max(N, words) + 255) / 256, 2048u)), dim3(256), 0, st, seeds, N,
-                         lps, data, bitmap, words, front_counts, dev_sized ? (hops - 1) * FRONTIER_WORDS : 0u, call);
+      hipLaunchKernelGGL(sample_init_kernel, dim3(std::min((std::max(N, bits) + 255) / 256, 2048u)), dim3(256), 0, st, seeds, N,
+                         lps, data, bitmap, bits, list_counts, counters, call);
     return SKY_OK;
   }
 
   // Online: the distinct parents of hop h whose rows this call has not built yet, into `list`; their number stays in
-  // the device word d_count (and is read by the host only when the build needs it there).
+  // the hop's device word d_count (and is read by the host only when the build needs it there).
   int frontier(uint32_t h) {
     frontier_upper = frontier_count = 0;
     if (!online || !N) return SKY_OK;
@@ -432,7 +440,7 @@ struct SampleSession {
     const HopGeom hg = geom(h);
     const uint64_t slots = (uint64_t)N * hg.width;
     frontier_upper = (uint32_t)std::min<uint64_t>(slots, g->V);
-    d_count = call->count + h;
+    d_count = list_counts + h;
     if (dev_sized) SKY_TRY(frontier_lists(g, frontier_upper, buffer(sky_graph::POOL_SEGMENTS), &front));
     hipLaunchKernelGGL(frontier_collect_kernel, dim3((uint32_t)((slots + COLLECT_T - 1) / COLLECT_T)), dim3(COLLECT_T), 0, st,
                        data, sample_lengths, slots, g->V, hg, bitmap, g->xadj, g->valid, front,
@@ -508,8 +516,8 @@ struct SampleSession {
   }
 
   int end(uint64_t* sampled, double* seconds) {
-    if (totals) return call_end(g, sampled, seconds, totals, N);
-    return call_end(g, sampled, seconds, sample_lengths, (uint64_t)N * slen);
+    if (totals) return call_end(g, words(), sampled, seconds, totals, N);
+    return call_end(g, words(), sampled, seconds, sample_lengths, (uint64_t)N * slen);
   }
 };
 

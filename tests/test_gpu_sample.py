@@ -282,3 +282,95 @@ def test_other_calls_between_the_steps_of_a_session(orc):
         assert np.array_equal(data.to_host((n, lps)), want[0]) and np.array_equal(sl.to_host((n, slen)), want[1])
         assert sampled.value == want[2]
     g.free()
+
+
+def open_session(capi, g, seeds, fan, seed, sl_fill=0):
+    """begin: (session, seeds, fanouts, data, sample_lengths), everything that has to stay alive."""
+    import ctypes as C
+    lps, slen = capi.sample_layout(fan)
+    seeds_d, fan = capi.DeviceArray.from_host(seeds), np.array(fan, np.uint32)
+    data = capi.DeviceArray(len(seeds) * lps, np.uint32, fill=capi.FILL)
+    sl = capi.DeviceArray(len(seeds) * slen, np.uint32, fill=sl_fill)
+    sess = C.c_void_p()
+    capi._ck(capi.lib().sky_sample_session_begin(g.h, seeds_d.ptr, C.c_uint32(len(seeds)), capi._p(fan), C.c_uint32(len(fan)),
+                                                 C.c_uint64(seed), data.ptr, sl.ptr, C.byref(sess)))
+    return sess, seeds_d, fan, data, sl
+
+
+def session_frontier(capi, sess, hop):
+    """Device addresses of list and count, and the bound."""
+    import ctypes as C
+    lst, cnt, upper = C.c_void_p(), C.c_void_p(), C.c_uint32()
+    capi._ck(capi.lib().sky_sample_session_frontier(sess, C.c_uint32(hop), C.byref(lst), C.byref(cnt), C.byref(upper)))
+    return lst, cnt, upper.value
+
+
+def session_end(capi, sess):
+    import ctypes as C
+    sampled, sec = C.c_uint64(), C.c_double()
+    capi._ck(capi.lib().sky_sample_session_end(sess, C.byref(sampled), C.byref(sec)))
+    return sampled.value, sec.value
+
+
+def read_list(capi, lst, cnt, room):
+    n = np.empty(1, np.uint32)
+    capi._ck(capi.lib().sky_memcpy_d2h(capi._p(n), cnt, 4))
+    assert n[0] <= room
+    out = np.empty(int(n[0]), np.uint32)
+    capi._ck(capi.lib().sky_memcpy_d2h(capi._p(out), lst, int(out.nbytes)))
+    return out
+
+
+def parents_by_hop(data, fan, V):
+    """Distinct vertices of every hop that no hop before held, from the sampled blocks."""
+    seen, out, off, width = np.zeros(0, np.uint32), [], 0, 1
+    for h in range(len(fan) - 1):
+        width *= int(fan[h])
+        block = np.unique(data[:, off:off + width])
+        fresh = np.setdiff1d(block[block < V], seen)
+        out.append(fresh)
+        seen = np.union1d(seen, fresh)
+        off += width
+    return out
+
+
+@pytest.mark.parametrize("device_sized", [1, 0])
+def test_lists_and_counts_of_sessions_open_at_the_same_time(orc, device_sized):
+    # two sessions at the same hop, other calls before the lists are read: every list holds the distinct parents of its own
+    # session, and weights given for the listed rows alone are all that the builds need
+    import ctypes as C
+    from skywalker_amd import capi
+    rng = np.random.default_rng(80)
+    degs = list(rng.integers(0, 60, 3000)) + [300, 700, 3000, 6000, 9000, 70001] * 3
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal")
+    V, fan = len(xadj) - 1, [1, 5, 4, 2]
+    lps, slen = capi.sample_layout(fan)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_device_sized", device_sized)
+    g.set_option("online_full_build", 0)
+    some = rng.integers(0, V, 700).astype(np.uint32)
+    runs = []
+    for n in (40, V):  # the second session's first frontier is every vertex: its list is full
+        seeds = rng.integers(0, V, n).astype(np.uint32) if n < V else np.arange(V, dtype=np.uint32)
+        want = orc.sample_online(xadj, adjncy, w, seeds, fan, 41)
+        runs.append((seeds, want, parents_by_hop(want[0], fan, V), np.zeros_like(w), open_session(capi, g, seeds, fan, 41)))
+    for hop in range(3):
+        lists = [session_frontier(capi, s[0], hop) for _, _, _, _, s in runs]
+        g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, some, 4, 0.0, 5)
+        got = g.sample_online(some, [1, 3, 2], 43)
+        want = orc.sample_online(xadj, adjncy, w, some, [1, 3, 2], 43)
+        assert np.array_equal(got[0].to_host(want[0].shape), want[0]) and got[2] == want[2]
+        for (seeds, _, parents, mine, s), (lst, cnt, upper) in zip(runs, lists):
+            listed = read_list(capi, lst, cnt, upper)
+            assert np.array_equal(np.sort(listed), parents[hop])
+            for v in listed:
+                mine[xadj[v]:xadj[v + 1]] = w[xadj[v]:xadj[v + 1]]
+            w_d = capi.DeviceArray.from_host(mine)
+            capi._ck(capi.lib().sky_sample_session_hop(s[0], C.c_uint32(hop), w_d.ptr))
+    for seeds, want, _, _, s in runs:
+        sampled, sec = session_end(capi, s[0])
+        n = len(seeds)
+        assert np.array_equal(s[3].to_host((n, lps)), want[0]) and np.array_equal(s[4].to_host((n, slen)), want[1])
+        assert sampled == want[2] and 0 < sec < 60
+    g.free()
