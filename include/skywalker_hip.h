@@ -199,7 +199,8 @@ int sky_sample_online(sky_graph* g, const uint32_t* seeds_device, uint32_t N, co
  *      row through a constructor that asks gpu_graph::getBias for each weight
  *      (include/alias_table_new.cuh:1090-1091, called from src/online_sample_new.cu:3-70); here the operator lives in
  *      another library, so the sampler hands out the frontier and takes the weights back:
- *        begin     outputs cleared, start vertices in place; the graph's tables count as not built
+ *        begin     sample_lengths cleared, start vertices in place in data (whose other slots stay as they are until
+ *                  they are reached); the graph's tables count as not built
  *        frontier  the distinct parents of `hop` (0 .. hops - 2) whose rows this session has not built: their vertex
  *                  ids in *list_device, their number in the device word *count_device (the host is not told it),
  *                  at most *upper of them
@@ -207,7 +208,8 @@ int sky_sample_online(sky_graph* g, const uint32_t* seeds_device, uint32_t N, co
  *                  the listed rows are read; an array whose allocation does not hold 16 more bytes, which
  *                  sky_device_malloc always adds, is copied first, as in sky_alias_build_from_weights; NULL: the
  *                  graph's own weights), then draws the children of `hop`
- *        end       sampled edges and kernel-region seconds; frees the session
+ *        end       sampled edges and kernel-region seconds; frees the session.  A session may end before its last hop:
+ *                  the outputs then hold the hops that were drawn
  *      Calls come in that order, frontier and hop once per hop, on one host thread.  Results are those of
  *      sky_sample_online on a graph whose weights are the ones supplied. ---- */
 typedef struct sky_sample_session sky_sample_session;

@@ -288,10 +288,13 @@ __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint3
   if (list) append_list(fresh, v, list, count, s_n);
 }
 
-// Start of an online call: start vertices in place, the bitmap of built rows and the counters cleared.
+// Start of an online call: start vertices in place, the bitmap of built rows and the counters cleared.  A call that runs
+// through all hops writes every length and total; one that is handed out hop by hop may end before, so those are cleared
+// for it (`sl`, nsl words, and `totals`, N; null: left alone).
 __global__ __launch_bounds__(256) void sample_init_kernel(const uint32_t* __restrict__ seeds, uint32_t N, uint64_t lps,
                                                           uint32_t* __restrict__ data, uint32_t* __restrict__ bitmap,
                                                           uint32_t words, uint32_t* __restrict__ counts, uint32_t ncounts,
+                                                          uint32_t* __restrict__ sl, uint64_t nsl, uint32_t* __restrict__ totals,
                                                           CallDevice* __restrict__ call) {
   call_stamp(call);
   if (blockIdx.x == 0)
@@ -299,9 +302,13 @@ __global__ __launch_bounds__(256) void sample_init_kernel(const uint32_t* __rest
   const uint64_t i0 = (uint64_t)blockIdx.x * 256u + threadIdx.x, step = (uint64_t)gridDim.x * 256u;
   for (uint64_t i = i0; i < words; i += step) bitmap[i] = 0;
   for (uint64_t i = i0; i < N; i += step) data[i * lps] = seeds[i];
+  if (sl)
+    for (uint64_t i = i0; i < nsl; i += step) sl[i] = 0;
+  if (totals)
+    for (uint64_t i = i0; i < N; i += step) totals[i] = 0;
 }
 
-// One call of the k-hop sampler, taken apart hop by hop: begin (outputs cleared, start vertices in place), then for
+// One call of the k-hop sampler, taken apart hop by hop: begin (start vertices in place), then for
 // every hop frontier (online: the distinct parents whose rows are not built yet), build (online: their rows) and
 // draw, then end (count, time).  sample_khop runs the steps in turn; sky_sample_session_* hands them to callers that
 // supply the weights of a frontier's rows themselves.
@@ -425,9 +432,12 @@ struct SampleSession {
     }
     SKY_TRY(call_begin(g, words(), &call));
     if (N && one_workgroup()) SKY_TRY(get(sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
+    const uint64_t lengths = want_list ? (uint64_t)N * slen : 0;  // to be cleared
+    const uint64_t items = std::max<uint64_t>(std::max(N, bits), lengths);
     if (online)
-      hipLaunchKernelGGL(sample_init_kernel, dim3(std::min((std::max(N, bits) + 255) / 256, 2048u)), dim3(256), 0, st, seeds, N,
-                         lps, data, bitmap, bits, list_counts, counters, call);
+      hipLaunchKernelGGL(sample_init_kernel, dim3((uint32_t)std::min<uint64_t>((items + 255) / 256, 2048)), dim3(256), 0, st, seeds,
+                         N, lps, data, bitmap, bits, list_counts, counters, lengths ? sample_lengths : nullptr, lengths,
+                         want_list ? totals : nullptr, call);
     return SKY_OK;
   }
 

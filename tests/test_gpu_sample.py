@@ -374,3 +374,29 @@ def test_lists_and_counts_of_sessions_open_at_the_same_time(orc, device_sized):
         assert np.array_equal(s[3].to_host((n, lps)), want[0]) and np.array_equal(s[4].to_host((n, slen)), want[1])
         assert sampled == want[2] and 0 < sec < 60
     g.free()
+
+
+@pytest.mark.parametrize("n,fan", [(40, [1, 5, 4]), (3, [1, 64, 64])])
+@pytest.mark.parametrize("distinct", [0, 1])
+def test_session_ended_before_its_last_hop(orc, n, fan, distinct):
+    # the count and the lengths are those of the hops that were drawn, whatever the caller's array held before; totals added
+    # up by the workgroups of the start vertices (40) and by the lengths (3 x 64 x 64, several workgroups each)
+    import ctypes as C
+    from skywalker_amd import capi
+    rng = np.random.default_rng(81)
+    xadj, adjncy, w = graph_from_degrees(rng.integers(3, 90, 500), rng, "lognormal")
+    seeds = rng.integers(0, 500, n).astype(np.uint32)
+    prob, alias, _ = orc.alias_build(xadj, w)
+    whole = orc.sample_offline(xadj, adjncy, prob, alias, seeds, fan, 47, distinct=bool(distinct))
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("sample_distinct", distinct)
+    for drawn in (0, 1):
+        s = open_session(capi, g, seeds, fan, 47, sl_fill=7)
+        for hop in range(drawn):
+            session_frontier(capi, s[0], hop)
+            capi._ck(capi.lib().sky_sample_session_hop(s[0], C.c_uint32(hop), None))
+        sampled, _ = session_end(capi, s[0])
+        sl = whole[1].copy()
+        sl[:, drawn:] = 0  # one length per start vertex at hop 0
+        assert np.array_equal(s[4].to_host(sl.shape), sl) and sampled == int(sl.sum())
+    g.free()
