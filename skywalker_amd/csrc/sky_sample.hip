@@ -433,7 +433,7 @@ struct SampleSession {
     SKY_TRY(call_begin(g, words(), &call));
     if (N && one_workgroup()) SKY_TRY(get(sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
     const uint64_t lengths = want_list ? (uint64_t)N * slen : 0;  // to be cleared
-    const uint64_t items = std::max<uint64_t>(std::max(N, bits), lengths);
+    const uint64_t items = std::max<uint64_t>(std::max(std::max(N, bits), 1u), lengths);  // an empty graph has counters too
     if (online)
       hipLaunchKernelGGL(sample_init_kernel, dim3((uint32_t)std::min<uint64_t>((items + 255) / 256, 2048)), dim3(256), 0, st, seeds,
                          N, lps, data, bitmap, bits, list_counts, counters, lengths ? sample_lengths : nullptr, lengths,

@@ -400,3 +400,17 @@ def test_session_ended_before_its_last_hop(orc, n, fan, distinct):
         sl[:, drawn:] = 0  # one length per start vertex at hop 0
         assert np.array_equal(s[4].to_host(sl.shape), sl) and sampled == int(sl.sum())
     g.free()
+
+
+def test_online_calls_on_a_graph_without_vertices_and_without_tables(orc):
+    from skywalker_amd import capi
+    none = np.zeros(0, np.uint32)
+    for V in (0, 300):
+        g = capi.Graph.upload(np.zeros(V + 1, np.uint32), none, np.zeros(0, np.float32))
+        for device_sized in (1, 0):
+            g.set_option("online_device_sized", device_sized)
+            assert g.sample_online(none, [1, 3, 2], 1)[2] == 0
+            assert g.sample_session(none, [1, 3, 2], 1)[2] == 0
+        assert g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, none, 4, 0.0, 1)[2] == 0
+        assert g.walk_online(capi.BIAS_NODE2VEC, 2.0, 0.5, none, 4, 0.0, 1)[2] == 0
+        g.free()
