@@ -27,6 +27,9 @@ struct BuildPlan {
   uint64_t *BL = nullptr, *BH = nullptr;
   uint32_t* nfh = nullptr;
   uint4* ranges = nullptr;
+  BuildPlan() = default;
+  BuildPlan(const BuildPlan&) = delete;
+  ~BuildPlan();
 };
 
 // Segments of a frontier's rows: class c from start[c] on, as many as the device word counts[c] says.  The classes
@@ -35,7 +38,6 @@ struct FrontierLists {
   RowRef* list = nullptr;
   uint32_t start[CLS_COUNT] = {0}, cap[CLS_COUNT] = {0};
   int tiled_from = 0;
-  uint32_t plan_serial = 0;  // the plan it was laid out for
 };
 constexpr uint32_t FRONTIER_WORDS = 32;  // device words of counts per frontier
 static_assert(FRONTIER_WORDS >= CLS_COUNT, "one word per class");
@@ -46,11 +48,12 @@ int ensure_plan(sky_graph* g);
 int build_all_fused(sky_graph* g, CallDevice* call);
 // The rows of at least min_degree entries alone (a class boundary of 33 or more); needs the plan.  `call` is stamped.
 int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call);
-// Segments for a frontier of at most n_upper rows, in `buf`, which grows when it has to.
-int frontier_lists(sky_graph* g, uint32_t n_upper, sky_graph::PoolBuf* buf, FrontierLists* f);
+// Segments for a frontier of at most n_upper rows, in `buf`, which grows when it has to.  `p` is a plan of the graph, the same
+// for all frontiers of a call.
+int frontier_lists(sky_graph* g, const BuildPlan& p, uint32_t n_upper, sky_graph::PoolBuf* buf, FrontierLists* f);
 // Builds the rows in the segments (counts: their lengths, on the device) and those of the tiled classes whose bit is set
 // and that no build of the same `epoch` has built yet.  Nothing waits for the device.
-int build_frontier(sky_graph* g, const FrontierLists& f, const uint32_t* counts, const uint32_t* bitmap, uint32_t epoch);
+int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, const uint32_t* counts, const uint32_t* bitmap, uint32_t epoch);
 
 // Appends the vertices of the calling workgroup's lanes whose `fresh` is set to their classes' segments: one global atomic
 // per class that occurs.  All threads of the workgroup call it; s_cnt and s_base hold CLS_COUNT words of LDS each.

@@ -484,22 +484,18 @@ int alloc(void** p, size_t bytes) {
 }
 }  // namespace
 
-void free_plan(sky_graph* g) {
-  if (!g->plan) return;
-  void* ptrs[] = {g->plan->rows, g->plan->trows, g->plan->tiles};
+BuildPlan::~BuildPlan() {
+  void* ptrs[] = {rows, trows, tiles};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
-  delete g->plan;
-  g->plan = nullptr;
 }
 
 int ensure_plan(sky_graph* g) {
   const long long narrow_limit = option(g, OPT_STREAM_MIN_EDGES);
   if (g->plan && g->plan->narrow_limit == narrow_limit) return SKY_OK;
-  free_plan(g);
+  g->plan.reset();
   hipStream_t st = g->stream;
-  g->plan = new BuildPlan();
-  ++g->plan_serial;
+  g->plan = std::make_shared<BuildPlan>();
   BuildPlan& p = *g->plan;
   auto body = [&]() -> int {
     SKY_TRY(bin_all_rows(g, CLS_G16, &p.rows, p.start));
@@ -563,7 +559,7 @@ int ensure_plan(sky_graph* g) {
     return SKY_OK;
   };
   const int rc = body();
-  if (rc != SKY_OK) free_plan(g);
+  if (rc != SKY_OK) g->plan.reset();
   return rc;
 }
 
@@ -591,8 +587,7 @@ struct Launch {
   }
 };
 
-FusedArgs common_args(sky_graph* g, int tiled_from) {
-  const BuildPlan& p = *g->plan;
+FusedArgs common_args(sky_graph* g, const BuildPlan& p, int tiled_from) {
   FusedArgs a = {};
   a.xadj = g->xadj;
   a.wgt = g->adjwgt;
@@ -615,7 +610,7 @@ FusedArgs common_args(sky_graph* g, int tiled_from) {
 
 // The four launches, in order on the graph's stream.
 template <bool DEV>
-int launch_all(sky_graph* g, Launch& wave, Launch& pair, Launch& wide, Launch& block, CallDevice* call) {
+int launch_all(sky_graph* g, const BuildPlan& p, Launch& wave, Launch& pair, Launch& wide, Launch& block, CallDevice* call) {
   hipStream_t st = g->stream;
   // the first launch that has anything to do is the call's first
   Launch* const order[4] = {&wave, &pair, &wide, &block};
@@ -628,8 +623,8 @@ int launch_all(sky_graph* g, Launch& wave, Launch& pair, Launch& wide, Launch& b
   // over what there is.
   auto grid = [&](const Launch& l, uint32_t cap) { return dim3((uint32_t)(DEV ? std::min<uint64_t>(l.units, cap) : l.units)); };
   if (wave.units) hipLaunchKernelGGL((fused_wave_kernel<DEV>), grid(wave, 5120), dim3(64), 0, st, wave.a);
-  if (wave.a.ledgers_done) hipLaunchKernelGGL(fused_ledger_kernel, dim3(g->plan->n_trows - wave.a.trow0), dim3(64), 0, st, g->plan->trows, wave.a.trow0,
-                                              g->plan->tsum, DEV);
+  if (wave.a.ledgers_done) hipLaunchKernelGGL(fused_ledger_kernel, dim3(p.n_trows - wave.a.trow0), dim3(64), 0, st, p.trows, wave.a.trow0,
+                                              p.tsum, DEV);
   if (pair.units) hipLaunchKernelGGL((fused_pair_kernel<DEV>), grid(pair, 2560), dim3(128), 0, st, pair.a);
   if (wide.units) hipLaunchKernelGGL((fused_wide_kernel<DEV>), grid(wide, 512), dim3(512), 0, st, wide.a);
   if (block.units) hipLaunchKernelGGL((fused_block_kernel<DEV>), grid(block, 1024), dim3(256), 0, st, block.a);
@@ -643,7 +638,7 @@ bool fused_possible(const sky_graph* g) { return option(g, OPT_ROW_MERGE) != 0 &
 static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call) {
   g->has_walk_index = false;
   const BuildPlan& p = *g->plan;
-  FusedArgs base = common_args(g, p.t_all);
+  FusedArgs base = common_args(g, p, p.t_all);
   const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
   base.list = p.rows;
   // at least 64 vertices a wavefront, 1024 at most, and enough wavefronts for every SIMD in between
@@ -674,15 +669,13 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   block.add(SEC_M10, rows(CLS_MW2 + 3), 1, p.start[CLS_MW2 + 3]);
   block.add(SEC_M8, rows(CLS_MW2 + 2), 1, p.start[CLS_MW2 + 2]);
   block.add(SEC_M6, rows(CLS_MW2 + 1), 1, p.start[CLS_MW2 + 1]);
-  return launch_all<false>(g, wave, pair, wide, block, call);
+  return launch_all<false>(g, p, wave, pair, wide, block, call);
 }
 int build_all_fused(sky_graph* g, CallDevice* call) { return build_host_sized(g, 0, call); }
 int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call) { return build_host_sized(g, min_degree, call); }
 
 // ---------------------------------------------------------------- rows of a frontier
-int frontier_lists(sky_graph* g, uint32_t n_upper, sky_graph::PoolBuf* buf, FrontierLists* f) {
-  SKY_TRY(ensure_plan(g));
-  const BuildPlan& p = *g->plan;
+int frontier_lists(sky_graph* g, const BuildPlan& p, uint32_t n_upper, sky_graph::PoolBuf* buf, FrontierLists* f) {
   // A workgroup needs 125 us to stream a row of 65,000 entries, which is as long as everything else that the build of a
   // small frontier does; the rows of a large one keep all workgroups streaming, and that is cheaper by the entry.
   f->tiled_from = n_upper <= SMALL_FRONTIER ? p.t_first : p.t_all;
@@ -694,18 +687,15 @@ int frontier_lists(sky_graph* g, uint32_t n_upper, sky_graph::PoolBuf* buf, Fron
     f->cap[c] = c == CLS_EMPTY || tiled ? 0u : (uint32_t)std::min<uint64_t>(n_upper, in_graph);
     at += f->cap[c];
   }
-  f->plan_serial = g->plan_serial;
   SKY_TRY(buf_grow(buf, at * sizeof(RowRef)));
   f->list = (RowRef*)buf->p;
   return SKY_OK;
 }
 
-int build_frontier(sky_graph* g, const FrontierLists& f, const uint32_t* counts, const uint32_t* bitmap, uint32_t epoch) {
-  if (!g->plan || f.plan_serial != g->plan_serial)
-    return fail(SKY_ERR_STATE, "a knob that decides how long rows are built was changed between a frontier and its build");
+int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, const uint32_t* counts, const uint32_t* bitmap,
+                   uint32_t epoch) {
   g->has_walk_index = false;
-  const BuildPlan& p = *g->plan;
-  FusedArgs base = common_args(g, f.tiled_from);
+  FusedArgs base = common_args(g, p, f.tiled_from);
   const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
   base.list = f.list;
   base.counts = counts;
@@ -742,7 +732,7 @@ int build_frontier(sky_graph* g, const FrontierLists& f, const uint32_t* counts,
   add(block, SEC_M10, 1, CLS_MW2 + 3);
   add(block, SEC_M8, 1, CLS_MW2 + 2);
   add(block, SEC_M6, 1, CLS_MW2 + 1);
-  return launch_all<true>(g, wave, pair, wide, block, nullptr);
+  return launch_all<true>(g, p, wave, pair, wide, block, nullptr);
 }
 
 }  // namespace sky

@@ -1,6 +1,7 @@
 // extern "C" surface of libskywalker_hip.so (declared in include/skywalker_hip.h).
 #include <cstring>
 
+#include "sky_build_fused.h"
 #include "sky_graph.h"
 
 namespace sky {
@@ -239,7 +240,7 @@ int sky_graph_free(sky_graph* g) {
     if (p) (void)hipFree(p);
   pool_release(g);
   call_release(&g->call);
-  free_plan(g);
+  g->plan.reset();
   free_build_scratch(g);
   free_tiled_scratch(g);
   delete g;

@@ -1,5 +1,6 @@
 // Internal definition of the opaque sky_graph handle.
 #pragma once
+#include <memory>
 #include <vector>
 
 #include "sky_call.h"
@@ -32,8 +33,7 @@ struct sky_graph {
   bool opt_own[OPT_COUNT] = {false};  // the graph has a value of its own for the knob
   // scratch memory of the table builds on this graph (allocated on first use, reused by every later build, freed
   // with the graph): row lists and counters of the binning pass, and the arrays of the tile-parallel path
-  sky::BuildPlan* plan = nullptr;  // sky_build_fused.h
-  uint32_t plan_serial = 0;        // plans made so far
+  std::shared_ptr<sky::BuildPlan> plan;  // sky_build_fused.h; a sampling session keeps the one it began with
   uint32_t frontier_epoch = 0;     // calls that have built frontiers
   void* build_scratch = nullptr;
   void* tiled_scratch = nullptr;
@@ -211,7 +211,6 @@ uint32_t tiled_max_tiles(const sky_graph* g);
 extern long long g_option_value[OPT_COUNT];
 inline long long option(const sky_graph* g, SkyOpt o) { return g && g->opt_own[o] ? g->opt_value[o] : g_option_value[o]; }
 void free_build_scratch(sky_graph* g);
-void free_plan(sky_graph* g);
 // Bins all vertices: the graph's class sizes, and the rows of the classes from `listed_from` on in a list of their own
 // (*rows, allocated here; class c starts at start[c]).
 int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start);

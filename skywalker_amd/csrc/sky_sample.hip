@@ -14,6 +14,7 @@
 // Online mode builds the table of every distinct frontier vertex, once, through the same
 // kernels as the offline build (into the graph's table storage), then samples the hop.
 #include <algorithm>
+#include <memory>
 #include <vector>
 
 #include "sky_build_fused.h"
@@ -329,6 +330,9 @@ struct SampleSession {
   // with the rows of every degree class (dev_sized).
   uint32_t *list_counts = nullptr, *front_counts = nullptr;
   FrontierLists front;
+  // The plan of the graph when the call began.  Another call between the steps of a session may make the graph a new one, when
+  // a knob that decides how long rows are built has changed.
+  std::shared_ptr<BuildPlan> plan;
   bool want_list = false;        // the caller is to see the frontier as a list of vertices
   uint32_t* totals = nullptr;    // children of each start vertex, when the kernels add them up
   uint32_t epoch = 0;            // this call's number, by which rows made tile by tile tell that it has built them
@@ -414,11 +418,12 @@ struct SampleSession {
       SKY_TRY(ensure_table_storage(g));
       if (dev_sized) {
         SKY_TRY(ensure_plan(g));
+        plan = g->plan;
         // room for the largest hop's rows from the start: growing it at a later hop would free and allocate with that
         // hop's predecessor running (first call on a graph, 40,000 seeds: 1.80 -> 1.45 ms)
         uint64_t most = 0;
         for (uint32_t h = 0; h + 1 < hops; ++h) most = std::max(most, (uint64_t)N * width[h]);
-        SKY_TRY(frontier_lists(g, (uint32_t)std::min<uint64_t>(most, g->V), buffer(sky_graph::POOL_SEGMENTS), &front));
+        SKY_TRY(frontier_lists(g, *plan, (uint32_t)std::min<uint64_t>(most, g->V), buffer(sky_graph::POOL_SEGMENTS), &front));
         epoch = ++g->frontier_epoch;
       } else {
         SKY_TRY(prepare_build_scratch(g, g->V));
@@ -451,7 +456,7 @@ struct SampleSession {
     const uint64_t slots = (uint64_t)N * hg.width;
     frontier_upper = (uint32_t)std::min<uint64_t>(slots, g->V);
     d_count = list_counts + h;
-    if (dev_sized) SKY_TRY(frontier_lists(g, frontier_upper, buffer(sky_graph::POOL_SEGMENTS), &front));
+    if (dev_sized) SKY_TRY(frontier_lists(g, *plan, frontier_upper, buffer(sky_graph::POOL_SEGMENTS), &front));
     hipLaunchKernelGGL(frontier_collect_kernel, dim3((uint32_t)((slots + COLLECT_T - 1) / COLLECT_T)), dim3(COLLECT_T), 0, st,
                        data, sample_lengths, slots, g->V, hg, bitmap, g->xadj, g->valid, front,
                        dev_sized ? front_counts + h * FRONTIER_WORDS : nullptr, list, d_count);
@@ -469,7 +474,7 @@ struct SampleSession {
     if (!online || !N || !frontier_upper) return SKY_OK;
     float* const own = g->adjwgt;
     if (weights) g->adjwgt = const_cast<float*>(weights);  // the build only reads it
-    const int rc = dev_sized ? build_frontier(g, front, front_counts + h * FRONTIER_WORDS, bitmap, epoch)
+    const int rc = dev_sized ? build_frontier(g, *plan, front, front_counts + h * FRONTIER_WORDS, bitmap, epoch)
                              : build_rows(g, list, frontier_count, nullptr);
     g->adjwgt = own;
     return rc;

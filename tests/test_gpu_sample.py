@@ -414,3 +414,36 @@ def test_online_calls_on_a_graph_without_vertices_and_without_tables(orc):
         assert g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, none, 4, 0.0, 1)[2] == 0
         assert g.walk_online(capi.BIAS_NODE2VEC, 2.0, 0.5, none, 4, 0.0, 1)[2] == 0
         g.free()
+
+
+def test_knobs_changed_between_the_steps_of_a_session(orc):
+    # stream_min_edges decides which rows a build makes tile by tile; a session goes on as it began when the knob changes and
+    # another call lays the graph's rows out anew
+    import ctypes as C
+    from skywalker_amd import capi
+    rng = np.random.default_rng(82)
+    degs = list(rng.integers(0, 60, 2000)) + [300, 3000, 6000, 9000, 25000, 70001] * 3
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal")
+    V, fan = len(xadj) - 1, [1, 5, 4, 2]
+    lps, slen = capi.sample_layout(fan)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_full_build", 0)
+    seeds = np.arange(V, dtype=np.uint32)
+    want = orc.sample_online(xadj, adjncy, w, seeds, fan, 53)
+    some = rng.integers(0, V, 300).astype(np.uint32)
+
+    def elsewhere(value):
+        g.set_option("stream_min_edges", value)
+        got, expect = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, some, 6, 0.0, 5), orc.walk_online(xadj, adjncy, w, 0, 1.0, 1.0, some, 6, 0.0, 5)
+        assert np.array_equal(got[0].to_host(expect[0].shape), expect[0])
+    s = open_session(capi, g, seeds, fan, 53)
+    for hop in range(3):
+        elsewhere(0 if hop % 2 else 1 << 30)
+        session_frontier(capi, s[0], hop)
+        elsewhere(1 << 30 if hop % 2 else 0)
+        capi._ck(capi.lib().sky_sample_session_hop(s[0], C.c_uint32(hop), None))
+    sampled, _ = session_end(capi, s[0])
+    assert np.array_equal(s[3].to_host((V, lps)), want[0]) and np.array_equal(s[4].to_host((V, slen)), want[1])
+    assert sampled == want[2]
+    g.free()
