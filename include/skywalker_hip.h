@@ -211,9 +211,8 @@ int sky_sample_online(sky_graph* g, const uint32_t* seeds_device, uint32_t N, co
  *        end       sampled edges and kernel-region seconds; frees the session.  A session may end before its last hop:
  *                  the outputs then hold the hops that were drawn
  *      Calls come in that order, frontier and hop once per hop, on one host thread.  Results are those of
- *      sky_sample_online on a graph whose weights are the ones supplied.  Tuning knobs that decide how rows are built count
- *      as they were at begin.  Other calls on the graph, other sessions among them, may come in between; they share its
- *      tables, so a row that such a call builds from other weights is the one that the session then draws from. ---- */
+ *      sky_sample_online on a graph whose weights are the ones supplied.  Other calls on the graph,
+ *      other sessions among them, may come in between, and knobs may change; all calls share the graph's tables, so a row that such a call builds from other weights is the one that the session then draws from. ---- */
 typedef struct sky_sample_session sky_sample_session;
 int sky_sample_session_begin(sky_graph* g, const uint32_t* seeds_device, uint32_t N, const uint32_t* fanout, uint32_t hops,
                              uint64_t philox_seed, uint32_t* data_device, uint32_t* sample_lengths_device,

@@ -65,7 +65,7 @@ struct FusedArgs {
   uint32_t* nfh;
   uint4* ranges;
   const uint32_t* bitmap;  // frontier: bit set for every vertex whose row has been asked for (null: every row is built)
-  uint32_t epoch;          // frontier: number of the call, to tell rows built earlier in it
+  uint32_t* built;         // frontier: by row of trows, set once a build of the same call has made it
   uint32_t tile0, trow0;  // first tile and row of those this build makes tile by tile
   bool ledgers_done;
   CallDevice* call;  // the call's first launch notes when it began
@@ -144,8 +144,9 @@ __device__ __forceinline__ bool row_at(const FusedArgs& a, const SectionRef& s, 
   return true;
 }
 
-__device__ __forceinline__ bool tile_active(const FusedArgs& a, const TiledRow& r) {
-  return !a.bitmap || (((a.bitmap[r.v >> 5] >> (r.v & 31)) & 1u) && r.done != a.epoch);
+__device__ __forceinline__ bool tile_active(const FusedArgs& a, uint32_t r) {
+  const uint32_t v = a.trows[r].v;
+  return ((a.bitmap[v >> 5] >> (v & 31)) & 1u) && !a.built[r];
 }
 
 // The exact sum of tile `tile` by a wavefront: 16 slots per lane.
@@ -153,9 +154,8 @@ __device__ __forceinline__ void tile_sum_wave(const FusedArgs& a, uint32_t tile)
   const uint32_t lane = threadIdx.x & 63;
   const TileGeom tg = a.geom[tile];
   if (tg.span == 0) return;  // there are fewer tiles than their bound
-  const TiledRow* row = a.trows + tg.row;
   if (a.bitmap) {
-    const bool active = tile_active(a, *row);
+    const bool active = tile_active(a, tg.row);
     if (tg.T == 0 && lane == 0) a.trows[tg.row].active = active ? 1u : 0u;
     if (!active) return;
   }
@@ -368,7 +368,7 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
         if (a.bitmap && !a.trows[r].active) break;
         if (a.trows[r].ntiles && a.trows[r].ok)
           tile_scan_row<512>(a.trows, r, a.ttot, a.BL, a.BH, a.nfh, a.ranges, *reinterpret_cast<TileScanLds<512>*>(smem));
-        if (threadIdx.x == 0) a.trows[r].done = a.epoch;
+        if (a.bitmap && threadIdx.x == 0) a.built[r] = 1;
         break;
       }
       default: break;
@@ -439,7 +439,7 @@ __global__ __launch_bounds__(1024) void plan_rows_kernel(const RowRef* __restric
       o.ntiles = nt;
       o.tile0 = before + inc - nt;
       o.bofs = o.tile0 + r;  // every row owns ntiles + 1 prefix slots
-      o.active = o.done = 0;
+      o.active = 0;
     }
     carry += total;
     __syncthreads();
@@ -693,14 +693,14 @@ int frontier_lists(sky_graph* g, const BuildPlan& p, uint32_t n_upper, sky_graph
 }
 
 int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, const uint32_t* counts, const uint32_t* bitmap,
-                   uint32_t epoch) {
+                   uint32_t* built) {
   g->has_walk_index = false;
   FusedArgs base = common_args(g, p, f.tiled_from);
   const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
   base.list = f.list;
   base.counts = counts;
   base.bitmap = bitmap;
-  base.epoch = epoch;
+  base.built = built;
   Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
   auto add = [&](Launch& l, Section k, uint32_t per, int cls, int ncls = 1) {
     uint32_t upper = 0;

@@ -17,7 +17,7 @@ struct TiledRow {
   double scale, fs, inv_fs;
   uint64_t one, total_h;
   uint32_t ok, last_heavy;  // last_heavy: span index
-  uint32_t active, done;    // builds of a frontier: whether its row is among those asked for; the call that built it
+  uint32_t active;          // builds of a frontier: whether the row is among those that the build makes
 };
 struct TileTotals {
   uint64_t d, u;

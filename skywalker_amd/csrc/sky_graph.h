@@ -34,7 +34,6 @@ struct sky_graph {
   // scratch memory of the table builds on this graph (allocated on first use, reused by every later build, freed
   // with the graph): row lists and counters of the binning pass, and the arrays of the tile-parallel path
   std::shared_ptr<sky::BuildPlan> plan;  // sky_build_fused.h; a sampling session keeps the one it began with
-  uint32_t frontier_epoch = 0;     // calls that have built frontiers
   void* build_scratch = nullptr;
   void* tiled_scratch = nullptr;
   int device = 0;  // the device that was current when the graph was created: its arrays live there

@@ -298,9 +298,8 @@ __global__ __launch_bounds__(256) void sample_init_kernel(const uint32_t* __rest
                                                           uint32_t* __restrict__ sl, uint64_t nsl, uint32_t* __restrict__ totals,
                                                           CallDevice* __restrict__ call) {
   call_stamp(call);
-  if (blockIdx.x == 0)
-    for (uint32_t i = threadIdx.x; i < ncounts; i += 256u) counts[i] = 0;
   const uint64_t i0 = (uint64_t)blockIdx.x * 256u + threadIdx.x, step = (uint64_t)gridDim.x * 256u;
+  for (uint64_t i = i0; i < ncounts; i += step) counts[i] = 0;
   for (uint64_t i = i0; i < words; i += step) bitmap[i] = 0;
   for (uint64_t i = i0; i < N; i += step) data[i * lps] = seeds[i];
   if (sl)
@@ -327,15 +326,16 @@ struct SampleSession {
   CallWords own_words;  // of a session whose steps are calls of their own
   uint32_t *bitmap = nullptr, *list = nullptr, *d_count = nullptr;
   // Counters of the frontiers, a hop's own each, cleared when the call begins: the length of its list, then FRONTIER_WORDS
-  // with the rows of every degree class (dev_sized).
-  uint32_t *list_counts = nullptr, *front_counts = nullptr;
+  // with the rows of every degree class (dev_sized).  Behind them a word for every row that can be made tile by tile, set when
+  // this call has built it: kept with the graph's rows instead, another call's build between two hops of a session made the
+  // session build the row again, from weights that its caller had not supplied.
+  uint32_t *list_counts = nullptr, *front_counts = nullptr, *built = nullptr;
   FrontierLists front;
   // The plan of the graph when the call began.  Another call between the steps of a session may make the graph a new one, when
   // a knob that decides how long rows are built has changed.
   std::shared_ptr<BuildPlan> plan;
   bool want_list = false;        // the caller is to see the frontier as a list of vertices
   uint32_t* totals = nullptr;    // children of each start vertex, when the kernels add them up
-  uint32_t epoch = 0;            // this call's number, by which rows made tile by tile tell that it has built them
   uint32_t frontier_upper = 0;   // most rows the last frontier can hold
   uint32_t frontier_count = 0;   // its size, when the host has read it (dev_sized false)
   // A session keeps its buffers while other calls, other sessions among them, use the same graph: the first to come holds
@@ -424,14 +424,16 @@ struct SampleSession {
         uint64_t most = 0;
         for (uint32_t h = 0; h + 1 < hops; ++h) most = std::max(most, (uint64_t)N * width[h]);
         SKY_TRY(frontier_lists(g, *plan, (uint32_t)std::min<uint64_t>(most, g->V), buffer(sky_graph::POOL_SEGMENTS), &front));
-        epoch = ++g->frontier_epoch;
       } else {
         SKY_TRY(prepare_build_scratch(g, g->V));
       }
-      counters = (hops - 1) * (1 + (dev_sized ? FRONTIER_WORDS : 0u));
+      counters = (hops - 1) * (1 + (dev_sized ? FRONTIER_WORDS : 0u)) + (dev_sized ? plan->n_trows : 0u);
       SKY_TRY(get(sky_graph::POOL_FRONT, (size_t)counters * 4, (void**)&list_counts));
       d_count = list_counts;
-      if (dev_sized) front_counts = list_counts + (hops - 1);
+      if (dev_sized) {
+        front_counts = list_counts + (hops - 1);
+        built = front_counts + (hops - 1) * FRONTIER_WORDS;
+      }
       SKY_TRY(get(sky_graph::POOL_BITMAP, (size_t)bits * 4, (void**)&bitmap));
       if (want_list || !dev_sized) SKY_TRY(get(sky_graph::POOL_LIST, (size_t)g->V * 4, (void**)&list));
     }
@@ -474,7 +476,7 @@ struct SampleSession {
     if (!online || !N || !frontier_upper) return SKY_OK;
     float* const own = g->adjwgt;
     if (weights) g->adjwgt = const_cast<float*>(weights);  // the build only reads it
-    const int rc = dev_sized ? build_frontier(g, *plan, front, front_counts + h * FRONTIER_WORDS, bitmap, epoch)
+    const int rc = dev_sized ? build_frontier(g, *plan, front, front_counts + h * FRONTIER_WORDS, bitmap, built)
                              : build_rows(g, list, frontier_count, nullptr);
     g->adjwgt = own;
     return rc;

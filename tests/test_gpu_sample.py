@@ -447,3 +447,35 @@ def test_knobs_changed_between_the_steps_of_a_session(orc):
     assert np.array_equal(s[3].to_host((V, lps)), want[0]) and np.array_equal(s[4].to_host((V, slen)), want[1])
     assert sampled == want[2]
     g.free()
+
+
+def test_rows_that_other_calls_build_between_the_hops_of_a_session(orc):
+    # weights are given for the rows that a hop lists and no others, as the interface asks: a long row that hop 0 has built,
+    # and that another call builds as well before hop 1 draws from it again, must not be built from hop 1's weights
+    import ctypes as C
+    from skywalker_amd import capi
+    rng = np.random.default_rng(83)
+    degs = list(rng.integers(3, 60, 400)) + [9000, 30000, 70001, 600001]
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal")
+    V, fan = len(xadj) - 1, [1, 8, 4]
+    adjncy[xadj[:-1]] = V - 4 + np.arange(V) % 4  # every row leads to a long one ...
+    w[xadj[:-1]] = 1000.0                                            # ... and mostly there
+    lps, slen = capi.sample_layout(fan)
+    seeds = np.arange(V - 60, V, dtype=np.uint32)
+    want = orc.sample_online(xadj, adjncy, w, seeds, fan, 59)
+    assert np.isin(want[0][:, 1:9], np.arange(V - 4, V)).any()
+    g = capi.Graph.upload(xadj, adjncy, w)
+    s = open_session(capi, g, seeds, fan, 59)
+    for hop in range(2):
+        lst, cnt, upper = session_frontier(capi, s[0], hop)
+        mine = np.zeros_like(w)
+        for v in read_list(capi, lst, cnt, upper):
+            mine[xadj[v]:xadj[v + 1]] = w[xadj[v]:xadj[v + 1]]
+        w_d = capi.DeviceArray.from_host(mine)
+        if hop:
+            g.sample_online(seeds, [1, 2], 61)
+        capi._ck(capi.lib().sky_sample_session_hop(s[0], C.c_uint32(hop), w_d.ptr))
+    sampled, _ = session_end(capi, s[0])
+    assert np.array_equal(s[3].to_host((60, lps)), want[0]) and np.array_equal(s[4].to_host((60, slen)), want[1])
+    assert sampled == want[2]
+    g.free()
