@@ -287,6 +287,7 @@ __global__ __launch_bounds__(ROWT) void build_lds_kernel(const RowRef* __restric
     if (tid == 0) valid[v] = 0;
     return;
   }
+  if (tid == 0) valid[v] = 1;
   const Ledger L = make_ledger(d, sum);
 
   // classify once; amounts -> prefix sums; first / last heavy of every (sub-tile, wave)
@@ -481,6 +482,7 @@ __global__ __launch_bounds__(HUGE_T) void build_huge_kernel(const RowRef* __rest
       if (tid == 0) valid[v] = 0;
       continue;
     }
+    if (tid == 0) valid[v] = 1;
     const Ledger L = make_ledger(d, sum);
 
     uint64_t carry_l = 0, carry_h = 0;

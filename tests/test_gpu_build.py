@@ -452,3 +452,31 @@ def test_large_builds_leave_short_rows_in_place_and_reuse_their_lists(orc):
         g.build_tables_from_weights(capi.DeviceArray.from_host(np.concatenate([w, np.zeros(4, np.float32)])))
         compare_tables(orc, g, xadj, w, "build %d" % seed)
     g.free()
+
+
+@pytest.mark.parametrize("knobs", [{"row_merge": 0}, {"tiled_max_tiles": 9}, {"row_merge": 0, "tiled_max_tiles": 9}, {}])
+@pytest.mark.parametrize("small_in_place", [-1, 0, 1])
+def test_flags_follow_the_weights_of_the_latest_build(orc, knobs, small_in_place):
+    # rows that had no weight in the build before, and rows uploaded as invalid, are valid again after a build from good
+    # weights, whichever kernels build them and whether or not the build bins the vertices anew
+    from helpers import weights
+    from skywalker_amd import capi
+    rng = np.random.default_rng(54)
+    degs = EDGE_DEGREES + [10_000, 24577, 66000] + list(rng.integers(0, 300, 300))
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "uniform")
+    half = w.copy()
+    for v in range(0, len(degs), 2):
+        half[xadj[v]:xadj[v + 1]] = 0.0
+    g = capi.Graph.upload(xadj, adjncy, w)
+    for k, value in knobs.items():
+        g.set_option(k, value)
+    g.set_option("small_in_place", small_in_place)
+    for seq, build in enumerate([np.zeros_like(w), w, half, w[::-1].copy(), half]):
+        g.build_tables_from_weights(capi.DeviceArray.from_host(build))
+        compare_tables(orc, g, xadj, build, "build %d with %s, small_in_place %d" % (seq, knobs, small_in_place))
+    n = len(w)
+    g.upload_tables(np.zeros(n, np.float32), np.full(n, capi.INVALID, np.uint32), np.zeros(len(degs), np.int8))
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, "uploaded as invalid, %s, small_in_place %d" % (knobs, small_in_place))
+    g.free()
