@@ -192,8 +192,9 @@ __global__ __launch_bounds__(256) void bin_scatter_kernel(const uint32_t* __rest
         vlist[atomicAdd(&s_cur[c], 1u)] = RowRef{v, off, d, 0};
       }
       nt += (uint32_t)__popcll(m);
-      // written here, next to its neighbours' flags; a row without weight clears it later
-      if (c >= listed_from || (c >= 0 && listed_from == CLS_G2)) valid[v] = c != CLS_EMPTY;
+      // Written here, next to its neighbours' flags; a row without weight clears it later.  Lists that a graph keeps for
+      // later builds are made without touching the flags: they belong to whatever tables there are.
+      if (c >= 0 && listed_from == CLS_G2) valid[v] = c != CLS_EMPTY;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();

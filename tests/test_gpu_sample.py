@@ -479,3 +479,29 @@ def test_rows_that_other_calls_build_between_the_hops_of_a_session(orc):
     assert np.array_equal(s[3].to_host((60, lps)), want[0]) and np.array_equal(s[4].to_host((60, slen)), want[1])
     assert sampled == want[2]
     g.free()
+
+
+def test_row_lists_made_anew_leave_the_flags_of_a_session_alone(orc):
+    # a row without weight that a session has built stays without children when another call makes the graph's row lists anew
+    import ctypes as C
+    from skywalker_amd import capi
+    rng = np.random.default_rng(84)
+    degs, fan = [40] * 8 + [1] * 8, [1, 64, 64]  # fanouts above the degree: all neighbours of a row with weight
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "uniform")
+    w[:8 * 40] = 0.0
+    adjncy[8 * 40:] = np.arange(8)  # hop 0 leads from the rows of one entry to those without weight
+    lps, slen = capi.sample_layout(fan)
+    seeds = np.arange(16, dtype=np.uint32)
+    want = orc.sample_online(xadj, adjncy, w, seeds, fan, 67)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_full_build", 0)
+    s = open_session(capi, g, seeds, fan, 67)
+    for hop in range(2):
+        session_frontier(capi, s[0], hop)
+        capi._ck(capi.lib().sky_sample_session_hop(s[0], C.c_uint32(hop), None))
+        g.set_option("stream_min_edges", 7 + hop)
+        g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds[15:], 1, 0.0, 5)
+    sampled, _ = session_end(capi, s[0])
+    assert np.array_equal(s[4].to_host((16, slen)), want[1]) and np.array_equal(s[3].to_host((16, lps)), want[0])
+    assert sampled == want[2] == 8
+    g.free()
