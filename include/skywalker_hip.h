@@ -18,7 +18,8 @@
  *     (from sky_device_malloc, or any other allocator of the same process).
  *   - `seconds` outputs report the kernel region only (start of the first kernel to the end of the last,
  *     by the device's constant-rate clock), like the gettimeofday bracket of the reference
- *     (src/util.cu:35-44).
+ *     (src/util.cu:35-44).  The first call on a graph that needs its rows listed by length makes those lists, which stay
+ *     with the graph, and its seconds contain that.
  *   - unreached output slots are never written; callers that want a sentinel
  *     pre-fill with sky_device_fill_u32.
  */

@@ -823,9 +823,9 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   // plan: they depend on the row offsets alone, and binning 67 M vertices again took 0.35 ms.
   const bool all_rows = src == nullptr && n == g->V;
   const bool planned = all_rows && small_in_place && n > 0;
-  if (planned) SKY_TRY(ensure_plan(g));
+  if (planned) SKY_TRY(ensure_plan(g, &call));
   RowRef* vlist = planned ? g->plan->rows : sc.vlist;
-  // clears the counters of the binning pass and notes when the call began
+  // clears the counters of the binning pass and, unless the plan's first kernel has, notes when the call began
   hipLaunchKernelGGL(build_begin_kernel, dim3(1), dim3(128), 0, st, sc.counters, (uint32_t)(COUNTER_BYTES / 4), call);
   if (n > 0) {
     if (small_in_place && !tm) {
@@ -1019,7 +1019,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   return fan.join();
 }
 
-int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start) {
+int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start, CallDevice** first) {
   hipStream_t st = g->stream;
   SKY_TRY(ensure_table_storage(g));
   SKY_TRY(prepare_build_scratch(g, 0));
@@ -1031,7 +1031,8 @@ int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start) 
   const uint32_t n = g->V, per_block = bin_per_block(n), blocks = n ? (n + per_block - 1) / per_block : 0;
   if (n) {
     hipLaunchKernelGGL(build_begin_kernel, dim3(1), dim3(128), 0, st, sc.counters, (uint32_t)(COUNTER_BYTES / 4),
-                       (CallDevice*)nullptr);
+                       *first);
+    *first = nullptr;
     hipLaunchKernelGGL(bin_count_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, (const uint32_t*)nullptr, n, per_block,
                        sc.blk_cnt, reinterpret_cast<unsigned long long*>(sc.counters + 2 * CLS_COUNT));
     hipLaunchKernelGGL(bin_offsets_kernel, dim3(CLS_COUNT), dim3(256), 0, st, sc.blk_cnt, blocks, sc.counters);
@@ -1059,10 +1060,10 @@ int build_all_tables(sky_graph* g, double* seconds) {
   const bool fused = fused_possible(g) && !option(g, OPT_BUILD_PROFILE) && option(g, OPT_SMALL_IN_PLACE) < 0 &&
                      option(g, OPT_BUILD_STREAMS) != 0 && g->E <= FUSED_MAX_ENTRIES && g->V;
   if (fused) {
-    SKY_TRY(ensure_plan(g));
     CallDevice* call = nullptr;
     double sec = 0;
     SKY_TRY(call_begin(g, &call));
+    SKY_TRY(ensure_plan(g, &call));
     SKY_TRY(build_all_fused(g, call));
     SKY_TRY(call_end(g, nullptr, &sec));
     g->build_profile.assign(1, {"build", (float)(sec * 1e3), g->E});

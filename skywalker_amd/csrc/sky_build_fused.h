@@ -43,10 +43,12 @@ constexpr uint32_t FRONTIER_WORDS = 32;  // device words of counts per frontier
 static_assert(FRONTIER_WORDS >= CLS_COUNT, "one word per class");
 
 bool fused_possible(const sky_graph* g);
-int ensure_plan(sky_graph* g);
+// The graph's plan, made if there is none or a knob has changed.  *first as in bin_all_rows: making the plan is part of the
+// call that needs it, and of its time.
+int ensure_plan(sky_graph* g, CallDevice** first);
 // All rows; needs the plan and vertices.
 int build_all_fused(sky_graph* g, CallDevice* call);
-// The rows of at least min_degree entries alone (a class boundary of 33 or more); needs the plan.  `call` is stamped.
+// The rows of at least min_degree entries alone (a class boundary of 33 or more); needs the plan.  `call` is stamped (null: another kernel was).
 int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call);
 // Segments for a frontier of at most n_upper rows, in `buf`, which grows when it has to.  `p` is a plan of the graph, the same
 // for all frontiers of a call.

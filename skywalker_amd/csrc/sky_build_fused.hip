@@ -490,7 +490,7 @@ BuildPlan::~BuildPlan() {
     if (p) (void)hipFree(p);
 }
 
-int ensure_plan(sky_graph* g) {
+int ensure_plan(sky_graph* g, CallDevice** first) {
   const long long narrow_limit = option(g, OPT_STREAM_MIN_EDGES);
   if (g->plan && g->plan->narrow_limit == narrow_limit) return SKY_OK;
   g->plan.reset();
@@ -498,7 +498,7 @@ int ensure_plan(sky_graph* g) {
   g->plan = std::make_shared<BuildPlan>();
   BuildPlan& p = *g->plan;
   auto body = [&]() -> int {
-    SKY_TRY(bin_all_rows(g, CLS_G16, &p.rows, p.start));
+    SKY_TRY(bin_all_rows(g, CLS_G16, &p.rows, p.start, first));
     p.listed = 0;
     for (int c = CLS_G16; c < CLS_COUNT; ++c) p.listed += g->bin_counts[c];
     p.narrow_limit = narrow_limit;

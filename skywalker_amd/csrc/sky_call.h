@@ -55,6 +55,8 @@ int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, con
 // With the graph's own words.
 int call_begin(sky_graph* g, CallDevice** call);
 int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);
+// Instead of call_end, for a call that has launched nothing after all.
+void call_cancel(sky_graph* g);
 void call_release(CallWords* w);
 
 }  // namespace sky

@@ -123,6 +123,8 @@ int call_begin(sky_graph* g, CallWords* w, CallDevice** call) {
 }
 int call_begin(sky_graph* g, CallDevice** call) { return call_begin(g, &g->call, call); }
 
+void call_cancel(sky_graph* g) { g->call.dirty = false; }
+
 // Up to this many counts are added up by the end kernel itself; more get a grid of their own.
 constexpr uint64_t END_COUNTS = 32768;
 // The host polls this long before it hands the wait to the runtime: a call that takes longer does not notice the

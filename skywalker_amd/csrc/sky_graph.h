@@ -211,8 +211,9 @@ extern long long g_option_value[OPT_COUNT];
 inline long long option(const sky_graph* g, SkyOpt o) { return g && g->opt_own[o] ? g->opt_value[o] : g_option_value[o]; }
 void free_build_scratch(sky_graph* g);
 // Bins all vertices: the graph's class sizes, and the rows of the classes from `listed_from` on in a list of their own
-// (*rows, allocated here; class c starts at start[c]).
-int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start);
+// (*rows, allocated here; class c starts at start[c]).  *first: the call's words if nothing of the call has run yet, else null;
+// the first kernel stamps them and leaves null there.
+int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start, CallDevice** first);
 void free_tiled_scratch(sky_graph* g);
 int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, float stop_prob, uint64_t seed,
                  uint32_t* paths, uint32_t* lengths, uint64_t* sampled, double* seconds);

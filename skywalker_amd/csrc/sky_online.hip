@@ -92,11 +92,11 @@ struct OnlinePlan {
   bool full;            // every row, then the offline walk
   uint32_t table_from;  // else: the rows of at least so many entries
 };
-static int online_plan(sky_graph* g, uint32_t N, uint32_t len, OnlinePlan* o) {
+static int online_plan(sky_graph* g, uint32_t N, uint32_t len, OnlinePlan* o, CallDevice** first) {
   const long long mode = option(g, OPT_ONLINE_FULL_BUILD);
   *o = OnlinePlan{mode > 0, 0xFFFFFFFFu};
   if (mode > 0) return SKY_OK;
-  SKY_TRY(ensure_plan(g));
+  SKY_TRY(ensure_plan(g, first));
   const double E = std::max(1u, g->E), draws = (double)N * len;
   const double draw_ps = N <= FEW_WALKERS ? DRAW_FEW_PS : DRAW_PS;
   const double from = BUILD_PS / draw_ps * E / std::max(1.0, draws);
@@ -130,23 +130,27 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
     return walk_online_node2vec(g, p, q, seeds, N, len, stop_prob, seed, paths, lengths, sampled, seconds);
   // Tables that already exist are used as they are.  Otherwise the rows that the walk will draw from often get theirs, all
   // of them when that is most of what it meets; the paths are the same either way.
-  double build_sec = 0;
+  double plan_sec = 0, build_sec = 0;
   OnlinePlan how{false, 0xFFFFFFFFu};
-  if (!g->has_tables && N && len) {
-    SKY_TRY(online_plan(g, N, len, &how));
-    if (how.full) SKY_TRY(build_all_tables(g, &build_sec));
+  CallDevice* call = nullptr;
+  if (!g->has_tables) {
+    SKY_TRY(call_begin(g, &call));
+    if (N && len) SKY_TRY(online_plan(g, N, len, &how, &call));
+    if (how.full) {  // the build is a call of its own, and so is the plan if it was made just now
+      if (call) call_cancel(g);
+      else SKY_TRY(call_end(g, nullptr, &plan_sec));
+      SKY_TRY(build_all_tables(g, &build_sec));
+    }
   }
   if (g->has_tables) {
     SKY_TRY(walk_offline(g, seeds, N, len, stop_prob, seed, paths, lengths, sampled, seconds));
-    if (seconds) *seconds += build_sec;
+    if (seconds) *seconds += plan_sec + build_sec;
     return SKY_OK;
   }
   hipStream_t st = g->stream;
-  CallDevice* call = nullptr;
-  SKY_TRY(call_begin(g, &call));
   if (how.table_from != 0xFFFFFFFFu) {
     SKY_TRY(build_rows_from(g, how.table_from, call));
-    call = nullptr;  // the build's first kernel is the call's
+    call = nullptr;  // the build's first kernel is the call's, or the plan's was
   }
   if (N) {
     // the fewer walkers, the larger the workgroup that takes one through a long row

@@ -414,10 +414,11 @@ struct SampleSession {
     if ((uint64_t)N * lps > (1ull << 40)) return fail(SKY_ERR_LIMIT, "sample: output too large");
     const uint32_t bits = (g->V + 31) / 32;  // words of the bitmap
     uint32_t counters = 0;
+    SKY_TRY(call_begin(g, words(), &call));
     if (online) {
       SKY_TRY(ensure_table_storage(g));
       if (dev_sized) {
-        SKY_TRY(ensure_plan(g));
+        SKY_TRY(ensure_plan(g, &call));
         plan = g->plan;
         // room for the largest hop's rows from the start: growing it at a later hop would free and allocate with that
         // hop's predecessor running (first call on a graph, 40,000 seeds: 1.80 -> 1.45 ms)
@@ -437,7 +438,6 @@ struct SampleSession {
       SKY_TRY(get(sky_graph::POOL_BITMAP, (size_t)bits * 4, (void**)&bitmap));
       if (want_list || !dev_sized) SKY_TRY(get(sky_graph::POOL_LIST, (size_t)g->V * 4, (void**)&list));
     }
-    SKY_TRY(call_begin(g, words(), &call));
     if (N && one_workgroup()) SKY_TRY(get(sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
     const uint64_t lengths = want_list ? (uint64_t)N * slen : 0;  // to be cleared
     const uint64_t items = std::max<uint64_t>(std::max(std::max(N, bits), 1u), lengths);  // an empty graph has counters too

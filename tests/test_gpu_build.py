@@ -480,3 +480,37 @@ def test_flags_follow_the_weights_of_the_latest_build(orc, knobs, small_in_place
     g.build_tables()
     compare_tables(orc, g, xadj, w, "uploaded as invalid, %s, small_in_place %d" % (knobs, small_in_place))
     g.free()
+
+
+@pytest.mark.parametrize("kind", ["build", "build by class", "walk", "walk on full tables", "sample", "session"])
+def test_seconds_of_a_call_that_lists_the_rows_contain_the_listing(kind):
+    # the first build on a graph, and the next one after a knob has changed how rows are built, lists the rows by class
+    # (two passes over the row offsets).  Against the same call that finds the lists in place, the least of five times each:
+    # at least as much longer as one pass over the offsets takes at 8 TB/s
+    from skywalker_amd import capi
+    V = 1 << 24
+    xadj = np.arange(V + 1, dtype=np.uint32) * np.uint32(2)
+    xadj[-1] += 40  # one row that is listed
+    g = capi.Graph.from_degrees(xadj, 7, capi.W_UNIFORM, 1.0, 2.0, 7)
+    seeds, one = (capi.DeviceArray.from_host(np.arange(n, dtype=np.uint32)) for n in (10, 1))
+    g.set_option("small_in_place", 1 if kind == "build by class" else -1)
+    g.set_option("online_full_build", 0 if kind == "walk" else -1)
+
+    def call(listing=None):
+        g.sample_session(np.zeros(0, np.uint32), [1, 2], 1)  # its begin leaves the graph without tables
+        if listing:
+            g.set_option("stream_min_edges", listing)
+        if kind.startswith("build"):
+            return g.build_tables()
+        if kind == "walk":
+            return g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 4, 0.0, 1)[3]
+        if kind == "walk on full tables":  # a thousand steps of one walker: cheaper with every row built
+            sec = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, one, 1000, 0.0, 1)[3]
+            g.tables()
+            return sec
+        return (g.sample_online if kind == "sample" else g.sample_session)(seeds, [1, 2, 2], 1)[3]
+    call()
+    again, listing = min(call() for _ in range(5)), min(call(10 + k) for k in range(5))
+    print(kind, "again %.1f us, with the listing %.1f us" % (again * 1e6, listing * 1e6))
+    assert listing - again > 4 * V / 8e12
+    g.free()
