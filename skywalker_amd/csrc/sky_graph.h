@@ -116,7 +116,7 @@ enum BuildClass : int {
 constexpr int MERGE_MAX_NW = 10;  // rows of at most 512 * 10 - 3 = 5117 entries pair by merge in LDS
 constexpr uint32_t HOLD_MAX_DEG = 8189;  // 512 threads x 16 slots hold such a row from any 16-byte phase
 constexpr uint32_t STREAM_MAX_DEG = 524287;  // longest row of the streaming classes (one workgroup takes 1.5 ms for it)
-__host__ __device__ __forceinline__ int degree_class(uint32_t d) {
+__host__ __device__ __forceinline__ constexpr int degree_class(uint32_t d) {
   if (d == 0) return CLS_EMPTY;
   if (d <= 2) return CLS_TINY;
   // rows of the group kernels start at any slot (their vector loads and stores only need 4-byte alignment)
@@ -146,7 +146,7 @@ __host__ __device__ __forceinline__ int degree_class(uint32_t d) {
 }
 
 // Shortest row of a class.
-inline uint32_t class_min_degree(int c) {
+constexpr uint32_t class_min_degree(int c) {
   switch (c) {
     case CLS_EMPTY: return 0;
     case CLS_TINY: return 1;
@@ -170,6 +170,19 @@ inline uint32_t class_min_degree(int c) {
     default: return c > CLS_MW2 && c <= CLS_MW2 + MERGE_MAX_NW - 2 ? 512u * (uint32_t)(c - CLS_MW2 + 1) - 2 : 0;
   }
 }
+
+// A walk that draws from the rows of at least so many entries reads tables that were never built if the two disagree: every
+// class starts where degree_class says it does, and the class below it is one that has a start too.
+constexpr bool class_starts_agree() {
+  auto has_start = [](int c) { return c == CLS_EMPTY || class_min_degree(c) > 0; };  // the numbers 22..24 are no classes
+  for (int c = 0; c < CLS_COUNT; ++c) {
+    if (c == CLS_EMPTY || !has_start(c)) continue;
+    const uint32_t d = class_min_degree(c);
+    if (degree_class(d) != c || degree_class(d - 1) == c || !has_start(degree_class(d - 1))) return false;
+  }
+  return degree_class(0) == CLS_EMPTY && has_start(degree_class(0xFFFFFFFFu));
+}
+static_assert(class_starts_agree(), "class_min_degree restates the boundaries of degree_class");
 
 // One listed row of a degree class: the build kernels read where the row lies from the list itself
 // instead of chasing xadj[v] after the list entry (one dependent global load less at every row start).
