@@ -252,7 +252,7 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      whose candidates were all kept already adds nothing, so sample_lengths may be below the fanout.  Fanouts of
  *      at most 64, at most 256 hops (SKY_ERR_LIMIT otherwise).
  *      "small_in_place" (default -1): 1 builds the rows of at most 32 entries in one kernel that walks the vertices
- *      in order and needs no row lists (it runs beside the binning pass and the kernels of the long rows); 0 builds
+ *      in order and needs no row lists (it runs beside the kernels of the long rows); 0 builds
  *      them by degree class like all other rows; -1 takes the former for builds of at least 2^25 rows or of all rows of a
  *      graph of more than 2^27 entries, and in the four launches that make all of a build of up to 2^27 entries.  0 or 1
  *      gives such a build its class kernels back.  Same tables.

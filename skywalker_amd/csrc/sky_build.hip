@@ -19,10 +19,10 @@
 // heavies in slot order) produces, written so that every entry is resolved by two
 // prefix sums and a binary search: no queues, no float atomics, no rollback.
 //
-// Dispatch is by degree class (sky_graph.h): one lane per vertex while binning (deg <= 2),
-// 4/8/16/32/64 lanes per vertex with the prefix arrays in a per-wave LDS strip,
-// 64 to 512 threads per vertex with the row's prefix arrays in LDS (rows up to 4093 entries),
-// and the tile-parallel path of sky_build_tiled.hip for longer rows.
+// Dispatch is by degree class (sky_graph.h): one lane per vertex (deg <= 2), 2 to 32 lanes per vertex with the prefix
+// arrays in a per-wave LDS strip (deg <= 192), 64 to 768 threads per vertex that pair by a merge in LDS (deg <= 5117),
+// 512 threads that hold or stream the row (sky_build_stream.hip), and the tile-parallel path of sky_build_tiled.hip for
+// longer rows.  Builds of up to FUSED_MAX_ENTRIES send the same row builders out in four launches (sky_build_fused.hip).
 #include <algorithm>
 #include <vector>
 

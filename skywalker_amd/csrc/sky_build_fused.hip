@@ -659,7 +659,10 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   pair.add(SEC_P6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
   wide.add(SEC_SCAN, n_trows, 1, 0);
   if (p.t_all != CLS_STREAM) wide.add(SEC_STREAM, rows(CLS_STREAM) + rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM]);
-  wide.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);  // hold_row beside the others would spill 190 registers
+  // Rows of 5118..8189 entries are streamed here: hold_row beside the others would spill 190 registers.  It is no loss: builds
+  // of such rows alone take 55 (4 M entries), 129 (17 M), 435..477 (67 M) and 840..902 us (134 M) this way, 121, 194, 554 and
+  // 1018 us with build_hold_kernel and the row lists in place.
+  wide.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);
   // two classes whose lists lie back to back; min_degree may leave out the first
   auto add_two = [&](Section k, int c) { wide.add(k, rows(c) + rows(c + 1), 1, p.start[rows(c) ? c : c + 1]); };
   add_two(SEC_B10, CLS_MW2 + 7);

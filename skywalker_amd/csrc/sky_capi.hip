@@ -59,7 +59,7 @@ long long g_option_value[OPT_COUNT] = {
     512ll * (sky::STREAM_MAX_DEG / 2),     // stream_wide_min_edges: 512 workgroups run at a time
     -1,                                    // walk_read_once: by the size of the tables
     0,                                     // sample_distinct
-    -1,                                    // small_in_place: builds of at least 2^25 rows
+    -1,                                    // small_in_place: by the size of the build
     1,                                     // build_streams
     0,                                     // build_profile
     0,                                     // walk_compact_every

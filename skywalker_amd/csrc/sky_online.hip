@@ -376,7 +376,7 @@ int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, 
   SKY_TRY(call_begin(g, &call));
   // Four wavefronts per walker, eight while that leaves CUs without one.  A window of 1024 ids per wavefront makes 37 KB
   // of LDS, four walkers to a CU; more walkers than that get windows of 512, 29 KB, five to a CU, so that fewer of them
-  // wait for a CU (2,000 walkers x 40 steps on the scale-18 graph 872 -> 703 us; 900 walkers on the scale-17 graph 538
+  // wait for a CU (2,000 walkers x 40 steps on the scale-18 graph 901 -> 761 us; 900 walkers on the scale-17 graph 538
   // with 1024 ids, 555 with 512).  Less LDS still, by fewer slots whose result is kept or smaller windows, was slower.
   constexpr uint32_t FEW = 512, RESIDENT = 1024;
   const uint32_t most = 0xFFFFFFFFu / 512;  // walkers of one launch: below 2^32 threads

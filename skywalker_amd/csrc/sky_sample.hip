@@ -421,7 +421,7 @@ struct SampleSession {
         SKY_TRY(ensure_plan(g, &call));
         plan = g->plan;
         // room for the largest hop's rows from the start: growing it at a later hop would free and allocate with that
-        // hop's predecessor running (first call on a graph, 40,000 seeds: 1.80 -> 1.45 ms)
+        // hop's predecessor running (first call on a graph, 40,000 seeds: 1.80 -> 1.20 ms)
         uint64_t most = 0;
         for (uint32_t h = 0; h + 1 < hops; ++h) most = std::max(most, (uint64_t)N * width[h]);
         SKY_TRY(frontier_lists(g, *plan, (uint32_t)std::min<uint64_t>(most, g->V), buffer(sky_graph::POOL_SEGMENTS), &front));

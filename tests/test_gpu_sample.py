@@ -155,7 +155,7 @@ def test_seeds_that_do_not_exist_have_no_children(orc):
 
 def test_online_sampling_builds_rows_of_every_class_without_waiting(orc):
     # frontiers whose rows fall into every degree class up to the streaming kernel's, their sizes known to the
-    # device alone; a second call on the same graph finds the class census in place
+    # device alone; a second call on the same graph finds the row lists in place
     from helpers import graph_from_degrees
     from skywalker_amd import capi
     rng = np.random.default_rng(77)
@@ -244,7 +244,7 @@ def test_batches_by_workgroup_and_by_hop(orc, n, fanout, distinct):
 
 def test_other_calls_between_the_steps_of_a_session(orc):
     # a larger batch with more hops, and a second session, on the same graph between the steps: buffers of the first
-    # session neither move nor change
+    # session neither move nor change (what the lists and counts hold: the next test)
     import ctypes as C
     from helpers import graph_from_degrees
     from skywalker_amd import capi

@@ -204,8 +204,8 @@ def test_read_once_gathers_give_the_same_paths(orc):
         g.free()
 
 
-def test_node2vec_rejection_one_walker_per_lane_for_large_batches(orc):
-    # up to 262,144 walkers take 8 lanes each (they search the previous row together); larger batches one lane each
+def test_node2vec_rejection_of_large_batches(orc):
+    # 300,000 walkers take two lanes each, 70,000 of them four: the paths do not depend on it
     from skywalker_amd import capi
     xadj, adjncy = orc.rmat_csr(12, 16, 35)
     w = orc.gen_weights(orc.W_LOGNORMAL, 35, len(adjncy), 0.0, 1.0)
