@@ -52,6 +52,80 @@ __device__ __forceinline__ bool walk_draw(const uint32_t* __restrict__ adjncy, c
   return true;
 }
 
+// Steps [s, s_end) of one walker that has a wavefront for itself; the arguments are the same in every lane.  Returns the step it
+// has come to, s_end unless it stopped.  Everything a step depends on is in scalar registers and its gathers are scalar
+// loads, the lanes hold the random numbers and the vertices of 64 steps, and the neighbour of the drawn column is requested
+// beside the table entry (half of the draws keep the column: two round trips to memory instead of three).
+// VEC: entry and neighbour through the vector cache instead: the scalar caches, one to two CUs, answer some 20 G misses a second
+// on the whole chip, which several thousand walkers ask for.
+template <bool INDEXED, bool VEC>
+__device__ __forceinline__ uint32_t walk_alone(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
+                                               const AliasEntry* __restrict__ table, const WalkEntry* __restrict__ index,
+                                               float stop_prob, uint64_t seed, uint32_t i, uint32_t v, uint32_t s,
+                                               uint32_t s_end, uint32_t* __restrict__ path) {
+  auto uniform = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); };
+  const uint32_t lane = threadIdx.x & 63;
+  while (s < s_end) {
+    const u32x4 r = philox(seed, i, s + lane, 0, DOM_WALK);
+    const uint32_t ubits = __float_as_uint(u24(r.y));
+    const unsigned long long stop = __ballot(u24(r.z) < stop_prob);
+    const uint32_t n = min(64u, s_end - s);
+    uint32_t mine = 0, k = 0;
+    for (; k < n; ++k) {
+      if ((stop >> k) & 1) break;
+      const bounds2u x = *reinterpret_cast<const bounds2u*>(xadj + v);
+      const uint32_t off = x.x, deg = x.y - x.x;
+      if (deg == 0) break;
+      const float u = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)ubits, (int)k));
+      uint32_t at = off + __umulhi((uint32_t)__builtin_amdgcn_readlane((int)r.x, (int)k), deg);
+      if (VEC) asm volatile("" : "+v"(at));
+      if (INDEXED) {
+        const WalkEntry e = index[at];
+        const bool keep = u < __uint_as_float(uniform(__float_as_uint(e.prob)));
+        if (!keep && uniform(e.alias) == SKY_INVALID) break;
+        v = uniform(keep ? e.nbr_col : e.nbr_alias);
+      } else {
+        const AliasEntry e = table[at];
+        uint32_t straight = adjncy[at];
+        if (VEC) asm volatile("" : "+v"(straight));  // here, not where it turns out to be needed
+        else asm volatile("" : "+s"(straight));
+        if (u < __uint_as_float(uniform(__float_as_uint(e.prob)))) {
+          v = uniform(straight);
+        } else {
+          const uint32_t alias = uniform(e.alias);
+          if (alias == SKY_INVALID) break;
+          v = uniform(adjncy[off + alias]);
+        }
+      }
+      if (lane == k) mine = v;
+    }
+    if (lane < k) path[s + 1 + lane] = mine;
+    s += k;
+    if (k < n) break;
+  }
+  return s;
+}
+
+// Few walkers, a wavefront each.  What bounds a walk of a few thousand walkers is the latency of its steps, and a wavefront of
+// 64 walkers waits in every one of them for the slowest of 64 gathers.  4,096 walkers x 80 steps on the scale-16 graph 94.8 ->
+// 55.8 us, 100 walkers 49.4 -> 34.8, 2,048 on the scale-24 graph 96 -> 49.
+template <bool INDEXED, bool VEC>
+__global__ __launch_bounds__(64) void walk_alone_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
+                                                        const AliasEntry* __restrict__ table,
+                                                        const WalkEntry* __restrict__ index,
+                                                        const uint32_t* __restrict__ seeds, uint32_t V, uint32_t len,
+                                                        float stop_prob, uint64_t seed, uint32_t* __restrict__ paths,
+                                                        uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
+  call_stamp(call);
+  const uint32_t i = blockIdx.x;
+  uint32_t* const path = paths + (size_t)i * (len + 1);
+  const uint32_t v = seeds[i];
+  if (threadIdx.x == 0) path[0] = v;
+  uint32_t s = 0;
+  if (v < V) s = walk_alone<INDEXED, VEC>(xadj, adjncy, table, index, stop_prob, seed, i, v, 0, len, path);
+  if (threadIdx.x == 0) lengths[i] = s;
+}
+
 // Steps [s_begin, s_end) of the walkers listed in `live` (null: walkers 0..n_live-1, which then also record
 // their start vertex).  A walker that is still walking at s_end is appended to `next_live` when that list is
 // given: the next launch then runs on full wavefronts again (walkers that reached a vertex without out-edges
@@ -70,26 +144,33 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
   if (n_live_dev) n_live = min(n_live, *n_live_dev);  // the list's length is only known on the device
   uint32_t steps = 0;
   bool walking = false;
-  uint32_t i = 0;
+  bool alone = false;  // the last of the wavefront that still walks
+  uint32_t i = 0, v = 0, s = s_begin;
+  auto finish = [&] {
+    steps = s - s_begin;
+    if (!walking || s_end == len) lengths[i] = s;
+    walking = walking && s_end < len;
+  };
   if (t < n_live) {
     i = live ? live[t] : t;
     uint32_t* path = paths + (size_t)i * (len + 1);
-    uint32_t v;
     if (s_begin == 0) {
       v = seeds[i];
       path[0] = v;
     } else {
       v = path[s_begin];
     }
-    uint32_t s = s_begin;
     walking = v < V;  // a start vertex that does not exist is recorded and never left
     // The random numbers of a step do not depend on where the walker stands: those of the next step are computed
-    // while the row bounds of this one are on their way (ten rounds, a fifth of a step's time otherwise: 4,096 walkers x
-    // 80 steps on the scale-16 graph 93 -> 85 us, 250,000 PPR walkers with the index 91 -> 74).  Spreading few walkers over
-    // more wavefronts, or requesting the neighbour of col beside the table entry, gained nothing: a step is two or
-    // three loads that miss L2, one after another.
+    // while the row bounds of this one are on their way (ten rounds, a tenth of a step's time: 250,000 PPR walkers with the
+    // index 91 -> 74 us).  Requesting the neighbour of col beside the table entry gains nothing here: of 64 walkers some
+    // take the alias in every step.
     u32x4 r = philox(seed, i, s, 0, DOM_WALK);
     while (walking && s < s_end) {
+      if (!ONCE) {
+        alone = __popcll(__ballot(true)) == 1;
+        if (alone) break;
+      }
       uint32_t b[WALK_STAGE];
       uint32_t got = 0;
 #pragma unroll
@@ -126,10 +207,22 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
       }
       s += got;
     }
-    steps = s - s_begin;
-    if (!walking || s_end == len) lengths[i] = s;
-    walking = walking && s_end < len;
+    if (ONCE) finish();
   }
+  if (const unsigned long long m = ONCE ? 0ull : __ballot(alone)) {
+    // The longest walks decide how long a launch lasts, and they end with their wavefronts to themselves (20,000 PPR walkers
+    // on the scale-24 graph 48 -> 43 us, 1 M 330 -> 310, 1 M walkers x 80 steps 1615 -> 1575).  Not where entries are read once:
+    // there the lines moved decide, and the scalar loads would keep what is not needed again.
+    const int l = __ffsll((long long)m) - 1;
+    auto of = [&](uint32_t x) { return (uint32_t)__builtin_amdgcn_readlane((int)x, l); };
+    const uint32_t to = walk_alone<INDEXED, false>(xadj, adjncy, table, index, stop_prob, seed, of(i), of(v), of(s), s_end,
+                                                   paths + (size_t)of(i) * (len + 1));
+    if (alone) {
+      s = to;
+      walking = to == s_end;
+    }
+  }
+  if (!ONCE && t < n_live) finish();
   if (next_live) {  // survivors, one atomic per wavefront
     const unsigned long long m = __ballot(walking);
     if (m) {
@@ -182,6 +275,12 @@ static void launch_walk(sky_graph* g, const uint32_t* seeds, const uint32_t* liv
                        seed, paths, lengths, next_live, n_next, call, partials);
 }
 
+// Up to ALONE_WALKERS walkers, as many wavefronts as the GPU holds, get a wavefront each (8,192 walkers x 80 steps on the
+// scale-16 graph 96 -> 69 us; twice as many would walk in two turns: 130, 97 with a lane each).  Beyond ALONE_SCALAR the
+// vector cache takes part (4,096 walkers 60.8 us all scalar, 54.9 with it; 1,000 walkers 35.4 and 37.5), and with the
+// walk index, whose entries leave no load to request ahead, a lane each is as fast (4,000 walkers on the scale-22
+// graph 70 us both ways; 2,000 walkers 45 -> 37).
+constexpr uint32_t ALONE_WALKERS = 8192, ALONE_SCALAR = 2048;
 int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, float stop_prob, uint64_t seed,
                  uint32_t* paths, uint32_t* lengths, uint64_t* sampled, double* seconds) {
   hipStream_t st = g->stream;
@@ -200,6 +299,16 @@ int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, 
     if (g->has_walk_index) launch_walk<true>(g, a...);
     else launch_walk<false>(g, a...);
   };
+  if (N && N <= (g->has_walk_index ? ALONE_SCALAR : ALONE_WALKERS) && !segmented) {
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(N), dim3(64), 0, st, g->xadj, g->adjncy, g->table, g->walk_index, seeds, g->V, len, stop_prob,
+                         seed, paths, lengths, call);
+    };
+    const bool vec = N > ALONE_SCALAR;
+    if (g->has_walk_index) go(walk_alone_kernel<true, false>);
+    else vec ? go(walk_alone_kernel<false, true>) : go(walk_alone_kernel<false, false>);
+    return call_end(g, sampled, seconds, lengths, N);
+  }
   if (N && !segmented) {
     run(seeds, (const uint32_t*)nullptr, (const uint32_t*)nullptr, N, len, 0u, len, stop_prob, seed, paths, lengths,
         (uint32_t*)nullptr, (uint32_t*)nullptr, call, (unsigned long long*)nullptr);

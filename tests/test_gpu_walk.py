@@ -47,6 +47,31 @@ def test_ppr_bit_exact_and_length_law(orc):
     assert chi_square_p(np.append(cnt, len(seeds) - cnt.sum()), np.append(pk, 1 - pk.sum())) > 0.01
 
 
+@pytest.mark.parametrize("n,length,stop", [(1, 1, 0.0), (63, 64, 0.0), (2048, 65, 0.02), (2049, 130, 0.0), (8192, 63, 0.15),
+                                           (8193, 129, 0.02), (70, 200, 0.0)])
+@pytest.mark.parametrize("index", [False, True])
+def test_walkers_with_a_wavefront_each(orc, n, length, stop, index):
+    # the limits between one walker to a wavefront and one to a lane, windows of 64 steps that end inside a walk, and
+    # walks that end at rows without weight, without entries and at start vertices that do not exist
+    from skywalker_amd import capi
+    rng = np.random.default_rng(n)
+    V = 3000
+    xadj, adjncy, w = graph_from_degrees(np.append(rng.integers(0, 40, V - 1), 5000), rng, "sparse", V=V)
+    w[xadj[10]:xadj[40]] = 0.0
+    seeds = rng.integers(0, V + 20, n, dtype=np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    if index:
+        g.build_walk_index()
+    prob, alias, _ = g.tables()
+    paths_d, len_d, sampled, _ = g.walk_offline(seeds, length, stop, 11)
+    paths, lengths = paths_d.to_host((n, length + 1)), len_d.to_host()
+    g.free()
+    opaths, olengths, osampled = orc.walk_offline(xadj, adjncy, prob, alias, seeds, length, stop, 11)
+    assert np.array_equal(lengths, olengths) and sampled == osampled
+    assert np.array_equal(paths, opaths)
+
+
 def test_dead_ends_and_zero_weight_rows(orc):
     # path graph 0 -> 1 -> 2 -> 3 (3 has no out-edge); vertex 4 has one zero-weight edge; 5 loops on itself
     xadj = np.array([0, 1, 2, 3, 3, 4, 5], np.uint32)
