@@ -20,7 +20,7 @@
 // prefix sums and a binary search: no queues, no float atomics, no rollback.
 //
 // Dispatch is by degree class (sky_graph.h): one lane per vertex (deg <= 2), 2 to 32 lanes per vertex with the prefix
-// arrays in a per-wave LDS strip (deg <= 192), 64 to 768 threads per vertex that pair by a merge in LDS (deg <= 5117),
+// arrays in a per-wave LDS strip (deg <= 192), 64 to 512 threads per vertex that pair by a merge in LDS (deg <= 5117),
 // 512 threads that hold or stream the row (sky_build_stream.hip), and the tile-parallel path of sky_build_tiled.hip for
 // longer rows.  Builds of up to FUSED_MAX_ENTRIES send the same row builders out in four launches (sky_build_fused.hip).
 #include <algorithm>
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(ROWT) void build_lds_kernel(const RowRef* __restric
                                                          AliasEntry* __restrict__ table, int8_t* __restrict__ valid) {
   constexpr int CAP = ROWT * 4 * T;
   constexpr int NW = ROWT / 64;
-  extern __shared__ uint64_t smem[];
+  extern __shared__ __align__(16) uint64_t smem[];
   uint64_t* s_sl = smem;
   uint64_t* s_sh = smem + CAP;
   __shared__ u128 s_wsum[NW];
@@ -422,11 +422,13 @@ __global__ __launch_bounds__(ROWT) void build_lds_kernel(const RowRef* __restric
 
 // ---------------------------------------------------------------- one row per workgroup, pairing by merge (merge_row)
 // MINW: wavefronts per SIMD the registers must leave room for; 3 where LDS (50 KB for 256 threads of 14 slots) allows no
-// more anyway.
+// more anyway.  Rows of one class each, 30 M entries, lognormal(0, 2), TB/s of 12 bytes an entry, with integer sums, masks and moves
+// of a thread's own slots, and as it is: 382..509 entries 2.57 and 3.26, 1022..1533 3.03 and 3.30, 2046..2557 2.70 and 3.34,
+// 4606..5117 2.37 and 3.09; on the scale-26 graph, whose rows fill their classes, 2.97 and 4.18, 3.75 and 4.12 for the first two.
 template <int ROWT, int PER, int MINW = 4>
 __global__ __launch_bounds__(ROWT, MINW) void build_merge_kernel(const RowRef* __restrict__ vlist, const float* __restrict__ wgt,
                                                            AliasEntry* __restrict__ table, int8_t* __restrict__ valid) {
-  extern __shared__ uint64_t smem[];
+  extern __shared__ __align__(16) uint64_t smem[];
   __shared__ uint64_t s_aux[8 * (ROWT / 64)];
   const RowRef rr = vlist[blockIdx.x];
   const bool ok = merge_row<ROWT, PER>(rr, smem, s_aux, wgt, table);
@@ -775,7 +777,6 @@ int prepare_build_scratch(sky_graph* g, uint32_t max_rows) {
   if (!g_lds_enabled) {
     SKY_TRY(enable_big_lds(build_lds_kernel<512, 2>, 512 * 4 * 2 * 16));
     SKY_TRY(enable_big_lds(build_merge_kernel<512, 10>, (int)merge_lds_bytes(512, 10)));
-    SKY_TRY(enable_big_lds(build_merge_kernel<768, 6>, (int)merge_lds_bytes(768, 6)));
     g_lds_enabled = true;
   }
   return SKY_OK;
@@ -928,9 +929,8 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
 #define SKY_MW(NW) SKY_TRY(mrg(CLS_MW2 + NW - 2, build_merge_kernel<64 * NW, 8>, 64 * NW, 8, mw_name[NW - 2]))
     // Class nw holds rows that fit 512 nw slots.  Where a shape with an even number of slots per thread and a
     // multiple of 4 wavefronts covers that span exactly, it is used instead of nw wavefronts of 8 slots: every
-    // SIMD of the CU then carries the same number of a workgroup's wavefronts, and 6..10 slots per thread need
-    // 70..110 registers (measured on rows of one class each: 13 % faster for nw = 3, 24 % for 5, 41 % for 6,
-    // 2 % for 7, 31 % for 9, 28 % for 10, where 10 wavefronts of 8 slots also spill).
+    // SIMD of the CU then carries the same number of a workgroup's wavefronts.  768 threads of 6 slots, which would cover
+    // nw = 9, need 86 registers: one workgroup per CU, 1.69 TB/s where 512 threads of 10 slots reach 2.85.
     SKY_MW(2);
     SKY_TRY(mrg(CLS_MW2 + 1, build_merge_kernel<256, 6>, 256, 6, mw_name[1]));
     SKY_MW(4);
@@ -938,7 +938,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     SKY_TRY(mrg(CLS_MW2 + 4, build_merge_kernel<512, 6>, 512, 6, mw_name[4]));
     SKY_TRY(mrg(CLS_MW2 + 5, (build_merge_kernel<256, 14, 3>), 256, 14, mw_name[5]));
     SKY_MW(8);
-    SKY_TRY(mrg(CLS_MW2 + 7, build_merge_kernel<768, 6>, 768, 6, mw_name[7]));
+    SKY_TRY(mrg(CLS_MW2 + 7, build_merge_kernel<512, 10>, 512, 10, mw_name[7]));
     SKY_TRY(mrg(CLS_MW2 + 8, build_merge_kernel<512, 10>, 512, 10, mw_name[8]));
 #undef SKY_MW
   } else {

@@ -276,7 +276,7 @@ constexpr size_t WAVE_LDS = cmax(cmax(SMALL_LDS_BYTES, 2 * 64 * 6 * 8 + 64 * 6),
 // 40,000-seed batch's second hop on the scale-22 graph: 79, 91 and 133 us, with the bounds 63, 70 and 81).
 template <bool DEV>
 __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
-  __shared__ uint64_t smem[(WAVE_LDS + 7) / 8];
+  __shared__ __align__(16) uint64_t smem[(WAVE_LDS + 7) / 8];
   __shared__ uint64_t s_aux[8];
   call_stamp(a.call);
   const UnitFinder<DEV> units(a);
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
 
 template <bool DEV>
 __global__ __launch_bounds__(128, 5) void fused_pair_kernel(FusedArgs a) {
-  __shared__ uint64_t smem[(merge_lds_bytes(128, 8) + 7) / 8];
+  __shared__ __align__(16) uint64_t smem[(merge_lds_bytes(128, 8) + 7) / 8];
   __shared__ uint64_t s_aux[16];
   call_stamp(a.call);
   const UnitFinder<DEV> units(a);

@@ -2,6 +2,8 @@
 // worth of rows) and that the kernels of sky_build.hip and sky_build_fused.hip launch.  The table is the pure function of
 // the weights that sky_build.hip defines.
 #pragma once
+#include <type_traits>
+
 #include "sky_build_common.h"
 #include "sky_graph.h"
 
@@ -11,6 +13,100 @@ namespace sky {
 typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float float2u __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(4)));
+
+// ---------------------------------------------------------------- slots of a wavefront
+// A thread works on PER consecutive slots, so that prefixes and pairing stay in registers, but memory wants the lanes of an
+// instruction side by side: 4 bytes read and 8 written per entry run at 3.1 TB/s when every lane moves its own 8 slots as
+// 16-byte pieces, at 1.8 with 16 slots, at 5.5 to 6.0 when the lanes' pieces are consecutive (4 GiB tables, one MI355X).  So
+// the wavefront's weights and entries change hands in LDS, in room of its own: 12 or 24 instructions of 16 bytes per lane
+// for 8 or 16 slots.
+// Pieces of 16 bytes lie where no two of eight lanes that follow one another meet in a bank: P pieces per lane.
+template <int P>
+__device__ __forceinline__ uint32_t piece_at(uint32_t c) {
+  return P % 8 == 0 ? c ^ ((c >> 3) & 7u) : P % 4 == 0 ? c ^ ((c >> 3) & 3u) : P % 2 == 0 ? c ^ ((c >> 3) & 1u) : c;
+}
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+// Values of the slots first + PER * lane + k of an array, 0 from `end` on (16 bytes behind that may be read).
+// `stage`: 64 * PER * 4 bytes of LDS for this wavefront, 16-byte aligned.
+template <int PER>
+__device__ __forceinline__ void wave_load(const float* __restrict__ src, uint32_t first, uint32_t end, void* stage,
+                                          uint32_t lane, float (&x)[PER]) {
+  static_assert(PER % 2 == 0, "whole pairs");
+  float4* const s4 = reinterpret_cast<float4*>(stage);
+  constexpr int Q = PER / 4, PIECES = 16 * PER;  // whole instructions; pieces of the wavefront
+  constexpr int N = (PIECES + 63) / 64;
+  float4 v[N];
+#pragma unroll
+  for (int t = 0; t < N; ++t) {
+    const uint32_t c = 64u * t + lane, pos = first + 4 * c;
+    v[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    if ((PIECES % 64 == 0 || c < PIECES) && pos < end) {
+      const float4u y = *reinterpret_cast<const float4u*>(src + pos);
+      v[t] = make_float4(y.x, y.y, y.z, y.w);
+    }
+    if (pos < end && pos + 4 > end) {  // one lane of a row
+      if (pos + 1 >= end) v[t].y = 0.f;
+      if (pos + 2 >= end) v[t].z = 0.f;
+      v[t].w = 0.f;
+    }
+  }
+  if constexpr (PER == 4) {
+    x[0] = v[0].x; x[1] = v[0].y; x[2] = v[0].z; x[3] = v[0].w;
+  } else {
+#pragma unroll
+    for (int t = 0; t < N; ++t) {
+      const uint32_t c = 64u * t + lane;
+      if (PIECES % 64 == 0 || c < PIECES) s4[PER % 4 == 0 ? piece_at<Q>(c) : c] = v[t];
+    }
+    wave_lds_sync();
+    if constexpr (PER % 4 == 0) {
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        const float4 y = s4[piece_at<Q>(Q * lane + q)];
+        x[4 * q] = y.x; x[4 * q + 1] = y.y; x[4 * q + 2] = y.z; x[4 * q + 3] = y.w;
+      }
+    } else {
+      const float2* const s2 = reinterpret_cast<const float2*>(stage);
+#pragma unroll
+      for (int h = 0; h < PER / 2; ++h) {
+        const float2 y = s2[PER / 2 * lane + h];
+        x[2 * h] = y.x; x[2 * h + 1] = y.y;
+      }
+    }
+  }
+}
+// Entries of the slots first + PER * lane + k that lie below `end`.
+// `stage`: 64 * PER * 8 bytes of LDS for this wavefront, 16-byte aligned.
+template <int PER>
+__device__ __forceinline__ void wave_store(AliasEntry* __restrict__ dst, uint32_t first, uint32_t end,
+                                           void* stage, uint32_t lane, const float (&p)[PER], const uint32_t (&a)[PER]) {
+  constexpr int P = PER / 2;
+  uint4* const s4 = reinterpret_cast<uint4*>(stage);
+  auto put = [&](uint32_t pos, const uint4u& y) {
+    if (pos + 2 <= end) *reinterpret_cast<uint4u*>(dst + pos) = y;
+    else if (pos < end) dst[pos] = AliasEntry{__uint_as_float(y.x), y.y};
+  };
+  if constexpr (PER == 4) {  // side by side enough
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      put(first + 4 * lane + 2 * h, uint4u{__float_as_uint(p[2 * h]), a[2 * h], __float_as_uint(p[2 * h + 1]), a[2 * h + 1]});
+    return;
+  }
+#pragma unroll
+  for (int h = 0; h < P; ++h)
+    s4[piece_at<P>(P * lane + h)] = make_uint4(__float_as_uint(p[2 * h]), a[2 * h], __float_as_uint(p[2 * h + 1]), a[2 * h + 1]);
+  wave_lds_sync();
+#pragma unroll
+  for (int t = 0; t < P; ++t) {
+    const uint32_t c = 64u * t + lane;
+    const uint4 y = s4[piece_at<P>(c)];
+    put(first + 2 * c, uint4u{y.x, y.y, y.z, y.w});
+  }
+}
 
 // ---------------------------------------------------------------- 2..32 lanes per row
 // G lanes share one row of at most PER * G slots; every lane holds PER consecutive weights, so a
@@ -339,13 +435,51 @@ __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __
 //   the alias of light r is the heavy rank reached when light r - 1 is taken (rank 0 for r = 0),
 //   the light that finishes heavy h is the light rank reached when heavy h is taken,
 // so each thread finds where its share of PER merged elements starts (one diagonal search) and
-// walks it.  The heavy count rides in bits 52..63 of the SH scan: a row of at most 4093 entries
-// keeps its sums below 2^52.
-constexpr uint64_t MERGE_CNT = 1ull << 52;
+// walks it.
+//
+// What bounds it is vector instructions, so
+// - prefix sums are doubles: whole numbers below 2^53 in a row of at most 2^13 slots.  An amount is one rounding instead of
+//   an addition and a mask, a residual one fused multiply-add instead of a conversion;
+// - slots behind the row's end in its last wavefront have weight 0 and go along as lights of deficit 2^40.  They come
+//   after every light of the row, in rank and in the merged order, so nothing of the row depends on them, and no step
+//   needs a mask; a heavy that only one of them reaches is one that nobody finishes;
+// - a slot takes part in the compaction on the side of its kind alone, and the merge reads both heads in every step, at
+//   addresses that differ by what the thread knows, instead of choosing between them.
 constexpr uint32_t MERGE_SELF = 0x80000000u;  // "prob 1, alias self" in the per-heavy result word
 
-// LDS of a row: 14 bytes a slot.
-constexpr size_t merge_lds_bytes(int rowt, int per) { return ((size_t)rowt * per + 2) * 14; }
+// LDS of a row: 14 bytes a slot, or 12 where that lets one more workgroup reside on a CU.  With 12, a heavy's residual takes the place of its
+// prefix sum, which the entries need last, and a row of several wavefronts pays a barrier for it (rows of 3582..4093
+// entries 2.68 -> 3.09 TB/s, of 2046..2557 3.16 -> 3.35; of 4606..5117 3.05 -> 2.94, so those keep 14).
+constexpr int merge_resident(int rowt, int per, int bytes) {
+  const int by_lds = 163840 / ((rowt * per + 2) * bytes + rowt), by_waves = (rowt <= 256 && per <= 8 ? 32 : 24) * 64 / rowt;
+  return by_lds < by_waves ? by_lds : by_waves;
+}
+constexpr bool merge_narrow(int rowt, int per) { return rowt == 64 || merge_resident(rowt, per, 12) > merge_resident(rowt, per, 14); }
+constexpr size_t merge_lds_bytes(int rowt, int per) { return ((size_t)rowt * per + 2) * (merge_narrow(rowt, per) ? 12 : 14); }
+
+// Inclusive prefix sum over the wavefront.
+__device__ __forceinline__ double wave_scan_f64(double v) {
+  auto from = [&](auto get) { v += __longlong_as_double((long long)get((uint64_t)__double_as_longlong(v))); };
+  from([](uint64_t b) { return dpp0_u64<DPP_ROW_SHR1, 0xF>(b); });
+  from([](uint64_t b) { return dpp0_u64<DPP_ROW_SHR2, 0xF>(b); });
+  from([](uint64_t b) { return dpp0_u64<DPP_ROW_SHR4, 0xF>(b); });
+  from([](uint64_t b) { return dpp0_u64<DPP_ROW_SHR8, 0xF>(b); });
+  from([](uint64_t b) { return dpp0_u64<DPP_ROW_BCAST15, 0xA>(b); });
+  from([](uint64_t b) { return dpp0_u64<DPP_ROW_BCAST31, 0xC>(b); });
+  return v;
+}
+__device__ __forceinline__ double lane_f64(double v, int lane) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+// max(|t|, m) in one instruction (fmax would quieten its operands first; neither is a NaN here).
+__device__ __forceinline__ double max_abs_f64(double t, double m) {
+  double x;
+  asm("v_max_f64 %0, |%1|, %2" : "=v"(x) : "v"(t), "v"(m));
+  return x;
+}
 
 // The row `rr` by ROWT threads that share `smem` and, for the wavefronts' sums, s_aux[8 * ROWT / 64].  Returns false when its weights sum to zero.  All threads of the
 // workgroup call it together; the arrays in LDS may be rewritten only after a barrier.
@@ -353,76 +487,62 @@ template <int ROWT, int PER>
 __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint64_t* s_aux,
                                           const float* __restrict__ wgt, AliasEntry* __restrict__ table,
                                           const int tid = threadIdx.x) {
-  // PER consecutive slots per thread, counted from the row's 16-byte aligned start; a thread moves them as
-  // quads when PER is a multiple of 4, as pairs otherwise (its first slot is then only 8-byte aligned)
-  constexpr int VEC = PER % 4 == 0 ? 4 : 2;
-  static_assert(PER % VEC == 0 && PER <= 16, "whole vectors, and `live` has one bit per slot");
   constexpr int CAP = ROWT * PER;
   constexpr int NW = ROWT / 64;
   constexpr uint32_t TOP = CAP + 1;  // heavy h lives at index TOP - h of the value array and of the result array
-  constexpr bool PACKED = CAP <= 4096;  // the heavy count rides in the SH scan; larger rows scan it separately
-  static_assert(CAP <= 8192, "sums and shifts below assume rows of fewer than 2^13 entries");
-  uint64_t* s_v = smem;                                             // [CAP + 2]
-  uint32_t* s_res = reinterpret_cast<uint32_t*>(smem + CAP + 2);  // [CAP + 2]
-  uint16_t* s_hs = reinterpret_cast<uint16_t*>(s_res + CAP + 2);   // [CAP + 2] row-local slot of heavy h
-  WSum3* s_wsum = reinterpret_cast<WSum3*>(s_aux);      // [NW]
-  double* s_fsum = reinterpret_cast<double*>(s_aux + 3 * NW);  // [NW]
-  uint64_t* s_ex = s_aux + 4 * NW;                       // [3 * NW]
-  uint32_t* s_mn = reinterpret_cast<uint32_t*>(s_aux + 7 * NW);  // [NW]
+  static_assert(CAP < 8192 && PER % 2 == 0, "prefix sums below 2^53, 8 * rank in 16 bits, whole pairs");
+  constexpr bool NARROW = merge_narrow(ROWT, PER);
+  using Rank = std::conditional_t<NARROW, uint16_t, uint32_t>;
+  constexpr int RSH = NARROW ? 2 : 1;                // from 8 * index to the place of a rank
+  constexpr uint32_t RB = sizeof(Rank);
+  // [CAP + 2] prefix sums; then [CAP + 2] ranks, times 8: of the heavy that is light r's alias, of the light that finishes heavy h;
+  // then [CAP + 2] the slot of heavy h.  A heavy's residual probability takes the place of its rank, or (NARROW) of its sum.
+  char* const s_v = reinterpret_cast<char*>(smem);
+  char* const s_rank = s_v + (CAP + 2) * 8;
+  char* const s_hs = s_rank + (CAP + 2) * RB;
+  auto val = [&](uint32_t at) -> double& { return *reinterpret_cast<double*>(s_v + at); };        // at: 8 * index
+  auto rank = [&](uint32_t at) -> Rank& { return *reinterpret_cast<Rank*>(s_rank + at); };  // RB * index
+  auto prob = [&](uint32_t at) -> uint32_t& {                                               // 8 * index
+    return *reinterpret_cast<uint32_t*>(NARROW ? s_v + at : s_rank + (at >> RSH));
+  };
+  auto slot_of = [&](uint32_t at) -> uint16_t& { return *reinterpret_cast<uint16_t*>(s_hs + at); };  // 2 * heavy rank
 
   const uint32_t off = rr.off, d = rr.d;
-  const uint32_t base = off & ~3u, lead = off - base, span = lead + d;
   const int wave = tid >> 6, lane = tid & 63;
-  const uint32_t pos0 = (uint32_t)PER * (uint32_t)tid;
-  const bool wave_on = (uint32_t)(PER * 64 * wave) < span;
+  const uint32_t k0 = (uint32_t)PER * (uint32_t)tid, wfirst = PER * 64u * (uint32_t)wave;
+  const bool wave_on = wfirst < d;
+  const uint32_t slots = min((uint32_t)CAP, (d + PER * 64u - 1) / (PER * 64u) * (PER * 64u));  // of the wavefronts that are on
 
-  double wd[PER];
-  uint32_t live = 0;  // bit j: slot pos0 + j belongs to the row
+  double wd[PER];  // clamped weights, then the amounts
   // the sum of the row as a plain fp64 sum where that is exact (plain_sum_is_exact), else as three limbs
   double rsum = 0.0;
   uint32_t mn = 0xFFFFFFFFu;
   if (wave_on) {
+    float xs[PER];
+    wave_load<PER>(wgt + off, wfirst, d, s_v + PER * 256 * wave, lane, xs);
 #pragma unroll
-    for (int t = 0; t < PER / VEC; ++t) {
-      const uint32_t pos = pos0 + (uint32_t)(VEC * t);
-      float xs[4] = {0.f, 0.f, 0.f, 0.f};
-      if (pos < span) {
-        if constexpr (VEC == 4) {
-          const float4 x = *reinterpret_cast<const float4*>(wgt + base + pos);
-          xs[0] = x.x; xs[1] = x.y; xs[2] = x.z; xs[3] = x.w;
-        } else {
-          const float2 x = *reinterpret_cast<const float2*>(wgt + base + pos);
-          xs[0] = x.x; xs[1] = x.y;
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) {
-        const uint32_t idx = pos + k;
-        const bool in = idx - lead < d;  // one unsigned compare: slots before the row wrap around
-        if (in) live |= 1u << (t * VEC + k);
-        const float cw = masked_weight(xs[k], in);
-        wd[t * VEC + k] = (double)cw;
-        rsum += wd[t * VEC + k];
-        mn = min(mn, __float_as_uint(cw) - 1u);
-      }
+    for (int j = 0; j < PER; ++j) {
+      const float cw = clamp_weight(xs[j]);
+      wd[j] = (double)cw;
+      rsum += wd[j];
+      mn = min(mn, __float_as_uint(cw) - 1u);
     }
-    rsum = group_sum_f64<64>(rsum);
+    rsum = lane_f64(wave_scan_f64(rsum), 63);
     mn = wave_min_u32(mn);
-  } else {
-#pragma unroll
-    for (int j = 0; j < PER; ++j) wd[j] = 0.0;
   }
   if (NW > 1) {
+    double* const s_sum = reinterpret_cast<double*>(s_aux);
+    uint32_t* const s_mn = reinterpret_cast<uint32_t*>(s_aux + NW);
     if (lane == 0) {
-      s_fsum[wave] = rsum;
+      s_sum[wave] = rsum;
       s_mn[wave] = mn;
     }
     __syncthreads();
-    rsum = s_fsum[0];
+    rsum = s_sum[0];
     mn = s_mn[0];
 #pragma unroll
     for (int i = 1; i < NW; ++i) {
-      rsum += s_fsum[i];
+      rsum += s_sum[i];
       mn = min(mn, s_mn[i]);
     }
   }
@@ -434,143 +554,165 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
       sum = group_sum_wsum3<64>(sum);
     }
     if (NW > 1) {
-      if (lane == 0) s_wsum[wave] = sum;
+      WSum3* const s_w = reinterpret_cast<WSum3*>(s_aux + 2 * NW);
+      if (lane == 0) s_w[wave] = sum;
       __syncthreads();
-      sum = s_wsum[0];
+      sum = s_w[0];
 #pragma unroll
       for (int i = 1; i < NW; ++i) {
-        sum.top += s_wsum[i].top;
-        sum.mid += s_wsum[i].mid;
-        sum.low += s_wsum[i].low;
+        sum.top += s_w[i].top;
+        sum.mid += s_w[i].mid;
+        sum.low += s_w[i].low;
       }
     }
     rsum = sum.top + sum.mid + sum.low != 0.0 ? wsum3_to_double(sum) : 0.0;
   }
   if (rsum == 0.0) {
-#pragma unroll
-    for (int j = 0; j < PER; ++j)
-      if ((live >> j) & 1) table[base + pos0 + j] = AliasEntry{0.0f, SKY_INVALID};
+    for (uint32_t k = tid; k < d; k += ROWT) table[off + k] = AliasEntry{0.0f, SKY_INVALID};
     return false;
   }
-  const Ledger L = make_ledger_small(d, rsum);
-  const double neg_fs = -L.fs;
 
   float op[PER];
-  uint32_t hcnt[PER];  // heavies up to and including this slot
-  uint32_t heavy = 0;
-  uint32_t nh, nl;
-  {
-    uint64_t dl[PER], dh[PER], sl[PER], sh[PER];
+  bool hv[PER];
+  double run = 0.0, run_u = 0.0;  // amounts of this thread's slots, of its heavies
+  uint32_t cnt = 0;
+  if (wave_on) {
+    const double scale = (double)d / rsum;
+    double fs = 1099511627776.0, neg_fs = -1099511627776.0;  // 2^40
+    asm("" : "+v"(fs), "+v"(neg_fs));  // in registers: as literals they would be moved into every sum's place
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const bool in = (live >> j) & 1;
-      const Entry e = PACKED ? classify_small_fma(wd[j], L, neg_fs) : classify_fast(wd[j], in, L);
-      dl[j] = (e.heavy || !in) ? 0 : e.amount;
-      dh[j] = e.heavy ? (PACKED ? (e.amount | MERGE_CNT) : e.amount) : 0;
-      op[j] = (float)e.p;
-      if (e.heavy) heavy |= 1u << j;
-    }
-    uint64_t total_l, total_h;
-    uint32_t ex_c = 0;
-    if constexpr (PACKED) {
-      block_scan2_flat<ROWT, PER>(dl, dh, s_ex, sl, sh, total_l, total_h, wave_on);
-      nh = (uint32_t)(total_h >> 52);
-    } else {
-      block_scan2c_flat<ROWT, PER>(dl, dh, (uint32_t)__popc(heavy), s_ex, sl, sh, ex_c, total_l, total_h, nh, wave_on);
-    }
-    nl = d - nh;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      const uint32_t hc = PACKED ? (uint32_t)(sh[j] >> 52) : ex_c + (uint32_t)__popc(heavy & ((2u << j) - 1));
-      hcnt[j] = hc;
-      if (!((live >> j) & 1)) continue;
-      const uint32_t li = pos0 + j - lead;
-      const bool hv = (heavy >> j) & 1;
-      s_v[hv ? TOP + 1 - hc : li - hc] = hv ? (PACKED ? (sh[j] & (MERGE_CNT - 1)) : sh[j]) : sl[j];
-      if (hv) s_hs[hc - 1] = (uint16_t)li;
+      const double p = wd[j] * scale, t = fma(p, fs, neg_fs);  // = (p - 1) * 2^F rounded once: the product is exact
+      hv[j] = t >= 0.5;
+      wd[j] = rint(max_abs_f64(t, hv[j] ? 1.0 : 0.0));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
+      op[j] = (float)p;
+      run += wd[j];
+      run_u += hv[j] ? wd[j] : 0.0;
+      cnt += hv[j] ? 1u : 0u;
     }
   }
-  if (tid == 0) {
-    s_v[nl] = ~0ull;
-    s_v[TOP - nh] = ~0ull;
+  // what lies before this thread's slots: amounts, surpluses, heavies
+  double ex, ex_u;
+  uint32_t ex_c, nh;
+  {
+    double* const s_p = reinterpret_cast<double*>(s_aux + 5 * NW);   // [2 * NW]
+    uint32_t* const s_c = reinterpret_cast<uint32_t*>(s_aux + 7 * NW);  // [NW]
+    const double i = wave_scan_f64(run), iu = wave_scan_f64(run_u);
+    const uint32_t ic = group_scan_u32<64>(cnt);
+    ex = i - run;
+    ex_u = iu - run_u;
+    ex_c = ic - cnt;
+    if (NW == 1) {
+      nh = (uint32_t)__builtin_amdgcn_readlane((int)ic, 63);
+    } else {
+      if (lane == 63) {
+        s_p[2 * wave] = i;
+        s_p[2 * wave + 1] = iu;
+        s_c[wave] = ic;
+      }
+      __syncthreads();
+      nh = 0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        if (w < wave) {
+          ex += s_p[2 * w];
+          ex_u += s_p[2 * w + 1];
+          ex_c += s_c[w];
+        }
+        nh += s_c[w];
+      }
+      nh = (uint32_t)__builtin_amdgcn_readfirstlane((int)nh);
+    }
+  }
+  const uint32_t nl = slots - nh;  // the row's own come first: d - nh of them
+  uint32_t at[PER];                // 8 * index of the slot's value
+  if (wave_on) {
+    uint32_t la = 8u * (k0 - ex_c), ha = 8u * (TOP - ex_c), hs = 2u * ex_c;
+    double sl = ex - ex_u, sh = ex_u;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      at[j] = hv[j] ? ha : la;
+      if (hv[j]) {
+        sh += wd[j];
+        val(ha) = sh;
+        slot_of(hs) = (uint16_t)(k0 + j);
+        ha -= 8u;
+        hs += 2u;
+      } else {
+        sl += wd[j];
+        val(la) = sl;
+        la += 8u;
+      }
+    }
+    if (lane == 63 && k0 + PER == slots) {
+      val(8u * nl) = __builtin_huge_val();
+      val(8u * (TOP - nh)) = __builtin_huge_val();
+    }
   }
   __syncthreads();
 
   if (nh) {
-    if (tid == 0) s_res[0] = s_hs[0];  // the first light starts in the first heavy
-    // merged positions [k0, k0 + PER) belong to this thread; a lights and k0 - a heavies come before them
-    const uint32_t k0 = pos0;
-    if (k0 < d) {
-      uint32_t lo = k0 > nh ? k0 - nh : 0u, hi = min(k0, nl);
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        if (s_v[mid - 1] < s_v[TOP - (k0 - mid)]) lo = mid; else hi = mid - 1;
-      }
-      uint32_t a = lo, b = k0 - lo;
-      const uint32_t steps = min((uint32_t)PER, d - k0);
-      uint64_t va = s_v[a], vb = s_v[TOP - b];  // heads of the two sequences: only the one taken is read again
+    if (wave_on) {
+      // merged positions [k0, k0 + PER) belong to this thread; a lights and k0 - a heavies come before them
+      uint32_t a8;
+      {
+        const uint32_t lo = k0 > nh ? k0 - nh : 0u, hi8 = 8u * min(k0, nl), dh = 8u * (TOP - k0);
+        a8 = 8u * lo;
+        const uint32_t most = min(nh, nl);
 #pragma unroll
-      for (int s = 0; s < PER; ++s) {
-        if ((uint32_t)s < steps) {
-          if (vb <= va) {
-            s_res[TOP - b] = a;
-            ++b;
-            vb = s_v[TOP - b];
-          } else {
-            ++a;
-            if (a < nl) s_res[a] = s_hs[min(b, nh - 1)];
-            va = s_v[a];
+        for (uint32_t step = 1u << (31 - __builtin_clz(CAP / 2)); step >= 1; step >>= 1) {
+          if (step <= most) {  // uniform
+            const uint32_t to = a8 + 8u * step;
+            const bool up = val(a8 + 8u * (step - 1)) < val(a8 + dh + 8u * step);
+            a8 = up && to <= hi8 ? to : a8;
           }
         }
       }
+      const uint32_t dh = 8u * (TOP - k0 - (PER - 1));  // the heavy at hand lies so far behind the light at hand, and 8 bytes less in every step
+      uint32_t rh = RB * (TOP - k0), k8 = 8u * k0;
+#pragma unroll
+      for (int s = 0; s < PER; ++s) {
+        const bool take = val(a8 + dh + 8u * (PER - 1 - s)) <= val(a8);  // the heavy
+        rank((a8 >> RSH) + (take ? rh : RB)) = (Rank)(take ? a8 : k8 - a8);
+        a8 += take ? 0u : 8u;
+        rh -= RB;
+        k8 += 8u;
+      }
+    }
+    if (tid == 0) {
+      rank(0) = 0;                                   // the first light starts in the first heavy
+      slot_of(2u * nh) = slot_of(2u * (nh - 1));    // a light beyond every heavy takes the last
     }
     __syncthreads();
     // heavies, densely by rank: residual probability from the light that finishes them
     for (uint32_t h = tid; h < nh; h += ROWT) {
-      const uint32_t r = s_res[TOP - h];
-      uint32_t out = MERGE_SELF;
-      if (h + 1 < nh && r < nl) out = __float_as_uint(residual_prob(L.one + s_v[TOP - h] - s_v[r], L));
-      s_res[TOP - h] = out;
+      const uint32_t i = TOP - h, r = rank(RB * i);
+      const float p = (float)fma(val(r) - val(8u * i), -1.0 / 1099511627776.0, 1.0);
+      prob(8u * i) = h + 1 < nh && r < 8u * (d - nh) ? __float_as_uint(p) : MERGE_SELF;
     }
     __syncthreads();
   }
 
-  if (pos0 < span) {
-    uint32_t oa[PER];
+  uint32_t oa[PER];
+  if (wave_on) {
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      const uint32_t li = pos0 + j - lead;
-      const uint32_t hc = hcnt[j];
-      oa[j] = li;
-      if (nh && ((live >> j) & 1)) {
-        if ((heavy >> j) & 1) {
-          const uint32_t x = s_res[TOP - (hc - 1)];
-          op[j] = x == MERGE_SELF ? 1.0f : __uint_as_float(x);
-          if (x != MERGE_SELF) oa[j] = s_hs[hc];
+      oa[j] = k0 + j;
+      if (nh) {
+        const uint32_t x = NARROW ? (hv[j] ? prob(at[j]) : (uint32_t)rank(at[j] >> RSH)) : (uint32_t)rank(at[j] >> RSH);
+        const uint32_t m = slot_of((hv[j] ? 8u * (TOP + 1) - at[j] : x) >> 2);
+        if (hv[j]) {
+          const bool self = x == MERGE_SELF;
+          op[j] = self ? 1.0f : __uint_as_float(x);
+          oa[j] = self ? oa[j] : m;
         } else {
-          oa[j] = s_res[li - hc];
+          oa[j] = m;
         }
-      }
-    }
-#pragma unroll
-    for (int t = 0; t < PER / VEC; ++t) {
-      const uint32_t pos = pos0 + (uint32_t)(VEC * t);
-      if (pos >= lead && pos + VEC <= span) {
-        if constexpr (VEC == 4) {
-          const float p4[4] = {op[4 * t], op[4 * t + 1], op[4 * t + 2], op[4 * t + 3]};
-          const uint32_t a4[4] = {oa[4 * t], oa[4 * t + 1], oa[4 * t + 2], oa[4 * t + 3]};
-          store_entries4(table + base + pos, p4, a4);
-        } else {
-          *reinterpret_cast<uint4*>(table + base + pos) =
-              make_uint4(__float_as_uint(op[2 * t]), oa[2 * t], __float_as_uint(op[2 * t + 1]), oa[2 * t + 1]);
-        }
-      } else {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k)
-          if ((live >> (t * VEC + k)) & 1) table[base + pos + k] = AliasEntry{op[VEC * t + k], oa[VEC * t + k]};
       }
     }
   }
+  if (NW > 1 && NARROW) __syncthreads();  // the entries take the place of the values
+  if (wave_on) wave_store<PER>(table + off, wfirst, d, s_v + PER * 512 * wave, lane, op, oa);
   return true;
 }
 

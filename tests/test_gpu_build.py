@@ -186,6 +186,38 @@ def test_rows_built_tile_by_tile(orc, dist):
     build_and_compare(orc, xadj, adjncy, w, "tiled/" + dist)
 
 
+@pytest.mark.parametrize("dist", ["uniform", "lognormal2", "nearequal", "sparse", "fewlights", "fewheavies", "alternating"])
+def test_rows_that_end_at_the_ends_of_wavefronts(orc, dist):
+    # rows paired by a merge: the last wavefront full, one slot short, one slot into the next; every row start; lights or
+    # heavies alone but for a few, which keeps one of the two sequences empty for whole wavefronts
+    from helpers import weights
+    from skywalker_amd import capi
+    rng = np.random.default_rng(23)
+    per = {253: (64, 4), 381: (64, 6), 509: (64, 8), 765: (128, 6), 1021: (128, 8), 1533: (256, 6), 2045: (256, 8),
+           2557: (256, 10), 3069: (512, 6), 3581: (256, 14), 4093: (512, 8), 5117: (512, 10)}
+    degs, lo = [], 193
+    for hi, (threads, slots) in per.items():
+        ends = [64 * slots * k + e for k in range(1, threads // 64 + 1) for e in (-1, 0, 1)]
+        degs += [d for d in ends if lo <= d <= hi] + [lo, hi]
+        lo = hi + 1
+    degs += [1, 1, 2, 3] * 8
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal", V=6000)
+    if dist == "fewlights":
+        w = np.where(rng.random(len(w)) < 0.01, 0.01, 1.01).astype(np.float32)
+    elif dist == "fewheavies":
+        w = np.where(rng.random(len(w)) < 0.005, 1000.0, 0.5).astype(np.float32)
+    elif dist == "alternating":  # lights first, then heavies, then lights: the merge runs along one of them for long
+        w = np.where((np.arange(len(w)) // 300) % 2 == 0, 1.0, 3.0).astype(np.float32)
+    else:
+        w = weights(len(w), rng, dist)
+    build_and_compare(orc, xadj, adjncy, w, "ends/" + dist)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, "ends in four launches/" + dist)
+    g.free()
+
+
 def test_streaming_kernel_for_rows_with_too_many_tiles(orc):
     from skywalker_amd import capi
     rng = np.random.default_rng(22)
