@@ -25,8 +25,7 @@
 #pragma once
 #include <type_traits>
 
-#include "sky_build_common.h"
-#include "sky_graph.h"
+#include "sky_build_rows.h"
 
 namespace sky {
 
@@ -47,19 +46,81 @@ __device__ __forceinline__ bool wave_in_row(const StreamRow& r, uint32_t c, int 
   return c * ST_CH + (uint32_t)(ST_PER * 64) * (uint32_t)wave < r.span;
 }
 
+// A thread works on 8 consecutive slots, but memory wants the lanes of an instruction side by side (sky_build_rows.h: every
+// lane its own 64 bytes as 16-byte stores runs at half the rate).  Here the four lanes of a quad move their common
+// 128 bytes of weights and 256 bytes of entries as whole 64-byte pieces and change hands by DPP, which needs no LDS: the
+// window takes all there is.  200 M entries in rows of 15,000 1143 -> 1100 us, of 30,000 1168 -> 1118, of 100,000 1460 -> 1410
+// (instruction issue bounds these rows).
 struct RawChunk {
-  float4 q[ST_PER / 4];
+  float4 q[ST_PER / 4];  // as loaded: quarter-slots quad_pos(c, tid, q) .. + 3
 };
+__device__ __forceinline__ uint32_t quad_pos(uint32_t c, int tid, int q) {
+  return c * ST_CH + 4u * (2u * ((uint32_t)tid & ~3u) + 4u * q + ((uint32_t)tid & 3u));
+}
 __device__ __forceinline__ RawChunk fetch_chunk(const float* __restrict__ wgt, const StreamRow& r, uint32_t c,
                                                 int tid) {
   RawChunk x;
 #pragma unroll
   for (int q = 0; q < ST_PER / 4; ++q) {
-    const uint32_t pos = c * ST_CH + (uint32_t)ST_PER * tid + 4u * q;
+    const uint32_t pos = quad_pos(c, tid, q);
     x.q[q] = make_float4(0.f, 0.f, 0.f, 0.f);
     if (pos < r.span) x.q[q] = *reinterpret_cast<const float4*>(wgt + r.base + pos);
   }
   return x;
+}
+template <int PERM>
+__device__ __forceinline__ uint32_t quad_get(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, PERM, 0xF, 0xF, true);
+}
+constexpr int quad_perm(int a, int b, int c, int d) { return a | b << 2 | c << 4 | d << 6; }
+// The thread's own 8 slots: quarter q of lane i of a quad was loaded as quarter i >> 1 of lane 2 * (i & 1) + q.  All lanes of the
+// wavefront call it together.
+__device__ __forceinline__ RawChunk own_slots(const RawChunk& x, int tid) {
+  const bool upper = (tid & 2) != 0;
+  auto get = [&](auto perm, float lo, float hi) {
+    constexpr int P = decltype(perm)::value;
+    const uint32_t a = quad_get<P>(__float_as_uint(lo)), b = quad_get<P>(__float_as_uint(hi));
+    return __uint_as_float(upper ? b : a);
+  };
+  auto get4 = [&](auto perm) {
+    return make_float4(get(perm, x.q[0].x, x.q[1].x), get(perm, x.q[0].y, x.q[1].y), get(perm, x.q[0].z, x.q[1].z),
+                       get(perm, x.q[0].w, x.q[1].w));
+  };
+  RawChunk o;
+  o.q[0] = get4(std::integral_constant<int, quad_perm(0, 2, 0, 2)>{});
+  o.q[1] = get4(std::integral_constant<int, quad_perm(1, 3, 1, 3)>{});
+  return o;
+}
+// The wavefront's 512 entries, all of which are written: t is where this thread's first one lies.
+__device__ __forceinline__ void quad_store(AliasEntry* t, int tid, const float (&p)[ST_PER], const uint32_t (&a)[ST_PER]) {
+  uint32_t v[4][4];  // [pair of entries][word]; afterwards [lane of the quad]: pair tid & 3 of that lane
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    v[h][0] = __float_as_uint(p[2 * h]);
+    v[h][1] = a[2 * h];
+    v[h][2] = __float_as_uint(p[2 * h + 1]);
+    v[h][3] = a[2 * h + 1];
+  }
+  const bool b0 = tid & 1, b1 = tid & 2;
+  auto swap = [&](auto perm, bool odd, uint32_t& lo, uint32_t& hi) {  // a 2 x 2 transpose between partner lanes
+    constexpr int P = decltype(perm)::value;
+    const uint32_t from_lo = quad_get<P>(lo), from_hi = quad_get<P>(hi);
+    lo = odd ? from_hi : lo;
+    hi = odd ? hi : from_lo;
+  };
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    using X1 = std::integral_constant<int, quad_perm(1, 0, 3, 2)>;
+    using X2 = std::integral_constant<int, quad_perm(2, 3, 0, 1)>;
+    swap(X1{}, b0, v[0][w], v[1][w]);
+    swap(X1{}, b0, v[2][w], v[3][w]);
+    swap(X2{}, b1, v[0][w], v[2][w]);
+    swap(X2{}, b1, v[1][w], v[3][w]);
+  }
+  AliasEntry* const t0 = t - 8 * (tid & 3) + 2 * (tid & 3);
+#pragma unroll
+  for (int h = 0; h < 4; ++h)
+    *reinterpret_cast<uint4*>(t0 + 8 * h) = make_uint4(v[h][0], v[h][1], v[h][2], v[h][3]);
 }
 // Makes the wavefront wait, here, until the chunk's loads have arrived.
 __device__ __forceinline__ void wait_for_chunk(const RawChunk& x) {
@@ -74,14 +135,15 @@ __device__ __forceinline__ bool wave_inside_row(const StreamRow& r, uint32_t c, 
   return w0 >= r.lead && w0 + (uint32_t)(ST_PER * 64) <= r.span;
 }
 // Clamped weights (0 outside the row) and the mask of slots that belong to the row.  EDGE false: the caller
-// knows that every slot does.
-template <bool EDGE>
-__device__ __forceinline__ uint32_t unpack_chunk(const RawChunk& x, const StreamRow& r, uint32_t c, int tid,
+// knows that every slot does.  OWN: the thread's own slots, in order; else those it has loaded, for the sums.
+template <bool EDGE, bool OWN = true>
+__device__ __forceinline__ uint32_t unpack_chunk(const RawChunk& raw, const StreamRow& r, uint32_t c, int tid,
                                                  float (&cw)[ST_PER]) {
   uint32_t live = EDGE ? 0u : (1u << ST_PER) - 1u;
+  const RawChunk x = OWN ? own_slots(raw, tid) : raw;
 #pragma unroll
   for (int q = 0; q < ST_PER / 4; ++q) {
-    const uint32_t pos = c * ST_CH + (uint32_t)ST_PER * tid + 4u * q;
+    const uint32_t pos = OWN ? c * ST_CH + (uint32_t)ST_PER * tid + 4u * q : quad_pos(c, tid, q);
     const float xs[4] = {x.q[q].x, x.q[q].y, x.q[q].z, x.q[q].w};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -202,7 +264,9 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
   auto& s_a = lds.s_a;
   auto& s_c = lds.s_c;
   auto& s_next = lds.s_next;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // what depends on the lane number stays inside this row's code
+  const int wave = tid >> 6, lane = tid & 63;
   StreamRow r;
   r.base = rr.off & ~3u;
   r.lead = rr.off - r.base;
@@ -221,9 +285,9 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
       if (!wave_in_row(r, c, wave)) continue;
       float cw[ST_PER];
       if (wave_inside_row(r, c, wave))
-        unpack_chunk<false>(cur, r, c, tid, cw);
+        unpack_chunk<false, false>(cur, r, c, tid, cw);
       else
-        unpack_chunk<true>(cur, r, c, tid, cw);
+        unpack_chunk<true, false>(cur, r, c, tid, cw);
 #pragma unroll
       for (int j = 0; j < ST_PER; j += 2) {
         fsum += (double)cw[j];
@@ -254,7 +318,7 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
         if (c + 1 < nch) nx = fetch_chunk(wgt, r, c + 1, tid);
         if (!wave_in_row(r, c, wave)) continue;
         float cw[ST_PER];
-        unpack_chunk<true>(cur, r, c, tid, cw);
+        unpack_chunk<true, false>(cur, r, c, tid, cw);
 #pragma unroll
         for (int j = 0; j < ST_PER; ++j) wsum3_add(sum, (double)cw[j]);
       }
@@ -373,11 +437,12 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
     uint64_t sh_hi;  // surplus prefix of the window's last heavy
     {
       // surplus prefix of the window: HP consecutive heavies per thread; the surplus takes the weight's place
-      // in s_sh first, the prefix takes the surplus's place after the scan
+      // in s_sh first, the prefix takes the surplus's place after the scan.  Unrolled by two: whole, the loops cost the
+      // device-sized launch 31 spilled registers.
       constexpr int HP = 12;
       static_assert(ST_CAP < (uint32_t)ST_T * HP, "one round covers the window");
       uint64_t su = 0;
-#pragma unroll
+#pragma unroll 2
       for (int k = 0; k < HP; ++k) {
         const uint32_t h = (uint32_t)HP * tid + k;
         if (h < nw) {
@@ -390,7 +455,7 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
       uint32_t ex_c, tot_c;
       stream_excl(su, 0u, s_a[0], s_c[0], ex_u, ex_c, tot_u, tot_c);
       uint64_t acc = sh_lo + ex_u;
-#pragma unroll
+#pragma unroll 2
       for (int k = 0; k < HP; ++k) {
         const uint32_t h = (uint32_t)HP * tid + k;
         if (h < nw) {
@@ -517,7 +582,9 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
       // chunk's stores are issued: loads and stores complete in one in-order count, so a wait for the load placed
       // after the stores (at its first use in the next iteration) would wait for the stores as well.
       wait_for_chunk(nx);
-      if (wr) {
+      if (__all(wr == (1u << ST_PER) - 1u)) {
+        quad_store(table + r.base + pos0, tid, op, oa);
+      } else if (wr) {  // the edges of the row and of a window
         AliasEntry* const t0 = table + r.base + pos0;
 #pragma unroll
         for (int q = 0; q < ST_PER / 4; ++q) {
@@ -567,14 +634,15 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
 // search per thread, its lights walk the list from there and leave the residual of every heavy they finish in the
 // list; after a barrier every thread completes its own heavies from the list and writes its 16 entries as whole
 // quads: each entry is written once.  A row with more heavies than the list holds repeats list, walk and completion
-// for the next ranks; everything it needs is still in registers.  (2.1 TB/s on such rows against 1.9 for the
-// streaming kernel.  The same with 1024 threads for rows of up to 16381 entries leaves one workgroup per CU, all
-// of whose wavefronts wait at the same barriers: 1.7 TB/s.)
+// for the next ranks; everything it needs is still in registers.  Weights and entries change hands in LDS
+// (wave_load, wave_store), the entries where the list was: with every lane moving its own 128 bytes 200 M entries in
+// rows of 6500 took 1435 us, so 1085 (2.2 TB/s of 12 bytes an entry).  (The same with 1024 threads for rows of up to
+// 16381 entries leaves one workgroup per CU, all of whose wavefronts wait at the same barriers: slower.)
 constexpr int HOLD_PER = 16;
 constexpr int HOLD_T = 512;
 constexpr uint32_t HOLD_CAP = 5632;  // heavies per list: two workgroups fill a CU's LDS
 constexpr size_t HOLD_LDS_BYTES = (size_t)(HOLD_CAP + 2) * 14;
-static_assert(HOLD_T * HOLD_PER >= HOLD_MAX_DEG + 3, "the row fits from any 16-byte phase");
+static_assert(HOLD_T * HOLD_PER >= HOLD_MAX_DEG && HOLD_T * HOLD_PER * 8 <= HOLD_LDS_BYTES, "the row fits, and so do its entries");
 
 // The row `rr` by a workgroup of HOLD_T threads with HOLD_LDS_BYTES of LDS and s_aux[8 * HOLD_T / 64].  Returns false
 // when its weights sum to zero.
@@ -590,31 +658,23 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
   uint64_t* s_ex = s_aux + 4 * NW;                             // [3 * NW]
   uint32_t* s_mn = reinterpret_cast<uint32_t*>(s_aux + 7 * NW);  // [NW]
 
-  const uint32_t d = rr.d;
-  const uint32_t base = rr.off & ~3u, lead = rr.off - base, span = lead + d;
+  const uint32_t d = rr.d, off = rr.off;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const uint32_t pos0 = (uint32_t)PER * (uint32_t)tid;
-  const bool wave_on = (uint32_t)(PER * 64 * wave) < span;
+  const uint32_t pos0 = (uint32_t)PER * (uint32_t)tid, wfirst = (uint32_t)(PER * 64) * (uint32_t)wave;
+  const bool wave_on = wfirst < d;
 
   float cw[PER];
   uint32_t live = 0;  // bit j: slot pos0 + j belongs to the row
   double rsum = 0.0;
   uint32_t mn = 0xFFFFFFFFu;
   if (wave_on) {
+    wave_load<PER>(wgt + off, wfirst, d, reinterpret_cast<char*>(smem) + PER * 256 * wave, lane, cw);
 #pragma unroll
-    for (int q = 0; q < PER / 4; ++q) {
-      const uint32_t pos = pos0 + 4u * q;
-      float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-      if (pos < span) x = *reinterpret_cast<const float4*>(wgt + base + pos);
-      const float xs[4] = {x.x, x.y, x.z, x.w};
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const bool in = pos + k - lead < d;  // one unsigned compare: slots before the row wrap around
-        if (in) live |= 1u << (q * 4 + k);
-        cw[q * 4 + k] = masked_weight(xs[k], in);
-        rsum += (double)cw[q * 4 + k];
-        mn = min(mn, __float_as_uint(cw[q * 4 + k]) - 1u);
-      }
+    for (int j = 0; j < PER; ++j) {
+      if (pos0 + j < d) live |= 1u << j;
+      cw[j] = clamp_weight(cw[j]);
+      rsum += (double)cw[j];
+      mn = min(mn, __float_as_uint(cw[j]) - 1u);
     }
     rsum = group_sum_f64<64>(rsum);
     mn = wave_min_u32(mn);
@@ -655,7 +715,7 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
   if (rsum == 0.0) {
 #pragma unroll
     for (int j = 0; j < PER; ++j)
-      if ((live >> j) & 1) table[base + pos0 + j] = AliasEntry{0.0f, SKY_INVALID};
+      if ((live >> j) & 1) table[off + pos0 + j] = AliasEntry{0.0f, SKY_INVALID};
     return false;
   }
   const Ledger L = make_ledger_small(d, rsum);
@@ -726,7 +786,7 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
 
   uint32_t oa[PER];
 #pragma unroll
-  for (int j = 0; j < PER; ++j) oa[j] = pos0 + (uint32_t)j - lead;  // a light of a row without heavies, and a heavy nobody finishes, point at themselves
+  for (int j = 0; j < PER; ++j) oa[j] = pos0 + (uint32_t)j;  // a light of a row without heavies, and a heavy nobody finishes, point at themselves
   uint64_t sh_lo = 0;  // surplus prefix of the heavies before the list
   for (uint32_t hb = 0; hb < nh; hb += CAPH) {
     const uint32_t nw = min(CAPH, nh - hb);
@@ -766,7 +826,7 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
       count_le<1>(s_sh, nw, k1, o1);
       uint32_t b = o1[0];
       uint64_t hv = s_sh[b], hvn = s_sh[b + 1];  // ~0 once the list is exhausted
-      uint32_t hal = (uint32_t)s_slot[b] - lead, haln = (uint32_t)s_slot[b + 1] - lead;
+      uint32_t hal = (uint32_t)s_slot[b], haln = (uint32_t)s_slot[b + 1];
 #pragma unroll
       for (int j = 0; j < PER; ++j) {
         const bool lt = ((live & ~heavy) >> j) & 1;  // a light of the row
@@ -781,7 +841,7 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
             hv = hvn;
             hal = haln;
             hvn = s_sh[b + 1];
-            haln = (uint32_t)s_slot[b + 1] - lead;
+            haln = (uint32_t)s_slot[b + 1];
           } while (hv <= sl);
         }
       }
@@ -799,7 +859,7 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
           if (r < nw) {
             const bool fin = (r + 1 < nw || more) && su <= tot_d;
             op[j] = fin ? s_prob[r] : 1.0f;
-            if (fin) oa[j] = (uint32_t)s_slot[r + 1] - lead;
+            if (fin) oa[j] = (uint32_t)s_slot[r + 1];
           }
           ++r;
         }
@@ -807,21 +867,8 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
     sh_lo = sh_hi;
   }
 
-  if (pos0 < span) {
-#pragma unroll
-    for (int q = 0; q < PER / 4; ++q) {
-      const uint32_t pos = pos0 + 4u * q;
-      if (pos >= lead && pos + 4 <= span) {
-        const float p4[4] = {op[4 * q], op[4 * q + 1], op[4 * q + 2], op[4 * q + 3]};
-        const uint32_t a4[4] = {oa[4 * q], oa[4 * q + 1], oa[4 * q + 2], oa[4 * q + 3]};
-        store_entries4(table + base + pos, p4, a4);
-      } else {
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          if ((live >> (4 * q + k)) & 1) table[base + pos + k] = AliasEntry{op[4 * q + k], oa[4 * q + k]};
-      }
-    }
-  }
+  __syncthreads();  // the entries take the list's place
+  if (wave_on) wave_store<PER>(table + off, wfirst, d, reinterpret_cast<char*>(smem) + PER * 512 * wave, lane, op, oa);
   return true;
 }
 

@@ -17,7 +17,7 @@ __global__ __launch_bounds__(ST_T, 4) void build_stream_kernel(const RowRef* __r
 
 __global__ __launch_bounds__(HOLD_T, 4) void build_hold_kernel(const RowRef* __restrict__ vlist, const float* __restrict__ wgt,
                                                        AliasEntry* __restrict__ table, int8_t* __restrict__ valid) {
-  extern __shared__ uint64_t smem[];
+  extern __shared__ __align__(16) uint64_t smem[];
   __shared__ uint64_t s_aux[8 * (HOLD_T / 64)];
   const RowRef rr = vlist[blockIdx.x];
   const bool ok = hold_row(rr, smem, s_aux, wgt, table);

@@ -263,6 +263,21 @@ def test_rows_streamed_by_one_workgroup(orc, dist):
     build_and_compare(orc, xadj, adjncy, w, "stream/" + dist)
 
 
+@pytest.mark.parametrize("dist", ["lognormal2", "nearequal", "fewlights"])
+def test_long_rows_that_end_at_the_ends_of_wavefronts(orc, dist):
+    # held rows change hands in LDS by wavefronts of 1024 slots, streamed ones by quads of lanes where all 512 slots of a
+    # wavefront are written and slot by slot elsewhere: ends at both sides of a wavefront's, of a quad's, every row start
+    from helpers import weights
+    rng = np.random.default_rng(37)
+    degs = [1024 * k + e for k in (5, 6, 7) for e in (-1, 0, 1)] + [8 * 1024 - e for e in (5, 4, 3)]
+    degs += [512 * k + e for k in (16, 17, 23, 24, 25, 32) for e in (-33, -4, -1, 0, 1, 2, 3, 31, 32)]
+    degs = [d for d in degs if d >= 5118] + [1, 1, 2, 3] * 12
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal", V=4096)
+    w = np.where(rng.random(len(w)) < 0.01, 0.01, 1.01).astype(np.float32) if dist == "fewlights" else weights(len(w), rng, dist)
+    build_and_compare(orc, xadj, adjncy, w, "ends of long rows/" + dist)
+
+
 def test_special_weight_values_in_every_kind_of_row(orc):
     # NaN, infinities, negatives, -0, denormals, values at and beyond the 2^32 clamp, and values whose
     # contribution to the exact sum is only a few units of 2^-64: same bits as the oracle in every class
