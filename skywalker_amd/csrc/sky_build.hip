@@ -39,12 +39,11 @@ __global__ __launch_bounds__(256) void build_group_kernel(const RowRef* __restri
                                                           const float* __restrict__ wgt,
                                                           AliasEntry* __restrict__ table,
                                                           int8_t* __restrict__ valid) {
-  __shared__ uint64_t s_pre[2 * 256 * PER];
-  __shared__ uint8_t s_hs[256 * PER];
+  __shared__ uint64_t smem[(group_lds_bytes(G, PER, 256) + 7) / 8];
   const uint32_t grp = blockIdx.x * (256 / G) + threadIdx.x / G;
   RowRef rr{0, 0, 0, 0};
   if (grp < count) rr = vlist[grp];
-  const bool ok = group_build_row<G, PER>(rr.off, rr.d, wgt, table, s_pre, s_hs);
+  const bool ok = group_build_row<G, PER>(rr.off, rr.d, wgt, table, smem);
   if ((threadIdx.x & (G - 1)) == 0 && grp < count) valid[rr.v] = ok ? 1 : 0;
 }
 

@@ -253,8 +253,7 @@ __device__ __forceinline__ void group_unit(const FusedArgs& a, const SectionRef&
   asm volatile("" : "+v"(t));  // what depends on the lane number stays inside this unit's code
   RowRef rr;
   const bool have = row_at<DEV>(a, s, unit * (64 / G) + t / G, rows, rr);
-  const bool ok = group_build_row<G, PER, 64>(rr.off, rr.d, a.wgt, a.table, smem,
-                                              reinterpret_cast<uint8_t*>(smem + 2 * 64 * PER), t);
+  const bool ok = group_build_row<G, PER, 64>(rr.off, rr.d, a.wgt, a.table, smem, t);
   if (have && (t & (G - 1)) == 0) a.valid[rr.v] = ok ? 1 : 0;
 }
 template <bool DEV, int ROWT, int PER>
@@ -269,7 +268,7 @@ __device__ __forceinline__ void merge_unit(const FusedArgs& a, const SectionRef&
 }
 
 constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
-constexpr size_t WAVE_LDS = cmax(cmax(SMALL_LDS_BYTES, 2 * 64 * 6 * 8 + 64 * 6), merge_lds_bytes(64, 8));
+constexpr size_t WAVE_LDS = cmax(cmax(SMALL_LDS_BYTES, group_lds_bytes(32, 6, 64)), merge_lds_bytes(64, 8));
 
 // The second launch bounds: what LDS lets reside anyway (21 wavefronts, 10 pairs, 4 workgroups of 256 to a CU).  Left alone the
 // device-sized kernels took 109, 104 and 132 registers, one workgroup in five and one in four less (the 134,652 rows of a

@@ -108,31 +108,71 @@ __device__ __forceinline__ void wave_store(AliasEntry* __restrict__ dst, uint32_
   }
 }
 
+// ---------------------------------------------------------------- sums as doubles
+// Prefix sums of a row's amounts are whole numbers below 2^53 in rows of at most 2^13 slots: doubles hold them exactly, an
+// amount is one rounding instead of an addition and a mask, a residual one fused multiply-add instead of a conversion.
+template <int G>
+__device__ __forceinline__ double group_scan_f64(double v) {
+  const int gl = lane_id() & (G - 1);
+  auto from = [&](int dist, auto get) {
+    const double o = __longlong_as_double((long long)get((uint64_t)__double_as_longlong(v)));
+    v += G >= 16 || gl >= dist ? o : 0.0;
+  };
+  from(1, [](uint64_t b) { return dpp0_u64<DPP_ROW_SHR1, 0xF>(b); });
+  if (G >= 4) from(2, [](uint64_t b) { return dpp0_u64<DPP_ROW_SHR2, 0xF>(b); });
+  if (G >= 8) from(4, [](uint64_t b) { return dpp0_u64<DPP_ROW_SHR4, 0xF>(b); });
+  if (G >= 16) from(8, [](uint64_t b) { return dpp0_u64<DPP_ROW_SHR8, 0xF>(b); });
+  if (G >= 32) from(16, [](uint64_t b) { return dpp0_u64<DPP_ROW_BCAST15, 0xA>(b); });
+  if (G >= 64) from(32, [](uint64_t b) { return dpp0_u64<DPP_ROW_BCAST31, 0xC>(b); });
+  return v;
+}
+__device__ __forceinline__ double wave_scan_f64(double v) { return group_scan_f64<64>(v); }
+__device__ __forceinline__ double lane_f64(double v, int lane) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+// max(|t|, m) in one instruction (fmax would quieten its operands first; neither is a NaN here).
+__device__ __forceinline__ double max_abs_f64(double t, double m) {
+  double x;
+  asm("v_max_f64 %0, |%1|, %2" : "=v"(x) : "v"(t), "v"(m));
+  return x;
+}
+
 // ---------------------------------------------------------------- 2..32 lanes per row
 // G lanes share one row of at most PER * G slots; every lane holds PER consecutive weights, so a
 // wavefront carries 64 / G rows and the per-row steps that do not depend on the row length (exact
-// sum, ledger, scans) are paid once per 64 / G rows.  Prefix sums run over the group by DPP; SL and
-// SH of every slot go to a per-group LDS strip padded to PER * G slots (slots outside the row add
-// nothing), which each entry then searches once with a fixed number of probes; the heavies' slots,
-// compacted by rank, give "next heavy" and "last heavy".  The rank rides in bits 52..63 of the SH scan.
+// sum, ledger, scans) are paid once per 64 / G rows.  The rows are paired by a merge, as merge_row below does it: lights' prefix
+// sums from the front of the row's strip in LDS, heavies' from its back, a sentinel after each; a lane finds by a search along the
+// diagonal where its PER merged elements start and walks them.  A step leaves, for the light it takes, how many heavies
+// come before the next light (whose alias that heavy is), and for the heavy it takes the residual that its light leaves.
+// Slots behind the row have weight 0 and so come out as lights of a whole bucket's deficit that rank after the row's own;
+// a heavy that only they reach has a surplus prefix above the row's own deficits.
+// (One search per entry over both prefix arrays took 131 to 153 instructions an entry.)
 // Every lane of the wavefront must call this together (DPP); a group without a row passes d = 0.
-// s_pre: [2 * BLOCK * PER] u64 ([0, BLK): SL of every slot of the block; [BLK, 2 * BLK): SH), s_hs: [BLOCK * PER]
-// (per group: row-local slot of its h-th heavy).  Returns false for a row whose weights sum to zero.
-constexpr uint64_t GROUP_CNT = 1ull << 52;
+// `smem`: group_lds_bytes(G, PER, BLOCK) of LDS for the BLOCK threads that call it.  Returns false for a row whose
+// weights sum to zero.
+constexpr size_t group_lds_bytes(int G, int PER, int BLOCK) { return (size_t)(BLOCK / G) * (G * PER + 2) * 13; }
 
 template <int G, int PER, int BLOCK = 256>
 __device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const float* __restrict__ wgt,
-                                                AliasEntry* __restrict__ table, uint64_t* __restrict__ s_pre,
-                                                uint8_t* __restrict__ s_hs, uint32_t tid = threadIdx.x) {
+                                                AliasEntry* __restrict__ table, void* __restrict__ smem, uint32_t tid = threadIdx.x) {
   static_assert(PER >= 4 && PER <= 6, "a lane loads one float4 (and one float), or three float2");
-  constexpr uint32_t SLOTS = PER * G;
-  constexpr uint32_t HB = PER == 4 ? SLOTS : PER == 5 ? SLOTS / 5 * 4 : SLOTS / 3 * 2;  // largest power of two <= SLOTS
-  static_assert((HB & (HB - 1)) == 0 && HB <= SLOTS && 2 * HB > SLOTS && SLOTS <= 256, "G is a power of two");
-  constexpr uint32_t BLK = BLOCK * PER;                      // slots of one block's strips (BLOCK threads)
-  const int gl = tid & (G - 1);
-  const int lane = tid & 63;
-  const uint32_t gbase = (uint32_t)PER * (tid - gl);  // first LDS slot of the group
+  constexpr uint32_t SLOTS = PER * G, STRIDE = SLOTS + 2, TOP = SLOTS + 1, STRIPS = BLOCK / G * STRIDE;
+  static_assert(SLOTS <= 256, "slots in 8 bits");
+  // Byte offsets into the prefix sums, `at` below, tell the place of everything else: the word of a light or a heavy lies at half
+  // the offset behind them, the slot of heavy h at an eighth of the offset of index h behind those.
+  char* const s_v = reinterpret_cast<char*>(smem);  // per row [STRIDE]: light r at r, heavy h at TOP - h
+  char* const s_w = s_v + STRIPS * 8;               // [STRIDE]: light r: offset of its alias' rank; heavy h: its residual
+  char* const s_hs = s_w + STRIPS * 4;              // [STRIDE]: slot of heavy h
+  auto val = [&](uint32_t at) -> double& { return *reinterpret_cast<double*>(s_v + at); };
+  auto word = [&](uint32_t at) -> uint32_t& { return *reinterpret_cast<uint32_t*>(s_w + (at >> 1)); };
+  auto slot_of = [&](uint32_t at) -> uint8_t& { return *reinterpret_cast<uint8_t*>(s_hs + (at >> 3)); };
+  const uint32_t gl = tid & (G - 1), lane = tid & 63;
+  const uint32_t g8 = 8u * STRIDE * (tid / G);  // offset of the row's strip
   const uint32_t pos = (uint32_t)PER * gl;
+  const uint32_t last_lane = lane - gl + G - 1;
 
   float xs[PER];
 #pragma unroll
@@ -152,17 +192,14 @@ __device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const 
       }
   }
   if (PER % 2 == 1 && pos + PER - 1 < d) xs[PER - 1] = wgt[off + pos + PER - 1];
-  double wd[PER];
-  uint32_t live = 0;
+  double wd[PER];  // clamped weights, then the amounts
   // the sum of the row as a plain fp64 sum where that is exact (plain_sum_is_exact); a wavefront in which some
   // group's is not falls back to the three-limb sum for all of its groups
   double Sd = 0.0;
   uint32_t mn = 0xFFFFFFFFu;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const bool in = pos + k < d;
-    if (in) live |= 1u << k;
-    const float cw = masked_weight(xs[k], in);
+    const float cw = masked_weight(xs[k], pos + k < d);
     wd[k] = (double)cw;
     Sd += wd[k];
     mn = min(mn, __float_as_uint(cw) - 1u);
@@ -178,79 +215,105 @@ __device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const 
     if (!plain) Sd = S.top + S.mid + S.low != 0.0 ? wsum3_to_double(S) : 0.0;
   }
   const bool row_ok = Sd != 0.0;
-  Ledger L = make_ledger_small(d, Sd);
-  if (!row_ok) L.scale = 0.0;
-  const double neg_fs = -L.fs;
+  const double scale = row_ok ? (double)d / Sd : 0.0;
+  double fs = 1099511627776.0, neg_fs = -1099511627776.0;  // 2^40
+  asm("" : "+v"(fs), "+v"(neg_fs));  // in registers: as literals they would be moved into every sum's place
 
-  uint64_t dl[PER], sl[PER], sh[PER];
   float op[PER];
-  uint32_t heavy = 0;
-  uint64_t ra = 0, rb = 0;
+  bool hv[PER];
+  double run = 0.0, run_u = 0.0;  // amounts of this lane's slots, of its heavies
+  uint32_t cnt = 0;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
-    const Entry e = classify_small_fma(wd[k], L, neg_fs);
-    dl[k] = (e.heavy || !((live >> k) & 1)) ? 0 : e.amount;
-    ra += dl[k];
-    rb += e.heavy ? (e.amount | GROUP_CNT) : 0;
-    sl[k] = ra;
-    sh[k] = rb;
-    op[k] = (float)e.p;
-    if (e.heavy) heavy |= 1u << k;
+    const double p = wd[k] * scale, t = fma(p, fs, neg_fs);  // = (p - 1) * 2^F rounded once: the product is exact
+    hv[k] = t >= 0.5;
+    wd[k] = rint(max_abs_f64(t, hv[k] ? 1.0 : 0.0));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
+    op[k] = (float)p;
+    run += wd[k];
+    run_u += hv[k] ? wd[k] : 0.0;
+    cnt += hv[k] ? 1u : 0u;
   }
-  const uint64_t ia = group_scan_u64<G>(ra), ib = group_scan_u64<G>(rb);
-  const uint32_t nh = (uint32_t)(shfl_u64(ib, (lane - gl) + G - 1) >> 52);
+  const double i = group_scan_f64<G>(run), iu = group_scan_f64<G>(run_u);
+  const uint32_t ic = group_scan_u32<G>(cnt);
+  const uint32_t nh = (uint32_t)__shfl((int)ic, (int)last_lane, 64);
+  // the deficits of the row's own lights: a slot behind the row counts 2^40
+  const double own = __longlong_as_double((long long)shfl_u64((uint64_t)__double_as_longlong(i - iu), (int)last_lane)) +
+                     (double)(SLOTS - d) * neg_fs;
+  const uint32_t nl = SLOTS - nh;
+  const uint32_t ex_c = ic - cnt;
+  uint32_t at[PER];  // of the slot's prefix sum
+  bool self[PER];    // a heavy that is the row's last or that no light finishes
+  {
+    uint32_t la = g8 + 8u * (pos - ex_c), ha = g8 + 8u * (TOP - ex_c), hs = g8 + 8u * ex_c;
+    const uint32_t last = g8 + 8u * (nh - 1);
+    double sh = iu - run_u, sl = i - run - sh;
 #pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    sl[k] += ia - ra;
-    sh[k] += ib - rb;
-    s_pre[gbase + pos + k] = sl[k];
-    s_pre[BLK + gbase + pos + k] = sh[k] & (GROUP_CNT - 1);
-    if ((heavy >> k) & 1) s_hs[gbase + (uint32_t)(sh[k] >> 52) - 1] = (uint8_t)(pos + k);
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-  // light: first slot with SH > SL - D.  heavy: first slot with SL >= SH, i.e. SL > SH - 1.
-  // The first probe narrows the answer to a window of HB slots that ends inside the strip.
-  uint32_t arr[PER], at[PER];
-  uint64_t key[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const bool hv = (heavy >> k) & 1;
-    arr[k] = gbase + (hv ? 0u : BLK);
-    key[k] = hv ? (sh[k] & (GROUP_CNT - 1)) - 1 : sl[k] - dl[k];
-    at[k] = HB == SLOTS ? 0u : (s_pre[arr[k] + HB - 1] <= key[k] ? SLOTS - HB : 0u);
-  }
-#pragma unroll
-  for (uint32_t step = HB / 2; step >= 1; step >>= 1) {
-    uint64_t v[PER];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) v[k] = s_pre[arr[k] + at[k] + step - 1];
-#pragma unroll
-    for (int k = 0; k < PER; ++k) at[k] += v[k] <= key[k] ? step : 0u;
-  }
-  uint32_t oa[PER];
-#pragma unroll
-  for (int k = 0; k < PER; ++k) {
-    const uint64_t v = s_pre[arr[k] + at[k]];
-    const bool found = v > key[k];
-    const uint32_t self = pos + k;
-    if (!((heavy >> k) & 1)) {
-      oa[k] = found ? at[k] : (nh ? (uint32_t)s_hs[gbase + nh - 1] : self);
-    } else {
-      const uint32_t hc = (uint32_t)(sh[k] >> 52);
-      if (hc < nh && found) {
-        op[k] = residual_prob(L.one + key[k] + 1 - v, L);
-        oa[k] = s_hs[gbase + hc];
+    for (int k = 0; k < PER; ++k) {
+      at[k] = hv[k] ? ha : la;
+      self[k] = false;
+      if (hv[k]) {
+        sh += wd[k];
+        val(ha) = sh;
+        slot_of(hs) = (uint8_t)(pos + k);
+        self[k] = hs == last || sh > own;
+        ha -= 8u;
+        hs += 8u;
       } else {
-        op[k] = 1.0f;
-        oa[k] = self;
+        sl += wd[k];
+        val(la) = sl;
+        la += 8u;
       }
     }
-    if (!row_ok) {
-      op[k] = 0.0f;
-      oa[k] = SKY_INVALID;
+    if (gl == G - 1) {
+      val(g8 + 8u * nl) = __builtin_huge_val();
+      val(g8 + 8u * (TOP - nh)) = __builtin_huge_val();
+    }
+    if (gl == 0) word(g8) = g8;  // the first light starts in the first heavy
+  }
+  wave_lds_sync();
+
+  // merged positions [pos, pos + PER) belong to this lane; a lights and pos - a heavies come before them
+  uint32_t a8;
+  {
+    const uint32_t hi8 = g8 + 8u * min(pos, nl), dh = 8u * (TOP - pos);
+    a8 = g8 + 8u * (pos > nh ? pos - nh : 0u);
+#pragma unroll
+    for (uint32_t step = 1u << (31 - __builtin_clz(SLOTS / 2)); step >= 1; step >>= 1) {
+      const uint32_t to = a8 + 8u * step;
+      const bool up = val(to - 8u) < val(to + dh);
+      a8 = up && to <= hi8 ? to : a8;
+    }
+  }
+  {
+    const uint32_t dh = 8u * (TOP - pos - (PER - 1));  // the heavy at hand lies so far behind the light at hand, and 8 bytes less in every step
+    uint32_t h2 = 8u * (TOP - pos), k8 = 2u * g8 + 8u * pos;
+#pragma unroll
+    for (int s = 0; s < PER; ++s) {
+      const double vl = val(a8), vh = val(a8 + dh + 8u * (PER - 1 - s));
+      const bool take = vh <= vl;  // the heavy
+      const float p = (float)fma(vl - vh, -1.0 / 1099511627776.0, 1.0);
+      word(a8 + (take ? h2 : 8u)) = take ? __float_as_uint(p) : k8 - a8;
+      a8 += take ? 0u : 8u;
+      h2 -= 8u;
+      k8 += 8u;
+    }
+  }
+  wave_lds_sync();
+
+  uint32_t oa[PER];
+  {
+    const uint32_t last = g8 + 8u * (nh - 1), k2 = 2u * g8 + 8u * (TOP + 1);
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+      const uint32_t x = word(at[k]);
+      // a light beyond every heavy takes the last
+      const uint32_t m = slot_of(hv[k] ? k2 - at[k] : min(x, last));
+      oa[k] = (hv[k] ? self[k] : nh == 0) ? pos + k : m;
+      if (hv[k]) op[k] = self[k] ? 1.0f : __uint_as_float(x);
+      if (!row_ok) {
+        op[k] = 0.0f;
+        oa[k] = SKY_INVALID;
+      }
     }
   }
   // the next row of this group reuses the strips: its writes must stay behind these reads
@@ -258,17 +321,16 @@ __device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const 
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
   for (int h = 0; h < PER / 2; ++h) {
-    const uint32_t m = (live >> (2 * h)) & 3u;
     AliasEntry* t = table + off + pos + 2 * h;
-    if (m == 3u) {
+    if (pos + 2 * h + 1 < d) {
       uint4u o;
       o.x = __float_as_uint(op[2 * h]); o.y = oa[2 * h]; o.z = __float_as_uint(op[2 * h + 1]); o.w = oa[2 * h + 1];
       *reinterpret_cast<uint4u*>(t) = o;
-    } else if (m == 1u) {
+    } else if (pos + 2 * h < d) {
       t[0] = AliasEntry{op[2 * h], oa[2 * h]};
     }
   }
-  if (PER % 2 == 1 && ((live >> (PER - 1)) & 1)) table[off + pos + PER - 1] = AliasEntry{op[PER - 1], oa[PER - 1]};
+  if (PER % 2 == 1 && pos + PER - 1 < d) table[off + pos + PER - 1] = AliasEntry{op[PER - 1], oa[PER - 1]};
   return row_ok || d == 0;
 }
 
@@ -316,16 +378,17 @@ __device__ __forceinline__ bool tiny_row(uint32_t off, uint32_t d, const float* 
 constexpr uint32_t SMALL_RANGE = 1024;  // most vertices per wavefront
 constexpr uint32_t SMALL_QBASE[4] = {0, 128, 224, 304};
 constexpr uint32_t SMALL_QTOTAL = 376;
-constexpr size_t SMALL_LDS_BYTES = 2 * 64 * 4 * 8 + 64 * 4 + SMALL_QTOTAL * 6;
+constexpr size_t SMALL_STRIPS = 4176;  // strips of the groups, the largest of three
+static_assert(SMALL_STRIPS >= group_lds_bytes(2, 4, 64) && SMALL_STRIPS >= group_lds_bytes(4, 4, 64) &&
+              SMALL_STRIPS >= group_lds_bytes(8, 4, 64) && SMALL_STRIPS % 8 == 0, "every group size fits");
+constexpr size_t SMALL_LDS_BYTES = SMALL_STRIPS + SMALL_QTOTAL * 6;
 // Vertices [lo, lo + per_wave) of the n (src null: the vertices themselves) by one wavefront that is a workgroup.
 __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __restrict__ xadj, const float* __restrict__ wgt,
                                                  const uint32_t* __restrict__ src, uint32_t n, uint32_t per_wave,
                                                  AliasEntry* __restrict__ table, int8_t* __restrict__ valid,
                                                  uint64_t* __restrict__ smem) {
-  uint64_t* s_pre = smem;                                           // [2 * 64 * 4]
-  uint32_t* q_off = reinterpret_cast<uint32_t*>(smem + 2 * 64 * 4);  // [SMALL_QTOTAL]
+  uint32_t* q_off = reinterpret_cast<uint32_t*>(smem + SMALL_STRIPS / 8);  // [SMALL_QTOTAL]
   uint16_t* q_it = reinterpret_cast<uint16_t*>(q_off + SMALL_QTOTAL);  // [SMALL_QTOTAL]
-  uint8_t* s_hs = reinterpret_cast<uint8_t*>(q_it + SMALL_QTOTAL);   // [64 * 4]
   const uint32_t lane = threadIdx.x;
   const uint32_t hi = min(n, lo + per_wave);
   uint32_t cnt[4] = {0, 0, 0, 0};  // wave-uniform queue lengths: rows of 1..2, 3..8, 9..16, 17..32 entries
@@ -359,21 +422,21 @@ __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __
   auto build_g2 = [&](uint32_t rows) {
     uint32_t t, off, it, d;
     take(1, rows, 2, t, off, it, d);
-    const bool ok = group_build_row<2, 4, 64>(off, d, wgt, table, s_pre, s_hs, t);
+    const bool ok = group_build_row<2, 4, 64>(off, d, wgt, table, smem, t);
     if ((t & 1) == 0 && !ok) clear_valid(it);
     cnt[1] -= rows;
   };
   auto build_g4 = [&](uint32_t rows) {
     uint32_t t, off, it, d;
     take(2, rows, 4, t, off, it, d);
-    const bool ok = group_build_row<4, 4, 64>(off, d, wgt, table, s_pre, s_hs, t);
+    const bool ok = group_build_row<4, 4, 64>(off, d, wgt, table, smem, t);
     if ((t & 3) == 0 && !ok) clear_valid(it);
     cnt[2] -= rows;
   };
   auto build_g8 = [&](uint32_t rows) {
     uint32_t t, off, it, d;
     take(3, rows, 8, t, off, it, d);
-    const bool ok = group_build_row<8, 4, 64>(off, d, wgt, table, s_pre, s_hs, t);
+    const bool ok = group_build_row<8, 4, 64>(off, d, wgt, table, smem, t);
     if ((t & 7) == 0 && !ok) clear_valid(it);
     cnt[3] -= rows;
   };
@@ -438,8 +501,7 @@ __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __
 // walks it.
 //
 // What bounds it is vector instructions, so
-// - prefix sums are doubles: whole numbers below 2^53 in a row of at most 2^13 slots.  An amount is one rounding instead of
-//   an addition and a mask, a residual one fused multiply-add instead of a conversion;
+// - prefix sums are doubles (above);
 // - slots behind the row's end in its last wavefront have weight 0 and go along as lights of deficit 2^40.  They come
 //   after every light of the row, in rank and in the merged order, so nothing of the row depends on them, and no step
 //   needs a mask; a heavy that only one of them reaches is one that nobody finishes;
@@ -456,30 +518,6 @@ constexpr int merge_resident(int rowt, int per, int bytes) {
 }
 constexpr bool merge_narrow(int rowt, int per) { return rowt == 64 || merge_resident(rowt, per, 12) > merge_resident(rowt, per, 14); }
 constexpr size_t merge_lds_bytes(int rowt, int per) { return ((size_t)rowt * per + 2) * (merge_narrow(rowt, per) ? 12 : 14); }
-
-// Inclusive prefix sum over the wavefront.
-__device__ __forceinline__ double wave_scan_f64(double v) {
-  auto from = [&](auto get) { v += __longlong_as_double((long long)get((uint64_t)__double_as_longlong(v))); };
-  from([](uint64_t b) { return dpp0_u64<DPP_ROW_SHR1, 0xF>(b); });
-  from([](uint64_t b) { return dpp0_u64<DPP_ROW_SHR2, 0xF>(b); });
-  from([](uint64_t b) { return dpp0_u64<DPP_ROW_SHR4, 0xF>(b); });
-  from([](uint64_t b) { return dpp0_u64<DPP_ROW_SHR8, 0xF>(b); });
-  from([](uint64_t b) { return dpp0_u64<DPP_ROW_BCAST15, 0xA>(b); });
-  from([](uint64_t b) { return dpp0_u64<DPP_ROW_BCAST31, 0xC>(b); });
-  return v;
-}
-__device__ __forceinline__ double lane_f64(double v, int lane) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v);
-  const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
-  const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
-  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-}
-// max(|t|, m) in one instruction (fmax would quieten its operands first; neither is a NaN here).
-__device__ __forceinline__ double max_abs_f64(double t, double m) {
-  double x;
-  asm("v_max_f64 %0, |%1|, %2" : "=v"(x) : "v"(t), "v"(m));
-  return x;
-}
 
 // The row `rr` by ROWT threads that share `smem` and, for the wavefronts' sums, s_aux[8 * ROWT / 64].  Returns false when its weights sum to zero.  All threads of the
 // workgroup call it together; the arrays in LDS may be rewritten only after a barrier.
