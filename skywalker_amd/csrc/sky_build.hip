@@ -962,13 +962,13 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     }
   }
 
-  SKY_TRY(grp(CLS_G2, build_group_kernel<2, 4>, 2, "g2"));
-  SKY_TRY(grp(CLS_G4, build_group_kernel<4, 4>, 4, "g4"));
-  SKY_TRY(grp(CLS_G8, build_group_kernel<8, 4>, 8, "g8"));
-  SKY_TRY(grp(CLS_G16, build_group_kernel<16, 4>, 16, "g16"));
-  SKY_TRY(grp(CLS_G32, build_group_kernel<32, 4>, 32, "g32"));
-  SKY_TRY(grp(CLS_G32S, build_group_kernel<32, 5>, 32, "g32s"));
-  SKY_TRY(grp(CLS_G32X, build_group_kernel<32, 6>, 32, "g32x"));
+  SKY_TRY(grp(CLS_G2, build_group_kernel<SHAPE_G2.lanes, SHAPE_G2.per>, SHAPE_G2.lanes, "g2"));
+  SKY_TRY(grp(CLS_G4, build_group_kernel<SHAPE_G4.lanes, SHAPE_G4.per>, SHAPE_G4.lanes, "g4"));
+  SKY_TRY(grp(CLS_G8, build_group_kernel<SHAPE_G8.lanes, SHAPE_G8.per>, SHAPE_G8.lanes, "g8"));
+  SKY_TRY(grp(CLS_G16, build_group_kernel<SHAPE_G16.lanes, SHAPE_G16.per>, SHAPE_G16.lanes, "g16"));
+  SKY_TRY(grp(CLS_G32, build_group_kernel<SHAPE_G32.lanes, SHAPE_G32.per>, SHAPE_G32.lanes, "g32"));
+  SKY_TRY(grp(CLS_G32S, build_group_kernel<SHAPE_G32S.lanes, SHAPE_G32S.per>, SHAPE_G32S.lanes, "g32s"));
+  SKY_TRY(grp(CLS_G32X, build_group_kernel<SHAPE_G32X.lanes, SHAPE_G32X.per>, SHAPE_G32X.lanes, "g32x"));
 
   // the lists HOLD, STREAM, STREAM_LAST, STREAM_WIDE, HUGE lie back to back (the class numbers between are unused)
   const uint32_t held_rows = row_merge ? 0 : counts[CLS_HOLD];

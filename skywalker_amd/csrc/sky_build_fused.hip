@@ -268,7 +268,7 @@ __device__ __forceinline__ void merge_unit(const FusedArgs& a, const SectionRef&
 }
 
 constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
-constexpr size_t WAVE_LDS = cmax(cmax(SMALL_LDS_BYTES, group_lds_bytes(32, 6, 64)), merge_lds_bytes(64, 8));
+constexpr size_t WAVE_LDS = cmax(cmax(SMALL_LDS_BYTES, group_lds_bytes(SHAPE_G32X.lanes, SHAPE_G32X.per, 64)), merge_lds_bytes(64, 8));
 
 // The second launch bounds: what LDS lets reside anyway (21 wavefronts, 10 pairs, 4 workgroups of 256 to a CU).  Left alone the
 // device-sized kernels took 109, 104 and 132 registers, one workgroup in five and one in four less (the 134,652 rows of a
@@ -294,13 +294,13 @@ __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
           if (row_at<DEV>(a, s, unit * 64 + threadIdx.x, rows, rr)) a.valid[rr.v] = tiny_row(rr.off, rr.d, a.wgt, a.table) ? 1 : 0;
         }
         break;
-      case SEC_G2: if constexpr (DEV) group_unit<DEV, 2, 4>(a, s, unit, rows, smem); break;
-      case SEC_G4: if constexpr (DEV) group_unit<DEV, 4, 4>(a, s, unit, rows, smem); break;
-      case SEC_G8: if constexpr (DEV) group_unit<DEV, 8, 4>(a, s, unit, rows, smem); break;
-      case SEC_G16: group_unit<DEV, 16, 4>(a, s, unit, rows, smem); break;
-      case SEC_G32: group_unit<DEV, 32, 4>(a, s, unit, rows, smem); break;
-      case SEC_G32S: group_unit<DEV, 32, 5>(a, s, unit, rows, smem); break;
-      case SEC_G32X: group_unit<DEV, 32, 6>(a, s, unit, rows, smem); break;
+      case SEC_G2: if constexpr (DEV) group_unit<DEV, SHAPE_G2.lanes, SHAPE_G2.per>(a, s, unit, rows, smem); break;
+      case SEC_G4: if constexpr (DEV) group_unit<DEV, SHAPE_G4.lanes, SHAPE_G4.per>(a, s, unit, rows, smem); break;
+      case SEC_G8: if constexpr (DEV) group_unit<DEV, SHAPE_G8.lanes, SHAPE_G8.per>(a, s, unit, rows, smem); break;
+      case SEC_G16: group_unit<DEV, SHAPE_G16.lanes, SHAPE_G16.per>(a, s, unit, rows, smem); break;
+      case SEC_G32: group_unit<DEV, SHAPE_G32.lanes, SHAPE_G32.per>(a, s, unit, rows, smem); break;
+      case SEC_G32S: group_unit<DEV, SHAPE_G32S.lanes, SHAPE_G32S.per>(a, s, unit, rows, smem); break;
+      case SEC_G32X: group_unit<DEV, SHAPE_G32X.lanes, SHAPE_G32X.per>(a, s, unit, rows, smem); break;
       case SEC_W1: merge_unit<DEV, 64, 4>(a, s, unit, rows, smem, s_aux); break;
       case SEC_W6: merge_unit<DEV, 64, 6>(a, s, unit, rows, smem, s_aux); break;
       case SEC_W2: merge_unit<DEV, 64, 8>(a, s, unit, rows, smem, s_aux); break;
@@ -649,10 +649,10 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   if (min_degree == 0) wave.add(SEC_SWEEP, g->V, base.per_wave, 0);
   wave.add(SEC_W6, rows(CLS_LDS_W6), 1, p.start[CLS_LDS_W6]);
   wave.add(SEC_W1, rows(CLS_LDS_W1), 1, p.start[CLS_LDS_W1]);
-  wave.add(SEC_G32X, rows(CLS_G32X), 2, p.start[CLS_G32X]);
-  wave.add(SEC_G32S, rows(CLS_G32S), 2, p.start[CLS_G32S]);
-  wave.add(SEC_G32, rows(CLS_G32), 2, p.start[CLS_G32]);
-  wave.add(SEC_G16, rows(CLS_G16), 4, p.start[CLS_G16]);
+  wave.add(SEC_G32X, rows(CLS_G32X), 64 / SHAPE_G32X.lanes, p.start[CLS_G32X]);
+  wave.add(SEC_G32S, rows(CLS_G32S), 64 / SHAPE_G32S.lanes, p.start[CLS_G32S]);
+  wave.add(SEC_G32, rows(CLS_G32), 64 / SHAPE_G32.lanes, p.start[CLS_G32]);
+  wave.add(SEC_G16, rows(CLS_G16), 64 / SHAPE_G16.lanes, p.start[CLS_G16]);
   pair.add(SEC_TOTALS, n_tiles, 2, 0);
   pair.add(SEC_P8, rows(CLS_MW2), 1, p.start[CLS_MW2]);
   pair.add(SEC_P6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
@@ -713,13 +713,13 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, con
   add(wave, SEC_W2, 1, CLS_LDS_W2);
   add(wave, SEC_W6, 1, CLS_LDS_W6);
   add(wave, SEC_W1, 1, CLS_LDS_W1);
-  add(wave, SEC_G32X, 2, CLS_G32X);
-  add(wave, SEC_G32S, 2, CLS_G32S);
-  add(wave, SEC_G32, 2, CLS_G32);
-  add(wave, SEC_G16, 4, CLS_G16);
-  add(wave, SEC_G8, 8, CLS_G8);
-  add(wave, SEC_G4, 16, CLS_G4);
-  add(wave, SEC_G2, 32, CLS_G2);
+  add(wave, SEC_G32X, 64 / SHAPE_G32X.lanes, CLS_G32X);
+  add(wave, SEC_G32S, 64 / SHAPE_G32S.lanes, CLS_G32S);
+  add(wave, SEC_G32, 64 / SHAPE_G32.lanes, CLS_G32);
+  add(wave, SEC_G16, 64 / SHAPE_G16.lanes, CLS_G16);
+  add(wave, SEC_G8, 64 / SHAPE_G8.lanes, CLS_G8);
+  add(wave, SEC_G4, 64 / SHAPE_G4.lanes, CLS_G4);
+  add(wave, SEC_G2, 64 / SHAPE_G2.lanes, CLS_G2);
   add(wave, SEC_TINY, 64, CLS_TINY);
   pair.add(SEC_TOTALS, n_tiles, 2, 0);
   add(pair, SEC_P8, 1, CLS_MW2);

@@ -68,11 +68,6 @@ __device__ __forceinline__ RawChunk fetch_chunk(const float* __restrict__ wgt, c
   }
   return x;
 }
-template <int PERM>
-__device__ __forceinline__ uint32_t quad_get(uint32_t x) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, PERM, 0xF, 0xF, true);
-}
-constexpr int quad_perm(int a, int b, int c, int d) { return a | b << 2 | c << 4 | d << 6; }
 // The thread's own 8 slots: quarter q of lane i of a quad was loaded as quarter i >> 1 of lane 2 * (i & 1) + q.  All lanes of the
 // wavefront call it together.
 __device__ __forceinline__ RawChunk own_slots(const RawChunk& x, int tid) {
@@ -93,30 +88,8 @@ __device__ __forceinline__ RawChunk own_slots(const RawChunk& x, int tid) {
 }
 // The wavefront's 512 entries, all of which are written: t is where this thread's first one lies.
 __device__ __forceinline__ void quad_store(AliasEntry* t, int tid, const float (&p)[ST_PER], const uint32_t (&a)[ST_PER]) {
-  uint32_t v[4][4];  // [pair of entries][word]; afterwards [lane of the quad]: pair tid & 3 of that lane
-#pragma unroll
-  for (int h = 0; h < 4; ++h) {
-    v[h][0] = __float_as_uint(p[2 * h]);
-    v[h][1] = a[2 * h];
-    v[h][2] = __float_as_uint(p[2 * h + 1]);
-    v[h][3] = a[2 * h + 1];
-  }
-  const bool b0 = tid & 1, b1 = tid & 2;
-  auto swap = [&](auto perm, bool odd, uint32_t& lo, uint32_t& hi) {  // a 2 x 2 transpose between partner lanes
-    constexpr int P = decltype(perm)::value;
-    const uint32_t from_lo = quad_get<P>(lo), from_hi = quad_get<P>(hi);
-    lo = odd ? from_hi : lo;
-    hi = odd ? hi : from_lo;
-  };
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    using X1 = std::integral_constant<int, quad_perm(1, 0, 3, 2)>;
-    using X2 = std::integral_constant<int, quad_perm(2, 3, 0, 1)>;
-    swap(X1{}, b0, v[0][w], v[1][w]);
-    swap(X1{}, b0, v[2][w], v[3][w]);
-    swap(X2{}, b1, v[0][w], v[2][w]);
-    swap(X2{}, b1, v[1][w], v[3][w]);
-  }
+  uint32_t v[4][4];
+  quad_exchange(tid, p, a, v);
   AliasEntry* const t0 = t - 8 * (tid & 3) + 2 * (tid & 3);
 #pragma unroll
   for (int h = 0; h < 4; ++h)

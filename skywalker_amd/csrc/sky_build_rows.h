@@ -108,6 +108,40 @@ __device__ __forceinline__ void wave_store(AliasEntry* __restrict__ dst, uint32_
   }
 }
 
+// ---------------------------------------------------------------- slots of a quad of lanes
+template <int PERM>
+__device__ __forceinline__ uint32_t quad_get(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, PERM, 0xF, 0xF, true);
+}
+constexpr int quad_perm(int a, int b, int c, int d) { return a | b << 2 | c << 4 | d << 6; }
+// The lanes of a quad exchange the entries of their 8 consecutive slots each: v[l] becomes pair tid & 3 of those of the quad's lane
+// l, so that one 16-byte store a lane moves 64 bytes in a row.  All lanes of the wavefront call it together.
+__device__ __forceinline__ void quad_exchange(uint32_t tid, const float (&p)[8], const uint32_t (&a)[8], uint32_t (&v)[4][4]) {
+#pragma unroll
+  for (int h = 0; h < 4; ++h) {
+    v[h][0] = __float_as_uint(p[2 * h]);
+    v[h][1] = a[2 * h];
+    v[h][2] = __float_as_uint(p[2 * h + 1]);
+    v[h][3] = a[2 * h + 1];
+  }
+  const bool b0 = tid & 1, b1 = tid & 2;
+  auto swap = [&](auto perm, bool odd, uint32_t& lo, uint32_t& hi) {  // a 2 x 2 transpose between partner lanes
+    constexpr int P = decltype(perm)::value;
+    const uint32_t from_lo = quad_get<P>(lo), from_hi = quad_get<P>(hi);
+    lo = odd ? from_hi : lo;
+    hi = odd ? hi : from_lo;
+  };
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    using X1 = std::integral_constant<int, quad_perm(1, 0, 3, 2)>;
+    using X2 = std::integral_constant<int, quad_perm(2, 3, 0, 1)>;
+    swap(X1{}, b0, v[0][w], v[1][w]);
+    swap(X1{}, b0, v[2][w], v[3][w]);
+    swap(X2{}, b1, v[0][w], v[2][w]);
+    swap(X2{}, b1, v[1][w], v[3][w]);
+  }
+}
+
 // ---------------------------------------------------------------- sums as doubles
 // Prefix sums of a row's amounts are whole numbers below 2^53 in rows of at most 2^13 slots: doubles hold them exactly, an
 // amount is one rounding instead of an addition and a mask, a residual one fused multiply-add instead of a conversion.
@@ -133,6 +167,9 @@ __device__ __forceinline__ double lane_f64(double v, int lane) {
   const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(b >> 32), lane);
   return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
+__device__ __forceinline__ double lane_shfl_f64(double v, int lane) {
+  return __longlong_as_double((long long)shfl_u64((uint64_t)__double_as_longlong(v), lane));
+}
 // max(|t|, m) in one instruction (fmax would quieten its operands first; neither is a NaN here).
 __device__ __forceinline__ double max_abs_f64(double t, double m) {
   double x;
@@ -145,43 +182,63 @@ __device__ __forceinline__ double max_abs_f64(double t, double m) {
 // wavefront carries 64 / G rows and the per-row steps that do not depend on the row length (exact
 // sum, ledger, scans) are paid once per 64 / G rows.  The rows are paired by a merge, as merge_row below does it: lights' prefix
 // sums from the front of the row's strip in LDS, heavies' from its back, a sentinel after each; a lane finds by a search along the
-// diagonal where its PER merged elements start and walks them.  A step leaves, for the light it takes, how many heavies
-// come before the next light (whose alias that heavy is), and for the heavy it takes the residual that its light leaves.
+// diagonal where its PER merged elements start and walks them.  A step leaves, for the light it takes, which heavy is the
+// next light's alias, and for the heavy it takes the residual that its light leaves.
 // Slots behind the row have weight 0 and so come out as lights of a whole bucket's deficit that rank after the row's own;
-// a heavy that only they reach has a surplus prefix above the row's own deficits.
-// (One search per entry over both prefix arrays took 131 to 153 instructions an entry.)
+// a heavy that only they reach has a prefix sum above the deficits of the row's own lights.
+// Instruction issue bounds it (94 % of the vector units' cycles for rows of 50 that lie side by side; scattered rows of a power-law
+// graph wait for lines that they use in part).
 // Every lane of the wavefront must call this together (DPP); a group without a row passes d = 0.
 // `smem`: group_lds_bytes(G, PER, BLOCK) of LDS for the BLOCK threads that call it.  Returns false for a row whose
 // weights sum to zero.
-constexpr size_t group_lds_bytes(int G, int PER, int BLOCK) { return (size_t)(BLOCK / G) * (G * PER + 2) * 13; }
+//
+// A strip has PER * G + 2 entries: light r at index r, heavy h at index TOP - h.  Every offset that a step needs is the offset of
+// the light or the heavy at hand, or of the next one:
+//   val   prefix sum of the light or heavy; once every lane has walked its share,
+//   word  of light r: the offset of its alias' heavy.  Of index TOP - h - 1: the residual of heavy h, below its own index because
+//         the entry there also holds
+//   slot  of index TOP - h: the slot of heavy h, which is the alias of heavy h - 1 (a byte, behind the sums)
+// (16-byte entries of all three save a shift a slot and lose more to bank conflicts; words of their own cost a
+// wavefront in six its place.)
+constexpr uint32_t group_entries(int G, int PER, int BLOCK) {
+  return ((uint32_t)(BLOCK / G) * (G * PER + 2) + 2 + 7) / 8 * 8;  // one more at either end is read
+}
+constexpr size_t group_lds_bytes(int G, int PER, int BLOCK) { return (size_t)group_entries(G, PER, BLOCK) * 9; }
+
+// Lanes and slots of a lane by class.  8 slots a lane where 4 would do for twice the lanes: what a lane does once for its row (sum, division,
+// scans, search) is half of its instructions with 4.  200 M entries in rows of 100 (32 lanes of 4 / 16 of 8) 739 / 630 us, of 50
+// 720 / 640, of 24 835 / 680, of 12 880 / 850; rows of 3..8 would be one lane's.
+struct GroupShape {
+  int lanes, per;
+};
+constexpr GroupShape SHAPE_G2{2, 4}, SHAPE_G4{2, 8}, SHAPE_G8{4, 8}, SHAPE_G16{8, 8}, SHAPE_G32{16, 8}, SHAPE_G32S{32, 5}, SHAPE_G32X{32, 6};
 
 template <int G, int PER, int BLOCK = 256>
 __device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const float* __restrict__ wgt,
                                                 AliasEntry* __restrict__ table, void* __restrict__ smem, uint32_t tid = threadIdx.x) {
-  static_assert(PER >= 4 && PER <= 6, "a lane loads one float4 (and one float), or three float2");
-  constexpr uint32_t SLOTS = PER * G, STRIDE = SLOTS + 2, TOP = SLOTS + 1, STRIPS = BLOCK / G * STRIDE;
+  static_assert((PER >= 4 && PER <= 6) || PER == 8, "a lane loads one float4 (and one float), two, or three float2");
+  constexpr uint32_t SLOTS = PER * G, STRIDE = SLOTS + 2, TOP = SLOTS + 1;
   static_assert(SLOTS <= 256, "slots in 8 bits");
-  // Byte offsets into the prefix sums, `at` below, tell the place of everything else: the word of a light or a heavy lies at half
-  // the offset behind them, the slot of heavy h at an eighth of the offset of index h behind those.
-  char* const s_v = reinterpret_cast<char*>(smem);  // per row [STRIDE]: light r at r, heavy h at TOP - h
-  char* const s_w = s_v + STRIPS * 8;               // [STRIDE]: light r: offset of its alias' rank; heavy h: its residual
-  char* const s_hs = s_w + STRIPS * 4;              // [STRIDE]: slot of heavy h
+  constexpr uint32_t SZ = 8, N = group_entries(G, PER, BLOCK);
+  char* const s_v = reinterpret_cast<char*>(smem);
   auto val = [&](uint32_t at) -> double& { return *reinterpret_cast<double*>(s_v + at); };
-  auto word = [&](uint32_t at) -> uint32_t& { return *reinterpret_cast<uint32_t*>(s_w + (at >> 1)); };
-  auto slot_of = [&](uint32_t at) -> uint8_t& { return *reinterpret_cast<uint8_t*>(s_hs + (at >> 3)); };
+  auto word = [&](uint32_t at) -> uint32_t& { return *reinterpret_cast<uint32_t*>(s_v + at); };
+  auto slot_of = [&](uint32_t at) -> uint8_t& { return *reinterpret_cast<uint8_t*>(s_v + N * 8 + (at >> 3)); };
   const uint32_t gl = tid & (G - 1), lane = tid & 63;
-  const uint32_t g8 = 8u * STRIDE * (tid / G);  // offset of the row's strip
+  const uint32_t strip = SZ * (STRIDE * (tid / G) + 1);  // its offset
   const uint32_t pos = (uint32_t)PER * gl;
   const uint32_t last_lane = lane - gl + G - 1;
 
   float xs[PER];
 #pragma unroll
   for (int k = 0; k < PER; ++k) xs[k] = 0.0f;
-  if (PER == 4 || PER == 5) {
-    if (pos < d) {
-      const float4u x = *reinterpret_cast<const float4u*>(wgt + off + pos);
-      xs[0] = x.x; xs[1] = x.y; xs[2] = x.z; xs[3] = x.w;
-    }
+  if (PER != 6) {
+#pragma unroll
+    for (int h = 0; h < PER / 4; ++h)
+      if (pos + 4 * h < d) {
+        const float4u x = *reinterpret_cast<const float4u*>(wgt + off + pos + 4 * h);
+        xs[4 * h] = x.x; xs[4 * h + 1] = x.y; xs[4 * h + 2] = x.z; xs[4 * h + 3] = x.w;
+      }
   } else {
 #pragma unroll
     for (int h = 0; h < PER / 2; ++h)
@@ -227,110 +284,113 @@ __device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const 
   for (int k = 0; k < PER; ++k) {
     const double p = wd[k] * scale, t = fma(p, fs, neg_fs);  // = (p - 1) * 2^F rounded once: the product is exact
     hv[k] = t >= 0.5;
-    wd[k] = rint(max_abs_f64(t, hv[k] ? 1.0 : 0.0));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
+    const double one = hv[k] ? 1.0 : 0.0;
+    wd[k] = rint(max_abs_f64(t, one));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
     op[k] = (float)p;
     run += wd[k];
-    run_u += hv[k] ? wd[k] : 0.0;
+    run_u = fma(wd[k], one, run_u);  // exact: whole numbers below 2^53
     cnt += hv[k] ? 1u : 0u;
   }
   const double i = group_scan_f64<G>(run), iu = group_scan_f64<G>(run_u);
   const uint32_t ic = group_scan_u32<G>(cnt);
-  const uint32_t nh = (uint32_t)__shfl((int)ic, (int)last_lane, 64);
-  // the deficits of the row's own lights: a slot behind the row counts 2^40
-  const double own = __longlong_as_double((long long)shfl_u64((uint64_t)__double_as_longlong(i - iu), (int)last_lane)) +
-                     (double)(SLOTS - d) * neg_fs;
-  const uint32_t nl = SLOTS - nh;
-  const uint32_t ex_c = ic - cnt;
-  uint32_t at[PER];  // of the slot's prefix sum
-  bool self[PER];    // a heavy that is the row's last or that no light finishes
+  const uint32_t nh = (uint32_t)__shfl((int)ic, (int)last_lane, 64), nl = SLOTS - nh;
+  // A heavy keeps itself when its prefix lies above the deficits of the row's own lights (a slot behind the row counts 2^40), or
+  // when it is the last, the only one whose prefix is all the surplus.
+  const double most = lane_shfl_f64(fmin(fma((double)(SLOTS - d), neg_fs, i - iu), iu - 1.0), (int)last_lane);
+  uint32_t at[PER];  // of a light's entry, of the one below a heavy's
+  bool self[PER];
   {
-    uint32_t la = g8 + 8u * (pos - ex_c), ha = g8 + 8u * (TOP - ex_c), hs = g8 + 8u * ex_c;
-    const uint32_t last = g8 + 8u * (nh - 1);
+    const uint32_t ex_c = ic - cnt;
+    uint32_t la = strip + SZ * (pos - ex_c), below = strip + SZ * (TOP - 1 - ex_c);
     double sh = iu - run_u, sl = i - run - sh;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-      at[k] = hv[k] ? ha : la;
+      at[k] = hv[k] ? below : la;
       self[k] = false;
       if (hv[k]) {
         sh += wd[k];
-        val(ha) = sh;
-        slot_of(hs) = (uint8_t)(pos + k);
-        self[k] = hs == last || sh > own;
-        ha -= 8u;
-        hs += 8u;
+        val(below + SZ) = sh;
+        slot_of(below + SZ) = (uint8_t)(pos + k);
+        self[k] = sh > most;
+        below -= SZ;
       } else {
         sl += wd[k];
         val(la) = sl;
-        la += 8u;
+        la += SZ;
       }
     }
     if (gl == G - 1) {
-      val(g8 + 8u * nl) = __builtin_huge_val();
-      val(g8 + 8u * (TOP - nh)) = __builtin_huge_val();
+      val(strip + SZ * nl) = __builtin_huge_val();
+      val(strip + SZ * (nl + 1)) = __builtin_huge_val();
     }
-    if (gl == 0) word(g8) = g8;  // the first light starts in the first heavy
   }
   wave_lds_sync();
+  if (gl == 0) slot_of(strip + SZ * (nl + 1)) = slot_of(strip + SZ * (nl + 2));  // a light beyond every heavy takes the last
 
-  // merged positions [pos, pos + PER) belong to this lane; a lights and pos - a heavies come before them
-  uint32_t a8;
+  // merged positions [pos, pos + PER) belong to this lane; some lights, the next of which is at a, and pos less so many
+  // heavies, the next of which is at q, come before them
+  uint32_t a = strip + SZ * (pos > nh ? pos - nh : 0u);
+  const uint32_t dq = SZ * (TOP - pos);
   {
-    const uint32_t hi8 = g8 + 8u * min(pos, nl), dh = 8u * (TOP - pos);
-    a8 = g8 + 8u * (pos > nh ? pos - nh : 0u);
+    const uint32_t hi = strip + SZ * min(pos, nl);
 #pragma unroll
     for (uint32_t step = 1u << (31 - __builtin_clz(SLOTS / 2)); step >= 1; step >>= 1) {
-      const uint32_t to = a8 + 8u * step;
-      const bool up = val(to - 8u) < val(to + dh);
-      a8 = up && to <= hi8 ? to : a8;
+      if (step >= SLOTS / 8 && step > 1 && !__any(min(nh, nl) >= step)) continue;  // few heavies, or few lights: never so far apart
+      const uint32_t to = min(a + SZ * step, hi);
+      a = val(to - SZ) < val(to + dq) ? to : a;
     }
   }
-  {
-    const uint32_t dh = 8u * (TOP - pos - (PER - 1));  // the heavy at hand lies so far behind the light at hand, and 8 bytes less in every step
-    uint32_t h2 = 8u * (TOP - pos), k8 = 2u * g8 + 8u * pos;
+  uint32_t q = a + dq;
+  uint32_t to[PER], x[PER];
 #pragma unroll
-    for (int s = 0; s < PER; ++s) {
-      const double vl = val(a8), vh = val(a8 + dh + 8u * (PER - 1 - s));
-      const bool take = vh <= vl;  // the heavy
-      const float p = (float)fma(vl - vh, -1.0 / 1099511627776.0, 1.0);
-      word(a8 + (take ? h2 : 8u)) = take ? __float_as_uint(p) : k8 - a8;
-      a8 += take ? 0u : 8u;
-      h2 -= 8u;
-      k8 += 8u;
-    }
+  for (int s = 0; s < PER; ++s) {
+    const double vl = val(a), vh = val(q);
+    const bool take = vh <= vl;  // the heavy
+    const float p = (float)fma(vl - vh, -1.0 / 1099511627776.0, 1.0);
+    const uint32_t an = a + SZ, qn = q - SZ;
+    to[s] = take ? qn : an;
+    x[s] = take ? __float_as_uint(p) : q;
+    a = take ? a : an;
+    q = take ? qn : q;
   }
+  wave_lds_sync();
+#pragma unroll
+  for (int s = 0; s < PER; ++s) word(to[s]) = x[s];
+  if (gl == 0) word(strip) = strip + SZ * TOP;  // the first light starts in the first heavy
   wave_lds_sync();
 
   uint32_t oa[PER];
-  {
-    const uint32_t last = g8 + 8u * (nh - 1), k2 = 2u * g8 + 8u * (TOP + 1);
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const uint32_t w = word(at[k]), m = slot_of(hv[k] ? at[k] : w);
+    oa[k] = self[k] ? pos + k : m;
+    if (hv[k]) op[k] = self[k] ? 1.0f : __uint_as_float(w);
+  }
+  if (__any(nh == 0)) {  // all weights alike, none that counts, or no row
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
-      const uint32_t x = word(at[k]);
-      // a light beyond every heavy takes the last
-      const uint32_t m = slot_of(hv[k] ? k2 - at[k] : min(x, last));
-      oa[k] = (hv[k] ? self[k] : nh == 0) ? pos + k : m;
-      if (hv[k]) op[k] = self[k] ? 1.0f : __uint_as_float(x);
-      if (!row_ok) {
-        op[k] = 0.0f;
-        oa[k] = SKY_INVALID;
-      }
+      if (nh == 0) oa[k] = row_ok ? pos + k : SKY_INVALID;
+      if (!row_ok) op[k] = 0.0f;
     }
   }
   // the next row of this group reuses the strips: its writes must stay behind these reads
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
+  auto put = [&](uint32_t k, const uint4u& o) {  // slots k and k + 1
+    if (k + 1 < d) *reinterpret_cast<uint4u*>(table + off + k) = o;
+    else if (k < d) table[off + k] = AliasEntry{__uint_as_float(o.x), o.y};
+  };
+  if constexpr (PER == 8 && G >= 4) {  // a quad of lanes moves its 256 bytes as whole 64-byte pieces
+    uint32_t v[4][4];
+    quad_exchange(tid, op, oa, v);
 #pragma unroll
-  for (int h = 0; h < PER / 2; ++h) {
-    AliasEntry* t = table + off + pos + 2 * h;
-    if (pos + 2 * h + 1 < d) {
-      uint4u o;
-      o.x = __float_as_uint(op[2 * h]); o.y = oa[2 * h]; o.z = __float_as_uint(op[2 * h + 1]); o.w = oa[2 * h + 1];
-      *reinterpret_cast<uint4u*>(t) = o;
-    } else if (pos + 2 * h < d) {
-      t[0] = AliasEntry{op[2 * h], oa[2 * h]};
-    }
+    for (int h = 0; h < 4; ++h) put(PER * (gl & ~3u) + 8 * h + 2 * (gl & 3u), uint4u{v[h][0], v[h][1], v[h][2], v[h][3]});
+  } else {
+#pragma unroll
+    for (int h = 0; h < PER / 2; ++h)
+      put(pos + 2 * h, uint4u{__float_as_uint(op[2 * h]), oa[2 * h], __float_as_uint(op[2 * h + 1]), oa[2 * h + 1]});
+    if (PER % 2 == 1 && pos + PER - 1 < d) table[off + pos + PER - 1] = AliasEntry{op[PER - 1], oa[PER - 1]};
   }
-  if (PER % 2 == 1 && pos + PER - 1 < d) table[off + pos + PER - 1] = AliasEntry{op[PER - 1], oa[PER - 1]};
   return row_ok || d == 0;
 }
 
@@ -367,20 +427,23 @@ __device__ __forceinline__ bool tiny_row(uint32_t off, uint32_t d, const float* 
 // ---------------------------------------------------------------- rows of at most 32 entries, where they lie
 // One wavefront walks a contiguous range of vertices, 64 at a time, and builds every row of 1..32 entries it
 // meets: the rows of a class queue up in LDS until they fill the wavefront (64 rows of 1..2 entries, 32 of 3..8 with
-// 2 lanes each, 16 of 9..16 with 4, 8 of 17..32 with 8) and are then built by the same code as in the class kernels.
+// 2 lanes each, 32 of 9..16 with 2, 16 of 17..32 with 4) and are then built by the same code as in the class kernels.
 // Neighbouring rows of different classes share their cache lines, and here the same wavefront touches them within a
 // few steps; no row list is written or read for these classes.  Also sets valid[] of the vertices it owns (rows of
 // 0..32 entries).  Workgroups are single wavefronts: nothing in here waits for another wavefront.
-// Queue capacities (128, 96, 80, 72): less than one batch left over plus the 64 vertices of a step
-// (64 + 63, 64 + 31, 64 + 15, 64 + 7), rounded up.  A queue entry is the row's offset and, in 16 bits, its degree (6 bits) above the vertex's position in
+// Queue capacities: less than one batch left over plus the 64 vertices of a step, rounded up.  A queue entry is the row's offset and, in 16 bits, its degree (6 bits) above the vertex's position in
 // the wavefront's range (10 bits): the vertex id itself is only needed for a row without weight, whose flag is
-// cleared.  6.5 KB of LDS per wavefront, so that six of them fit every SIMD (the kernel's registers allow six).
+// cleared.  7.5 KB of LDS per wavefront, so that five of them fit every SIMD, as many as the kernel's registers allow.
 constexpr uint32_t SMALL_RANGE = 1024;  // most vertices per wavefront
-constexpr uint32_t SMALL_QBASE[4] = {0, 128, 224, 304};
-constexpr uint32_t SMALL_QTOTAL = 376;
-constexpr size_t SMALL_STRIPS = 4176;  // strips of the groups, the largest of three
-static_assert(SMALL_STRIPS >= group_lds_bytes(2, 4, 64) && SMALL_STRIPS >= group_lds_bytes(4, 4, 64) &&
-              SMALL_STRIPS >= group_lds_bytes(8, 4, 64) && SMALL_STRIPS % 8 == 0, "every group size fits");
+constexpr uint32_t SMALL_BATCH[4] = {64, 64 / SHAPE_G2.lanes, 64 / SHAPE_G4.lanes, 64 / SHAPE_G8.lanes};
+constexpr uint32_t small_cap(int q) { return (SMALL_BATCH[q] + 63 + 7) / 8 * 8; }
+constexpr uint32_t SMALL_QBASE[4] = {0, small_cap(0), small_cap(0) + small_cap(1), small_cap(0) + small_cap(1) + small_cap(2)};
+constexpr uint32_t SMALL_QTOTAL = SMALL_QBASE[3] + small_cap(3);
+constexpr size_t smax(size_t a, size_t b) { return a > b ? a : b; }
+// strips of the groups, the largest of three
+constexpr size_t SMALL_STRIPS = smax(group_lds_bytes(SHAPE_G2.lanes, SHAPE_G2.per, 64),
+                                     smax(group_lds_bytes(SHAPE_G4.lanes, SHAPE_G4.per, 64), group_lds_bytes(SHAPE_G8.lanes, SHAPE_G8.per, 64)));
+static_assert(SMALL_STRIPS % 8 == 0);
 constexpr size_t SMALL_LDS_BYTES = SMALL_STRIPS + SMALL_QTOTAL * 6;
 // Vertices [lo, lo + per_wave) of the n (src null: the vertices themselves) by one wavefront that is a workgroup.
 __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __restrict__ xadj, const float* __restrict__ wgt,
@@ -421,23 +484,23 @@ __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __
   };
   auto build_g2 = [&](uint32_t rows) {
     uint32_t t, off, it, d;
-    take(1, rows, 2, t, off, it, d);
-    const bool ok = group_build_row<2, 4, 64>(off, d, wgt, table, smem, t);
-    if ((t & 1) == 0 && !ok) clear_valid(it);
+    take(1, rows, SHAPE_G2.lanes, t, off, it, d);
+    const bool ok = group_build_row<SHAPE_G2.lanes, SHAPE_G2.per, 64>(off, d, wgt, table, smem, t);
+    if ((t & (SHAPE_G2.lanes - 1)) == 0 && !ok) clear_valid(it);
     cnt[1] -= rows;
   };
   auto build_g4 = [&](uint32_t rows) {
     uint32_t t, off, it, d;
-    take(2, rows, 4, t, off, it, d);
-    const bool ok = group_build_row<4, 4, 64>(off, d, wgt, table, smem, t);
-    if ((t & 3) == 0 && !ok) clear_valid(it);
+    take(2, rows, SHAPE_G4.lanes, t, off, it, d);
+    const bool ok = group_build_row<SHAPE_G4.lanes, SHAPE_G4.per, 64>(off, d, wgt, table, smem, t);
+    if ((t & (SHAPE_G4.lanes - 1)) == 0 && !ok) clear_valid(it);
     cnt[2] -= rows;
   };
   auto build_g8 = [&](uint32_t rows) {
     uint32_t t, off, it, d;
-    take(3, rows, 8, t, off, it, d);
-    const bool ok = group_build_row<8, 4, 64>(off, d, wgt, table, smem, t);
-    if ((t & 7) == 0 && !ok) clear_valid(it);
+    take(3, rows, SHAPE_G8.lanes, t, off, it, d);
+    const bool ok = group_build_row<SHAPE_G8.lanes, SHAPE_G8.per, 64>(off, d, wgt, table, smem, t);
+    if ((t & (SHAPE_G8.lanes - 1)) == 0 && !ok) clear_valid(it);
     cnt[3] -= rows;
   };
 
@@ -477,9 +540,9 @@ __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     while (cnt[0] >= 64u) build_tiny(64);
-    while (cnt[1] >= 32u) build_g2(32);
-    while (cnt[2] >= 16u) build_g4(16);
-    while (cnt[3] >= 8u) build_g8(8);
+    while (cnt[1] >= SMALL_BATCH[1]) build_g2(SMALL_BATCH[1]);
+    while (cnt[2] >= SMALL_BATCH[2]) build_g4(SMALL_BATCH[2]);
+    while (cnt[3] >= SMALL_BATCH[3]) build_g8(SMALL_BATCH[3]);
     // the next step's queue entries stay behind this step's reads of the queues
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();

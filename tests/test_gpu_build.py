@@ -218,6 +218,31 @@ def test_rows_that_end_at_the_ends_of_wavefronts(orc, dist):
     g.free()
 
 
+@pytest.mark.parametrize("dist", ["lognormal2", "nearequal", "sparse", "fewlights", "fewheavies", "alternating", "equal"])
+def test_rows_that_share_a_wavefront(orc, dist):
+    # rows of 3..192 entries, paired by a merge in strips of their own: every length a few times, so that full, partly filled
+    # and empty strips meet; rows without heavies, with one, with nothing but heavies around one light
+    from helpers import weights
+    from skywalker_amd import capi
+    rng = np.random.default_rng(29)
+    degs = [d for d in range(1, 196) for _ in range(3)] + [8, 16, 32, 64, 128, 160, 192] * 20
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal", V=len(degs) + 5)
+    if dist == "fewlights":
+        w = np.where(rng.random(len(w)) < 0.03, 0.01, 1.01).astype(np.float32)
+    elif dist == "fewheavies":
+        w = np.where(rng.random(len(w)) < 0.02, 1000.0, 0.5).astype(np.float32)
+    elif dist == "alternating":
+        w = np.where((np.arange(len(w)) // 20) % 2 == 0, 1.0, 3.0).astype(np.float32)
+    else:
+        w = weights(len(w), rng, dist)
+    build_and_compare(orc, xadj, adjncy, w, "short/" + dist)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, "short in four launches/" + dist)
+    g.free()
+
+
 def test_streaming_kernel_for_rows_with_too_many_tiles(orc):
     from skywalker_amd import capi
     rng = np.random.default_rng(22)
