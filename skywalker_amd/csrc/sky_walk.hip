@@ -471,18 +471,18 @@ int walk_offline_noalloc(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32
 // (src/unbiased_walk.cu:14-60).
 //
 // G lanes per walker, which hold its state alike and share the work of a step: the random numbers, which cost more
-// instructions than everything else in a trial, are computed for TRIALS trials of STEPS steps at once, one lane each, and
+// instructions than everything else in a trial, are computed for several trials of several steps at once, one lane each, and
 // all search the previous row together, G probes per round.  Most trials need no search at all: whether the candidate is
 // kept depends on its being a neighbour of the previous vertex only when the drawn number lies between the two cases'
 // limits.  The bounds of the candidate's own row are requested before the search, for the step after.  Leaving the first
 // probe until it is known to be needed, or reading the next step's entry during the search as if the candidate were
 // kept, was slower.
 //
+// A turn of the loop is one trial of every walker of the wavefront, whichever step each of them is in: where a turn was a step,
+// every walker waited in each for the one with the most trials.
+//
 // A walk lasts as long as its longest chain of dependent loads, so G is the largest whose wavefronts are all resident at
-// once (seven on each of the 1024 SIMDs); once the walkers alone fill the GPU the lanes are worth more as walkers.  80 steps
-// with p = 2, q = 0.5 on a scale-24 graph, in us (the best G for the size, then 8 lanes without the other points above,
-// or one lane above 262,144 walkers): 100 walkers 102 / 175, 10,000 254 / 325, 40,000 401 / 433, 100,000 573 / 900,
-// 1,000,000 (40 steps) 2213 / 2796.
+// once (seven on each of the 1024 SIMDs); once the walkers alone fill the GPU the lanes are worth more as walkers.
 constexpr uint64_t N2V_LANES = 7ull * 1024 * 64;
 template <int G>
 __device__ __forceinline__ unsigned long long group_ballot(bool p) {
@@ -523,7 +523,8 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
     const AliasEntry* __restrict__ table, const uint32_t* __restrict__ seeds, uint32_t walker0, uint32_t N, uint32_t V, uint32_t len,
     float fp, float fq, float fmax, float stop_prob, uint64_t seed, bool once, uint32_t* __restrict__ paths,
     uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
-  constexpr uint32_t TRIALS = G < 16 ? 2 : G < 32 ? 4 : 8, STEPS = G / TRIALS;
+  // Numbers kept of a step, a lane each, of the last one fewer: at least the next trial's and the next step's first.
+  constexpr uint32_t TRIALS = G < 4 ? 1 : 3;
   if (walker0 == 0) call_stamp(call);
   const uint64_t wi = walker0 + ((uint64_t)blockIdx.x * WALK_BLOCK + threadIdx.x) / G;
   const uint32_t i = (uint32_t)wi, gl = threadIdx.x & (G - 1);
@@ -532,59 +533,63 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
   uint32_t s = 0;
   if (wi < N) {
     uint32_t* path = paths + (size_t)i * (len + 1);
-    uint32_t v = seeds[i], prev = 0, prev_off = 0, prev_deg = 0;
+    uint32_t v = seeds[i];
     if (first) path[0] = v;
     if (v < V && len) {
       bounds2u x = *reinterpret_cast<const bounds2u*>(xadj + v);
-      // trial gl % TRIALS of step s0 + gl / TRIALS, where s0 is the last multiple of STEPS
-      u32x4 mine = philox(seed, i, gl / TRIALS, gl % TRIALS, DOM_WALK);
+      uint32_t off = x.x, deg = x.y - x.x, t = 0;
+      uint32_t prev = 0, prev_off = 0, prev_deg = 0, x0 = 0xFFFFFFFFu;
+      // lane gl: trial sb_t + gl of step sb, then trial gl % TRIALS of step sb + gl / TRIALS
+      uint32_t sb = 0, tb = 0;
+      auto numbers = [&] { return philox(seed, i, sb + gl / TRIALS, gl % TRIALS + (gl < TRIALS ? tb : 0u), DOM_WALK); };
+      auto lane_of = [&](uint32_t step, uint32_t trial) -> uint32_t {  // G or more: not among the kept ones
+        const uint32_t k = step == sb ? trial - tb : trial;
+        return k < TRIALS ? (step - sb) * TRIALS + k : (uint32_t)G;
+      };
+      u32x4 mine = numbers();
       const float lo = fminf(1.0f, fq), hi = fmaxf(1.0f, fq);
       for (;;) {
-        const uint32_t x0 = group_first_probe<G>(adjncy + prev_off, prev_deg);  // in flight during the loads below
-        const uint32_t off = x.x, deg = x.y - x.x;
-        const int from = base + (int)(s % STEPS * TRIALS);
-        if ((stop_prob > 0.0f && u24((uint32_t)__shfl((int)mine.z, from, 64)) < stop_prob) || deg == 0) break;
-        uint32_t next = 0;
-        bool dead = false;
-        u32x4 ahead = mine, more = mine;
-        for (uint32_t t = 0;; ++t) {
-          if (t >= TRIALS && (t - TRIALS) % G == 0) more = philox(seed, i, s, t + gl, DOM_WALK);
-          const bool late = t >= TRIALS;
-          const int lane = late ? base + (int)((t - TRIALS) % G) : from + (int)t;
-          const uint32_t rx = (uint32_t)__shfl((int)(late ? more.x : mine.x), lane, 64);
-          const uint32_t ry = (uint32_t)__shfl((int)(late ? more.y : mine.y), lane, 64);
-          const uint32_t rw = (uint32_t)__shfl((int)(late ? more.w : mine.w), lane, 64);
-          const uint32_t col = __umulhi(rx, deg);
-          const AliasEntry e = once ? load_entry_once(table + off + col) : table[off + col];
-          if (t == 0 && (s + 1) % STEPS == 0) {  // the numbers of the steps ahead, while the entry is on its way
-            ahead = philox(seed, i, s + 1 + gl / TRIALS, gl % TRIALS, DOM_WALK);
-            asm volatile("" : "+v"(ahead.x), "+v"(ahead.y), "+v"(ahead.z), "+v"(ahead.w));
-          }
-          const uint32_t cand = u24(ry) < e.prob ? col : e.alias;
-          if (cand == SKY_INVALID) {
-            dead = true;
-            break;
-          }
-          next = adjncy[off + cand];
-          x = *reinterpret_cast<const bounds2u*>(xadj + next);
-          if (s == 0 || t >= 65536u) break;
+        const int from = base + (int)lane_of(s, t);
+        if (t == 0 && ((stop_prob > 0.0f && u24((uint32_t)__shfl((int)mine.z, from, 64)) < stop_prob) || deg == 0)) break;
+        const uint32_t rx = (uint32_t)__shfl((int)mine.x, from, 64);
+        const uint32_t ry = (uint32_t)__shfl((int)mine.y, from, 64);
+        const uint32_t rw = (uint32_t)__shfl((int)mine.w, from, 64);
+        const uint32_t col = __umulhi(rx, deg);
+        const AliasEntry e = once ? load_entry_once(table + off + col) : table[off + col];
+        // The numbers of what may come next, while the entry is on its way: all walkers of the wavefront together.
+        if (__any(lane_of(s, t + 1) >= (uint32_t)G || lane_of(s + 1, 0) >= (uint32_t)G)) {
+          sb = s;
+          tb = t + 1;
+          mine = numbers();
+          asm volatile("" : "+v"(mine.x), "+v"(mine.y), "+v"(mine.z), "+v"(mine.w));
+        }
+        const uint32_t cand = u24(ry) < e.prob ? col : e.alias;
+        if (cand == SKY_INVALID) break;
+        const uint32_t next = adjncy[off + cand];
+        x = *reinterpret_cast<const bounds2u*>(xadj + next);
+        bool keep = s == 0 || t >= 65536u;
+        if (!keep) {
           const float need = u24(rw) * fmax;
-          bool keep;
           if (next == prev) keep = need < fp;
           else if (need < lo) keep = true;
           else if (!(need < hi)) keep = false;
           else keep = need < (group_row_has<G>(adjncy + prev_off, prev_deg, next, x0) ? 1.0f : fq);
-          if (keep) break;
         }
-        if (dead) break;
-        mine = ahead;
-        prev = v;
-        prev_off = off;
-        prev_deg = deg;
-        v = next;
-        ++s;
-        if (first) path[s] = v;
-        if (s == len) break;
+        if (keep) {
+          prev = v;
+          prev_off = off;
+          prev_deg = deg;
+          x0 = group_first_probe<G>(adjncy + off, deg);  // in flight during the loads of the step
+          v = next;
+          off = x.x;
+          deg = x.y - x.x;
+          t = 0;
+          ++s;
+          if (first) path[s] = v;
+          if (s == len) break;
+        } else {
+          ++t;
+        }
       }
     }
     if (first) lengths[i] = s;
