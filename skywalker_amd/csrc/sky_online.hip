@@ -179,6 +179,7 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
 // in every pass, and a launch per step that waited for its slowest walker: 480 us a step for 2,000 walkers on the scale-18
 // graph, 1.1 M entries.)  What the search found stays in LDS, two bits per slot, for the passes that follow.
 constexpr uint32_t N2V_CODES = 65536;    // slots of a row whose result is kept
+constexpr uint32_t N2V_WEIGHTS = N2V_CODES / 16;  // slots of a row whose weights are, in the same LDS
 constexpr uint32_t N2V_SPARSE = 32;      // previous row longer than the current one by this factor: searched in memory
 
 // number of ids of row[lo .. n) that lie below key, plus lo; a wavefront probes 64 places at a time
@@ -205,7 +206,8 @@ struct N2vRow {
   bool has_prev;
   float p, q;
   uint32_t* win;   // [WIN], this wavefront's own
-  uint8_t* codes;  // [N2V_CODES / 4]: per slot 0 neighbour of both, 1 the previous vertex, 2 neither
+  uint8_t* codes;  // [N2V_CODES / 4]: per slot 0 neighbour of both, 1 the previous vertex, 2 neither.  Or the weights of a row
+                   // of up to N2V_WEIGHTS slots: what follows the first pass then waits for no memory
   uint32_t wpos, wlen;  // window: ids wpos .. wpos + wlen of the previous row
 
   // weight of the edge in slot k after the second-order factor (src/api/bias_node2vec.cu:15-27)
@@ -300,14 +302,20 @@ struct N2vRow {
     uint32_t code = 0;
     if (has_prev) {
       code = find(k, t);
-      if (d <= N2V_CODES && k < d) codes[k >> 2] = (uint8_t)code;
+      if (d > N2V_WEIGHTS && d <= N2V_CODES && k < d) codes[k >> 2] = (uint8_t)code;
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) x[j] = k + j < d ? weigh(x[j], (code >> (2 * j)) & 3u) : 0.0f;
+    if (d <= N2V_WEIGHTS && k < d) reinterpret_cast<float4*>(codes)[k >> 2] = make_float4(x[0], x[1], x[2], x[3]);
   }
   __device__ __forceinline__ void again(uint32_t k, float (&x)[4]) const {
     x[0] = x[1] = x[2] = x[3] = 0.0f;
     if (k >= d) return;
+    if (d <= N2V_WEIGHTS) {
+      const float4 c = reinterpret_cast<const float4*>(codes)[k >> 2];
+      x[0] = c.x; x[1] = c.y; x[2] = c.z; x[3] = c.w;
+      return;
+    }
     const float4u a = *reinterpret_cast<const float4u*>(w + k);
     x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
     uint32_t code = 0;
@@ -333,7 +341,7 @@ __global__ __launch_bounds__(T) void walk_n2v_table_kernel(const uint32_t* __res
                                                            uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
   __shared__ DrawLds<T> lds;
   __shared__ uint32_t s_win[T / 64][WIN];
-  __shared__ uint8_t s_codes[N2V_CODES / 4];
+  __shared__ __align__(16) uint8_t s_codes[N2V_CODES / 4];
   call_stamp(call);
   const uint32_t i = first + blockIdx.x;
   uint32_t* const path = paths + (size_t)i * (len + 1);
