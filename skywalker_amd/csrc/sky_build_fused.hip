@@ -65,6 +65,7 @@ struct FusedArgs {
   uint32_t* nfh;
   uint4* ranges;
   const uint32_t* bitmap;  // frontier: bit set for every vertex whose row has been asked for (null: every row is built)
+  uint32_t bit_mask;       // of the bitmap (frontier_bit)
   uint32_t* built;         // frontier: by row of trows, set once a build of the same call has made it
   uint32_t tile0, trow0;  // first tile and row of those this build makes tile by tile
   bool ledgers_done;
@@ -145,8 +146,8 @@ __device__ __forceinline__ bool row_at(const FusedArgs& a, const SectionRef& s, 
 }
 
 __device__ __forceinline__ bool tile_active(const FusedArgs& a, uint32_t r) {
-  const uint32_t v = a.trows[r].v;
-  return ((a.bitmap[v >> 5] >> (v & 31)) & 1u) && !a.built[r];
+  const uint32_t b = frontier_bit(a.trows[r].v, a.bit_mask);
+  return ((a.bitmap[b >> 5] >> (b & 31)) & 1u) && !a.built[r];
 }
 
 // The exact sum of tile `tile` by a wavefront: 16 slots per lane.
@@ -702,6 +703,7 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, con
   base.list = f.list;
   base.counts = counts;
   base.bitmap = bitmap;
+  base.bit_mask = frontier_mask(g->V);
   base.built = built;
   Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
   auto add = [&](Launch& l, Section k, uint32_t per, int cls, int ncls = 1) {

@@ -252,7 +252,7 @@ __global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
 constexpr int COLLECT_T = 1024;
 __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint32_t* __restrict__ data,
                                                                      const uint32_t* __restrict__ sl, uint64_t total,
-                                                                     uint32_t V, HopGeom g, uint32_t* bitmap,
+                                                                     uint32_t V, HopGeom g, uint32_t* bitmap, uint32_t bit_mask,
                                                                      const uint32_t* __restrict__ xadj,
                                                                      int8_t* __restrict__ valid, FrontierLists f,
                                                                      uint32_t* __restrict__ counts,
@@ -282,8 +282,8 @@ __global__ __launch_bounds__(COLLECT_T) void frontier_collect_kernel(const uint3
   // atomic: bits are never cleared during a call, and one that another XCD has just set and that still reads as clear
   // is decided by the atomic.
   if (live) {
-    const uint32_t bit = 1u << (v & 31);
-    if (!(bitmap[v >> 5] & bit)) fresh = !(atomicOr(&bitmap[v >> 5], bit) & bit);
+    const uint32_t b = frontier_bit(v, bit_mask), bit = 1u << (b & 31);
+    if (!(bitmap[b >> 5] & bit)) fresh = !(atomicOr(&bitmap[b >> 5], bit) & bit);
   }
   if (counts) append_rows(fresh, v, xadj, valid, f, counts, s_cnt, s_base);
   if (list) append_list(fresh, v, list, count, s_n);
@@ -412,7 +412,7 @@ struct SampleSession {
       }
     }
     if ((uint64_t)N * lps > (1ull << 40)) return fail(SKY_ERR_LIMIT, "sample: output too large");
-    const uint32_t bits = (g->V + 31) / 32;  // words of the bitmap
+    const uint32_t bits = frontier_mask(g->V) / 32 + 1;  // words of the bitmap
     uint32_t counters = 0;
     SKY_TRY(call_begin(g, words(), &call));
     if (online) {
@@ -460,7 +460,7 @@ struct SampleSession {
     d_count = list_counts + h;
     if (dev_sized) SKY_TRY(frontier_lists(g, *plan, frontier_upper, buffer(sky_graph::POOL_SEGMENTS), &front));
     hipLaunchKernelGGL(frontier_collect_kernel, dim3((uint32_t)((slots + COLLECT_T - 1) / COLLECT_T)), dim3(COLLECT_T), 0, st,
-                       data, sample_lengths, slots, g->V, hg, bitmap, g->xadj, g->valid, front,
+                       data, sample_lengths, slots, g->V, hg, bitmap, frontier_mask(g->V), g->xadj, g->valid, front,
                        dev_sized ? front_counts + h * FRONTIER_WORDS : nullptr, list, d_count);
     if (!dev_sized) {
       SKY_HIP(hipMemcpyAsync(&frontier_count, d_count, 4, hipMemcpyDeviceToHost, st));
