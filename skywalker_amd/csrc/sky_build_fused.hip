@@ -12,7 +12,8 @@
 //   fused_wide_kernel    512 threads   rows of 2558 and more             scan over a row's tiles
 //   fused_block_kernel   256 threads   rows of 1022..2557                entries of the tiles
 //
-// A launch whose classes are empty is left out.  Every row builder is the one the class kernels call, so the
+// A launch whose classes are empty is left out.  A small build with rows for more than the first of them, and none for tiles, goes
+// out in one launch of 512 threads instead (fused_all_kernel).  Every row builder is the one the class kernels call, so the
 // tables are the same bits.  The lists of rows by class and the geometry of the tiles depend on the row offsets alone:
 // they are made by the first build of a graph and kept with it.
 #include <algorithm>
@@ -250,7 +251,7 @@ __device__ __forceinline__ void tile_totals_wave(const FusedArgs& a, uint32_t ti
 template <bool DEV, int G, int PER>
 __device__ __forceinline__ void group_unit(const FusedArgs& a, const SectionRef& s, uint32_t unit, uint32_t rows,
                                            uint64_t* smem) {
-  uint32_t t = threadIdx.x;
+  uint32_t t = threadIdx.x & 63;
   asm volatile("" : "+v"(t));  // what depends on the lane number stays inside this unit's code
   RowRef rr;
   const bool have = row_at<DEV>(a, s, unit * (64 / G) + t / G, rows, rr);
@@ -262,10 +263,10 @@ __device__ __forceinline__ void merge_unit(const FusedArgs& a, const SectionRef&
                                            uint64_t* smem, uint64_t* s_aux) {
   RowRef rr;
   if (!row_at<DEV>(a, s, unit, rows, rr)) return;
-  int t = threadIdx.x;
+  int t = ROWT == 64 ? threadIdx.x & 63 : threadIdx.x;
   asm volatile("" : "+v"(t));  // see group_unit
   const bool ok = merge_row<ROWT, PER>(rr, smem, s_aux, a.wgt, a.table, t);
-  if (threadIdx.x == 0) a.valid[rr.v] = ok ? 1 : 0;
+  if (t == 0) a.valid[rr.v] = ok ? 1 : 0;
 }
 
 constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
@@ -406,6 +407,46 @@ __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
     __syncthreads();
   }
 }
+
+// Small builds in one launch.  Rows of up to 509 entries are a wavefront's, eight of which share a
+// workgroup, any longer one has the workgroup to itself.
+constexpr uint32_t ALL_WAVES = 8;
+constexpr size_t ALL_SLICE = (WAVE_LDS + 64 + 15) / 16 * 16;  // of a wavefront, and its sums
+static_assert(ALL_WAVES * ALL_SLICE <= WIDE_LDS, "eight wavefronts fit the same LDS");
+__global__ __launch_bounds__(512, 4) void fused_all_kernel(FusedArgs a) {
+  __shared__ __align__(16) uint64_t smem[(WIDE_LDS + 7) / 8];
+  call_stamp(a.call);
+  const UnitFinder<false> units(a);
+  SectionRef s;
+  uint32_t unit = 0, rows = 0;
+  units.find(a, blockIdx.x, s, unit, rows);
+  uint64_t* const s_aux = smem + (WIDE_LDS - 512) / 8;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), wunit = unit * ALL_WAVES + wave;
+  uint64_t* const wmem = smem + wave * (ALL_SLICE / 8);
+  uint64_t* const w_aux = wmem + (ALL_SLICE - 64) / 8;
+  switch (s.kind) {
+    case SEC_SWEEP: small_rows_range(wunit * a.per_wave, a.xadj, a.wgt, nullptr, a.V, a.per_wave, a.table, a.valid, wmem); break;
+    case SEC_G16: group_unit<false, SHAPE_G16.lanes, SHAPE_G16.per>(a, s, wunit, rows, wmem); break;
+    case SEC_G32: group_unit<false, SHAPE_G32.lanes, SHAPE_G32.per>(a, s, wunit, rows, wmem); break;
+    case SEC_G32S: group_unit<false, SHAPE_G32S.lanes, SHAPE_G32S.per>(a, s, wunit, rows, wmem); break;
+    case SEC_G32X: group_unit<false, SHAPE_G32X.lanes, SHAPE_G32X.per>(a, s, wunit, rows, wmem); break;
+    case SEC_W1: merge_unit<false, 64, 4>(a, s, wunit, rows, wmem, w_aux); break;
+    case SEC_W6: merge_unit<false, 64, 6>(a, s, wunit, rows, wmem, w_aux); break;
+    case SEC_W2: merge_unit<false, 64, 8>(a, s, wunit, rows, wmem, w_aux); break;
+    case SEC_B6: merge_unit<false, 512, 6>(a, s, unit, rows, smem, s_aux); break;
+    case SEC_B10: merge_unit<false, 512, 10>(a, s, unit, rows, smem, s_aux); break;
+    case SEC_STREAM: {
+      RowRef rr;
+      if (row_at<false>(a, s, unit, rows, rr)) {
+        const bool ok = stream_row(rr, *reinterpret_cast<StreamLds*>(smem), a.wgt, a.table);
+        if (threadIdx.x == 0) a.valid[rr.v] = ok ? 1 : 0;
+      }
+      break;
+    }
+    default: break;
+  }
+}
+
 // ---------------------------------------------------------------- plan of a graph
 // Geometry of the rows that are built tile by tile, in list order: one workgroup, once per graph.
 __global__ __launch_bounds__(1024) void plan_rows_kernel(const RowRef* __restrict__ list, uint32_t n, TiledRow* __restrict__ rows) {
@@ -474,6 +515,15 @@ namespace {
 // Rows of more tiles than this get their ledger from a launch of its own: 2048 tiles add up 2048 x 2048 sums of 16
 // bytes, 67 MB out of L2, when every tile does it.
 constexpr uint32_t LEDGER_TILES = 2048;
+
+// Builds of at most so many workgroups of 512 threads, and without longer rows than this (one is streamed in 39 us), go out in one
+// launch: each of the others costs 5 to 15 us, mostly of waiting for the last row.  Above, a workgroup's LDS and registers leave
+// fewer wavefronts on a CU than the four kernels do.  (Four launches / one, us: scale 10 with 8 edges a vertex 32 / 23, scale
+// 13 with 16 45 / 24, scale 16 with 4 51 / 24, scale 20 with 3 80 / 59; 40,000 .. 6 M entries in rows of up to 15,000 by most
+// workgroups: 2,300 53 / 75, 4,000 110 / 86, 12,000 141 / 151.)
+constexpr uint64_t ALL_MOST = 4096;
+constexpr uint32_t ALL_LONGEST = 16384;
+static_assert(ALL_LONGEST <= 24576, "none is of class CLS_STREAM");
 
 // Frontiers of at most this many rows make the rows of 8190..65533 entries tile by tile.
 constexpr uint32_t SMALL_FRONTIER = 65536;
@@ -643,8 +693,44 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   base.list = p.rows;
   // at least 64 vertices a wavefront, 1024 at most, and enough wavefronts for every SIMD in between
   base.per_wave = std::max(64u, std::min(SMALL_RANGE, g->V / 8192u / 64u * 64u));
-  Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
   auto rows = [&](int c) { return class_min_degree(c) >= min_degree ? g->bin_counts[c] : 0u; };
+  uint32_t past_wave = 0;  // rows of more than 509 entries: what a second launch would be for
+  for (int c = CLS_COUNT - 1; c > CLS_LDS_W2; --c)
+    if (class_min_degree(c) >= 510) past_wave += rows(c);
+  if (past_wave && g->max_degree <= ALL_LONGEST) {
+    Launch all(base, 512);
+    auto waves = [&](Section k, int c, uint32_t per) { all.add(k, rows(c), per * ALL_WAVES, p.start[c]); };
+    all.add(SEC_STREAM, rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM_LAST]);
+    all.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);
+    auto range = [&](Section k, int c0, int c1) {  // classes whose lists lie back to back; min_degree may leave out the first ones
+      uint32_t n = 0;
+      int c = c0;
+      for (int i = c1; i >= c0; --i)
+        if (rows(i)) {
+          n += rows(i);
+          c = i;
+        }
+      all.add(k, n, 1, p.start[c]);
+    };
+    range(SEC_B10, CLS_MW2 + 5, CLS_MW2 + 8);
+    range(SEC_B6, CLS_MW2, CLS_MW2 + 4);
+    all.add(SEC_B6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
+    waves(SEC_W2, CLS_LDS_W2, 1);
+    if (min_degree == 0) all.add(SEC_SWEEP, g->V, base.per_wave * ALL_WAVES, 0);
+    waves(SEC_W6, CLS_LDS_W6, 1);
+    waves(SEC_W1, CLS_LDS_W1, 1);
+    waves(SEC_G32X, CLS_G32X, 64 / SHAPE_G32X.lanes);
+    waves(SEC_G32S, CLS_G32S, 64 / SHAPE_G32S.lanes);
+    waves(SEC_G32, CLS_G32, 64 / SHAPE_G32.lanes);
+    waves(SEC_G16, CLS_G16, 64 / SHAPE_G16.lanes);
+    if (all.units <= ALL_MOST) {
+      all.a.call = call;
+      if (all.units) hipLaunchKernelGGL(fused_all_kernel, dim3((uint32_t)all.units), dim3(512), 0, g->stream, all.a);
+      SKY_HIP(hipGetLastError());
+      return SKY_OK;
+    }
+  }
+  Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
   wave.add(SEC_SUM, n_tiles, 1, 0);
   wave.add(SEC_W2, rows(CLS_LDS_W2), 1, p.start[CLS_LDS_W2]);
   if (min_degree == 0) wave.add(SEC_SWEEP, g->V, base.per_wave, 0);

@@ -430,7 +430,7 @@ __device__ __forceinline__ bool tiny_row(uint32_t off, uint32_t d, const float* 
 // 2 lanes each, 32 of 9..16 with 2, 16 of 17..32 with 4) and are then built by the same code as in the class kernels.
 // Neighbouring rows of different classes share their cache lines, and here the same wavefront touches them within a
 // few steps; no row list is written or read for these classes.  Also sets valid[] of the vertices it owns (rows of
-// 0..32 entries).  Workgroups are single wavefronts: nothing in here waits for another wavefront.
+// 0..32 entries).  Nothing in here waits for another wavefront.
 // Queue capacities: less than one batch left over plus the 64 vertices of a step, rounded up.  A queue entry is the row's offset and, in 16 bits, its degree (6 bits) above the vertex's position in
 // the wavefront's range (10 bits): the vertex id itself is only needed for a row without weight, whose flag is
 // cleared.  7.5 KB of LDS per wavefront, so that five of them fit every SIMD, as many as the kernel's registers allow.
@@ -445,14 +445,14 @@ constexpr size_t SMALL_STRIPS = smax(group_lds_bytes(SHAPE_G2.lanes, SHAPE_G2.pe
                                      smax(group_lds_bytes(SHAPE_G4.lanes, SHAPE_G4.per, 64), group_lds_bytes(SHAPE_G8.lanes, SHAPE_G8.per, 64)));
 static_assert(SMALL_STRIPS % 8 == 0);
 constexpr size_t SMALL_LDS_BYTES = SMALL_STRIPS + SMALL_QTOTAL * 6;
-// Vertices [lo, lo + per_wave) of the n (src null: the vertices themselves) by one wavefront that is a workgroup.
+// Vertices [lo, lo + per_wave) of the n (src null: the vertices themselves) by one wavefront.
 __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __restrict__ xadj, const float* __restrict__ wgt,
                                                  const uint32_t* __restrict__ src, uint32_t n, uint32_t per_wave,
                                                  AliasEntry* __restrict__ table, int8_t* __restrict__ valid,
                                                  uint64_t* __restrict__ smem) {
   uint32_t* q_off = reinterpret_cast<uint32_t*>(smem + SMALL_STRIPS / 8);  // [SMALL_QTOTAL]
   uint16_t* q_it = reinterpret_cast<uint16_t*>(q_off + SMALL_QTOTAL);  // [SMALL_QTOTAL]
-  const uint32_t lane = threadIdx.x;
+  const uint32_t lane = threadIdx.x & 63;
   const uint32_t hi = min(n, lo + per_wave);
   uint32_t cnt[4] = {0, 0, 0, 0};  // wave-uniform queue lengths: rows of 1..2, 3..8, 9..16, 17..32 entries
 
@@ -583,12 +583,16 @@ constexpr bool merge_narrow(int rowt, int per) { return rowt == 64 || merge_resi
 constexpr size_t merge_lds_bytes(int rowt, int per) { return ((size_t)rowt * per + 2) * (merge_narrow(rowt, per) ? 12 : 14); }
 
 // The row `rr` by ROWT threads that share `smem` and, for the wavefronts' sums, s_aux[8 * ROWT / 64].  Returns false when its weights sum to zero.  All threads of the
-// workgroup call it together; the arrays in LDS may be rewritten only after a barrier.
+// workgroup (the wavefront, for ROWT = 64) call it together; the arrays in LDS may be rewritten only after a barrier.
 template <int ROWT, int PER>
 __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint64_t* s_aux,
                                           const float* __restrict__ wgt, AliasEntry* __restrict__ table,
                                           const int tid = threadIdx.x) {
   constexpr int CAP = ROWT * PER;
+  auto row_sync = [] {  // a row of one wavefront waits for no other: its workgroup may have more
+    if (ROWT > 64) __syncthreads();
+    else wave_lds_sync();
+  };
   constexpr int NW = ROWT / 64;
   constexpr uint32_t TOP = CAP + 1;  // heavy h lives at index TOP - h of the value array and of the result array
   static_assert(CAP < 8192 && PER % 2 == 0, "prefix sums below 2^53, 8 * rank in 16 bits, whole pairs");
@@ -638,7 +642,7 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
       s_sum[wave] = rsum;
       s_mn[wave] = mn;
     }
-    __syncthreads();
+    row_sync();
     rsum = s_sum[0];
     mn = s_mn[0];
 #pragma unroll
@@ -657,7 +661,7 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
     if (NW > 1) {
       WSum3* const s_w = reinterpret_cast<WSum3*>(s_aux + 2 * NW);
       if (lane == 0) s_w[wave] = sum;
-      __syncthreads();
+      row_sync();
       sum = s_w[0];
 #pragma unroll
       for (int i = 1; i < NW; ++i) {
@@ -711,7 +715,7 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
         s_p[2 * wave + 1] = iu;
         s_c[wave] = ic;
       }
-      __syncthreads();
+      row_sync();
       nh = 0;
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
@@ -750,7 +754,7 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
       val(8u * (TOP - nh)) = __builtin_huge_val();
     }
   }
-  __syncthreads();
+  row_sync();
 
   if (nh) {
     if (wave_on) {
@@ -784,14 +788,14 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
       rank(0) = 0;                                   // the first light starts in the first heavy
       slot_of(2u * nh) = slot_of(2u * (nh - 1));    // a light beyond every heavy takes the last
     }
-    __syncthreads();
+    row_sync();
     // heavies, densely by rank: residual probability from the light that finishes them
     for (uint32_t h = tid; h < nh; h += ROWT) {
       const uint32_t i = TOP - h, r = rank(RB * i);
       const float p = (float)fma(val(r) - val(8u * i), -1.0 / 1099511627776.0, 1.0);
       prob(8u * i) = h + 1 < nh && r < 8u * (d - nh) ? __float_as_uint(p) : MERGE_SELF;
     }
-    __syncthreads();
+    row_sync();
   }
 
   uint32_t oa[PER];
@@ -812,7 +816,7 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
       }
     }
   }
-  if (NW > 1 && NARROW) __syncthreads();  // the entries take the place of the values
+  if (NW > 1 && NARROW) row_sync();  // the entries take the place of the values
   if (wave_on) wave_store<PER>(table + off, wfirst, d, s_v + PER * 512 * wave, lane, op, oa);
   return true;
 }

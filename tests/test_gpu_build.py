@@ -239,7 +239,7 @@ def test_rows_that_share_a_wavefront(orc, dist):
     build_and_compare(orc, xadj, adjncy, w, "short/" + dist)
     g = capi.Graph.upload(xadj, adjncy, w)
     g.build_tables()
-    compare_tables(orc, g, xadj, w, "short in four launches/" + dist)
+    compare_tables(orc, g, xadj, w, "short by default/" + dist)
     g.free()
 
 
@@ -489,6 +489,30 @@ def test_builds_in_four_launches(orc, dist, stream_min_edges):
     compare_tables(orc, g, xadj, w2, dist + ", other weights")
     g.build_tables()
     compare_tables(orc, g, xadj, w, dist + ", again")
+    g.free()
+
+
+@pytest.mark.parametrize("longest", [509, 510, 16384, 16385])
+@pytest.mark.parametrize("dist", ["lognormal2", "fewlights", "sparse"])
+def test_small_builds_in_one_launch(orc, dist, longest):
+    # rows of every class up to 16,384 entries share workgroups of 512 threads, a wavefront or a workgroup each; a longer row,
+    # or none that needs more than a wavefront, takes the four launches; twice, the second time from weights without a row's
+    from helpers import weights
+    from skywalker_amd import capi
+    rng = np.random.default_rng(43)
+    degs = [d for d in EDGE_DEGREES if d < longest] + [longest] + list(rng.integers(0, min(longest, 2000), 300))
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal", V=len(degs) + 3)
+    w = np.where(rng.random(len(w)) < 0.01, 0.01, 1.01).astype(np.float32) if dist == "fewlights" else weights(len(w), rng, dist)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, "one launch/%s/%d" % (dist, longest))
+    g.free()
+    for v in rng.integers(0, len(degs), 20):
+        w[xadj[v]:xadj[v + 1]] = 0.0
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, "one launch, rows without weight/%s/%d" % (dist, longest))
     g.free()
 
 
