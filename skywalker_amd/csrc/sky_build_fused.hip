@@ -516,13 +516,14 @@ namespace {
 // bytes, 67 MB out of L2, when every tile does it.
 constexpr uint32_t LEDGER_TILES = 2048;
 
-// Builds of at most so many workgroups of 512 threads, and without longer rows than this (one is streamed in 39 us), go out in one
-// launch: each of the others costs 5 to 15 us, mostly of waiting for the last row.  Above, a workgroup's LDS and registers leave
-// fewer wavefronts on a CU than the four kernels do.  (Four launches / one, us: scale 10 with 8 edges a vertex 32 / 23, scale
-// 13 with 16 45 / 24, scale 16 with 4 51 / 24, scale 20 with 3 80 / 59; 40,000 .. 6 M entries in rows of up to 15,000 by most
-// workgroups: 2,300 53 / 75, 4,000 110 / 86, 12,000 141 / 151.)
+// Builds of at most so many workgroups of 512 threads, and without longer rows than this, go out in one launch: each of the
+// others costs 5 to 15 us, mostly of waiting for the last row.  With more workgroups their LDS and registers, which leave fewer
+// wavefronts on a CU than the four kernels do, cost more; a longer row takes longer to stream (29 us for this one) than the
+// passes over its tiles.  (Four launches / one, us: scale 10 with 8 edges a vertex 32 / 23, scale 13 with 16 45 / 24, scale 16 with 4
+// 51 / 24, scale 20 with 3 80 / 59; rebuilds by workgroups: 2,300 75 / 53, 4,000 110 / 86, 12,000 141 / 151; by the longest
+// row: 8,600 56 / 36, 15,400 with few others 62 / 76.)
 constexpr uint64_t ALL_MOST = 4096;
-constexpr uint32_t ALL_LONGEST = 16384;
+constexpr uint32_t ALL_LONGEST = 12288;
 static_assert(ALL_LONGEST <= 24576, "none is of class CLS_STREAM");
 
 // Frontiers of at most this many rows make the rows of 8190..65533 entries tile by tile.
@@ -691,8 +692,10 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   FusedArgs base = common_args(g, p, p.t_all);
   const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
   base.list = p.rows;
-  // at least 64 vertices a wavefront, 1024 at most, and enough wavefronts for every SIMD in between
-  base.per_wave = std::max(64u, std::min(SMALL_RANGE, g->V / 8192u / 64u * 64u));
+  // Vertices of a wavefront: enough wavefronts for every SIMD, but 256 rather than fewer where four wavefronts a SIMD remain: the
+  // rows of a few vertices fill no batch of their class.  (4.4 M entries in 870,000 rows 51 us with 64, 40 with 192; 6.3 M in
+  // 2 M rows 113 with 256, 124 with 512; 20 M in 4 M rows 115 with 448, 125 with 960.)
+  base.per_wave = std::max(64u, std::min(SMALL_RANGE, std::max(g->V / 8192u, std::min(256u, g->V / 4096u)) / 64u * 64u));
   auto rows = [&](int c) { return class_min_degree(c) >= min_degree ? g->bin_counts[c] : 0u; };
   uint32_t past_wave = 0;  // rows of more than 509 entries: what a second launch would be for
   for (int c = CLS_COUNT - 1; c > CLS_LDS_W2; --c)

@@ -207,11 +207,12 @@ constexpr size_t group_lds_bytes(int G, int PER, int BLOCK) { return (size_t)gro
 
 // Lanes and slots of a lane by class.  8 slots a lane where 4 would do for twice the lanes: what a lane does once for its row (sum, division,
 // scans, search) is half of its instructions with 4.  200 M entries in rows of 100 (32 lanes of 4 / 16 of 8) 739 / 630 us, of 50
-// 720 / 640, of 24 835 / 680, of 12 880 / 850; rows of 3..8 would be one lane's.
+// 720 / 640.  Not for the rows of up to 32: 200 M entries in rows of 24 835 / 680, but where they lie among others half as many
+// lanes means batches that are half as full (scale 20 with 16 edges a vertex 140 / 150, scale 22 with 10 316 / 333).
 struct GroupShape {
   int lanes, per;
 };
-constexpr GroupShape SHAPE_G2{2, 4}, SHAPE_G4{2, 8}, SHAPE_G8{4, 8}, SHAPE_G16{8, 8}, SHAPE_G32{16, 8}, SHAPE_G32S{32, 5}, SHAPE_G32X{32, 6};
+constexpr GroupShape SHAPE_G2{2, 4}, SHAPE_G4{4, 4}, SHAPE_G8{8, 4}, SHAPE_G16{8, 8}, SHAPE_G32{16, 8}, SHAPE_G32S{32, 5}, SHAPE_G32X{32, 6};
 
 template <int G, int PER, int BLOCK = 256>
 __device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const float* __restrict__ wgt,
@@ -427,13 +428,13 @@ __device__ __forceinline__ bool tiny_row(uint32_t off, uint32_t d, const float* 
 // ---------------------------------------------------------------- rows of at most 32 entries, where they lie
 // One wavefront walks a contiguous range of vertices, 64 at a time, and builds every row of 1..32 entries it
 // meets: the rows of a class queue up in LDS until they fill the wavefront (64 rows of 1..2 entries, 32 of 3..8 with
-// 2 lanes each, 32 of 9..16 with 2, 16 of 17..32 with 4) and are then built by the same code as in the class kernels.
+// 2 lanes each, 16 of 9..16 with 4, 8 of 17..32 with 8) and are then built by the same code as in the class kernels.
 // Neighbouring rows of different classes share their cache lines, and here the same wavefront touches them within a
 // few steps; no row list is written or read for these classes.  Also sets valid[] of the vertices it owns (rows of
 // 0..32 entries).  Nothing in here waits for another wavefront.
 // Queue capacities: less than one batch left over plus the 64 vertices of a step, rounded up.  A queue entry is the row's offset and, in 16 bits, its degree (6 bits) above the vertex's position in
 // the wavefront's range (10 bits): the vertex id itself is only needed for a row without weight, whose flag is
-// cleared.  7.5 KB of LDS per wavefront, so that five of them fit every SIMD, as many as the kernel's registers allow.
+// cleared.  5 KB of LDS per wavefront: the kernel's registers decide how many fit a SIMD.
 constexpr uint32_t SMALL_RANGE = 1024;  // most vertices per wavefront
 constexpr uint32_t SMALL_BATCH[4] = {64, 64 / SHAPE_G2.lanes, 64 / SHAPE_G4.lanes, 64 / SHAPE_G8.lanes};
 constexpr uint32_t small_cap(int q) { return (SMALL_BATCH[q] + 63 + 7) / 8 * 8; }

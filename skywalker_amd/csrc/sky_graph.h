@@ -91,8 +91,8 @@ enum BuildClass : int {
   CLS_EMPTY = 0,    // deg 0            handled while binning
   CLS_TINY = 1,     // deg 1..2         one lane per vertex, handled while binning
   CLS_G2 = 2,       // deg 3..8         2 lanes per row, 4 slots per lane
-  CLS_G4 = 3,       // deg <= 16        2 lanes, 8 slots per lane
-  CLS_G8 = 4,       // deg <= 32        4 lanes, 8 slots per lane
+  CLS_G4 = 3,       // deg <= 16        4 lanes
+  CLS_G8 = 4,       // deg <= 32        8 lanes
   CLS_G16 = 5,      // deg <= 64        8 lanes, 8 slots per lane
   CLS_G32 = 6,      // deg <= 128       16 lanes, 8 slots per lane
   CLS_G32X = 7,     // deg 161..192     32 lanes, 6 slots per lane

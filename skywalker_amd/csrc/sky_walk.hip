@@ -275,12 +275,18 @@ static void launch_walk(sky_graph* g, const uint32_t* seeds, const uint32_t* liv
                        seed, paths, lengths, next_live, n_next, call, partials);
 }
 
-// Up to ALONE_WALKERS walkers, as many wavefronts as the GPU holds, get a wavefront each (8,192 walkers x 80 steps on the
-// scale-16 graph 96 -> 69 us; twice as many would walk in two turns: 130, 97 with a lane each).  Beyond ALONE_SCALAR the
-// vector cache takes part (4,096 walkers 60.8 us all scalar, 54.9 with it; 1,000 walkers 35.4 and 37.5), and with the
-// walk index, whose entries leave no load to request ahead, a lane each is as fast (4,000 walkers on the scale-22
-// graph 70 us both ways; 2,000 walkers 45 -> 37).
-constexpr uint32_t ALONE_WALKERS = 8192, ALONE_SCALAR = 2048;
+// Few walkers get a wavefront each.  Beyond ALONE_SCALAR the vector cache takes part (4,096 walkers x 80 steps on the scale-16 graph
+// 60.8 us all scalar, 54.9 with it; 1,000 walkers 35.4 and 37.5), and with the walk index, whose entries leave no load to
+// request ahead, a lane each is as fast (4,000 walkers on the scale-22 graph 70 us both ways; 2,000 walkers 45 -> 37).
+// Up to 8,192 are as many wavefronts as the GPU holds (twice as many walk in two turns: 130 us, 97 with a lane each), but
+// where a lane's gathers come from L2 or the walk is short half as many are the limit (8,000 walkers, a lane / a wavefront each:
+// scale 14, 30 steps 31.6 / 36.8; scale 21, 30 steps 47.8 / 38.5, 6 steps 20.4 / 23; 4,000: scale 14, 6 steps 19.3 / 20.1,
+// 16 steps 24.0 / 23.9, 30 steps 31 / 29).
+constexpr uint32_t ALONE_SCALAR = 2048;
+static uint32_t alone_walkers(const sky_graph* g, uint32_t len) {
+  if (g->has_walk_index || len < 16) return ALONE_SCALAR;
+  return len >= 24 && (uint64_t)g->E * sizeof(AliasEntry) > (4u << 20) ? 8192u : 4096u;
+}
 int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, float stop_prob, uint64_t seed,
                  uint32_t* paths, uint32_t* lengths, uint64_t* sampled, double* seconds) {
   hipStream_t st = g->stream;
@@ -299,7 +305,7 @@ int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, 
     if (g->has_walk_index) launch_walk<true>(g, a...);
     else launch_walk<false>(g, a...);
   };
-  if (N && N <= (g->has_walk_index ? ALONE_SCALAR : ALONE_WALKERS) && !segmented) {
+  if (N && N <= alone_walkers(g, len) && !segmented) {
     auto go = [&](auto kernel) {
       hipLaunchKernelGGL(kernel, dim3(N), dim3(64), 0, st, g->xadj, g->adjncy, g->table, g->walk_index, seeds, g->V, len, stop_prob,
                          seed, paths, lengths, call);
@@ -524,7 +530,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
     float fp, float fq, float fmax, float stop_prob, uint64_t seed, bool once, uint32_t* __restrict__ paths,
     uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
   // Numbers kept of a step, a lane each, of the last one fewer: at least the next trial's and the next step's first.
-  constexpr uint32_t TRIALS = G < 4 ? 1 : 3;
+  constexpr uint32_t TRIALS = G < 4 ? 1 : G < 16 ? 3 : G < 32 ? 4 : 8;
   if (walker0 == 0) call_stamp(call);
   const uint64_t wi = walker0 + ((uint64_t)blockIdx.x * WALK_BLOCK + threadIdx.x) / G;
   const uint32_t i = (uint32_t)wi, gl = threadIdx.x & (G - 1);
@@ -546,14 +552,17 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
         const uint32_t k = step == sb ? trial - tb : trial;
         return k < TRIALS ? (step - sb) * TRIALS + k : (uint32_t)G;
       };
+      // what lane l holds; the only walker of a wavefront needs no exchange through LDS for it
+      auto of = [&](uint32_t x, int l) -> uint32_t {
+        if (G == 64) return (uint32_t)__builtin_amdgcn_readlane((int)x, __builtin_amdgcn_readfirstlane(l));
+        return (uint32_t)__shfl((int)x, l, 64);
+      };
       u32x4 mine = numbers();
       const float lo = fminf(1.0f, fq), hi = fmaxf(1.0f, fq);
       for (;;) {
         const int from = base + (int)lane_of(s, t);
-        if (t == 0 && ((stop_prob > 0.0f && u24((uint32_t)__shfl((int)mine.z, from, 64)) < stop_prob) || deg == 0)) break;
-        const uint32_t rx = (uint32_t)__shfl((int)mine.x, from, 64);
-        const uint32_t ry = (uint32_t)__shfl((int)mine.y, from, 64);
-        const uint32_t rw = (uint32_t)__shfl((int)mine.w, from, 64);
+        if (t == 0 && ((stop_prob > 0.0f && u24(of(mine.z, from)) < stop_prob) || deg == 0)) break;
+        const uint32_t rx = of(mine.x, from), ry = of(mine.y, from), rw = of(mine.w, from);
         const uint32_t col = __umulhi(rx, deg);
         const AliasEntry e = once ? load_entry_once(table + off + col) : table[off + col];
         // The numbers of what may come next, while the entry is on its way: all walkers of the wavefront together.

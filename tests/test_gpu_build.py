@@ -492,10 +492,10 @@ def test_builds_in_four_launches(orc, dist, stream_min_edges):
     g.free()
 
 
-@pytest.mark.parametrize("longest", [509, 510, 16384, 16385])
+@pytest.mark.parametrize("longest", [509, 510, 12288, 12289])
 @pytest.mark.parametrize("dist", ["lognormal2", "fewlights", "sparse"])
 def test_small_builds_in_one_launch(orc, dist, longest):
-    # rows of every class up to 16,384 entries share workgroups of 512 threads, a wavefront or a workgroup each; a longer row,
+    # rows of every class up to 12,288 entries share workgroups of 512 threads, a wavefront or a workgroup each; a longer row,
     # or none that needs more than a wavefront, takes the four launches; twice, the second time from weights without a row's
     from helpers import weights
     from skywalker_amd import capi
