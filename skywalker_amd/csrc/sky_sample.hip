@@ -156,9 +156,13 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_draw_kernel(SampleArgs a) {
 // fanout 25 197 -> 17 us.
 constexpr uint32_t DISTINCT_MAX_K = 64;  // largest fanout of this rule
 constexpr uint32_t DISTINCT_ROUNDS = 11;
-__device__ __forceinline__ uint32_t distinct_lanes(uint32_t k) { return k <= 4 ? 4u : k == 64u ? 64u : 1u << (32 - __clz((int)(k - 1))); }
+__host__ __device__ inline uint32_t distinct_lanes(uint32_t k) {
+  uint32_t g = 4;
+  while (g < k) g *= 2;
+  return g;
+}
 
-// T = 256 spreads the parents of one start vertex over four wavefronts, for batches of a few start vertices.
+// T spreads the parents of one start vertex over several wavefronts, for batches of a few start vertices.
 template <int T>
 __global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
   __shared__ __align__(16) uint32_t s_c[T];
@@ -186,16 +190,29 @@ __global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
       }
       uint32_t cand = 0, child = 0, t = 0;
       bool live = i < min(deg, k);  // a draw that keeps something, as far as is known
+      // The entry of the next try is requested when this one's candidate is taken (1,024 seeds, 25 x 10 on the scale-20 graph 60 -> 58 us,
+      // 806 with 4 edges a vertex 43 -> 38; several tries at once cost more in random numbers than they save: 65).
+      uint32_t col = 0;
+      float u = 0.0f;
+      AliasEntry e{0.0f, 0};
+      auto request = [&](uint32_t round) {
+        const u32x4 r = philox(a.seed, (uint32_t)si, s * k + i, g.h + 256u * round, DOM_SAMPLE);
+        col = __umulhi(r.x, deg);
+        u = u24(r.y);
+        e = a.table[o + col];
+      };
       auto take = [&] {
-        const u32x4 r = philox(a.seed, (uint32_t)si, s * k + i, g.h + 256u * t, DOM_SAMPLE);
-        const uint32_t col = __umulhi(r.x, deg);
-        const AliasEntry e = a.table[o + col];
-        cand = u24(r.y) < e.prob ? col : e.alias;
+        cand = u < e.prob ? col : e.alias;
         child = a.adjncy[o + cand];
+        if (t + 1 < DISTINCT_ROUNDS) request(t + 1);
       };
       if (live) {
-        if (deg > k) take();
-        else child = a.adjncy[o + (cand = i)];  // all neighbours
+        if (deg > k) {
+          request(0);
+          take();
+        } else {
+          child = a.adjncy[o + (cand = i)];  // all neighbours
+        }
       }
       for (;;) {
         s_c[tid] = cand;
@@ -519,14 +536,27 @@ struct SampleSession {
       const uint64_t draws = width[h1 - 1] * fanout[h1];
       while (a.lanes > 1 && draws <= a.lanes / 2) a.lanes /= 2;
     }
-    // T = 64 as soon as that fills the GPU with wavefronts
-    const uint32_t T = distinct && (N < 4096 || parts > 1) ? 256 : 64, per_block = distinct ? 1 : SAMPLE_T / a.lanes;
+    // Distinct children: lanes for every parent of the widest hop at once, as long as the GPU holds all wavefronts (2,500 seeds,
+    // 10 x 10 on the scale-18 graph 46 -> 42 us; 5,000, 25 x 10 on the scale-20 graph 79 -> 78).
+    uint32_t T = 64;
+    if (distinct && parts > 1) {
+      T = 256;
+    } else if (distinct) {
+      uint64_t lanes = 0;
+      for (uint32_t h = h0; h < h1; ++h) lanes = std::max(lanes, width[h] * distinct_lanes(fanout[h + 1]));
+      while (T < 1024 && T < lanes && (uint64_t)N * (2 * T / 64) <= 8192) T *= 2;
+    }
+    const uint32_t per_block = distinct ? 1 : SAMPLE_T / a.lanes;
     const uint64_t most = 0xFFFFFFFFull / T / parts * per_block;  // start vertices of one launch (below 2^32 threads)
     for (a.first = 0; a.first < N; a.first += most) {
       const dim3 grid((uint32_t)((std::min<uint64_t>(most, N - a.first) + per_block - 1) / per_block * parts));
-      if (!distinct) hipLaunchKernelGGL(sample_draw_kernel, grid, dim3(SAMPLE_T), 0, st, a);
-      else if (T == 64) hipLaunchKernelGGL(sample_distinct_kernel<64>, grid, dim3(64), 0, st, a);
-      else hipLaunchKernelGGL(sample_distinct_kernel<256>, grid, dim3(256), 0, st, a);
+      auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(T), 0, st, a); };
+      if (!distinct) go(sample_draw_kernel);
+      else if (T == 64) go(sample_distinct_kernel<64>);
+      else if (T == 128) go(sample_distinct_kernel<128>);
+      else if (T == 256) go(sample_distinct_kernel<256>);
+      else if (T == 512) go(sample_distinct_kernel<512>);
+      else go(sample_distinct_kernel<1024>);
       a.call = nullptr;
     }
     return SKY_OK;
