@@ -887,20 +887,6 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   const bool stream_to_tiled = !row_merge || all_stream_edges <= (uint64_t)option(g, OPT_STREAM_MIN_EDGES);
   const bool wide_streamed = !stream_to_tiled && all_stream_edges >= (uint64_t)option(g, OPT_STREAM_WIDE_MIN_EDGES);
   const uint32_t wide_rows = wide_streamed ? counts[CLS_STREAM_WIDE] : 0;
-  if (!stream_to_tiled && narrow_rows + wide_rows) {
-    // the streaming kernel takes three times as long for an entry as the others when it shares the GPU with them
-    StreamSwap sw(g, fan.next(3 * (narrow_edges + (wide_streamed ? host.edges[CLS_STREAM_WIDE] : 0))));
-    SKY_TRY(build_rows_stream(g, vlist + starts[CLS_STREAM_WIDE], wide_rows, vlist + starts[CLS_STREAM], narrow_rows));
-    if (tm) SKY_TRY(tm->mark("stream", narrow_edges + (wide_streamed ? host.edges[CLS_STREAM_WIDE] : 0)));
-  }
-  // Rows of 5118..8189 entries: one workgroup holds the row (without row_merge they are built tile by tile).
-  if (row_merge && counts[CLS_HOLD]) {
-    {
-      StreamSwap sw(g, fan.next(2 * host.edges[CLS_HOLD]));
-      SKY_TRY(build_rows_hold(g, vlist + starts[CLS_HOLD], counts[CLS_HOLD]));
-    }
-    if (tm) SKY_TRY(tm->mark("hold", host.edges[CLS_HOLD]));
-  }
   auto lds = [&](int cls, auto kernel, int rowt, int t, const char* name) -> int {
     const uint32_t cnt = counts[cls];
     if (cnt) {
@@ -962,6 +948,22 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     }
   }
 
+  // After the merge kernels: two workgroups of it fill a CU's LDS, so nothing of small_rows_kernel would run beside it on a CU
+  // (scale 26 8.25 -> 8.18 ms, scale 25 with 56 edges a vertex 8.8 -> 8.6); last of all, its longest rows would have no company.
+  if (!stream_to_tiled && narrow_rows + wide_rows) {
+    // the streaming kernel takes three times as long for an entry as the others when it shares the GPU with them
+    StreamSwap sw(g, fan.next(3 * (narrow_edges + (wide_streamed ? host.edges[CLS_STREAM_WIDE] : 0))));
+    SKY_TRY(build_rows_stream(g, vlist + starts[CLS_STREAM_WIDE], wide_rows, vlist + starts[CLS_STREAM], narrow_rows));
+    if (tm) SKY_TRY(tm->mark("stream", narrow_edges + (wide_streamed ? host.edges[CLS_STREAM_WIDE] : 0)));
+  }
+  // Rows of 5118..8189 entries: one workgroup holds the row (without row_merge they are built tile by tile).
+  if (row_merge && counts[CLS_HOLD]) {
+    {
+      StreamSwap sw(g, fan.next(2 * host.edges[CLS_HOLD]));
+      SKY_TRY(build_rows_hold(g, vlist + starts[CLS_HOLD], counts[CLS_HOLD]));
+    }
+    if (tm) SKY_TRY(tm->mark("hold", host.edges[CLS_HOLD]));
+  }
   SKY_TRY(grp(CLS_G2, build_group_kernel<SHAPE_G2.lanes, SHAPE_G2.per>, SHAPE_G2.lanes, "g2"));
   SKY_TRY(grp(CLS_G4, build_group_kernel<SHAPE_G4.lanes, SHAPE_G4.per>, SHAPE_G4.lanes, "g4"));
   SKY_TRY(grp(CLS_G8, build_group_kernel<SHAPE_G8.lanes, SHAPE_G8.per>, SHAPE_G8.lanes, "g8"));
