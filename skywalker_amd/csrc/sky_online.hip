@@ -80,11 +80,12 @@ __global__ __launch_bounds__(T) void walk_direct_kernel(const uint32_t* __restri
 // How to serve a static-bias walk on a graph without tables.  Every row drawn from costs either its table (about
 // BUILD_PS a entry, once) or two sweeps over its weights (about DRAW_PS a entry, each time).  A step leads to a row
 // with a probability that grows with its length, so a row of d entries is drawn from about N * len * d / E times, and
-// its table pays from the length on at which N * len * d / E * DRAW_PS exceeds BUILD_PS.  Measured on one MI355X.
-// A few thousand walkers do not fill the GPU: what counts then is how long one walker's draw takes, on four wavefronts, and
-// tables pay from half that length on (R-MAT scale 18 to 24, 10 to 40,000 walkers, 4 to 16 steps: both lie within 10 % of
-// the best of a sweep over the ratio, but for single walkers in long rows).
-constexpr double BUILD_PS = 8.0, DRAW_PS = 2.5, DRAW_FEW_PS = 5.0;
+// its table pays from the length on at which N * len * d / E * DRAW_PS exceeds BUILD_PS.  Measured on one MI355X.  The launches of
+// a build cost BUILD_US whatever they build, so it has to save as much (531 walkers x 6 steps on the scale-16 graph 75 ->
+// 54 us, 110 x 9 on the scale-20 graph with 32 edges a vertex 161 -> 114, 400 x 8 on the scale-22 graph 180 -> 134).  The same
+// ratio for a few thousand walkers and for many: tables from half that length on for the former made 3,000 x 16 steps on the
+// scale-23 graph 390 us, now 334, and 2,000 x 10 on the scale-24 graph 305, now 259.
+constexpr double BUILD_PS = 8.0, DRAW_PS = 2.5;
 constexpr uint32_t FEW_WALKERS = 4096;
 constexpr double BUILD_US = 40.0, STEP_US = 4.0;  // launches of a build; the chain of loads and scans of a step
 
@@ -98,24 +99,27 @@ static int online_plan(sky_graph* g, uint32_t N, uint32_t len, OnlinePlan* o, Ca
   if (mode > 0) return SKY_OK;
   SKY_TRY(ensure_plan(g, first));
   const double E = std::max(1u, g->E), draws = (double)N * len;
-  const double draw_ps = N <= FEW_WALKERS ? DRAW_FEW_PS : DRAW_PS;
-  const double from = BUILD_PS / draw_ps * E / std::max(1.0, draws);
+  const double from = BUILD_PS / DRAW_PS * E / std::max(1.0, draws);
   // the shortest class whose rows are all that long; the classes below G16 (33 entries) are not built apart from the rest
-  double built = 0, direct = 0;
-  bool any = false;
+  double built = 0, direct = 0, tabled = 0;  // entries of tables, entries that draws from other rows read, and from these without tables
   for (int c = CLS_TINY; c < CLS_COUNT; ++c) {
     const double entries = (double)g->bin_edges[c], lo = class_min_degree(c);
     if (entries == 0) continue;
-    const double mean = c == CLS_TINY ? 1.5 : entries / std::max(1u, g->bin_counts[c]);
+    const double read = draws * entries / E * (c == CLS_TINY ? 1.5 : entries / std::max(1u, g->bin_counts[c]));
     if (c >= CLS_G16 && lo >= from) {
       built += entries;
+      tabled += read;
       o->table_from = std::min(o->table_from, class_min_degree(c));
-      any = true;
     } else {
-      direct += draws * entries / E * mean;
+      direct += read;
     }
   }
-  const double hybrid_us = (any ? BUILD_US : 0.0) + (built * BUILD_PS + direct * draw_ps) * 1e-6 + STEP_US * len;
+  if (built && tabled * DRAW_PS * 1e-6 < BUILD_US + built * BUILD_PS * 1e-6) {  // not worth the launches
+    o->table_from = 0xFFFFFFFFu;
+    direct += tabled;
+    built = 0;
+  }
+  const double hybrid_us = (built ? BUILD_US : 0.0) + (built * BUILD_PS + direct * DRAW_PS) * 1e-6 + STEP_US * len;
   const double full_us = BUILD_US + E * BUILD_PS * 1e-6 + 1.2 * len;
   o->full = mode < 0 && full_us < hybrid_us;
   return SKY_OK;
