@@ -270,7 +270,10 @@ __device__ __forceinline__ void merge_unit(const FusedArgs& a, const SectionRef&
 }
 
 constexpr size_t cmax(size_t a, size_t b) { return a > b ? a : b; }
-constexpr size_t WAVE_LDS = cmax(cmax(SMALL_LDS_BYTES, group_lds_bytes(SHAPE_G32X.lanes, SHAPE_G32X.per, 64)), merge_lds_bytes(64, 8));
+constexpr size_t WAVE_LDS = cmax(cmax(SMALL_LDS_BYTES, group_lds_bytes(SHAPE_G32X.lanes, SHAPE_G32X.per, 64)),
+                                 cmax(merge_lds_bytes(64, 8), cmax(merge_lds_bytes(64, 6), merge_lds_bytes(64, 4))));
+constexpr size_t PAIR_LDS = cmax(merge_lds_bytes(128, 8), merge_lds_bytes(128, 6));
+constexpr size_t BLOCK_LDS = cmax(cmax(merge_lds_bytes(256, 10), merge_lds_bytes(256, 8)), cmax(merge_lds_bytes(256, 6), sizeof(TileEmitLds)));
 
 // The second launch bounds: what LDS lets reside anyway (21 wavefronts, 10 pairs, 4 workgroups of 256 to a CU).  Left alone the
 // device-sized kernels took 109, 104 and 132 registers, one workgroup in five and one in four less (the 134,652 rows of a
@@ -316,7 +319,7 @@ __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
 
 template <bool DEV>
 __global__ __launch_bounds__(128, 5) void fused_pair_kernel(FusedArgs a) {
-  __shared__ __align__(16) uint64_t smem[(merge_lds_bytes(128, 8) + 7) / 8];
+  __shared__ __align__(16) uint64_t smem[(PAIR_LDS + 7) / 8];
   __shared__ uint64_t s_aux[16];
   call_stamp(a.call);
   const UnitFinder<DEV> units(a);
@@ -340,7 +343,8 @@ __global__ __launch_bounds__(128, 5) void fused_pair_kernel(FusedArgs a) {
 }
 
 constexpr size_t WIDE_LDS = sizeof(StreamLds);  // two workgroups of it fill a CU
-static_assert(WIDE_LDS % 8 == 0 && merge_lds_bytes(512, 10) + 512 <= WIDE_LDS, "everything fits the same LDS");
+static_assert(WIDE_LDS % 8 == 0 && cmax(merge_lds_bytes(512, 10), cmax(merge_lds_bytes(512, 8), merge_lds_bytes(512, 6))) + 512 <= WIDE_LDS,
+              "everything fits the same LDS");
 template <bool DEV>
 __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[(WIDE_LDS + 7) / 8];
@@ -381,7 +385,7 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
 
 template <bool DEV>
 __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
-  __shared__ __align__(16) uint64_t smem[(cmax(merge_lds_bytes(256, 10), sizeof(TileEmitLds)) + 7) / 8];
+  __shared__ __align__(16) uint64_t smem[(BLOCK_LDS + 7) / 8];
   __shared__ uint64_t s_aux[32];
   call_stamp(a.call);
   const UnitFinder<DEV> units(a);

@@ -569,19 +569,16 @@ __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __
 // - slots behind the row's end in its last wavefront have weight 0 and go along as lights of deficit 2^40.  They come
 //   after every light of the row, in rank and in the merged order, so nothing of the row depends on them, and no step
 //   needs a mask; a heavy that only one of them reaches is one that nobody finishes;
-// - a slot takes part in the compaction on the side of its kind alone, and the merge reads both heads in every step, at
-//   addresses that differ by what the thread knows, instead of choosing between them.
-constexpr uint32_t MERGE_SELF = 0x80000000u;  // "prob 1, alias self" in the per-heavy result word
-
-// LDS of a row: 14 bytes a slot, or 12 where that lets one more workgroup reside on a CU.  With 12, a heavy's residual takes the place of its
-// prefix sum, which the entries need last, and a row of several wavefronts pays a barrier for it (rows of 3582..4093
-// entries 2.68 -> 3.09 TB/s, of 2046..2557 3.16 -> 3.35; of 4606..5117 3.05 -> 2.94, so those keep 14).
-constexpr int merge_resident(int rowt, int per, int bytes) {
-  const int by_lds = 163840 / ((rowt * per + 2) * bytes + rowt), by_waves = (rowt <= 256 && per <= 8 ? 32 : 24) * 64 / rowt;
-  return by_lds < by_waves ? by_lds : by_waves;
-}
-constexpr bool merge_narrow(int rowt, int per) { return rowt == 64 || merge_resident(rowt, per, 12) > merge_resident(rowt, per, 14); }
-constexpr size_t merge_lds_bytes(int rowt, int per) { return ((size_t)rowt * per + 2) * (merge_narrow(rowt, per) ? 12 : 14); }
+// - a slot takes part in the compaction on the side of its kind alone;
+// - the offsets of a step are those of the strips of group_build_row above: of the light and the heavy at hand and of the next ones,
+//   and a step leaves the residual of the heavy that it takes: no pass over the heavies follows.
+//
+// LDS of a row: 10 bytes a slot (sum, slot of a heavy): the words take the place of the sums once every thread has walked its
+// share.  That costs two barriers, and words apart (14 bytes) cost rows that reside on a CU.  200 M entries, before (a pass
+// over the heavies, 12 or 14 bytes) / with 10 / with 14 bytes: rows of 230 692 / 730 / 690 us, 350 605 / 596 / 640, 500 585 / 573
+// / -, 700 651 / 668 / 680, 1,400 637 / 680 / 650, 2,500 610 / 572 / -, 3,000 752 / 727 / 750, 3,500 758 / 635 / -, 4,800 750 / 675 / -.
+constexpr bool merge_words(int rowt, int per) { return rowt * per == 256 || rowt * per == 1536; }
+constexpr size_t merge_lds_bytes(int rowt, int per) { return (((size_t)rowt * per + 4) * (merge_words(rowt, per) ? 14 : 10) + 15) / 16 * 16; }
 
 // The row `rr` by ROWT threads that share `smem` and, for the wavefronts' sums, s_aux[8 * ROWT / 64].  Returns false when its weights sum to zero.  All threads of the
 // workgroup (the wavefront, for ROWT = 64) call it together; the arrays in LDS may be rewritten only after a barrier.
@@ -595,23 +592,15 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
     else wave_lds_sync();
   };
   constexpr int NW = ROWT / 64;
-  constexpr uint32_t TOP = CAP + 1;  // heavy h lives at index TOP - h of the value array and of the result array
-  static_assert(CAP < 8192 && PER % 2 == 0, "prefix sums below 2^53, 8 * rank in 16 bits, whole pairs");
-  constexpr bool NARROW = merge_narrow(ROWT, PER);
-  using Rank = std::conditional_t<NARROW, uint16_t, uint32_t>;
-  constexpr int RSH = NARROW ? 2 : 1;                // from 8 * index to the place of a rank
-  constexpr uint32_t RB = sizeof(Rank);
-  // [CAP + 2] prefix sums; then [CAP + 2] ranks, times 8: of the heavy that is light r's alias, of the light that finishes heavy h;
-  // then [CAP + 2] the slot of heavy h.  A heavy's residual probability takes the place of its rank, or (NARROW) of its sum.
-  char* const s_v = reinterpret_cast<char*>(smem);
-  char* const s_rank = s_v + (CAP + 2) * 8;
-  char* const s_hs = s_rank + (CAP + 2) * RB;
-  auto val = [&](uint32_t at) -> double& { return *reinterpret_cast<double*>(s_v + at); };        // at: 8 * index
-  auto rank = [&](uint32_t at) -> Rank& { return *reinterpret_cast<Rank*>(s_rank + at); };  // RB * index
-  auto prob = [&](uint32_t at) -> uint32_t& {                                               // 8 * index
-    return *reinterpret_cast<uint32_t*>(NARROW ? s_v + at : s_rank + (at >> RSH));
-  };
-  auto slot_of = [&](uint32_t at) -> uint16_t& { return *reinterpret_cast<uint16_t*>(s_hs + at); };  // 2 * heavy rank
+  constexpr uint32_t TOP = CAP + 1, SZ = 8, B0 = SZ;  // light r at B0 + SZ * r, heavy h at B0 + SZ * (TOP - h)
+  static_assert(CAP < 8000 && PER % 2 == 0, "prefix sums below 2^53, offsets in 16 bits, whole pairs");
+  char* const s_v = reinterpret_cast<char*>(smem);  // one more at either end is read
+  constexpr bool WORDS = merge_words(ROWT, PER);
+  char* const s_w = s_v + (CAP + 4) * SZ;
+  char* const s_hs = WORDS ? s_w + (CAP + 4) * 4 : s_w;
+  auto val = [&](uint32_t at) -> double& { return *reinterpret_cast<double*>(s_v + at); };
+  auto word = [&](uint32_t at) -> uint32_t& { return *reinterpret_cast<uint32_t*>(WORDS ? s_w + (at >> 1) : s_v + at); };
+  auto slot_of = [&](uint32_t at) -> uint16_t& { return *reinterpret_cast<uint16_t*>(s_hs + (at >> 2)); };
 
   const uint32_t off = rr.off, d = rr.d;
   const int wave = tid >> 6, lane = tid & 63;
@@ -690,15 +679,16 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
     for (int j = 0; j < PER; ++j) {
       const double p = wd[j] * scale, t = fma(p, fs, neg_fs);  // = (p - 1) * 2^F rounded once: the product is exact
       hv[j] = t >= 0.5;
-      wd[j] = rint(max_abs_f64(t, hv[j] ? 1.0 : 0.0));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
+      const double one = hv[j] ? 1.0 : 0.0;
+      wd[j] = rint(max_abs_f64(t, one));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
       op[j] = (float)p;
       run += wd[j];
-      run_u += hv[j] ? wd[j] : 0.0;
+      run_u = fma(wd[j], one, run_u);  // exact: whole numbers below 2^53
       cnt += hv[j] ? 1u : 0u;
     }
   }
-  // what lies before this thread's slots: amounts, surpluses, heavies
-  double ex, ex_u;
+  // what lies before this thread's slots, and in the whole row: amounts, surpluses, heavies
+  double ex, ex_u, all, all_u;
   uint32_t ex_c, nh;
   {
     double* const s_p = reinterpret_cast<double*>(s_aux + 5 * NW);   // [2 * NW]
@@ -710,114 +700,116 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
     ex_c = ic - cnt;
     if (NW == 1) {
       nh = (uint32_t)__builtin_amdgcn_readlane((int)ic, 63);
+      all = lane_f64(i, 63);
+      all_u = lane_f64(iu, 63);
     } else {
       if (lane == 63) {
         s_p[2 * wave] = i;
         s_p[2 * wave + 1] = iu;
         s_c[wave] = ic;
       }
-      row_sync();
+      __syncthreads();
       nh = 0;
+      all = all_u = 0.0;
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
-        if (w < wave) {
-          ex += s_p[2 * w];
-          ex_u += s_p[2 * w + 1];
-          ex_c += s_c[w];
+        if (w == wave) {
+          ex += all;
+          ex_u += all_u;
+          ex_c += nh;
         }
+        all += s_p[2 * w];
+        all_u += s_p[2 * w + 1];
         nh += s_c[w];
       }
       nh = (uint32_t)__builtin_amdgcn_readfirstlane((int)nh);
     }
   }
   const uint32_t nl = slots - nh;  // the row's own come first: d - nh of them
-  uint32_t at[PER];                // 8 * index of the slot's value
+  const uint32_t end_l = B0 + SZ * nl, end_h = B0 + SZ * (TOP - nh);
+  // A heavy keeps itself when its prefix lies above the deficits of the row's own lights (a slot behind the row counts 2^40), or
+  // when it is the last, the only one whose prefix is all the surplus.
+  const double most = fmin(fma((double)(slots - d), -1099511627776.0, all - all_u), all_u - 1.0);
+  uint32_t at[PER];  // of a light's entry, of the one below a heavy's
+  bool self[PER];
   if (wave_on) {
-    uint32_t la = 8u * (k0 - ex_c), ha = 8u * (TOP - ex_c), hs = 2u * ex_c;
+    uint32_t la = B0 + SZ * (k0 - ex_c), below = B0 + SZ * (TOP - 1 - ex_c);
     double sl = ex - ex_u, sh = ex_u;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
-      at[j] = hv[j] ? ha : la;
+      at[j] = hv[j] ? below : la;
+      self[j] = false;
       if (hv[j]) {
         sh += wd[j];
-        val(ha) = sh;
-        slot_of(hs) = (uint16_t)(k0 + j);
-        ha -= 8u;
-        hs += 2u;
+        val(below + SZ) = sh;
+        slot_of(below + SZ) = (uint16_t)(k0 + j);
+        self[j] = sh > most;
+        below -= SZ;
       } else {
         sl += wd[j];
         val(la) = sl;
-        la += 8u;
+        la += SZ;
       }
     }
     if (lane == 63 && k0 + PER == slots) {
-      val(8u * nl) = __builtin_huge_val();
-      val(8u * (TOP - nh)) = __builtin_huge_val();
+      val(end_l) = __builtin_huge_val();
+      val(end_h) = __builtin_huge_val();
     }
   }
   row_sync();
 
+  uint32_t oa[PER];
   if (nh) {
+    uint32_t to[PER], x[PER];
     if (wave_on) {
-      // merged positions [k0, k0 + PER) belong to this thread; a lights and k0 - a heavies come before them
-      uint32_t a8;
-      {
-        const uint32_t lo = k0 > nh ? k0 - nh : 0u, hi8 = 8u * min(k0, nl), dh = 8u * (TOP - k0);
-        a8 = 8u * lo;
-        const uint32_t most = min(nh, nl);
+      // merged positions [k0, k0 + PER) belong to this thread; some lights, the next of which is at a, and k0 less so many
+      // heavies, the next of which is at q, come before them
+      const uint32_t hi = B0 + SZ * min(k0, nl), dq = SZ * (TOP - k0), fewer = min(nh, nl);
+      uint32_t a = B0 + SZ * (k0 > nh ? k0 - nh : 0u);
 #pragma unroll
-        for (uint32_t step = 1u << (31 - __builtin_clz(CAP / 2)); step >= 1; step >>= 1) {
-          if (step <= most) {  // uniform
-            const uint32_t to = a8 + 8u * step;
-            const bool up = val(a8 + 8u * (step - 1)) < val(a8 + dh + 8u * step);
-            a8 = up && to <= hi8 ? to : a8;
-          }
+      for (uint32_t step = 1u << (31 - __builtin_clz(CAP / 2)); step >= 1; step >>= 1) {
+        if (step <= fewer) {  // uniform
+          const uint32_t up = min(a + SZ * step, hi);
+          a = val(up - SZ) < val(up + dq) ? up : a;
         }
       }
-      const uint32_t dh = 8u * (TOP - k0 - (PER - 1));  // the heavy at hand lies so far behind the light at hand, and 8 bytes less in every step
-      uint32_t rh = RB * (TOP - k0), k8 = 8u * k0;
+      uint32_t q = a + dq;
 #pragma unroll
       for (int s = 0; s < PER; ++s) {
-        const bool take = val(a8 + dh + 8u * (PER - 1 - s)) <= val(a8);  // the heavy
-        rank((a8 >> RSH) + (take ? rh : RB)) = (Rank)(take ? a8 : k8 - a8);
-        a8 += take ? 0u : 8u;
-        rh -= RB;
-        k8 += 8u;
+        const double vl = val(a), vh = val(q);
+        const bool take = vh <= vl;  // the heavy
+        const float p = (float)fma(vl - vh, -1.0 / 1099511627776.0, 1.0);
+        const uint32_t an = a + SZ, qn = q - SZ;
+        to[s] = take ? qn : an;
+        x[s] = take ? __float_as_uint(p) : q;
+        if (WORDS) word(to[s]) = x[s];
+        a = take ? a : an;
+        q = take ? qn : q;
       }
     }
-    if (tid == 0) {
-      rank(0) = 0;                                   // the first light starts in the first heavy
-      slot_of(2u * nh) = slot_of(2u * (nh - 1));    // a light beyond every heavy takes the last
-    }
-    row_sync();
-    // heavies, densely by rank: residual probability from the light that finishes them
-    for (uint32_t h = tid; h < nh; h += ROWT) {
-      const uint32_t i = TOP - h, r = rank(RB * i);
-      const float p = (float)fma(val(r) - val(8u * i), -1.0 / 1099511627776.0, 1.0);
-      prob(8u * i) = h + 1 < nh && r < 8u * (d - nh) ? __float_as_uint(p) : MERGE_SELF;
-    }
-    row_sync();
-  }
-
-  uint32_t oa[PER];
-  if (wave_on) {
+    if (tid == 0) slot_of(end_h) = slot_of(end_h + SZ);  // a light beyond every heavy takes the last
+    if (!WORDS) {
+      row_sync();
+      if (wave_on) {
 #pragma unroll
-    for (int j = 0; j < PER; ++j) {
-      oa[j] = k0 + j;
-      if (nh) {
-        const uint32_t x = NARROW ? (hv[j] ? prob(at[j]) : (uint32_t)rank(at[j] >> RSH)) : (uint32_t)rank(at[j] >> RSH);
-        const uint32_t m = slot_of((hv[j] ? 8u * (TOP + 1) - at[j] : x) >> 2);
-        if (hv[j]) {
-          const bool self = x == MERGE_SELF;
-          op[j] = self ? 1.0f : __uint_as_float(x);
-          oa[j] = self ? oa[j] : m;
-        } else {
-          oa[j] = m;
-        }
+        for (int s = 0; s < PER; ++s) word(to[s]) = x[s];
       }
     }
+    if (tid == 0) word(B0) = B0 + SZ * TOP;  // the first light starts in the first heavy
+    row_sync();
+    if (wave_on) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const uint32_t w = word(at[j]), m = slot_of(hv[j] ? at[j] : w);
+        oa[j] = self[j] ? k0 + j : m;
+        if (hv[j]) op[j] = self[j] ? 1.0f : __uint_as_float(w);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < PER; ++j) oa[j] = k0 + j;
   }
-  if (NW > 1 && NARROW) row_sync();  // the entries take the place of the values
+  if (!WORDS || NW == 1) row_sync();  // the entries take the place of the sums
   if (wave_on) wave_store<PER>(table + off, wfirst, d, s_v + PER * 512 * wave, lane, op, oa);
   return true;
 }
