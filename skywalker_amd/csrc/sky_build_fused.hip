@@ -530,6 +530,10 @@ constexpr uint64_t ALL_MOST = 4096;
 constexpr uint32_t ALL_LONGEST = 12288;
 static_assert(ALL_LONGEST <= 24576, "none is of class CLS_STREAM");
 
+// Rows of 5118..8189 entries from which they are a launch of their own (10,000 rows of 6,500 streamed 478 us, held 402; 20,000
+// 885 and 745): fewer save less than a launch costs.
+constexpr uint32_t HOLD_ALONE = 2048;
+
 // Frontiers of at most this many rows make the rows of 8190..65533 entries tile by tile.
 constexpr uint32_t SMALL_FRONTIER = 65536;
 
@@ -752,10 +756,10 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   pair.add(SEC_P6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
   wide.add(SEC_SCAN, n_trows, 1, 0);
   if (p.t_all != CLS_STREAM) wide.add(SEC_STREAM, rows(CLS_STREAM) + rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM]);
-  // Rows of 5118..8189 entries are streamed here: hold_row beside the others would spill 190 registers.  It is no loss: builds
-  // of such rows alone take 55 (4 M entries), 129 (17 M), 435..477 (67 M) and 840..902 us (134 M) this way, 121, 194, 554 and
-  // 1018 us with build_hold_kernel and the row lists in place.
-  wide.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);
+  // Rows of 5118..8189 entries: streamed beside the others, where hold_row would spill, or, where they are enough for a launch,
+  // HOLD_ALONE, by build_hold_kernel.
+  const bool hold_alone = min_degree == 0 && rows(CLS_HOLD) >= HOLD_ALONE;  // behind the sweep, which notes when the call began
+  if (!hold_alone) wide.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);
   // two classes whose lists lie back to back; min_degree may leave out the first
   auto add_two = [&](Section k, int c) { wide.add(k, rows(c) + rows(c + 1), 1, p.start[rows(c) ? c : c + 1]); };
   add_two(SEC_B10, CLS_MW2 + 7);
@@ -765,7 +769,8 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   block.add(SEC_M10, rows(CLS_MW2 + 3), 1, p.start[CLS_MW2 + 3]);
   block.add(SEC_M8, rows(CLS_MW2 + 2), 1, p.start[CLS_MW2 + 2]);
   block.add(SEC_M6, rows(CLS_MW2 + 1), 1, p.start[CLS_MW2 + 1]);
-  return launch_all<false>(g, p, wave, pair, wide, block, call);
+  SKY_TRY(launch_all<false>(g, p, wave, pair, wide, block, call));
+  return hold_alone ? build_rows_hold(g, p.rows + p.start[CLS_HOLD], rows(CLS_HOLD)) : SKY_OK;
 }
 int build_all_fused(sky_graph* g, CallDevice* call) { return build_host_sized(g, 0, call); }
 int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call) { return build_host_sized(g, min_degree, call); }

@@ -492,6 +492,21 @@ def test_builds_in_four_launches(orc, dist, stream_min_edges):
     g.free()
 
 
+@pytest.mark.parametrize("n", [2047, 2048])
+def test_many_rows_that_one_workgroup_holds(orc, n):
+    # from 2,048 rows of 5,118..8,189 entries on they are a launch of their own behind the four
+    rng = np.random.default_rng(47)
+    degs = [5118, 5119, 8188, 8189] * (n // 4) + [6000] * (n % 4) + [12289, 1, 2, 3, 40, 700] + list(rng.integers(0, 40, 3000))
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal", V=len(degs))
+    w[xadj[100]:xadj[110]] = 0.0
+    from skywalker_amd import capi
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, "held rows/%d" % n)
+    g.free()
+
+
 @pytest.mark.parametrize("longest", [509, 510, 12288, 12289])
 @pytest.mark.parametrize("dist", ["lognormal2", "fewlights", "sparse"])
 def test_small_builds_in_one_launch(orc, dist, longest):
