@@ -73,12 +73,13 @@ KERNEL_OF = {  # build_profile entry -> kernel symbol
     "tiled_totals": "tiled_totals_kernel", "tiled_emit": "tiled_scan_kernel+tiled_emit_kernel",
     "streamed": "huge_prefix_kernel+build_huge_kernel", "stream": "build_stream_kernel", "hold": "build_hold_kernel",
 }
-KERNEL_OF.update({"g%d%s" % (g, x): "build_group_kernel<%d,%d>" % (g, 6 if x else 4)
-                  for g in (2, 4, 8, 16, 32) for x in ("", "x")})
-KERNEL_OF.update({"g32s": "build_group_kernel<32,5>"})
+KERNEL_OF.update({"g2": "build_group_kernel<2,4>", "g4": "build_group_kernel<4,4>", "g8": "build_group_kernel<8,4>",
+                  "g16": "build_group_kernel<8,8>", "g32": "build_group_kernel<16,8>", "g32s": "build_group_kernel<32,5>",
+                  "g32x": "build_group_kernel<32,6>"})
 KERNEL_OF.update({"mw%d" % nw: "build_merge_kernel<%d,8>" % (64 * nw) for nw in range(2, 11)})
 KERNEL_OF.update({"mw3": "build_merge_kernel<256,6>", "mw5": "build_merge_kernel<256,10>", "mw6": "build_merge_kernel<512,6>",
-                  "mw7": "build_merge_kernel<256,14>", "mw9": "build_merge_kernel<768,6>", "mw10": "build_merge_kernel<512,10>"})
+                  "mw7": "build_merge_kernel<256,14>", "mw10": "build_merge_kernel<512,10>"})
+SAME_KERNEL = {"mw9": "mw10"}  # two classes of rows, one kernel
 
 
 def cpu_model():
@@ -386,8 +387,10 @@ def main():
     for _ in range(psteps):
         g.build_tables()
         for nm, ms, edges in g.build_profile():
-            p = prof.setdefault(nm, [0.0, edges])
+            p = prof.setdefault(SAME_KERNEL.get(nm, nm), [0.0, {}])
             p[0] += ms / psteps
+            p[1][nm] = edges
+    prof = {k: [ms, sum(edges.values())] for k, (ms, edges) in prof.items()}
     capi.set_option("build_profile", 0)
 
     # the same walks with the optional 16-byte walk index, and with live walkers handed from launch to launch:
