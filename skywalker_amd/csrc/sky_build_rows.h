@@ -143,8 +143,12 @@ __device__ __forceinline__ void quad_exchange(uint32_t tid, const float (&p)[8],
 }
 
 // ---------------------------------------------------------------- sums as doubles
-// Prefix sums of a row's amounts are whole numbers below 2^53 in rows of at most 2^13 slots: doubles hold them exactly, an
-// amount is one rounding instead of an addition and a mask, a residual one fused multiply-add instead of a conversion.
+// An amount is one rounding instead of an addition and a mask, a residual one fused multiply-add instead of a conversion.
+// Deficits and surpluses are summed apart.  A light, and a slot behind the row, has a deficit of at most 2^40: in fewer than 2^13
+// slots every sum of deficits is a whole number below 2^53, which a double holds.  The surpluses add up to as much where every
+// weight counts, so that both together pass 2^53; where weights below 2^-64, which add nothing to the row's sum, have shares
+// all the same they add up to more by themselves.  A sum of surpluses below 2^53 is exact in whatever order it was added, and
+// one that was rounded is at least 2^53 (rounding is monotone): above every deficit prefix, which is all that is asked of it.
 template <int G>
 __device__ __forceinline__ double group_scan_f64(double v) {
   const int gl = lane_id() & (G - 1);
@@ -279,31 +283,31 @@ __device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const 
 
   float op[PER];
   bool hv[PER];
-  double run = 0.0, run_u = 0.0;  // amounts of this lane's slots, of its heavies
+  double run_d = 0.0, run_u = 0.0;  // deficits and surpluses of this lane's slots
   uint32_t cnt = 0;
 #pragma unroll
   for (int k = 0; k < PER; ++k) {
     const double p = wd[k] * scale, t = fma(p, fs, neg_fs);  // = (p - 1) * 2^F rounded once: the product is exact
     hv[k] = t >= 0.5;
-    const double one = hv[k] ? 1.0 : 0.0;
-    wd[k] = rint(max_abs_f64(t, one));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
+    const double heavy = hv[k] ? 1.0 : 0.0, light = hv[k] ? 0.0 : 1.0;
+    wd[k] = rint(max_abs_f64(t, heavy));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
     op[k] = (float)p;
-    run += wd[k];
-    run_u = fma(wd[k], one, run_u);  // exact: whole numbers below 2^53
+    run_d = fma(wd[k], light, run_d);
+    run_u = fma(wd[k], heavy, run_u);
     cnt += hv[k] ? 1u : 0u;
   }
-  const double i = group_scan_f64<G>(run), iu = group_scan_f64<G>(run_u);
+  const double id = group_scan_f64<G>(run_d), iu = group_scan_f64<G>(run_u);
   const uint32_t ic = group_scan_u32<G>(cnt);
   const uint32_t nh = (uint32_t)__shfl((int)ic, (int)last_lane, 64), nl = SLOTS - nh;
   // A heavy keeps itself when its prefix lies above the deficits of the row's own lights (a slot behind the row counts 2^40), or
   // when it is the last, the only one whose prefix is all the surplus.
-  const double most = lane_shfl_f64(fmin(fma((double)(SLOTS - d), neg_fs, i - iu), iu - 1.0), (int)last_lane);
+  const double most = lane_shfl_f64(fmin(fma((double)(SLOTS - d), neg_fs, id), iu - 1.0), (int)last_lane);
   uint32_t at[PER];  // of a light's entry, of the one below a heavy's
   bool self[PER];
   {
     const uint32_t ex_c = ic - cnt;
     uint32_t la = strip + SZ * (pos - ex_c), below = strip + SZ * (TOP - 1 - ex_c);
-    double sh = iu - run_u, sl = i - run - sh;
+    double sh = iu - run_u, sl = id - run_d;
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       at[k] = hv[k] ? below : la;
@@ -593,7 +597,7 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
   };
   constexpr int NW = ROWT / 64;
   constexpr uint32_t TOP = CAP + 1, SZ = 8, B0 = SZ;  // light r at B0 + SZ * r, heavy h at B0 + SZ * (TOP - h)
-  static_assert(CAP < 8000 && PER % 2 == 0, "prefix sums below 2^53, offsets in 16 bits, whole pairs");
+  static_assert(CAP < 8000 && PER % 2 == 0, "sums of deficits below 2^53, offsets in 16 bits, whole pairs");
   char* const s_v = reinterpret_cast<char*>(smem);  // one more at either end is read
   constexpr bool WORDS = merge_words(ROWT, PER);
   char* const s_w = s_v + (CAP + 4) * SZ;
@@ -669,7 +673,7 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
 
   float op[PER];
   bool hv[PER];
-  double run = 0.0, run_u = 0.0;  // amounts of this thread's slots, of its heavies
+  double run_d = 0.0, run_u = 0.0;  // deficits and surpluses of this thread's slots
   uint32_t cnt = 0;
   if (wave_on) {
     const double scale = (double)d / rsum;
@@ -679,46 +683,46 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
     for (int j = 0; j < PER; ++j) {
       const double p = wd[j] * scale, t = fma(p, fs, neg_fs);  // = (p - 1) * 2^F rounded once: the product is exact
       hv[j] = t >= 0.5;
-      const double one = hv[j] ? 1.0 : 0.0;
-      wd[j] = rint(max_abs_f64(t, one));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
+      const double heavy = hv[j] ? 1.0 : 0.0, light = hv[j] ? 0.0 : 1.0;
+      wd[j] = rint(max_abs_f64(t, heavy));  // |t| < 0.5 for a light with t > 0: rounds to the deficit 0
       op[j] = (float)p;
-      run += wd[j];
-      run_u = fma(wd[j], one, run_u);  // exact: whole numbers below 2^53
+      run_d = fma(wd[j], light, run_d);
+      run_u = fma(wd[j], heavy, run_u);
       cnt += hv[j] ? 1u : 0u;
     }
   }
-  // what lies before this thread's slots, and in the whole row: amounts, surpluses, heavies
-  double ex, ex_u, all, all_u;
+  // what lies before this thread's slots, and in the whole row: deficits, surpluses, heavies
+  double ex_d, ex_u, all_d, all_u;
   uint32_t ex_c, nh;
   {
     double* const s_p = reinterpret_cast<double*>(s_aux + 5 * NW);   // [2 * NW]
     uint32_t* const s_c = reinterpret_cast<uint32_t*>(s_aux + 7 * NW);  // [NW]
-    const double i = wave_scan_f64(run), iu = wave_scan_f64(run_u);
+    const double id = wave_scan_f64(run_d), iu = wave_scan_f64(run_u);
     const uint32_t ic = group_scan_u32<64>(cnt);
-    ex = i - run;
+    ex_d = id - run_d;
     ex_u = iu - run_u;
     ex_c = ic - cnt;
     if (NW == 1) {
       nh = (uint32_t)__builtin_amdgcn_readlane((int)ic, 63);
-      all = lane_f64(i, 63);
+      all_d = lane_f64(id, 63);
       all_u = lane_f64(iu, 63);
     } else {
       if (lane == 63) {
-        s_p[2 * wave] = i;
+        s_p[2 * wave] = id;
         s_p[2 * wave + 1] = iu;
         s_c[wave] = ic;
       }
       __syncthreads();
       nh = 0;
-      all = all_u = 0.0;
+      all_d = all_u = 0.0;
 #pragma unroll
       for (int w = 0; w < NW; ++w) {
         if (w == wave) {
-          ex += all;
+          ex_d += all_d;
           ex_u += all_u;
           ex_c += nh;
         }
-        all += s_p[2 * w];
+        all_d += s_p[2 * w];
         all_u += s_p[2 * w + 1];
         nh += s_c[w];
       }
@@ -729,12 +733,12 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
   const uint32_t end_l = B0 + SZ * nl, end_h = B0 + SZ * (TOP - nh);
   // A heavy keeps itself when its prefix lies above the deficits of the row's own lights (a slot behind the row counts 2^40), or
   // when it is the last, the only one whose prefix is all the surplus.
-  const double most = fmin(fma((double)(slots - d), -1099511627776.0, all - all_u), all_u - 1.0);
+  const double most = fmin(fma((double)(slots - d), -1099511627776.0, all_d), all_u - 1.0);
   uint32_t at[PER];  // of a light's entry, of the one below a heavy's
   bool self[PER];
   if (wave_on) {
     uint32_t la = B0 + SZ * (k0 - ex_c), below = B0 + SZ * (TOP - 1 - ex_c);
-    double sl = ex - ex_u, sh = ex_u;
+    double sl = ex_d, sh = ex_u;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       at[j] = hv[j] ? below : la;

@@ -531,6 +531,70 @@ def test_small_builds_in_one_launch(orc, dist, longest):
     g.free()
 
 
+def few_carry_the_mass(d, k0, e):
+    """Shares of the mean weight, in units of 2^-40 all whole: one heavy, then lights whose deficits reach its surplus as the last
+    of them is taken, e units more.  Deficits and surpluses together pass 2^53 on the way there for d > 4103, at an odd number."""
+    u, n0 = 2.0 ** -40, d - 8
+    share = np.zeros(d)
+    share[:4] = [k0 * u, n0 + 4 - 2.0 ** -10, 1.5, (2 ** 30 - 2 ** 24) * u]
+    share[4 + n0:] = [(2 ** 24 - k0 - e) * u, 2.0, 0.5 - 2.0 ** -20, (2 ** 20 + e) * u]
+    w = share.astype(np.float32)
+    assert np.array_equal(w.astype(np.float64), share) and share.sum() == d  # so that the scale is 1
+    return w
+
+
+def below_the_grid(d, k0, e):
+    """The same meeting of a light and a heavy, d a power of two, with heavies between that add nothing to the row's sum (their
+    weights are below 2^-64) and have a surplus of 0.75 d each: 0.6 d^2 altogether, past 2^53 units for d >= 128."""
+    u, share = 2.0 ** -40, np.full(d, 0.25)
+    h = d - d // 8
+    share[:3] = [k0 * u, 3 - 2.0 ** -22, 1.5]
+    share[3:h] = 0.75 * d
+    share[3] = d  # a weight of 2^-64: the row's sum
+    share[h] = (2 ** 18 - k0 - e) * u
+    w = (share * (2.0 ** -64 / d)).astype(np.float32)
+    assert np.array_equal(w.astype(np.float64), share * (2.0 ** -64 / d))
+    return w
+
+
+def skewed_rows():
+    rows = [few_carry_the_mass(d, k0, e) for d in (3777, 4093, 4094, 4103, 4104, 4605, 4606, 5117) for k0 in (1, 3) for e in (-1, 0)]
+    # in rows like these the last bit of one probability differed
+    rows += [np.random.default_rng(s).lognormal(0, sigma, 5117).astype(np.float32) for s, sigma in ((49, 4), (2891, 3), (3448, 6))]
+    rng = np.random.default_rng(61)
+    return rows + [rng.lognormal(0, sigma, d).astype(np.float32) for sigma in (3, 4, 6) for d in rng.integers(3070, 5118, 20)]
+
+
+def vanishing_rows():
+    rows = [below_the_grid(d, k0, e) for d in (64, 128, 256, 512, 1024, 2048, 4096) for k0 in (1, 3, 5, 7) for e in (-1, 0)]
+    rng, u = np.random.default_rng(62), 2.0 ** -64
+    for d in [100, 128, 129, 192, 193, 381, 509, 765, 1021, 2045, 3069, 3581, 4093, 5117] + list(rng.integers(100, 5118, 20)):
+        share = np.concatenate([1 + rng.uniform(0, 2.0 ** -19, d // 5), rng.uniform(0.5, 0.99, d // 2) * d,
+                                rng.uniform(0, 0.001, d - d // 5 - d // 2)])
+        share[d // 3] = d
+        rows.append((share * (u / d)).astype(np.float32))
+    return rows
+
+
+@pytest.mark.parametrize("route", ["by class", "four launches", "one launch"])
+@pytest.mark.parametrize("make", [skewed_rows, vanishing_rows])
+def test_rows_whose_sums_need_every_bit(orc, make, route):
+    # rows whose deficits and surpluses together, or whose surpluses alone, add up to 2^53 units and more: the sums that decide
+    # aliases and residuals are below that and exact in every kernel
+    from skywalker_amd import capi
+    rows = make()
+    if route == "four launches":  # a row too long for one
+        rows.append(np.ones(12289, np.float32))
+    w = np.concatenate(rows)
+    xadj = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.uint32)
+    g = capi.Graph.upload(xadj, np.zeros(len(w), np.uint32), w)
+    if route == "by class":
+        g.set_option("small_in_place", 0)
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, "%s, %s" % (make.__name__, route))
+    g.free()
+
+
 @pytest.mark.parametrize("degree", [2048 * 1024 - 3, 2048 * 1024 + 1])
 def test_ledger_of_rows_of_very_many_tiles_in_four_launches(orc, degree):
     # up to 2048 tiles every tile adds up its row's sums itself, above a launch in between does
