@@ -165,6 +165,10 @@ __device__ __forceinline__ double group_scan_f64(double v) {
   return v;
 }
 __device__ __forceinline__ double wave_scan_f64(double v) { return group_scan_f64<64>(v); }
+// The value of the lane before, 0 in lane 0.
+__device__ __forceinline__ double lane_before_f64(double v) {
+  return __longlong_as_double((long long)dpp0_u64<DPP_WAVE_SHR1, 0xF>((uint64_t)__double_as_longlong(v)));
+}
 __device__ __forceinline__ double lane_f64(double v, int lane) {
   const uint64_t b = (uint64_t)__double_as_longlong(v);
   const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)b, lane);
@@ -224,6 +228,10 @@ __device__ __forceinline__ bool group_build_row(uint32_t off, uint32_t d, const 
   static_assert((PER >= 4 && PER <= 6) || PER == 8, "a lane loads one float4 (and one float), two, or three float2");
   constexpr uint32_t SLOTS = PER * G, STRIDE = SLOTS + 2, TOP = SLOTS + 1;
   static_assert(SLOTS <= 256, "slots in 8 bits");
+  // A lane's surpluses are at most (PER + 2) d shares of 2^40 (a weight that counts in part has up to 2 d shares, all of them
+  // together): where the prefix up to them was rounded, the one before them lies above every deficit prefix too, and so does
+  // their difference.
+  static_assert((PER + 3) * SLOTS < 8192, "the surpluses before a lane may be got by subtraction");
   constexpr uint32_t SZ = 8, N = group_entries(G, PER, BLOCK);
   char* const s_v = reinterpret_cast<char*>(smem);
   auto val = [&](uint32_t at) -> double& { return *reinterpret_cast<double*>(s_v + at); };
@@ -700,7 +708,7 @@ __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint6
     const double id = wave_scan_f64(run_d), iu = wave_scan_f64(run_u);
     const uint32_t ic = group_scan_u32<64>(cnt);
     ex_d = id - run_d;
-    ex_u = iu - run_u;
+    ex_u = lane_before_f64(iu);  // not iu - run_u: a thread's own surpluses may take the prefix past 2^53
     ex_c = ic - cnt;
     if (NW == 1) {
       nh = (uint32_t)__builtin_amdgcn_readlane((int)ic, 63);

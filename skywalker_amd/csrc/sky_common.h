@@ -279,7 +279,8 @@ __device__ __forceinline__ uint64_t shfl_up_u64(uint64_t v, int delta) {
   return ((uint64_t)hi << 32) | lo;
 }
 // ---- DPP building blocks.  A wave is four rows of 16 lanes; row_shr:n moves data n lanes up inside a
-// row, row_bcast15 / row_bcast31 carry the last lane of a row (of the first half) to the next row(s).
+// row, wave_shr:1 one lane up in the whole wave, row_bcast15 / row_bcast31 carry the last lane of a row (of the first half) to
+// the next row(s).
 // Lanes without a source, and rows masked off, receive 0.  Callers must be convergent (all 64 lanes
 // active): a DPP read from a disabled lane is not defined.
 template <int CTRL, int ROW_MASK>
@@ -293,7 +294,7 @@ __device__ __forceinline__ uint64_t dpp0_u64(uint64_t v) {
   return (uint64_t)__builtin_amdgcn_update_dpp((uint64_t)0, v, CTRL, ROW_MASK, 0xF, true);
 }
 constexpr int DPP_ROW_SHR1 = 0x111, DPP_ROW_SHR2 = 0x112, DPP_ROW_SHR4 = 0x114, DPP_ROW_SHR8 = 0x118;
-constexpr int DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143;
+constexpr int DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143, DPP_WAVE_SHR1 = 0x138;
 constexpr int DPP_QUAD_XOR1 = 0xB1 /* quad_perm [1,0,3,2] */, DPP_QUAD_XOR2 = 0x4E /* quad_perm [2,3,0,1] */;
 constexpr int DPP_ROW_HALF_MIRROR = 0x141, DPP_ROW_MIRROR = 0x140;
 

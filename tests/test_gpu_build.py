@@ -576,8 +576,28 @@ def vanishing_rows():
     return rows
 
 
+def surpluses_that_leap(d, k, rng):
+    """Heavies of a little surplus up to slot k, one light that all of them fall to, then forty heavies of some d / 3 shares each: the
+    prefix of a thread that holds some of both kinds passes 2^53, what lies before it is a small odd number of units."""
+    u, one = np.float32(2.0 ** -64), np.float32(3 * 2.0 ** -64 / d)  # one: the least heavy weight, or the largest light one
+    w = (rng.uniform(0, 1, d) * one).astype(np.float32)
+    w[0] = 0.0
+    w[1:k] = one
+    for i in range(1, k):
+        for _ in range(1 + int(rng.integers(3))):
+            w[i] = np.nextafter(w[i], np.float32(1))
+    w[k:k + 40] = rng.uniform(0.9, 0.99, 40) * u
+    w[k + 40] = 3 * u  # the row's sum
+    return w
+
+
+def leaping_rows():
+    return [surpluses_that_leap(d, k, np.random.default_rng(k)) for d in (1021, 2557, 3100, 3581, 3800, 4093, 4094, 5117)
+            for k in range(5, 30)]
+
+
 @pytest.mark.parametrize("route", ["by class", "four launches", "one launch"])
-@pytest.mark.parametrize("make", [skewed_rows, vanishing_rows])
+@pytest.mark.parametrize("make", [skewed_rows, vanishing_rows, leaping_rows])
 def test_rows_whose_sums_need_every_bit(orc, make, route):
     # rows whose deficits and surpluses together, or whose surpluses alone, add up to 2^53 units and more: the sums that decide
     # aliases and residuals are below that and exact in every kernel
