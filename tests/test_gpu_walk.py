@@ -72,6 +72,31 @@ def test_walkers_with_a_wavefront_each(orc, n, length, stop, index):
     assert np.array_equal(paths, opaths)
 
 
+@pytest.mark.parametrize("entries", [(4 << 20) // 8, (4 << 20) // 8 + 1])
+@pytest.mark.parametrize("n,length", [(4096, 24), (4097, 23), (4097, 24), (8192, 70), (8193, 24)])
+def test_thousands_of_walkers_with_a_wavefront_each(orc, n, length, entries):
+    # where the tables take more than 4 MB and the walk has 24 steps or more, up to 8,192 walkers have a wavefront each: both sides
+    # of each of the three limits
+    from skywalker_amd import capi
+    rng = np.random.default_rng(n + length)
+    V = 20000
+    degs = rng.integers(0, 50, V)
+    degs[-1] = entries - degs[:-1].sum()
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "sparse", V=V)
+    assert len(w) == entries and degs[-1] > 0
+    w[xadj[10]:xadj[40]] = 0.0
+    seeds = rng.integers(0, V + 20, n, dtype=np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    prob, alias, _ = g.tables()
+    paths_d, len_d, sampled, _ = g.walk_offline(seeds, length, 0.01, 13)
+    paths, lengths = paths_d.to_host((n, length + 1)), len_d.to_host()
+    g.free()
+    opaths, olengths, osampled = orc.walk_offline(xadj, adjncy, prob, alias, seeds, length, 0.01, 13)
+    assert np.array_equal(lengths, olengths) and sampled == osampled
+    assert np.array_equal(paths, opaths)
+
+
 def test_dead_ends_and_zero_weight_rows(orc):
     # path graph 0 -> 1 -> 2 -> 3 (3 has no out-edge); vertex 4 has one zero-weight edge; 5 loops on itself
     xadj = np.array([0, 1, 2, 3, 3, 4, 5], np.uint32)
