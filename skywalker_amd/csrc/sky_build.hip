@@ -339,7 +339,7 @@ __global__ __launch_bounds__(ROWT) void build_lds_kernel(const RowRef* __restric
     }
   }
   uint64_t total_l, total_h;
-  block_scan2<ROWT, T>(dl, dh, s_ex, sl, sh, total_l, total_h, wave_live);  // its barrier also publishes s_fh / s_lh
+  block_scan2<ROWT, T, false>(dl, dh, s_ex, sl, sh, total_l, total_h, wave_live);  // its barrier also publishes s_fh / s_lh
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     const uint32_t pos = 4u * (t * ROWT + tid);
@@ -495,22 +495,22 @@ __global__ __launch_bounds__(HUGE_T) void build_huge_kernel(const RowRef* __rest
         const Entry e = classify(clamp_weight(wr[i]), L);
         if (e.heavy) dh = e.amount; else dl = e.amount;
       }
-      const uint64_t il = group_scan_u64<64>(dl), ih = group_scan_u64<64>(dh);
+      const uint64_t il = group_scan_u64<64>(dl), ih = group_scan_sat_u64<64>(dh);
       __syncthreads();
       if (lane == 63) { s_wl[wave] = il; s_wh[wave] = ih; }
       __syncthreads();
       uint64_t bl = carry_l, bh = carry_h, tl = 0, th = 0;
       for (int k = 0; k < NW; ++k) {
-        if (k == wave) { bl += tl; bh += th; }
+        if (k == wave) { bl += tl; bh = add_sat(bh, th); }
         tl += s_wl[k];
-        th += s_wh[k];
+        th = add_sat(th, s_wh[k]);
       }
       if (i < d) {
         g_sl[i] = bl + il;
-        g_sh[i] = bh + ih;
+        g_sh[i] = add_sat(bh, ih);
       }
       carry_l += tl;
-      carry_h += th;
+      carry_h = add_sat(carry_h, th);
     }
     const uint64_t total_h = carry_h;
     __threadfence();

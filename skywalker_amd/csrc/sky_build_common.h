@@ -8,10 +8,10 @@ namespace sky {
 constexpr uint32_t NONE32 = 0xFFFFFFFFu;
 
 // Inclusive prefixes of two quantities over the slots of a tile held as [Q][4] per thread (slot order:
-// quad q of thread tid, then thread tid + 1; sub-tile q before q + 1).  One barrier.
+// quad q of thread tid, then thread tid + 1; sub-tile q before q + 1).  The second is surpluses (SAT: add_sat).  One barrier.
 // Bit q of `wave_live` (wave-uniform) clear means every value of this wave in sub-tile q is zero:
 // the wave then skips that sub-tile's scan.
-template <int ROWT, int Q>
+template <int ROWT, int Q, bool SAT>
 __device__ __forceinline__ void block_scan2(const uint64_t (&a)[Q][4], const uint64_t (&b)[Q][4],
                                             uint64_t* __restrict__ s_ex /* [2 * Q * ROWT/64] */,
                                             uint64_t (&oa)[Q][4], uint64_t (&ob)[Q][4], uint64_t& tot_a,
@@ -32,18 +32,18 @@ __device__ __forceinline__ void block_scan2(const uint64_t (&a)[Q][4], const uin
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       ra += a[q][k];
-      rb += b[q][k];
+      rb = add_sat<SAT>(rb, b[q][k]);
       oa[q][k] = ra;
       ob[q][k] = rb;
     }
     ia[q] = group_scan_u64<64>(ra);
-    ib[q] = group_scan_u64<64>(rb);
+    ib[q] = group_scan_sat_u64<64, SAT>(rb);
     if (lane == 63) {
       s_ex[(q * NW + wave) * 2] = ia[q];
       s_ex[(q * NW + wave) * 2 + 1] = ib[q];
     }
-    ia[q] -= ra;  // exclusive over the lanes of this wave
-    ib[q] -= rb;
+    ia[q] -= ra;
+    ib[q] = before_own<SAT>(ib[q], rb);  // exclusive over the lanes of this wave
   }
   __syncthreads();
   uint64_t run_a = 0, run_b = 0;
@@ -53,15 +53,15 @@ __device__ __forceinline__ void block_scan2(const uint64_t (&a)[Q][4], const uin
     for (int w = 0; w < NW; ++w) {
       if (w == wave) {
         ia[q] += run_a;
-        ib[q] += run_b;
+        ib[q] = add_sat<SAT>(ib[q], run_b);
       }
       run_a += s_ex[(q * NW + w) * 2];
-      run_b += s_ex[(q * NW + w) * 2 + 1];
+      run_b = add_sat<SAT>(run_b, s_ex[(q * NW + w) * 2 + 1]);
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       oa[q][k] += ia[q];
-      ob[q][k] += ib[q];
+      ob[q][k] = add_sat<SAT>(ob[q][k], ib[q]);
     }
   }
   tot_a = run_a;
@@ -93,8 +93,8 @@ __device__ __forceinline__ void search4(const uint64_t* s, const uint32_t (&base
 }
 
 
-// Single-quantity form of block_scan2.
-template <int ROWT, int Q>
+// Single-quantity form of block_scan2.  SAT: of surpluses.
+template <int ROWT, int Q, bool SAT>
 __device__ __forceinline__ void block_scan1(const uint64_t (&a)[Q][4], uint64_t* __restrict__ s_ex /* [Q * ROWT/64] */,
                                             uint64_t base, uint64_t (&oa)[Q][4]) {
   constexpr int NW = ROWT / 64;
@@ -105,12 +105,12 @@ __device__ __forceinline__ void block_scan1(const uint64_t (&a)[Q][4], uint64_t*
     uint64_t ra = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-      ra += a[q][k];
+      ra = add_sat<SAT>(ra, a[q][k]);
       oa[q][k] = ra;
     }
-    ia[q] = group_scan_u64<64>(ra);
+    ia[q] = group_scan_sat_u64<64, SAT>(ra);
     if (lane == 63) s_ex[q * NW + wave] = ia[q];
-    ia[q] -= ra;
+    ia[q] = before_own<SAT>(ia[q], ra);
   }
   __syncthreads();
   uint64_t run = base;
@@ -118,11 +118,11 @@ __device__ __forceinline__ void block_scan1(const uint64_t (&a)[Q][4], uint64_t*
   for (int q = 0; q < Q; ++q) {
 #pragma unroll
     for (int w = 0; w < NW; ++w) {
-      if (w == wave) ia[q] += run;
-      run += s_ex[q * NW + w];
+      if (w == wave) ia[q] = add_sat<SAT>(ia[q], run);
+      run = add_sat<SAT>(run, s_ex[q * NW + w]);
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) oa[q][k] += ia[q];
+    for (int k = 0; k < 4; ++k) oa[q][k] = add_sat<SAT>(oa[q][k], ia[q]);
   }
 }
 

@@ -218,34 +218,39 @@ __device__ __forceinline__ void tile_totals_wave(const FusedArgs& a, uint32_t ti
     }
   }
   if (!ok) return;
-  uint64_t sd = 0, su = 0;
-  uint32_t fh = NONE32, lh = 0;  // lh holds idx + 1 so that 0 means none
+  auto totals = [&](auto may_wrap) {
+    constexpr bool SAT = decltype(may_wrap)::value;
+    uint64_t sd = 0, su = 0;
+    uint32_t fh = NONE32, lh = 0;  // lh holds idx + 1 so that 0 means none
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const float xs[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
+    for (int k = 0; k < 4; ++k) {
+      const float xs[4] = {x[k].x, x[k].y, x[k].z, x[k].w};
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t idx = tg.T * TILE + 256u * k + 4u * lane + j;
-      const bool in = idx - tg.lead < tg.span - tg.lead;
-      const Entry e = classify_fast((double)masked_weight(xs[j], in), in, L);
-      if (!in) continue;
-      if (e.heavy) {
-        su += e.amount;
-        fh = min(fh, idx);
-        lh = max(lh, idx + 1);
-      } else {
-        sd += e.amount;
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t idx = tg.T * TILE + 256u * k + 4u * lane + j;
+        const bool in = idx - tg.lead < tg.span - tg.lead;
+        const Entry e = classify_fast((double)masked_weight(xs[j], in), in, L);
+        if (!in) continue;
+        if (e.heavy) {
+          su = add_sat<SAT>(su, e.amount);
+          fh = min(fh, idx);
+          lh = max(lh, idx + 1);
+        } else {
+          sd += e.amount;
+        }
       }
     }
-  }
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    sd += shfl_xor_u64(sd, m);
-    su += shfl_xor_u64(su, m);
-    fh = min(fh, (uint32_t)__shfl_xor((int)fh, m, 64));
-    lh = max(lh, (uint32_t)__shfl_xor((int)lh, m, 64));
-  }
-  if (lane == 0) a.ttot[tile] = TileTotals{sd, su, fh, lh ? lh - 1 : NONE32};
+    for (int m = 32; m >= 1; m >>= 1) {
+      sd += shfl_xor_u64(sd, m);
+      su = add_sat<SAT>(su, shfl_xor_u64(su, m));
+      fh = min(fh, (uint32_t)__shfl_xor((int)fh, m, 64));
+      lh = max(lh, (uint32_t)__shfl_xor((int)lh, m, 64));
+    }
+    if (lane == 0) a.ttot[tile] = TileTotals{sd, su, fh, lh ? lh - 1 : NONE32};
+  };
+  if (surpluses_may_wrap(L.scale)) totals(std::true_type{});
+  else totals(std::false_type{});
 }
 
 template <bool DEV, int G, int PER>

@@ -165,9 +165,8 @@ __device__ __forceinline__ double group_scan_f64(double v) {
   return v;
 }
 __device__ __forceinline__ double wave_scan_f64(double v) { return group_scan_f64<64>(v); }
-// The value of the lane before, 0 in lane 0.
 __device__ __forceinline__ double lane_before_f64(double v) {
-  return __longlong_as_double((long long)dpp0_u64<DPP_WAVE_SHR1, 0xF>((uint64_t)__double_as_longlong(v)));
+  return __longlong_as_double((long long)lane_before_u64((uint64_t)__double_as_longlong(v)));
 }
 __device__ __forceinline__ double lane_f64(double v, int lane) {
   const uint64_t b = (uint64_t)__double_as_longlong(v);

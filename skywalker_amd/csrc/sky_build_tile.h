@@ -79,7 +79,7 @@ struct TileScanLds {
   uint64_t s_wl[T / 64], s_wh[T / 64];
   uint32_t s_wm[T / 64];
 };
-template <int TS_T>
+template <int TS_T, bool SAT>
 __device__ __forceinline__ void tile_scan_row(TiledRow* __restrict__ rows, uint32_t r, const TileTotals* __restrict__ ttot,
                                               uint64_t* __restrict__ BL, uint64_t* __restrict__ BH,
                                               uint32_t* __restrict__ nfh, uint4* __restrict__ ranges,
@@ -104,7 +104,7 @@ __device__ __forceinline__ void tile_scan_row(TiledRow* __restrict__ rows, uint3
       u = x.u;
       lh = x.last_heavy == NONE32 ? 0 : x.last_heavy + 1;
     }
-    const uint64_t il = group_scan_u64<64>(d), ih = group_scan_u64<64>(u);
+    const uint64_t il = group_scan_u64<64>(d), ih = group_scan_sat_u64<64, SAT>(u);
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) lh = max(lh, (uint32_t)__shfl_xor((int)lh, m, 64));
     if (lane == 63) {
@@ -119,18 +119,19 @@ __device__ __forceinline__ void tile_scan_row(TiledRow* __restrict__ rows, uint3
     for (int w = 0; w < NW; ++w) {
       if (w == wave) {
         bl += tl;
-        bh += th;
+        bh = add_sat<SAT>(bh, th);
       }
       tl += s_wl[w];
-      th += s_wh[w];
+      th = add_sat<SAT>(th, s_wh[w]);
       lm = max(lm, s_wm[w]);
     }
+    const uint64_t eh = before_own<SAT>(ih, u);  // all lanes together
     if (t < nt) {
       BL[b0 + t] = bl + il - d;
-      BH[b0 + t] = bh + ih - u;
+      BH[b0 + t] = add_sat<SAT>(bh, eh);
     }
     cl += tl;
-    ch += th;
+    ch = add_sat<SAT>(ch, th);
     if (lm) last = lm - 1;
     __syncthreads();  // the wavefront totals are rewritten by the next round
   }
@@ -186,6 +187,15 @@ __device__ __forceinline__ void tile_scan_row(TiledRow* __restrict__ rows, uint3
   }
 }
 
+template <int TS_T>
+__device__ __forceinline__ void tile_scan_row(TiledRow* __restrict__ rows, uint32_t r, const TileTotals* __restrict__ ttot,
+                                              uint64_t* __restrict__ BL, uint64_t* __restrict__ BH,
+                                              uint32_t* __restrict__ nfh, uint4* __restrict__ ranges,
+                                              TileScanLds<TS_T>& lds) {
+  if (surpluses_may_wrap(rows[r].scale)) tile_scan_row<TS_T, true>(rows, r, ttot, BL, BH, nfh, ranges, lds);
+  else tile_scan_row<TS_T, false>(rows, r, ttot, BL, BH, nfh, ranges, lds);
+}
+
 // ---------------------------------------------------------------- pass 3: every entry of a tile
 // Resolves the own entries of one kind whose key lies in [lo, hi) against the per-slot prefix of tile
 // `pt` held in smem[0..TILE).  OWN_HEAVY = false: lights, key = exclusive deficit prefix, prefix = surplus.
@@ -231,7 +241,7 @@ __device__ __forceinline__ void resolve_in_tile(const TiledRow& r, const Ledger&
 
 // One pass over the partner tiles of one kind other than the own tile T: their per-slot prefix is
 // recomputed from the weights into LDS.
-template <bool OWN_HEAVY>
+template <bool OWN_HEAVY, bool SAT>
 __device__ __forceinline__ void partner_pass(const TiledRow& r, const Ledger& L, const float* __restrict__ wgt,
                                              const uint64_t* __restrict__ B, uint32_t t_lo, uint32_t t_hi,
                                              uint64_t* smem,
@@ -256,7 +266,7 @@ __device__ __forceinline__ void partner_pass(const TiledRow& r, const Ledger& L,
         pv[q][k] = e.heavy != OWN_HEAVY ? e.amount : 0;
       }
     __syncthreads();  // searches of the previous partner are done: s_ex and the prefix may be overwritten
-    block_scan1<TL_T, TL_Q>(pv, s_ex, lo, ps);
+    block_scan1<TL_T, TL_Q, SAT && !OWN_HEAVY>(pv, s_ex, lo, ps);
 #pragma unroll
     for (int q = 0; q < TL_Q; ++q)
 #pragma unroll
@@ -271,37 +281,17 @@ struct TileEmitLds {
   uint64_t s_ex[2 * TL_Q * (TL_T / 64)];
   uint32_t s_fh[TL_Q][TL_T / 64];
 };
-// Every entry of tile `tile` (tg.span not 0) by TL_T threads.
-__device__ __forceinline__ void tile_emit(const TileGeom& tg, uint32_t tile, const TiledRow* __restrict__ rows,
-                                          const float* __restrict__ wgt, const uint64_t* __restrict__ gBL,
-                                          const uint64_t* __restrict__ gBH, const uint32_t* __restrict__ nfh,
-                                          const uint4* __restrict__ ranges, AliasEntry* __restrict__ table,
-                                          int8_t* __restrict__ valid, TileEmitLds& lds) {
+// Every entry of tile T of row `r`, whose weights are w.  SAT: the row's surpluses may wrap (surpluses_may_wrap).
+template <bool SAT>
+__device__ __forceinline__ void tile_entries(const TiledRow& r, const Ledger& L, uint32_t tile, uint32_t T, const float (&w)[TL_Q][4],
+                                             const float* __restrict__ wgt, const uint64_t* __restrict__ gBL,
+                                             const uint64_t* __restrict__ gBH, const uint32_t* __restrict__ nfh,
+                                             const uint4* __restrict__ ranges, AliasEntry* __restrict__ table, TileEmitLds& lds) {
   constexpr int NW = TL_T / 64;
   auto& smem = lds.smem;
   auto& s_ex = lds.s_ex;
   auto& s_fh = lds.s_fh;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const uint32_t T = tg.T;
-
-  float w[TL_Q][4];
-  load_tile(wgt, geom_row(tg, tile), T, tid, w);  // requested before the row record arrives
-  const TiledRow r = rows[tg.row];
-  if (!r.ok) {
-#pragma unroll
-    for (int q = 0; q < TL_Q; ++q)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t idx = T * TILE + 4u * (q * TL_T + tid) + k;
-        if (in_row(r, idx)) {
-          table[r.base + idx] = AliasEntry{0.0f, SKY_INVALID};
-        }
-      }
-    if (T == 0 && tid == 0) valid[r.v] = 0;
-    return;
-  }
-  if (T == 0 && tid == 0) valid[r.v] = 1;
-  const Ledger L = row_ledger(r);
   const uint64_t* BL = gBL + r.bofs;  // tile prefixes of this row
   const uint64_t* BH = gBH + r.bofs;
   const uint64_t bl = BL[T], bl1 = BL[T + 1], bh = BH[T], bh1 = BH[T + 1];
@@ -340,13 +330,13 @@ __device__ __forceinline__ void tile_emit(const TileGeom& tg, uint32_t tile, con
       if (lane == 0) s_fh[q][wave] = fh;
     }
     uint64_t tl, th;
-    block_scan2<TL_T, TL_Q>(dl, dh, s_ex, sl, sh, tl, th);  // its barrier also publishes s_fh
+    block_scan2<TL_T, TL_Q, SAT>(dl, dh, s_ex, sl, sh, tl, th);  // its barrier also publishes s_fh
 #pragma unroll
     for (int q = 0; q < TL_Q; ++q)
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
         sl[q][k] += bl;
-        sh[q][k] += bh;
+        sh[q][k] = add_sat<SAT>(sh[q][k], bh);
         key[q][k] = ((heavy_mask >> (q * 4 + k)) & 1) ? sh[q][k] - 1 : sl[q][k] - dl[q][k];
       }
   }
@@ -396,8 +386,8 @@ __device__ __forceinline__ void tile_emit(const TileGeom& tg, uint32_t tile, con
   resolve_in_tile<true>(r, L, smem, T, bl, bl1, heavy_mask, live_mask, nh_after, T, key, op, oa);
 
   // the other partner tiles (ranges precomputed per tile by tiled_scan_kernel)
-  partner_pass<false>(r, L, wgt, BH, rg.x, rg.y, smem, s_ex, heavy_mask, live_mask, nh_after, T, key, op, oa);
-  partner_pass<true>(r, L, wgt, BL, rg.z, rg.w, smem, s_ex, heavy_mask, live_mask, nh_after, T, key, op, oa);
+  partner_pass<false, SAT>(r, L, wgt, BH, rg.x, rg.y, smem, s_ex, heavy_mask, live_mask, nh_after, T, key, op, oa);
+  partner_pass<true, SAT>(r, L, wgt, BL, rg.z, rg.w, smem, s_ex, heavy_mask, live_mask, nh_after, T, key, op, oa);
 
 #pragma unroll
   for (int q = 0; q < TL_Q; ++q) {
@@ -413,6 +403,36 @@ __device__ __forceinline__ void tile_emit(const TileGeom& tg, uint32_t tile, con
         }
     }
   }
+}
+// Every entry of tile `tile` (tg.span not 0) by TL_T threads.
+__device__ __forceinline__ void tile_emit(const TileGeom& tg, uint32_t tile, const TiledRow* __restrict__ rows,
+                                          const float* __restrict__ wgt, const uint64_t* __restrict__ gBL,
+                                          const uint64_t* __restrict__ gBH, const uint32_t* __restrict__ nfh,
+                                          const uint4* __restrict__ ranges, AliasEntry* __restrict__ table,
+                                          int8_t* __restrict__ valid, TileEmitLds& lds) {
+  const int tid = threadIdx.x;
+  const uint32_t T = tg.T;
+
+  float w[TL_Q][4];
+  load_tile(wgt, geom_row(tg, tile), T, tid, w);  // requested before the row record arrives
+  const TiledRow r = rows[tg.row];
+  if (!r.ok) {
+#pragma unroll
+    for (int q = 0; q < TL_Q; ++q)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t idx = T * TILE + 4u * (q * TL_T + tid) + k;
+        if (in_row(r, idx)) {
+          table[r.base + idx] = AliasEntry{0.0f, SKY_INVALID};
+        }
+      }
+    if (T == 0 && tid == 0) valid[r.v] = 0;
+    return;
+  }
+  if (T == 0 && tid == 0) valid[r.v] = 1;
+  const Ledger L = row_ledger(r);
+  if (surpluses_may_wrap(L.scale)) tile_entries<true>(r, L, tile, T, w, wgt, gBL, gBH, nfh, ranges, table, lds);
+  else tile_entries<false>(r, L, tile, T, w, wgt, gBL, gBH, nfh, ranges, table, lds);
 }
 
 }  // namespace sky

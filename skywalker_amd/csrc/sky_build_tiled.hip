@@ -153,28 +153,33 @@ __global__ __launch_bounds__(TL_T) void tiled_totals_kernel(const TileGeom* __re
   const Ledger L = row_ledger(r);
   uint64_t sd = 0, su = 0;
   uint32_t fh = NONE32, lh = 0;  // lh holds idx + 1 so that 0 means none
+  auto add_up = [&](auto may_wrap) {
+    constexpr bool SAT = decltype(may_wrap)::value;
 #pragma unroll
-  for (int q = 0; q < TL_Q; ++q)
+    for (int q = 0; q < TL_Q; ++q)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t idx = t * TILE + 4u * (q * TL_T + tid) + k;
-      if (!in_row(r, idx)) continue;
-      const Entry e = classify_fast((double)w[q][k], true, L);
-      if (e.heavy) {
-        su += e.amount;
-        fh = min(fh, idx);
-        lh = max(lh, idx + 1);
-      } else {
-        sd += e.amount;
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t idx = t * TILE + 4u * (q * TL_T + tid) + k;
+        if (!in_row(r, idx)) continue;
+        const Entry e = classify_fast((double)w[q][k], true, L);
+        if (e.heavy) {
+          su = add_sat<SAT>(su, e.amount);
+          fh = min(fh, idx);
+          lh = max(lh, idx + 1);
+        } else {
+          sd += e.amount;
+        }
       }
-    }
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) {
-    sd += shfl_xor_u64(sd, m);
-    su += shfl_xor_u64(su, m);
-    fh = min(fh, (uint32_t)__shfl_xor((int)fh, m, 64));
-    lh = max(lh, (uint32_t)__shfl_xor((int)lh, m, 64));
-  }
+    for (int m = 32; m >= 1; m >>= 1) {
+      sd += shfl_xor_u64(sd, m);
+      su = add_sat<SAT>(su, shfl_xor_u64(su, m));
+      fh = min(fh, (uint32_t)__shfl_xor((int)fh, m, 64));
+      lh = max(lh, (uint32_t)__shfl_xor((int)lh, m, 64));
+    }
+  };
+  if (surpluses_may_wrap(L.scale)) add_up(std::true_type{});
+  else add_up(std::false_type{});
   if ((tid & 63) == 0) {
     s_d[tid >> 6] = sd;
     s_u[tid >> 6] = su;
@@ -186,7 +191,7 @@ __global__ __launch_bounds__(TL_T) void tiled_totals_kernel(const TileGeom* __re
     TileTotals o{0, 0, NONE32, 0};
     for (int i = 0; i < TL_T / 64; ++i) {
       o.d += s_d[i];
-      o.u += s_u[i];
+      o.u = add_sat(o.u, s_u[i]);
       o.first_heavy = min(o.first_heavy, s_f[i]);
       o.last_heavy = max(o.last_heavy, s_l[i]);
     }

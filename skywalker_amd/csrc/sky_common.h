@@ -298,6 +298,9 @@ constexpr int DPP_ROW_BCAST15 = 0x142, DPP_ROW_BCAST31 = 0x143, DPP_WAVE_SHR1 = 
 constexpr int DPP_QUAD_XOR1 = 0xB1 /* quad_perm [1,0,3,2] */, DPP_QUAD_XOR2 = 0x4E /* quad_perm [2,3,0,1] */;
 constexpr int DPP_ROW_HALF_MIRROR = 0x141, DPP_ROW_MIRROR = 0x140;
 
+// The value of the lane before, 0 in lane 0.
+__device__ __forceinline__ uint64_t lane_before_u64(uint64_t v) { return dpp0_u64<DPP_WAVE_SHR1, 0xF>(v); }
+
 // Inclusive prefix sum over aligned groups of G lanes (G = 4, 8, 16, 32, 64).
 template <int G>
 __device__ __forceinline__ uint64_t group_scan_u64(uint64_t v) {
@@ -322,6 +325,39 @@ __device__ __forceinline__ uint64_t group_scan_u64(uint64_t v) {
     }
   }
   return v;
+}
+// Sums of surpluses, with saturation.  Weights below 2^-64 add nothing to the sum of their row of d and can have nearly d shares each:
+// in rows of 4,096 entries and more their surpluses may pass 2^64.  No deficit prefix reaches 2^63, so that a prefix that stays
+// at 2^64 - 1 decides what the true one does (its heavies are never reached); one that wraps would be taken for a small one.
+// A weight loses less than 2^-64 to the floor, so that all shares together are at most d (S + d) / S in units of that: twice the
+// row's d, which leaves every sum below 2^64, unless S < d.  That is a scale above 2^64, and such rows alone need saturation: it costs
+// four instructions for two (a walk with the table of every step 693 -> 718 us when every row's sums had it).
+// Where sums may be at their limit, what lies before a lane is the prefix of the lane before, not its own less its amount.
+// SAT false: ordinary sums.
+template <bool SAT = true>
+__device__ __forceinline__ uint64_t add_sat(uint64_t a, uint64_t b) {
+  if constexpr (SAT) return __builtin_elementwise_add_sat(a, b);
+  return a + b;
+}
+__device__ __forceinline__ bool surpluses_may_wrap(double scale) {
+  return __builtin_expect(__builtin_amdgcn_readfirstlane(scale > 18446744073709551616.0) != 0, 0);  // uniform: a row's scale
+}
+template <int G, bool SAT = true>
+__device__ __forceinline__ uint64_t group_scan_sat_u64(uint64_t v) {
+  if constexpr (!SAT) return group_scan_u64<G>(v);
+  static_assert(G == 16 || G == 64, "whole rows of 16 lanes, or all of them");
+  v = add_sat(v, dpp0_u64<DPP_ROW_SHR1, 0xF>(v));
+  v = add_sat(v, dpp0_u64<DPP_ROW_SHR2, 0xF>(v));
+  v = add_sat(v, dpp0_u64<DPP_ROW_SHR4, 0xF>(v));
+  v = add_sat(v, dpp0_u64<DPP_ROW_SHR8, 0xF>(v));
+  if (G >= 64) v = add_sat(v, dpp0_u64<DPP_ROW_BCAST15, 0xA>(v));
+  if (G >= 64) v = add_sat(v, dpp0_u64<DPP_ROW_BCAST31, 0xC>(v));
+  return v;
+}
+// What lies before a lane: of its inclusive prefix over the wavefront and its own amount.
+template <bool SAT = true>
+__device__ __forceinline__ uint64_t before_own(uint64_t inclusive, uint64_t own) {
+  return SAT ? lane_before_u64(inclusive) : inclusive - own;
 }
 template <int G>
 __device__ __forceinline__ uint32_t group_scan_u32(uint32_t v) {

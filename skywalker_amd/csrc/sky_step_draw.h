@@ -46,6 +46,186 @@ __device__ __forceinline__ bool row_contains(const uint32_t* __restrict__ row, u
   return false;
 }
 
+// Rest of the draw below: column `col` of class `ec` with the acceptance number u.  SAT: the row's surpluses may wrap.
+template <bool SAT, int T, class Row>
+__device__ __forceinline__ uint32_t draw_entry(Row& row, const uint32_t d, const Ledger& L, const uint32_t col, const Entry& ec,
+                                               const float u, const uint32_t csz, const uint32_t nc, const uint32_t c0,
+                                               const uint32_t c1, DrawLds<T>& lds) {
+  constexpr int NW = T / 64;
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // the four slots of this lane in the 256 from `base` on: amounts of the two kinds
+  auto amounts = [&](uint32_t base, uint64_t (&dd)[4], uint64_t (&uu)[4]) {
+    float w[4];
+    row.again(base + 4 * lane, w);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool in = base + 4 * lane + k < d;
+      const Entry e = classify_fast((double)w[k], in, L);
+      dd[k] = in && !e.heavy ? e.amount : 0;
+      uu[k] = e.heavy ? e.amount : 0;
+    }
+  };
+
+  // pass 2: totals of the chunks
+  for (uint32_t c = c0; c < c1; ++c) {
+    uint64_t sd = 0, su = 0;
+    const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
+    for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
+      uint64_t dd[4], uu[4];
+      amounts(base, dd, uu);
+      sd += (dd[0] + dd[1]) + (dd[2] + dd[3]);
+      su = add_sat<SAT>(su, add_sat<SAT>(add_sat<SAT>(uu[0], uu[1]), add_sat<SAT>(uu[2], uu[3])));
+    }
+    sd = group_scan_u64<64>(sd);
+    su = group_scan_sat_u64<64, SAT>(su);
+    if (lane == 63) {
+      lds.d[c] = sd;
+      lds.u[c] = su;
+    }
+  }
+  __syncthreads();
+
+  if (wave == 0) {
+    {  // prefixes over the chunks: 4 consecutive ones per lane
+      constexpr int PER = DRAW_CHUNKS / 64;
+      uint64_t pd[PER], pu[PER], rd = 0, ru = 0;
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const uint32_t c = lane * PER + j;
+        rd += c < nc ? lds.d[c] : 0;
+        ru = add_sat<SAT>(ru, c < nc ? lds.u[c] : 0);
+        pd[j] = rd;
+        pu[j] = ru;
+      }
+      const uint64_t bd = group_scan_u64<64>(rd) - rd, bu = before_own<SAT>(group_scan_sat_u64<64, SAT>(ru), ru);
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        lds.d[lane * PER + j] = bd + pd[j];
+        lds.u[lane * PER + j] = add_sat<SAT>(bu, pu[j]);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    // first chunk of the row whose inclusive prefix in p exceeds key, nc if none
+    auto chunk_above = [&](const uint64_t* p, uint64_t key) -> uint32_t {
+#pragma unroll
+      for (int j = 0; j < DRAW_CHUNKS / 64; ++j) {
+        const uint32_t c = 64 * j + lane;
+        const unsigned long long m = __ballot(c < nc && p[c] > key);
+        if (m) return 64 * j + (uint32_t)__ffsll((long long)m) - 1;
+      }
+      return nc;
+    };
+    // first slot of chunk c whose inclusive prefix (of surpluses or deficits) exceeds key, and that prefix
+    auto slot_above = [&](uint32_t c, bool surplus, uint64_t key, uint64_t& at) -> uint32_t {
+      const uint64_t* p = surplus ? lds.u : lds.d;
+      const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
+      uint64_t before = c ? p[c - 1] : 0;
+      for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
+        uint64_t dd[4], uu[4], run[4];
+        amounts(base, dd, uu);
+        uint64_t t = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          t = add_sat<SAT>(t, surplus ? uu[k] : dd[k]);
+          run[k] = t;
+        }
+        const uint64_t inc = group_scan_sat_u64<64, SAT>(t), mine = add_sat<SAT>(before, before_own<SAT>(inc, t));
+        const unsigned long long m = __ballot(add_sat<SAT>(before, inc) > key);
+        if (m) {
+          const int l = __ffsll((long long)m) - 1;
+          uint32_t k = 3;
+          uint64_t x = add_sat<SAT>(mine, run[3]);
+#pragma unroll
+          for (int j = 2; j >= 0; --j)
+            if (add_sat<SAT>(mine, run[j]) > key) {
+              k = j;
+              x = add_sat<SAT>(mine, run[j]);
+            }
+          at = shfl_u64(x, l);
+          return (uint32_t)__shfl((int)(base + 4 * lane + k), l, 64);
+        }
+        before = add_sat<SAT>(before, shfl_u64(inc, 63));
+      }
+      // not reached while the weights stay what they were in pass 2; a bias operator that answers differently each
+      // time must not keep the wavefront here
+      at = key + 1;
+      return end - 1;
+    };
+    // first (last) heavy slot of [from, end), both inside chunk c; NONE_SLOT if there is none
+    auto heavy_in = [&](uint32_t c, uint32_t from, bool last) -> uint32_t {
+      const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
+      uint32_t got = NONE_SLOT;
+      for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
+        if (base + DRAW_CHUNK <= from) continue;
+        uint64_t dd[4], uu[4];
+        amounts(base, dd, uu);
+        uint32_t mine = NONE_SLOT;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t slot = base + 4 * lane + k;
+          if (uu[k] && slot >= from && (last || mine == NONE_SLOT)) mine = slot;
+        }
+        const unsigned long long m = __ballot(mine != NONE_SLOT);
+        if (m) {
+          const int l = last ? 63 - __clzll((long long)m) : __ffsll((long long)m) - 1;
+          got = (uint32_t)__shfl((int)mine, l, 64);
+          if (!last) break;
+        }
+      }
+      return got;
+    };
+
+    // key: deficits before a light col, surpluses up to and with a heavy col
+    const uint32_t cc = col / csz;
+    uint64_t key = ec.heavy ? (cc ? lds.u[cc - 1] : 0) : (cc ? lds.d[cc - 1] : 0), part = 0;
+    for (uint32_t base = cc * csz; base <= col; base += DRAW_CHUNK) {
+      uint64_t dd[4], uu[4];
+      amounts(base, dd, uu);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t slot = base + 4 * lane + k;
+        part = add_sat<SAT>(part, ec.heavy ? (slot <= col ? uu[k] : 0) : (slot < col ? dd[k] : 0));
+      }
+    }
+    key = add_sat<SAT>(key, shfl_u64(group_scan_sat_u64<64, SAT>(part), 63));
+
+    uint32_t cand = col;
+    const uint64_t total_u = lds.u[nc - 1];
+    if (!ec.heavy) {
+      // first heavy whose surplus prefix exceeds the key; the last heavy if there is none; col itself without any heavy
+      const uint32_t cm = chunk_above(lds.u, key);
+      if (cm < nc) {
+        uint64_t at;
+        cand = slot_above(cm, true, key, at);
+      } else if (total_u) {
+        cand = heavy_in(chunk_above(lds.u, total_u - 1), 0, true);
+      }
+    } else {
+      // next heavy after col (none: col is the last heavy and keeps the draw), then the first light l with
+      // SL(l) >= y: prob = (one + y - SL(l)) / one
+      uint32_t nxt = col + 1 < d ? heavy_in(cc, col + 1, false) : NONE_SLOT;
+      if (nxt == NONE_SLOT) {
+        const uint32_t cn = chunk_above(lds.u, lds.u[cc]);
+        if (cn < nc) nxt = heavy_in(cn, 0, false);
+      }
+      const uint32_t cl = nxt != NONE_SLOT ? chunk_above(lds.d, key - 1) : nc;
+      if (cl < nc) {
+        uint64_t sl = 0;
+        (void)slot_above(cl, false, key - 1, sl);
+        cand = u < residual_prob(L.one + key - sl, L) ? col : nxt;
+      }
+    }
+    if (NW == 1) return cand;
+    if (lane == 0) lds.result = cand;
+  }
+  __syncthreads();
+  const uint32_t cand = lds.result;
+  __syncthreads();  // the next draw rewrites what the others still read
+  return cand;
+}
+
 // Row-local slot that (walker, step) with random numbers r draws from the row of d >= 1 entries, or NONE_SLOT when
 // their weights sum to zero.  Called by every thread of a workgroup of T.  `row`:
 //   row.first(k, w)   clamped weights of slots k .. k + 3 (k a multiple of 4; zeros past the row).  A wavefront goes
@@ -139,177 +319,8 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
   }
   if (!ec.heavy && u < (float)ec.p) return col;  // the light keeps the draw: its alias is never read
 
-  // the four slots of this lane in the 256 from `base` on: amounts of the two kinds
-  auto amounts = [&](uint32_t base, uint64_t (&dd)[4], uint64_t (&uu)[4]) {
-    float w[4];
-    row.again(base + 4 * lane, w);
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const bool in = base + 4 * lane + k < d;
-      const Entry e = classify_fast((double)w[k], in, L);
-      dd[k] = in && !e.heavy ? e.amount : 0;
-      uu[k] = e.heavy ? e.amount : 0;
-    }
-  };
-
-  // pass 2: totals of the chunks
-  for (uint32_t c = c0; c < c1; ++c) {
-    uint64_t sd = 0, su = 0;
-    const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
-    for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
-      uint64_t dd[4], uu[4];
-      amounts(base, dd, uu);
-      sd += (dd[0] + dd[1]) + (dd[2] + dd[3]);
-      su += (uu[0] + uu[1]) + (uu[2] + uu[3]);
-    }
-    sd = group_scan_u64<64>(sd);
-    su = group_scan_u64<64>(su);
-    if (lane == 63) {
-      lds.d[c] = sd;
-      lds.u[c] = su;
-    }
-  }
-  __syncthreads();
-
-  if (wave == 0) {
-    {  // prefixes over the chunks: 4 consecutive ones per lane
-      constexpr int PER = DRAW_CHUNKS / 64;
-      uint64_t pd[PER], pu[PER], rd = 0, ru = 0;
-#pragma unroll
-      for (int j = 0; j < PER; ++j) {
-        const uint32_t c = lane * PER + j;
-        rd += c < nc ? lds.d[c] : 0;
-        ru += c < nc ? lds.u[c] : 0;
-        pd[j] = rd;
-        pu[j] = ru;
-      }
-      const uint64_t bd = group_scan_u64<64>(rd) - rd, bu = group_scan_u64<64>(ru) - ru;
-#pragma unroll
-      for (int j = 0; j < PER; ++j) {
-        lds.d[lane * PER + j] = bd + pd[j];
-        lds.u[lane * PER + j] = bu + pu[j];
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    // first chunk of the row whose inclusive prefix in p exceeds key, nc if none
-    auto chunk_above = [&](const uint64_t* p, uint64_t key) -> uint32_t {
-#pragma unroll
-      for (int j = 0; j < DRAW_CHUNKS / 64; ++j) {
-        const uint32_t c = 64 * j + lane;
-        const unsigned long long m = __ballot(c < nc && p[c] > key);
-        if (m) return 64 * j + (uint32_t)__ffsll((long long)m) - 1;
-      }
-      return nc;
-    };
-    // first slot of chunk c whose inclusive prefix (of surpluses or deficits) exceeds key, and that prefix
-    auto slot_above = [&](uint32_t c, bool surplus, uint64_t key, uint64_t& at) -> uint32_t {
-      const uint64_t* p = surplus ? lds.u : lds.d;
-      const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
-      uint64_t before = c ? p[c - 1] : 0;
-      for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
-        uint64_t dd[4], uu[4], run[4];
-        amounts(base, dd, uu);
-        uint64_t t = 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          t += surplus ? uu[k] : dd[k];
-          run[k] = t;
-        }
-        const uint64_t inc = group_scan_u64<64>(t), mine = before + inc - t;
-        const unsigned long long m = __ballot(before + inc > key);
-        if (m) {
-          const int l = __ffsll((long long)m) - 1;
-          uint32_t k = 3;
-          uint64_t x = mine + run[3];
-#pragma unroll
-          for (int j = 2; j >= 0; --j)
-            if (mine + run[j] > key) {
-              k = j;
-              x = mine + run[j];
-            }
-          at = shfl_u64(x, l);
-          return (uint32_t)__shfl((int)(base + 4 * lane + k), l, 64);
-        }
-        before += shfl_u64(inc, 63);
-      }
-      // not reached while the weights stay what they were in pass 2; a bias operator that answers differently each
-      // time must not keep the wavefront here
-      at = key + 1;
-      return end - 1;
-    };
-    // first (last) heavy slot of [from, end), both inside chunk c; NONE_SLOT if there is none
-    auto heavy_in = [&](uint32_t c, uint32_t from, bool last) -> uint32_t {
-      const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
-      uint32_t got = NONE_SLOT;
-      for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
-        if (base + DRAW_CHUNK <= from) continue;
-        uint64_t dd[4], uu[4];
-        amounts(base, dd, uu);
-        uint32_t mine = NONE_SLOT;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          const uint32_t slot = base + 4 * lane + k;
-          if (uu[k] && slot >= from && (last || mine == NONE_SLOT)) mine = slot;
-        }
-        const unsigned long long m = __ballot(mine != NONE_SLOT);
-        if (m) {
-          const int l = last ? 63 - __clzll((long long)m) : __ffsll((long long)m) - 1;
-          got = (uint32_t)__shfl((int)mine, l, 64);
-          if (!last) break;
-        }
-      }
-      return got;
-    };
-
-    // key: deficits before a light col, surpluses up to and with a heavy col
-    const uint32_t cc = col / csz;
-    uint64_t key = ec.heavy ? (cc ? lds.u[cc - 1] : 0) : (cc ? lds.d[cc - 1] : 0), part = 0;
-    for (uint32_t base = cc * csz; base <= col; base += DRAW_CHUNK) {
-      uint64_t dd[4], uu[4];
-      amounts(base, dd, uu);
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t slot = base + 4 * lane + k;
-        part += ec.heavy ? (slot <= col ? uu[k] : 0) : (slot < col ? dd[k] : 0);
-      }
-    }
-    key += shfl_u64(group_scan_u64<64>(part), 63);
-
-    uint32_t cand = col;
-    const uint64_t total_u = lds.u[nc - 1];
-    if (!ec.heavy) {
-      // first heavy whose surplus prefix exceeds the key; the last heavy if there is none; col itself without any heavy
-      const uint32_t cm = chunk_above(lds.u, key);
-      if (cm < nc) {
-        uint64_t at;
-        cand = slot_above(cm, true, key, at);
-      } else if (total_u) {
-        cand = heavy_in(chunk_above(lds.u, total_u - 1), 0, true);
-      }
-    } else {
-      // next heavy after col (none: col is the last heavy and keeps the draw), then the first light l with
-      // SL(l) >= y: prob = (one + y - SL(l)) / one
-      uint32_t nxt = col + 1 < d ? heavy_in(cc, col + 1, false) : NONE_SLOT;
-      if (nxt == NONE_SLOT) {
-        const uint32_t cn = chunk_above(lds.u, lds.u[cc]);
-        if (cn < nc) nxt = heavy_in(cn, 0, false);
-      }
-      const uint32_t cl = nxt != NONE_SLOT ? chunk_above(lds.d, key - 1) : nc;
-      if (cl < nc) {
-        uint64_t sl = 0;
-        (void)slot_above(cl, false, key - 1, sl);
-        cand = u < residual_prob(L.one + key - sl, L) ? col : nxt;
-      }
-    }
-    if (NW == 1) return cand;
-    if (lane == 0) lds.result = cand;
-  }
-  __syncthreads();
-  const uint32_t cand = lds.result;
-  __syncthreads();  // the next draw rewrites what the others still read
-  return cand;
+  return surpluses_may_wrap(L.scale) ? draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, c0, c1, lds)
+                                     : draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, c0, c1, lds);
 }
 
 // A row whose weights are computed by a function of the slot (row(k): clamped weight of slot k < d): those of a row of up

@@ -615,6 +615,46 @@ def test_rows_whose_sums_need_every_bit(orc, make, route):
     g.free()
 
 
+def long_vanishing_rows(longest):
+    """Rows whose surpluses add up to 2^64 units and more."""
+    rows = [below_the_grid(d, k0, e) for d in (8192, 16384, 65536) if d <= longest for k0 in (1, 3) for e in (-1, 0)]
+    rng, u = np.random.default_rng(63), 2.0 ** -64
+    for d in (5100, 5117, 5118, 6000, 8188, 8189, 8190, 9000, 12288, 12289, 30000, 70001, 600001):
+        if d > longest:
+            break
+        share = np.concatenate([1 + rng.uniform(0, 2.0 ** -19, d // 10), rng.uniform(0.9, 0.99, d - 2 * (d // 10)) * d,
+                                rng.uniform(0, 0.1, d // 10)])
+        share[d // 3] = d
+        rows.append((share * (u / d)).astype(np.float32))
+    return rows
+
+
+@pytest.mark.parametrize("longest", [12288, 600001])
+@pytest.mark.parametrize("knobs", [{}, {"stream_min_edges": 0, "stream_wide_min_edges": 0}, {"small_in_place": 0},
+                                   {"small_in_place": 0, "stream_min_edges": 0, "stream_wide_min_edges": 0}, {"row_merge": 0},
+                                   {"tiled_max_tiles": 9}])
+def test_surpluses_beyond_64_bits(orc, knobs, longest):
+    # by default in one launch or four, streamed or tile by tile, by class (rows of 5,118..8,189 entries held), by the kernels that the
+    # tests alone select; and the draws of a walk that builds no table against those from the tables
+    from skywalker_amd import capi
+    rows = long_vanishing_rows(longest)
+    w = np.concatenate(rows)
+    V = max(len(r) for r in rows)  # every slot of a row leads to a vertex of its own
+    xadj = np.full(V + 1, len(w), np.uint32)
+    xadj[:len(rows) + 1] = np.concatenate([[0], np.cumsum([len(r) for r in rows])])
+    g = capi.Graph.upload(xadj, np.concatenate([np.arange(len(r), dtype=np.uint32) for r in rows]), w)
+    for k, value in knobs.items():
+        g.set_option(k, value)
+    seeds = np.repeat(np.arange(len(rows), dtype=np.uint32), 40)
+    g.set_option("online_full_build", 0)
+    online = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 1, 0.0, 5)
+    g.build_tables()
+    compare_tables(orc, g, xadj, w, "surpluses beyond 64 bits, %s" % knobs)
+    offline = g.walk_offline(seeds, 1, 0.0, 5)
+    assert np.array_equal(online[0].to_host(), offline[0].to_host())
+    g.free()
+
+
 @pytest.mark.parametrize("degree", [2048 * 1024 - 3, 2048 * 1024 + 1])
 def test_ledger_of_rows_of_very_many_tiles_in_four_launches(orc, degree):
     # up to 2048 tiles every tile adds up its row's sums itself, above a launch in between does
