@@ -133,16 +133,14 @@ __device__ __forceinline__ uint32_t unpack_chunk(const RawChunk& raw, const Stre
   return live;
 }
 
-// Exclusive prefix over the workgroup (thread order) of one u64 and one u32 per thread, plus totals.  SAT: the u64 is surpluses
-// (add_sat).
+// Exclusive prefix over the workgroup (thread order) of one u64 and one u32 per thread, plus totals.
 // One barrier: consecutive calls must alternate between two sets of s_a / s_c (a wavefront may start
 // the next call while others still read this one's sums; it cannot start the one after that before
 // every wavefront has passed the next call's barrier).
-template <bool SAT>
 __device__ __forceinline__ void stream_excl(uint64_t a, uint32_t c, uint64_t* s_a, uint32_t* s_c, uint64_t& ex_a,
                                             uint32_t& ex_c, uint64_t& tot_a, uint32_t& tot_c) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint64_t ia = group_scan_sat_u64<64, SAT>(a);
+  const uint64_t ia = group_scan_u64<64>(a);
   const uint32_t ic = group_scan_u32<64>(c);
   if (lane == 63) {
     s_a[wave] = ia;
@@ -151,15 +149,15 @@ __device__ __forceinline__ void stream_excl(uint64_t a, uint32_t c, uint64_t* s_
   __syncthreads();
   uint64_t ra = 0;
   uint32_t rc = 0;
-  ex_a = before_own<SAT>(ia, a);
+  ex_a = ia - a;
   ex_c = ic - c;
 #pragma unroll
   for (int w = 0; w < ST_NW; ++w) {
     if (w == wave) {
-      ex_a = add_sat<SAT>(ex_a, ra);
+      ex_a += ra;
       ex_c += rc;
     }
-    ra = add_sat<SAT>(ra, s_a[w]);
+    ra += s_a[w];
     rc += s_c[w];
   }
   tot_a = ra;
@@ -423,22 +421,42 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
         if (h < nw) {
           const uint64_t a = classify_fast((double)s_w32[2 * h], true, L).amount;
           s_sh[h] = a;
-          su = add_sat(su, a);
+          su += a;
         }
       }
       uint64_t ex_u, tot_u;
       uint32_t ex_c, tot_c;
-      stream_excl<true>(su, 0u, s_a[0], s_c[0], ex_u, ex_c, tot_u, tot_c);
-      uint64_t acc = add_sat(sh_lo, ex_u);
+      stream_excl(su, 0u, s_a[0], s_c[0], ex_u, ex_c, tot_u, tot_c);
+      uint64_t acc = sh_lo + ex_u;
 #pragma unroll 2
       for (int k = 0; k < HP; ++k) {
         const uint32_t h = (uint32_t)HP * tid + k;
         if (h < nw) {
-          acc = add_sat(acc, s_sh[h]);
+          acc += s_sh[h];
           s_sh[h] = acc;
         }
       }
-      sh_hi = add_sat(sh_lo, uniform_u64(tot_u));
+      sh_hi = sh_lo + uniform_u64(tot_u);
+    }
+    double scale = L.scale;
+    asm volatile("" : "+v"(scale));  // asked anew for every window: no scalar register holds the answer meanwhile
+    if (surpluses_may_wrap(scale)) {
+      // The prefixes may have wrapped, but what two neighbours differ by has not: one thread adds it up with saturation (in rows of next
+      // to no weight at all, so it may take its time; saturating sums above cost a build of 753 K entries with rows of up to
+      // 12,000 1.3 of 40 us).
+      __syncthreads();
+      if (tid == 0) {
+        uint64_t wrapped = sh_lo, acc = sh_lo;
+#pragma unroll 1
+        for (uint32_t h = 0; h < nw; ++h) {
+          const uint64_t x = s_sh[h];
+          acc = add_sat(acc, x - wrapped);
+          wrapped = x;
+          s_sh[h] = acc;
+        }
+      }
+      __syncthreads();
+      if (nw) sh_hi = uniform_u64(s_sh[nw - 1]);
     }
     const bool any_heavy = hb + nw != 0;
     const bool whole_row = hb == 0 && !more;  // the usual case: one window holds every heavy of the row
@@ -504,7 +522,7 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
       }
       uint64_t ex_d, tot_d;
       uint32_t ex_c, tot_c;
-      stream_excl<false>(run, nheavy, s_a[c & 1], s_c[c & 1], ex_d, ex_c, tot_d, tot_c);
+      stream_excl(run, nheavy, s_a[c & 1], s_c[c & 1], ex_d, ex_c, tot_d, tot_c);
       const uint32_t pos0 = c * ST_CH + (uint32_t)ST_PER * tid;
       uint32_t oa[ST_PER];
       uint32_t wr = 0;  // entries this window writes: its lights, and heavies as placeholders unless an earlier window owns them
@@ -724,7 +742,12 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
   uint32_t ex_c, nh;
   {
     const uint32_t c = (uint32_t)__popc(heavy);
-    const uint64_t id = group_scan_u64<64>(run_d), iu = group_scan_sat_u64<64>(run_u);  // run_u is below 2^59
+    // Surpluses may add up to more than 64 bits hold (surpluses_may_wrap): no more of a thread's or a wavefront's are counted than lie
+    // above every deficit prefix of so short a row (2^53).
+    static_assert(HOLD_MAX_DEG < (1u << 13));
+    auto counted = [](uint64_t x) { return x < (1ull << 54) ? x : (uint64_t)(1ull << 54); };
+    run_u = counted(run_u);
+    const uint64_t id = group_scan_u64<64>(run_d), iu = group_scan_u64<64>(run_u);
     const uint32_t ic = group_scan_u32<64>(c);
     if (lane == 63) {
       s_ex[3 * wave] = id;
@@ -741,7 +764,7 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
       wc = (uint32_t)s_ex[3 * lane + 2];
     }
     wd = group_scan_u64<16>(wd);
-    wu = group_scan_sat_u64<16>(wu);
+    wu = group_scan_u64<16>(counted(wu));
     wc = group_scan_u32<16>(wc);
     const int prev = max(wave - 1, 0);
     uint64_t bd = shfl_u64(wd, prev), bu = shfl_u64(wu, prev);
@@ -753,7 +776,7 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
     tot_d = shfl_u64(wd, NW - 1);
     nh = (uint32_t)__shfl((int)wc, NW - 1, 64);
     ex_d = bd + id - run_d;
-    ex_u = add_sat(bu, lane_before_u64(iu));
+    ex_u = bu + iu - run_u;
     ex_c = bc + ic - c;
   }
   nh = uniform_u32(nh);
@@ -776,7 +799,7 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
 #pragma unroll
       for (int j = 0; j < PER; ++j)
         if ((heavy >> j) & 1) {
-          su = add_sat(su, amt[j]);
+          su += amt[j];
           if (r <= nw) {  // ranks before the list wrap around
             if (r < nw) s_sh[r] = su;
             s_slot[r] = (uint16_t)(pos0 + j);
@@ -830,7 +853,7 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
 #pragma unroll
       for (int j = 0; j < PER; ++j)
         if ((heavy >> j) & 1) {
-          su = add_sat(su, amt[j]);
+          su += amt[j];
           if (r < nw) {
             const bool fin = (r + 1 < nw || more) && su <= tot_d;
             op[j] = fin ? s_prob[r] : 1.0f;

@@ -345,13 +345,13 @@ __device__ __forceinline__ bool surpluses_may_wrap(double scale) {
 template <int G, bool SAT = true>
 __device__ __forceinline__ uint64_t group_scan_sat_u64(uint64_t v) {
   if constexpr (!SAT) return group_scan_u64<G>(v);
-  static_assert(G == 16 || G == 64, "whole rows of 16 lanes, or all of them");
+  static_assert(G == 64, "all lanes of the wavefront");
   v = add_sat(v, dpp0_u64<DPP_ROW_SHR1, 0xF>(v));
   v = add_sat(v, dpp0_u64<DPP_ROW_SHR2, 0xF>(v));
   v = add_sat(v, dpp0_u64<DPP_ROW_SHR4, 0xF>(v));
   v = add_sat(v, dpp0_u64<DPP_ROW_SHR8, 0xF>(v));
-  if (G >= 64) v = add_sat(v, dpp0_u64<DPP_ROW_BCAST15, 0xA>(v));
-  if (G >= 64) v = add_sat(v, dpp0_u64<DPP_ROW_BCAST31, 0xC>(v));
+  v = add_sat(v, dpp0_u64<DPP_ROW_BCAST15, 0xA>(v));
+  v = add_sat(v, dpp0_u64<DPP_ROW_BCAST31, 0xC>(v));
   return v;
 }
 // What lies before a lane: of its inclusive prefix over the wavefront and its own amount.
