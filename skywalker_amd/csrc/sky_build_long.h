@@ -441,9 +441,9 @@ __device__ __forceinline__ bool stream_row(const RowRef rr, StreamLds& lds, cons
     double scale = L.scale;
     asm volatile("" : "+v"(scale));  // asked anew for every window: no scalar register holds the answer meanwhile
     if (surpluses_may_wrap(scale)) {
-      // The prefixes may have wrapped, but what two neighbours differ by has not: one thread adds it up with saturation (in rows of next
-      // to no weight at all, so it may take its time; saturating sums above cost a build of 753 K entries with rows of up to
-      // 12,000 1.3 of 40 us).
+      // The prefixes may have wrapped, but what two neighbours differ by has not: one thread adds it up with saturation
+      // (in rows of next to no weight at all, so it may take its time; a build of 753 K entries with rows of up to 12,000
+      // took 39.7 us without, 40.0 with this and 41.0 with saturating sums above).
       __syncthreads();
       if (tid == 0) {
         uint64_t wrapped = sh_lo, acc = sh_lo;
@@ -742,8 +742,8 @@ __device__ __forceinline__ bool hold_row(const RowRef rr, uint64_t* smem, uint64
   uint32_t ex_c, nh;
   {
     const uint32_t c = (uint32_t)__popc(heavy);
-    // Surpluses may add up to more than 64 bits hold (surpluses_may_wrap): no more of a thread's or a wavefront's are counted than lie
-    // above every deficit prefix of so short a row (2^53).
+    // Surpluses may add up to more than 64 bits hold (surpluses_may_wrap): no more of a thread's or a wavefront's are
+    // counted than lie above every deficit prefix of so short a row (2^53).
     static_assert(HOLD_MAX_DEG < (1u << 13));
     auto counted = [](uint64_t x) { return x < (1ull << 54) ? x : (uint64_t)(1ull << 54); };
     run_u = counted(run_u);

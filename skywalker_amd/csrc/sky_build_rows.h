@@ -212,10 +212,14 @@ constexpr uint32_t group_entries(int G, int PER, int BLOCK) {
 }
 constexpr size_t group_lds_bytes(int G, int PER, int BLOCK) { return (size_t)group_entries(G, PER, BLOCK) * 9; }
 
-// Lanes and slots of a lane by class.  8 slots a lane where 4 would do for twice the lanes: what a lane does once for its row (sum, division,
-// scans, search) is half of its instructions with 4.  200 M entries in rows of 100 (32 lanes of 4 / 16 of 8) 739 / 630 us, of 50
-// 720 / 640.  Not for the rows of up to 32: 200 M entries in rows of 24 835 / 680, but where they lie among others half as many
-// lanes means batches that are half as full (scale 20 with 16 edges a vertex 140 / 150, scale 22 with 10 316 / 333).
+// Lanes and slots of a lane by class.  8 slots a lane where 4 would do for twice the lanes: what a lane does once for its row
+// (sum, division, scans, search) is half of its instructions with 4.  Rows that lie side by side, 200 M entries in rows of
+// 100 (32 lanes of 4 / 16 of 8) 739 / 630 us, of 50 (16 of 4 / 8 of 8) 720 / 640.  Rows of 33..64 that lie scattered in a graph
+// built by class wait for their lines, of which half as many lanes ask for fewer at a time: they lose some 5 and 2 % (the scale-26
+// graph 0.615 / 0.650 ms, rows of every length in random order 0.261 / 0.267, five processes a side that differ by as much), 0.4 % of
+// such a build; rows of 65..128 gain there too (scale 25 with 56 edges a vertex 0.255 / 0.22 ms).
+// Not for the rows of up to 32: 200 M entries in rows of 24 835 / 680, but where they lie among others half as many lanes
+// means batches that are half as full (scale 20 with 16 edges a vertex 140 / 150, scale 22 with 10 316 / 333).
 struct GroupShape {
   int lanes, per;
 };
@@ -443,9 +447,10 @@ __device__ __forceinline__ bool tiny_row(uint32_t off, uint32_t d, const float* 
 // Neighbouring rows of different classes share their cache lines, and here the same wavefront touches them within a
 // few steps; no row list is written or read for these classes.  Also sets valid[] of the vertices it owns (rows of
 // 0..32 entries).  Nothing in here waits for another wavefront.
-// Queue capacities: less than one batch left over plus the 64 vertices of a step, rounded up.  A queue entry is the row's offset and, in 16 bits, its degree (6 bits) above the vertex's position in
-// the wavefront's range (10 bits): the vertex id itself is only needed for a row without weight, whose flag is
-// cleared.  5 KB of LDS per wavefront: the kernel's registers decide how many fit a SIMD.
+// Queue capacities: less than one batch left over plus the 64 vertices of a step, rounded up.  A queue entry is the row's
+// offset and, in 16 bits, its degree (6 bits) above the vertex's position in the wavefront's range (10 bits): the vertex
+// id itself is only needed for a row without weight, whose flag is cleared.  5 KB of LDS per wavefront: the kernel's
+// registers decide how many fit a SIMD.
 constexpr uint32_t SMALL_RANGE = 1024;  // most vertices per wavefront
 constexpr uint32_t SMALL_BATCH[4] = {64, 64 / SHAPE_G2.lanes, 64 / SHAPE_G4.lanes, 64 / SHAPE_G8.lanes};
 constexpr uint32_t small_cap(int q) { return (SMALL_BATCH[q] + 63 + 7) / 8 * 8; }
@@ -591,8 +596,9 @@ __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __
 constexpr bool merge_words(int rowt, int per) { return rowt * per == 256 || rowt * per == 1536; }
 constexpr size_t merge_lds_bytes(int rowt, int per) { return (((size_t)rowt * per + 4) * (merge_words(rowt, per) ? 14 : 10) + 15) / 16 * 16; }
 
-// The row `rr` by ROWT threads that share `smem` and, for the wavefronts' sums, s_aux[8 * ROWT / 64].  Returns false when its weights sum to zero.  All threads of the
-// workgroup (the wavefront, for ROWT = 64) call it together; the arrays in LDS may be rewritten only after a barrier.
+// The row `rr` by ROWT threads that share `smem` and, for the wavefronts' sums, s_aux[8 * ROWT / 64].  Returns false when its
+// weights sum to zero.  All threads of the workgroup (the wavefront, for ROWT = 64) call it together; the arrays in LDS may
+// be rewritten only after a barrier.
 template <int ROWT, int PER>
 __device__ __forceinline__ bool merge_row(const RowRef rr, uint64_t* smem, uint64_t* s_aux,
                                           const float* __restrict__ wgt, AliasEntry* __restrict__ table,

@@ -273,11 +273,6 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int mask) {
   const uint32_t hi = __shfl_xor((int)(uint32_t)(v >> 32), mask, 64);
   return ((uint64_t)hi << 32) | lo;
 }
-__device__ __forceinline__ uint64_t shfl_up_u64(uint64_t v, int delta) {
-  const uint32_t lo = __shfl_up((int)(uint32_t)v, delta, 64);
-  const uint32_t hi = __shfl_up((int)(uint32_t)(v >> 32), delta, 64);
-  return ((uint64_t)hi << 32) | lo;
-}
 // ---- DPP building blocks.  A wave is four rows of 16 lanes; row_shr:n moves data n lanes up inside a
 // row, wave_shr:1 one lane up in the whole wave, row_bcast15 / row_bcast31 carry the last lane of a row (of the first half) to
 // the next row(s).
@@ -326,12 +321,14 @@ __device__ __forceinline__ uint64_t group_scan_u64(uint64_t v) {
   }
   return v;
 }
-// Sums of surpluses, with saturation.  Weights below 2^-64 add nothing to the sum of their row of d and can have nearly d shares each:
-// in rows of 4,096 entries and more their surpluses may pass 2^64.  No deficit prefix reaches 2^63, so that a prefix that stays
-// at 2^64 - 1 decides what the true one does (its heavies are never reached); one that wraps would be taken for a small one.
-// A weight loses less than 2^-64 to the floor, so that all shares together are at most d (S + d) / S in units of that: twice the
-// row's d, which leaves every sum below 2^64, unless S < d.  That is a scale above 2^64, and such rows alone need saturation: it costs
-// four instructions for two (a walk with the table of every step 693 -> 718 us when every row's sums had it).
+// Sums of surpluses, with saturation.  Weights below 2^-64 add nothing to the sum of their row of d and can have nearly d
+// shares each: in rows of 4,096 entries and more their surpluses may pass 2^64.  No deficit prefix reaches 2^63, so that a
+// prefix that stays at 2^64 - 1 decides what the true one does (its heavies are never reached); one that wraps would be
+// taken for a small one.
+// A weight loses less than 2^-64 to the floor, so that all shares together are at most d (S + d) / S, S in units of that:
+// twice d, which leaves every sum below 2^64, unless S < d.  That is a scale above 2^64, and such rows alone need
+// saturation: it costs four instructions for two (walks, us: with the table of every step 693 -> 718 when every row's sums
+// had it, online without tables 232 -> 246; with two forms of the draw 716 -> 712 and 232 -> 235).
 // Where sums may be at their limit, what lies before a lane is the prefix of the lane before, not its own less its amount.
 // SAT false: ordinary sums.
 template <bool SAT = true>

@@ -135,7 +135,7 @@ __host__ __device__ __forceinline__ constexpr int degree_class(uint32_t d) {
   if (d <= 509) return CLS_LDS_W2;
   if (d <= 765) return CLS_MW2_6;
   const uint32_t nw = (d + 3 + 511) / 512;  // wavefronts of 512 slots that hold the row from any 16-byte phase
-  // The arrays of a longer row (12 to 14 bytes of LDS per slot) would leave room for one workgroup per CU only: such a row
+  // The arrays of a longer row (10 or 14 bytes of LDS per slot) would leave room for one workgroup per CU only: such a row
   // keeps its heavies alone in LDS, and its entries in registers as long as 512 threads can hold them (1024 threads
   // for rows of up to 16381 entries, one workgroup per CU, ran at 1.7 TB/s where the streaming kernel reaches 1.95).
   if (nw <= MERGE_MAX_NW) return CLS_MW2 + (int)nw - 2;

@@ -81,12 +81,13 @@ __global__ __launch_bounds__(T) void walk_direct_kernel(const uint32_t* __restri
 // BUILD_PS a entry, once) or two sweeps over its weights (about DRAW_PS a entry, each time).  A step leads to a row
 // with a probability that grows with its length, so a row of d entries is drawn from about N * len * d / E times, and
 // its table pays from the length on at which N * len * d / E * DRAW_PS exceeds BUILD_PS.  Measured on one MI355X.  The launches of
-// a build cost BUILD_US whatever they build, so it has to save as much; a step waits for the sweep of its row, so what is saved
-// counts CHAIN times what its bandwidth comes to (counted once, 1,873 x 11 steps on the scale-22 graph with 7 edges a
-// vertex went without tables, 176 us for 138; from 2 on it is right there, 4 is on the scale-17 graph with 43, 98 for 92).  (531 walkers x 6 steps on the scale-16 graph 75 ->
-// 54 us, 110 x 9 on the scale-20 graph with 32 edges a vertex 161 -> 114, 400 x 8 on the scale-22 graph 180 -> 134).  The same
-// ratio for a few thousand walkers and for many: tables from half that length on for the former made 3,000 x 16 steps on the
-// scale-23 graph 390 us, now 334, and 2,000 x 10 on the scale-24 graph 305, now 259.
+// a build cost BUILD_US whatever they build, so it has to save as much: without this rule 531 walkers x 6 steps on the scale-16
+// graph took 75 us, with it 54, 110 x 9 on the scale-20 graph with 32 edges a vertex 161 and 114, 400 x 8 on the scale-22 graph
+// 180 and 134.  A step waits for the sweep of its row, so what is saved counts CHAIN times what its bandwidth comes to: counted
+// once, 1,873 x 11 steps on the scale-22 graph with 7 edges a vertex go without tables, 176 us for 138.  From 2 on that is right;
+// 4 is right on the scale-17 graph with 43 as well, 98 us for 92 the other way.
+// The same ratio for a few thousand walkers and for many: tables from half that length on for the former made 3,000 x 16 steps on
+// the scale-23 graph 390 us, now 334, and 2,000 x 10 on the scale-24 graph 305, now 259.
 constexpr double BUILD_PS = 8.0, DRAW_PS = 2.5, CHAIN = 4.0;
 constexpr uint32_t FEW_WALKERS = 4096;
 constexpr double BUILD_US = 40.0, STEP_US = 4.0;  // launches of a build; the chain of loads and scans of a step
