@@ -635,23 +635,37 @@ def long_vanishing_rows(longest):
                                    {"tiled_max_tiles": 9}])
 def test_surpluses_beyond_64_bits(orc, knobs, longest):
     # by default in one launch or four, streamed or tile by tile, by class (rows of 5,118..8,189 entries held), by the kernels that the
-    # tests alone select; and the draws of a walk that builds no table against those from the tables
+    # tests alone select
     from skywalker_amd import capi
     rows = long_vanishing_rows(longest)
     w = np.concatenate(rows)
-    V = max(len(r) for r in rows)  # every slot of a row leads to a vertex of its own
-    xadj = np.full(V + 1, len(w), np.uint32)
-    xadj[:len(rows) + 1] = np.concatenate([[0], np.cumsum([len(r) for r in rows])])
-    g = capi.Graph.upload(xadj, np.concatenate([np.arange(len(r), dtype=np.uint32) for r in rows]), w)
+    xadj = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.uint32)
+    g = capi.Graph.upload(xadj, np.zeros(len(w), np.uint32), w)
     for k, value in knobs.items():
         g.set_option(k, value)
-    seeds = np.repeat(np.arange(len(rows), dtype=np.uint32), 40)
-    g.set_option("online_full_build", 0)
-    online = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 1, 0.0, 5)
     g.build_tables()
     compare_tables(orc, g, xadj, w, "surpluses beyond 64 bits, %s" % knobs)
-    offline = g.walk_offline(seeds, 1, 0.0, 5)
-    assert np.array_equal(online[0].to_host(), offline[0].to_host())
+    g.free()
+
+
+@pytest.mark.parametrize("walkers", [200, 1000, 5000])
+def test_draws_from_rows_with_surpluses_beyond_64_bits(walkers):
+    # evaluated from the weights, by workgroups of every size, against those from the tables.  20 M entries in rows of 32 beside
+    # them: of a graph so large this walk builds no row of up to 12,288 entries
+    from skywalker_amd import capi
+    rows = long_vanishing_rows(12288)
+    lens = np.concatenate([[len(r) for r in rows], np.full(625000, 32)])
+    w = np.concatenate(rows + [np.ones(32 * 625000, np.float32)])
+    xadj = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    local = np.arange(len(w), dtype=np.uint32) - np.repeat(xadj[:-1], lens)  # a vertex of its own for every slot of a row
+    g = capi.Graph.upload(xadj, local, w)
+    g.set_option("online_full_build", 0)
+    seeds = np.arange(walkers, dtype=np.uint32) % len(rows)
+    direct = [g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 1, 0.0, 5), g.walk_online(capi.BIAS_NODE2VEC, 2.0, 0.5, seeds, 1, 0.0, 5)]
+    g.build_tables()
+    tabled = g.walk_offline(seeds, 1, 0.0, 5)[0].to_host()
+    for paths, _, _, _ in direct:
+        assert np.array_equal(paths.to_host(), tabled)
     g.free()
 
 
