@@ -339,7 +339,7 @@ __global__ __launch_bounds__(ROWT) void build_lds_kernel(const RowRef* __restric
     }
   }
   uint64_t total_l, total_h;
-  block_scan2<ROWT, T, false>(dl, dh, s_ex, sl, sh, total_l, total_h, wave_live);  // its barrier also publishes s_fh / s_lh
+  block_scan2_as<ROWT, T, false>(dl, dh, s_ex, sl, sh, total_l, total_h, wave_live);  // its barrier also publishes s_fh / s_lh
 #pragma unroll
   for (int t = 0; t < T; ++t) {
     const uint32_t pos = 4u * (t * ROWT + tid);

@@ -12,10 +12,10 @@ constexpr uint32_t NONE32 = 0xFFFFFFFFu;
 // Bit q of `wave_live` (wave-uniform) clear means every value of this wave in sub-tile q is zero:
 // the wave then skips that sub-tile's scan.
 template <int ROWT, int Q, bool SAT>
-__device__ __forceinline__ void block_scan2(const uint64_t (&a)[Q][4], const uint64_t (&b)[Q][4],
-                                            uint64_t* __restrict__ s_ex /* [2 * Q * ROWT/64] */,
-                                            uint64_t (&oa)[Q][4], uint64_t (&ob)[Q][4], uint64_t& tot_a,
-                                            uint64_t& tot_b, uint32_t wave_live = 0xFFFFFFFFu) {
+__device__ __forceinline__ void block_scan2_as(const uint64_t (&a)[Q][4], const uint64_t (&b)[Q][4],
+                                               uint64_t* __restrict__ s_ex /* [2 * Q * ROWT/64] */,
+                                               uint64_t (&oa)[Q][4], uint64_t (&ob)[Q][4], uint64_t& tot_a,
+                                               uint64_t& tot_b, uint32_t wave_live = 0xFFFFFFFFu) {
   constexpr int NW = ROWT / 64;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   uint64_t ia[Q], ib[Q];
@@ -66,6 +66,15 @@ __device__ __forceinline__ void block_scan2(const uint64_t (&a)[Q][4], const uin
   }
   tot_a = run_a;
   tot_b = run_b;
+}
+// SAT where the row's surpluses may wrap: chosen here, where two forms of everything that follows would spill scalar registers (357
+// instructions an entry of a tile, 340 so, 337 without).
+template <int ROWT, int Q>
+__device__ __forceinline__ void block_scan2(bool may_wrap, const uint64_t (&a)[Q][4], const uint64_t (&b)[Q][4],
+                                            uint64_t* __restrict__ s_ex, uint64_t (&oa)[Q][4], uint64_t (&ob)[Q][4],
+                                            uint64_t& tot_a, uint64_t& tot_b) {
+  if (may_wrap) block_scan2_as<ROWT, Q, true>(a, b, s_ex, oa, ob, tot_a, tot_b);
+  else block_scan2_as<ROWT, Q, false>(a, b, s_ex, oa, ob, tot_a, tot_b);
 }
 
 // For four keys at once: number of entries of the sorted array that starts `base_k` bytes into the LDS

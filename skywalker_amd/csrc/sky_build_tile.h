@@ -241,7 +241,7 @@ __device__ __forceinline__ void resolve_in_tile(const TiledRow& r, const Ledger&
 
 // One pass over the partner tiles of one kind other than the own tile T: their per-slot prefix is
 // recomputed from the weights into LDS.
-template <bool OWN_HEAVY, bool SAT>
+template <bool OWN_HEAVY>
 __device__ __forceinline__ void partner_pass(const TiledRow& r, const Ledger& L, const float* __restrict__ wgt,
                                              const uint64_t* __restrict__ B, uint32_t t_lo, uint32_t t_hi,
                                              uint64_t* smem,
@@ -266,7 +266,8 @@ __device__ __forceinline__ void partner_pass(const TiledRow& r, const Ledger& L,
         pv[q][k] = e.heavy != OWN_HEAVY ? e.amount : 0;
       }
     __syncthreads();  // searches of the previous partner are done: s_ex and the prefix may be overwritten
-    block_scan1<TL_T, TL_Q, SAT && !OWN_HEAVY>(pv, s_ex, lo, ps);
+    if (!OWN_HEAVY && surpluses_may_wrap(L.scale)) block_scan1<TL_T, TL_Q, true>(pv, s_ex, lo, ps);
+    else block_scan1<TL_T, TL_Q, false>(pv, s_ex, lo, ps);
 #pragma unroll
     for (int q = 0; q < TL_Q; ++q)
 #pragma unroll
@@ -281,17 +282,37 @@ struct TileEmitLds {
   uint64_t s_ex[2 * TL_Q * (TL_T / 64)];
   uint32_t s_fh[TL_Q][TL_T / 64];
 };
-// Every entry of tile T of row `r`, whose weights are w.  SAT: the row's surpluses may wrap (surpluses_may_wrap).
-template <bool SAT>
-__device__ __forceinline__ void tile_entries(const TiledRow& r, const Ledger& L, uint32_t tile, uint32_t T, const float (&w)[TL_Q][4],
-                                             const float* __restrict__ wgt, const uint64_t* __restrict__ gBL,
-                                             const uint64_t* __restrict__ gBH, const uint32_t* __restrict__ nfh,
-                                             const uint4* __restrict__ ranges, AliasEntry* __restrict__ table, TileEmitLds& lds) {
+// Every entry of tile `tile` (tg.span not 0) by TL_T threads.
+__device__ __forceinline__ void tile_emit(const TileGeom& tg, uint32_t tile, const TiledRow* __restrict__ rows,
+                                          const float* __restrict__ wgt, const uint64_t* __restrict__ gBL,
+                                          const uint64_t* __restrict__ gBH, const uint32_t* __restrict__ nfh,
+                                          const uint4* __restrict__ ranges, AliasEntry* __restrict__ table,
+                                          int8_t* __restrict__ valid, TileEmitLds& lds) {
   constexpr int NW = TL_T / 64;
   auto& smem = lds.smem;
   auto& s_ex = lds.s_ex;
   auto& s_fh = lds.s_fh;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const uint32_t T = tg.T;
+
+  float w[TL_Q][4];
+  load_tile(wgt, geom_row(tg, tile), T, tid, w);  // requested before the row record arrives
+  const TiledRow r = rows[tg.row];
+  if (!r.ok) {
+#pragma unroll
+    for (int q = 0; q < TL_Q; ++q)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t idx = T * TILE + 4u * (q * TL_T + tid) + k;
+        if (in_row(r, idx)) {
+          table[r.base + idx] = AliasEntry{0.0f, SKY_INVALID};
+        }
+      }
+    if (T == 0 && tid == 0) valid[r.v] = 0;
+    return;
+  }
+  if (T == 0 && tid == 0) valid[r.v] = 1;
+  const Ledger L = row_ledger(r);
   const uint64_t* BL = gBL + r.bofs;  // tile prefixes of this row
   const uint64_t* BH = gBH + r.bofs;
   const uint64_t bl = BL[T], bl1 = BL[T + 1], bh = BH[T], bh1 = BH[T + 1];
@@ -330,13 +351,19 @@ __device__ __forceinline__ void tile_entries(const TiledRow& r, const Ledger& L,
       if (lane == 0) s_fh[q][wave] = fh;
     }
     uint64_t tl, th;
-    block_scan2<TL_T, TL_Q, SAT>(dl, dh, s_ex, sl, sh, tl, th);  // its barrier also publishes s_fh
+    const bool may_wrap = surpluses_may_wrap(L.scale);
+    block_scan2<TL_T, TL_Q>(may_wrap, dl, dh, s_ex, sl, sh, tl, th);  // its barrier also publishes s_fh
 #pragma unroll
     for (int q = 0; q < TL_Q; ++q)
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
+        const uint64_t inside = sh[q][k];
         sl[q][k] += bl;
-        sh[q][k] = add_sat<SAT>(sh[q][k], bh);
+        sh[q][k] += bh;
+        if (may_wrap) {
+          asm volatile("");  // a branch, not a select in every row
+          sh[q][k] = add_sat(inside, bh);
+        }
         key[q][k] = ((heavy_mask >> (q * 4 + k)) & 1) ? sh[q][k] - 1 : sl[q][k] - dl[q][k];
       }
   }
@@ -386,8 +413,8 @@ __device__ __forceinline__ void tile_entries(const TiledRow& r, const Ledger& L,
   resolve_in_tile<true>(r, L, smem, T, bl, bl1, heavy_mask, live_mask, nh_after, T, key, op, oa);
 
   // the other partner tiles (ranges precomputed per tile by tiled_scan_kernel)
-  partner_pass<false, SAT>(r, L, wgt, BH, rg.x, rg.y, smem, s_ex, heavy_mask, live_mask, nh_after, T, key, op, oa);
-  partner_pass<true, SAT>(r, L, wgt, BL, rg.z, rg.w, smem, s_ex, heavy_mask, live_mask, nh_after, T, key, op, oa);
+  partner_pass<false>(r, L, wgt, BH, rg.x, rg.y, smem, s_ex, heavy_mask, live_mask, nh_after, T, key, op, oa);
+  partner_pass<true>(r, L, wgt, BL, rg.z, rg.w, smem, s_ex, heavy_mask, live_mask, nh_after, T, key, op, oa);
 
 #pragma unroll
   for (int q = 0; q < TL_Q; ++q) {
@@ -403,36 +430,6 @@ __device__ __forceinline__ void tile_entries(const TiledRow& r, const Ledger& L,
         }
     }
   }
-}
-// Every entry of tile `tile` (tg.span not 0) by TL_T threads.
-__device__ __forceinline__ void tile_emit(const TileGeom& tg, uint32_t tile, const TiledRow* __restrict__ rows,
-                                          const float* __restrict__ wgt, const uint64_t* __restrict__ gBL,
-                                          const uint64_t* __restrict__ gBH, const uint32_t* __restrict__ nfh,
-                                          const uint4* __restrict__ ranges, AliasEntry* __restrict__ table,
-                                          int8_t* __restrict__ valid, TileEmitLds& lds) {
-  const int tid = threadIdx.x;
-  const uint32_t T = tg.T;
-
-  float w[TL_Q][4];
-  load_tile(wgt, geom_row(tg, tile), T, tid, w);  // requested before the row record arrives
-  const TiledRow r = rows[tg.row];
-  if (!r.ok) {
-#pragma unroll
-    for (int q = 0; q < TL_Q; ++q)
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const uint32_t idx = T * TILE + 4u * (q * TL_T + tid) + k;
-        if (in_row(r, idx)) {
-          table[r.base + idx] = AliasEntry{0.0f, SKY_INVALID};
-        }
-      }
-    if (T == 0 && tid == 0) valid[r.v] = 0;
-    return;
-  }
-  if (T == 0 && tid == 0) valid[r.v] = 1;
-  const Ledger L = row_ledger(r);
-  if (surpluses_may_wrap(L.scale)) tile_entries<true>(r, L, tile, T, w, wgt, gBL, gBH, nfh, ranges, table, lds);
-  else tile_entries<false>(r, L, tile, T, w, wgt, gBL, gBH, nfh, ranges, table, lds);
 }
 
 }  // namespace sky
