@@ -67,8 +67,8 @@ __device__ __forceinline__ void block_scan2_as(const uint64_t (&a)[Q][4], const 
   tot_a = run_a;
   tot_b = run_b;
 }
-// SAT where the row's surpluses may wrap: chosen here, where two forms of everything that follows would spill scalar registers (357
-// instructions an entry of a tile, 340 so, 337 without).
+// SAT where the row's surpluses may wrap: chosen here, where two forms of everything that follows would spill scalar
+// registers (357 instructions an entry of the tiles of the scale-26 graph, 345 so, 342 without).
 template <int ROWT, int Q>
 __device__ __forceinline__ void block_scan2(bool may_wrap, const uint64_t (&a)[Q][4], const uint64_t (&b)[Q][4],
                                             uint64_t* __restrict__ s_ex, uint64_t (&oa)[Q][4], uint64_t (&ob)[Q][4],
