@@ -328,7 +328,7 @@ __device__ __forceinline__ uint64_t group_scan_u64(uint64_t v) {
 // A weight loses less than 2^-64 to the floor, so that all shares together are at most d (S + d) / S, S in units of that:
 // twice d, which leaves every sum below 2^64, unless S < d.  That is a scale above 2^64, and such rows alone need
 // saturation: it costs four instructions for two (walks, us: with the table of every step 693 -> 718 when every row's sums
-// had it, online without tables 232 -> 246; with two forms of the draw 716 -> 712 and 232 -> 235).
+// had it, online without tables 232 -> 246; with two forms of the draw 687 -> 680 and 232 -> 234).
 // Where sums may be at their limit, what lies before a lane is the prefix of the lane before, not its own less its amount.
 // SAT false: ordinary sums.
 template <bool SAT = true>

@@ -52,7 +52,9 @@ __device__ __forceinline__ uint32_t draw_entry(Row& row, const uint32_t d, const
                                                const float u, const uint32_t csz, const uint32_t nc, const uint32_t c0,
                                                const uint32_t c1, DrawLds<T>& lds) {
   constexpr int NW = T / 64;
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  uint32_t tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // what depends on the lane number stays inside this form's code
+  const uint32_t wave = tid >> 6, lane = tid & 63;
   // the four slots of this lane in the 256 from `base` on: amounts of the two kinds
   auto amounts = [&](uint32_t base, uint64_t (&dd)[4], uint64_t (&uu)[4]) {
     float w[4];
