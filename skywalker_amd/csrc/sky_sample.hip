@@ -56,7 +56,8 @@ struct SampleArgs {
 // The parent in slot s of hop g.h, V when the slot is not filled.
 __device__ __forceinline__ uint32_t parent_of(const SampleArgs& a, const HopGeom& g, uint64_t si, uint32_t s) {
   if (g.h == 0 && a.seeds) return a.seeds[si];
-  return slot_filled(g, a.sl, si, s) ? a.data[si * g.lps + g.off + s] : 0xFFFFFFFFu;
+  const uint32_t v = a.data[si * g.lps + g.off + s];  // beside the count that says whether it is one
+  return slot_filled(g, a.sl, si, s) ? v : 0xFFFFFFFFu;
 }
 
 // Children with replacement: one lane per (slot, draw), U of them at a time so that their chains of four dependent
@@ -154,8 +155,16 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_draw_kernel(SampleArgs a) {
 // until no two candidates are equal.  The sequential rule comes out of this exactly, in as many rounds of dependent
 // loads as candidates collide in a row, where one lane per parent took one per try: hop 1 of a 1024-seed batch with
 // fanout 25 197 -> 17 us.
+// What bounds a batch is the start vertex with the most rounds, and rounds are many where a row is hardly longer than k (25
+// draws from 29 entries took 47, with 1.8 the mean of 1,024 start vertices).  Such a row, of up to 64 entries, is therefore held in
+// LDS, entries and neighbours both, which also makes one dependent load of two.  A bit for every entry then says what is taken:
+// a prefix over the draws of their candidates' bits finds f, the bits before f are final, and a draw that meets one of
+// them goes on until it meets none, in the same round.  No more than k rounds, none of which leaves the CU: 1,024 seeds, 25 x 10 on the
+// scale-20 graph 50 -> 36 us.
 constexpr uint32_t DISTINCT_MAX_K = 64;  // largest fanout of this rule
 constexpr uint32_t DISTINCT_ROUNDS = 11;
+// Entries a lane of a row that its group holds in LDS: 24 KB for 512 threads, four workgroups of which are all wavefronts that a CU takes.
+constexpr uint32_t DISTINCT_ROW = 4;
 __host__ __device__ inline uint32_t distinct_lanes(uint32_t k) {
   uint32_t g = 4;
   while (g < k) g *= 2;
@@ -166,6 +175,8 @@ __host__ __device__ inline uint32_t distinct_lanes(uint32_t k) {
 template <int T>
 __global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
   __shared__ __align__(16) uint32_t s_c[T];
+  __shared__ AliasEntry s_row[T * DISTINCT_ROW];
+  __shared__ uint32_t s_adj[T * DISTINCT_ROW];
   __shared__ uint32_t s_n[T / 64];
   if (a.h0 == 0) call_stamp(a.call);
   const uint64_t si = a.first + blockIdx.x / a.parts;
@@ -184,58 +195,117 @@ __global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
       const bool in = slot < g.width;
       const uint32_t v = in ? parent_of(a, g, si, s) : 0xFFFFFFFFu;
       uint32_t o = 0, deg = 0;
-      if (v < a.V && a.valid[v]) {
+      if (v < a.V) {
+        const int8_t ok = a.valid[v];  // beside the bounds
         o = a.xadj[v];
         deg = a.xadj[v + 1] - o;
+        if (!ok) deg = 0;
+      }
+      // Five draws and fewer collide so seldom that only a start vertex with several wavefronts, which wait for the slowest of
+      // them, gains (3,000 seeds, 5 x 3 on the scale-18 graph 27 -> 25 us; one wavefront each, 5,000 seeds, 15 x 10 x 5 217 -> 223).
+      const bool held = G >= (T > 64 ? 8u : 16u) && deg > k && deg <= min(64u, DISTINCT_ROW * G);
+      const uint32_t rbase = DISTINCT_ROW * gbase;
+      if (held) {
+#pragma unroll
+        for (uint32_t m = 0; m < DISTINCT_ROW; ++m) {
+          const uint32_t j = m * G + i;
+          if (j < deg) {
+            s_row[rbase + j] = a.table[o + j];
+            s_adj[rbase + j] = a.adjncy[o + j];
+          }
+        }
       }
       uint32_t cand = 0, child = 0, t = 0;
       bool live = i < min(deg, k);  // a draw that keeps something, as far as is known
-      // The entry of the next try is requested when this one's candidate is taken (1,024 seeds, 25 x 10 on the scale-20 graph 60 -> 58 us,
-      // 806 with 4 edges a vertex 43 -> 38; several tries at once cost more in random numbers than they save: 65).
+      const bool direct = deg > k && !held;
       uint32_t col = 0;
       float u = 0.0f;
-      AliasEntry e{0.0f, 0};
-      auto request = [&](uint32_t round) {
+      auto numbers = [&](uint32_t round) {
         const u32x4 r = philox(a.seed, (uint32_t)si, s * k + i, g.h + 256u * round, DOM_SAMPLE);
         col = __umulhi(r.x, deg);
         u = u24(r.y);
-        e = a.table[o + col];
       };
-      auto take = [&] {
-        cand = u < e.prob ? col : e.alias;
-        child = a.adjncy[o + cand];
-        if (t + 1 < DISTINCT_ROUNDS) request(t + 1);
-      };
-      if (live) {
-        if (deg > k) {
-          request(0);
-          take();
-        } else {
-          child = a.adjncy[o + (cand = i)];  // all neighbours
-        }
+      if (live && deg > k) numbers(0);
+      AliasEntry e{0.0f, 0};
+      if (live && !held) {  // on its way meanwhile
+        if (direct) e = a.table[o + col];
+        else child = a.adjncy[o + (cand = i)];  // all neighbours
       }
-      for (;;) {
-        s_c[tid] = cand;
+      if (__any(held)) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        unsigned long long same = 0;  // earlier draws of the group with this draw's candidate
-        for (uint32_t j = 0; j < k; j += 4) {
-          const uint4 c = *reinterpret_cast<const uint4*>(s_c + gbase + j);
-          const uint32_t m = (c.x == cand ? 1u : 0u) | (c.y == cand ? 2u : 0u) | (c.z == cand ? 4u : 0u) | (c.w == cand ? 8u : 0u);
-          same |= (unsigned long long)m << j;
+        auto take = [&] {
+          const AliasEntry x = s_row[rbase + col];
+          cand = u < x.prob ? col : x.alias;
+        };
+        if (held && live) take();
+        for (;;) {
+          const uint64_t bit = held && live ? 1ull << cand : 0ull;
+          uint64_t before = bit;  // candidates of this draw and the earlier ones of its group, then of the earlier ones
+          auto from = [&](uint32_t dist, uint64_t x) { before |= i >= dist ? x : 0ull; };
+          from(1, dpp0_u64<DPP_ROW_SHR1, 0xF>(before));
+          from(2, dpp0_u64<DPP_ROW_SHR2, 0xF>(before));
+          from(4, dpp0_u64<DPP_ROW_SHR4, 0xF>(before));
+          from(8, dpp0_u64<DPP_ROW_SHR8, 0xF>(before));
+          if (G >= 32) before |= dpp0_u64<DPP_ROW_BCAST15, 0xA>(before);
+          if (G >= 64) before |= dpp0_u64<DPP_ROW_BCAST31, 0xC>(before);
+          before = lane_before_u64(before);
+          if (i == 0) before = 0;
+          const unsigned long long bad = group_mask((before & bit) != 0);
+          if (!__any(bad != 0)) break;
+          const uint32_t f = bad ? (uint32_t)__ffsll((long long)bad) - 1 : 0u;
+          const uint64_t final = bad ? shfl_u64(before, (int)((lane & ~(G - 1)) + f)) : 0ull;
+          bool taken = i >= f && (bit & final);
+          while (__any(taken)) {
+            if (taken) {
+              if (++t == DISTINCT_ROUNDS) {
+                live = taken = false;
+              } else {
+                numbers(t);
+                take();
+                taken = (final >> cand) & 1;
+              }
+            }
+          }
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the next round's candidates stay behind these reads
-        __builtin_amdgcn_wave_barrier();
-        const unsigned long long alive = group_mask(live);
-        same &= alive & ((1ull << i) - 1ull);
-        const unsigned long long bad = group_mask(live && same != 0);
-        if (!__any(bad != 0)) break;
-        if (bad) {
-          const uint32_t f = (uint32_t)__ffsll((long long)bad) - 1;
-          if (live && i >= f && (same & ((1ull << f) - 1ull))) {  // a final draw holds the candidate
-            if (++t == DISTINCT_ROUNDS) live = false;
-            else take();
+        if (held && live) child = s_adj[rbase + cand];
+      }
+      if (__any(live && !held)) {
+        // The entry of the next try is requested when this one's candidate is taken (1,024 seeds, 25 x 10 on the scale-20 graph 60 -> 58 us,
+        // 806 with 4 edges a vertex 43 -> 38; several tries at once cost more in random numbers than they save: 65).
+        auto take = [&] {
+          cand = u < e.prob ? col : e.alias;
+          child = a.adjncy[o + cand];
+          if (t + 1 < DISTINCT_ROUNDS) {
+            numbers(t + 1);
+            e = a.table[o + col];
+          }
+        };
+        if (live && direct) take();
+        for (;;) {
+          s_c[tid] = cand;
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          unsigned long long same = 0;  // earlier draws of the group with this draw's candidate
+          for (uint32_t j = 0; j < k; j += 4) {
+            const uint4 c = *reinterpret_cast<const uint4*>(s_c + gbase + j);
+            const uint32_t m = (c.x == cand ? 1u : 0u) | (c.y == cand ? 2u : 0u) | (c.z == cand ? 4u : 0u) | (c.w == cand ? 8u : 0u);
+            same |= (unsigned long long)m << j;
+          }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the next round's candidates stay behind these reads
+          __builtin_amdgcn_wave_barrier();
+          const unsigned long long alive = group_mask(live);
+          same &= alive & ((1ull << i) - 1ull);
+          const unsigned long long bad = group_mask(live && direct && same != 0);
+          if (!__any(bad != 0)) break;
+          if (bad) {
+            const uint32_t f = (uint32_t)__ffsll((long long)bad) - 1;
+            if (live && i >= f && (same & ((1ull << f) - 1ull))) {  // a final draw holds the candidate
+              if (++t == DISTINCT_ROUNDS) live = false;
+              else take();
+            }
           }
         }
       }

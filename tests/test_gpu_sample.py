@@ -76,6 +76,30 @@ def test_distinct_children_match_oracle(orc, fanout):
         assert (osl[big, 0] < fanout[1]).any()  # a parent that ended with fewer children than its fanout is among the cases
 
 
+@pytest.mark.parametrize("weights", ["lognormal2", "sparse"])
+@pytest.mark.parametrize("fanout", [[1, 1, 2], [1, 3, 5], [1, 9, 16], [1, 17, 2], [1, 33, 1], [1, 63], [1, 64]])
+def test_distinct_children_of_rows_held_in_lds(orc, fanout, weights):
+    # a group of lanes holds a row of at most four entries a lane, and of at most 64, and finds taken slots by their bits: rows
+    # at both limits and at the fan-out's, with draws that run out of tries (a few entries with most of the weight)
+    from skywalker_amd import capi
+    rng = np.random.default_rng(61)
+    degs = [0, 1, 2, 3, 4, 5, 15, 16, 17, 18, 31, 32, 33, 34, 35, 62, 63, 64, 65, 66, 130]
+    xadj, adjncy, w = graph_from_degrees(degs * 12, rng, weights)
+    V = len(xadj) - 1
+    prob, alias, valid = orc.alias_build(xadj, w)
+    seeds = rng.integers(0, V + 1, 700).astype(np.uint32)
+    lps, slen = capi.sample_layout(fanout)
+    want = orc.sample_offline(xadj, adjncy, prob, alias, seeds, fanout, 29, distinct=True)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    g.set_option("sample_distinct", 1)
+    for call in (g.sample_offline, g.sample_online):
+        data, sl, sampled, _ = call(seeds, fanout, 29)
+        assert np.array_equal(sl.to_host((700, slen)), want[1]) and np.array_equal(data.to_host((700, lps)), want[0])
+        assert sampled == want[2]
+    g.free()
+
+
 def test_online_sampling_with_short_rows_built_in_vertex_order(orc):
     # option small_in_place = 1 on a list of frontier vertices (by default only builds of 2^25 rows and more use it)
     from skywalker_amd import capi
