@@ -16,12 +16,14 @@ struct CallDevice {
   unsigned long long sampled;  // edges sampled so far
   unsigned long long pad[6];
 };
-// Pinned host words of a call, written by the end kernel.
+// Pinned host words of a call, written by the end kernel: each carries the number of the call in its upper 16 bits, so that the
+// host knows which of them has arrived and neither waits for the other on its way over PCIe (results first, then, released, a
+// number of their own: a round trip more, 0.4 to 0.8 us of a call of 15 to 30).
 struct CallHost {
-  unsigned long long seq;  // number of the last call that has ended
   unsigned long long sampled, ticks;
-  unsigned long long pad[5];
+  unsigned long long pad[6];
 };
+constexpr int CALL_VALUE_BITS = 48;  // 2^48 edges fill the GPU's memory a thousand times over; 2^48 ticks of 10 ns are a month
 static_assert(sizeof(CallDevice) == 64 && sizeof(CallHost) == 64, "one cache line each");
 // Where a call reports.  A graph has one for the calls that begin and end within one entry point; a call that stays open
 // between entry points (a sampling session) has its own, because other calls on the graph begin and end meanwhile.
@@ -40,11 +42,12 @@ __device__ __forceinline__ void call_stamp(CallDevice* call) {
 // Last statement of the call's last kernel, by one thread that has seen every other thread's contribution.
 __device__ __forceinline__ void call_report(CallDevice* call, CallHost* host, unsigned long long seq,
                                             unsigned long long sampled) {
-  host->sampled = sampled;
-  host->ticks = call->start ? wall_clock64() - call->start : 0;  // 0: the call had nothing to launch
+  const unsigned long long start = call->start, ticks = start ? wall_clock64() - start : 0;  // 0: the call had nothing to launch
+  constexpr unsigned long long VALUE = (1ull << CALL_VALUE_BITS) - 1;
+  __hip_atomic_store(&host->sampled, (sampled & VALUE) | seq << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  __hip_atomic_store(&host->ticks, (ticks & VALUE) | seq << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   call->start = 0;
   call->sampled = 0;
-  __hip_atomic_store(&host->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // The device words of `w` (taken on first use), cleared; a call that ended in an error may have left something in them.

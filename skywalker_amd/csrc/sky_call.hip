@@ -88,7 +88,7 @@ int take_words(int device, CallWords* w) {
   w->dev = use->dev + k;
   w->host = use->host + k;
   w->khz = use->khz;
-  w->seq = use->host[k].seq;
+  w->seq = use->host[k].sampled >> CALL_VALUE_BITS;  // not the next call's
   return SKY_OK;
 }
 }  // namespace
@@ -142,7 +142,13 @@ int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, con
   hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, st, w->dev, w->host, seq, counts,
                      (uint32_t)n);
   SKY_HIP(hipGetLastError());
-  auto ended = [&] { return __atomic_load_n(&w->host->seq, __ATOMIC_ACQUIRE) == seq; };
+  unsigned long long words[2];
+  auto ended = [&] {
+    words[0] = __atomic_load_n(&w->host->sampled, __ATOMIC_ACQUIRE);
+    words[1] = __atomic_load_n(&w->host->ticks, __ATOMIC_ACQUIRE);
+    constexpr unsigned long long NUMBER = 0xFFFFull << CALL_VALUE_BITS;
+    return !(((words[0] ^ seq << CALL_VALUE_BITS) | (words[1] ^ seq << CALL_VALUE_BITS)) & NUMBER);
+  };
   bool done = ended();
   if (!done) {
     const auto t0 = std::chrono::steady_clock::now();
@@ -158,8 +164,9 @@ int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, con
     if (!ended()) return fail(SKY_ERR_HIP, "the call's end was not reported");
   }
   w->dirty = false;
-  if (sampled) *sampled = w->host->sampled;
-  if (seconds) *seconds = (double)w->host->ticks / ((double)w->khz * 1e3);
+  constexpr unsigned long long VALUE = (1ull << CALL_VALUE_BITS) - 1;
+  if (sampled) *sampled = words[0] & VALUE;
+  if (seconds) *seconds = (double)(words[1] & VALUE) / ((double)w->khz * 1e3);
   return SKY_OK;
 }
 int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
