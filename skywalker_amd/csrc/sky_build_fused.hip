@@ -57,6 +57,7 @@ struct FusedArgs {
   AliasEntry* table;
   int8_t* valid;
   uint32_t V, per_wave;  // SEC_SWEEP
+  bool split;            // a wavefront for every class of a range's rows, four that follow one another (SPLIT_SWEEP)
   // rows built tile by tile
   TiledRow* trows;
   const TileGeom* geom;
@@ -253,6 +254,11 @@ __device__ __forceinline__ void tile_totals_wave(const FusedArgs& a, uint32_t ti
   else totals(std::false_type{});
 }
 
+__device__ __forceinline__ void sweep_unit(const FusedArgs& a, uint32_t unit, uint64_t* smem) {
+  small_rows_range((a.split ? unit / 4 : unit) * a.per_wave, a.xadj, a.wgt, nullptr, a.V, a.per_wave, a.table, a.valid, smem,
+                   a.split ? 1u << (unit % 4) : 15u);
+}
+
 template <bool DEV, int G, int PER>
 __device__ __forceinline__ void group_unit(const FusedArgs& a, const SectionRef& s, uint32_t unit, uint32_t rows,
                                            uint64_t* smem) {
@@ -296,7 +302,7 @@ __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
     switch (s.kind) {
       case SEC_SWEEP:
         if constexpr (!DEV)
-          small_rows_range(unit * a.per_wave, a.xadj, a.wgt, nullptr, a.V, a.per_wave, a.table, a.valid, smem);
+          sweep_unit(a, unit, smem);
         break;
       case SEC_TINY:
         if constexpr (DEV) {
@@ -434,7 +440,7 @@ __global__ __launch_bounds__(512, 4) void fused_all_kernel(FusedArgs a) {
   uint64_t* const wmem = smem + wave * (ALL_SLICE / 8);
   uint64_t* const w_aux = wmem + (ALL_SLICE - 64) / 8;
   switch (s.kind) {
-    case SEC_SWEEP: small_rows_range(wunit * a.per_wave, a.xadj, a.wgt, nullptr, a.V, a.per_wave, a.table, a.valid, wmem); break;
+    case SEC_SWEEP: sweep_unit(a, wunit, wmem); break;
     case SEC_G16: group_unit<false, SHAPE_G16.lanes, SHAPE_G16.per>(a, s, wunit, rows, wmem); break;
     case SEC_G32: group_unit<false, SHAPE_G32.lanes, SHAPE_G32.per>(a, s, wunit, rows, wmem); break;
     case SEC_G32S: group_unit<false, SHAPE_G32S.lanes, SHAPE_G32S.per>(a, s, wunit, rows, wmem); break;
@@ -534,6 +540,13 @@ constexpr uint32_t LEDGER_TILES = 2048;
 constexpr uint64_t ALL_MOST = 4096;
 constexpr uint32_t ALL_LONGEST = 12288;
 static_assert(ALL_LONGEST <= 24576, "none is of class CLS_STREAM");
+
+// Graphs of at most so many vertices sweep their rows of up to 32 entries with four wavefronts a range, one to a class: nothing but
+// the chain of a wavefront's batches bounds so few rows, and there one batch is left of four.  More vertices keep the GPU busy
+// without, and four wavefronts that share their lines read and write them four times (one wavefront / four, us: scale 9 with 5
+// edges a vertex 17.2 / 13.6, scale 10 with 8 17.7 / 13.6, scale 13 with 8 19.6 / 14.9, scale 15 with 3 19.0 / 15.5, with 20 32.3 / 32.5,
+// scale 16 with 8 25.5 / 26, scale 17 with 4 19.7 / 20.5, scale 18 with 3 25.7 / 28, scale 20 with 16 137 / 171).
+constexpr uint32_t SPLIT_SWEEP = 1u << 15;
 
 // Rows of 5118..8189 entries from which they are a launch of their own (10,000 rows of 6,500 streamed 478 us, held 402; 20,000
 // 885 and 745): fewer save less than a launch costs.
@@ -708,7 +721,9 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   // Vertices of a wavefront: enough wavefronts for every SIMD, but 256 rather than fewer where four wavefronts a SIMD remain: the
   // rows of a few vertices fill no batch of their class.  (4.4 M entries in 870,000 rows 51 us with 64, 40 with 192; 6.3 M in
   // 2 M rows 113 with 256, 124 with 512; 20 M in 4 M rows 115 with 448, 125 with 960.)
-  base.per_wave = std::max(64u, std::min(SMALL_RANGE, std::max(g->V / 8192u, std::min(256u, g->V / 4096u)) / 64u * 64u));
+  base.split = g->V <= SPLIT_SWEEP;
+  base.per_wave = base.split ? 64u : std::max(64u, std::min(SMALL_RANGE, std::max(g->V / 8192u, std::min(256u, g->V / 4096u)) / 64u * 64u));
+  const uint32_t ranges = (g->V + base.per_wave - 1) / base.per_wave, sweeps = base.split ? 4 * ranges : ranges;
   auto rows = [&](int c) { return class_min_degree(c) >= min_degree ? g->bin_counts[c] : 0u; };
   uint32_t past_wave = 0;  // rows of more than 509 entries: what a second launch would be for
   for (int c = CLS_COUNT - 1; c > CLS_LDS_W2; --c)
@@ -732,7 +747,7 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
     range(SEC_B6, CLS_MW2, CLS_MW2 + 4);
     all.add(SEC_B6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
     waves(SEC_W2, CLS_LDS_W2, 1);
-    if (min_degree == 0) all.add(SEC_SWEEP, g->V, base.per_wave * ALL_WAVES, 0);
+    if (min_degree == 0) all.add(SEC_SWEEP, sweeps, ALL_WAVES, 0);
     waves(SEC_W6, CLS_LDS_W6, 1);
     waves(SEC_W1, CLS_LDS_W1, 1);
     waves(SEC_G32X, CLS_G32X, 64 / SHAPE_G32X.lanes);
@@ -749,7 +764,7 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
   wave.add(SEC_SUM, n_tiles, 1, 0);
   wave.add(SEC_W2, rows(CLS_LDS_W2), 1, p.start[CLS_LDS_W2]);
-  if (min_degree == 0) wave.add(SEC_SWEEP, g->V, base.per_wave, 0);
+  if (min_degree == 0) wave.add(SEC_SWEEP, sweeps, 1, 0);
   wave.add(SEC_W6, rows(CLS_LDS_W6), 1, p.start[CLS_LDS_W6]);
   wave.add(SEC_W1, rows(CLS_LDS_W1), 1, p.start[CLS_LDS_W1]);
   wave.add(SEC_G32X, rows(CLS_G32X), 64 / SHAPE_G32X.lanes, p.start[CLS_G32X]);

@@ -462,11 +462,12 @@ constexpr size_t SMALL_STRIPS = smax(group_lds_bytes(SHAPE_G2.lanes, SHAPE_G2.pe
                                      smax(group_lds_bytes(SHAPE_G4.lanes, SHAPE_G4.per, 64), group_lds_bytes(SHAPE_G8.lanes, SHAPE_G8.per, 64)));
 static_assert(SMALL_STRIPS % 8 == 0);
 constexpr size_t SMALL_LDS_BYTES = SMALL_STRIPS + SMALL_QTOTAL * 6;
-// Vertices [lo, lo + per_wave) of the n (src null: the vertices themselves) by one wavefront.
+// Vertices [lo, lo + per_wave) of the n (src null: the vertices themselves) by one wavefront.  `queues`: bit q set for the rows of queue q,
+// rows of no entries with those of 1..2; the others are left to other wavefronts.
 __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __restrict__ xadj, const float* __restrict__ wgt,
                                                  const uint32_t* __restrict__ src, uint32_t n, uint32_t per_wave,
                                                  AliasEntry* __restrict__ table, int8_t* __restrict__ valid,
-                                                 uint64_t* __restrict__ smem) {
+                                                 uint64_t* __restrict__ smem, uint32_t queues = 15u) {
   uint32_t* q_off = reinterpret_cast<uint32_t*>(smem + SMALL_STRIPS / 8);  // [SMALL_QTOTAL]
   uint16_t* q_it = reinterpret_cast<uint16_t*>(q_off + SMALL_QTOTAL);  // [SMALL_QTOTAL]
   const uint32_t lane = threadIdx.x & 63;
@@ -539,8 +540,10 @@ __device__ __forceinline__ void small_rows_range(uint32_t lo, const uint32_t* __
     if (base + 64u < hi) fetch(base + 64u, nv, noff, nend);
     int q = -1;
     if (v != 0xFFFFFFFFu && d <= 32u) {
-      valid[v] = d != 0;  // a row without weight clears it when it is built
-      q = d == 0 ? -1 : d <= 2 ? 0 : d <= 8 ? 1 : d <= 16 ? 2 : 3;
+      q = d <= 2 ? 0 : d <= 8 ? 1 : d <= 16 ? 2 : 3;
+      if ((queues >> q) & 1) valid[v] = d != 0;  // a row without weight clears it when it is built
+      else q = -1;
+      if (d == 0) q = -1;
     }
     const uint32_t packed = (d << 10) | (base - lo + lane);
 #pragma unroll

@@ -531,6 +531,25 @@ def test_small_builds_in_one_launch(orc, dist, longest):
     g.free()
 
 
+@pytest.mark.parametrize("vertices", [1, 63, 64, 65, 32767, 32768, 32769])
+@pytest.mark.parametrize("longest", [32, 510])
+def test_short_rows_swept_by_class(orc, vertices, longest):
+    # up to 32,768 vertices: a wavefront for every class of a range's rows (longest 32: the launch of single wavefronts, 510: the one
+    # launch of eight); one more vertex: one wavefront for all of them.  Flags too: rows without entries and without weight
+    from skywalker_amd import capi
+    rng = np.random.default_rng(vertices + longest)
+    degs = rng.integers(0, 33, vertices)
+    degs[-1] = longest
+    xadj, _, w = graph_from_degrees(degs, rng, "lognormal2", V=max(vertices, 2))
+    w[rng.random(len(w)) < 0.3] = 0.0
+    adjncy = np.zeros(len(w), np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    for _ in range(2):
+        g.build_tables()
+        compare_tables(orc, g, xadj, w, vertices)
+    g.free()
+
+
 def few_carry_the_mass(d, k0, e):
     """Shares of the mean weight, in units of 2^-40 all whole: one heavy, then lights whose deficits reach its surplus as the last
     of them is taken, e units more.  Deficits and surpluses together pass 2^53 on the way there for d > 4103, at an odd number."""
