@@ -484,12 +484,21 @@ int walk_offline_noalloc(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32
 // probe until it is known to be needed, or reading the next step's entry during the search as if the candidate were
 // kept, was slower.
 //
-// A turn of the loop is one trial of every walker of the wavefront, whichever step each of them is in: where a turn was a step,
+// A turn of the loop is TR trials of every walker of the wavefront, whichever step each of them is in: where a turn was a step,
 // every walker waited in each for the one with the most trials.
 //
 // A walk lasts as long as its longest chain of dependent loads, so G is the largest whose wavefronts are all resident at
 // once (seven on each of the 1024 SIMDs); once the walkers alone fill the GPU the lanes are worth more as walkers.
+// Where no trial is in need of a search (q = 1) two lanes, that hold the next trial's numbers and the next step's, are as good as many
+// (p = 4, 50,000 walkers x 40 on the scale-20 graph: 2 lanes 110 us, 8 191; 8,000 x 30 on the scale-22 graph: 2 59, 4 60, 32 102;
+// 500 x 60, scale 16: 2 89, 4 74, 64 77).
+// TR: where half of the trials fail or more, four are drawn at once, a lane each, and the first that is kept ends the step, or, of
+// two that depend on the previous row, the first is searched for and the other left to the next turn.  (One at a time / four, us: p = 1/4,
+// q = 1: 500 x 60, scale 16, 224 / 121, 8,000 x 30, scale 22, 256 / 143, 50,000 x 40, scale 20, 371 / 273; p = 1/2, q = 2: 220 / 143, 275 / 178,
+// 490 / 396.  Where three in four are kept, p = 2, q = 1/2: 91 / 101, 120 / 134, 222 / 294; where the walkers alone fill the GPU, 150,000 x 30,
+// scale 22, p = 1/4, q = 1: 482 / 637.)
 constexpr uint64_t N2V_LANES = 7ull * 1024 * 64;
+constexpr int N2V_TRIALS = 4;
 template <int G>
 __device__ __forceinline__ unsigned long long group_ballot(bool p) {
   const unsigned long long b = __ballot(p) >> (lane_id() & (64u - G));
@@ -523,17 +532,19 @@ __device__ __forceinline__ bool group_row_has(const uint32_t* __restrict__ row, 
   return group_ballot<G>(gl < len && row[lo + gl] == key) != 0;
 }
 
-template <int G>
+template <int G, int TR>
 __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
     const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
     const AliasEntry* __restrict__ table, const uint32_t* __restrict__ seeds, uint32_t walker0, uint32_t N, uint32_t V, uint32_t len,
     float fp, float fq, float fmax, float stop_prob, uint64_t seed, bool once, uint32_t* __restrict__ paths,
     uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
-  // Numbers kept of a step, a lane each, of the last one fewer: at least the next trial's and the next step's first.
-  constexpr uint32_t TRIALS = G < 4 ? 1 : G < 16 ? 3 : G < 32 ? 4 : 8;
+  // One trial a turn: the numbers of the next one and of the next step's first are kept, which takes two lanes.  Four: those of the turn.
+  static_assert(TR == 1 ? G >= 2 : TR == N2V_TRIALS && G >= TR, "a lane for every number that is kept");
+  // Numbers kept of a step, a lane each, of the last one fewer.
+  constexpr uint32_t TRIALS = TR == 1 ? (G < 4 ? 1 : G < 16 ? 3 : G < 32 ? 4 : 8) : G < 16 ? TR : 2 * TR;
   if (walker0 == 0) call_stamp(call);
   const uint64_t wi = walker0 + ((uint64_t)blockIdx.x * WALK_BLOCK + threadIdx.x) / G;
-  const uint32_t i = (uint32_t)wi, gl = threadIdx.x & (G - 1);
+  const uint32_t i = (uint32_t)wi, gl = threadIdx.x & (G - 1), my = gl & (TR - 1);
   const int base = (int)(lane_id() & (64u - G));  // first lane of the group
   const bool first = gl == 0;                     // the lane that writes for the group
   uint32_t s = 0;
@@ -554,35 +565,71 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
       };
       // what lane l holds; the only walker of a wavefront needs no exchange through LDS for it
       auto of = [&](uint32_t x, int l) -> uint32_t {
-        if (G == 64) return (uint32_t)__builtin_amdgcn_readlane((int)x, __builtin_amdgcn_readfirstlane(l));
+        if (G == 64 && TR == 1) return (uint32_t)__builtin_amdgcn_readlane((int)x, __builtin_amdgcn_readfirstlane(l));
         return (uint32_t)__shfl((int)x, l, 64);
       };
       u32x4 mine = numbers();
       const float lo = fminf(1.0f, fq), hi = fmaxf(1.0f, fq);
       for (;;) {
+        if (TR > 1 && __any(lane_of(s, t) >= (uint32_t)G || lane_of(s, t + TR - 1) >= (uint32_t)G)) {
+          sb = s;
+          tb = t;
+          mine = numbers();
+        }
         const int from = base + (int)lane_of(s, t);
         if (t == 0 && ((stop_prob > 0.0f && u24(of(mine.z, from)) < stop_prob) || deg == 0)) break;
-        const uint32_t rx = of(mine.x, from), ry = of(mine.y, from), rw = of(mine.w, from);
+        const uint32_t rx = of(mine.x, from + (int)my), ry = of(mine.y, from + (int)my), rw = of(mine.w, from + (int)my);
         const uint32_t col = __umulhi(rx, deg);
         const AliasEntry e = once ? load_entry_once(table + off + col) : table[off + col];
         // The numbers of what may come next, while the entry is on its way: all walkers of the wavefront together.
-        if (__any(lane_of(s, t + 1) >= (uint32_t)G || lane_of(s + 1, 0) >= (uint32_t)G)) {
+        if (G > TR && __any((TR == 1 && lane_of(s, t + 1) >= (uint32_t)G) || lane_of(s + 1, TR - 1) >= (uint32_t)G)) {
           sb = s;
           tb = t + 1;
           mine = numbers();
           asm volatile("" : "+v"(mine.x), "+v"(mine.y), "+v"(mine.z), "+v"(mine.w));
         }
         const uint32_t cand = u24(ry) < e.prob ? col : e.alias;
-        if (cand == SKY_INVALID) break;
-        const uint32_t next = adjncy[off + cand];
+        if (cand == SKY_INVALID) break;  // a row without weight: every entry says so
+        uint32_t next = adjncy[off + cand];
         x = *reinterpret_cast<const bounds2u*>(xadj + next);
-        bool keep = s == 0 || t >= 65536u;
+        bool keep = s == 0 || t + my >= 65536u, ask = false;
+        const float need = u24(rw) * fmax;
         if (!keep) {
-          const float need = u24(rw) * fmax;
           if (next == prev) keep = need < fp;
           else if (need < lo) keep = true;
-          else if (!(need < hi)) keep = false;
-          else keep = need < (group_row_has<G>(adjncy + prev_off, prev_deg, next, x0) ? 1.0f : fq);
+          else ask = need < hi;
+        }
+        uint32_t went = 1;  // trials that this turn has decided
+        if (TR == 1) {
+          if (ask) keep = need < (group_row_has<G>(adjncy + prev_off, prev_deg, next, x0) ? 1.0f : fq);
+        } else {
+          // bit j: trial t + j is kept; bit 8 + j: that depends on the previous row
+          uint32_t b = (keep ? 1u : ask ? 256u : 0u) << my;
+          b |= dpp0<DPP_QUAD_XOR1, 0xF>(b);
+          b |= dpp0<DPP_QUAD_XOR2, 0xF>(b);
+          const uint32_t kept = b & 255u;
+          uint32_t left = kept | b >> 8 | 1u << TR;
+          went = (uint32_t)__ffs((int)left) - 1u;
+          if (went < TR && !((kept >> went) & 1u)) {
+            const int l = base + (int)went;
+            const uint32_t key = (uint32_t)__shfl((int)next, l, 64);
+            const float limit = __shfl(need, l, 64);
+            if (!(limit < (group_row_has<G>(adjncy + prev_off, prev_deg, key, x0) ? 1.0f : fq))) {  // on to the next one that may be kept
+              left &= left - 1u;
+              went = (uint32_t)__ffs((int)left) - 1u;
+              keep = went < TR && ((kept >> went) & 1u);
+            } else {
+              keep = true;
+            }
+          } else {
+            keep = went < TR;
+          }
+          if (keep) {
+            const int l = base + (int)went;
+            next = (uint32_t)__shfl((int)next, l, 64);
+            x.x = (uint32_t)__shfl((int)x.x, l, 64);
+            x.y = (uint32_t)__shfl((int)x.y, l, 64);
+          }
         }
         if (keep) {
           prev = v;
@@ -597,7 +644,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
           if (first) path[s] = v;
           if (s == len) break;
         } else {
-          ++t;
+          t += went;
         }
       }
     }
@@ -617,25 +664,39 @@ int walk_node2vec_reject(sky_graph* g, float p, float q, const uint32_t* seeds, 
   if (!g->has_tables) SKY_TRY(build_all_tables(g, &build_sec));  // first-order tables, built on demand
   const float fp = 1.0f / p, fq = 1.0f / q;
   const float fmax = fmaxf(1.0f, fmaxf(fp, fq));
+  if (fp == 1.0f && fq == 1.0f) {  // every candidate is kept: the first-order walk, whose trial 0 shares the counters
+    SKY_TRY(walk_offline(g, seeds, N, len, stop_prob, seed, paths, lengths, sampled, seconds));
+    if (seconds) *seconds += build_sec;
+    return SKY_OK;
+  }
   CallDevice* call = nullptr;
   SKY_TRY(call_begin(g, &call));
-  auto run = [&](auto lanes) {
+  auto run = [&](auto lanes, auto trials) {
     constexpr int G = decltype(lanes)::value;
     const uint64_t most = 0x80000000ull / G;  // walkers of one launch: below 2^32 threads
     for (uint64_t f = 0; f < N; f += most) {
       const uint64_t threads = std::min<uint64_t>(most, N - f) * G;
-      hipLaunchKernelGGL(walk_n2v_reject_group_kernel<G>, dim3((uint32_t)((threads + WALK_BLOCK - 1) / WALK_BLOCK)),
+      hipLaunchKernelGGL((walk_n2v_reject_group_kernel<G, decltype(trials)::value>), dim3((uint32_t)((threads + WALK_BLOCK - 1) / WALK_BLOCK)),
                          dim3(WALK_BLOCK), 0, st, g->xadj, g->adjncy, g->table, seeds, (uint32_t)f, N, g->V, len, fp, fq, fmax,
                          stop_prob, seed, walk_reads_once(g), paths, lengths, call);
     }
   };
-  const uint64_t lanes = N ? N2V_LANES / N : 0;  // per walker
-  if (lanes >= 64) run(std::integral_constant<int, 64>{});
-  else if (lanes >= 32) run(std::integral_constant<int, 32>{});
-  else if (lanes >= 16) run(std::integral_constant<int, 16>{});
-  else if (lanes >= 8) run(std::integral_constant<int, 8>{});
-  else if (lanes >= 4) run(std::integral_constant<int, 4>{});
-  else if (N) run(std::integral_constant<int, 2>{});
+  using One = std::integral_constant<int, 1>;
+  using Four = std::integral_constant<int, N2V_TRIALS>;
+  uint64_t lanes = N ? N2V_LANES / N : 0;  // per walker
+  // (1 + 1 / q) / 2 / fmax of the candidates are kept where one in two is a neighbour of the previous vertex.
+  const bool four = lanes >= 8 && (1.0f + fq) <= fmax;
+  if (fq == 1.0f) lanes = four ? std::max<uint64_t>(N2V_TRIALS, lanes / 2) : lanes >= 32 ? 4 : 2;
+  auto pick = [&](auto width) {
+    if (four) run(width, Four{});
+    else run(width, One{});
+  };
+  if (lanes >= 64) pick(std::integral_constant<int, 64>{});
+  else if (lanes >= 32) pick(std::integral_constant<int, 32>{});
+  else if (lanes >= 16) pick(std::integral_constant<int, 16>{});
+  else if (lanes >= 8) pick(std::integral_constant<int, 8>{});
+  else if (lanes >= 4) pick(std::integral_constant<int, 4>{});
+  else if (N) run(std::integral_constant<int, 2>{}, One{});
   SKY_TRY(call_end(g, sampled, seconds));
   if (seconds) *seconds += build_sec;
   return SKY_OK;

@@ -228,6 +228,25 @@ def test_node2vec_rejection_bit_exact(orc, scale, ef, stop, p, q):
     assert sampled == osampled
 
 
+@pytest.mark.parametrize("walkers", [1, 700, 10000, 15000, 40000, 60000, 240000])
+@pytest.mark.parametrize("p,q", [(0.25, 1.0), (0.5, 2.0), (0.5, 1.0), (4.0, 1.0), (1.0, 1.0), (0.0625, 8.0), (8.0, 0.0625)])
+def test_node2vec_trials_by_how_many_are_kept(orc, walkers, p, q):
+    # one trial a turn or four, with 64 lanes a walker to 2; q = 1: no trial needs the previous row; p = q = 1: the first-order walk
+    from skywalker_amd import capi
+    xadj, adjncy = orc.rmat_csr(11, 12, 35)
+    w = orc.gen_weights(orc.W_LOGNORMAL, 35, len(adjncy), 0.0, 2.0)
+    w[xadj[3]:xadj[9]] = 0.0  # rows without weight
+    prob, alias, _ = orc.alias_build(xadj, w)
+    seeds = orc.gen_seeds(6, (1 << 11) + 1, walkers)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    for stop, length in ((0.0, 7), (0.05, 12)):
+        paths, lengths, sampled, _ = g.walk_online(capi.BIAS_NODE2VEC_REJECT, p, q, seeds, length, stop, 19)
+        want = orc.walk_node2vec_reject(xadj, adjncy, prob, alias, p, q, seeds, length, stop, 19)
+        assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host((walkers, length + 1)), want[0])
+        assert sampled == want[2]
+    g.free()
+
+
 def test_read_once_gathers_give_the_same_paths(orc):
     from skywalker_amd import capi
     xadj, adjncy = orc.rmat_csr(12, 16, 36)
