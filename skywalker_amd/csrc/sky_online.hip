@@ -7,6 +7,8 @@
 //
 // node2vec: the weights of a step depend on the walker's previous vertex
 // (src/api/bias_node2vec.cu:15-27), so each (walker, step) has a table of its own, of which one entry is evaluated.
+#include <cmath>
+
 #include "sky_build_fused.h"
 #include "sky_graph.h"
 #include "sky_step_draw.h"
@@ -25,19 +27,24 @@ typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(4)));
 // The graph's own weights of a row (the weight array has 16 spare bytes, so four slots can be read from any).
 struct PlainRow {
   static constexpr int U = 4;
+  static constexpr bool HELD = true;
   const float* w;
   uint32_t d;
-  __device__ __forceinline__ void first(uint32_t k, float (&x)[4]) const {
-    x[0] = x[1] = x[2] = x[3] = 0.0f;
-    if (k < d) {
-      const float4u q = *reinterpret_cast<const float4u*>(w + k);
-      x[0] = clamp_weight(q.x);
-      x[1] = masked_weight(q.y, k + 1 < d);
-      x[2] = masked_weight(q.z, k + 2 < d);
-      x[3] = masked_weight(q.w, k + 3 < d);
-    }
+  // Without a branch, so that all loads are on their way before the first is waited for.
+  __device__ __forceinline__ void many(uint32_t k, uint32_t end, bool, float (&x)[U][4]) const {
+    float4u q[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) q[j] = *reinterpret_cast<const float4u*>(w + min(k + 256u * j, (d - 1) & ~3u));
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x[j][t] = masked_weight(q[j][t], k + 256u * j + t < end);
   }
-  __device__ __forceinline__ void again(uint32_t k, float (&x)[4]) const { first(k, x); }
+  __device__ __forceinline__ void again(uint32_t k, float (&x)[4]) const {
+    const float4u q = *reinterpret_cast<const float4u*>(w + min(k, (d - 1) & ~3u));
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[t] = masked_weight(q[t], k + t < d);
+  }
 };
 
 // A walker per workgroup of T threads, for the whole walk.  Rows of table_from entries and more have tables; from the
@@ -206,11 +213,13 @@ __device__ __forceinline__ uint32_t wave_lower_bound(const uint32_t* __restrict_
 template <uint32_t WIN>
 struct N2vRow {
   static constexpr int U = 1;
+  static constexpr bool HELD = true;
   const float* w;
   const uint32_t* nbr;
   const uint32_t* prow;
   uint32_t d, pdeg, prev;
   bool has_prev;
+  bool times;  // p and q are reciprocals, which are exact: products instead of quotients
   float p, q;
   uint32_t* win;   // [WIN], this wavefront's own
   uint8_t* codes;  // [N2V_CODES / 4]: per slot 0 neighbour of both, 1 the previous vertex, 2 neither.  Or the weights of a row
@@ -219,9 +228,8 @@ struct N2vRow {
 
   // weight of the edge in slot k after the second-order factor (src/api/bias_node2vec.cu:15-27)
   __device__ __forceinline__ float weigh(float x, uint32_t code) const {
-    if (code == 1u) x = __fdiv_rn(x, p);
-    else if (code == 2u) x = __fdiv_rn(x, q);
-    return clamp_weight(x);
+    const float by = code == 1u ? p : code == 2u ? q : 1.0f;
+    return clamp_weight(times ? x * by : __fdiv_rn(x, by));
   }
   __device__ __forceinline__ void load_window(uint32_t from) {
     const uint32_t lane = threadIdx.x & 63;
@@ -341,10 +349,10 @@ struct N2vRow {
 };
 
 template <int T, uint32_t WIN>
-__global__ __launch_bounds__(T) void walk_n2v_table_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
+__global__ __launch_bounds__(T, WIN == 512 ? 5 : 4) void walk_n2v_table_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
                                                            const float* __restrict__ wgt, const uint32_t* __restrict__ seeds,
                                                            uint32_t first, uint32_t V, uint32_t len, float p, float q,
-                                                           float stop_prob, uint64_t seed, uint32_t* __restrict__ paths,
+                                                           float stop_prob, uint64_t seed, bool times, uint32_t* __restrict__ paths,
                                                            uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
   __shared__ DrawLds<T> lds;
   __shared__ uint32_t s_win[T / 64][WIN];
@@ -367,11 +375,162 @@ __global__ __launch_bounds__(T) void walk_n2v_table_kernel(const uint32_t* __res
     row.pdeg = prev_deg;
     row.prev = prev;
     row.has_prev = s > 0;
+    row.times = times;
     row.p = p;
     row.q = q;
     row.win = s_win[threadIdx.x >> 6];
     row.codes = s_codes;
     row.wpos = row.wlen = 0;
+    const uint32_t cand = draw_slot<T>(row, d, r, lds);
+    if (cand == NONE_SLOT) break;
+    prev = v;
+    prev_off = off;
+    prev_deg = d;
+    v = row.nbr[cand];
+    if (threadIdx.x == 0) path[s + 1] = v;
+  }
+  if (threadIdx.x == 0) lengths[i] = s;
+}
+
+// The same walk on a graph of few enough vertices that a bit for each fits beside the walkers of a CU in LDS: the bits of the
+// previous row's vertices are set once a step, and a slot then tests one bit, where the search of the window is ten dependent
+// reads; with no state from slot to slot the loads of U times 256 slots are in flight at once.
+// Four walkers of four wavefronts to a CU, or two of eight while these hold all of them that walk (700 walkers x 20 on the scale-17 graph
+// 242 us with four wavefronts, 201 with eight; 2,000 x 40 there 452 and 667): twice as many bits would leave two walkers to a CU.
+// Against the windows: 2,000 x 40 with p = 2, q = 1/2 on the scale-18 graph 736 -> 550 us, on the scale-17 graph 617 -> 456, 1,500 x 30
+// with 40 edges a vertex, scale 13, 482 -> 320, 200 x 40 with 30, scale 16, 526 -> 358.
+constexpr uint32_t MAP_VERTICES = 1u << 18;  // 32 KB
+constexpr uint32_t MAP_ROW = 32768;          // longer previous rows of N2V_SPARSE times the current one are searched in memory
+constexpr uint32_t MAP_KEEP = 4096;          // slots of a row whose weights are kept, or what room there is
+constexpr uint32_t MAP_FEW = 768;
+struct N2vMapRow {
+  static constexpr int U = 2;
+  static constexpr bool HELD = true;
+  const float* w;
+  const uint32_t* nbr;
+  const uint32_t* prow;
+  const uint32_t* map;  // bit t: vertex t is a neighbour of prev
+  float* kept;          // weights of the row's slots, if it has at most `keep`
+  uint32_t d, pdeg, prev, keep;
+  bool has_prev, search;
+  bool times;  // p and q are reciprocals, which are exact: products instead of quotients
+  float p, q;
+
+  // weight of the edge to t after the second-order factor (src/api/bias_node2vec.cu:15-27)
+  __device__ __forceinline__ float weigh(float x, uint32_t t, bool in) const {
+    if (has_prev) {
+      const bool both = search ? in && row_contains(prow, pdeg, t) : (map[t >> 5] >> (t & 31)) & 1u;
+      const float by = t == prev ? p : both ? 1.0f : q;
+      x = times ? x * by : __fdiv_rn(x, by);
+    }
+    return masked_weight(x, in);
+  }
+  __device__ __forceinline__ void many(uint32_t k, uint32_t end, bool again, float (&x)[U][4]) const {
+    if (again && d <= keep) {
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const uint32_t at = min(k + 256u * j, (d - 1) & ~3u);
+        const float4 c = reinterpret_cast<const float4*>(kept)[at >> 2];
+        const float y[4] = {c.x, c.y, c.z, c.w};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) x[j][t] = k + 256u * j + t < end ? y[t] : 0.0f;
+      }
+      return;
+    }
+    float4u a[U];
+    uint4u b[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const uint32_t at = min(k + 256u * j, (d - 1) & ~3u);
+      a[j] = *reinterpret_cast<const float4u*>(w + at);
+      b[j] = *reinterpret_cast<const uint4u*>(nbr + at);
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      const uint32_t at = k + 256u * j;
+      x[j][0] = x[j][1] = x[j][2] = x[j][3] = 0.0f;
+      if (at - 4 * (threadIdx.x & 63) >= end) continue;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const bool in = at + t < end;
+        x[j][t] = weigh(a[j][t], in ? b[j][t] : 0u, in);  // past the row's end lies another's vertex, or none
+      }
+      if (!again && d <= keep && at < end) reinterpret_cast<float4*>(kept)[at >> 2] = make_float4(x[j][0], x[j][1], x[j][2], x[j][3]);
+    }
+  }
+  __device__ __forceinline__ void again(uint32_t k, float (&x)[4]) const {
+    x[0] = x[1] = x[2] = x[3] = 0.0f;
+    if (k >= d) return;
+    if (d <= keep) {
+      const float4 c = reinterpret_cast<const float4*>(kept)[k >> 2];
+      x[0] = c.x; x[1] = c.y; x[2] = c.z; x[3] = c.w;
+      return;
+    }
+    const float4u a = *reinterpret_cast<const float4u*>(w + k);
+    const uint4u b = *reinterpret_cast<const uint4u*>(nbr + k);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[t] = weigh(a[t], k + t < d ? b[t] : 0u, k + t < d);
+  }
+};
+
+template <int T>
+__global__ __launch_bounds__(T) void walk_n2v_map_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
+                                                         const float* __restrict__ wgt, const uint32_t* __restrict__ seeds,
+                                                         uint32_t first, uint32_t V, uint32_t len, float p, float q,
+                                                         float stop_prob, uint64_t seed, bool times, uint32_t map_words, uint32_t keep,
+                                                         uint32_t* __restrict__ paths, uint32_t* __restrict__ lengths,
+                                                         CallDevice* __restrict__ call) {
+  __shared__ DrawLds<T> lds;
+  extern __shared__ __align__(16) uint32_t s_map[];  // [map_words], a multiple of 4, then the kept weights
+  call_stamp(call);
+  const uint32_t i = first + blockIdx.x;
+  uint32_t* const path = paths + (size_t)i * (len + 1);
+  uint32_t v = seeds[i], s = 0, prev = 0, prev_off = 0, prev_deg = 0;
+  if (threadIdx.x == 0) path[0] = v;
+  for (; s < len && v < V; ++s) {
+    const u32x4 r = philox(seed, i, s, 0, DOM_WALK);
+    if (stop_prob > 0.0f && u24(r.z) < stop_prob) break;
+    const uint32_t off = xadj[v], end = xadj[v + 1];
+    auto mark = [&] {  // the previous row, while the bounds of this one are on their way
+      constexpr int M = 2;
+      const uint32_t* const prow = adjncy + prev_off;
+      for (uint64_t from = 0; from < prev_deg; from += 4 * T * M) {
+        const uint32_t k = (uint32_t)from + 4 * threadIdx.x;
+        uint4u x[M];
+#pragma unroll
+        for (int j = 0; j < M; ++j) x[j] = *reinterpret_cast<const uint4u*>(prow + min(k + 4 * T * j, (prev_deg - 1) & ~3u));
+        if (from == 0) {
+          __syncthreads();  // the draw before may still be reading bits
+          for (uint32_t c = threadIdx.x; c < map_words / 4; c += T) reinterpret_cast<uint4*>(s_map)[c] = make_uint4(0, 0, 0, 0);
+          __syncthreads();
+        }
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+#pragma unroll
+          for (int t = 0; t < 4; ++t)
+            if (k + 4 * T * j + t < prev_deg) atomicOr(&s_map[x[j][t] >> 5], 1u << (x[j][t] & 31));
+      }
+    };  // the draw starts with a barrier
+    if (s > 0 && prev_deg <= MAP_ROW) mark();
+    const uint32_t d = end - off;
+    if (d == 0) break;
+    const bool search = prev_deg > MAP_ROW && prev_deg / N2V_SPARSE > d;
+    if (prev_deg > MAP_ROW && !search) mark();
+    N2vMapRow row;
+    row.w = wgt + off;
+    row.nbr = adjncy + off;
+    row.prow = adjncy + prev_off;
+    row.map = s_map;
+    row.kept = reinterpret_cast<float*>(s_map + map_words);
+    row.d = d;
+    row.pdeg = prev_deg;
+    row.prev = prev;
+    row.keep = keep;
+    row.has_prev = s > 0;
+    row.search = search;
+    row.times = times;
+    row.p = p;
+    row.q = q;
     const uint32_t cand = draw_slot<T>(row, d, r, lds);
     if (cand == NONE_SLOT) break;
     prev = v;
@@ -394,14 +553,30 @@ int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, 
   // wait for a CU (2,000 walkers x 40 steps on the scale-18 graph 901 -> 761 us; 900 walkers on the scale-17 graph 538
   // with 1024 ids, 555 with 512).  Less LDS still, by fewer slots whose result is kept or smaller windows, was slower.
   constexpr uint32_t FEW = 512, RESIDENT = 1024;
+  // A power of two divides as its reciprocal multiplies, to the last bit: 12 instructions an entry fewer.
+  auto power = [](float x) {
+    int e;
+    return std::frexp(x, &e) == 0.5f && std::abs(e) < 100;
+  };
+  const bool times = power(p) && power(q);
+  const float by_p = times ? 1.0f / p : p, by_q = times ? 1.0f / q : q;
   const uint32_t most = 0xFFFFFFFFu / 512;  // walkers of one launch: below 2^32 threads
   for (uint32_t f = 0; f < N; f += std::min(most, N - f)) {
     const dim3 grid(std::min(most, N - f));
     auto go = [&](auto kernel, uint32_t threads) {
-      hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, st, g->xadj, g->adjncy, g->adjwgt, seeds, f, g->V, len, p, q, stop_prob,
-                         seed, paths, lengths, call);
+      hipLaunchKernelGGL(kernel, grid, dim3(threads), 0, st, g->xadj, g->adjncy, g->adjwgt, seeds, f, g->V, len, by_p, by_q, stop_prob,
+                         seed, times, paths, lengths, call);
     };
-    if (N <= FEW) go(walk_n2v_table_kernel<512, 1024>, 512);
+    if (g->V <= MAP_VERTICES) {
+      const uint32_t words = (g->V + 127u) / 128u * 4u;
+      auto map = [&](auto kernel, uint32_t threads, uint32_t walkers, size_t fixed) {  // walkers of a CU
+        const uint32_t keep = std::min(MAP_KEEP, ((160u << 10) / walkers - (uint32_t)fixed - 4u * words) / 16u * 4u);
+        hipLaunchKernelGGL(kernel, grid, dim3(threads), 4u * (words + keep), st, g->xadj, g->adjncy, g->adjwgt, seeds, f, g->V, len,
+                           by_p, by_q, stop_prob, seed, times, words, keep, paths, lengths, call);
+      };
+      if (N <= MAP_FEW) map(walk_n2v_map_kernel<512>, 512, 2, sizeof(DrawLds<512>));
+      else map(walk_n2v_map_kernel<256>, 256, 4, sizeof(DrawLds<256>));
+    } else if (N <= FEW) go(walk_n2v_table_kernel<512, 1024>, 512);
     else if (N <= RESIDENT) go(walk_n2v_table_kernel<256, 1024>, 256);
     else go(walk_n2v_table_kernel<256, 512>, 256);
     call = nullptr;

@@ -2,6 +2,9 @@
 // the threads of a workgroup evaluate that entry alone, from the same prefix-sum definition the offline build uses:
 //   pass 1  exact sum of the row's weights -> ledger, class of entry col
 //           (a light col whose own share accepts the draw needs nothing more)
+// in rows of up to 16 slots a thread
+//   scan    of deficits and surpluses over the workgroup, whose prefixes each thread has for its own slots (draw_held)
+// and in longer ones
 //   pass 2  deficits and surpluses of every chunk of the row; their prefixes over the chunks
 //   then    the one chunk that holds col gives the prefix up to col, and the one chunk in which the other kind's
 //           prefix crosses it gives the slot (and the chunk with the next or last heavy that heavy)
@@ -27,6 +30,8 @@ struct DrawLds {
   double fsum[T / 64];
   u128 sum[T / 64];
   uint32_t mn[T / 64];
+  uint64_t key;
+  uint32_t heavy[T / 64];
   uint32_t result;
 };
 
@@ -46,11 +51,23 @@ __device__ __forceinline__ bool row_contains(const uint32_t* __restrict__ row, u
   return false;
 }
 
+// Weights of the U times 256 slots from `base` on, four consecutive ones of each 256 per lane, zeros from `end` on.
+template <int U, class Row>
+__device__ __forceinline__ void row_weights(Row& row, uint32_t base, uint32_t end, bool again, float (&w)[U][4]) {
+  const uint32_t k = base + 4 * (threadIdx.x & 63);
+  if constexpr (U > 1) {
+    row.many(k, end, again, w);
+  } else {
+    if (again) row.again(k, w[0]);
+    else row.first(k, w[0]);
+  }
+}
+
 // Rest of the draw below: column `col` of class `ec` with the acceptance number u.  SAT: the row's surpluses may wrap.
 template <bool SAT, int T, class Row>
 __device__ __forceinline__ uint32_t draw_entry(Row& row, const uint32_t d, const Ledger& L, const uint32_t col, const Entry& ec,
-                                               const float u, const uint32_t csz, const uint32_t nc, const uint32_t c0,
-                                               const uint32_t c1, DrawLds<T>& lds) {
+                                               const float u, const uint32_t csz, const uint32_t nc, const uint32_t k0,
+                                               const uint32_t k1, DrawLds<T>& lds) {
   constexpr int NW = T / 64;
   uint32_t tid = threadIdx.x;
   asm volatile("" : "+v"(tid));  // what depends on the lane number stays inside this form's code
@@ -69,20 +86,33 @@ __device__ __forceinline__ uint32_t draw_entry(Row& row, const uint32_t d, const
   };
 
   // pass 2: totals of the chunks
-  for (uint32_t c = c0; c < c1; ++c) {
+  {
+    constexpr int U = Row::U;
     uint64_t sd = 0, su = 0;
-    const uint32_t end = c + 1 == nc ? d : (c + 1) * csz;
-    for (uint32_t base = c * csz; base < end; base += DRAW_CHUNK) {
-      uint64_t dd[4], uu[4];
-      amounts(base, dd, uu);
-      sd += (dd[0] + dd[1]) + (dd[2] + dd[3]);
-      su = add_sat<SAT>(su, add_sat<SAT>(add_sat<SAT>(uu[0], uu[1]), add_sat<SAT>(uu[2], uu[3])));
-    }
-    sd = group_scan_u64<64>(sd);
-    su = group_scan_sat_u64<64, SAT>(su);
-    if (lane == 63) {
-      lds.d[c] = sd;
-      lds.u[c] = su;
+    for (uint32_t base = k0; base < k1; base += DRAW_CHUNK * U) {
+      float w[U][4];
+      row_weights<U>(row, base, k1, true, w);
+#pragma unroll
+      for (int j = 0; j < U; ++j) {
+        const uint32_t at = base + DRAW_CHUNK * j;
+        if (at >= k1) continue;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const bool in = at + 4 * lane + k < d;
+          const Entry e = classify_fast((double)w[j][k], in, L);
+          sd += in && !e.heavy ? e.amount : 0;
+          su = add_sat<SAT>(su, e.heavy ? e.amount : 0);
+        }
+        if (((at + DRAW_CHUNK) & (csz - 1)) && at + DRAW_CHUNK < k1) continue;  // the chunk goes on
+        sd = group_scan_u64<64>(sd);
+        su = group_scan_sat_u64<64, SAT>(su);
+        if (lane == 63) {
+          const uint32_t c = at / csz;
+          lds.d[c] = sd;
+          lds.u[c] = su;
+        }
+        sd = su = 0;
+      }
     }
   }
   __syncthreads();
@@ -223,9 +253,122 @@ __device__ __forceinline__ uint32_t draw_entry(Row& row, const uint32_t d, const
     if (lane == 0) lds.result = cand;
   }
   __syncthreads();
-  const uint32_t cand = lds.result;
-  __syncthreads();  // the next draw rewrites what the others still read
-  return cand;
+  return lds.result;  // the next draw starts with a barrier
+}
+
+// The same for a row of at most 4 Q T slots, Q quads of consecutive ones a thread: one scan over the workgroup gives every prefix,
+// the thread of col the key, and the thread whose prefixes it falls between the slot.  Three barriers and some 3,000 cycles, where the
+// sweep over chunks and the chain on one wavefront behind it take 9,000 (counted in the table-per-step walk, rows of 800 entries on
+// average).  The amounts of four quads held in registers would make them 147, three wavefronts to a SIMD: they are computed again.
+template <bool SAT, int Q, int T, class Row>
+__device__ __forceinline__ uint32_t draw_held(Row& row, const uint32_t d, const Ledger& L, const uint32_t col, const Entry& ec,
+                                              const float u, DrawLds<T>& lds) {
+  constexpr int NW = T / 64, S = 4 * Q;
+  uint32_t tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));  // what depends on the lane number stays inside this form's code
+  const uint32_t wave = tid >> 6, lane = tid & 63, k0 = S * tid, owner = col / S, own = col % S;
+  // f(slot within the thread's, heavy, amount)
+  uint64_t a[4];
+  uint32_t ah = 0;
+  auto each = [&](bool again, auto&& f) {
+#pragma unroll 1
+    for (int q = 0; q < Q; ++q) {
+      if (Q > 1 || !again) {
+        float w[4];
+        row.again(k0 + 4 * q, w);
+        ah = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const Entry e = classify_fast((double)w[k], k0 + 4 * q + k < d, L);
+          a[k] = e.amount;
+          ah |= (e.heavy ? 1u : 0u) << k;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) f(4 * q + k, (ah >> k) & 1, a[k]);
+    }
+  };
+  uint64_t sd = 0, su = 0;
+  uint32_t heavy = 0;  // bit k: slot k0 + k
+  each(false, [&](int k, bool h, uint64_t x) {
+    heavy |= (h ? 1u : 0u) << k;
+    sd += h ? 0 : x;
+    su = add_sat<SAT>(su, h ? x : 0);
+  });
+  const uint64_t id = group_scan_u64<64>(sd), iu = group_scan_sat_u64<64, SAT>(su);
+  uint64_t bd = id - sd, bu = before_own<SAT>(iu, su);  // before the thread's slots
+  uint64_t tu = 0;                                      // surpluses of the row
+  if (lane == 63) {
+    lds.d[wave] = id;
+    lds.u[wave] = iu;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NW; ++i) {
+    const uint64_t x = lds.d[i], y = lds.u[i];
+    tu = add_sat<SAT>(tu, y);
+    if (i < (int)wave) {
+      bd += x;
+      bu = add_sat<SAT>(bu, y);
+    }
+  }
+  if (tid == owner) {  // deficits before a light col, surpluses up to and with a heavy col
+    uint64_t key = ec.heavy ? bu : bd;
+    each(true, [&](int k, bool h, uint64_t x) {
+      key = add_sat<SAT>(key, ec.heavy ? (h && k <= (int)own ? x : 0) : (!h && k < (int)own ? x : 0));
+    });
+    lds.key = key;
+    lds.result = col;
+  }
+  // first (last) heavy slot of each wavefront among those in `mask`
+  auto heavies = [&](uint32_t mask, bool last) {
+    const unsigned long long m = __ballot(mask != 0);
+    const int l = last ? 63 - __clzll((long long)(m | 1)) : __ffsll((long long)(m | 1ull << 63)) - 1;
+    const uint32_t slot = (uint32_t)__shfl((int)(k0 + (last ? 31 - __clz((int)(mask | 1)) : __ffs((int)(mask | 1u << 31)) - 1)), l, 64);
+    if (lane == 0) lds.heavy[wave] = m ? slot : NONE_SLOT;
+  };
+  if (ec.heavy) heavies(tid < owner ? 0u : tid == owner ? heavy & ~((2u << own) - 1u) : heavy, false);
+  __syncthreads();
+  const uint64_t key = lds.key;
+  if (!ec.heavy) {
+    // first heavy whose surplus prefix exceeds the key; the last heavy if there is none; col itself without any heavy
+    if (key < tu) {
+      if (bu <= key && key < add_sat<SAT>(bu, su)) {
+        uint32_t at = S;
+        each(true, [&](int k, bool h, uint64_t x) {
+          if (h) bu = add_sat<SAT>(bu, x);
+          at = at == S && bu > key ? k : at;
+        });
+        lds.result = min(k0 + at, d - 1);  // a bias operator may answer differently each time
+      }
+    } else if (tu) {
+      heavies(heavy, true);
+      __syncthreads();
+      if (tid == 0) {
+        uint32_t slot = NONE_SLOT;
+#pragma unroll
+        for (int i = 0; i < NW; ++i)
+          if (lds.heavy[i] != NONE_SLOT) slot = lds.heavy[i];
+        lds.result = slot;
+      }
+    }
+  } else {
+    // next heavy after col (none: col is the last heavy and keeps the draw), then the first light l with
+    // SL(l) >= y: prob = (one + y - SL(l)) / one
+    uint32_t nxt = NONE_SLOT;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) nxt = min(nxt, lds.heavy[i]);
+    if (nxt != NONE_SLOT && bd < key && key <= bd + sd) {
+      uint64_t sl = 0;
+      each(true, [&](int k, bool h, uint64_t x) {
+        if (!h) bd += x;
+        sl = sl == 0 && bd >= key ? bd : sl;  // the key of a heavy is at least 1
+      });
+      lds.result = u < residual_prob(L.one + key - sl, L) ? col : nxt;
+    }
+  }
+  __syncthreads();
+  return lds.result;
 }
 
 // Row-local slot that (walker, step) with random numbers r draws from the row of d >= 1 entries, or NONE_SLOT when
@@ -233,7 +376,9 @@ __device__ __forceinline__ uint32_t draw_entry(Row& row, const uint32_t d, const
 //   row.first(k, w)   clamped weights of slots k .. k + 3 (k a multiple of 4; zeros past the row).  A wavefront goes
 //                     through its part of the row in slot order, once, all lanes together (k advances by 4 per lane)
 //   row.again(k, w)   the same, afterwards, for any slots and by any wavefront
-//   Row::U            how many chunks' worth of first() may be in flight at once
+//   Row::U            how many times 256 slots are in flight at once; if that is more than one, instead of first():
+//   Row::HELD         rows of up to 16 slots a thread by draw_held
+//   row.many(k, end, again, w)  slots k + 256 j .. k + 256 j + 3 for j < U, zeros from slot `end` on, in both sweeps
 template <int T, class Row>
 __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const u32x4& r, DrawLds<T>& lds) {
   constexpr int NW = T / 64, U = Row::U;
@@ -250,18 +395,15 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
   uint32_t mn = 0xFFFFFFFFu;
   for (uint32_t base = k0; base < k1; base += DRAW_CHUNK * U) {
     float w[U][4];
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      w[j][0] = w[j][1] = w[j][2] = w[j][3] = 0.0f;
-      if (base + DRAW_CHUNK * j < k1) row.first(base + DRAW_CHUNK * j + 4 * lane, w[j]);
-    }
+    row_weights<U>(row, base, k1, false, w);
 #pragma unroll
     for (int j = 0; j < U; ++j)
+      if (base + DRAW_CHUNK * j < k1)
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        fsum += (double)w[j][k];
-        mn = min(mn, __float_as_uint(w[j][k]) - 1u);
-      }
+        for (int k = 0; k < 4; ++k) {
+          fsum += (double)w[j][k];
+          mn = min(mn, __float_as_uint(w[j][k]) - 1u);
+        }
   }
   fsum = group_sum_f64<64>(fsum);
   mn = wave_min_u32(mn);
@@ -321,8 +463,18 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
   }
   if (!ec.heavy && u < (float)ec.p) return col;  // the light keeps the draw: its alias is never read
 
-  return surpluses_may_wrap(L.scale) ? draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, c0, c1, lds)
-                                     : draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, c0, c1, lds);
+  if constexpr (!Row::HELD) {
+    return surpluses_may_wrap(L.scale) ? draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds)
+                                       : draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
+  }
+  if (surpluses_may_wrap(L.scale)) {
+    if (d <= 4 * T) return draw_held<true, 1, T>(row, d, L, col, ec, u, lds);
+    if (d <= 16 * T) return draw_held<true, 4, T>(row, d, L, col, ec, u, lds);
+    return draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
+  }
+  if (d <= 4 * T) return draw_held<false, 1, T>(row, d, L, col, ec, u, lds);
+  if (d <= 16 * T) return draw_held<false, 4, T>(row, d, L, col, ec, u, lds);
+  return draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
 }
 
 // A row whose weights are computed by a function of the slot (row(k): clamped weight of slot k < d): those of a row of up
@@ -331,6 +483,7 @@ constexpr uint32_t FN_CACHE = 4096;
 template <class Fn>
 struct FunctionRow {
   static constexpr int U = 1;
+  static constexpr bool HELD = false;  // the operator is called where it is linked in: node2vec's, 8,000 walkers x 20, scale 16, 5.5 ms, 6.0 with
   Fn fn;
   uint32_t d;
   float* cache;  // [FN_CACHE]

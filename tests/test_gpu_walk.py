@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from helpers import chi_square_p, graph_from_degrees
+from helpers import chi_square_p, graph_from_degrees, weights
 
 pytestmark = pytest.mark.gpu
 
@@ -467,3 +467,33 @@ def test_node2vec_table_rows_beyond_the_window(orc, walkers):
     assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host((walkers, 8)), want[0])
     assert sampled == want[2]
     g.free()
+
+
+@pytest.mark.parametrize("V", [1200, (1 << 18) - 1, 1 << 18, (1 << 18) + 1])
+@pytest.mark.parametrize("walkers,p,q", [(768, 2.0, 0.5), (769, 3.0, 0.7), (2000, 0.25, 4.0)])
+def test_node2vec_table_with_a_bit_per_vertex(orc, V, walkers, p, q):
+    # eight and four wavefronts per walker, the largest graph whose vertices have bits and the first without; quotients by powers of two
+    # and by others; rows around the 4 and 16 slots a thread of the draw and around the weights kept; previous rows of more than
+    # 32,768 entries before short ones (searched in memory) and long ones; surpluses beyond 64 bits
+    from skywalker_amd import capi
+    rng = np.random.default_rng(47)
+    degs = [1, 2, 3, 4, 5, 987, 988, 989, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097, 8191, 8192, 8193] * 4 + \
+        [32767, 32768, 32769, 40000, 66001] + list(rng.integers(1, 900, 500))
+    n = len(degs)
+    ids = np.sort(np.append(rng.choice(np.arange(1, V - 1), n - 2, replace=False), [0, V - 1]))  # the vertices with rows
+    rng.shuffle(degs)
+    lens = np.zeros(V, np.int64)
+    lens[ids] = degs
+    xadj = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    adjncy = np.concatenate([np.sort(rng.choice(ids, k)) for k in degs]).astype(np.uint32)
+    w = weights(len(adjncy), rng, "sparse")
+    for v in ids[::3]:
+        w[xadj[v]:xadj[v + 1]] *= np.float32(1e-19)
+    seeds = np.append(rng.choice(ids, walkers - 2), [V - 1, 0]).astype(np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    paths, lengths, sampled, _ = g.walk_online(capi.BIAS_NODE2VEC, p, q, seeds, 8, 0.02, 37)
+    got = paths.to_host((walkers, 9)), lengths.to_host()
+    g.free()
+    want = orc.walk_online(xadj, adjncy, w, 1, p, q, seeds, 8, 0.02, 37)
+    assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
+    assert sampled == want[2]
