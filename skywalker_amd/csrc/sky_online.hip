@@ -7,6 +7,7 @@
 //
 // node2vec: the weights of a step depend on the walker's previous vertex
 // (src/api/bias_node2vec.cu:15-27), so each (walker, step) has a table of its own, of which one entry is evaluated.
+#include <algorithm>
 #include <cmath>
 
 #include "sky_build_fused.h"
@@ -27,14 +28,18 @@ typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(4)));
 // The graph's own weights of a row (the weight array has 16 spare bytes, so four slots can be read from any).
 struct PlainRow {
   static constexpr int U = 4;
-  static constexpr bool HELD = true;
+  static constexpr int HELD = 4;
   const float* w;
   uint32_t d;
-  // Without a branch, so that all loads are on their way before the first is waited for.
+  // Branches that a wavefront takes as one: all loads are on their way before the first is waited for.
   __device__ __forceinline__ void many(uint32_t k, uint32_t end, bool, float (&x)[U][4]) const {
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
     float4u q[U];
 #pragma unroll
-    for (int j = 0; j < U; ++j) q[j] = *reinterpret_cast<const float4u*>(w + min(k + 256u * j, (d - 1) & ~3u));
+    for (int j = 0; j < U; ++j) {
+      q[j] = float4u{0, 0, 0, 0};
+      if (first + 256u * j < end) q[j] = *reinterpret_cast<const float4u*>(w + min(k + 256u * j, (d - 1) & ~3u));
+    }
 #pragma unroll
     for (int j = 0; j < U; ++j)
 #pragma unroll
@@ -84,54 +89,74 @@ __global__ __launch_bounds__(T) void walk_direct_kernel(const uint32_t* __restri
   if (threadIdx.x == 0) lengths[i] = s;
 }
 
-// How to serve a static-bias walk on a graph without tables.  Every row drawn from costs either its table (about
-// BUILD_PS a entry, once) or two sweeps over its weights (about DRAW_PS a entry, each time).  A step leads to a row
-// with a probability that grows with its length, so a row of d entries is drawn from about N * len * d / E times, and
-// its table pays from the length on at which N * len * d / E * DRAW_PS exceeds BUILD_PS.  Measured on one MI355X.  The launches of
-// a build cost BUILD_US whatever they build, so it has to save as much: without this rule 531 walkers x 6 steps on the scale-16
-// graph took 75 us, with it 54, 110 x 9 on the scale-20 graph with 32 edges a vertex 161 and 114, 400 x 8 on the scale-22 graph
-// 180 and 134.  A step waits for the sweep of its row, so what is saved counts CHAIN times what its bandwidth comes to: counted
-// once, 1,873 x 11 steps on the scale-22 graph with 7 edges a vertex go without tables, 176 us for 138.  From 2 on that is right;
-// 4 is right on the scale-17 graph with 43 as well, 98 us for 92 the other way.
-// The same ratio for a few thousand walkers and for many: tables from half that length on for the former made 3,000 x 16 steps on
-// the scale-23 graph 390 us, now 334, and 2,000 x 10 on the scale-24 graph 305, now 259.
-constexpr double BUILD_PS = 8.0, DRAW_PS = 2.5, CHAIN = 4.0;
-constexpr uint32_t FEW_WALKERS = 4096;
-constexpr double BUILD_US = 40.0, STEP_US = 4.0;  // launches of a build; the chain of loads and scans of a step
+// Threads of a walker: the walk ends with the walker that meets the longest rows without a table, so the longer these may be the more
+// threads, and the more walkers the fewer, down to what fills the GPU.  (64 / 128 / 256 / 512 / 1024 threads, us.  Longest row of
+// 300,000: 207 walkers x 3 233 / 137 / 86 / 69 / 69; 5,000 x 2 1137 / 604 / 328 / 226; 7,000 x 2 1410 / 774 / 413 / 303 / 307.  Of 50,000
+// to 65,000: 352 x 8 269 / 158 / 102 / 84 / 89; 8,500 x 1 91 / 61 / 46 / 66; 20,000 x 2 233 / 190 / 195 / 288.  Of 25,000: 1,000 x 6
+// 155 / 135 / 122 / 133 / 180; 3,000 x 10 471 / 348 / 274 / 333.  Of 5,000 to 8,000: 100 x 10 80 / 65 / 57 / 59 / 73; 1,000 x 12 135 / 119 / 119 / 142;
+// 3,800 x 8 172 / 156 / 168 / 211; 7,000 x 10 237 / 221 / 252 / 371.)
+static uint32_t walker_threads(uint32_t N, uint32_t longest) {
+  if (longest > 65533) return N <= 256 ? 1024 : N <= 8192 ? 512 : 256;
+  if (longest > 16384) return N <= 512 ? 512 : N <= 16384 ? 256 : 128;
+  return N <= 1024 ? 256 : N <= 8192 ? 128 : 64;
+}
+
+// How to serve a static-bias walk on a graph without tables.  Every row drawn from costs either its table (BUILD_PS an entry, once, and
+// BUILD_US the launches of a build) or two sweeps over its weights (DRAW_PS an entry, each time).  A start vertex is any vertex; a
+// later step leads to a row with a probability that grows with its length, so a row of d entries is drawn from N * (len - 1) * d / E
+// times, and its table pays from some length on.  But a walk also lasts as long as the walker that meets the longest row without
+// a table, ROW_NS an entry with 512 threads, inversely more with fewer and down to ROW_LEAST_NS with more.  What every choice would
+// take is added up, from no tables over those of the longest class alone to those of every class from 33 entries on, and the least is taken.
+// The figures were fitted to 36 walks on graphs of 1 M to 260 M entries with ten choices each: what is taken is 2 % slower than the best
+// of the ten in the mean, 25 % at most.  (Tables where N * len * d / E * 2.5 ps exceeds 8 ps, as before, and now, us: 5,000 walkers x 2 on the
+// scale-24 graph 1301 / 169, 4,000 x 2 on the scale-22 graph with 40 edges a vertex 640 / 186, 500 x 8 with 30 288 / 192, 8,500 x 1 on the
+// scale-23 graph 180 / 46, 20,000 x 12 there 415 / 375.)
+constexpr double BUILD_PS = 7.5, DRAW_PS = 2.4, BUILD_US = 31.0, ROW_NS = 0.39, ROW_LEAST_NS = 0.25, STEP_US = 2.4;
 
 struct OnlinePlan {
   bool full;            // every row, then the offline walk
   uint32_t table_from;  // else: the rows of at least so many entries
 };
-static int online_plan(sky_graph* g, uint32_t N, uint32_t len, OnlinePlan* o, CallDevice** first) {
+static int online_plan(sky_graph* g, uint32_t N, uint32_t len, float stop_prob, OnlinePlan* o, CallDevice** first) {
   const long long mode = option(g, OPT_ONLINE_FULL_BUILD);
   *o = OnlinePlan{mode > 0, 0xFFFFFFFFu};
   if (mode > 0) return SKY_OK;
   SKY_TRY(ensure_plan(g, first));
-  const double E = std::max(1u, g->E), draws = (double)N * len;
-  const double from = BUILD_PS / DRAW_PS * E / std::max(1.0, draws);
-  // the shortest class whose rows are all that long; the classes below G16 (33 entries) are not built apart from the rest
-  double built = 0, direct = 0, tabled = 0;  // entries of tables, entries that draws from other rows read, and from these without tables
-  for (int c = CLS_TINY; c < CLS_COUNT; ++c) {
-    const double entries = (double)g->bin_edges[c], lo = class_min_degree(c);
-    if (entries == 0) continue;
-    const double read = draws * entries / E * (c == CLS_TINY ? 1.5 : entries / std::max(1u, g->bin_counts[c]));
-    if (c >= CLS_G16 && lo >= from) {
-      built += entries;
-      tabled += read;
-      o->table_from = std::min(o->table_from, class_min_degree(c));
-    } else {
-      direct += read;
+  const double E = std::max(1u, g->E), V = std::max(1u, g->V), go = 1.0 - std::min(1.0f, std::max(0.0f, stop_prob)), starts = N * go;
+  const double edges = N * (go < 1.0 ? go * go * (1.0 - std::pow(go, len - 1.0)) / (1.0 - go) : len - 1.0);  // steps along an edge
+  struct Rows {
+    uint32_t from;
+    double entries, read, chain;  // of all rows; of those drawn from, with repeats; of the one walker's that meets the most
+  } rows[CLS_COUNT + 1];
+  int n = 0;
+  for (int c = CLS_G2; c < CLS_COUNT; ++c) {
+    const double entries = (double)g->bin_edges[c], count = g->bin_counts[c];
+    if (entries == 0 || count == 0) continue;
+    const double mean = entries / count, times = edges * entries / E + starts * count / V;
+    const double most = std::min(1.5 * mean, (double)g->max_degree);
+    rows[n++] = Rows{class_min_degree(c), entries, times * mean, most * (std::min(1.0, times) + times / std::max(1u, N))};
+  }
+  std::sort(rows, rows + n, [](const Rows& a, const Rows& b) { return a.from < b.from; });
+  const double to_max = edges * g->max_degree / E;
+  double best = 1e30, built = 0;
+  for (int k = n; k >= 0; --k) {  // tables of rows[k] .. rows[n - 1]
+    if (k < n) built += rows[k].entries;
+    if (k < n && rows[k].from < 33) break;  // the shorter classes are not built apart from the rest
+    const uint32_t from = k < n ? rows[k].from : 0xFFFFFFFFu;
+    double read = 0, chain = k < n ? 0.0 : g->max_degree * (std::min(1.0, to_max) + to_max / std::max(1u, N));
+    for (int i = 0; i < k; ++i) {
+      read += rows[i].read;
+      chain = std::max(chain, rows[i].chain);
+    }
+    const double row_ns = std::max(ROW_LEAST_NS, ROW_NS * 512 / walker_threads(N, std::min(from - 1, g->max_degree)));
+    const double us = (k < n ? BUILD_US + built * BUILD_PS * 1e-6 : 0.0) + read * DRAW_PS * 1e-6 + chain * row_ns * 1e-3 + STEP_US * len;
+    if (us < best) {
+      best = us;
+      o->table_from = from;
     }
   }
-  if (built && CHAIN * tabled * DRAW_PS * 1e-6 < BUILD_US + built * BUILD_PS * 1e-6) {  // not worth the launches
-    o->table_from = 0xFFFFFFFFu;
-    direct += tabled;
-    built = 0;
-  }
-  const double hybrid_us = (built ? BUILD_US : 0.0) + (built * BUILD_PS + direct * DRAW_PS) * 1e-6 + STEP_US * len;
   const double full_us = BUILD_US + E * BUILD_PS * 1e-6 + 1.2 * len;
-  o->full = mode < 0 && full_us < hybrid_us;
+  o->full = mode < 0 && full_us < best;
   return SKY_OK;
 }
 
@@ -149,7 +174,7 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
   CallDevice* call = nullptr;
   if (!g->has_tables) {
     SKY_TRY(call_begin(g, &call));
-    if (N && len) SKY_TRY(online_plan(g, N, len, &how, &call));
+    if (N && len) SKY_TRY(online_plan(g, N, len, stop_prob, &how, &call));
     if (how.full) {  // the build is a call of its own, and so is the plan if it was made just now
       if (call) call_cancel(g);
       else SKY_TRY(call_end(g, nullptr, &plan_sec));
@@ -167,8 +192,7 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
     call = nullptr;  // the build's first kernel is the call's, or the plan's was
   }
   if (N) {
-    // the fewer walkers, the larger the workgroup that takes one through a long row
-    const uint32_t T = N <= 256 ? 1024 : N <= FEW_WALKERS ? 256 : 64;
+    const uint32_t T = walker_threads(N, std::min(how.table_from - 1, g->max_degree));
     const uint32_t most = 0xFFFFFFFFu / T;  // walkers of one launch: below 2^32 threads
     for (uint32_t f = 0; f < N; f += std::min(most, N - f)) {
       auto go = [&](auto kernel) {
@@ -176,7 +200,9 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
                            how.table_from, seeds, f, g->V, len, stop_prob, seed, paths, lengths, call);
       };
       if (T == 1024) go(walk_direct_kernel<1024>);
+      else if (T == 512) go(walk_direct_kernel<512>);
       else if (T == 256) go(walk_direct_kernel<256>);
+      else if (T == 128) go(walk_direct_kernel<128>);
       else go(walk_direct_kernel<64>);
       call = nullptr;
     }
@@ -213,7 +239,7 @@ __device__ __forceinline__ uint32_t wave_lower_bound(const uint32_t* __restrict_
 template <uint32_t WIN>
 struct N2vRow {
   static constexpr int U = 1;
-  static constexpr bool HELD = true;
+  static constexpr int HELD = 16;
   const float* w;
   const uint32_t* nbr;
   const uint32_t* prow;
@@ -405,7 +431,7 @@ constexpr uint32_t MAP_KEEP = 4096;          // slots of a row whose weights are
 constexpr uint32_t MAP_FEW = 768;
 struct N2vMapRow {
   static constexpr int U = 2;
-  static constexpr bool HELD = true;
+  static constexpr int HELD = 16;
   const float* w;
   const uint32_t* nbr;
   const uint32_t* prow;

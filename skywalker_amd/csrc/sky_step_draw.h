@@ -377,7 +377,7 @@ __device__ __forceinline__ uint32_t draw_held(Row& row, const uint32_t d, const 
 //                     through its part of the row in slot order, once, all lanes together (k advances by 4 per lane)
 //   row.again(k, w)   the same, afterwards, for any slots and by any wavefront
 //   Row::U            how many times 256 slots are in flight at once; if that is more than one, instead of first():
-//   Row::HELD         rows of up to 16 slots a thread by draw_held
+//   Row::HELD         0, 4 or 16: rows of up to so many slots a thread by draw_held
 //   row.many(k, end, again, w)  slots k + 256 j .. k + 256 j + 3 for j < U, zeros from slot `end` on, in both sweeps
 template <int T, class Row>
 __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const u32x4& r, DrawLds<T>& lds) {
@@ -463,17 +463,17 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
   }
   if (!ec.heavy && u < (float)ec.p) return col;  // the light keeps the draw: its alias is never read
 
-  if constexpr (!Row::HELD) {
+  if constexpr (Row::HELD == 0) {
     return surpluses_may_wrap(L.scale) ? draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds)
                                        : draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
   }
   if (surpluses_may_wrap(L.scale)) {
     if (d <= 4 * T) return draw_held<true, 1, T>(row, d, L, col, ec, u, lds);
-    if (d <= 16 * T) return draw_held<true, 4, T>(row, d, L, col, ec, u, lds);
+    if constexpr (Row::HELD == 16) if (d <= 16 * T) return draw_held<true, 4, T>(row, d, L, col, ec, u, lds);
     return draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
   }
   if (d <= 4 * T) return draw_held<false, 1, T>(row, d, L, col, ec, u, lds);
-  if (d <= 16 * T) return draw_held<false, 4, T>(row, d, L, col, ec, u, lds);
+  if constexpr (Row::HELD == 16) if (d <= 16 * T) return draw_held<false, 4, T>(row, d, L, col, ec, u, lds);
   return draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
 }
 
@@ -483,7 +483,7 @@ constexpr uint32_t FN_CACHE = 4096;
 template <class Fn>
 struct FunctionRow {
   static constexpr int U = 1;
-  static constexpr bool HELD = false;  // the operator is called where it is linked in: node2vec's, 8,000 walkers x 20, scale 16, 5.5 ms, 6.0 with
+  static constexpr int HELD = 0;  // the operator is called where it is linked in: node2vec's, 8,000 walkers x 20, scale 16, 5.5 ms, 6.0 with
   Fn fn;
   uint32_t d;
   float* cache;  // [FN_CACHE]

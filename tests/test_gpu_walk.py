@@ -497,3 +497,29 @@ def test_node2vec_table_with_a_bit_per_vertex(orc, V, walkers, p, q):
     want = orc.walk_online(xadj, adjncy, w, 1, p, q, seeds, 8, 0.02, 37)
     assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
     assert sampled == want[2]
+
+
+@pytest.mark.parametrize("longest,walkers", [(70001, 256), (70001, 257), (70001, 8193), (40001, 512), (40001, 513), (40001, 16385),
+                                             (12289, 1024), (12289, 1025), (12289, 8193)])
+def test_online_static_draws_by_workgroups_of_every_size(longest, walkers):
+    # 64 to 1024 threads a walker by the longest row and the number of walkers; rows around 256 slots a wavefront and 4 a thread,
+    # beside 20 M entries in rows of 32: of a graph so large a walk of one step builds no row
+    from skywalker_amd import capi
+    rng = np.random.default_rng(longest)
+    lens = [1, 2, 3, 4, 5, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097, longest] + \
+        list(rng.integers(1, 5000, 100))
+    n = len(lens)
+    lens = np.concatenate([lens, np.full(625000, 32)])
+    xadj = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    local = np.arange(xadj[-1], dtype=np.uint32) - np.repeat(xadj[:-1], lens)  # a vertex of its own for every slot of a row
+    w = np.ones(xadj[-1], np.float32)
+    w[:xadj[n]] = weights(int(xadj[n]), rng, "sparse")
+    g = capi.Graph.upload(xadj, local, w)
+    g.set_option("online_full_build", 0)
+    seeds = (np.arange(walkers) % n).astype(np.uint32)
+    direct = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 1, 0.0, 7)
+    g.build_tables()
+    tabled = g.walk_offline(seeds, 1, 0.0, 7)
+    assert np.array_equal(direct[0].to_host(), tabled[0].to_host()) and np.array_equal(direct[1].to_host(), tabled[1].to_host())
+    assert direct[2] == tabled[2]
+    g.free()
