@@ -268,7 +268,7 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      faster.  The paths are the same.
  *      "online_device_sized" (default 1): sky_sample_online builds the rows of a frontier without the host ever
  *      learning how many they are: the sizes of its degree classes stay on the device, every build kernel finds its rows through them, and the call waits for
- *      the device only once, at its end.  0 makes the host read the size of every frontier and size the launches
+ *      the device only once, at its end; hops whose rows are few are drawn from the weights and build none.  0 makes the host read the size of every frontier and size the launches
  *      exactly, which waits twice per hop.  Same results.
  *      "walk_compact_every" (default 0): k > 0 makes sky_walk_offline run k steps per launch and hand the next
  *      launch the list of walkers that are still walking (the reference's walker queue,

@@ -20,38 +20,7 @@ int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, 
                          float stop_prob, uint64_t seed, uint32_t* paths, uint32_t* lengths, uint64_t* sampled,
                          double* seconds);
 
-// Vectors that are only 4-byte aligned: global loads of 16 bytes need no more on gfx950.
-typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(4)));
-
 // ---------------------------------------------------------------- static bias
-// The graph's own weights of a row (the weight array has 16 spare bytes, so four slots can be read from any).
-struct PlainRow {
-  static constexpr int U = 4;
-  static constexpr int HELD = 4;
-  const float* w;
-  uint32_t d;
-  // Branches that a wavefront takes as one: all loads are on their way before the first is waited for.
-  __device__ __forceinline__ void many(uint32_t k, uint32_t end, bool, float (&x)[U][4]) const {
-    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
-    float4u q[U];
-#pragma unroll
-    for (int j = 0; j < U; ++j) {
-      q[j] = float4u{0, 0, 0, 0};
-      if (first + 256u * j < end) q[j] = *reinterpret_cast<const float4u*>(w + min(k + 256u * j, (d - 1) & ~3u));
-    }
-#pragma unroll
-    for (int j = 0; j < U; ++j)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) x[j][t] = masked_weight(q[j][t], k + 256u * j + t < end);
-  }
-  __device__ __forceinline__ void again(uint32_t k, float (&x)[4]) const {
-    const float4u q = *reinterpret_cast<const float4u*>(w + min(k, (d - 1) & ~3u));
-#pragma unroll
-    for (int t = 0; t < 4; ++t) x[t] = masked_weight(q[t], k + t < d);
-  }
-};
-
 // A walker per workgroup of T threads, for the whole walk.  Rows of table_from entries and more have tables; from the
 // others the draw is evaluated directly.
 template <int T>

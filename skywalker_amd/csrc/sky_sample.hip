@@ -12,13 +12,15 @@
 // result does not depend on scheduling.
 //
 // Online mode builds the table of every distinct frontier vertex, once, through the same
-// kernels as the offline build (into the graph's table storage), then samples the hop.
+// kernels as the offline build (into the graph's table storage), then samples the hop; or, where that takes less (choose_direct),
+// evaluates the draws of a hop from the weights.
 #include <algorithm>
 #include <memory>
 #include <vector>
 
 #include "sky_build_fused.h"
 #include "sky_graph.h"
+#include "sky_step_draw.h"
 
 namespace sky {
 
@@ -140,6 +142,209 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_draw_kernel(SampleArgs a) {
       if ((uint32_t)m < T) mine += o;
     }
     if (tid == 0 && own) a.totals[si] = (a.h0 ? a.totals[si] : 0u) + mine;
+  }
+}
+
+// Online, without a table: the children of a slot from the weights of its row, by T threads that have S consecutive slots of it each.
+// With the deficits and surpluses up to the last of them in LDS every lane evaluates a draw of its own, by searches over the threads'
+// prefixes and the slots of the one they end at.
+template <int T>
+struct DirectLds {
+  uint64_t d[T], u[T];  // inclusive prefixes by thread
+  u128 sum[T / 64];
+  double fsum[T / 64];
+  uint64_t wd[T / 64], wu[T / 64];
+  uint32_t mn[T / 64], any;
+};
+// Children that the row of d > 0 entries yields: g.k, d if it has no more, none if they weigh nothing.  tid: of the T threads, a
+// workgroup or one of its wavefronts.
+template <int T>
+__device__ __forceinline__ uint32_t direct_children(const SampleArgs& a, const HopGeom& g, const float* __restrict__ wgt, uint64_t si,
+                                                    uint32_t s, uint32_t off, uint32_t d, uint32_t tid, DirectLds<T>& lds) {
+  constexpr int NW = T / 64;
+  const uint32_t wave = tid >> 6, lane = tid & 63;
+  const uint32_t* const nbr = a.adjncy + off;
+  uint32_t* const out = a.data + si * g.lps + g.off_next + (uint64_t)s * g.k;
+  PlainRow row{wgt + off, d};
+  auto sync = [] {
+    if constexpr (NW > 1) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  };
+  sync();  // the row before has been drawn from
+  if (d <= g.k) {
+    // all of them, of a row that weighs something: 2^-64 is the least a weight counts for
+    bool any = false;
+    for (uint32_t k = tid; k < d; k += T) any = any || clamp_weight(row.w[k]) >= 5.421010862427522e-20f;
+    if (NW > 1) {
+      if (tid == 0) lds.any = 0;
+      __syncthreads();
+      if (any) lds.any = 1;
+      __syncthreads();
+      any = lds.any;
+    } else {
+      any = __any(any);
+    }
+    if (!any) return 0;
+    for (uint32_t k = tid; k < d; k += T) out[k] = nbr[k];
+    return d;
+  }
+  uint32_t csz = DRAW_CHUNK;
+  while ((uint64_t)csz * NW < d) csz *= 2;
+  const uint32_t k0 = (uint32_t)min((uint64_t)d, (uint64_t)wave * csz), k1 = (uint32_t)min((uint64_t)d, (uint64_t)(wave + 1) * csz);
+  Ledger L;
+  if (!row_ledger<T>(row, d, k0, k1, lds, L)) return 0;
+  const uint32_t S = ((d - 1) / T + 4) & ~3u;
+  // f(slot, heavy, amount) of the slots [from, to), `from` a multiple of 4, until it says true
+  auto slots = [&](uint32_t from, uint32_t to, auto&& f) {
+    auto go = [&](auto quads) {  // that are requested together
+      constexpr int Q = decltype(quads)::value;
+      for (uint32_t k = from; k < to; k += 4 * Q) {
+        float w[Q][4];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) row.again(k + 4 * q, w[q]);
+#pragma unroll
+        for (int j = 0; j < 4 * Q; ++j) {
+          const Entry e = classify_fast((double)w[j / 4][j % 4], k + j < d, L);
+          if (k + j < to && f(k + j, e.heavy, e.amount)) return;
+        }
+      }
+    };
+    if (S > 4) go(std::integral_constant<int, 4>{});
+    else go(std::integral_constant<int, 1>{});
+  };
+  uint64_t sd = 0, su = 0;
+  const uint32_t own = (uint32_t)min((uint64_t)d, (uint64_t)tid * S), end = (uint32_t)min((uint64_t)d, (uint64_t)(tid + 1) * S);
+  slots(own, end, [&](uint32_t, bool heavy, uint64_t x) {
+    sd += heavy ? 0 : x;
+    su = add_sat<true>(su, heavy ? x : 0);
+    return false;
+  });
+  sd = group_scan_u64<64>(sd);
+  su = group_scan_sat_u64<64, true>(su);
+  if (NW > 1) {
+    if (lane == 63) {
+      lds.wd[wave] = sd;
+      lds.wu[wave] = su;
+    }
+    sync();
+#pragma unroll
+    for (int i = 0; i + 1 < NW; ++i)
+      if (i < (int)wave) {
+        sd += lds.wd[i];
+        su = add_sat<true>(su, lds.wu[i]);
+      }
+  }
+  lds.d[tid] = sd;
+  lds.u[tid] = su;
+  sync();
+  const uint64_t total_u = lds.u[T - 1], total_d = lds.d[T - 1];
+  // first slot of the kind whose inclusive prefix exceeds the key, which the kind's total does, and that prefix
+  auto above = [&](bool surplus, uint64_t key, uint64_t& at) -> uint32_t {
+    const uint64_t* p = surplus ? lds.u : lds.d;
+    const uint32_t t = first_greater(p, 0, T, key);
+    uint64_t run = t ? p[t - 1] : 0;
+    uint32_t got = d - 1;
+    slots(t * S, (uint32_t)min((uint64_t)d, (uint64_t)(t + 1) * S), [&](uint32_t k, bool heavy, uint64_t x) {
+      if (heavy == surplus) run = add_sat<true>(run, x);
+      if (run > key) got = k;
+      return run > key;
+    });
+    at = run;
+    return got;
+  };
+  for (uint32_t i = tid; i < g.k; i += T) {
+    const u32x4 r = philox(a.seed, (uint32_t)si, s * g.k + i, g.h, DOM_SAMPLE);
+    const uint32_t col = __umulhi(r.x, d), t = col / S;
+    const float u = u24(r.y);
+    // deficits before a light col, surpluses up to and with a heavy col
+    uint64_t key_d = t ? lds.d[t - 1] : 0, key_u = t ? lds.u[t - 1] : 0;
+    bool heavy = false;
+    float p = 0.0f;
+    {
+      float w[4];
+      row.again(col & ~3u, w);
+      const uint32_t j = col & 3u;
+      const Entry e = classify_fast((double)(j == 0 ? w[0] : j == 1 ? w[1] : j == 2 ? w[2] : w[3]), true, L);
+      heavy = e.heavy;
+      p = (float)e.p;
+    }
+    uint32_t cand = col;
+    if (heavy || !(u < p)) {
+      slots(t * S, col + 1, [&](uint32_t k, bool h, uint64_t x) {
+        if (h) key_u = add_sat<true>(key_u, x);
+        else if (k < col) key_d += x;
+        return false;
+      });
+      uint64_t at;
+      if (!heavy) {
+        // first heavy whose surplus prefix exceeds the key; the last heavy if there is none; col itself without any heavy
+        if (total_u) cand = above(true, min(key_d, total_u - 1), at);
+      } else if (key_u < total_u && key_u <= total_d) {
+        // the first light l with SL(l) >= the key, and the next heavy: prob = (one + key - SL(l)) / one
+        (void)above(false, key_u - 1, at);
+        if (!(u < residual_prob(L.one + key_u - at, L))) cand = above(true, key_u, at);
+      }
+    }
+    out[i] = nbr[cand];
+  }
+  return g.k;
+}
+
+// A wavefront a slot; the slots of a workgroup whose rows are too long for one are left to all eight together.  What bounds it is the chain
+// of some six dependent loads of a slot and the longest row (1,676 seeds x 20 on the scale-22 graph, the longest row met of 100,000 entries:
+// 382 us with a wavefront a slot throughout, 106 with four, 77 like this).
+constexpr int DIRECT_T = 512;
+constexpr uint32_t DIRECT_LONG = 1024;
+__global__ __launch_bounds__(DIRECT_T) void sample_direct_kernel(SampleArgs a, const float* __restrict__ wgt) {
+  constexpr int NW = DIRECT_T / 64;
+  __shared__ __align__(16) unsigned char smem[std::max(sizeof(DirectLds<DIRECT_T>), NW * sizeof(DirectLds<64>))];
+  __shared__ uint32_t s_off[NW], s_d[NW];
+  call_stamp(a.call);
+  const HopGeom& g = a.hop[a.h0];
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  auto done = [&](uint64_t si, uint32_t s, uint32_t cnt) {
+    a.sl[si * g.slen + g.loff + s] = cnt;
+    if (!a.totals) return;
+    if (g.h == 0) a.totals[si] = cnt;
+    else atomicAdd(&a.totals[si], cnt);
+  };
+  const uint64_t first = a.first + (uint64_t)blockIdx.x * NW, slots = a.N * g.width;
+  {
+    const uint64_t slot = first + wave, si = slot / g.width;
+    const uint32_t s = (uint32_t)(slot - si * g.width);
+    uint32_t off = 0, d = 0;
+    if (slot < slots) {
+      const uint32_t v = parent_of(a, g, si, s);
+      if (g.h == 0 && a.seeds && lane == 0) a.data[si * g.lps] = v;
+      if (v < a.V) {
+        off = a.xadj[v];
+        d = a.xadj[v + 1] - off;
+      }
+      off = (uint32_t)__builtin_amdgcn_readfirstlane((int)off);
+      d = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
+      if (d <= DIRECT_LONG) {
+        const uint32_t cnt = d ? direct_children<64>(a, g, wgt, si, s, off, d, lane, reinterpret_cast<DirectLds<64>*>(smem)[wave]) : 0u;
+        if (lane == 0) done(si, s, cnt);
+      }
+    }
+    if (lane == 0) {
+      s_off[wave] = off;
+      s_d[wave] = d > DIRECT_LONG ? d : 0u;
+    }
+  }
+  __syncthreads();
+  for (uint32_t w = 0; w < NW; ++w) {
+    const uint32_t d = s_d[w];
+    if (d == 0) continue;
+    const uint64_t slot = first + w, si = slot / g.width;
+    const uint32_t s = (uint32_t)(slot - si * g.width);
+    const uint32_t cnt = direct_children<DIRECT_T>(a, g, wgt, si, s, s_off[w], d, threadIdx.x, *reinterpret_cast<DirectLds<DIRECT_T>*>(smem));
+    if (threadIdx.x == 0) done(si, s, cnt);
   }
 }
 
@@ -402,6 +607,7 @@ __global__ __launch_bounds__(256) void sample_init_kernel(const uint32_t* __rest
 struct SampleSession {
   sky_graph* g = nullptr;
   bool online = false, dev_sized = false, distinct = false;
+  std::vector<char> direct;  // by hop: drawn from the weights, without tables
   const uint32_t* seeds = nullptr;
   uint32_t N = 0, hops = 0;
   uint64_t seed = 0;
@@ -421,6 +627,7 @@ struct SampleSession {
   // The plan of the graph when the call began.  Another call between the steps of a session may make the graph a new one, when
   // a knob that decides how long rows are built has changed.
   std::shared_ptr<BuildPlan> plan;
+  bool stamped = false;          // the call's first kernel is on its way
   bool want_list = false;        // the caller is to see the frontier as a list of vertices
   uint32_t* totals = nullptr;    // children of each start vertex, when the kernels add them up
   uint32_t frontier_upper = 0;   // most rows the last frontier can hold
@@ -528,7 +735,10 @@ struct SampleSession {
     if (N && one_workgroup()) SKY_TRY(get(sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
     const uint64_t lengths = want_list ? (uint64_t)N * slen : 0;  // to be cleared
     const uint64_t items = std::max<uint64_t>(std::max(std::max(N, bits), 1u), lengths);  // an empty graph has counters too
-    if (online)
+    if (dev_sized && !want_list && !distinct && N) choose_direct();
+    const bool init = online && (direct.empty() || std::find(direct.begin(), direct.end(), 0) != direct.end());
+    stamped = init;
+    if (init)
       hipLaunchKernelGGL(sample_init_kernel, dim3((uint32_t)std::min<uint64_t>((items + 255) / 256, 2048)), dim3(256), 0, st, seeds,
                          N, lps, data, bitmap, bits, list_counts, counters, lengths ? sample_lengths : nullptr, lengths,
                          want_list ? totals : nullptr, call);
@@ -539,7 +749,7 @@ struct SampleSession {
   // the hop's device word d_count (and is read by the host only when the build needs it there).
   int frontier(uint32_t h) {
     frontier_upper = frontier_count = 0;
-    if (!online || !N) return SKY_OK;
+    if (!online || !N || (!direct.empty() && direct[h])) return SKY_OK;
     hipStream_t st = g->stream;
     const HopGeom hg = geom(h);
     const uint64_t slots = (uint64_t)N * hg.width;
@@ -582,6 +792,7 @@ struct SampleSession {
 
   int draw(uint32_t h0, uint32_t h1) {
     if (!N) return SKY_OK;
+    if (!direct.empty() && direct[h0]) return draw_direct(h0);
     hipStream_t st = g->stream;
     SampleArgs a = {};
     a.xadj = g->xadj;
@@ -627,6 +838,52 @@ struct SampleSession {
       else if (T == 256) go(sample_distinct_kernel<256>);
       else if (T == 512) go(sample_distinct_kernel<512>);
       else go(sample_distinct_kernel<1024>);
+      a.call = nullptr;
+    }
+    return SKY_OK;
+  }
+
+  // Which hops do without tables.  The six launches that collect, build and draw take 50 us even of a few rows; start vertices are any
+  // vertices, whose rows are short, and a draw from the weights of one costs little more than the draw from its table.  Of a call of
+  // several hops only up to DIRECT_FEW of them, and no more than there are vertices: rows built for the first hop are met again at the
+  // second.  (Built / direct, us: 10,000 seeds x 20 on the scale-14 graph 66 / 48, 39,000 on the scale-22 graph 125 / 92; 700 x 5 x 3, scale 13,
+  // 103 / 91; 3,000 x 5 x 3, scale 16, 134 / 115; 401 x 10 x 10, scale 22, 299 / 249; 15,900 x 5 x 3 on 4,096 vertices 111 / 145, 36,000 x
+  // 5 x 3 on the scale-20 graph 402 / 450.)  Later hops lead to long rows, again and again: the call does without tables altogether where they
+  // come to few entries and none is very long (70 x 5 x 3, scale 18, 97 / 68; 200 x 25 x 10, scale 15, 106 / 75; 400 x 10 x 10 with 3.4 M
+  // entries, scale 14, 107 / 122; 100 x 5 x 3 on the scale-20 graph, whose longest row has 69,000 entries, 107 / 145).
+  static constexpr uint32_t DIRECT_SEEDS = 65536, DIRECT_FEW = 8192, DIRECT_ROW = 52000;
+  static constexpr double DIRECT_ENTRIES = 2e6;
+  void choose_direct() {
+    if (N > DIRECT_SEEDS || (hops > 2 && N > std::min(DIRECT_FEW, g->V))) return;
+    double mean = 0;  // entries of the row that an edge leads to
+    for (int c = CLS_G2; c < CLS_COUNT; ++c)
+      if (g->bin_counts[c]) mean += (double)g->bin_edges[c] * g->bin_edges[c] / g->bin_counts[c] / std::max(1u, g->E);
+    bool all = g->max_degree <= DIRECT_ROW;
+    for (uint32_t h = 1; h + 1 < hops; ++h) all = all && (double)N * width[h] * mean <= DIRECT_ENTRIES;
+    direct.assign(hops - 1, all);
+    direct[0] = 1;
+  }
+  int draw_direct(uint32_t h) {
+    SampleArgs a = {};
+    a.xadj = g->xadj;
+    a.adjncy = g->adjncy;
+    a.seeds = h == 0 ? seeds : nullptr;
+    a.call = stamped ? nullptr : call;
+    stamped = true;
+    a.data = data;
+    a.sl = sample_lengths;
+    a.totals = totals;
+    a.V = g->V;
+    a.h0 = h;
+    a.h1 = h + 1;
+    a.seed = seed;
+    a.hop[h] = geom(h);
+    a.N = N;
+    constexpr uint64_t PER = DIRECT_T / 64;
+    const uint64_t slots = (uint64_t)N * width[h], most = PER << 22;  // slots of one launch: below 2^32 threads
+    for (a.first = 0; a.first < slots; a.first += most) {
+      const dim3 grid((uint32_t)((std::min<uint64_t>(most, slots - a.first) + PER - 1) / PER));
+      hipLaunchKernelGGL(sample_direct_kernel, grid, dim3(DIRECT_T), 0, g->stream, a, g->adjwgt);
       a.call = nullptr;
     }
     return SKY_OK;

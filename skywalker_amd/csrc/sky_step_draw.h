@@ -19,6 +19,10 @@
 
 namespace sky {
 
+// Vectors that are only 4-byte aligned: global loads of 16 bytes need no more on gfx950.
+typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t uint4u __attribute__((ext_vector_type(4), aligned(4)));
+
 constexpr int N2V_T = 256;
 constexpr uint32_t NONE_SLOT = 0xFFFFFFFFu;
 constexpr uint32_t DRAW_CHUNK = 256;  // slots a wavefront takes at a time: 4 consecutive ones per lane
@@ -371,25 +375,12 @@ __device__ __forceinline__ uint32_t draw_held(Row& row, const uint32_t d, const 
   return lds.result;
 }
 
-// Row-local slot that (walker, step) with random numbers r draws from the row of d >= 1 entries, or NONE_SLOT when
-// their weights sum to zero.  Called by every thread of a workgroup of T.  `row`:
-//   row.first(k, w)   clamped weights of slots k .. k + 3 (k a multiple of 4; zeros past the row).  A wavefront goes
-//                     through its part of the row in slot order, once, all lanes together (k advances by 4 per lane)
-//   row.again(k, w)   the same, afterwards, for any slots and by any wavefront
-//   Row::U            how many times 256 slots are in flight at once; if that is more than one, instead of first():
-//   Row::HELD         0, 4 or 16: rows of up to so many slots a thread by draw_held
-//   row.many(k, end, again, w)  slots k + 256 j .. k + 256 j + 3 for j < U, zeros from slot `end` on, in both sweeps
-template <int T, class Row>
-__device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const u32x4& r, DrawLds<T>& lds) {
+// Ledger of the row of d >= 1 entries by a workgroup of T, of which this wavefront has slots [k0, k1); false when the weights sum to
+// zero.
+template <int T, class Row, class Lds>
+__device__ __forceinline__ bool row_ledger(Row& row, const uint32_t d, const uint32_t k0, const uint32_t k1, Lds& lds, Ledger& L) {
   constexpr int NW = T / 64, U = Row::U;
-  const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  uint32_t csz = DRAW_CHUNK;
-  while ((uint64_t)csz * DRAW_CHUNKS < d) csz *= 2;
-  const uint32_t nc = (uint32_t)(((uint64_t)d + csz - 1) / csz), cpw = (nc + NW - 1) / NW;
-  const uint32_t c0 = wave * cpw, c1 = min(nc, c0 + cpw);
-  __syncthreads();  // the draw before has been read by everyone
-  const uint32_t k0 = c0 < nc ? c0 * csz : d, k1 = c0 < nc ? (c1 == nc ? d : c1 * csz) : d;  // this wavefront's slots
-
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // pass 1: the sum as a plain fp64 sum where that is exact (plain_sum_is_exact), else in 128 bits
   double fsum = 0.0;
   uint32_t mn = 0xFFFFFFFFu;
@@ -420,12 +411,13 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
       fsum += lds.fsum[i];
       mn = min(mn, lds.mn[i]);
     }
-  } else {
-    __syncthreads();  // what first() has left in LDS
+  } else {  // what first() has left in LDS
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
-  Ledger L;
   if (plain_sum_is_exact(fsum, mn)) {
-    if (fsum == 0.0) return NONE_SLOT;
+    if (fsum == 0.0) return false;
     L = make_ledger_small(d, fsum);
     if (d >= (1u << 22)) {
       const int F = 62 - (31 - __clz((int)d));
@@ -449,9 +441,33 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
 #pragma unroll
       for (int i = 1; i < NW; ++i) sum = add128(sum, lds.sum[i]);
     }
-    if ((sum.lo | sum.hi) == 0) return NONE_SLOT;
+    if ((sum.lo | sum.hi) == 0) return false;
     L = make_ledger(d, sum);
   }
+  return true;
+}
+
+// Row-local slot that (walker, step) with random numbers r draws from the row of d >= 1 entries, or NONE_SLOT when
+// their weights sum to zero.  Called by every thread of a workgroup of T.  `row`:
+//   row.first(k, w)   clamped weights of slots k .. k + 3 (k a multiple of 4; zeros past the row).  A wavefront goes
+//                     through its part of the row in slot order, once, all lanes together (k advances by 4 per lane)
+//   row.again(k, w)   the same, afterwards, for any slots and by any wavefront
+//   Row::U            how many times 256 slots are in flight at once; if that is more than one, instead of first():
+//   Row::HELD         0, 4 or 16: rows of up to so many slots a thread by draw_held
+//   row.many(k, end, again, w)  slots k + 256 j .. k + 256 j + 3 for j < U, zeros from slot `end` on, in both sweeps
+template <int T, class Row>
+__device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const u32x4& r, DrawLds<T>& lds) {
+  constexpr int NW = T / 64;
+  const uint32_t wave = threadIdx.x >> 6;
+  uint32_t csz = DRAW_CHUNK;
+  while ((uint64_t)csz * DRAW_CHUNKS < d) csz *= 2;
+  const uint32_t nc = (uint32_t)(((uint64_t)d + csz - 1) / csz), cpw = (nc + NW - 1) / NW;
+  const uint32_t c0 = wave * cpw, c1 = min(nc, c0 + cpw);
+  __syncthreads();  // the draw before has been read by everyone
+  const uint32_t k0 = c0 < nc ? c0 * csz : d, k1 = c0 < nc ? (c1 == nc ? d : c1 * csz) : d;  // this wavefront's slots
+
+  Ledger L;
+  if (!row_ledger<T>(row, d, k0, k1, lds, L)) return NONE_SLOT;
   const uint32_t col = __umulhi(r.x, d);
   const float u = u24(r.y);
   Entry ec;
@@ -476,6 +492,33 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
   if constexpr (Row::HELD == 16) if (d <= 16 * T) return draw_held<false, 4, T>(row, d, L, col, ec, u, lds);
   return draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
 }
+
+// The graph's own weights of a row (the weight array has 16 spare bytes, so four slots can be read from any).
+struct PlainRow {
+  static constexpr int U = 4;
+  static constexpr int HELD = 4;
+  const float* w;
+  uint32_t d;
+  // Branches that a wavefront takes as one: all loads are on their way before the first is waited for.
+  __device__ __forceinline__ void many(uint32_t k, uint32_t end, bool, float (&x)[U][4]) const {
+    const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
+    float4u q[U];
+#pragma unroll
+    for (int j = 0; j < U; ++j) {
+      q[j] = float4u{0, 0, 0, 0};
+      if (first + 256u * j < end) q[j] = *reinterpret_cast<const float4u*>(w + min(k + 256u * j, (d - 1) & ~3u));
+    }
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) x[j][t] = masked_weight(q[j][t], k + 256u * j + t < end);
+  }
+  __device__ __forceinline__ void again(uint32_t k, float (&x)[4]) const {
+    const float4u q = *reinterpret_cast<const float4u*>(w + min(k, (d - 1) & ~3u));
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[t] = masked_weight(q[t], k + t < d);
+  }
+};
 
 // A row whose weights are computed by a function of the slot (row(k): clamped weight of slot k < d): those of a row of up
 // to CAP entries stay in LDS after the first pass, those of a longer one are computed again.

@@ -529,3 +529,29 @@ def test_row_lists_made_anew_leave_the_flags_of_a_session_alone(orc):
     assert np.array_equal(s[4].to_host((16, slen)), want[1]) and np.array_equal(s[3].to_host((16, lps)), want[0])
     assert sampled == want[2] == 8
     g.free()
+
+
+@pytest.mark.parametrize("fanout", [[1, 20], [1, 5, 3], [1, 70], [1, 600], [1, 1]])
+@pytest.mark.parametrize("dist,seeds_n", [("lognormal2", 333), ("sparse", 1601), ("nearequal", 40)])
+def test_children_drawn_from_the_weights(orc, fanout, dist, seeds_n):
+    # without tables, a wavefront or a workgroup a slot: rows around the fan-out, around 4 and 16 slots a thread and around the rows that a
+    # workgroup shares; rows without weight, and with surpluses beyond 64 bits; workgroups partly empty; start vertices that do not exist
+    from skywalker_amd import capi
+    rng = np.random.default_rng(53)
+    degs = [0, 1, 2, 3, 4, 5, 19, 20, 21, 63, 64, 65, 69, 70, 71, 255, 256, 257, 260, 511, 513, 599, 600, 601, 1021, 1023, 1024, 1025,
+            2047, 2048, 2049, 4097, 8191, 8193, 40001] + list(rng.integers(1, 700, 40))
+    xadj, adjncy, w = graph_from_degrees(degs, rng, dist)
+    n = len(degs)
+    for v in range(0, n, 3):
+        if dist == "sparse":
+            w[xadj[v]:xadj[v + 1]] *= np.float32(1e-19)
+    for v in (7, 20, 31):
+        w[xadj[v]:xadj[v + 1]] = 0.0
+    seeds = np.append((np.arange(seeds_n - 1) * 7) % n, n + 5).astype(np.uint32)
+    lps, slen = capi.sample_layout(fanout)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    d, sl, sampled, _ = g.sample_online(seeds, fanout, 61)
+    got = d.to_host((seeds_n, lps)), sl.to_host((seeds_n, slen))
+    g.free()
+    want = orc.sample_online(xadj, adjncy, w, seeds, fanout, 61)
+    assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0]) and sampled == want[2]
