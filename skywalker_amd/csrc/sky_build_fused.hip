@@ -37,7 +37,7 @@ enum Section : uint32_t {
   SEC_TOTALS,                                  //             two tiles
   SEC_STREAM, SEC_B6, SEC_B8, SEC_B10,  // 512 threads
   SEC_SCAN,                                    //             a row's tiles
-  SEC_M6, SEC_M8, SEC_M10,                     // 256 threads
+  SEC_M6, SEC_M8, SEC_M10, SEC_M14,            // 256 threads
   SEC_EMIT                                     //             a tile
 };
 struct SectionRef {
@@ -394,9 +394,10 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
   }
 }
 
-template <bool DEV>
+// LONGER: rows of 2558..3581 entries as well (block_takes_longer), for which a CU holds four workgroups instead of five.
+template <bool DEV, bool LONGER>
 __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
-  __shared__ __align__(16) uint64_t smem[(BLOCK_LDS + 7) / 8];
+  __shared__ __align__(16) uint64_t smem[((LONGER ? cmax(merge_lds_bytes(256, 14), BLOCK_LDS) : BLOCK_LDS) + 7) / 8];
   __shared__ uint64_t s_aux[32];
   call_stamp(a.call);
   const UnitFinder<DEV> units(a);
@@ -407,6 +408,9 @@ __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
     switch (s.kind) {
       case SEC_M6: merge_unit<DEV, 256, 6>(a, s, unit, rows, smem, s_aux); break;
       case SEC_M8: merge_unit<DEV, 256, 8>(a, s, unit, rows, smem, s_aux); break;
+      case SEC_M14:
+        if constexpr (LONGER) merge_unit<DEV, 256, 14>(a, s, unit, rows, smem, s_aux);
+        break;
       case SEC_M10: merge_unit<DEV, 256, 10>(a, s, unit, rows, smem, s_aux); break;
       case SEC_EMIT: {
         const uint32_t tile = a.tile0 + unit;
@@ -685,9 +689,21 @@ FusedArgs common_args(sky_graph* g, const BuildPlan& p, int tiled_from) {
   return a;
 }
 
+// Whether the rows of 2558..3581 entries (CLS_MW2 + 4 and + 5) go out with the launch of 256 threads, 14 slots each, rather than beside
+// the streamed rows, whose LDS leaves two workgroups of 512 to a CU (23 M entries in such rows of the scale-22 graph with 32 edges a
+// vertex: 120 us there, 94 here; its build 725 -> 700).  With their LDS a CU holds four workgroups of that launch instead of five,
+// which costs tiles more (16 M entries in tiles 543 -> 570 us).
+constexpr double LONGER_ENTRIES = 4e6, LONGER_PER_TILED = 2;
+bool block_takes_longer(const sky_graph* g, int tiled_from) {
+  double tiled = 0;
+  for (int c = tiled_from; c <= CLS_HUGE; ++c) tiled += (double)g->bin_edges[c];
+  const double longer = (double)g->bin_edges[CLS_MW2 + 4] + (double)g->bin_edges[CLS_MW2 + 5];
+  return longer >= std::max(LONGER_ENTRIES, LONGER_PER_TILED * tiled);
+}
+
 // The four launches, in order on the graph's stream.
 template <bool DEV>
-int launch_all(sky_graph* g, const BuildPlan& p, Launch& wave, Launch& pair, Launch& wide, Launch& block, CallDevice* call) {
+int launch_all(sky_graph* g, const BuildPlan& p, Launch& wave, Launch& pair, Launch& wide, Launch& block, bool longer, CallDevice* call) {
   hipStream_t st = g->stream;
   // the first launch that has anything to do is the call's first
   Launch* const order[4] = {&wave, &pair, &wide, &block};
@@ -704,7 +720,8 @@ int launch_all(sky_graph* g, const BuildPlan& p, Launch& wave, Launch& pair, Lau
                                               p.tsum, DEV);
   if (pair.units) hipLaunchKernelGGL((fused_pair_kernel<DEV>), grid(pair, 2560), dim3(128), 0, st, pair.a);
   if (wide.units) hipLaunchKernelGGL((fused_wide_kernel<DEV>), grid(wide, 512), dim3(512), 0, st, wide.a);
-  if (block.units) hipLaunchKernelGGL((fused_block_kernel<DEV>), grid(block, 1024), dim3(256), 0, st, block.a);
+  if (block.units && longer) hipLaunchKernelGGL((fused_block_kernel<DEV, true>), grid(block, 1024), dim3(256), 0, st, block.a);
+  else if (block.units) hipLaunchKernelGGL((fused_block_kernel<DEV, false>), grid(block, 1024), dim3(256), 0, st, block.a);
   SKY_HIP(hipGetLastError());
   return SKY_OK;
 }
@@ -781,15 +798,21 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   const bool hold_alone = min_degree == 0 && rows(CLS_HOLD) >= HOLD_ALONE;  // behind the sweep, which notes when the call began
   if (!hold_alone) wide.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);
   // two classes whose lists lie back to back; min_degree may leave out the first
-  auto add_two = [&](Section k, int c) { wide.add(k, rows(c) + rows(c + 1), 1, p.start[rows(c) ? c : c + 1]); };
-  add_two(SEC_B10, CLS_MW2 + 7);
-  add_two(SEC_B8, CLS_MW2 + 5);
-  wide.add(SEC_B6, rows(CLS_MW2 + 4), 1, p.start[CLS_MW2 + 4]);
+  auto add_two = [&](Launch& l, Section k, int c) { l.add(k, rows(c) + rows(c + 1), 1, p.start[rows(c) ? c : c + 1]); };
+  add_two(wide, SEC_B10, CLS_MW2 + 7);
+  const bool longer = block_takes_longer(g, p.t_all);
+  if (longer) {
+    wide.add(SEC_B8, rows(CLS_MW2 + 6), 1, p.start[CLS_MW2 + 6]);
+  } else {
+    add_two(wide, SEC_B8, CLS_MW2 + 5);
+    wide.add(SEC_B6, rows(CLS_MW2 + 4), 1, p.start[CLS_MW2 + 4]);
+  }
   block.add(SEC_EMIT, n_tiles, 1, 0);
+  if (longer) add_two(block, SEC_M14, CLS_MW2 + 4);
   block.add(SEC_M10, rows(CLS_MW2 + 3), 1, p.start[CLS_MW2 + 3]);
   block.add(SEC_M8, rows(CLS_MW2 + 2), 1, p.start[CLS_MW2 + 2]);
   block.add(SEC_M6, rows(CLS_MW2 + 1), 1, p.start[CLS_MW2 + 1]);
-  SKY_TRY(launch_all<false>(g, p, wave, pair, wide, block, call));
+  SKY_TRY(launch_all<false>(g, p, wave, pair, wide, block, longer, call));
   return hold_alone ? build_rows_hold(g, p.rows + p.start[CLS_HOLD], rows(CLS_HOLD)) : SKY_OK;
 }
 int build_all_fused(sky_graph* g, CallDevice* call) { return build_host_sized(g, 0, call); }
@@ -848,13 +871,19 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, con
   if (f.tiled_from != CLS_STREAM) add(wide, SEC_STREAM, 1, CLS_STREAM, 2);
   add(wide, SEC_STREAM, 1, CLS_HOLD);
   add(wide, SEC_B10, 1, CLS_MW2 + 7, 2);
-  add(wide, SEC_B8, 1, CLS_MW2 + 5, 2);
-  add(wide, SEC_B6, 1, CLS_MW2 + 4);
+  const bool longer = block_takes_longer(g, f.tiled_from);
+  if (longer) {
+    add(wide, SEC_B8, 1, CLS_MW2 + 6);
+  } else {
+    add(wide, SEC_B8, 1, CLS_MW2 + 5, 2);
+    add(wide, SEC_B6, 1, CLS_MW2 + 4);
+  }
   block.add(SEC_EMIT, n_tiles, 1, 0);
+  if (longer) add(block, SEC_M14, 1, CLS_MW2 + 4, 2);
   add(block, SEC_M10, 1, CLS_MW2 + 3);
   add(block, SEC_M8, 1, CLS_MW2 + 2);
   add(block, SEC_M6, 1, CLS_MW2 + 1);
-  return launch_all<true>(g, p, wave, pair, wide, block, nullptr);
+  return launch_all<true>(g, p, wave, pair, wide, block, longer, nullptr);
 }
 
 }  // namespace sky
