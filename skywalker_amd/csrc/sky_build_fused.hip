@@ -69,6 +69,7 @@ struct FusedArgs {
   const uint32_t* bitmap;  // frontier: bit set for every vertex whose row has been asked for (null: every row is built)
   uint32_t bit_mask;       // of the bitmap (frontier_bit)
   uint32_t* built;         // frontier: by row of trows, set once a build of the same call has made it
+  uint32_t* next;          // frontier: units of the wide launch that are taken, 0 at first (null: every grid-th for each workgroup)
   uint32_t tile0, trow0;  // first tile and row of those this build makes tile by tile
   bool ledgers_done;
   CallDevice* call;  // the call's first launch notes when it began
@@ -126,6 +127,14 @@ struct UnitFinder<true> {
     return true;
   }
 };
+// The next unit that no workgroup of the launch has.
+__device__ __forceinline__ uint32_t next_unit(uint32_t* taken) {
+  __shared__ uint32_t s_unit;
+  __syncthreads();  // the unit before is done with LDS, and s_unit has been read
+  if (threadIdx.x == 0) s_unit = gridDim.x + atomicAdd(taken, 1u);
+  __syncthreads();
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)s_unit);
+}
 // Row `i` of a section (host-sized: `rows` holds none, the section's last unit may be partly empty).
 template <bool DEV>
 __device__ __forceinline__ bool row_at(const FusedArgs& a, const SectionRef& s, uint32_t i, uint32_t rows, RowRef& rr) {
@@ -363,7 +372,9 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
   uint64_t* const s_aux = smem + (WIDE_LDS - 512) / 8;
   call_stamp(a.call);
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = blockIdx.x;; u += gridDim.x) {
+  // Rows of tiles by every grid-th workgroup; the rows behind them, where a.next is given, by the workgroup that is first free.
+  const uint32_t scans = DEV && a.next && a.sec[0].kind == SEC_SCAN ? a.sec[0].units : 0u;
+  for (uint32_t u = blockIdx.x < scans ? blockIdx.x : scans + blockIdx.x;;) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -390,7 +401,16 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
       default: break;
     }
     if (!DEV) return;
-    __syncthreads();
+    if (!a.next) {
+      u += gridDim.x;
+      __syncthreads();
+    } else if (u < scans) {
+      u += gridDim.x;
+      if (u >= scans) u = scans + blockIdx.x;
+      __syncthreads();
+    } else {
+      u = scans + next_unit(a.next);
+    }
   }
 }
 
@@ -701,6 +721,17 @@ bool block_takes_longer(const sky_graph* g, int tiled_from) {
   return longer >= std::max(LONGER_ENTRIES, LONGER_PER_TILED * tiled);
 }
 
+// Whether the workgroups of a frontier's wide launch ask for their next unit instead of taking every 512th.  A streamed row of 60,000
+// entries takes seven times as long as one of 8,000, and who asks waits 2 us: not where merges, of some 8 us, are most of the units.
+// (40,000 seeds 25 x 10 on the scale-22 graph with 32 edges a vertex, 1,800 streamed rows: 177 us, asked for 162; with 7,300 merges
+// beside them 297, asked for 330.)
+bool streams_by_queue(const sky_graph* g, int tiled_from, bool longer) {
+  if (tiled_from == CLS_STREAM) return false;
+  uint64_t merges = 0;
+  for (int c = CLS_MW2 + (longer ? 6 : 4); c <= CLS_MW2 + 8; ++c) merges += g->bin_counts[c];
+  return merges <= (uint64_t)g->bin_counts[CLS_STREAM] + g->bin_counts[CLS_STREAM_LAST];
+}
+
 // The four launches, in order on the graph's stream.
 template <bool DEV>
 int launch_all(sky_graph* g, const BuildPlan& p, Launch& wave, Launch& pair, Launch& wide, Launch& block, bool longer, CallDevice* call) {
@@ -836,7 +867,7 @@ int frontier_lists(sky_graph* g, const BuildPlan& p, uint32_t n_upper, sky_graph
   return SKY_OK;
 }
 
-int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, const uint32_t* counts, const uint32_t* bitmap,
+int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uint32_t* counts, const uint32_t* bitmap,
                    uint32_t* built) {
   g->has_walk_index = false;
   FusedArgs base = common_args(g, p, f.tiled_from);
@@ -872,6 +903,7 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, con
   add(wide, SEC_STREAM, 1, CLS_HOLD);
   add(wide, SEC_B10, 1, CLS_MW2 + 7, 2);
   const bool longer = block_takes_longer(g, f.tiled_from);
+  if (streams_by_queue(g, f.tiled_from, longer)) wide.a.next = counts + CLS_COUNT;
   if (longer) {
     add(wide, SEC_B8, 1, CLS_MW2 + 6);
   } else {

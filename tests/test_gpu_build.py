@@ -782,3 +782,25 @@ def test_seconds_of_a_call_that_lists_the_rows_contain_the_listing(kind):
     print(kind, "again %.1f us, with the listing %.1f us" % (again * 1e6, listing * 1e6))
     assert listing - again > 4 * V / 8e12
     g.free()
+
+
+def test_rows_of_2558_to_3581_entries_beside_shorter_ones(orc):
+    # enough of them for the launch of 256 threads, 14 slots each, in a build and in that of a frontier, whose streamed rows the workgroups
+    # ask for; the edges of their classes, and of those around them
+    from skywalker_amd import capi
+    rng = np.random.default_rng(59)
+    degs = list(rng.integers(2558, 3582, 1400)) + [2556, 2557, 2558, 2559, 3069, 3070, 3071, 3580, 3581, 3582, 3583, 4093, 4094, 5117] * 3 + \
+        list(rng.integers(8190, 65534, 40)) + [8190, 24576, 24577, 65533] + list(rng.integers(1, 300, 3000))
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal")
+    g = capi.Graph.upload(xadj, adjncy, w)
+    seeds = (np.arange(70000) % len(degs)).astype(np.uint32)
+    d, sl, sampled, _ = g.sample_online(seeds, [1, 2], 3)
+    got = d.to_host(), sl.to_host()
+    g.build_tables()
+    prob, alias, valid = g.tables()
+    g.free()
+    oprob, oalias, ovalid = orc.alias_build(xadj, w)
+    assert np.array_equal(prob.view(np.uint32), oprob.view(np.uint32)) and np.array_equal(alias, oalias) and np.array_equal(valid, ovalid)
+    want = orc.sample_offline(xadj, adjncy, oprob, oalias, seeds, [1, 2], 3)
+    assert np.array_equal(got[0], want[0].ravel()) and np.array_equal(got[1], want[1].ravel()) and sampled == want[2]
