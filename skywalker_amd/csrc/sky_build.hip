@@ -214,7 +214,7 @@ __global__ __launch_bounds__(64) void small_rows_kernel(const uint32_t* __restri
                                                         uint32_t per_wave, AliasEntry* __restrict__ table,
                                                         int8_t* __restrict__ valid) {
   __shared__ uint64_t smem[(SMALL_LDS_BYTES + 7) / 8];
-  small_rows_range(blockIdx.x * per_wave, xadj, wgt, src, n, per_wave, table, valid, smem);
+  small_rows_range(spread_units(blockIdx.x, gridDim.x) * per_wave, xadj, wgt, src, n, per_wave, table, valid, smem);
 }
 
 // ---------------------------------------------------------------- one row per workgroup, prefix arrays in LDS

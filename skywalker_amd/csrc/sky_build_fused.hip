@@ -264,7 +264,8 @@ __device__ __forceinline__ void tile_totals_wave(const FusedArgs& a, uint32_t ti
 }
 
 __device__ __forceinline__ void sweep_unit(const FusedArgs& a, uint32_t unit, uint64_t* smem) {
-  small_rows_range((a.split ? unit / 4 : unit) * a.per_wave, a.xadj, a.wgt, nullptr, a.V, a.per_wave, a.table, a.valid, smem,
+  const uint32_t range = a.split ? unit / 4 : spread_units(unit, (a.V + a.per_wave - 1) / a.per_wave);
+  small_rows_range(range * a.per_wave, a.xadj, a.wgt, nullptr, a.V, a.per_wave, a.table, a.valid, smem,
                    a.split ? 1u << (unit % 4) : 15u);
 }
 

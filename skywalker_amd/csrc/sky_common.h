@@ -81,6 +81,13 @@ __device__ __forceinline__ float clamp_weight(float w) {
 __device__ __forceinline__ float masked_weight(float w, bool in) {
   return __builtin_amdgcn_fmed3f(w, 0.0f, in ? 4294967296.0f : 0.0f);
 }
+// A permutation of the units u < n of a launch that are ranges of a graph's vertices.  Workgroup u runs on XCD u mod 8, and in a graph whose
+// ids say something about degrees (every bit of an R-MAT id does) so would the last bits of u: the XCD of the ranges that end in
+// 000 had several times the entries of the others.  (Builds, us, in order / spread: 2^26 vertices with 5 edges each 2312 / 1769, 2^25 with 20
+// 3600 / 3350, 2^24 with 7 780 / 670, 2^22 with 10 312 / 274, 2^20 with 16 138 / 132; rows in random order 352 / 352.)
+__device__ __forceinline__ uint32_t spread_units(uint32_t u, uint32_t n) {
+  return (u | 63u) < n ? u ^ ((u >> 6) * 0x9E3779B1u) >> 26 : u;
+}
 // floor(w * 2^64) of a clamped weight.
 __device__ __forceinline__ u128 weight_fixed(float w) {
   const uint32_t bits = __float_as_uint(w);

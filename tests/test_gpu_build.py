@@ -804,3 +804,23 @@ def test_rows_of_2558_to_3581_entries_beside_shorter_ones(orc):
     assert np.array_equal(prob.view(np.uint32), oprob.view(np.uint32)) and np.array_equal(alias, oalias) and np.array_equal(valid, ovalid)
     want = orc.sample_offline(xadj, adjncy, oprob, oalias, seeds, [1, 2], 3)
     assert np.array_equal(got[0], want[0].ravel()) and np.array_equal(got[1], want[1].ravel()) and sampled == want[2]
+
+
+@pytest.mark.parametrize("V", [32769, 36863, 36864, 36865, 40959, 200001])
+def test_short_rows_of_ranges_in_another_order(orc, V):
+    # whole and partial groups of 64 ranges of vertices
+    from skywalker_amd import capi
+    rng = np.random.default_rng(V)
+    degs = np.where(rng.random(V) < 0.02, rng.integers(33, 300, V), rng.integers(0, 34, V))
+    xadj = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    E = int(xadj[-1])
+    adjncy = rng.integers(0, V, E, dtype=np.uint32)
+    w = rng.lognormal(0, 1, E).astype(np.float32)
+    w[rng.random(E) < 0.3] = 0.0
+    g = capi.Graph.upload(xadj, adjncy, w)
+    for _ in range(2):
+        g.build_tables()
+    prob, alias, valid = g.tables()
+    g.free()
+    oprob, oalias, ovalid = orc.alias_build(xadj, w)
+    assert np.array_equal(prob.view(np.uint32), oprob.view(np.uint32)) and np.array_equal(alias, oalias) and np.array_equal(valid, ovalid)
