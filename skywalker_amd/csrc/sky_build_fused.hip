@@ -415,6 +415,12 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
   }
 }
 
+// Tiles in an order in which neighbours run on the same XCD (workgroup u on u mod 8), 64 in a row: a tile reads the weights of those
+// it is paired with once more, and finds them in that XCD's cache.  (40 M entries, 11 M of them in tiles: 350 -> 345 us; 60 M: 531 -> 523.)
+__device__ __forceinline__ uint32_t near_tile(uint32_t u, uint32_t n) {
+  return (u | 511u) < n ? (u & ~511u) + (u & 7u) * 64u + ((u >> 3) & 63u) : u;
+}
+
 // LONGER: rows of 2558..3581 entries as well (block_takes_longer), for which a CU holds four workgroups instead of five.
 template <bool DEV, bool LONGER>
 __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
@@ -434,7 +440,7 @@ __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
         break;
       case SEC_M10: merge_unit<DEV, 256, 10>(a, s, unit, rows, smem, s_aux); break;
       case SEC_EMIT: {
-        const uint32_t tile = a.tile0 + unit;
+        const uint32_t tile = a.tile0 + near_tile(unit, s.units);
         const TileGeom tg = a.geom[tile];
         if (tg.span == 0 || (a.bitmap && !a.trows[tg.row].active)) break;
         tile_emit(tg, tile, a.trows, a.wgt, a.BL, a.BH, a.nfh, a.ranges, a.table, a.valid,
