@@ -880,7 +880,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   // own launch (too few workgroups to fill the GPU): its rows then go to the tile-parallel path together with the
   // HUGE class.  The rows above 65533 entries keep one workgroup busy for up to 1.5 ms; they join the launch (and
   // start first) only when it holds enough other rows to run that long anyway, else they are built tile by tile.
-  // The lists lie back to back: STREAM, STREAM_LAST, STREAM_WIDE, HUGE.
+  // The lists lie back to back: STREAM_LAST, STREAM, STREAM_WIDE, HUGE.
   const uint32_t narrow_rows = counts[CLS_STREAM] + counts[CLS_STREAM_LAST];
   const uint64_t narrow_edges = host.edges[CLS_STREAM] + host.edges[CLS_STREAM_LAST];
   const uint64_t all_stream_edges = narrow_edges + host.edges[CLS_STREAM_WIDE];
@@ -953,7 +953,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   if (!stream_to_tiled && narrow_rows + wide_rows) {
     // the streaming kernel takes three times as long for an entry as the others when it shares the GPU with them
     StreamSwap sw(g, fan.next(3 * (narrow_edges + (wide_streamed ? host.edges[CLS_STREAM_WIDE] : 0))));
-    SKY_TRY(build_rows_stream(g, vlist + starts[CLS_STREAM_WIDE], wide_rows, vlist + starts[CLS_STREAM], narrow_rows));
+    SKY_TRY(build_rows_stream(g, vlist + starts[CLS_STREAM_WIDE], wide_rows, vlist + starts[CLS_STREAM_LAST], narrow_rows));
     if (tm) SKY_TRY(tm->mark("stream", narrow_edges + (wide_streamed ? host.edges[CLS_STREAM_WIDE] : 0)));
   }
   // Rows of 5118..8189 entries: one workgroup holds the row (without row_merge they are built tile by tile).
@@ -972,7 +972,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   SKY_TRY(grp(CLS_G32S, build_group_kernel<SHAPE_G32S.lanes, SHAPE_G32S.per>, SHAPE_G32S.lanes, "g32s"));
   SKY_TRY(grp(CLS_G32X, build_group_kernel<SHAPE_G32X.lanes, SHAPE_G32X.per>, SHAPE_G32X.lanes, "g32x"));
 
-  // the lists HOLD, STREAM, STREAM_LAST, STREAM_WIDE, HUGE lie back to back (the class numbers between are unused)
+  // the lists HOLD, STREAM_LAST, STREAM, STREAM_WIDE, HUGE lie back to back (the class numbers between are unused)
   const uint32_t held_rows = row_merge ? 0 : counts[CLS_HOLD];
   const uint32_t tiled_rows =
       counts[CLS_HUGE] + (wide_streamed ? 0 : counts[CLS_STREAM_WIDE]) + (stream_to_tiled ? narrow_rows : 0) + held_rows;
@@ -981,7 +981,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
                                (row_merge ? 0 : host.edges[CLS_HOLD]);
   const RowRef* tiled_list =
       vlist + (held_rows ? starts[CLS_HOLD]
-                         : stream_to_tiled ? starts[CLS_STREAM] : (wide_streamed ? starts[CLS_HUGE] : starts[CLS_STREAM_WIDE]));
+                         : stream_to_tiled ? starts[CLS_STREAM_LAST] : (wide_streamed ? starts[CLS_HUGE] : starts[CLS_STREAM_WIDE]));
   if (tiled_rows) {
     const uint32_t cnt = tiled_rows;
     uint32_t skipped = 0;

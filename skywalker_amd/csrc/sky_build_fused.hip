@@ -495,7 +495,8 @@ __global__ __launch_bounds__(512, 4) void fused_all_kernel(FusedArgs a) {
 
 // ---------------------------------------------------------------- plan of a graph
 // Geometry of the rows that are built tile by tile, in list order: one workgroup, once per graph.
-__global__ __launch_bounds__(1024) void plan_rows_kernel(const RowRef* __restrict__ list, uint32_t n, TiledRow* __restrict__ rows) {
+__global__ __launch_bounds__(1024) void plan_rows_kernel(const RowRef* __restrict__ list, uint32_t n, TiledRow* __restrict__ rows,
+                                                         uint32_t row0, uint32_t tile0) {
   __shared__ uint32_t s_w[16];
   const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   uint32_t carry = 0;
@@ -516,7 +517,7 @@ __global__ __launch_bounds__(1024) void plan_rows_kernel(const RowRef* __restric
       total += s_w[w];
     }
     if (r < n) {
-      TiledRow& o = rows[r];
+      TiledRow& o = rows[row0 + r];
       o.v = rr.v;
       o.off = rr.off;
       o.d = rr.d;
@@ -524,8 +525,8 @@ __global__ __launch_bounds__(1024) void plan_rows_kernel(const RowRef* __restric
       o.lead = rr.off & 3u;
       o.span = o.lead + rr.d;
       o.ntiles = nt;
-      o.tile0 = before + inc - nt;
-      o.bofs = o.tile0 + r;  // every row owns ntiles + 1 prefix slots
+      o.tile0 = tile0 + before + inc - nt;
+      o.bofs = o.tile0 + row0 + r;  // every row owns ntiles + 1 prefix slots
       o.active = 0;
     }
     carry += total;
@@ -611,27 +612,43 @@ int ensure_plan(sky_graph* g, CallDevice** first) {
     for (int c = CLS_G16; c < CLS_COUNT; ++c) p.listed += g->bin_counts[c];
     p.narrow_limit = narrow_limit;
     // Rows of 8190..65533 entries are streamed, one workgroup each, by builds that hold enough of them to fill the GPU that
-    // way; other builds, and those of small frontiers, make them tile by tile, for which they need geometry.  A graph
-    // with very many of them does without: 65536 tiles that a frontier may have to pass over take 20 us a launch.
-    const uint64_t narrow = g->bin_edges[CLS_STREAM] + g->bin_edges[CLS_STREAM_LAST];
+    // way; other builds, and those of small frontiers, make them tile by tile, all of them or those of more than 24,576, for which
+    // they need geometry.  A graph with very many of them does without: 65536 tiles that a frontier may have to pass over take 20 us
+    // a launch.
     // A workgroup takes 2.4 ns an entry for such a row, and the launch lasts at least as long as the longest of them.
     // The launch of the rows of 2558..65533 entries as a whole takes 6 ps an entry, the tile passes 13 ps (one
     // MI355X; this tells the faster way for 13 of 13 graphs of 4 to 117 M entries: 40 M entries in rows of 1..300,000
-    // 409 -> 367 us by tiles, R-MAT scale 22 edge factor 28 754 us streamed, 888 by tiles).
-    uint64_t wide = narrow + g->bin_edges[CLS_HOLD];
+    // 409 -> 367 us by tiles, R-MAT scale 22 edge factor 28 754 us streamed, 888 by tiles).  Rows of up to 24,576 streamed and the longer ones
+    // by tiles: an online walk of 10,000 x 8 on the scale-22 graph with 16 edges a vertex 222 -> 197 us, a build with 10 272 -> 264.
+    const uint64_t last = g->bin_edges[CLS_STREAM_LAST], narrow = g->bin_edges[CLS_STREAM] + last;
+    uint64_t wide = g->bin_edges[CLS_HOLD];
     for (int c = CLS_MW2 + 4; c <= CLS_MW2 + MERGE_MAX_NW - 2; ++c) wide += g->bin_edges[c];
-    const uint32_t longest = std::min(g->max_degree, g->bin_counts[CLS_STREAM] ? 65533u : 24576u);
-    const double stream_us = std::max(longest * 2.4e-3, wide * 6e-6), tiles_us = (wide - narrow) * 6e-6 + narrow * 13e-6;
-    p.t_all = (long long)narrow <= narrow_limit || (narrow_limit > 0 && tiles_us < stream_us) ? CLS_STREAM : CLS_STREAM_WIDE;
-    p.t_first = p.t_all == CLS_STREAM || narrow <= 65536ull * TILE ? CLS_STREAM : CLS_STREAM_WIDE;
-    uint64_t edges = 0;
+    auto us = [&](uint64_t streamed, uint32_t longest) {
+      return std::max(std::min(g->max_degree, longest) * 2.4e-3, (wide + streamed) * 6e-6) + (narrow - streamed) * 13e-6;
+    };
+    const double none_us = us(0, HOLD_MAX_DEG), last_us = us(last, 24576u), all_us = us(narrow, g->bin_counts[CLS_STREAM] ? 65533u : 24576u);
+    const bool some = narrow_limit > 0 && last > 0 && g->bin_counts[CLS_STREAM] > 0 && last_us < none_us;
+    if ((long long)narrow <= narrow_limit || (narrow_limit > 0 && std::min(none_us, some ? last_us : none_us) < all_us))
+      p.t_all = some ? CLS_STREAM : CLS_STREAM_LAST;
+    else
+      p.t_all = CLS_STREAM_WIDE;
+    p.t_first = p.t_all == CLS_STREAM_LAST || narrow <= 65536ull * TILE ? CLS_STREAM_LAST : p.t_all;
+    // Tiles of the rows that only small frontiers make tile by tile, then those of the others, from a bound of the former on: that is
+    // known without asking the device, and the places between are no tiles.
+    uint64_t edges = 0, early_edges = 0;
     for (int c = p.t_first; c <= CLS_HUGE; ++c) {
       p.n_trows += g->bin_counts[c];
       edges += g->bin_edges[c];
+      if (c < p.t_all) {
+        p.wide_row += g->bin_counts[c];
+        early_edges += g->bin_edges[c];
+      }
     }
     if (!p.n_trows) return SKY_OK;
-    const uint64_t bound = edges / TILE + 2ull * p.n_trows;
+    const uint64_t wide_tile = early_edges / TILE + 2ull * p.wide_row;
+    const uint64_t bound = wide_tile + (edges - early_edges) / TILE + 2ull * (p.n_trows - p.wide_row);
     if (bound >= (1ull << 31)) return fail(SKY_ERR_LIMIT, "the number of tiles has no usable bound");
+    p.wide_tile = (uint32_t)wide_tile;
     p.n_tiles = (uint32_t)bound;
     SKY_TRY(alloc((void**)&p.trows, (size_t)p.n_trows * sizeof(TiledRow)));
     const size_t nb = (size_t)p.n_tiles + p.n_trows;
@@ -652,18 +669,13 @@ int ensure_plan(sky_graph* g, CallDevice** first) {
     take(p.BH, nb);
     take(p.nfh, p.n_tiles);
     SKY_HIP(hipMemsetAsync(p.geom, 0, (size_t)p.n_tiles * sizeof(TileGeom), st));  // span 0: no such tile
-    hipLaunchKernelGGL(plan_rows_kernel, dim3(1), dim3(1024), 0, st, p.rows + p.start[p.t_first], p.n_trows, p.trows);
+    const RowRef* const list = p.rows + p.start[p.t_first];
+    if (p.wide_row) hipLaunchKernelGGL(plan_rows_kernel, dim3(1), dim3(1024), 0, st, list, p.wide_row, p.trows, 0u, 0u);
+    if (p.wide_row < p.n_trows)
+      hipLaunchKernelGGL(plan_rows_kernel, dim3(1), dim3(1024), 0, st, list + p.wide_row, p.n_trows - p.wide_row, p.trows, p.wide_row,
+                         p.wide_tile);
     hipLaunchKernelGGL(plan_tiles_kernel, dim3(p.n_trows), dim3(256), 0, st, p.trows, p.geom);
     SKY_HIP(hipGetLastError());
-    if (p.t_first != p.t_all) {  // the rows that every build makes tile by tile come after the others
-      p.wide_row = g->bin_counts[CLS_STREAM] + g->bin_counts[CLS_STREAM_LAST];
-      if (p.wide_row < p.n_trows) {
-        SKY_HIP(hipMemcpyAsync(&p.wide_tile, &p.trows[p.wide_row].tile0, 4, hipMemcpyDeviceToHost, st));
-        SKY_HIP(hipStreamSynchronize(st));
-      } else {
-        p.wide_tile = p.n_tiles;
-      }
-    }
     return SKY_OK;
   };
   const int rc = body();
@@ -733,10 +745,10 @@ bool block_takes_longer(const sky_graph* g, int tiled_from) {
 // (40,000 seeds 25 x 10 on the scale-22 graph with 32 edges a vertex, 1,800 streamed rows: 177 us, asked for 162; with 7,300 merges
 // beside them 297, asked for 330.)
 bool streams_by_queue(const sky_graph* g, int tiled_from, bool longer) {
-  if (tiled_from == CLS_STREAM) return false;
+  if (tiled_from == CLS_STREAM_LAST) return false;
   uint64_t merges = 0;
   for (int c = CLS_MW2 + (longer ? 6 : 4); c <= CLS_MW2 + 8; ++c) merges += g->bin_counts[c];
-  return merges <= (uint64_t)g->bin_counts[CLS_STREAM] + g->bin_counts[CLS_STREAM_LAST];
+  return merges <= (uint64_t)g->bin_counts[CLS_STREAM_LAST] + (tiled_from > CLS_STREAM ? g->bin_counts[CLS_STREAM] : 0u);
 }
 
 // The four launches, in order on the graph's stream.
@@ -830,7 +842,8 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   pair.add(SEC_P8, rows(CLS_MW2), 1, p.start[CLS_MW2]);
   pair.add(SEC_P6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
   wide.add(SEC_SCAN, n_trows, 1, 0);
-  if (p.t_all != CLS_STREAM) wide.add(SEC_STREAM, rows(CLS_STREAM) + rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM]);
+  if (p.t_all > CLS_STREAM) wide.add(SEC_STREAM, rows(CLS_STREAM), 1, p.start[CLS_STREAM]);
+  if (p.t_all > CLS_STREAM_LAST) wide.add(SEC_STREAM, rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM_LAST]);
   // Rows of 5118..8189 entries: streamed beside the others, where hold_row would spill, or, where they are enough for a launch,
   // HOLD_ALONE, by build_hold_kernel.
   const bool hold_alone = min_degree == 0 && rows(CLS_HOLD) >= HOLD_ALONE;  // behind the sweep, which notes when the call began
@@ -906,7 +919,8 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
   add(pair, SEC_P8, 1, CLS_MW2);
   add(pair, SEC_P6, 1, CLS_MW2_6);
   wide.add(SEC_SCAN, n_trows, 1, 0);
-  if (f.tiled_from != CLS_STREAM) add(wide, SEC_STREAM, 1, CLS_STREAM, 2);
+  if (f.tiled_from > CLS_STREAM) add(wide, SEC_STREAM, 1, CLS_STREAM);
+  if (f.tiled_from > CLS_STREAM_LAST) add(wide, SEC_STREAM, 1, CLS_STREAM_LAST);
   add(wide, SEC_STREAM, 1, CLS_HOLD);
   add(wide, SEC_B10, 1, CLS_MW2 + 7, 2);
   const bool longer = block_takes_longer(g, f.tiled_from);

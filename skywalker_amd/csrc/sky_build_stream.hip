@@ -3,14 +3,14 @@
 
 namespace sky {
 
-// The first n_first workgroups take the rows of first_list (the longest ones), the others those of vlist.
+// The first n_first workgroups take the rows of first_list (the longest ones), the others the n of vlist from the last one on.
 __global__ __launch_bounds__(ST_T, 4) void build_stream_kernel(const RowRef* __restrict__ first_list, uint32_t n_first,
-                                                            const RowRef* __restrict__ vlist,
+                                                            const RowRef* __restrict__ vlist, uint32_t n,
                                                             const float* __restrict__ wgt,
                                                             AliasEntry* __restrict__ table,
                                                             int8_t* __restrict__ valid) {
   __shared__ StreamLds lds;
-  const RowRef rr = blockIdx.x < n_first ? first_list[blockIdx.x] : vlist[blockIdx.x - n_first];
+  const RowRef rr = blockIdx.x < n_first ? first_list[blockIdx.x] : vlist[n - 1 - (blockIdx.x - n_first)];
   const bool ok = stream_row(rr, lds, wgt, table);
   if (threadIdx.x == 0) valid[rr.v] = ok ? 1 : 0;
 }
@@ -38,10 +38,10 @@ int build_rows_hold(sky_graph* g, const RowRef* rows, uint32_t n) {
 }
 
 // Builds the n_first rows of `first_list` and the n rows of `rows_list` (8190..STREAM_MAX_DEG entries each) in one
-// launch that starts with the former.
+// launch that starts with the former and goes through the latter backwards: their lists have the longer ones last.
 int build_rows_stream(sky_graph* g, const RowRef* first_list, uint32_t n_first, const RowRef* rows_list, uint32_t n) {
   if (n + n_first == 0) return SKY_OK;
-  hipLaunchKernelGGL(build_stream_kernel, dim3(n + n_first), dim3(ST_T), 0, g->stream, first_list, n_first, rows_list, g->adjwgt,
+  hipLaunchKernelGGL(build_stream_kernel, dim3(n + n_first), dim3(ST_T), 0, g->stream, first_list, n_first, rows_list, n, g->adjwgt,
                      g->table, g->valid);
   return SKY_OK;
 }

@@ -103,8 +103,8 @@ enum BuildClass : int {
   CLS_LDS_W6 = 19,  // deg 254..381     one wavefront per row, 6 slots per lane (the lower half of what CLS_LDS_W2 would hold)
   CLS_MW2_6 = 20,   // deg 510..765     two wavefronts per row, 6 slots per lane (the lower half of what CLS_MW2 would hold)
   CLS_HOLD = 21,         // deg 5118..8189     one workgroup holds the row in registers, its heavies in LDS
-  CLS_STREAM = 25,       // deg 24577..65533   one workgroup streams the row, a window of its heavies stays in LDS.
-  CLS_STREAM_LAST = 26,  // deg 8190..24576    Three classes built by one launch that takes the longest rows first
+  CLS_STREAM_LAST = 25,  // deg 8190..24576    one workgroup streams the row, a window of its heavies stays in LDS.
+  CLS_STREAM = 26,       // deg 24577..65533   Three classes built by one launch that takes the longest rows first
   CLS_STREAM_WIDE = 27,  // deg 65534..524287  and so
                     //                  does not end on its longest rows
   CLS_HUGE = 28,    // above            built tile by tile by the whole GPU

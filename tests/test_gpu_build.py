@@ -824,3 +824,29 @@ def test_short_rows_of_ranges_in_another_order(orc, V):
     g.free()
     oprob, oalias, ovalid = orc.alias_build(xadj, w)
     assert np.array_equal(prob.view(np.uint32), oprob.view(np.uint32)) and np.array_equal(alias, oalias) and np.array_equal(valid, ovalid)
+
+
+@pytest.mark.parametrize("seeds_n", [3000, 70000])
+def test_rows_of_8190_to_24576_entries_streamed_and_longer_ones_by_tiles(orc, seeds_n):
+    # in a build of all rows, in one of the rows of 8,190 entries and more, and in those of a small frontier (all by tiles) and a large one
+    from skywalker_amd import capi
+    rng = np.random.default_rng(61)
+    degs = list(rng.integers(8190, 24577, 270)) + [8189, 8190, 8191, 24576, 24577, 24578, 30000, 65533, 65534, 70001] + list(rng.integers(1, 200, 2000))
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal2")
+    seeds = (np.arange(seeds_n) % len(degs)).astype(np.uint32)
+    oprob, oalias, ovalid = orc.alias_build(xadj, w)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_full_build", 0)
+    d, sl, sampled, _ = g.sample_online(seeds, [1, 2, 2], 3)
+    got = d.to_host(), sl.to_host()
+    walk = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 9, 0.0, 5)
+    walked = walk[0].to_host(), walk[1].to_host()
+    g.build_tables()
+    prob, alias, valid = g.tables()
+    g.free()
+    assert np.array_equal(prob.view(np.uint32), oprob.view(np.uint32)) and np.array_equal(alias, oalias) and np.array_equal(valid, ovalid)
+    want = orc.sample_offline(xadj, adjncy, oprob, oalias, seeds, [1, 2, 2], 3)
+    assert np.array_equal(got[0], want[0].ravel()) and np.array_equal(got[1], want[1].ravel()) and sampled == want[2]
+    paths, lengths, steps = orc.walk_offline(xadj, adjncy, oprob, oalias, seeds, 9, 0.0, 5)
+    assert np.array_equal(walked[0], paths.ravel()) and np.array_equal(walked[1], lengths) and walk[2] == steps
