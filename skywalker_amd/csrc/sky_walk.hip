@@ -493,7 +493,8 @@ int walk_offline_noalloc(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32
 // (p = 4, 50,000 walkers x 40 on the scale-20 graph: 2 lanes 110 us, 8 191; 8,000 x 30 on the scale-22 graph: 2 59, 4 60, 32 102;
 // 500 x 60, scale 16: 2 89, 4 74, 64 77).
 // TR: where half of the trials fail or more, four are drawn at once, a lane each, and the first that is kept ends the step, or, of
-// two that depend on the previous row, the first is searched for and the other left to the next turn.  (One at a time / four, us: p = 1/4,
+// two that depend on the previous row, the first is searched for and the other left to the next turn; the first that ends the walk, if it
+// comes before, ends it.  (One at a time / four, us: p = 1/4,
 // q = 1: 500 x 60, scale 16, 224 / 121, 8,000 x 30, scale 22, 256 / 143, 50,000 x 40, scale 20, 371 / 273; p = 1/2, q = 2: 220 / 143, 275 / 178,
 // 490 / 396.  Where three in four are kept, p = 2, q = 1/2: 91 / 101, 120 / 134, 222 / 294; where the walkers alone fill the GPU, 150,000 x 30,
 // scale 22, p = 1/4, q = 1: 482 / 637.)
@@ -589,8 +590,11 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
           asm volatile("" : "+v"(mine.x), "+v"(mine.y), "+v"(mine.z), "+v"(mine.w));
         }
         const uint32_t cand = u24(ry) < e.prob ? col : e.alias;
-        if (cand == SKY_INVALID) break;  // a row without weight: every entry says so
-        uint32_t next = adjncy[off + cand];
+        // The walk ends at a row without weight.  A table from outside may keep the column in some of its entries, or for some numbers: in
+        // a turn of several trials a lane then ends the walk while its neighbours do not, and the group decides below.
+        const bool ends = cand == SKY_INVALID;
+        if (TR == 1 && ends) break;
+        uint32_t next = adjncy[off + (TR > 1 && ends ? col : cand)];
         x = *reinterpret_cast<const bounds2u*>(xadj + next);
         bool keep = s == 0 || t + my >= 65536u, ask = false;
         const float need = u24(rw) * fmax;
@@ -603,27 +607,28 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
         if (TR == 1) {
           if (ask) keep = need < (group_row_has<G>(adjncy + prev_off, prev_deg, next, x0) ? 1.0f : fq);
         } else {
-          // bit j: trial t + j is kept; bit 8 + j: that depends on the previous row
-          uint32_t b = (keep ? 1u : ask ? 256u : 0u) << my;
+          // bit j: trial t + j is kept; bit 8 + j: that depends on the previous row; bit 16 + j: it ends the walk
+          uint32_t b = (ends ? 65536u : keep ? 1u : ask ? 256u : 0u) << my;
           b |= dpp0<DPP_QUAD_XOR1, 0xF>(b);
           b |= dpp0<DPP_QUAD_XOR2, 0xF>(b);
-          const uint32_t kept = b & 255u;
-          uint32_t left = kept | b >> 8 | 1u << TR;
+          const uint32_t kept = b & 255u, asked = (b >> 8) & 255u, ended = b >> 16;
+          uint32_t left = kept | asked | ended | 1u << TR;
           went = (uint32_t)__ffs((int)left) - 1u;
-          if (went < TR && !((kept >> went) & 1u)) {
+          if ((asked >> went) & 1u) {
             const int l = base + (int)went;
             const uint32_t key = (uint32_t)__shfl((int)next, l, 64);
             const float limit = __shfl(need, l, 64);
             if (!(limit < (group_row_has<G>(adjncy + prev_off, prev_deg, key, x0) ? 1.0f : fq))) {  // on to the next one that may be kept
               left &= left - 1u;
               went = (uint32_t)__ffs((int)left) - 1u;
-              keep = went < TR && ((kept >> went) & 1u);
+              keep = (kept >> went) & 1u;
             } else {
               keep = true;
             }
           } else {
-            keep = went < TR;
+            keep = (kept >> went) & 1u;
           }
+          if ((ended >> went) & 1u) break;
           if (keep) {
             const int l = base + (int)went;
             next = (uint32_t)__shfl((int)next, l, 64);

@@ -247,6 +247,33 @@ def test_node2vec_trials_by_how_many_are_kept(orc, walkers, p, q):
     g.free()
 
 
+@pytest.mark.parametrize("walkers", [1, 700, 7168, 7169, 14337, 28673, 57344, 57345])
+@pytest.mark.parametrize("p,q", [(0.25, 1.0), (0.5, 2.0), (0.0625, 8.0), (2.0, 0.5), (1.0, 1.0)])
+def test_node2vec_rejection_on_an_uploaded_table_whose_rows_without_weight_keep_some_columns(orc, walkers, p, q):
+    # sky_alias_upload takes any prob in [0, 1] in a row flagged invalid: a trial that keeps its column goes on from there, and
+    # the first one that does not ends the walk if no earlier trial of its step was kept; one trial a turn and four, 64 lanes a walker to 4
+    from skywalker_amd import capi
+    rng = np.random.default_rng(17)
+    xadj, adjncy = orc.rmat_csr(11, 12, 35)
+    w = orc.gen_weights(orc.W_LOGNORMAL, 35, len(adjncy), 0.0, 2.0)
+    V = len(xadj) - 1
+    for v in np.flatnonzero(rng.random(V) < 0.3):
+        w[xadj[v]:xadj[v + 1]] = 0.0
+    prob, alias, valid = orc.alias_build(xadj, w)
+    free = alias == 0xFFFFFFFF
+    assert free.sum() > len(w) // 8
+    prob[free] = rng.choice(np.float32([0.0, 0.3, 0.7, 0.95, 1.0]), free.sum())
+    seeds = orc.gen_seeds(6, V + 1, walkers)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.upload_tables(prob, alias, valid)
+    for stop, length in ((0.0, 12), (0.02, 30)):
+        paths, lengths, sampled, _ = g.walk_online(capi.BIAS_NODE2VEC_REJECT, p, q, seeds, length, stop, 19)
+        want = orc.walk_node2vec_reject(xadj, adjncy, prob, alias, p, q, seeds, length, stop, 19)
+        assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host((walkers, length + 1)), want[0])
+        assert sampled == want[2]
+    g.free()
+
+
 def test_read_once_gathers_give_the_same_paths(orc):
     from skywalker_amd import capi
     xadj, adjncy = orc.rmat_csr(12, 16, 36)
