@@ -887,7 +887,9 @@ int frontier_lists(sky_graph* g, const BuildPlan& p, uint32_t n_upper, sky_graph
   return SKY_OK;
 }
 
-int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uint32_t* counts, const uint32_t* bitmap,
+__global__ void clear_taken_kernel(uint32_t* taken) { *taken = 0; }
+
+int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uint32_t* counts, bool again, const uint32_t* bitmap,
                    uint32_t* built) {
   g->has_walk_index = false;
   FusedArgs base = common_args(g, p, f.tiled_from);
@@ -924,7 +926,10 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
   add(wide, SEC_STREAM, 1, CLS_HOLD);
   add(wide, SEC_B10, 1, CLS_MW2 + 7, 2);
   const bool longer = block_takes_longer(g, f.tiled_from);
-  if (streams_by_queue(g, f.tiled_from, longer)) wide.a.next = counts + CLS_COUNT;
+  if (streams_by_queue(g, f.tiled_from, longer)) {
+    wide.a.next = counts + CLS_COUNT;
+    if (again) hipLaunchKernelGGL(clear_taken_kernel, dim3(1), dim3(1), 0, g->stream, wide.a.next);
+  }
   if (longer) {
     add(wide, SEC_B8, 1, CLS_MW2 + 6);
   } else {

@@ -624,6 +624,7 @@ struct SampleSession {
   // session build the row again, from weights that its caller had not supplied.
   uint32_t *list_counts = nullptr, *front_counts = nullptr, *built = nullptr;
   FrontierLists front;
+  std::vector<char> made;  // by hop: its rows have been built (a session's caller may have a hop built and drawn once more)
   // The plan of the graph when the call began.  Another call between the steps of a session may make the graph a new one, when
   // a knob that decides how long rows are built has changed.
   std::shared_ptr<BuildPlan> plan;
@@ -694,6 +695,7 @@ struct SampleSession {
     width.assign(hops, 0);
     off.assign(hops, 0);
     loff.assign(hops, 0);
+    made.assign(hops, 0);
     uint64_t wd = 1;
     for (uint32_t h = 0; h < hops; ++h) {
       wd *= fanout[h];
@@ -773,8 +775,9 @@ struct SampleSession {
     if (!online || !N || !frontier_upper) return SKY_OK;
     float* const own = g->adjwgt;
     if (weights) g->adjwgt = const_cast<float*>(weights);  // the build only reads it
-    const int rc = dev_sized ? build_frontier(g, *plan, front, front_counts + h * FRONTIER_WORDS, bitmap, built)
+    const int rc = dev_sized ? build_frontier(g, *plan, front, front_counts + h * FRONTIER_WORDS, made[h], bitmap, built)
                              : build_rows(g, list, frontier_count, nullptr);
+    made[h] = 1;
     g->adjwgt = own;
     return rc;
   }

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from helpers import chi_square_p, graph_from_degrees
+from helpers import chi_square_p, graph_from_degrees, weights
 
 pytestmark = pytest.mark.gpu
 
@@ -528,6 +528,33 @@ def test_row_lists_made_anew_leave_the_flags_of_a_session_alone(orc):
     sampled, _ = session_end(capi, s[0])
     assert np.array_equal(s[4].to_host((16, slen)), want[1]) and np.array_equal(s[3].to_host((16, lps)), want[0])
     assert sampled == want[2] == 8
+    g.free()
+
+
+def test_hop_of_a_session_taken_once_more(orc):
+    # a frontier of more than 65,536 rows, 1,100 of which are streamed by the workgroup that is first free: the second time, from other
+    # weights, every one of them is built again
+    import ctypes as C
+    from skywalker_amd import capi
+    rng = np.random.default_rng(85)
+    degs = list(rng.integers(8190, 9500, 1100)) + list(rng.integers(1, 4, 70000))
+    rng.shuffle(degs)
+    xadj = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    V, E, fan = len(degs), int(xadj[-1]), [1, 3]
+    adjncy = rng.integers(0, V, E, dtype=np.uint32)
+    w = [weights(E, rng, "lognormal2") for _ in range(2)]
+    seeds = rng.permutation(V).astype(np.uint32)
+    lps, slen = capi.sample_layout(fan)
+    g = capi.Graph.upload(xadj, adjncy, w[0])
+    s = open_session(capi, g, seeds, fan, 71)
+    session_frontier(capi, s[0], 0)
+    for x in w:
+        w_d = capi.DeviceArray.from_host(x)
+        capi._ck(capi.lib().sky_sample_session_hop(s[0], C.c_uint32(0), w_d.ptr))
+        capi.synchronize()
+    session_end(capi, s[0])
+    want = orc.sample_online(xadj, adjncy, w[1], seeds, fan, 71)
+    assert np.array_equal(s[4].to_host((V, slen)), want[1]) and np.array_equal(s[3].to_host((V, lps)), want[0])
     g.free()
 
 
