@@ -268,8 +268,13 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      faster.  The paths are the same.
  *      "online_device_sized" (default 1): sky_sample_online builds the rows of a frontier without the host ever
  *      learning how many they are: the sizes of its degree classes stay on the device, every build kernel finds its rows through them, and the call waits for
- *      the device only once, at its end; hops whose rows are few are drawn from the weights and build none.  0 makes the host read the size of every frontier and size the launches
+ *      the device only once, at its end (or after its first hop as well: "online_direct").  0 makes the host read the size of every frontier and size the launches
  *      exactly, which waits twice per hop.  Same results.
+ *      "online_direct" (default -1): sky_sample_online evaluates the draws of a hop from the weights and builds none of its
+ *      rows.  -1: the first hop of up to 8,192 start vertices, or of 40,960 where there is no other, and all hops where later ones
+ *      are expected to lead to few entries; a hop whose rows turn out to be long, or to hold many entries together, is drawn from
+ *      tables after all.  0: never.  1: every hop, whatever it meets.  Draws with replacement and online_device_sized only.  Same
+ *      results.
  *      "walk_compact_every" (default 0): k > 0 makes sky_walk_offline run k steps per launch and hand the next
  *      launch the list of walkers that are still walking (the reference's walker queue,
  *      include/sampler_result.cuh:646-669), so that walkers that have stopped no longer hold a lane; 0 keeps every

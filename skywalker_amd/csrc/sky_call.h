@@ -14,14 +14,16 @@ namespace sky {
 struct CallDevice {
   unsigned long long start;    // wall clock of the first kernel
   unsigned long long sampled;  // edges sampled so far
-  unsigned long long pad[6];
+  unsigned long long entries, arrived, refused;  // sample_check_kernel; the last is left as it is
+  unsigned long long pad[3];
 };
 // Pinned host words of a call, written by the end kernel: each carries the number of the call in its upper 16 bits, so that the
 // host knows which of them has arrived and neither waits for the other on its way over PCIe (results first, then, released, a
 // number of their own: a round trip more, 0.4 to 0.8 us of a call of 15 to 30).
 struct CallHost {
   unsigned long long sampled, ticks;
-  unsigned long long pad[6];
+  unsigned long long answer;  // in the course of a call, with a number of its own (call_ask)
+  unsigned long long pad[5];
 };
 constexpr int CALL_VALUE_BITS = 48;  // 2^48 edges fill the GPU's memory a thousand times over; 2^48 ticks of 10 ns are a month
 static_assert(sizeof(CallDevice) == 64 && sizeof(CallHost) == 64, "one cache line each");
@@ -30,7 +32,7 @@ static_assert(sizeof(CallDevice) == 64 && sizeof(CallHost) == 64, "one cache lin
 struct CallWords {
   CallDevice* dev = nullptr;
   CallHost* host = nullptr;
-  unsigned long long seq = 0;
+  unsigned long long seq = 0, asked = 0;  // numbers of the last end and of the last question
   int khz = 0;
   bool dirty = false;  // a call has begun and not ended well: its device words may not be zero
 };
@@ -39,7 +41,9 @@ struct CallWords {
 __device__ __forceinline__ void call_stamp(CallDevice* call) {
   if (call && blockIdx.x == 0 && threadIdx.x == 0) call->start = wall_clock64();
 }
-// Last statement of the call's last kernel, by one thread that has seen every other thread's contribution.
+// Last statement of the call's last kernel, by one thread that has seen every other thread's contribution.  The host may go on
+// before the device words are zero again; who uses them next is a kernel behind this one on the device's null stream, whichever graph
+// it belongs to.
 __device__ __forceinline__ void call_report(CallDevice* call, CallHost* host, unsigned long long seq,
                                             unsigned long long sampled) {
   const unsigned long long start = call->start, ticks = start ? wall_clock64() - start : 0;  // 0: the call had nothing to launch
@@ -55,6 +59,13 @@ int call_begin(sky_graph* g, CallWords* w, CallDevice** call);
 // Enqueues the end kernel behind what the call has put on the graph's stream, waits for it and hands out the results.
 // Outputs may be null.  `counts` (n of them, device, may be null) are added to the sampled edges.
 int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);
+// The host's questions in the course of a call: a kernel answers question number call_ask(w) by call_answer, and call_answered waits
+// for it.
+inline unsigned long long call_ask(CallWords* w) { return ++w->asked; }
+__device__ __forceinline__ void call_answer(CallHost* host, unsigned long long number, unsigned long long value) {
+  __hip_atomic_store(&host->answer, value | number << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+int call_answered(sky_graph* g, CallWords* w, unsigned long long* value);
 // With the graph's own words.
 int call_begin(sky_graph* g, CallDevice** call);
 int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);

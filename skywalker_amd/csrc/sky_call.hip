@@ -1,5 +1,6 @@
 // End of a call: results and completion through pinned host words (sky_call.h).
 #include <chrono>
+#include <cstddef>
 #include <mutex>
 #include <vector>
 
@@ -89,6 +90,7 @@ int take_words(int device, CallWords* w) {
   w->host = use->host + k;
   w->khz = use->khz;
   w->seq = use->host[k].sampled >> CALL_VALUE_BITS;  // not the next call's
+  w->asked = use->host[k].answer >> CALL_VALUE_BITS;
   return SKY_OK;
 }
 }  // namespace
@@ -131,6 +133,39 @@ constexpr uint64_t END_COUNTS = 32768;
 // five microseconds, and one whose kernels fault ends with the runtime's error instead of polling for ever.
 constexpr auto POLL_FOR = std::chrono::microseconds(3000);
 
+// Waits until n host words from `from` on carry the number `seq`, and takes their values.
+static int take_values(hipStream_t st, const unsigned long long* from, int n, unsigned long long seq, unsigned long long* values) {
+  constexpr unsigned long long VALUE = (1ull << CALL_VALUE_BITS) - 1;
+  auto there = [&] {
+    unsigned long long other = 0;
+    for (int i = 0; i < n; ++i) {
+      const unsigned long long x = __atomic_load_n(from + i, __ATOMIC_ACQUIRE);
+      other |= (x ^ seq << CALL_VALUE_BITS) & ~VALUE;
+      values[i] = x & VALUE;
+    }
+    return !other;
+  };
+  bool done = there();
+  if (!done) {
+    const auto t0 = std::chrono::steady_clock::now();
+    do {
+      for (int k = 0; k < 64 && !done; ++k) {
+        __builtin_ia32_pause();
+        done = there();
+      }
+    } while (!done && std::chrono::steady_clock::now() - t0 < POLL_FOR);
+  }
+  if (!done) {
+    SKY_HIP(hipStreamSynchronize(st));
+    if (!there()) return fail(SKY_ERR_HIP, "the call's end was not reported");
+  }
+  return SKY_OK;
+}
+
+int call_answered(sky_graph* g, CallWords* w, unsigned long long* value) {
+  return take_values(g->stream, &w->host->answer, 1, w->asked, value);
+}
+
 int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
   hipStream_t st = g->stream;
   if (n > END_COUNTS) {
@@ -142,31 +177,12 @@ int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, con
   hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, st, w->dev, w->host, seq, counts,
                      (uint32_t)n);
   SKY_HIP(hipGetLastError());
+  static_assert(offsetof(CallHost, ticks) == offsetof(CallHost, sampled) + 8, "taken together");
   unsigned long long words[2];
-  auto ended = [&] {
-    words[0] = __atomic_load_n(&w->host->sampled, __ATOMIC_ACQUIRE);
-    words[1] = __atomic_load_n(&w->host->ticks, __ATOMIC_ACQUIRE);
-    constexpr unsigned long long NUMBER = 0xFFFFull << CALL_VALUE_BITS;
-    return !(((words[0] ^ seq << CALL_VALUE_BITS) | (words[1] ^ seq << CALL_VALUE_BITS)) & NUMBER);
-  };
-  bool done = ended();
-  if (!done) {
-    const auto t0 = std::chrono::steady_clock::now();
-    do {
-      for (int k = 0; k < 64 && !done; ++k) {
-        __builtin_ia32_pause();
-        done = ended();
-      }
-    } while (!done && std::chrono::steady_clock::now() - t0 < POLL_FOR);
-  }
-  if (!done) {
-    SKY_HIP(hipStreamSynchronize(st));
-    if (!ended()) return fail(SKY_ERR_HIP, "the call's end was not reported");
-  }
+  SKY_TRY(take_values(st, &w->host->sampled, 2, seq, words));
   w->dirty = false;
-  constexpr unsigned long long VALUE = (1ull << CALL_VALUE_BITS) - 1;
-  if (sampled) *sampled = words[0] & VALUE;
-  if (seconds) *seconds = (double)(words[1] & VALUE) / ((double)w->khz * 1e3);
+  if (sampled) *sampled = words[0];
+  if (seconds) *seconds = (double)words[1] / ((double)w->khz * 1e3);
   return SKY_OK;
 }
 int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {

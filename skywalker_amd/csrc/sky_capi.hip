@@ -65,6 +65,7 @@ long long g_option_value[OPT_COUNT] = {
     0,                                     // walk_compact_every
     -1,                                    // online_full_build: by estimate
     1,                                     // online_device_sized
+    -1,                                    // online_direct: by the rows that are met
 };
 }  // namespace sky
 
@@ -543,6 +544,7 @@ static const OptionSpec g_option_spec[OPT_COUNT] = {
     {"walk_compact_every", 0, 1ll << 31},
     {"online_full_build", -1, 1},
     {"online_device_sized", 0, 1},
+    {"online_direct", -1, 1},
 };
 static int parse_option(const char* who, const char* name, long value, int* index, long long* stored) {
   if (!name) return fail(SKY_ERR_ARG, std::string(who) + ": null name");

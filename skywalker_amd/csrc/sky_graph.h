@@ -21,6 +21,7 @@ enum SkyOpt : int {
   OPT_WALK_COMPACT_EVERY,
   OPT_ONLINE_FULL_BUILD,
   OPT_ONLINE_DEVICE_SIZED,
+  OPT_ONLINE_DIRECT,
   OPT_COUNT
 };
 

@@ -15,6 +15,7 @@
 // kernels as the offline build (into the graph's table storage), then samples the hop; or, where that takes less (choose_direct),
 // evaluates the draws of a hop from the weights.
 #include <algorithm>
+#include <functional>
 #include <memory>
 #include <vector>
 
@@ -51,6 +52,7 @@ struct SampleArgs {
   uint32_t lanes;      // lanes per start vertex (a power of two; 64 when parts > 1)
   uint64_t first, N;   // start vertices [first, N)
   CallDevice* call;    // stamped by the call's first kernel (null: another kernel was)
+  CallDevice* words;   // without tables: where a hop is refused (null: none is)
   uint64_t seed;
   HopGeom hop[SAMPLE_HOPS];
 };
@@ -295,16 +297,82 @@ __device__ __forceinline__ uint32_t direct_children(const SampleArgs& a, const H
   return g.k;
 }
 
+constexpr int DIRECT_T = 512;
+constexpr uint32_t DIRECT_LONG = 1024;
+
+// Whether a hop is drawn from the weights after all.  Its parents are the caller's: well connected vertices, or one of them again and
+// again, whose rows are swept for every slot where a build makes each once, and long ones with the whole GPU.  Refused
+// is a hop with a workgroup of more than `most_chain` entries in long rows, counting DIRECT_PER_ROW more for each (they follow one another,
+// 1.1 ns each), or with more than `budget` entries altogether (18 ps each).  The answer reaches the host while the draws run, which are
+// 4 to 8 us later for it.  (All hops from tables / from the weights whatever they meet / by this rule, us.  8,192 seeds x 20, the scale-16
+// graph, any vertices 55 / 38 / 44, the first 8,192 64 / 106 / 73, ends of edges 67 / 127 / 78, one vertex of 12,938 entries 138 / 432 / 147;
+// the scale-22 graph with 32 edges a vertex 91 / 46 / 53, 221 / 989 / 231, 406 / 846 / 399, one of 319,795 161 / 7,192 / 184.  1,024 x 10 x
+// 10 there 360 / 332 / 323, 537 / 1,255 / 522, 564 / 835 / 539, 508 / 3,626 / 495.)
+constexpr int CHECK_T = 256, CHECK_U = 4;
+constexpr uint32_t DIRECT_CHAIN = 32768, DIRECT_PER_ROW = 4096;
+constexpr unsigned long long DIRECT_TOO_LONG = 1ull << 54;  // above any sum of the entries, 2^21 slots of less than 2^32
+__global__ __launch_bounds__(CHECK_T) void sample_check_kernel(SampleArgs a, uint64_t budget, uint32_t most_chain,
+                                                               CallHost* __restrict__ host, unsigned long long number) {
+  __shared__ unsigned long long s_sum[CHECK_T / 64];
+  __shared__ uint32_t s_chain[CHECK_T / 64];
+  call_stamp(a.call);
+  const HopGeom& g = a.hop[a.h0];
+  const uint64_t slots = a.N * g.width;
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t v[CHECK_U], d[CHECK_U];
+#pragma unroll
+  for (int u = 0; u < CHECK_U; ++u) {
+    const uint64_t slot = ((uint64_t)blockIdx.x * CHECK_U + u) * CHECK_T + threadIdx.x, si = slot / g.width;
+    v[u] = slot < slots ? parent_of(a, g, si, (uint32_t)(slot - si * g.width)) : 0xFFFFFFFFu;
+  }
+#pragma unroll
+  for (int u = 0; u < CHECK_U; ++u) d[u] = v[u] < a.V ? a.xadj[v[u] + 1] - a.xadj[v[u]] : 0u;
+  unsigned long long sum = 0;
+  uint32_t chain = 0;  // of the longest of the workgroups whose slots these are
+#pragma unroll
+  for (int u = 0; u < CHECK_U; ++u) {
+    sum += d[u];
+    uint32_t c = d[u] > DIRECT_LONG ? min(d[u], most_chain) + DIRECT_PER_ROW : 0u;
+#pragma unroll
+    for (int m = 1; m < DIRECT_T / 64; m *= 2) c += (uint32_t)__shfl_xor((int)c, m, 64);
+    chain = max(chain, c);
+  }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    sum += shfl_xor_u64(sum, m);
+    chain = max(chain, (uint32_t)__shfl_xor((int)chain, m, 64));
+  }
+  if (lane == 0) {
+    s_sum[wave] = sum;
+    s_chain[wave] = chain;
+  }
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int w = 1; w < CHECK_T / 64; ++w) {
+    sum += s_sum[w];
+    chain = max(chain, s_chain[w]);
+  }
+  if (chain > most_chain) sum += DIRECT_TOO_LONG;
+  if (gridDim.x > 1) {
+    atomicAdd(&a.words->entries, sum);
+    __threadfence();
+    if (atomicAdd(&a.words->arrived, 1ull) != gridDim.x - 1) return;
+    sum = atomicExch(&a.words->entries, 0ull);
+    a.words->arrived = 0;
+  }
+  a.words->refused = sum > budget;
+  call_answer(host, number, sum > budget);
+}
+
 // A wavefront a slot; the slots of a workgroup whose rows are too long for one are left to all eight together.  What bounds it is the chain
 // of some six dependent loads of a slot and the longest row (1,676 seeds x 20 on the scale-22 graph, the longest row met of 100,000 entries:
 // 382 us with a wavefront a slot throughout, 106 with four, 77 like this).
-constexpr int DIRECT_T = 512;
-constexpr uint32_t DIRECT_LONG = 1024;
 __global__ __launch_bounds__(DIRECT_T) void sample_direct_kernel(SampleArgs a, const float* __restrict__ wgt) {
   constexpr int NW = DIRECT_T / 64;
   __shared__ __align__(16) unsigned char smem[std::max(sizeof(DirectLds<DIRECT_T>), NW * sizeof(DirectLds<64>))];
   __shared__ uint32_t s_off[NW], s_d[NW];
   call_stamp(a.call);
+  const bool refused = a.words && a.words->refused;
   const HopGeom& g = a.hop[a.h0];
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   auto done = [&](uint64_t si, uint32_t s, uint32_t cnt) {
@@ -327,6 +395,7 @@ __global__ __launch_bounds__(DIRECT_T) void sample_direct_kernel(SampleArgs a, c
       }
       off = (uint32_t)__builtin_amdgcn_readfirstlane((int)off);
       d = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);
+      if (refused) return;  // the whole workgroup, here or below
       if (d <= DIRECT_LONG) {
         const uint32_t cnt = d ? direct_children<64>(a, g, wgt, si, s, off, d, lane, reinterpret_cast<DirectLds<64>*>(smem)[wave]) : 0u;
         if (lane == 0) done(si, s, cnt);
@@ -337,6 +406,7 @@ __global__ __launch_bounds__(DIRECT_T) void sample_direct_kernel(SampleArgs a, c
       s_d[wave] = d > DIRECT_LONG ? d : 0u;
     }
   }
+  if (refused) return;
   __syncthreads();
   for (uint32_t w = 0; w < NW; ++w) {
     const uint32_t d = s_d[w];
@@ -628,7 +698,9 @@ struct SampleSession {
   // The plan of the graph when the call began.  Another call between the steps of a session may make the graph a new one, when
   // a knob that decides how long rows are built has changed.
   std::shared_ptr<BuildPlan> plan;
+  std::vector<uint64_t> budget;  // by hop without tables: entries beyond which it is refused (0: never)
   bool stamped = false;          // the call's first kernel is on its way
+  std::function<void()> init;    // enqueues sample_init_kernel, for an online call that is not direct throughout
   bool want_list = false;        // the caller is to see the frontier as a list of vertices
   uint32_t* totals = nullptr;    // children of each start vertex, when the kernels add them up
   uint32_t frontier_upper = 0;   // most rows the last frontier can hold
@@ -737,13 +809,34 @@ struct SampleSession {
     if (N && one_workgroup()) SKY_TRY(get(sky_graph::POOL_TOTALS, (size_t)N * 4, (void**)&totals));
     const uint64_t lengths = want_list ? (uint64_t)N * slen : 0;  // to be cleared
     const uint64_t items = std::max<uint64_t>(std::max(std::max(N, bits), 1u), lengths);  // an empty graph has counters too
-    if (dev_sized && !want_list && !distinct && N) choose_direct();
-    const bool init = online && (direct.empty() || std::find(direct.begin(), direct.end(), 0) != direct.end());
-    stamped = init;
-    if (init)
+    init = [=] {
       hipLaunchKernelGGL(sample_init_kernel, dim3((uint32_t)std::min<uint64_t>((items + 255) / 256, 2048)), dim3(256), 0, st, seeds,
                          N, lps, data, bitmap, bits, list_counts, counters, lengths ? sample_lengths : nullptr, lengths,
-                         want_list ? totals : nullptr, call);
+                         want_list ? totals : nullptr, stamped ? nullptr : call);
+      stamped = true;
+    };
+    if (dev_sized && !want_list && !distinct && N) choose_direct();
+    if (online && !all_direct()) init();
+    return SKY_OK;
+  }
+  bool is_direct(uint32_t h) const { return !direct.empty() && direct[h]; }
+  bool all_direct() const { return !direct.empty() && std::find(direct.begin(), direct.end(), 0) == direct.end(); }
+
+  // All hops in turn.
+  int run() {
+    if (!online && totals) return draw(0, hops - 1);
+    for (uint32_t h = 0; h + 1 < hops; ++h) {
+      SKY_TRY(frontier(h));
+      SKY_TRY(build(h, nullptr));
+      SKY_TRY(draw(h, h + 1));
+      if (!is_direct(h) || !budget[h]) continue;
+      unsigned long long refused = 0;
+      SKY_TRY(call_answered(g, words(), &refused));
+      if (!refused) continue;
+      if (all_direct()) init();
+      direct.clear();  // the hop once more, with tables, and those behind it
+      --h;
+    }
     return SKY_OK;
   }
 
@@ -751,7 +844,7 @@ struct SampleSession {
   // the hop's device word d_count (and is read by the host only when the build needs it there).
   int frontier(uint32_t h) {
     frontier_upper = frontier_count = 0;
-    if (!online || !N || (!direct.empty() && direct[h])) return SKY_OK;
+    if (!online || !N || is_direct(h)) return SKY_OK;
     hipStream_t st = g->stream;
     const HopGeom hg = geom(h);
     const uint64_t slots = (uint64_t)N * hg.width;
@@ -795,7 +888,7 @@ struct SampleSession {
 
   int draw(uint32_t h0, uint32_t h1) {
     if (!N) return SKY_OK;
-    if (!direct.empty() && direct[h0]) return draw_direct(h0);
+    if (is_direct(h0)) return draw_direct(h0);
     hipStream_t st = g->stream;
     SampleArgs a = {};
     a.xadj = g->xadj;
@@ -846,23 +939,37 @@ struct SampleSession {
     return SKY_OK;
   }
 
-  // Which hops do without tables.  The six launches that collect, build and draw take 50 us even of a few rows; start vertices are any
-  // vertices, whose rows are short, and a draw from the weights of one costs little more than the draw from its table.  Of a call of
-  // several hops only up to DIRECT_FEW of them, and no more than there are vertices: rows built for the first hop are met again at the
-  // second.  (Built / direct, us: 10,000 seeds x 20 on the scale-14 graph 66 / 48, 39,000 on the scale-22 graph 125 / 92; 700 x 5 x 3, scale 13,
+  // Which hops do without tables, unless their rows turn out to be long (sample_check_kernel).  The six launches that collect, build and
+  // draw take 50 us even of a few rows; start vertices are mostly any vertices, whose rows are short, and a draw from the weights of one
+  // costs little more than the draw from its table.  Up to DIRECT_SEEDS of them (40,000 x 20 on the scale-16 graph 81 / 79, 60,000 86 / 98);
+  // of a call of several hops only up to DIRECT_FEW, and no more than there are vertices: rows built for the first hop are met again at
+  // the second.  (Built / direct, us: 10,000 seeds x 20 on the scale-14 graph 66 / 48, 39,000 on the scale-22 graph 125 / 92; 700 x 5 x 3, scale 13,
   // 103 / 91; 3,000 x 5 x 3, scale 16, 134 / 115; 401 x 10 x 10, scale 22, 299 / 249; 15,900 x 5 x 3 on 4,096 vertices 111 / 145, 36,000 x
   // 5 x 3 on the scale-20 graph 402 / 450.)  Later hops lead to long rows, again and again: the call does without tables altogether where they
   // come to few entries and none is very long (70 x 5 x 3, scale 18, 97 / 68; 200 x 25 x 10, scale 15, 106 / 75; 400 x 10 x 10 with 3.4 M
   // entries, scale 14, 107 / 122; 100 x 5 x 3 on the scale-20 graph, whose longest row has 69,000 entries, 107 / 145).
-  static constexpr uint32_t DIRECT_SEEDS = 65536, DIRECT_FEW = 8192, DIRECT_ROW = 52000;
-  static constexpr double DIRECT_ENTRIES = 2e6;
+  static constexpr uint32_t DIRECT_SEEDS = 40960, DIRECT_FEW = 8192, DIRECT_ROW = 52000;
+  static constexpr double DIRECT_ENTRIES = 2e6, DIRECT_SPARE = 1e6;
   void choose_direct() {
+    const long long mode = option(g, OPT_ONLINE_DIRECT);
+    if (mode == 0) return;
+    budget.assign(hops - 1, 0);
+    if (mode > 0) return direct.assign(hops - 1, 1);
     if (N > DIRECT_SEEDS || (hops > 2 && N > std::min(DIRECT_FEW, g->V))) return;
     double mean = 0;  // entries of the row that an edge leads to
     for (int c = CLS_G2; c < CLS_COUNT; ++c)
       if (g->bin_counts[c]) mean += (double)g->bin_edges[c] * g->bin_edges[c] / g->bin_counts[c] / std::max(1u, g->E);
     bool all = g->max_degree <= DIRECT_ROW;
-    for (uint32_t h = 1; h + 1 < hops; ++h) all = all && (double)N * width[h] * mean <= DIRECT_ENTRIES;
+    auto limit = [&](uint32_t h, double entries) {  // rows that are all short and few are not looked at
+      const uint64_t most = (uint64_t)(DIRECT_SPARE + entries);
+      if (g->max_degree > DIRECT_LONG || (double)N * width[h] * g->max_degree > (double)most) budget[h] = most;
+    };
+    limit(0, (double)N * g->E / std::max(1u, g->V));
+    for (uint32_t h = 1; h + 1 < hops; ++h) {
+      const double entries = (double)N * width[h] * std::max(1.0, mean);
+      all = all && entries <= DIRECT_ENTRIES;
+      limit(h, entries);
+    }
     direct.assign(hops - 1, all);
     direct[0] = 1;
   }
@@ -872,6 +979,7 @@ struct SampleSession {
     a.adjncy = g->adjncy;
     a.seeds = h == 0 ? seeds : nullptr;
     a.call = stamped ? nullptr : call;
+    a.words = budget[h] ? words()->dev : nullptr;
     stamped = true;
     a.data = data;
     a.sl = sample_lengths;
@@ -884,6 +992,12 @@ struct SampleSession {
     a.N = N;
     constexpr uint64_t PER = DIRECT_T / 64;
     const uint64_t slots = (uint64_t)N * width[h], most = PER << 22;  // slots of one launch: below 2^32 threads
+    if (budget[h]) {  // of few enough slots, by choose_direct, for one launch
+      const uint32_t chain = DIRECT_CHAIN + std::min(plan->n_tiles, 65536u);  // a build passes over the plan's tiles, 1.1 ns each too
+      hipLaunchKernelGGL(sample_check_kernel, dim3((uint32_t)((slots + CHECK_T * CHECK_U - 1) / (CHECK_T * CHECK_U))), dim3(CHECK_T), 0,
+                         g->stream, a, budget[h], chain, words()->host, call_ask(words()));
+      a.call = nullptr;
+    }
     for (a.first = 0; a.first < slots; a.first += most) {
       const dim3 grid((uint32_t)((std::min<uint64_t>(most, slots - a.first) + PER - 1) / PER));
       hipLaunchKernelGGL(sample_direct_kernel, grid, dim3(DIRECT_T), 0, g->stream, a, g->adjwgt);
@@ -902,15 +1016,7 @@ int sample_khop(sky_graph* g, bool online, const uint32_t* seeds, uint32_t N, co
                 uint64_t seed, uint32_t* data, uint32_t* sample_lengths, uint64_t* sampled, double* seconds) {
   SampleSession s(g);
   SKY_TRY(s.begin(online, seeds, N, fanout, hops, seed, data, sample_lengths));
-  if (!s.online && s.totals) {
-    SKY_TRY(s.draw(0, hops - 1));
-    return s.end(sampled, seconds);
-  }
-  for (uint32_t h = 0; h + 1 < hops; ++h) {
-    SKY_TRY(s.frontier(h));
-    SKY_TRY(s.build(h, nullptr));
-    SKY_TRY(s.draw(h, h + 1));
-  }
+  SKY_TRY(s.run());
   return s.end(sampled, seconds);
 }
 

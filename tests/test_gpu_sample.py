@@ -14,11 +14,12 @@ def test_layout_closed_form():
     assert capi.sample_layout([1, 20, 20]) == (421, 21)
 
 
-@pytest.mark.parametrize("device_sized", [1, 0])
+@pytest.mark.parametrize("device_sized,direct", [(1, 0), (1, -1), (0, -1)])
 @pytest.mark.parametrize("fanout", [[1, 25, 10], [1, 3, 2, 2], [1, 5]])
-def test_offline_and_online_match_oracle(orc, fanout, device_sized):
+def test_offline_and_online_match_oracle(orc, fanout, device_sized, direct):
     # device_sized 1 (the default): the size of every frontier stays on the device and the host never waits inside
-    # the call; 0: the host reads it before it launches the build of the frontier's rows
+    # the call, or, where the first hop is drawn from the weights (direct), once behind that; 0: the host reads it before it launches the
+    # build of the frontier's rows
     from skywalker_amd import capi
     xadj, adjncy = orc.rmat_csr(13, 8, 21)
     w = orc.gen_weights(orc.W_LOGNORMAL, 21, len(adjncy), 0.0, 1.0)
@@ -26,6 +27,7 @@ def test_offline_and_online_match_oracle(orc, fanout, device_sized):
     lps, slen = capi.sample_layout(fanout)
     g = capi.Graph.upload(xadj, adjncy, w)
     capi.set_option("online_device_sized", device_sized)
+    g.set_option("online_direct", direct)
     try:
         d_on, sl_on, s_on, _ = g.sample_online(seeds, fanout, 17)
     finally:
@@ -192,8 +194,9 @@ def test_online_sampling_builds_rows_of_every_class_without_waiting(orc):
     fanout = [1, 4, 3]
     lps, slen = capi.sample_layout(fanout)
     g = capi.Graph.upload(xadj, adjncy, w)
-    for rep, n in enumerate((V, 50)):
-        seeds = np.arange(n, dtype=np.uint32) if rep == 0 else rng.integers(0, V, n).astype(np.uint32)
+    for rep, (n, mode) in enumerate(((V, 0), (50, 0), (V, -1), (50, -1))):
+        g.set_option("online_direct", mode)
+        seeds = np.arange(n, dtype=np.uint32) if n == V else rng.integers(0, V, n).astype(np.uint32)
         d_on, sl_on, s_on, _ = g.sample_online(seeds, fanout, 31 + rep)
         odata, osl, osampled = orc.sample_online(xadj, adjncy, w, seeds, fanout, 31 + rep)
         assert np.array_equal(d_on.to_host((n, lps)), odata) and np.array_equal(sl_on.to_host((n, slen)), osl)
@@ -576,9 +579,59 @@ def test_children_drawn_from_the_weights(orc, fanout, dist, seeds_n):
         w[xadj[v]:xadj[v + 1]] = 0.0
     seeds = np.append((np.arange(seeds_n - 1) * 7) % n, n + 5).astype(np.uint32)
     lps, slen = capi.sample_layout(fanout)
-    g = capi.Graph.upload(xadj, adjncy, w)
-    d, sl, sampled, _ = g.sample_online(seeds, fanout, 61)
-    got = d.to_host((seeds_n, lps)), sl.to_host((seeds_n, slen))
-    g.free()
     want = orc.sample_online(xadj, adjncy, w, seeds, fanout, 61)
-    assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0]) and sampled == want[2]
+    g = capi.Graph.upload(xadj, adjncy, w)
+    for mode in (1, -1, 0):  # whatever the rows, unless they are long, never
+        g.set_option("online_direct", mode)
+        d, sl, sampled, _ = g.sample_online(seeds, fanout, 61)
+        assert np.array_equal(sl.to_host((seeds_n, slen)), want[1]) and np.array_equal(d.to_host((seeds_n, lps)), want[0])
+        assert sampled == want[2]
+    g.free()
+
+
+@pytest.mark.parametrize("fanout", [[1, 20], [1, 10, 10], [1, 10, 300]])
+@pytest.mark.parametrize("longest", [40001, 60001])
+def test_parents_whose_rows_are_too_long_to_draw_from_the_weights(orc, fanout, longest):
+    # one long row again and again, beside others, and behind rows of one entry: the first hop is drawn from tables after all, or the
+    # second where the longest row is short enough for a call that begins without any
+    from skywalker_amd import capi
+    rng = np.random.default_rng(89)
+    degs = np.full(105001, 10)
+    degs[0], degs[1:5001] = longest, 1
+    xadj = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    V, E = len(degs), int(xadj[-1])
+    adjncy = rng.integers(0, V, E, dtype=np.uint32)
+    adjncy[longest:longest + 5000] = 0  # rows 1 to 5000 lead to the long one
+    w = weights(E, rng, "lognormal2")
+    lps, slen = capi.sample_layout(fanout)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    short = rng.integers(5001, V, 4000).astype(np.uint32)
+    mixed = short.copy()
+    mixed[3000] = 0
+    for seeds in (np.zeros(30, np.uint32), np.zeros(3000, np.uint32), np.arange(1, 31, dtype=np.uint32), short[:30], short, mixed):
+        want = orc.sample_online(xadj, adjncy, w, seeds, fanout, 73)
+        for _ in range(2):
+            d, sl, sampled, _ = g.sample_online(seeds, fanout, 73)
+            assert np.array_equal(sl.to_host((len(seeds), slen)), want[1]) and np.array_equal(d.to_host((len(seeds), lps)), want[0])
+            assert sampled == want[2]
+    g.free()
+
+
+def test_a_vertex_that_starts_every_sample_is_not_swept_for_each_of_them():
+    # 8,192 times a row of 60,000 entries: its table takes microseconds, and by default it is made once
+    from skywalker_amd import capi
+    rng = np.random.default_rng(90)
+    degs = np.full(100001, 10)
+    degs[0] = 60000
+    xadj = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    E = int(xadj[-1])
+    g = capi.Graph.upload(xadj, rng.integers(0, len(degs), E, dtype=np.uint32), weights(E, rng, "lognormal"))
+    seeds = np.zeros(8192, np.uint32)
+
+    def seconds(mode):
+        g.set_option("online_direct", mode)
+        return min(g.sample_online(seeds, [1, 20], 1)[3] for _ in range(5))
+    never, default, always = seconds(0), seconds(-1), seconds(1)
+    print("never %.1f us, by default %.1f us, always %.1f us" % (never * 1e6, default * 1e6, always * 1e6))
+    assert default < 2 * never and 2 * default < always
+    g.free()
