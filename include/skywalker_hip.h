@@ -263,8 +263,8 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      "build_profile" (default 0): 1 records a HIP event after every kernel of sky_alias_build_all for
  *      sky_last_build_profile (about 3 microseconds each; a small graph pays 20 % of its build for them).
  *      "online_full_build" (default -1): how sky_walk_online serves a static bias on a graph without tables:
- *      0 builds the long rows that the walk is expected to draw from often and evaluates the draws from all others
- *      directly; 1 builds every row first and walks as sky_walk_offline does; -1 takes whichever is estimated to be
+ *      0 builds the long rows that the walk is expected to draw from often (short walks look at the rows of up to 4,096 of their
+ *      start vertices for that) and evaluates the draws from all others directly; 1 builds every row first and walks as sky_walk_offline does; -1 takes whichever is estimated to be
  *      faster.  The paths are the same.
  *      "online_device_sized" (default 1): sky_sample_online builds the rows of a frontier without the host ever
  *      learning how many they are: the sizes of its degree classes stay on the device, every build kernel finds its rows through them, and the call waits for
@@ -273,8 +273,8 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      "online_direct" (default -1): sky_sample_online evaluates the draws of a hop from the weights and builds none of its
  *      rows.  -1: the first hop of up to 8,192 start vertices, or of 40,960 where there is no other, and all hops where later ones
  *      are expected to lead to few entries; a hop whose rows turn out to be long, or to hold many entries together, is drawn from
- *      tables after all.  0: never.  1: every hop, whatever it meets.  Draws with replacement and online_device_sized only.  Same
- *      results.
+ *      tables after all.  0: never.  1: every hop, whatever it meets.  Draws with replacement and online_device_sized only.  1 also
+ *      keeps sky_walk_online with a static bias from building any row, unless online_full_build is 1.  Same results.
  *      "walk_compact_every" (default 0): k > 0 makes sky_walk_offline run k steps per launch and hand the next
  *      launch the list of walkers that are still walking (the reference's walker queue,
  *      include/sampler_result.cuh:646-669), so that walkers that have stopped no longer hold a lane; 0 keeps every

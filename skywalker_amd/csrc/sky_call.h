@@ -17,16 +17,17 @@ struct CallDevice {
   unsigned long long entries, arrived, refused;  // sample_check_kernel; the last is left as it is
   unsigned long long pad[3];
 };
+constexpr int CALL_ANSWERS = 10;
 // Pinned host words of a call, written by the end kernel: each carries the number of the call in its upper 16 bits, so that the
 // host knows which of them has arrived and neither waits for the other on its way over PCIe (results first, then, released, a
 // number of their own: a round trip more, 0.4 to 0.8 us of a call of 15 to 30).
 struct CallHost {
   unsigned long long sampled, ticks;
-  unsigned long long answer;  // in the course of a call, with a number of its own (call_ask)
-  unsigned long long pad[5];
+  unsigned long long answer[CALL_ANSWERS];  // in the course of a call, with a number of their own (call_ask)
+  unsigned long long pad[4];
 };
 constexpr int CALL_VALUE_BITS = 48;  // 2^48 edges fill the GPU's memory a thousand times over; 2^48 ticks of 10 ns are a month
-static_assert(sizeof(CallDevice) == 64 && sizeof(CallHost) == 64, "one cache line each");
+static_assert(sizeof(CallDevice) == 64 && sizeof(CallHost) == 128, "cache lines of their own");
 // Where a call reports.  A graph has one for the calls that begin and end within one entry point; a call that stays open
 // between entry points (a sampling session) has its own, because other calls on the graph begin and end meanwhile.
 struct CallWords {
@@ -59,13 +60,13 @@ int call_begin(sky_graph* g, CallWords* w, CallDevice** call);
 // Enqueues the end kernel behind what the call has put on the graph's stream, waits for it and hands out the results.
 // Outputs may be null.  `counts` (n of them, device, may be null) are added to the sampled edges.
 int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);
-// The host's questions in the course of a call: a kernel answers question number call_ask(w) by call_answer, and call_answered waits
-// for it.
+// The host's questions in the course of a call: a kernel answers question number call_ask(w) by call_answer, word by word, and
+// call_answered waits for the first n.
 inline unsigned long long call_ask(CallWords* w) { return ++w->asked; }
-__device__ __forceinline__ void call_answer(CallHost* host, unsigned long long number, unsigned long long value) {
-  __hip_atomic_store(&host->answer, value | number << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+__device__ __forceinline__ void call_answer(CallHost* host, unsigned long long number, int word, unsigned long long value) {
+  __hip_atomic_store(&host->answer[word], value | number << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-int call_answered(sky_graph* g, CallWords* w, unsigned long long* value);
+int call_answered(sky_graph* g, CallWords* w, unsigned long long* values, int n);
 // With the graph's own words.
 int call_begin(sky_graph* g, CallDevice** call);
 int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);

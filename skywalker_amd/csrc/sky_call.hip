@@ -90,7 +90,7 @@ int take_words(int device, CallWords* w) {
   w->host = use->host + k;
   w->khz = use->khz;
   w->seq = use->host[k].sampled >> CALL_VALUE_BITS;  // not the next call's
-  w->asked = use->host[k].answer >> CALL_VALUE_BITS;
+  w->asked = use->host[k].answer[0] >> CALL_VALUE_BITS;
   return SKY_OK;
 }
 }  // namespace
@@ -162,8 +162,8 @@ static int take_values(hipStream_t st, const unsigned long long* from, int n, un
   return SKY_OK;
 }
 
-int call_answered(sky_graph* g, CallWords* w, unsigned long long* value) {
-  return take_values(g->stream, &w->host->answer, 1, w->asked, value);
+int call_answered(sky_graph* g, CallWords* w, unsigned long long* values, int n) {
+  return take_values(g->stream, w->host->answer, n, w->asked, values);
 }
 
 int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {

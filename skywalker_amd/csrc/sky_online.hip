@@ -71,8 +71,8 @@ static uint32_t walker_threads(uint32_t N, uint32_t longest) {
 }
 
 // How to serve a static-bias walk on a graph without tables.  Every row drawn from costs either its table (BUILD_PS an entry, once, and
-// BUILD_US the launches of a build) or two sweeps over its weights (DRAW_PS an entry, each time).  A start vertex is any vertex; a
-// later step leads to a row with a probability that grows with its length, so a row of d entries is drawn from N * (len - 1) * d / E
+// BUILD_US the launches of a build) or two sweeps over its weights (DRAW_PS an entry, each time).  A start vertex is any vertex, or as
+// online_plan finds; a later step leads to a row with a probability that grows with its length, so a row of d entries is drawn from N * (len - 1) * d / E
 // times, and its table pays from some length on.  But a walk also lasts as long as the walker that meets the longest row without
 // a table, ROW_NS an entry with 512 threads, inversely more with fewer and down to ROW_LEAST_NS with more.  What every choice would
 // take is added up, from no tables over those of the longest class alone to those of every class from 33 entries on, and the least is taken.
@@ -85,13 +85,13 @@ constexpr double BUILD_PS = 7.5, DRAW_PS = 2.4, BUILD_US = 31.0, ROW_NS = 0.39, 
 struct OnlinePlan {
   bool full;            // every row, then the offline walk
   uint32_t table_from;  // else: the rows of at least so many entries
+  double us;
 };
-static int online_plan(sky_graph* g, uint32_t N, uint32_t len, float stop_prob, OnlinePlan* o, CallDevice** first) {
-  const long long mode = option(g, OPT_ONLINE_FULL_BUILD);
-  *o = OnlinePlan{mode > 0, 0xFFFFFFFFu};
-  if (mode > 0) return SKY_OK;
-  SKY_TRY(ensure_plan(g, first));
-  const double E = std::max(1u, g->E), V = std::max(1u, g->V), go = 1.0 - std::min(1.0f, std::max(0.0f, stop_prob)), starts = N * go;
+// starts: walkers whose first row is of each class.  `only`: null, or the plan that is to be rated.
+static OnlinePlan plan_for(const sky_graph* g, uint32_t N, uint32_t len, double go, const double (&starts)[CLS_COUNT],
+                           const OnlinePlan* only = nullptr) {
+  OnlinePlan o{false, 0xFFFFFFFFu, 1e30};
+  const double E = std::max(1u, g->E);
   const double edges = N * (go < 1.0 ? go * go * (1.0 - std::pow(go, len - 1.0)) / (1.0 - go) : len - 1.0);  // steps along an edge
   struct Rows {
     uint32_t from;
@@ -101,17 +101,18 @@ static int online_plan(sky_graph* g, uint32_t N, uint32_t len, float stop_prob, 
   for (int c = CLS_G2; c < CLS_COUNT; ++c) {
     const double entries = (double)g->bin_edges[c], count = g->bin_counts[c];
     if (entries == 0 || count == 0) continue;
-    const double mean = entries / count, times = edges * entries / E + starts * count / V;
+    const double mean = entries / count, times = edges * entries / E + starts[c];
     const double most = std::min(1.5 * mean, (double)g->max_degree);
     rows[n++] = Rows{class_min_degree(c), entries, times * mean, most * (std::min(1.0, times) + times / std::max(1u, N))};
   }
   std::sort(rows, rows + n, [](const Rows& a, const Rows& b) { return a.from < b.from; });
   const double to_max = edges * g->max_degree / E;
-  double best = 1e30, built = 0;
+  double built = 0;
   for (int k = n; k >= 0; --k) {  // tables of rows[k] .. rows[n - 1]
     if (k < n) built += rows[k].entries;
     if (k < n && rows[k].from < 33) break;  // the shorter classes are not built apart from the rest
     const uint32_t from = k < n ? rows[k].from : 0xFFFFFFFFu;
+    if (only && (only->full || only->table_from != from)) continue;
     double read = 0, chain = k < n ? 0.0 : g->max_degree * (std::min(1.0, to_max) + to_max / std::max(1u, N));
     for (int i = 0; i < k; ++i) {
       read += rows[i].read;
@@ -119,13 +120,79 @@ static int online_plan(sky_graph* g, uint32_t N, uint32_t len, float stop_prob, 
     }
     const double row_ns = std::max(ROW_LEAST_NS, ROW_NS * 512 / walker_threads(N, std::min(from - 1, g->max_degree)));
     const double us = (k < n ? BUILD_US + built * BUILD_PS * 1e-6 : 0.0) + read * DRAW_PS * 1e-6 + chain * row_ns * 1e-3 + STEP_US * len;
-    if (us < best) {
-      best = us;
-      o->table_from = from;
+    if (us < o.us) {
+      o.us = us;
+      o.table_from = from;
     }
   }
   const double full_us = BUILD_US + E * BUILD_PS * 1e-6 + 1.2 * len;
-  o->full = mode < 0 && full_us < best;
+  if (only ? only->full : option(g, OPT_ONLINE_FULL_BUILD) < 0 && full_us < o.us) {
+    o.full = true;
+    o.us = full_us;
+  }
+  return o;
+}
+
+// Classes of the rows of start vertices, all of them or 4,096 spread over them, 16 bits each.
+constexpr uint32_t STARTS_T = 1024, STARTS_SEEN = 4096;
+static_assert(3 * CALL_ANSWERS >= CLS_COUNT && 16 * 3 <= CALL_VALUE_BITS, "three classes a word");
+__global__ __launch_bounds__(STARTS_T) void walk_starts_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ seeds,
+                                                               uint32_t N, uint32_t V, CallHost* __restrict__ host,
+                                                               unsigned long long number, CallDevice* __restrict__ call) {
+  __shared__ uint32_t s_n[3 * CALL_ANSWERS];
+  call_stamp(call);
+  if (threadIdx.x < 3 * CALL_ANSWERS) s_n[threadIdx.x] = 0;
+  __syncthreads();
+  const uint32_t seen = min(N, STARTS_SEEN);
+  uint32_t v[STARTS_SEEN / STARTS_T];
+#pragma unroll
+  for (int u = 0; u < (int)(STARTS_SEEN / STARTS_T); ++u) {
+    const uint32_t i = u * STARTS_T + threadIdx.x;
+    v[u] = i < seen ? seeds[(uint64_t)i * N / seen] : V;
+  }
+#pragma unroll
+  for (int u = 0; u < (int)(STARTS_SEEN / STARTS_T); ++u)
+    if (v[u] < V) atomicAdd(&s_n[degree_class(xadj[v[u] + 1] - xadj[v[u]])], 1u);
+  __syncthreads();
+  const uint32_t t = threadIdx.x;
+  if (t < CALL_ANSWERS)
+    call_answer(host, number, (int)t, s_n[3 * t] | (unsigned long long)s_n[3 * t + 1] << 16 | (unsigned long long)s_n[3 * t + 2] << 32);
+}
+
+// Start vertices are the caller's.  Where the plan for any vertices is within ASK_US of the best for ends of edges they are not looked
+// at, unless it is one without tables and they might all be the vertex with the longest row; else what their rows are is asked for, which the
+// call waits 10 us for.  (As planned for any vertices / as asked, us: 40,000 walkers x 1 on the scale-20 graph, any vertices 85 / 95, ends of
+// edges 250 / 123, the longest row 2487 / 73; 8,500 x 1 there 32 / 41, 87 / 93, 610 / 62, on the scale-22 graph with 32 edges a vertex
+// 33 / 42, 275 / 214, 2427 / 95; 5,000 x 2, scale 20, 90 / 103, 135 / 101, 457 / 86.)
+constexpr double ASK_US = 15.0;
+static int online_plan(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, float stop_prob, OnlinePlan* o, CallDevice** first) {
+  const long long mode = option(g, OPT_ONLINE_FULL_BUILD);
+  *o = OnlinePlan{mode > 0, 0xFFFFFFFFu, 0.0};
+  if (mode > 0 || option(g, OPT_ONLINE_DIRECT) > 0) return SKY_OK;
+  SKY_TRY(ensure_plan(g, first));
+  const double go = 1.0 - std::min(1.0f, std::max(0.0f, stop_prob));
+  double any[CLS_COUNT], ends[CLS_COUNT], longest[CLS_COUNT] = {0.0};
+  longest[degree_class(g->max_degree)] = N * go;
+  for (int c = 0; c < CLS_COUNT; ++c) {
+    any[c] = N * go * g->bin_counts[c] / std::max(1u, g->V);
+    ends[c] = N * go * g->bin_edges[c] / std::max(1u, g->E);
+  }
+  *o = plan_for(g, N, len, go, any);
+  const OnlinePlan other = plan_for(g, N, len, go, ends);
+  auto loss = [&](const double (&starts)[CLS_COUNT], const OnlinePlan& best) { return plan_for(g, N, len, go, starts, o).us - best.us; };
+  const bool none = !o->full && o->table_from == 0xFFFFFFFFu, other_none = !other.full && other.table_from == 0xFFFFFFFFu;
+  if (o->full || (loss(ends, other) < ASK_US &&
+                  !(none && !other_none && loss(longest, plan_for(g, N, len, go, longest)) > 4 * ASK_US)))
+    return SKY_OK;
+  hipLaunchKernelGGL(walk_starts_kernel, dim3(1), dim3(STARTS_T), 0, g->stream, g->xadj, seeds, N, g->V, g->call.host, call_ask(&g->call),
+                     *first);
+  SKY_HIP(hipGetLastError());
+  *first = nullptr;
+  unsigned long long counts[CALL_ANSWERS];
+  SKY_TRY(call_answered(g, &g->call, counts, CALL_ANSWERS));
+  for (int c = 0; c < CLS_COUNT; ++c)
+    any[c] = N * go * (double)(counts[c / 3] >> 16 * (c % 3) & 0xFFFF) / std::min(N, STARTS_SEEN);
+  *o = plan_for(g, N, len, go, any);
   return SKY_OK;
 }
 
@@ -139,11 +206,11 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
   // Tables that already exist are used as they are.  Otherwise the rows that the walk will draw from often get theirs, all
   // of them when that is most of what it meets; the paths are the same either way.
   double plan_sec = 0, build_sec = 0;
-  OnlinePlan how{false, 0xFFFFFFFFu};
+  OnlinePlan how{false, 0xFFFFFFFFu, 0.0};
   CallDevice* call = nullptr;
   if (!g->has_tables) {
     SKY_TRY(call_begin(g, &call));
-    if (N && len) SKY_TRY(online_plan(g, N, len, stop_prob, &how, &call));
+    if (N && len) SKY_TRY(online_plan(g, seeds, N, len, stop_prob, &how, &call));
     if (how.full) {  // the build is a call of its own, and so is the plan if it was made just now
       if (call) call_cancel(g);
       else SKY_TRY(call_end(g, nullptr, &plan_sec));

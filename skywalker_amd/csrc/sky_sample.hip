@@ -361,7 +361,7 @@ __global__ __launch_bounds__(CHECK_T) void sample_check_kernel(SampleArgs a, uin
     a.words->arrived = 0;
   }
   a.words->refused = sum > budget;
-  call_answer(host, number, sum > budget);
+  call_answer(host, number, 0, sum > budget);
 }
 
 // A wavefront a slot; the slots of a workgroup whose rows are too long for one are left to all eight together.  What bounds it is the chain
@@ -831,7 +831,7 @@ struct SampleSession {
       SKY_TRY(draw(h, h + 1));
       if (!is_direct(h) || !budget[h]) continue;
       unsigned long long refused = 0;
-      SKY_TRY(call_answered(g, words(), &refused));
+      SKY_TRY(call_answered(g, words(), &refused, 1));
       if (!refused) continue;
       if (all_direct()) init();
       direct.clear();  // the hop once more, with tables, and those behind it

@@ -530,7 +530,7 @@ def test_node2vec_table_with_a_bit_per_vertex(orc, V, walkers, p, q):
                                              (12289, 1024), (12289, 1025), (12289, 8193)])
 def test_online_static_draws_by_workgroups_of_every_size(longest, walkers):
     # 64 to 1024 threads a walker by the longest row and the number of walkers; rows around 256 slots a wavefront and 4 a thread,
-    # beside 20 M entries in rows of 32: of a graph so large a walk of one step builds no row
+    # none of which is built (online_direct 1), or those that a walk from these vertices is expected to gain by (-1)
     from skywalker_amd import capi
     rng = np.random.default_rng(longest)
     lens = [1, 2, 3, 4, 5, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 4095, 4096, 4097, longest] + \
@@ -544,9 +544,44 @@ def test_online_static_draws_by_workgroups_of_every_size(longest, walkers):
     g = capi.Graph.upload(xadj, local, w)
     g.set_option("online_full_build", 0)
     seeds = (np.arange(walkers) % n).astype(np.uint32)
-    direct = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 1, 0.0, 7)
+    online = []
+    for mode in (1, -1):
+        g.set_option("online_direct", mode)
+        online.append(g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 1, 0.0, 7))
     g.build_tables()
     tabled = g.walk_offline(seeds, 1, 0.0, 7)
-    assert np.array_equal(direct[0].to_host(), tabled[0].to_host()) and np.array_equal(direct[1].to_host(), tabled[1].to_host())
-    assert direct[2] == tabled[2]
+    for direct in online:
+        assert np.array_equal(direct[0].to_host(), tabled[0].to_host()) and np.array_equal(direct[1].to_host(), tabled[1].to_host())
+        assert direct[2] == tabled[2]
+    g.free()
+
+
+@pytest.mark.parametrize("full_build", [0, -1])
+@pytest.mark.parametrize("length", [1, 2])
+def test_short_walks_from_well_connected_vertices_build_their_rows(orc, length, full_build):
+    # a walk of a few steps from any vertices needs no tables; from the longest row for every walker it does, and sweeping it
+    # for each of them takes ten times as long as the others
+    from skywalker_amd import capi
+    xadj, adjncy = orc.rmat_csr(16, 16, 44)
+    w = orc.gen_weights(orc.W_LOGNORMAL, 44, len(adjncy), 0.0, 1.0)
+    deg = np.diff(xadj.astype(np.int64))
+    prob, alias, _ = orc.alias_build(xadj, w)
+    rng = np.random.default_rng(44)
+    N = 40000
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_full_build", full_build)
+    starts = {"any": rng.integers(0, len(deg) + 1, N), "ends": adjncy[rng.integers(0, len(adjncy), N)], "first": np.arange(N) % 5000,
+              "hub": np.full(N, deg.argmax()), "none": np.full(N, len(deg)), "few": np.argsort(-deg)[:7]}
+    took = {}
+    for name, seeds in starts.items():
+        seeds = seeds.astype(np.uint32)
+        paths, lengths, sampled = orc.walk_offline(xadj, adjncy, prob, alias, seeds, length, 0.0, 5)
+        for _ in range(4):
+            got = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, length, 0.0, 5)
+            took[name] = min(took.get(name, 1e9), got[3])
+            assert np.array_equal(got[0].to_host(paths.shape), paths) and np.array_equal(got[1].to_host(), lengths) and got[2] == sampled
+            if full_build:
+                g.sample_session(np.zeros(0, np.uint32), [1, 2], 1)  # its begin leaves the graph without tables
+    print({k: "%.1f us" % (v * 1e6) for k, v in took.items()})
+    assert took["hub"] < 3 * took["any"]
     g.free()
