@@ -236,8 +236,9 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      "stream_min_edges" (default 4000000): rows of 8190..524287 entries have a kernel of their own (one workgroup
  *      streams a row); when a build holds no more than this many entries in such rows, too few to fill the GPU
  *      with one workgroup each, they go to the tile-parallel path instead.  Builds that go out in four launches take
- *      that path also above the limit where the longest such row would outlast everything else.  Tests set 0: always
- *      by one workgroup.
+ *      that path also above the limit, for all of these rows or for those of more than 24576 entries, where the longest such row would
+ *      outlast everything else, and at the default, and no other value, stream those of up to 24576 entries below it where
+ *      that takes less.  Tests set 0: always by one workgroup.
  *      "stream_wide_min_edges" (default 134217216): the rows of more than 65533 entries among them keep a workgroup
  *      busy for up to 1.5 ms; they join that kernel only when the build holds at least this many entries in rows
  *      of 8190..524287 entries (the launch then runs that long anyway), else they are built tile by tile.  Tests set 0.

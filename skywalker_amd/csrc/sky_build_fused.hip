@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "sky_build_fused.h"
+#include "sky_build_rules.h"
 #include "sky_build_long.h"
 #include "sky_build_rows.h"
 #include "sky_build_tile.h"
@@ -611,27 +612,16 @@ int ensure_plan(sky_graph* g, CallDevice** first) {
     p.listed = 0;
     for (int c = CLS_G16; c < CLS_COUNT; ++c) p.listed += g->bin_counts[c];
     p.narrow_limit = narrow_limit;
-    // Rows of 8190..65533 entries are streamed, one workgroup each, by builds that hold enough of them to fill the GPU that
-    // way; other builds, and those of small frontiers, make them tile by tile, all of them or those of more than 24,576, for which
-    // they need geometry.  A graph with very many of them does without: 65536 tiles that a frontier may have to pass over take 20 us
-    // a launch.
-    // A workgroup takes 2.4 ns an entry for such a row, and the launch lasts at least as long as the longest of them.
-    // The launch of the rows of 2558..65533 entries as a whole takes 6 ps an entry, the tile passes 13 ps (one
-    // MI355X; this tells the faster way for 13 of 13 graphs of 4 to 117 M entries: 40 M entries in rows of 1..300,000
-    // 409 -> 367 us by tiles, R-MAT scale 22 edge factor 28 754 us streamed, 888 by tiles).  Rows of up to 24,576 streamed and the longer ones
-    // by tiles: an online walk of 10,000 x 8 on the scale-22 graph with 16 edges a vertex 222 -> 197 us, a build with 10 272 -> 264.
+    // Those of 8190..65533 entries by narrow_rows; small frontiers make them tile by tile, for which they need geometry.  A graph with very
+    // many of them does without: 65536 tiles that a frontier may have to pass over take 20 us a launch.
     const uint64_t last = g->bin_edges[CLS_STREAM_LAST], narrow = g->bin_edges[CLS_STREAM] + last;
     uint64_t wide = g->bin_edges[CLS_HOLD];
     for (int c = CLS_MW2 + 4; c <= CLS_MW2 + MERGE_MAX_NW - 2; ++c) wide += g->bin_edges[c];
-    auto us = [&](uint64_t streamed, uint32_t longest) {
-      return std::max(std::min(g->max_degree, longest) * 2.4e-3, (wide + streamed) * 6e-6) + (narrow - streamed) * 13e-6;
-    };
-    const double none_us = us(0, HOLD_MAX_DEG), last_us = us(last, 24576u), all_us = us(narrow, g->bin_counts[CLS_STREAM] ? 65533u : 24576u);
-    const bool some = narrow_limit > 0 && last > 0 && g->bin_counts[CLS_STREAM] > 0 && last_us < none_us;
-    if ((long long)narrow <= narrow_limit || (narrow_limit > 0 && std::min(none_us, some ? last_us : none_us) < all_us))
-      p.t_all = some ? CLS_STREAM : CLS_STREAM_LAST;
-    else
-      p.t_all = CLS_STREAM_WIDE;
+    switch (narrow_rows(narrow_limit, last, g->bin_edges[CLS_STREAM], wide, g->max_degree)) {
+      case NarrowRows::STREAMED: p.t_all = CLS_STREAM_WIDE; break;
+      case NarrowRows::TO_24576_STREAMED: p.t_all = CLS_STREAM; break;
+      case NarrowRows::TILED: p.t_all = CLS_STREAM_LAST; break;
+    }
     p.t_first = p.t_all == CLS_STREAM_LAST || narrow <= 65536ull * TILE ? CLS_STREAM_LAST : p.t_all;
     // Tiles of the rows that only small frontiers make tile by tile, then those of the others, from a bound of the former on: that is
     // known without asking the device, and the places between are no tiles.

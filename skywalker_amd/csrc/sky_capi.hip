@@ -2,6 +2,7 @@
 #include <cstring>
 
 #include "sky_build_fused.h"
+#include "sky_build_rules.h"
 #include "sky_graph.h"
 
 namespace sky {
@@ -55,7 +56,7 @@ namespace sky {
 long long g_option_value[OPT_COUNT] = {
     1ll << 22,                             // tiled_max_tiles: no limit
     1,                                     // row_merge
-    4000000,                               // stream_min_edges
+    STREAM_MIN_EDGES,                      // stream_min_edges
     512ll * (sky::STREAM_MAX_DEG / 2),     // stream_wide_min_edges: 512 workgroups run at a time
     -1,                                    // walk_read_once: by the size of the tables
     0,                                     // sample_distinct
