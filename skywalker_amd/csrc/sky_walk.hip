@@ -669,7 +669,8 @@ int walk_node2vec_reject(sky_graph* g, float p, float q, const uint32_t* seeds, 
   if (!g->has_tables) SKY_TRY(build_all_tables(g, &build_sec));  // first-order tables, built on demand
   const float fp = 1.0f / p, fq = 1.0f / q;
   const float fmax = fmaxf(1.0f, fmaxf(fp, fq));
-  if (fp == 1.0f && fq == 1.0f) {  // every candidate is kept: the first-order walk, whose trial 0 shares the counters
+  // every candidate is kept: the first-order walk, whose trial 0 shares the counters, and whose one launch has a lane for each walker
+  if (fp == 1.0f && fq == 1.0f && N <= 0xFFFFFFFFu / WALK_BLOCK * WALK_BLOCK) {
     SKY_TRY(walk_offline(g, seeds, N, len, stop_prob, seed, paths, lengths, sampled, seconds));
     if (seconds) *seconds += build_sec;
     return SKY_OK;

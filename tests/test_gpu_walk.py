@@ -556,6 +556,29 @@ def test_online_static_draws_by_workgroups_of_every_size(longest, walkers):
     g.free()
 
 
+def test_node2vec_rejection_without_bias_by_more_walkers_than_one_launch_has():
+    # p = q = 1 goes by the first-order walk, whose grid for so many walkers would be empty
+    from skywalker_amd import capi
+    N = 0xFFFFFF10
+    if capi.mem_info()[0] < 14 * N:
+        pytest.skip("56 GB of device memory")
+    xadj, adjncy = np.array([0, 1, 2], np.uint32), np.array([1, 0], np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, np.ones(2, np.float32))
+    g.build_tables()
+    seeds = capi.DeviceArray(N, np.uint32, fill=1)
+    paths, lengths = capi.DeviceArray(N, np.uint32, fill=7), capi.DeviceArray(N, np.uint32, fill=7)
+    sampled = g.walk_online(capi.BIAS_NODE2VEC_REJECT, 1.0, 1.0, seeds, 0, 0.0, 5, out=(paths, lengths))[2]
+    assert sampled == 0
+    import ctypes as C
+    for first in (0, (1 << 31) - 500, (1 << 32) - 2000, N - 1000):
+        for array, want in ((paths, 1), (lengths, 0)):
+            part = np.empty(1000 if first + 1000 <= N else N - first, np.uint32)
+            capi._ck(capi.lib().sky_memcpy_d2h(capi._p(part), C.c_void_p(array.ptr.value + 4 * first), C.c_size_t(part.nbytes)))
+            assert (part == want).all()
+    for x in (seeds, paths, lengths, g):
+        x.free()
+
+
 @pytest.mark.parametrize("full_build", [0, -1])
 @pytest.mark.parametrize("length", [1, 2])
 def test_short_walks_from_well_connected_vertices_build_their_rows(orc, length, full_build):
