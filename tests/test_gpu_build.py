@@ -669,8 +669,7 @@ def test_surpluses_beyond_64_bits(orc, knobs, longest):
 
 @pytest.mark.parametrize("walkers", [200, 1000, 5000])
 def test_draws_from_rows_with_surpluses_beyond_64_bits(walkers):
-    # evaluated from the weights, by workgroups of every size, against those from the tables.  20 M entries in rows of 32 beside
-    # them: of a graph so large this walk builds no row of up to 12,288 entries
+    # evaluated from the weights, by workgroups of 256 and 128 threads, against those from the tables; 20 M entries in rows of 32 beside them
     from skywalker_amd import capi
     rows = long_vanishing_rows(12288)
     lens = np.concatenate([[len(r) for r in rows], np.full(625000, 32)])
@@ -679,6 +678,7 @@ def test_draws_from_rows_with_surpluses_beyond_64_bits(walkers):
     local = np.arange(len(w), dtype=np.uint32) - np.repeat(xadj[:-1], lens)  # a vertex of its own for every slot of a row
     g = capi.Graph.upload(xadj, local, w)
     g.set_option("online_full_build", 0)
+    g.set_option("online_direct", 1)  # no row is built
     seeds = np.arange(walkers, dtype=np.uint32) % len(rows)
     direct = [g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 1, 0.0, 5), g.walk_online(capi.BIAS_NODE2VEC, 2.0, 0.5, seeds, 1, 0.0, 5)]
     g.build_tables()
@@ -785,16 +785,18 @@ def test_seconds_of_a_call_that_lists_the_rows_contain_the_listing(kind):
 
 
 def test_rows_of_2558_to_3581_entries_beside_shorter_ones(orc):
-    # enough of them for the launch of 256 threads, 14 slots each, in a build and in that of a frontier, whose streamed rows the workgroups
-    # ask for; the edges of their classes, and of those around them
+    # enough of them for the launch of 256 threads, 14 slots each, in a build and in that of a frontier of more than 65,536 rows, whose
+    # 700 streamed rows the workgroups ask for; the edges of their classes, and of those around them
     from skywalker_amd import capi
     rng = np.random.default_rng(59)
     degs = list(rng.integers(2558, 3582, 1400)) + [2556, 2557, 2558, 2559, 3069, 3070, 3071, 3580, 3581, 3582, 3583, 4093, 4094, 5117] * 3 + \
-        list(rng.integers(8190, 65534, 40)) + [8190, 24576, 24577, 65533] + list(rng.integers(1, 300, 3000))
+        list(rng.integers(8190, 12000, 650)) + list(rng.integers(8190, 65534, 50)) + [8190, 24576, 24577, 65533] + \
+        list(rng.integers(1, 300, 3000)) + list(rng.integers(1, 4, 65000))
     rng.shuffle(degs)
     xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal")
     g = capi.Graph.upload(xadj, adjncy, w)
-    seeds = (np.arange(70000) % len(degs)).astype(np.uint32)
+    g.set_option("stream_min_edges", 0)  # 50 rows of up to 65,533 entries would take as long as all others
+    seeds = rng.permutation(len(degs)).astype(np.uint32)
     d, sl, sampled, _ = g.sample_online(seeds, [1, 2], 3)
     got = d.to_host(), sl.to_host()
     g.build_tables()
@@ -826,18 +828,25 @@ def test_short_rows_of_ranges_in_another_order(orc, V):
     assert np.array_equal(prob.view(np.uint32), oprob.view(np.uint32)) and np.array_equal(alias, oalias) and np.array_equal(valid, ovalid)
 
 
+@pytest.mark.parametrize("limit", [None, 0, 1 << 30])
 @pytest.mark.parametrize("seeds_n", [3000, 70000])
-def test_rows_of_8190_to_24576_entries_streamed_and_longer_ones_by_tiles(orc, seeds_n):
-    # in a build of all rows, in one of the rows of 8,190 entries and more, and in those of a small frontier (all by tiles) and a large one
+def test_rows_of_8190_to_24576_entries_streamed_and_longer_ones_by_tiles(orc, seeds_n, limit):
+    # or all of them streamed (limit 0), or none: in a build of all rows, in one of the longer rows for a walk, and in those of small
+    # frontiers (all by tiles) and of large ones, of more than 65,536 rows, the streamed ones and those with tiles among them
     from skywalker_amd import capi
     rng = np.random.default_rng(61)
-    degs = list(rng.integers(8190, 24577, 270)) + [8189, 8190, 8191, 24576, 24577, 24578, 30000, 65533, 65534, 70001] + list(rng.integers(1, 200, 2000))
+    degs = list(rng.integers(8190, 24577, 270)) + list(rng.integers(8190, 9000, 350)) + \
+        [8189, 8190, 8191, 24576, 24577, 24578, 30000, 65533, 65534, 70001, 600001] + list(rng.integers(1, 200, 2000)) + [1, 2] * 34000
     rng.shuffle(degs)
     xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal2")
-    seeds = (np.arange(seeds_n) % len(degs)).astype(np.uint32)
+    # every vertex but a few, or the first ones and all long rows
+    seeds = rng.permutation(len(degs))[:seeds_n] if seeds_n > 65536 else np.append(np.flatnonzero(np.diff(xadj) > 8000), np.arange(seeds_n))[:seeds_n]
+    seeds = seeds.astype(np.uint32)
     oprob, oalias, ovalid = orc.alias_build(xadj, w)
     g = capi.Graph.upload(xadj, adjncy, w)
     g.set_option("online_full_build", 0)
+    g.set_option("online_direct", 0)
+    g.set_option("stream_min_edges", limit)
     d, sl, sampled, _ = g.sample_online(seeds, [1, 2, 2], 3)
     got = d.to_host(), sl.to_host()
     walk = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 9, 0.0, 5)

@@ -245,25 +245,31 @@ def test_sampling_hop_by_hop_with_the_callers_weights(orc):
                                       (70001, [1, 7, 4])])
 def test_batches_by_workgroup_and_by_hop(orc, n, fanout, distinct):
     # few start vertices share workgroups hop by hop, many take one each or part of a wavefront; fanouts of every group
-    # width; a frontier of more than 65,536 slots streams its long rows instead of making them tile by tile
+    # width; a frontier of more than 65,536 rows streams its long rows instead of making them tile by tile; with the first hop from
+    # tables and, by default, from the weights
     from helpers import graph_from_degrees
     from skywalker_amd import capi
     rng = np.random.default_rng(78)
     degs = [0, 1, 2, 3, 4, 5, 16, 17, 32, 33, 34, 63, 64, 65, 66, 200, 600, 1500, 3000, 5200, 8190, 9001, 25003, 66001, 530001]
-    degs += list(rng.integers(0, 90, 400))
+    degs += list(rng.integers(0, 90, 400)) + ([1, 2, 3] * 24000 if n > 65536 else [])
     xadj, adjncy, w = graph_from_degrees(degs, rng, "sparse")
     V = len(xadj) - 1
-    seeds = rng.integers(0, V + 1, n).astype(np.uint32)
+    seeds = (np.append(V, rng.permutation(V)) if n > 65536 else rng.integers(0, V + 1, n)).astype(np.uint32)[:n]
+    if n > 65536:
+        seeds[1:26] = np.arange(25)
     lps, slen = capi.sample_layout(fanout)
     g = capi.Graph.upload(xadj, adjncy, w)
     g.set_option("stream_min_edges", 0)
     g.set_option("sample_distinct", int(distinct))
+    g.set_option("online_direct", 0)
+    tabled = g.sample_online(seeds, fanout, 37)
+    g.set_option("online_direct", -1)
     on = g.sample_online(seeds, fanout, 37)
     g.build_tables()
     off = g.sample_offline(seeds, fanout, 37)
     prob, alias, _ = g.tables()
     want = orc.sample_offline(xadj, adjncy, prob, alias, seeds, fanout, 37, distinct=distinct)
-    for data, sl, sampled, _ in (on, off):
+    for data, sl, sampled, _ in (tabled, on, off):
         assert np.array_equal(sl.to_host((n, slen)), want[1]) and np.array_equal(data.to_host((n, lps)), want[0])
         assert sampled == want[2]
     g.free()

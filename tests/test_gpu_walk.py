@@ -458,8 +458,8 @@ def test_walk_index_goes_stale_when_tables_change(orc):
 @pytest.mark.parametrize("dist", ["lognormal2", "nearequal", "sparse"])
 @pytest.mark.parametrize("walkers", [1, 256, 257, 4096, 4097])
 def test_online_static_draws_evaluated_from_the_weights(orc, walkers, dist):
-    # workgroups of 1024, 256 and 64 threads; rows around a chunk of 256 slots, and rows of more than 256 chunks; the
-    # fewer draws are expected, the fewer rows get a table
+    # workgroups of 1024 threads to 256; rows around a chunk of 256 slots, and rows of more than 256 chunks; no row with a table, and those
+    # that the walk is expected to gain by
     from skywalker_amd import capi
     rng = np.random.default_rng(45)
     degs = [1, 2, 3, 4, 5, 63, 64, 65, 255, 256, 257, 511, 513, 1023, 1025, 4097, 65535, 65536, 65537, 140001, 0] + \
@@ -469,10 +469,12 @@ def test_online_static_draws_evaluated_from_the_weights(orc, walkers, dist):
     g = capi.Graph.upload(xadj, adjncy, w)
     g.set_option("online_full_build", 0)
     for length, stop in ((1, 0.0), (9, 0.03)):
-        paths, lengths, sampled, _ = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, length, stop, 29)
         want = orc.walk_online(xadj, adjncy, w, 0, 1.0, 1.0, seeds, length, stop, 29)
-        assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host((walkers, length + 1)), want[0])
-        assert sampled == want[2]
+        for mode in (1, -1):
+            g.set_option("online_direct", mode)
+            paths, lengths, sampled, _ = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, length, stop, 29)
+            assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host((walkers, length + 1)), want[0])
+            assert sampled == want[2]
     g.free()
 
 
