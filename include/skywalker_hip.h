@@ -264,7 +264,7 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      "build_profile" (default 0): 1 records a HIP event after every kernel of sky_alias_build_all for
  *      sky_last_build_profile (about 3 microseconds each; a small graph pays 20 % of its build for them).
  *      "online_full_build" (default -1): how sky_walk_online serves a static bias on a graph without tables:
- *      0 builds the long rows that the walk is expected to draw from often (short walks look at the rows of up to 4,096 of their
+ *      0 builds the long rows that the walk is expected to draw from often (short walks look at the rows of up to 1,024 of their
  *      start vertices for that) and evaluates the draws from all others directly; 1 builds every row first and walks as sky_walk_offline does; -1 takes whichever is estimated to be
  *      faster.  The paths are the same.
  *      "online_device_sized" (default 1): sky_sample_online builds the rows of a frontier without the host ever

@@ -29,12 +29,14 @@ __global__ __launch_bounds__(T) void walk_direct_kernel(const uint32_t* __restri
                                                         uint32_t table_from, const uint32_t* __restrict__ seeds, uint32_t first,
                                                         uint32_t V, uint32_t len, float stop_prob, uint64_t seed,
                                                         uint32_t* __restrict__ paths, uint32_t* __restrict__ lengths,
-                                                        CallDevice* __restrict__ call) {
+                                                        CallDevice* __restrict__ call, const CallDevice* __restrict__ words) {
   __shared__ DrawLds<T> lds;
   call_stamp(call);
   const uint32_t i = first + blockIdx.x;
   uint32_t* const path = paths + (size_t)i * (len + 1);
+  const bool refused = words && words->refused;  // beside the start vertex
   uint32_t v = seeds[i], s = 0;
+  if (refused) return;  // another plan is on its way
   if (threadIdx.x == 0) path[0] = v;
   for (; s < len && v < V; ++s) {
     const u32x4 r = philox(seed, i, s, 0, DOM_WALK);
@@ -86,11 +88,12 @@ struct OnlinePlan {
   bool full;            // every row, then the offline walk
   uint32_t table_from;  // else: the rows of at least so many entries
   double us;
+  bool enqueued = false;  // of no tables: the walk goes out at once, and is refused if the rows of its start vertices are long
 };
 // starts: walkers whose first row is of each class.  `only`: null, or the plan that is to be rated.
 static OnlinePlan plan_for(const sky_graph* g, uint32_t N, uint32_t len, double go, const double (&starts)[CLS_COUNT],
                            const OnlinePlan* only = nullptr) {
-  OnlinePlan o{false, 0xFFFFFFFFu, 1e30};
+  OnlinePlan o{false, 0xFFFFFFFFu, 1e30, false};
   const double E = std::max(1u, g->E);
   const double edges = N * (go < 1.0 ? go * go * (1.0 - std::pow(go, len - 1.0)) / (1.0 - go) : len - 1.0);  // steps along an edge
   struct Rows {
@@ -133,15 +136,19 @@ static OnlinePlan plan_for(const sky_graph* g, uint32_t N, uint32_t len, double 
   return o;
 }
 
-// Classes of the rows of start vertices, all of them or 4,096 spread over them, 16 bits each.
-constexpr uint32_t STARTS_T = 1024, STARTS_SEEN = 4096;
-static_assert(3 * CALL_ANSWERS >= CLS_COUNT && 16 * 3 <= CALL_VALUE_BITS, "three classes a word");
+// Classes of the rows of start vertices, all of them or 1,024 spread over them, 16 bits each; and, in the place of a class that is none,
+// whether a walk without tables is refused: these rows hold more than `budget` entries, or one of them more than `longest`.
+constexpr uint32_t STARTS_T = 512, STARTS_SEEN = 1024, STARTS_REFUSED = 22;
+static_assert(3 * CALL_ANSWERS >= CLS_COUNT && 16 * 3 <= CALL_VALUE_BITS && class_min_degree(STARTS_REFUSED) == 0, "three classes a word");
 __global__ __launch_bounds__(STARTS_T) void walk_starts_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ seeds,
-                                                               uint32_t N, uint32_t V, CallHost* __restrict__ host,
+                                                               uint32_t N, uint32_t V, unsigned long long budget, uint32_t longest,
+                                                               CallDevice* __restrict__ words, CallHost* __restrict__ host,
                                                                unsigned long long number, CallDevice* __restrict__ call) {
   __shared__ uint32_t s_n[3 * CALL_ANSWERS];
+  __shared__ unsigned long long s_entries;
   call_stamp(call);
   if (threadIdx.x < 3 * CALL_ANSWERS) s_n[threadIdx.x] = 0;
+  if (threadIdx.x == 0) s_entries = 0;
   __syncthreads();
   const uint32_t seen = min(N, STARTS_SEEN);
   uint32_t v[STARTS_SEEN / STARTS_T];
@@ -150,32 +157,58 @@ __global__ __launch_bounds__(STARTS_T) void walk_starts_kernel(const uint32_t* _
     const uint32_t i = u * STARTS_T + threadIdx.x;
     v[u] = i < seen ? seeds[(uint64_t)i * N / seen] : V;
   }
+  unsigned long long entries = 0;
 #pragma unroll
   for (int u = 0; u < (int)(STARTS_SEEN / STARTS_T); ++u)
-    if (v[u] < V) atomicAdd(&s_n[degree_class(xadj[v[u] + 1] - xadj[v[u]])], 1u);
+    if (v[u] < V) {
+      const uint32_t d = xadj[v[u] + 1] - xadj[v[u]];
+      atomicAdd(&s_n[degree_class(d)], 1u);
+      entries += d > longest ? budget + 1 : d;
+    }
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) entries += shfl_xor_u64(entries, m);
+  if ((threadIdx.x & 63) == 0) atomicAdd(&s_entries, entries);
   __syncthreads();
   const uint32_t t = threadIdx.x;
-  if (t < CALL_ANSWERS)
-    call_answer(host, number, (int)t, s_n[3 * t] | (unsigned long long)s_n[3 * t + 1] << 16 | (unsigned long long)s_n[3 * t + 2] << 32);
+  const bool refused = s_entries > budget;
+  if (t == 0) words->refused = refused;
+  if (t < CALL_ANSWERS) {
+    unsigned long long x = 0;
+    for (uint32_t k = 0; k < 3; ++k) x |= (unsigned long long)(3 * t + k == STARTS_REFUSED ? (uint32_t)refused : s_n[3 * t + k]) << 16 * k;
+    call_answer(host, number, (int)t, x);
+  }
+}
+
+// The plan by what walk_starts_kernel has seen; *o as it is if it has been enqueued and is not refused.
+static int plan_for_starts(sky_graph* g, uint32_t N, uint32_t len, double go, OnlinePlan* o) {
+  unsigned long long counts[CALL_ANSWERS];
+  SKY_TRY(call_answered(g, &g->call, counts, CALL_ANSWERS));
+  auto of = [&](uint32_t c) { return (uint32_t)(counts[c / 3] >> 16 * (c % 3)) & 0xFFFFu; };
+  if (o->enqueued && !of(STARTS_REFUSED)) return SKY_OK;
+  double starts[CLS_COUNT];
+  for (uint32_t c = 0; c < CLS_COUNT; ++c) starts[c] = c == STARTS_REFUSED ? 0.0 : N * go * of(c) / std::min(N, STARTS_SEEN);
+  *o = plan_for(g, N, len, go, starts);
+  return SKY_OK;
 }
 
 // Start vertices are the caller's.  Where the plan for any vertices is within ASK_US of the best for ends of edges they are not looked
-// at, unless it is one without tables and they might all be the vertex with the longest row; else what their rows are is asked for, which the
-// call waits 10 us for.  (As planned for any vertices / as asked, us: 40,000 walkers x 1 on the scale-20 graph, any vertices 85 / 95, ends of
-// edges 250 / 123, the longest row 2487 / 73; 8,500 x 1 there 32 / 41, 87 / 93, 610 / 62, on the scale-22 graph with 32 edges a vertex
-// 33 / 42, 275 / 214, 2427 / 95; 5,000 x 2, scale 20, 90 / 103, 135 / 101, 457 / 86.)
+// at, unless it is one without tables and they might all be the vertex with the longest row.  Else 1,024 of their rows are: for a plan without
+// tables while the walk is on its way, 4 us later, unless it is refused; for another before the build, which waits 10 us for it.  (As planned
+// for any vertices / as seen, us: 40,000 walkers x 1 on the scale-20 graph, any vertices 86 / 90, ends of edges 253 / 127, the longest row
+// 2477 / 76; 8,500 x 1 there 32 / 37, 88 / 91, 606 / 61, on the scale-22 graph with 32 edges a vertex 33 / 37, 270 / 211, 2427 / 94;
+// 5,000 x 2, scale 20, 89 / 95, 135 / 98, 454 / 83.)
 constexpr double ASK_US = 15.0;
-static int online_plan(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, float stop_prob, OnlinePlan* o, CallDevice** first) {
+static int online_plan(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, double go, OnlinePlan* o, CallDevice** first) {
   const long long mode = option(g, OPT_ONLINE_FULL_BUILD);
-  *o = OnlinePlan{mode > 0, 0xFFFFFFFFu, 0.0};
+  *o = OnlinePlan{mode > 0, 0xFFFFFFFFu, 0.0, false};
   if (mode > 0 || option(g, OPT_ONLINE_DIRECT) > 0) return SKY_OK;
   SKY_TRY(ensure_plan(g, first));
-  const double go = 1.0 - std::min(1.0f, std::max(0.0f, stop_prob));
+  const double E = std::max(1u, g->E), V = std::max(1u, g->V);
   double any[CLS_COUNT], ends[CLS_COUNT], longest[CLS_COUNT] = {0.0};
   longest[degree_class(g->max_degree)] = N * go;
   for (int c = 0; c < CLS_COUNT; ++c) {
-    any[c] = N * go * g->bin_counts[c] / std::max(1u, g->V);
-    ends[c] = N * go * g->bin_edges[c] / std::max(1u, g->E);
+    any[c] = N * go * g->bin_counts[c] / V;
+    ends[c] = N * go * g->bin_edges[c] / E;
   }
   *o = plan_for(g, N, len, go, any);
   const OnlinePlan other = plan_for(g, N, len, go, ends);
@@ -184,16 +217,16 @@ static int online_plan(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t
   if (o->full || (loss(ends, other) < ASK_US &&
                   !(none && !other_none && loss(longest, plan_for(g, N, len, go, longest)) > 4 * ASK_US)))
     return SKY_OK;
-  hipLaunchKernelGGL(walk_starts_kernel, dim3(1), dim3(STARTS_T), 0, g->stream, g->xadj, seeds, N, g->V, g->call.host, call_ask(&g->call),
-                     *first);
+  // Without tables the start rows may take 10 us more than those of any vertices, and the longest 15, or as long as one that is met later.
+  const double seen = std::min(N, STARTS_SEEN), row_ns = std::max(ROW_LEAST_NS, ROW_NS * 512 / walker_threads(N, g->max_degree));
+  const double budget = 1.5 * seen * E / V + 10e6 / DRAW_PS * seen / N;
+  const double most = std::max(15e3 / row_ns, g->max_degree * std::min(1.0, (len - 1.0) * N * g->max_degree / E));
+  hipLaunchKernelGGL(walk_starts_kernel, dim3(1), dim3(STARTS_T), 0, g->stream, g->xadj, seeds, N, g->V, (unsigned long long)budget,
+                     (uint32_t)std::min(most, 4294967295.0), g->call.dev, g->call.host, call_ask(&g->call), *first);
   SKY_HIP(hipGetLastError());
   *first = nullptr;
-  unsigned long long counts[CALL_ANSWERS];
-  SKY_TRY(call_answered(g, &g->call, counts, CALL_ANSWERS));
-  for (int c = 0; c < CLS_COUNT; ++c)
-    any[c] = N * go * (double)(counts[c / 3] >> 16 * (c % 3) & 0xFFFF) / std::min(N, STARTS_SEEN);
-  *o = plan_for(g, N, len, go, any);
-  return SKY_OK;
+  o->enqueued = none;
+  return none ? SKY_OK : plan_for_starts(g, N, len, go, o);
 }
 
 int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* seeds, uint32_t N, uint32_t len,
@@ -206,11 +239,33 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
   // Tables that already exist are used as they are.  Otherwise the rows that the walk will draw from often get theirs, all
   // of them when that is most of what it meets; the paths are the same either way.
   double plan_sec = 0, build_sec = 0;
-  OnlinePlan how{false, 0xFFFFFFFFu, 0.0};
+  OnlinePlan how{false, 0xFFFFFFFFu, 0.0, false};
   CallDevice* call = nullptr;
+  auto walk = [&] {
+    const uint32_t T = walker_threads(N, std::min(how.table_from - 1, g->max_degree));
+    const uint32_t most = 0xFFFFFFFFu / T;  // walkers of one launch: below 2^32 threads
+    for (uint32_t f = 0; f < N; f += std::min(most, N - f)) {
+      auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(std::min(most, N - f)), dim3(T), 0, g->stream, g->xadj, g->adjncy, g->adjwgt, g->table,
+                           how.table_from, seeds, f, g->V, len, stop_prob, seed, paths, lengths, call, how.enqueued ? g->call.dev : nullptr);
+      };
+      if (T == 1024) go(walk_direct_kernel<1024>);
+      else if (T == 512) go(walk_direct_kernel<512>);
+      else if (T == 256) go(walk_direct_kernel<256>);
+      else if (T == 128) go(walk_direct_kernel<128>);
+      else go(walk_direct_kernel<64>);
+      call = nullptr;
+    }
+  };
   if (!g->has_tables) {
     SKY_TRY(call_begin(g, &call));
-    if (N && len) SKY_TRY(online_plan(g, seeds, N, len, stop_prob, &how, &call));
+    const double go = 1.0 - std::min(1.0f, std::max(0.0f, stop_prob));
+    if (N && len) SKY_TRY(online_plan(g, seeds, N, len, go, &how, &call));
+    if (how.enqueued) {
+      walk();
+      SKY_TRY(plan_for_starts(g, N, len, go, &how));
+      if (how.enqueued) return call_end(g, sampled, seconds, lengths, N);
+    }
     if (how.full) {  // the build is a call of its own, and so is the plan if it was made just now
       if (call) call_cancel(g);
       else SKY_TRY(call_end(g, nullptr, &plan_sec));
@@ -222,27 +277,11 @@ int walk_online(sky_graph* g, int bias_kind, float p, float q, const uint32_t* s
     if (seconds) *seconds += plan_sec + build_sec;
     return SKY_OK;
   }
-  hipStream_t st = g->stream;
   if (how.table_from != 0xFFFFFFFFu) {
     SKY_TRY(build_rows_from(g, how.table_from, call));
     call = nullptr;  // the build's first kernel is the call's, or the plan's was
   }
-  if (N) {
-    const uint32_t T = walker_threads(N, std::min(how.table_from - 1, g->max_degree));
-    const uint32_t most = 0xFFFFFFFFu / T;  // walkers of one launch: below 2^32 threads
-    for (uint32_t f = 0; f < N; f += std::min(most, N - f)) {
-      auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(std::min(most, N - f)), dim3(T), 0, st, g->xadj, g->adjncy, g->adjwgt, g->table,
-                           how.table_from, seeds, f, g->V, len, stop_prob, seed, paths, lengths, call);
-      };
-      if (T == 1024) go(walk_direct_kernel<1024>);
-      else if (T == 512) go(walk_direct_kernel<512>);
-      else if (T == 256) go(walk_direct_kernel<256>);
-      else if (T == 128) go(walk_direct_kernel<128>);
-      else go(walk_direct_kernel<64>);
-      call = nullptr;
-    }
-  }
+  walk();
   return call_end(g, sampled, seconds, lengths, N);
 }
 
@@ -458,7 +497,9 @@ __global__ __launch_bounds__(T, WIN == 512 ? 5 : 4) void walk_n2v_table_kernel(c
 // previous row's vertices are set once a step, and a slot then tests one bit, where the search of the window is ten dependent
 // reads; with no state from slot to slot the loads of U times 256 slots are in flight at once.
 // Four walkers of four wavefronts to a CU, or two of eight while these hold all of them that walk (700 walkers x 20 on the scale-17 graph
-// 242 us with four wavefronts, 201 with eight; 2,000 x 40 there 452 and 667): twice as many bits would leave two walkers to a CU.
+// 242 us with four wavefronts, 201 with eight; 2,000 x 40 there 452 and 667): twice as many bits leave two walkers to a CU.  The line
+// is where four go, not where the bits stop to pay: with two of eight wavefronts to a CU the scale-19 graph would take 371 us for 490 with
+// 200 walkers x 40, 409 for 739 with 768, 767 for 863 with 2,000.
 // Against the windows: 2,000 x 40 with p = 2, q = 1/2 on the scale-18 graph 736 -> 550 us, on the scale-17 graph 617 -> 456, 1,500 x 30
 // with 40 edges a vertex, scale 13, 482 -> 320, 200 x 40 with 30, scale 16, 526 -> 358.
 constexpr uint32_t MAP_VERTICES = 1u << 18;  // 32 KB
