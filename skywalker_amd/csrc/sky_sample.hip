@@ -310,7 +310,8 @@ constexpr uint32_t DIRECT_LONG = 1024;
 // 10 there 360 / 332 / 323, 537 / 1,255 / 522, 564 / 835 / 539, 508 / 3,626 / 495.)
 constexpr int CHECK_T = 256, CHECK_U = 4;
 constexpr uint32_t DIRECT_CHAIN = 32768, DIRECT_PER_ROW = 4096;
-constexpr unsigned long long DIRECT_TOO_LONG = 1ull << 54;  // above any sum of the entries, 2^21 slots of less than 2^32
+// Above any sum of entries (40,960 slots of less than 2^32, or 2 M of up to DIRECT_ROW), and 2,000 workgroups may add it.
+constexpr unsigned long long DIRECT_TOO_LONG = 1ull << 50;
 __global__ __launch_bounds__(CHECK_T) void sample_check_kernel(SampleArgs a, uint64_t budget, uint32_t most_chain,
                                                                CallHost* __restrict__ host, unsigned long long number) {
   __shared__ unsigned long long s_sum[CHECK_T / 64];
