@@ -157,21 +157,36 @@ __device__ __forceinline__ bool row_at(const FusedArgs& a, const SectionRef& s, 
   return true;
 }
 
-__device__ __forceinline__ bool tile_active(const FusedArgs& a, uint32_t r) {
-  const uint32_t b = frontier_bit(a.trows[r].v, a.bit_mask);
-  return ((a.bitmap[b >> 5] >> (b & 31)) & 1u) && !a.built[r];
+// Units first, first + stride, ... below n that are wanted, by a workgroup (each wavefront of it looks for itself and finds the same), 64
+// of them looked at together, a lane each.  A build of a frontier passes over the tiles of every long row of the graph, of which it
+// makes few: one after another that is a chain of two to four dependent loads for each (28,500 tiles of the scale-22 graph with 32
+// edges a vertex, 43 us of a launch of 1,024 workgroups).
+template <class Wanted, class Work>
+__device__ __forceinline__ void each_wanted(uint32_t n, uint32_t first, uint32_t stride, Wanted wanted, Work work) {
+  for (uint32_t u0 = first; u0 < n; u0 += 64u * stride) {
+    const uint32_t u = u0 + (threadIdx.x & 63) * stride;
+    for (unsigned long long m = __ballot(u < n && wanted(u)); m; m &= m - 1ull) work(u0 + ((uint32_t)__ffsll((long long)m) - 1u) * stride);
+  }
+}
+// Whether the tile belongs to a row that the frontier asks for; its first tile says so to the passes behind.
+__device__ __forceinline__ bool tile_asked(const FusedArgs& a, uint32_t tile) {
+  const TileGeom tg = a.geom[tile];
+  if (tg.span == 0) return false;  // there are fewer tiles than their bound
+  const uint32_t b = frontier_bit(a.trows[tg.row].v, a.bit_mask);
+  const bool active = ((a.bitmap[b >> 5] >> (b & 31)) & 1u) && !a.built[tg.row];
+  if (tg.T == 0) a.trows[tg.row].active = active ? 1u : 0u;
+  return active;
+}
+__device__ __forceinline__ bool tile_active(const FusedArgs& a, uint32_t tile) {
+  const TileGeom tg = a.geom[tile];
+  return tg.span != 0 && a.trows[tg.row].active;
 }
 
 // The exact sum of tile `tile` by a wavefront: 16 slots per lane.
 __device__ __forceinline__ void tile_sum_wave(const FusedArgs& a, uint32_t tile) {
   const uint32_t lane = threadIdx.x & 63;
   const TileGeom tg = a.geom[tile];
-  if (tg.span == 0) return;  // there are fewer tiles than their bound
-  if (a.bitmap) {
-    const bool active = tile_active(a, tg.row);
-    if (tg.T == 0 && lane == 0) a.trows[tg.row].active = active ? 1u : 0u;
-    if (!active) return;
-  }
+  if (tg.span == 0) return;
   float4 x[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -200,7 +215,6 @@ __device__ __forceinline__ void tile_totals_wave(const FusedArgs& a, uint32_t ti
   const TileGeom tg = a.geom[tile];
   if (tg.span == 0) return;
   TiledRow* row = a.trows + tg.row;
-  if (a.bitmap && !row->active) return;
   float4 x[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -305,8 +319,12 @@ __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[(WAVE_LDS + 7) / 8];
   __shared__ uint64_t s_aux[8];
   call_stamp(a.call);
+  const uint32_t tiles = DEV && a.sec[0].kind == SEC_SUM ? a.sec[0].units : 0u;
+  if constexpr (DEV)
+    each_wanted(tiles, blockIdx.x, gridDim.x, [&](uint32_t t) { return tile_asked(a, a.tile0 + t); },
+                [&](uint32_t t) { tile_sum_wave(a, a.tile0 + t); });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = blockIdx.x;; u += gridDim.x) {
+  for (uint32_t u = tiles + blockIdx.x;; u += gridDim.x) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -331,7 +349,9 @@ __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
       case SEC_W1: merge_unit<DEV, 64, 4>(a, s, unit, rows, smem, s_aux); break;
       case SEC_W6: merge_unit<DEV, 64, 6>(a, s, unit, rows, smem, s_aux); break;
       case SEC_W2: merge_unit<DEV, 64, 8>(a, s, unit, rows, smem, s_aux); break;
-      case SEC_SUM: tile_sum_wave(a, a.tile0 + unit); break;
+      case SEC_SUM:
+        if constexpr (!DEV) tile_sum_wave(a, a.tile0 + unit);
+        break;
       default: break;
     }
     if (!DEV) return;
@@ -344,19 +364,25 @@ __global__ __launch_bounds__(128, 5) void fused_pair_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[(PAIR_LDS + 7) / 8];
   __shared__ uint64_t s_aux[16];
   call_stamp(a.call);
+  const uint32_t pairs = DEV && a.sec[0].kind == SEC_TOTALS ? a.sec[0].units : 0u;
+  if constexpr (DEV)
+    each_wanted(pairs * 2, blockIdx.x * 2 + (threadIdx.x >> 6), gridDim.x * 2,
+                [&](uint32_t t) { return t < a.sec[0].stride && tile_active(a, a.tile0 + t); },
+                [&](uint32_t t) { tile_totals_wave(a, a.tile0 + t); });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = blockIdx.x;; u += gridDim.x) {
+  for (uint32_t u = pairs + blockIdx.x;; u += gridDim.x) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
     switch (s.kind) {
       case SEC_P6: merge_unit<DEV, 128, 6>(a, s, unit, rows, smem, s_aux); break;
       case SEC_P8: merge_unit<DEV, 128, 8>(a, s, unit, rows, smem, s_aux); break;
-      case SEC_TOTALS: {
-        const uint32_t t = unit * 2 + (threadIdx.x >> 6);
-        if (t < s.stride) tile_totals_wave(a, a.tile0 + t);
+      case SEC_TOTALS:
+        if constexpr (!DEV) {
+          const uint32_t t = unit * 2 + (threadIdx.x >> 6);
+          if (t < s.stride) tile_totals_wave(a, a.tile0 + t);
+        }
         break;
-      }
       default: break;
     }
     if (!DEV) return;
@@ -373,10 +399,21 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
   // the wavefronts' sums of merge_row, past the end of their arrays
   uint64_t* const s_aux = smem + (WIDE_LDS - 512) / 8;
   call_stamp(a.call);
-  const UnitFinder<DEV> units(a);
+  auto scan = [&](uint32_t r) {
+    if (a.trows[r].ntiles && a.trows[r].ok)
+      tile_scan_row<512>(a.trows, r, a.ttot, a.BL, a.BH, a.nfh, a.ranges, *reinterpret_cast<TileScanLds<512>*>(smem));
+  };
   // Rows of tiles by every grid-th workgroup; the rows behind them, where a.next is given, by the workgroup that is first free.
-  const uint32_t scans = DEV && a.next && a.sec[0].kind == SEC_SCAN ? a.sec[0].units : 0u;
-  for (uint32_t u = blockIdx.x < scans ? blockIdx.x : scans + blockIdx.x;;) {
+  const uint32_t scans = DEV && a.sec[0].kind == SEC_SCAN ? a.sec[0].units : 0u;
+  if constexpr (DEV)
+    each_wanted(scans, blockIdx.x, gridDim.x, [&](uint32_t r) { return a.trows[a.trow0 + r].active != 0; },
+                [&](uint32_t r) {
+                  scan(a.trow0 + r);
+                  if (threadIdx.x == 0) a.built[a.trow0 + r] = 1;
+                  __syncthreads();
+                });
+  const UnitFinder<DEV> units(a);
+  for (uint32_t u = scans + blockIdx.x;;) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -392,23 +429,14 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
       case SEC_B6: merge_unit<DEV, 512, 6>(a, s, unit, rows, smem, s_aux); break;
       case SEC_B8: merge_unit<DEV, 512, 8>(a, s, unit, rows, smem, s_aux); break;
       case SEC_B10: merge_unit<DEV, 512, 10>(a, s, unit, rows, smem, s_aux); break;
-      case SEC_SCAN: {
-        const uint32_t r = a.trow0 + unit;
-        if (a.bitmap && !a.trows[r].active) break;
-        if (a.trows[r].ntiles && a.trows[r].ok)
-          tile_scan_row<512>(a.trows, r, a.ttot, a.BL, a.BH, a.nfh, a.ranges, *reinterpret_cast<TileScanLds<512>*>(smem));
-        if (a.bitmap && threadIdx.x == 0) a.built[r] = 1;
+      case SEC_SCAN:
+        if constexpr (!DEV) scan(a.trow0 + unit);
         break;
-      }
       default: break;
     }
     if (!DEV) return;
     if (!a.next) {
       u += gridDim.x;
-      __syncthreads();
-    } else if (u < scans) {
-      u += gridDim.x;
-      if (u >= scans) u = scans + blockIdx.x;
       __syncthreads();
     } else {
       u = scans + next_unit(a.next);
@@ -428,8 +456,18 @@ __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[((LONGER ? cmax(merge_lds_bytes(256, 14), BLOCK_LDS) : BLOCK_LDS) + 7) / 8];
   __shared__ uint64_t s_aux[32];
   call_stamp(a.call);
+  auto emit = [&](uint32_t tile) {
+    tile_emit(a.geom[tile], tile, a.trows, a.wgt, a.BL, a.BH, a.nfh, a.ranges, a.table, a.valid, *reinterpret_cast<TileEmitLds*>(smem));
+  };
+  const uint32_t tiles = DEV && a.sec[0].kind == SEC_EMIT ? a.sec[0].units : 0u;
+  if constexpr (DEV)
+    each_wanted(tiles, blockIdx.x, gridDim.x, [&](uint32_t t) { return tile_active(a, a.tile0 + near_tile(t, tiles)); },
+                [&](uint32_t t) {
+                  emit(a.tile0 + near_tile(t, tiles));
+                  __syncthreads();
+                });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = blockIdx.x;; u += gridDim.x) {
+  for (uint32_t u = tiles + blockIdx.x;; u += gridDim.x) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -440,14 +478,12 @@ __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
         if constexpr (LONGER) merge_unit<DEV, 256, 14>(a, s, unit, rows, smem, s_aux);
         break;
       case SEC_M10: merge_unit<DEV, 256, 10>(a, s, unit, rows, smem, s_aux); break;
-      case SEC_EMIT: {
-        const uint32_t tile = a.tile0 + near_tile(unit, s.units);
-        const TileGeom tg = a.geom[tile];
-        if (tg.span == 0 || (a.bitmap && !a.trows[tg.row].active)) break;
-        tile_emit(tg, tile, a.trows, a.wgt, a.BL, a.BH, a.nfh, a.ranges, a.table, a.valid,
-                  *reinterpret_cast<TileEmitLds*>(smem));
+      case SEC_EMIT:
+        if constexpr (!DEV) {
+          const uint32_t tile = a.tile0 + near_tile(unit, s.units);
+          if (a.geom[tile].span) emit(tile);
+        }
         break;
-      }
       default: break;
     }
     if (!DEV) return;

@@ -641,3 +641,26 @@ def test_a_vertex_that_starts_every_sample_is_not_swept_for_each_of_them():
     print("never %.1f us, by default %.1f us, always %.1f us" % (never * 1e6, default * 1e6, always * 1e6))
     assert default < 2 * never and 2 * default < always
     g.free()
+
+
+@pytest.mark.parametrize("asked", ["one", "tenth", "all", "none"])
+def test_frontiers_that_ask_for_some_of_many_rows_made_by_tiles(orc, asked):
+    # 500 rows of 9 to 13 tiles each, five tiles to a workgroup of the launch with the fewest, of which the frontier wants some
+    from skywalker_amd import capi
+    rng = np.random.default_rng(91)
+    degs = np.concatenate([rng.integers(8190, 12500, 500), np.full(20000, 3)])
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal2")
+    long_rows = np.flatnonzero(degs > 3).astype(np.uint32)
+    long_rows = {"one": long_rows[250:251], "tenth": long_rows[::10], "all": long_rows, "none": long_rows[:0]}[asked]
+    seeds = np.concatenate([long_rows, rng.permutation(np.flatnonzero(degs == 3))[:2000].astype(np.uint32)])
+    fan = [1, 7]
+    lps, slen = capi.sample_layout(fan)
+    want = orc.sample_online(xadj, adjncy, w, seeds, fan, 75)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_direct", 0)
+    for _ in range(2):
+        d, sl, sampled, _ = g.sample_online(seeds, fan, 75)
+        assert np.array_equal(sl.to_host((len(seeds), slen)), want[1]) and np.array_equal(d.to_host((len(seeds), lps)), want[0])
+        assert sampled == want[2]
+    g.free()
