@@ -664,3 +664,26 @@ def test_frontiers_that_ask_for_some_of_many_rows_made_by_tiles(orc, asked):
         assert np.array_equal(sl.to_host((len(seeds), slen)), want[1]) and np.array_equal(d.to_host((len(seeds), lps)), want[0])
         assert sampled == want[2]
     g.free()
+
+
+@pytest.mark.parametrize("kind", ["one", "two", "pairs", "far"])
+def test_vertices_that_a_workgroup_of_the_collection_meets_again(orc, kind):
+    # every lane the same vertex, two of them in turn, every vertex twice in a row, and vertices that share their places in LDS (the
+    # bits of 4,096 places apart, by the factor's inverse)
+    from skywalker_amd import capi
+    rng = np.random.default_rng(92)
+    V, n = 1 << 15, 2500
+    xadj, adjncy, w = graph_from_degrees(rng.integers(1, 9, V), rng, "uniform")
+    inverse = pow(2654435769, -1, V)
+    seeds = {"one": np.full(n, 77), "two": np.arange(n) % 2, "pairs": np.arange(n) // 2,
+             "far": np.array([(5 + 4096 * (i % 8)) * inverse % V for i in range(n)])}[kind].astype(np.uint32)
+    fan = [1, 2]
+    lps, slen = capi.sample_layout(fan)
+    want = orc.sample_online(xadj, adjncy, w, seeds, fan, 76)
+    for mode in (1, 0):  # by class in device-sized builds, and as a list
+        g = capi.Graph.upload(xadj, adjncy, w)
+        g.set_option("online_direct", 0)
+        g.set_option("online_device_sized", mode)
+        d, sl, sampled, _ = g.sample_online(seeds, fan, 76)
+        assert np.array_equal(sl.to_host((n, slen)), want[1]) and np.array_equal(d.to_host((n, lps)), want[0]) and sampled == want[2]
+        g.free()
