@@ -4,7 +4,7 @@
 // The class kernels of sky_build.hip give every degree class a launch of its own.  That is right where a class fills
 // the GPU for a millisecond; a build of 17 M entries spent 220 us on 27 launches of 5 to 25 us each, 2.4 us apart on
 // the host and each with a tail of its own, and spreading them over four streams costs 30 us for the fork and the
-// join alone.  Here one launch takes all classes whose rows need the same number of threads, and the passes of the
+// join by events alone.  Here one launch takes all classes whose rows need the same number of threads, and the passes of the
 // rows that are built tile by tile, which depend on one another, ride along in the same four launches:
 //
 //   fused_wave_kernel    64 threads    rows of up to 509 entries         tile sums
@@ -16,6 +16,16 @@
 // out in one launch of 512 threads instead (fused_all_kernel).  Every row builder is the one the class kernels call, so the
 // tables are the same bits.  The lists of rows by class and the geometry of the tiles depend on the row offsets alone:
 // they are made by the first build of a graph and kept with it.
+//
+// Only the passes over tiles depend on one another.  In a whole build the sweep over the rows of up to 32 entries, and behind it the rows
+// of 2558 and more, go out beside the rest (Beside, sky_call.h), so that the tails of four launches no longer follow one another.
+// (In order / beside, us, three graphs in turn: scale 16 with 16 edges a vertex 46 / 42, scale 20 with 16 131 / 120, with 6 96 / 82, with 3
+// 69 / 54, scale 23 with 4 253 / 233, with 10 437 / 433, 3 M entries in rows of up to 20,000 70 / 58, 40 M in rows of up to 300,007 331 / 319.
+// From 60 M entries on the tails no longer count: scale 22 with 31 649 / 655, scale 24 with 6 530 / 530.  On one graph again and again, with
+// the long rows in front of the sweep scale 23 with 10 483 instead of 430; those on a third stream scale 20 with 6 69 instead of 82, with 16 110
+// instead of 104, scale 16 with 16 45 instead of 42; rows of up to 107 entries alone, one launch in order, 128 / 138.)  The
+// workgroups of a frontier's launches stay until all units are done and leave no room beside them: those follow one another.  (The second
+// hop of 40,000 seeds on the scale-22 graph with 32 edges a vertex takes 10 to 90 us longer beside one another.)
 #include <algorithm>
 #include <cstddef>
 #include <type_traits>
@@ -74,6 +84,7 @@ struct FusedArgs {
   uint32_t tile0, trow0;  // first tile and row of those this build makes tile by tile
   bool ledgers_done;
   CallDevice* call;  // the call's first launch notes when it began
+  ForkMark fork;     // and the first of a fork that it runs
   uint32_t nsec;
   uint32_t first[MAX_SECTIONS];  // host-sized: first unit of every section, 2^32 - 1 past the last
   SectionRef sec[MAX_SECTIONS];
@@ -319,6 +330,7 @@ __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[(WAVE_LDS + 7) / 8];
   __shared__ uint64_t s_aux[8];
   call_stamp(a.call);
+  fork_mark(a.fork);
   const uint32_t tiles = DEV && a.sec[0].kind == SEC_SUM ? a.sec[0].units : 0u;
   if constexpr (DEV)
     each_wanted(tiles, blockIdx.x, gridDim.x, [&](uint32_t t) { return tile_asked(a, a.tile0 + t); },
@@ -364,6 +376,7 @@ __global__ __launch_bounds__(128, 5) void fused_pair_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[(PAIR_LDS + 7) / 8];
   __shared__ uint64_t s_aux[16];
   call_stamp(a.call);
+  fork_mark(a.fork);
   const uint32_t pairs = DEV && a.sec[0].kind == SEC_TOTALS ? a.sec[0].units : 0u;
   if constexpr (DEV)
     each_wanted(pairs * 2, blockIdx.x * 2 + (threadIdx.x >> 6), gridDim.x * 2,
@@ -399,6 +412,7 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
   // the wavefronts' sums of merge_row, past the end of their arrays
   uint64_t* const s_aux = smem + (WIDE_LDS - 512) / 8;
   call_stamp(a.call);
+  fork_mark(a.fork);
   auto scan = [&](uint32_t r) {
     if (a.trows[r].ntiles && a.trows[r].ok)
       tile_scan_row<512>(a.trows, r, a.ttot, a.BL, a.BH, a.nfh, a.ranges, *reinterpret_cast<TileScanLds<512>*>(smem));
@@ -456,6 +470,7 @@ __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
   __shared__ __align__(16) uint64_t smem[((LONGER ? cmax(merge_lds_bytes(256, 14), BLOCK_LDS) : BLOCK_LDS) + 7) / 8];
   __shared__ uint64_t s_aux[32];
   call_stamp(a.call);
+  fork_mark(a.fork);
   auto emit = [&](uint32_t tile) {
     tile_emit(a.geom[tile], tile, a.trows, a.wgt, a.BL, a.BH, a.nfh, a.ranges, a.table, a.valid, *reinterpret_cast<TileEmitLds*>(smem));
   };
@@ -777,27 +792,20 @@ bool streams_by_queue(const sky_graph* g, int tiled_from, bool longer) {
   return merges <= (uint64_t)g->bin_counts[CLS_STREAM_LAST] + (tiled_from > CLS_STREAM ? g->bin_counts[CLS_STREAM] : 0u);
 }
 
-// The four launches, in order on the graph's stream.
+// One launch, if it has anything to do.  Device-sized ones know a bound of their units only: as many workgroups as the GPU holds at a time
+// stride over what there is.
 template <bool DEV>
-int launch_all(sky_graph* g, const BuildPlan& p, Launch& wave, Launch& pair, Launch& wide, Launch& block, bool longer, CallDevice* call) {
-  hipStream_t st = g->stream;
-  // the first launch that has anything to do is the call's first
-  Launch* const order[4] = {&wave, &pair, &wide, &block};
-  for (Launch* l : order)
-    if (l->units) {
-      l->a.call = call;
-      break;
-    }
-  // Device-sized launches know a bound of their units only: as many workgroups as the GPU holds at a time stride
-  // over what there is.
-  auto grid = [&](const Launch& l, uint32_t cap) { return dim3((uint32_t)(DEV ? std::min<uint64_t>(l.units, cap) : l.units)); };
-  if (wave.units) hipLaunchKernelGGL((fused_wave_kernel<DEV>), grid(wave, 5120), dim3(64), 0, st, wave.a);
-  if (wave.a.ledgers_done) hipLaunchKernelGGL(fused_ledger_kernel, dim3(p.n_trows - wave.a.trow0), dim3(64), 0, st, p.trows, wave.a.trow0,
-                                              p.tsum, DEV);
-  if (pair.units) hipLaunchKernelGGL((fused_pair_kernel<DEV>), grid(pair, 2560), dim3(128), 0, st, pair.a);
-  if (wide.units) hipLaunchKernelGGL((fused_wide_kernel<DEV>), grid(wide, 512), dim3(512), 0, st, wide.a);
-  if (block.units && longer) hipLaunchKernelGGL((fused_block_kernel<DEV, true>), grid(block, 1024), dim3(256), 0, st, block.a);
-  else if (block.units) hipLaunchKernelGGL((fused_block_kernel<DEV, false>), grid(block, 1024), dim3(256), 0, st, block.a);
+int enqueue(const BuildPlan& p, const Launch& l, bool longer, hipStream_t st) {
+  if (!l.units) return SKY_OK;
+  const uint32_t resident = l.threads == 64 ? 5120 : l.threads == 128 ? 2560 : l.threads == 256 ? 1024 : 512;
+  const dim3 grid((uint32_t)(DEV ? std::min<uint64_t>(l.units, resident) : l.units));
+  if (l.threads == 64) hipLaunchKernelGGL((fused_wave_kernel<DEV>), grid, dim3(64), 0, st, l.a);
+  else if (l.threads == 128) hipLaunchKernelGGL((fused_pair_kernel<DEV>), grid, dim3(128), 0, st, l.a);
+  else if (l.threads == 512) hipLaunchKernelGGL((fused_wide_kernel<DEV>), grid, dim3(512), 0, st, l.a);
+  else if (longer) hipLaunchKernelGGL((fused_block_kernel<DEV, true>), grid, dim3(256), 0, st, l.a);
+  else hipLaunchKernelGGL((fused_block_kernel<DEV, false>), grid, dim3(256), 0, st, l.a);
+  if (l.a.nsec && l.a.sec[0].kind == SEC_SUM && l.a.ledgers_done)
+    hipLaunchKernelGGL(fused_ledger_kernel, dim3(p.n_trows - l.a.trow0), dim3(64), 0, st, p.trows, l.a.trow0, p.tsum, DEV);
   SKY_HIP(hipGetLastError());
   return SKY_OK;
 }
@@ -854,20 +862,11 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
       return SKY_OK;
     }
   }
-  Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
-  wave.add(SEC_SUM, n_tiles, 1, 0);
-  wave.add(SEC_W2, rows(CLS_LDS_W2), 1, p.start[CLS_LDS_W2]);
-  if (min_degree == 0) wave.add(SEC_SWEEP, sweeps, 1, 0);
-  wave.add(SEC_W6, rows(CLS_LDS_W6), 1, p.start[CLS_LDS_W6]);
-  wave.add(SEC_W1, rows(CLS_LDS_W1), 1, p.start[CLS_LDS_W1]);
-  wave.add(SEC_G32X, rows(CLS_G32X), 64 / SHAPE_G32X.lanes, p.start[CLS_G32X]);
-  wave.add(SEC_G32S, rows(CLS_G32S), 64 / SHAPE_G32S.lanes, p.start[CLS_G32S]);
-  wave.add(SEC_G32, rows(CLS_G32), 64 / SHAPE_G32.lanes, p.start[CLS_G32]);
-  wave.add(SEC_G16, rows(CLS_G16), 64 / SHAPE_G16.lanes, p.start[CLS_G16]);
+  Launch pair(base, 128), scan(base, 512), block(base, 256), rest(base, 64), wide(base, 512);
   pair.add(SEC_TOTALS, n_tiles, 2, 0);
   pair.add(SEC_P8, rows(CLS_MW2), 1, p.start[CLS_MW2]);
   pair.add(SEC_P6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
-  wide.add(SEC_SCAN, n_trows, 1, 0);
+  scan.add(SEC_SCAN, n_trows, 1, 0);
   if (p.t_all > CLS_STREAM) wide.add(SEC_STREAM, rows(CLS_STREAM), 1, p.start[CLS_STREAM]);
   if (p.t_all > CLS_STREAM_LAST) wide.add(SEC_STREAM, rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM_LAST]);
   // Rows of 5118..8189 entries: streamed beside the others, where hold_row would spill, or, where they are enough for a launch,
@@ -889,8 +888,39 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   block.add(SEC_M10, rows(CLS_MW2 + 3), 1, p.start[CLS_MW2 + 3]);
   block.add(SEC_M8, rows(CLS_MW2 + 2), 1, p.start[CLS_MW2 + 2]);
   block.add(SEC_M6, rows(CLS_MW2 + 1), 1, p.start[CLS_MW2 + 1]);
-  SKY_TRY(launch_all<false>(g, p, wave, pair, wide, block, longer, call));
-  return hold_alone ? build_rows_hold(g, p.rows + p.start[CLS_HOLD], rows(CLS_HOLD)) : SKY_OK;
+  // Rows of up to 509 entries alone are one launch; beside others the sweep goes to the side.
+  const bool sides = pair.units + scan.units + block.units + wide.units > 0;
+  Launch wave(base, 64);
+  wave.add(SEC_SUM, n_tiles, 1, 0);
+  wave.add(SEC_W2, rows(CLS_LDS_W2), 1, p.start[CLS_LDS_W2]);
+  if (min_degree == 0) (sides ? rest : wave).add(SEC_SWEEP, sweeps, 1, 0);
+  wave.add(SEC_W6, rows(CLS_LDS_W6), 1, p.start[CLS_LDS_W6]);
+  wave.add(SEC_W1, rows(CLS_LDS_W1), 1, p.start[CLS_LDS_W1]);
+  wave.add(SEC_G32X, rows(CLS_G32X), 64 / SHAPE_G32X.lanes, p.start[CLS_G32X]);
+  wave.add(SEC_G32S, rows(CLS_G32S), 64 / SHAPE_G32S.lanes, p.start[CLS_G32S]);
+  wave.add(SEC_G32, rows(CLS_G32), 64 / SHAPE_G32.lanes, p.start[CLS_G32]);
+  wave.add(SEC_G16, rows(CLS_G16), 64 / SHAPE_G16.lanes, p.start[CLS_G16]);
+  Launch* const order[] = {&wave, &pair, &scan, &block, &rest, &wide};  // the last two beside the others, which depend on one another
+  Launch* first = nullptr;
+  for (Launch* l : order)
+    if (l->units && !first) first = l;
+  if (!first) return hold_alone ? build_rows_hold(g, p.rows + p.start[CLS_HOLD], rows(CLS_HOLD)) : SKY_OK;
+  first->a.call = call;
+  Beside side;
+  if (rest.units + wide.units && first != &rest && first != &wide) SKY_TRY(beside_begin(g, &side, &first->a.fork));
+  SKY_TRY(enqueue<false>(p, *first, longer, g->stream));
+  auto others = [&]() -> int {
+    if (side.stream) SKY_TRY(beside_fork(side));
+    for (Launch* l : {&rest, &wide})
+      if (l != first) SKY_TRY(enqueue<false>(p, *l, longer, side.stream ? side.stream : g->stream));
+    for (Launch* l : {&wave, &pair, &scan, &block})
+      if (l != first) SKY_TRY(enqueue<false>(p, *l, longer, g->stream));
+    if (hold_alone) SKY_TRY(build_rows_hold(g, p.rows + p.start[CLS_HOLD], rows(CLS_HOLD)));
+    return side.stream ? beside_join(side) : SKY_OK;
+  };
+  const int rc = others();
+  if (rc != SKY_OK && side.stream) beside_drop(side);
+  return rc;
 }
 int build_all_fused(sky_graph* g, CallDevice* call) { return build_host_sized(g, 0, call); }
 int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call) { return build_host_sized(g, min_degree, call); }
@@ -967,7 +997,8 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
   add(block, SEC_M10, 1, CLS_MW2 + 3);
   add(block, SEC_M8, 1, CLS_MW2 + 2);
   add(block, SEC_M6, 1, CLS_MW2 + 1);
-  return launch_all<true>(g, p, wave, pair, wide, block, longer, nullptr);
+  for (const Launch* l : {&wave, &pair, &wide, &block}) SKY_TRY(enqueue<true>(p, *l, longer, g->stream));
+  return SKY_OK;
 }
 
 }  // namespace sky

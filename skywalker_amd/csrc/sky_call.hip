@@ -91,6 +91,7 @@ int take_words(int device, CallWords* w) {
   w->khz = use->khz;
   w->seq = use->host[k].sampled >> CALL_VALUE_BITS;  // not the next call's
   w->asked = use->host[k].answer[0] >> CALL_VALUE_BITS;
+  w->forks = use->host[k].begun;
   return SKY_OK;
 }
 }  // namespace
@@ -127,6 +128,55 @@ int call_begin(sky_graph* g, CallDevice** call) { return call_begin(g, &g->call,
 
 void call_cancel(sky_graph* g) { g->call.dirty = false; }
 
+// ---------------------------------------------------------------- beside the graph's stream
+namespace {
+constexpr int MAX_DEVICES = 64;
+struct SideStream {
+  hipStream_t stream = nullptr;
+  bool tried = false;
+} g_side[MAX_DEVICES];  // one per device, which it keeps until the process ends
+}  // namespace
+
+__global__ void beside_done_kernel(CallHost* host, uint32_t number) {
+  __hip_atomic_store(&host->done, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
+  *b = Beside{};
+  *mark = ForkMark{nullptr, 0};
+  if (g->device < 0 || g->device >= MAX_DEVICES) return SKY_OK;
+  if (!g->call.host) SKY_TRY(take_words(g->device, &g->call));
+  {
+    std::lock_guard<std::mutex> lock(g_mutex);
+    SideStream& side = g_side[g->device];
+    if (!side.tried) {
+      int can = 0;
+      SKY_HIP(hipDeviceGetAttribute(&can, hipDeviceAttributeCanUseStreamWaitValue, g->device));
+      if (can) SKY_HIP(hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking));
+      side.tried = true;
+    }
+    b->stream = side.stream;
+  }
+  if (!b->stream) return SKY_OK;
+  b->g = g;
+  b->host = g->call.host;
+  b->number = ++g->call.forks;
+  *mark = ForkMark{&b->host->begun, b->number};
+  return SKY_OK;
+}
+int beside_fork(const Beside& b) {
+  SKY_HIP(hipStreamWaitValue32(b.stream, &b.host->begun, b.number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+  return SKY_OK;
+}
+int beside_join(const Beside& b) {
+  hipLaunchKernelGGL(beside_done_kernel, dim3(1), dim3(1), 0, b.stream, b.host, b.number);
+  SKY_HIP(hipGetLastError());
+  SKY_HIP(hipStreamWaitValue32(b.g->stream, &b.host->done, b.number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+  return SKY_OK;
+}
+void beside_drop(const Beside& b) { (void)hipStreamSynchronize(b.stream); }
+
+// ---------------------------------------------------------------- the end
 // Up to this many counts are added up by the end kernel itself; more get a grid of their own.
 constexpr uint64_t END_COUNTS = 32768;
 // The host polls this long before it hands the wait to the runtime: a call that takes longer does not notice the

@@ -859,3 +859,43 @@ def test_rows_of_8190_to_24576_entries_streamed_and_longer_ones_by_tiles(orc, se
     assert np.array_equal(got[0], want[0].ravel()) and np.array_equal(got[1], want[1].ravel()) and sampled == want[2]
     paths, lengths, steps = orc.walk_offline(xadj, adjncy, oprob, oalias, seeds, 9, 0.0, 5)
     assert np.array_equal(walked[0], paths.ravel()) and np.array_equal(walked[1], lengths) and walk[2] == steps
+
+
+@pytest.mark.parametrize("longest", [600, 13000, 30000, 70001])
+def test_builds_over_two_streams_one_after_another_and_from_two_threads(orc, longest):
+    # the sweep and the long rows beside the other launches, a tile path among these for the longest: two weight arrays in turn, so that
+    # what an earlier build left shows, written just before each build and read just after it; two graphs, a thread each
+    import threading
+    from helpers import weights
+    from skywalker_amd import capi
+    made, errors = [], []
+    for k in range(2):
+        rng = np.random.default_rng(longest + k)
+        degs = np.concatenate([rng.integers(0, 33, 40000), rng.integers(33, 510, 4000), rng.integers(510, min(longest, 6000) + 1, 1500),
+                               rng.integers(min(longest, 8190), longest + 1, 12), [longest]])
+        rng.shuffle(degs)
+        xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal")
+        sets = [w, weights(len(w), rng, "lognormal2")]
+        made.append((capi.Graph.upload(xadj, adjncy, w), sets, [orc.alias_build(xadj, x) for x in sets]))
+
+    def builds(g, sets, want):
+        try:
+            for n in range(6):
+                x = capi.DeviceArray.from_host(np.concatenate([sets[n % 2], np.zeros(4, np.float32)]))
+                g.build_tables_from_weights(x)
+                prob, alias, valid = g.tables()
+                oprob, oalias, ovalid = want[n % 2]
+                assert np.array_equal(prob.view(np.uint32), oprob.view(np.uint32)) and np.array_equal(alias, oalias), n
+                assert np.array_equal(valid, ovalid), n
+        except BaseException as e:  # a thread's failure is the test's
+            errors.append(e)
+    builds(*made[0])
+    threads = [threading.Thread(target=builds, args=m) for m in made]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for g, _, _ in made:
+        g.free()
+    if errors:
+        raise errors[0]
