@@ -48,8 +48,9 @@ __global__ __launch_bounds__(256) void build_group_kernel(const RowRef* __restri
 }
 
 __global__ __launch_bounds__(128) void build_begin_kernel(uint32_t* __restrict__ counters, uint32_t words,
-                                                          CallDevice* call) {
+                                                          CallDevice* call, ForkMark fork) {
   call_stamp(call);
+  fork_mark(fork);
   for (uint32_t i = threadIdx.x; i < words; i += 128u) counters[i] = 0;
 }
 
@@ -638,88 +639,47 @@ void pool_release(sky_graph* g) {
     b.p = nullptr;
     b.cap = 0;
   }
-  for (hipStream_t& s : g->side) {
-    if (s) (void)hipStreamDestroy(s);
-    s = nullptr;
-  }
-  for (hipEvent_t& e : g->join_ev) {
-    if (e) (void)hipEventDestroy(e);
-    e = nullptr;
-  }
-  if (g->fork_ev) (void)hipEventDestroy(g->fork_ev);
-  g->fork_ev = nullptr;
 }
 
-// The class kernels of one build are independent of one another once their lists are there.  A build of up to 1 G entries
-// sends them out over the graph's stream and three side streams (a class of few rows takes as long as one row, and
-// the tail of one kernel is filled by another); the graph's stream waits for the others at the end.  Not used when
-// every kernel is timed on its own.
-constexpr uint64_t FAN_MIN_EDGES = 2000000, FAN_MAX_EDGES = 1ull << 30;
+// The class kernels of one build are independent of one another once their lists are there: they go out over the graph's stream
+// and three side streams (a class of few rows takes as long as one row, and the tail of one kernel is filled by another), and the
+// graph's stream waits for the others at the end.  Not used when every kernel is timed on its own.
+// (With events for the waits, and one stream for the classes of builds of 1 G entries and more / now, us: scale 26 with 8 edges a vertex
+// 2,452 / 2,379, with 28 8,083 / 8,036, means of five processes a side, of which those of the latter differ by 200; scale 23 with 40
+// 1,535 / 1,495, scale 22 with 50 965 / 937, scale 24 with 16 1,235 / 1,230.  The streaming kernel in front of the merge kernels, the
+// short rows behind them, or two streams instead of four: the same or up to 5 % slower.)
+constexpr uint64_t FAN_MIN_EDGES = 2000000;
 struct StreamFan {
-  sky_graph* g;
+  Beside b;
   hipStream_t main;
-  bool on = false, joinable = false, used[sky_graph::SIDE_STREAMS] = {false, false, false};
-  int turn = 0;
-  StreamFan(sky_graph* g_, hipStream_t m) : g(g_), main(m) {}
-  int ensure() {
-    for (int k = 0; k < sky_graph::SIDE_STREAMS; ++k) {
-      if (!g->side[k]) SKY_HIP(hipStreamCreateWithFlags(&g->side[k], hipStreamNonBlocking));
-      if (!g->join_ev[k]) SKY_HIP(hipEventCreateWithFlags(&g->join_ev[k], hipEventDisableTiming));
-    }
-    if (!g->fork_ev) SKY_HIP(hipEventCreateWithFlags(&g->fork_ev, hipEventDisableTiming));
-    return SKY_OK;
-  }
-  // One side stream that starts from the present end of the graph's stream, whatever start() does later; join()
-  // waits for it.
+  bool on = false;
+  uint64_t load[SIDE_STREAMS + 1] = {0, 0, 0, 0};
+  explicit StreamFan(hipStream_t m) : main(m) {}
+  // One side stream, whatever start() does later; join() waits for it.
   int branch(int k, hipStream_t* out) {
-    SKY_TRY(ensure());
-    SKY_HIP(hipEventRecord(g->fork_ev, main));
-    SKY_HIP(hipStreamWaitEvent(g->side[k], g->fork_ev, 0));
-    used[k] = true;
-    joinable = true;
-    *out = g->side[k];
+    *out = main;
+    if (!b.stream[k]) return SKY_OK;
+    SKY_TRY(beside_fork(&b, k));
+    *out = b.stream[k];
     return SKY_OK;
   }
-  int start() {  // after the binning pass has been enqueued on the graph's stream
-    SKY_TRY(ensure());
-    SKY_HIP(hipEventRecord(g->fork_ev, main));
-    for (int k = 0; k < sky_graph::SIDE_STREAMS; ++k) SKY_HIP(hipStreamWaitEvent(g->side[k], g->fork_ev, 0));
-    on = true;
-    joinable = true;
-    return SKY_OK;
-  }
-  hipStream_t next() {
-    if (!on) return main;
-    const int k = turn++ % (sky_graph::SIDE_STREAMS + 1);
-    if (k == sky_graph::SIDE_STREAMS) return main;
-    used[k] = true;
-    return g->side[k];
-  }
+  void start() { on = b.stream[0] != nullptr; }
   // The stream that carries the least work so far (`work`: the launch's entries, weighted by the caller where a
   // kernel is slow): a kernel queued behind a long one waits for it while other streams run dry.
-  uint64_t load[sky_graph::SIDE_STREAMS + 1] = {0, 0, 0, 0};
-  hipStream_t next(uint64_t work) {
-    if (!on) return main;
+  int next(uint64_t work, hipStream_t* out) {
+    *out = main;
+    if (!on) return SKY_OK;
     int k = 0;
-    for (int i = 1; i <= sky_graph::SIDE_STREAMS; ++i)
+    for (int i = 1; i <= SIDE_STREAMS; ++i)
       if (load[i] < load[k]) k = i;
     load[k] += work + 1;
-    if (k == sky_graph::SIDE_STREAMS) return main;
-    used[k] = true;
-    return g->side[k];
+    return k == SIDE_STREAMS ? SKY_OK : branch(k, out);
   }
   int join() {
-    if (!joinable) return SKY_OK;
-    on = joinable = false;
-    for (int k = 0; k < sky_graph::SIDE_STREAMS; ++k)
-      if (used[k]) {
-        used[k] = false;
-        SKY_HIP(hipEventRecord(g->join_ev[k], g->side[k]));
-        SKY_HIP(hipStreamWaitEvent(main, g->join_ev[k], 0));
-      }
-    return SKY_OK;
+    on = false;
+    return beside_join(&b);
   }
-  ~StreamFan() { (void)join(); }  // an error in between still leaves the graph's stream behind every kernel
+  ~StreamFan() { beside_drop(&b); }  // after an error in between
 };
 // The graph's stream replaced for the duration of a call that takes it from the graph.
 struct StreamSwap {
@@ -813,7 +773,7 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   static_assert(sizeof(host) == COUNTER_BYTES, "counter block layout");
   const bool small_in_place = small_rows_in_place(g, src, n);
   const int listed_from = small_in_place ? CLS_G16 : CLS_G2;
-  StreamFan fan(g, st);
+  StreamFan fan(st);
   auto launch_small = [&](hipStream_t s) {
     const uint32_t per_wave = std::max(256u, std::min(SMALL_RANGE, n / 16384u / 64u * 64u));
     hipLaunchKernelGGL(small_rows_kernel, dim3((n + per_wave - 1) / per_wave), dim3(64), 0, s, g->xadj, g->adjwgt, src, n,
@@ -826,11 +786,14 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   if (planned) SKY_TRY(ensure_plan(g, &call));
   RowRef* vlist = planned ? g->plan->rows : sc.vlist;
   // clears the counters of the binning pass and, unless the plan's first kernel has, notes when the call began
-  hipLaunchKernelGGL(build_begin_kernel, dim3(1), dim3(128), 0, st, sc.counters, (uint32_t)(COUNTER_BYTES / 4), call);
+  ForkMark fork{nullptr, 0};
+  if (!tm && n > 0) SKY_TRY(beside_begin(g, &fan.b, &fork));
+  hipLaunchKernelGGL(build_begin_kernel, dim3(1), dim3(128), 0, st, sc.counters, (uint32_t)(COUNTER_BYTES / 4), call, fork);
+  SKY_HIP(hipGetLastError());
   if (n > 0) {
     if (small_in_place && !tm) {
       hipStream_t side;
-      SKY_TRY(fan.branch(sky_graph::SIDE_STREAMS - 1, &side));
+      SKY_TRY(fan.branch(SIDE_STREAMS - 1, &side));
       launch_small(side);
     }
     if (planned) {
@@ -864,13 +827,15 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   }
   uint64_t call_edges = 0;
   for (int c = 0; c < CLS_COUNT; ++c) call_edges += host.edges[c];
-  if (!tm && option(g, OPT_BUILD_STREAMS) && call_edges >= FAN_MIN_EDGES && call_edges < FAN_MAX_EDGES) SKY_TRY(fan.start());
+  if (!tm && option(g, OPT_BUILD_STREAMS) && call_edges >= FAN_MIN_EDGES) fan.start();
 
   auto grp = [&](int cls, auto kernel, int G, const char* name) -> int {
     const uint32_t cnt = counts[cls];
     if (cnt) {
       const uint32_t per_block = 256 / G;
-      hipLaunchKernelGGL(kernel, dim3((cnt + per_block - 1) / per_block), dim3(256), 0, fan.next(host.edges[cls]), vlist + starts[cls],
+      hipStream_t on;
+      SKY_TRY(fan.next(host.edges[cls], &on));
+      hipLaunchKernelGGL(kernel, dim3((cnt + per_block - 1) / per_block), dim3(256), 0, on, vlist + starts[cls],
                          cnt, g->adjwgt, g->table, g->valid);
     }
     return (tm && cnt) ? tm->mark(name, host.edges[cls]) : SKY_OK;  // no bracket for an empty class
@@ -891,7 +856,9 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     const uint32_t cnt = counts[cls];
     if (cnt) {
       const size_t bytes = (size_t)rowt * 4 * t * 16;
-      hipLaunchKernelGGL(kernel, dim3(cnt), dim3(rowt), bytes, fan.next(host.edges[cls]), vlist + starts[cls], g->xadj, g->adjwgt,
+      hipStream_t on;
+      SKY_TRY(fan.next(host.edges[cls], &on));
+      hipLaunchKernelGGL(kernel, dim3(cnt), dim3(rowt), bytes, on, vlist + starts[cls], g->xadj, g->adjwgt,
                          g->table, g->valid);
     }
     return (tm && cnt) ? tm->mark(name, host.edges[cls]) : SKY_OK;  // no bracket for an empty class
@@ -900,7 +867,9 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     const uint32_t cnt = counts[cls];
     if (cnt) {
       const size_t bytes = merge_lds_bytes(rowt, per);
-      hipLaunchKernelGGL(kernel, dim3(cnt), dim3(rowt), bytes, fan.next(host.edges[cls]), vlist + starts[cls],
+      hipStream_t on;
+      SKY_TRY(fan.next(host.edges[cls], &on));
+      hipLaunchKernelGGL(kernel, dim3(cnt), dim3(rowt), bytes, on, vlist + starts[cls],
                          g->adjwgt, g->table, g->valid);
     }
     return (tm && cnt) ? tm->mark(name, host.edges[cls]) : SKY_OK;  // no bracket for an empty class
@@ -952,14 +921,18 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   // (scale 26 8.25 -> 8.18 ms, scale 25 with 56 edges a vertex 8.8 -> 8.6); last of all, its longest rows would have no company.
   if (!stream_to_tiled && narrow_rows + wide_rows) {
     // the streaming kernel takes three times as long for an entry as the others when it shares the GPU with them
-    StreamSwap sw(g, fan.next(3 * (narrow_edges + (wide_streamed ? host.edges[CLS_STREAM_WIDE] : 0))));
+    hipStream_t on;
+    SKY_TRY(fan.next(3 * (narrow_edges + (wide_streamed ? host.edges[CLS_STREAM_WIDE] : 0)), &on));
+    StreamSwap sw(g, on);
     SKY_TRY(build_rows_stream(g, vlist + starts[CLS_STREAM_WIDE], wide_rows, vlist + starts[CLS_STREAM_LAST], narrow_rows));
     if (tm) SKY_TRY(tm->mark("stream", narrow_edges + (wide_streamed ? host.edges[CLS_STREAM_WIDE] : 0)));
   }
   // Rows of 5118..8189 entries: one workgroup holds the row (without row_merge they are built tile by tile).
   if (row_merge && counts[CLS_HOLD]) {
     {
-      StreamSwap sw(g, fan.next(2 * host.edges[CLS_HOLD]));
+      hipStream_t on;
+      SKY_TRY(fan.next(2 * host.edges[CLS_HOLD], &on));
+      StreamSwap sw(g, on);
       SKY_TRY(build_rows_hold(g, vlist + starts[CLS_HOLD], counts[CLS_HOLD]));
     }
     if (tm) SKY_TRY(tm->mark("hold", host.edges[CLS_HOLD]));
@@ -986,7 +959,9 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
     const uint32_t cnt = tiled_rows;
     uint32_t skipped = 0;
     {
-      StreamSwap sw(g, fan.next(2 * tiled_edges));
+      hipStream_t on;
+      SKY_TRY(fan.next(2 * tiled_edges, &on));
+      StreamSwap sw(g, on);
       SKY_TRY(build_rows_tiled(g, tiled_list, cnt, &skipped, tm, tiled_edges));
     }
     SKY_TRY(fan.join());
@@ -1032,7 +1007,7 @@ int bin_all_rows(sky_graph* g, int listed_from, RowRef** rows, uint32_t* start, 
   const uint32_t n = g->V, per_block = bin_per_block(n), blocks = n ? (n + per_block - 1) / per_block : 0;
   if (n) {
     hipLaunchKernelGGL(build_begin_kernel, dim3(1), dim3(128), 0, st, sc.counters, (uint32_t)(COUNTER_BYTES / 4),
-                       *first);
+                       *first, ForkMark{nullptr, 0});
     *first = nullptr;
     hipLaunchKernelGGL(bin_count_kernel, dim3(blocks), dim3(256), 0, st, g->xadj, (const uint32_t*)nullptr, n, per_block,
                        sc.blk_cnt, reinterpret_cast<unsigned long long*>(sc.counters + 2 * CLS_COUNT));

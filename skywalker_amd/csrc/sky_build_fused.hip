@@ -910,16 +910,16 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   if (rest.units + wide.units && first != &rest && first != &wide) SKY_TRY(beside_begin(g, &side, &first->a.fork));
   SKY_TRY(enqueue<false>(p, *first, longer, g->stream));
   auto others = [&]() -> int {
-    if (side.stream) SKY_TRY(beside_fork(side));
+    if (side.stream[0]) SKY_TRY(beside_fork(&side, 0));
     for (Launch* l : {&rest, &wide})
-      if (l != first) SKY_TRY(enqueue<false>(p, *l, longer, side.stream ? side.stream : g->stream));
+      if (l != first) SKY_TRY(enqueue<false>(p, *l, longer, side.stream[0] ? side.stream[0] : g->stream));
     for (Launch* l : {&wave, &pair, &scan, &block})
       if (l != first) SKY_TRY(enqueue<false>(p, *l, longer, g->stream));
     if (hold_alone) SKY_TRY(build_rows_hold(g, p.rows + p.start[CLS_HOLD], rows(CLS_HOLD)));
-    return side.stream ? beside_join(side) : SKY_OK;
+    return beside_join(&side);
   };
   const int rc = others();
-  if (rc != SKY_OK && side.stream) beside_drop(side);
+  if (rc != SKY_OK) beside_drop(&side);
   return rc;
 }
 int build_all_fused(sky_graph* g, CallDevice* call) { return build_host_sized(g, 0, call); }

@@ -24,8 +24,8 @@ constexpr int CALL_ANSWERS = 10;
 struct CallHost {
   unsigned long long sampled, ticks;
   unsigned long long answer[CALL_ANSWERS];  // in the course of a call, with a number of their own (call_ask)
-  uint32_t begun, done;  // what two streams wait for (Beside)
-  unsigned long long pad[3];
+  uint32_t begun, done[3];                  // what streams wait for (Beside)
+  unsigned long long pad[2];
 };
 constexpr int CALL_VALUE_BITS = 48;  // 2^48 edges fill the GPU's memory a thousand times over; 2^48 ticks of 10 ns are a month
 static_assert(sizeof(CallDevice) == 64 && sizeof(CallHost) == 128, "cache lines of their own");
@@ -69,15 +69,17 @@ __device__ __forceinline__ void call_answer(CallHost* host, unsigned long long n
   __hip_atomic_store(&host->answer[word], value | number << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 int call_answered(sky_graph* g, CallWords* w, unsigned long long* values, int n);
-// Kernels beside those of the graph's stream, on a stream that all graphs of a device share.  Each of the two waits for the other by a
-// word in pinned memory that a kernel writes and the waiting queue's command processor reads: the first kernel of the fork notes that
-// it runs (fork_mark), so that everything in front of it has ended, and a small last one that everything in front of it on the side has.
-// 2 us each way, where events and stream waits take 9 (two kernels of 40 us side by side 55 us in all, with events 68, one after
-// the other 89).  Who waits is enqueued behind the kernel that writes, so that every wait ends also where other threads' calls lie
-// between, and where both streams share a hardware queue.
+// Kernels beside those of the graph's stream, on streams that all graphs of a device share.  These and the graph's stream wait for one
+// another by words in pinned memory that a kernel writes and the waiting queue's command processor reads: a kernel on the graph's stream
+// notes that it runs (fork_mark), so that everything in front of it has ended, and a small last one on each of the others that everything
+// in front of it has.  2 us each way, where events and stream waits take 9 (two kernels of 40 us side by side 55 us in all, with
+// events 68, one after the other 89).  Who waits is enqueued behind the kernel that writes, so that every wait ends also where other
+// threads' calls lie between, and where streams share a hardware queue.
+constexpr int SIDE_STREAMS = 3;
 struct Beside {
-  sky_graph* g = nullptr;
-  hipStream_t stream = nullptr;  // null: no fork
+  hipStream_t main = nullptr;
+  hipStream_t stream[SIDE_STREAMS] = {nullptr, nullptr, nullptr};  // null: no fork
+  bool used[SIDE_STREAMS] = {false, false, false};
   CallHost* host = nullptr;
   uint32_t number = 0;
 };
@@ -90,12 +92,12 @@ __device__ __forceinline__ void fork_mark(const ForkMark& f) {
 }
 // A fork, and the mark for the next kernel on the graph's stream.  b->stream stays null on a device whose queues know no such wait.
 int beside_begin(sky_graph* g, Beside* b, ForkMark* mark);
-// With that kernel on its way: the side stream waits for its mark.
-int beside_fork(const Beside& b);
-// The graph's stream waits for what the side stream holds.
-int beside_join(const Beside& b);
-// Instead of a join, after an error: the host waits for the side stream.
-void beside_drop(const Beside& b);
+// With that kernel on its way: side stream k waits for its mark, if it does not already.
+int beside_fork(Beside* b, int k);
+// The graph's stream waits for what the side streams of the fork hold.
+int beside_join(Beside* b);
+// Instead of a join, after an error: the host waits for them.
+void beside_drop(Beside* b);
 // With the graph's own words.
 int call_begin(sky_graph* g, CallDevice** call);
 int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);

@@ -131,14 +131,15 @@ void call_cancel(sky_graph* g) { g->call.dirty = false; }
 // ---------------------------------------------------------------- beside the graph's stream
 namespace {
 constexpr int MAX_DEVICES = 64;
-struct SideStream {
-  hipStream_t stream = nullptr;
+struct SideStreams {
+  hipStream_t stream[SIDE_STREAMS] = {nullptr, nullptr, nullptr};
   bool tried = false;
-} g_side[MAX_DEVICES];  // one per device, which it keeps until the process ends
+} g_side[MAX_DEVICES];  // of every device, which keeps them until the process ends
+static_assert(sizeof(CallHost::done) / sizeof(CallHost::done[0]) == SIDE_STREAMS, "a word for each");
 }  // namespace
 
-__global__ void beside_done_kernel(CallHost* host, uint32_t number) {
-  __hip_atomic_store(&host->done, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+__global__ void beside_done_kernel(uint32_t* word, uint32_t number) {
+  __hip_atomic_store(word, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
@@ -146,35 +147,45 @@ int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
   *mark = ForkMark{nullptr, 0};
   if (g->device < 0 || g->device >= MAX_DEVICES) return SKY_OK;
   if (!g->call.host) SKY_TRY(take_words(g->device, &g->call));
-  {
-    std::lock_guard<std::mutex> lock(g_mutex);
-    SideStream& side = g_side[g->device];
-    if (!side.tried) {
-      int can = 0;
-      SKY_HIP(hipDeviceGetAttribute(&can, hipDeviceAttributeCanUseStreamWaitValue, g->device));
-      if (can) SKY_HIP(hipStreamCreateWithFlags(&side.stream, hipStreamNonBlocking));
-      side.tried = true;
-    }
-    b->stream = side.stream;
+  std::lock_guard<std::mutex> lock(g_mutex);
+  SideStreams& side = g_side[g->device];
+  if (!side.tried) {
+    int can = 0;
+    SKY_HIP(hipDeviceGetAttribute(&can, hipDeviceAttributeCanUseStreamWaitValue, g->device));
+    if (can)
+      for (hipStream_t& s : side.stream)
+        if (!s) SKY_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    side.tried = true;
   }
-  if (!b->stream) return SKY_OK;
-  b->g = g;
+  if (!side.stream[0]) return SKY_OK;
+  for (int k = 0; k < SIDE_STREAMS; ++k) b->stream[k] = side.stream[k];
+  b->main = g->stream;
   b->host = g->call.host;
   b->number = ++g->call.forks;
   *mark = ForkMark{&b->host->begun, b->number};
   return SKY_OK;
 }
-int beside_fork(const Beside& b) {
-  SKY_HIP(hipStreamWaitValue32(b.stream, &b.host->begun, b.number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+int beside_fork(Beside* b, int k) {
+  if (b->used[k]) return SKY_OK;
+  SKY_HIP(hipStreamWaitValue32(b->stream[k], &b->host->begun, b->number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+  b->used[k] = true;
   return SKY_OK;
 }
-int beside_join(const Beside& b) {
-  hipLaunchKernelGGL(beside_done_kernel, dim3(1), dim3(1), 0, b.stream, b.host, b.number);
-  SKY_HIP(hipGetLastError());
-  SKY_HIP(hipStreamWaitValue32(b.g->stream, &b.host->done, b.number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+int beside_join(Beside* b) {
+  for (int k = 0; k < SIDE_STREAMS; ++k) {
+    if (!b->used[k]) continue;
+    hipLaunchKernelGGL(beside_done_kernel, dim3(1), dim3(1), 0, b->stream[k], &b->host->done[k], b->number);
+    SKY_HIP(hipGetLastError());
+    SKY_HIP(hipStreamWaitValue32(b->main, &b->host->done[k], b->number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+    b->used[k] = false;
+  }
   return SKY_OK;
 }
-void beside_drop(const Beside& b) { (void)hipStreamSynchronize(b.stream); }
+void beside_drop(Beside* b) {
+  for (int k = 0; k < SIDE_STREAMS; ++k)
+    if (b->used[k]) (void)hipStreamSynchronize(b->stream[k]);
+  for (bool& u : b->used) u = false;
+}
 
 // ---------------------------------------------------------------- the end
 // Up to this many counts are added up by the end kernel itself; more get a grid of their own.

@@ -73,13 +73,6 @@ struct sky_graph {
   };
   PoolBuf pool[POOL_SLOTS];
   bool sampler_busy = false;  // a sampling session holds the slots from POOL_BITMAP on; other calls bring their own
-  // Side streams (default priority) over which a small build spreads its class kernels, the event they wait for
-  // and the events the graph's stream waits for afterwards; created on first use.
-  static constexpr int SIDE_STREAMS = 3;
-  hipStream_t side[SIDE_STREAMS] = {nullptr, nullptr, nullptr};
-  hipEvent_t fork_ev = nullptr;
-  hipEvent_t join_ev[SIDE_STREAMS] = {nullptr, nullptr, nullptr};
-
   // Class sizes of all vertices (of the classes from CLS_G2 on; entries also of CLS_TINY), valid once there is a plan.
   uint32_t bin_counts[32] = {0};
   unsigned long long bin_edges[32] = {0};

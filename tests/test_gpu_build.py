@@ -861,10 +861,12 @@ def test_rows_of_8190_to_24576_entries_streamed_and_longer_ones_by_tiles(orc, se
     assert np.array_equal(walked[0], paths.ravel()) and np.array_equal(walked[1], lengths) and walk[2] == steps
 
 
+@pytest.mark.parametrize("by_class", [False, True])
 @pytest.mark.parametrize("longest", [600, 13000, 30000, 70001])
-def test_builds_over_two_streams_one_after_another_and_from_two_threads(orc, longest):
-    # the sweep and the long rows beside the other launches, a tile path among these for the longest: two weight arrays in turn, so that
-    # what an earlier build left shows, written just before each build and read just after it; two graphs, a thread each
+def test_builds_over_several_streams_one_after_another_and_from_two_threads(orc, longest, by_class):
+    # the sweep and the long rows beside the other launches, a tile path among these for the longest, or the class kernels on four
+    # streams: two weight arrays in turn, so that what an earlier build left shows, written just before each build and read just after
+    # it; two graphs, a thread each
     import threading
     from helpers import weights
     from skywalker_amd import capi
@@ -877,6 +879,8 @@ def test_builds_over_two_streams_one_after_another_and_from_two_threads(orc, lon
         xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal")
         sets = [w, weights(len(w), rng, "lognormal2")]
         made.append((capi.Graph.upload(xadj, adjncy, w), sets, [orc.alias_build(xadj, x) for x in sets]))
+        if by_class:
+            made[k][0].set_option("small_in_place", k)
 
     def builds(g, sets, want):
         try:
