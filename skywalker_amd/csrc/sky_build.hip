@@ -645,7 +645,7 @@ void pool_release(sky_graph* g) {
 // and three side streams (a class of few rows takes as long as one row, and the tail of one kernel is filled by another), and the
 // graph's stream waits for the others at the end.  Not used when every kernel is timed on its own.
 // (With events for the waits, and one stream for the classes of builds of 1 G entries and more / now, us: scale 26 with 8 edges a vertex
-// 2,452 / 2,379, with 28 8,083 / 8,036, means of five processes a side, of which those of the latter differ by 200; scale 23 with 40
+// 2,435 / 2,368, with 28 8,013 / 8,010, means of ten processes a side, of which those of the latter differ by 200; scale 23 with 40
 // 1,535 / 1,495, scale 22 with 50 965 / 937, scale 24 with 16 1,235 / 1,230.  The streaming kernel in front of the merge kernels, the
 // short rows behind them, or two streams instead of four: the same or up to 5 % slower.)
 constexpr uint64_t FAN_MIN_EDGES = 2000000;

@@ -458,6 +458,23 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
   }
 }
 
+// The rows of up to 5117 entries of that launch by themselves: without the streamed rows' LDS a CU holds three workgroups instead of two.
+constexpr size_t MID_LDS = cmax(merge_lds_bytes(512, 10), cmax(merge_lds_bytes(512, 8), merge_lds_bytes(512, 6)));
+__global__ __launch_bounds__(512, 6) void fused_mid_kernel(FusedArgs a) {
+  __shared__ __align__(16) uint64_t smem[(MID_LDS + 7) / 8];
+  __shared__ uint64_t s_aux[64];
+  const UnitFinder<false> units(a);
+  SectionRef s;
+  uint32_t unit = 0, rows = 0;
+  if (!units.find(a, blockIdx.x, s, unit, rows)) return;
+  switch (s.kind) {
+    case SEC_B6: merge_unit<false, 512, 6>(a, s, unit, rows, smem, s_aux); break;
+    case SEC_B8: merge_unit<false, 512, 8>(a, s, unit, rows, smem, s_aux); break;
+    case SEC_B10: merge_unit<false, 512, 10>(a, s, unit, rows, smem, s_aux); break;
+    default: break;
+  }
+}
+
 // Tiles in an order in which neighbours run on the same XCD (workgroup u on u mod 8), 64 in a row: a tile reads the weights of those
 // it is paired with once more, and finds them in that XCD's cache.  (40 M entries, 11 M of them in tiles: 350 -> 345 us; 60 M: 531 -> 523.)
 __device__ __forceinline__ uint32_t near_tile(uint32_t u, uint32_t n) {
@@ -631,6 +648,13 @@ static_assert(ALL_LONGEST <= 24576, "none is of class CLS_STREAM");
 // edges a vertex 17.2 / 13.6, scale 10 with 8 17.7 / 13.6, scale 13 with 8 19.6 / 14.9, scale 15 with 3 19.0 / 15.5, with 20 32.3 / 32.5,
 // scale 16 with 8 25.5 / 26, scale 17 with 4 19.7 / 20.5, scale 18 with 3 25.7 / 28, scale 20 with 16 137 / 171).
 constexpr uint32_t SPLIT_SWEEP = 1u << 15;
+
+// Whole builds of at least so many entries send out the rows of 2558..5117 entries (3582.. beside block_takes_longer) in a launch of
+// their own, beside the others on a third stream, which costs smaller ones more (in the launch of the longer rows / by
+// themselves, us: scale 16 with 16 edges a vertex 43 / 46, scale 20 with 6 82 / 86, 10 M entries in rows of up to 50,000 100 / 103, of
+// up to 7,000 87 / 87, scale 20 with 16 119 / 119, with 30 193 / 187, scale 22 with 16 357 / 348, scale 23 with 10 432 / 421, 40 M entries in rows of
+// up to 5,000 249 / 232, of up to 300,007 319 / 314, 60 M of up to 9,000 362 / 365, scale 21 with 40 456 / 461).
+constexpr uint32_t MID_ALONE = 1u << 24;
 
 // Rows of 5118..8189 entries from which they are a launch of their own (10,000 rows of 6,500 streamed 478 us, held 402; 20,000
 // 885 and 745): fewer save less than a launch costs.
@@ -862,7 +886,8 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
       return SKY_OK;
     }
   }
-  Launch pair(base, 128), scan(base, 512), block(base, 256), rest(base, 64), wide(base, 512);
+  Launch pair(base, 128), scan(base, 512), block(base, 256), rest(base, 64), wide(base, 512), alone(base, 512);
+  Launch& mid = min_degree == 0 && g->E >= MID_ALONE ? alone : wide;
   pair.add(SEC_TOTALS, n_tiles, 2, 0);
   pair.add(SEC_P8, rows(CLS_MW2), 1, p.start[CLS_MW2]);
   pair.add(SEC_P6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
@@ -875,13 +900,13 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   if (!hold_alone) wide.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);
   // two classes whose lists lie back to back; min_degree may leave out the first
   auto add_two = [&](Launch& l, Section k, int c) { l.add(k, rows(c) + rows(c + 1), 1, p.start[rows(c) ? c : c + 1]); };
-  add_two(wide, SEC_B10, CLS_MW2 + 7);
+  add_two(mid, SEC_B10, CLS_MW2 + 7);
   const bool longer = block_takes_longer(g, p.t_all);
   if (longer) {
-    wide.add(SEC_B8, rows(CLS_MW2 + 6), 1, p.start[CLS_MW2 + 6]);
+    mid.add(SEC_B8, rows(CLS_MW2 + 6), 1, p.start[CLS_MW2 + 6]);
   } else {
-    add_two(wide, SEC_B8, CLS_MW2 + 5);
-    wide.add(SEC_B6, rows(CLS_MW2 + 4), 1, p.start[CLS_MW2 + 4]);
+    add_two(mid, SEC_B8, CLS_MW2 + 5);
+    mid.add(SEC_B6, rows(CLS_MW2 + 4), 1, p.start[CLS_MW2 + 4]);
   }
   block.add(SEC_EMIT, n_tiles, 1, 0);
   if (longer) add_two(block, SEC_M14, CLS_MW2 + 4);
@@ -889,7 +914,7 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   block.add(SEC_M8, rows(CLS_MW2 + 2), 1, p.start[CLS_MW2 + 2]);
   block.add(SEC_M6, rows(CLS_MW2 + 1), 1, p.start[CLS_MW2 + 1]);
   // Rows of up to 509 entries alone are one launch; beside others the sweep goes to the side.
-  const bool sides = pair.units + scan.units + block.units + wide.units > 0;
+  const bool sides = pair.units + scan.units + block.units + wide.units + alone.units > 0;
   Launch wave(base, 64);
   wave.add(SEC_SUM, n_tiles, 1, 0);
   wave.add(SEC_W2, rows(CLS_LDS_W2), 1, p.start[CLS_LDS_W2]);
@@ -900,19 +925,28 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   wave.add(SEC_G32S, rows(CLS_G32S), 64 / SHAPE_G32S.lanes, p.start[CLS_G32S]);
   wave.add(SEC_G32, rows(CLS_G32), 64 / SHAPE_G32.lanes, p.start[CLS_G32]);
   wave.add(SEC_G16, rows(CLS_G16), 64 / SHAPE_G16.lanes, p.start[CLS_G16]);
-  Launch* const order[] = {&wave, &pair, &scan, &block, &rest, &wide};  // the last two beside the others, which depend on one another
+  // The passes over tiles depend on one another, the last three launches on nothing; only a build without the others has one of them first.
+  Launch* const order[] = {&wave, &pair, &scan, &block, &rest, &wide};
   Launch* first = nullptr;
   for (Launch* l : order)
     if (l->units && !first) first = l;
-  if (!first) return hold_alone ? build_rows_hold(g, p.rows + p.start[CLS_HOLD], rows(CLS_HOLD)) : SKY_OK;
-  first->a.call = call;
   Beside side;
-  if (rest.units + wide.units && first != &rest && first != &wide) SKY_TRY(beside_begin(g, &side, &first->a.fork));
-  SKY_TRY(enqueue<false>(p, *first, longer, g->stream));
+  if (first) {
+    first->a.call = call;
+    if (rest.units + wide.units + alone.units && first != &rest && first != &wide) SKY_TRY(beside_begin(g, &side, &first->a.fork));
+    SKY_TRY(enqueue<false>(p, *first, longer, g->stream));
+  }
   auto others = [&]() -> int {
-    if (side.stream[0]) SKY_TRY(beside_fork(&side, 0));
+    hipStream_t on[2] = {g->stream, g->stream};
+    for (int k = 0; k < 2; ++k)
+      if (side.stream[k] && (k ? alone.units : rest.units + wide.units)) {
+        SKY_TRY(beside_fork(&side, k));
+        on[k] = side.stream[k];
+      }
     for (Launch* l : {&rest, &wide})
-      if (l != first) SKY_TRY(enqueue<false>(p, *l, longer, side.stream[0] ? side.stream[0] : g->stream));
+      if (l != first) SKY_TRY(enqueue<false>(p, *l, longer, on[0]));
+    if (alone.units) hipLaunchKernelGGL(fused_mid_kernel, dim3((uint32_t)alone.units), dim3(512), 0, on[1], alone.a);
+    SKY_HIP(hipGetLastError());
     for (Launch* l : {&wave, &pair, &scan, &block})
       if (l != first) SKY_TRY(enqueue<false>(p, *l, longer, g->stream));
     if (hold_alone) SKY_TRY(build_rows_hold(g, p.rows + p.start[CLS_HOLD], rows(CLS_HOLD)));

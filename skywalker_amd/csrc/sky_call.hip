@@ -145,7 +145,9 @@ __global__ void beside_done_kernel(uint32_t* word, uint32_t number) {
 int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
   *b = Beside{};
   *mark = ForkMark{nullptr, 0};
-  if (g->device < 0 || g->device >= MAX_DEVICES) return SKY_OK;
+  int current = -1;
+  SKY_HIP(hipGetDevice(&current));
+  if (g->device != current || current < 0 || current >= MAX_DEVICES) return SKY_OK;  // the graph's stream is the current device's
   if (!g->call.host) SKY_TRY(take_words(g->device, &g->call));
   std::lock_guard<std::mutex> lock(g_mutex);
   SideStreams& side = g_side[g->device];

@@ -903,3 +903,25 @@ def test_builds_over_several_streams_one_after_another_and_from_two_threads(orc,
         g.free()
     if errors:
         raise errors[0]
+
+
+@pytest.mark.parametrize("E", [(1 << 24) - 1, 1 << 24])
+def test_rows_of_2558_to_5117_entries_in_a_launch_of_their_own(orc, E):
+    # the smallest build that gives them one and the largest that does not; the edges of their classes
+    from skywalker_amd import capi
+    rng = np.random.default_rng(61)
+    degs = list(rng.integers(2558, 5118, 300)) + [2557, 2558, 3069, 3070, 3581, 3582, 4093, 4094, 4605, 4606, 5117, 5118] * 2 + \
+        list(rng.integers(1, 300, 20000)) + list(rng.integers(8190, 9000, 20))
+    left = E - sum(degs)
+    degs += [31] * (left // 31) + [left % 31]
+    rng.shuffle(degs)
+    xadj = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    adjncy = np.zeros(E, np.uint32)
+    w = rng.lognormal(0, 2, E).astype(np.float32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    for _ in range(2):
+        g.build_tables()
+    prob, alias, valid = g.tables()
+    g.free()
+    oprob, oalias, ovalid = orc.alias_build(xadj, w)
+    assert np.array_equal(prob.view(np.uint32), oprob.view(np.uint32)) and np.array_equal(alias, oalias) and np.array_equal(valid, ovalid)
