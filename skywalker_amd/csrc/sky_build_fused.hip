@@ -843,11 +843,15 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   FusedArgs base = common_args(g, p, p.t_all);
   const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
   base.list = p.rows;
-  // Vertices of a wavefront: enough wavefronts for every SIMD, but 256 rather than fewer where four wavefronts a SIMD remain: the
-  // rows of a few vertices fill no batch of their class.  (4.4 M entries in 870,000 rows 51 us with 64, 40 with 192; 6.3 M in
-  // 2 M rows 113 with 256, 124 with 512; 20 M in 4 M rows 115 with 448, 125 with 960.)
+  // Vertices of a wavefront: enough wavefronts for every SIMD, but 128 to 256 rather than fewer where four wavefronts a SIMD remain: the
+  // rows of a few vertices fill no batch of their class.  The last wavefronts of a sweep are what is left of it behind the launches beside
+  // it, so no more than that either where it makes 12,288 wavefronts.  (64 where there were fewer than 4,096 wavefronts of 128, 256 up to
+  // 2 M vertices, an 8,192th above / now, us: 3 M entries in 478,000 rows 44 / 36, scale 20 with 6 edges a vertex 83 / 78, scale 22 with 3
+  // 115 / 110, scale 23 with 4 232 / 219, 19 M entries in 4.8 M rows of up to 107, one launch, 133 / 130; scale 22 with 4 127 / 129, with 10
+  // 242 / 245; most others within 1 %.)
   base.split = g->V <= SPLIT_SWEEP;
-  base.per_wave = base.split ? 64u : std::max(64u, std::min(SMALL_RANGE, std::max(g->V / 8192u, std::min(256u, g->V / 4096u)) / 64u * 64u));
+  const uint32_t least = g->V > 1u << 20 ? 256u : std::min(192u, std::max(g->V / 4096u, std::min(128u, g->V / 2048u)));
+  base.per_wave = base.split ? 64u : std::max(64u, std::min(SMALL_RANGE, std::max(g->V / 12288u, least) / 64u * 64u));
   const uint32_t ranges = (g->V + base.per_wave - 1) / base.per_wave, sweeps = base.split ? 4 * ranges : ranges;
   auto rows = [&](int c) { return class_min_degree(c) >= min_degree ? g->bin_counts[c] : 0u; };
   uint32_t past_wave = 0;  // rows of more than 509 entries: what a second launch would be for
