@@ -436,9 +436,15 @@ __global__ __launch_bounds__(DIRECT_T) void sample_direct_kernel(SampleArgs a, c
 // LDS, entries and neighbours both, which also makes one dependent load of two.  A bit for every entry then says what is taken:
 // a prefix over the draws of their candidates' bits finds f, the bits before f are final, and a draw that meets one of
 // them goes on until it meets none, in the same round.  No more than k rounds, none of which leaves the CU: 1,024 seeds, 25 x 10 on the
-// scale-20 graph 50 -> 36 us.
+// scale-20 graph 50 -> 36 us.  The first draw that needs its next try takes that one and the one behind it for all draws of the
+// wavefront, which keep the candidates: a lane's random numbers take a wavefront as long as those of all, and ten tries are then drawn
+// five times, not as often as draws need them (1,024 seeds x 25 27.3 -> 24.2 us, 25 x 10 34.7 -> 33.5, 300 x 32 x 7 on the scale-21 graph 31.9 -> 28.6,
+// 5,000 x 15 x 10 x 5 154.5 -> 147; one at a time or five 1 to 2 % behind two.  Draw after draw instead of rounds: 34.4; tries taken
+// by the idle groups of a hop with one parent: 25.2).
 constexpr uint32_t DISTINCT_MAX_K = 64;  // largest fanout of this rule
 constexpr uint32_t DISTINCT_ROUNDS = 11;
+constexpr uint32_t DISTINCT_AHEAD = 2;  // tries that are taken together in a row in LDS
+static_assert((DISTINCT_ROUNDS - 1) % DISTINCT_AHEAD == 0 && 6 * (DISTINCT_ROUNDS - 1) <= 64, "the candidates of all tries fit 64 bits");
 // Entries a lane of a row that its group holds in LDS: 24 KB for 512 threads, four workgroups of which are all wavefronts that a CU takes.
 constexpr uint32_t DISTINCT_ROW = 4;
 __host__ __device__ inline uint32_t distinct_lanes(uint32_t k) {
@@ -482,12 +488,20 @@ __global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
       const bool held = G >= (T > 64 ? 8u : 16u) && deg > k && deg <= min(64u, DISTINCT_ROW * G);
       const uint32_t rbase = DISTINCT_ROW * gbase;
       if (held) {
+        AliasEntry x[DISTINCT_ROW];
+        uint32_t y[DISTINCT_ROW];
+#pragma unroll
+        for (uint32_t m = 0; m < DISTINCT_ROW; ++m) {  // all on their way before the first is waited for
+          const uint32_t j = min(m * G + i, deg - 1);
+          x[m] = a.table[o + j];
+          y[m] = a.adjncy[o + j];
+        }
 #pragma unroll
         for (uint32_t m = 0; m < DISTINCT_ROW; ++m) {
           const uint32_t j = m * G + i;
           if (j < deg) {
-            s_row[rbase + j] = a.table[o + j];
-            s_adj[rbase + j] = a.adjncy[o + j];
+            s_row[rbase + j] = x[m];
+            s_adj[rbase + j] = y[m];
           }
         }
       }
@@ -511,11 +525,23 @@ __global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        auto take = [&] {
+        auto drawn = [&] {
           const AliasEntry x = s_row[rbase + col];
-          cand = u < x.prob ? col : x.alias;
+          return u < x.prob ? col : x.alias;
         };
-        if (held && live) take();
+        if (held && live) cand = drawn();
+        uint64_t next = 0;  // candidates of the tries behind the first, 6 bits each, `filled` of them
+        uint32_t filled = 0;
+        auto fill = [&] {
+          if (held && live) {
+#pragma unroll
+            for (uint32_t m = 0; m < DISTINCT_AHEAD; ++m) {
+              numbers(filled + 1 + m);
+              next |= (uint64_t)drawn() << (6 * (filled + m));
+            }
+          }
+          filled += DISTINCT_AHEAD;
+        };
         for (;;) {
           const uint64_t bit = held && live ? 1ull << cand : 0ull;
           uint64_t before = bit;  // candidates of this draw and the earlier ones of its group, then of the earlier ones
@@ -534,14 +560,11 @@ __global__ __launch_bounds__(T) void sample_distinct_kernel(SampleArgs a) {
           const uint64_t final = bad ? shfl_u64(before, (int)((lane & ~(G - 1)) + f)) : 0ull;
           bool taken = i >= f && (bit & final);
           while (__any(taken)) {
+            if (taken && ++t == DISTINCT_ROUNDS) live = taken = false;
+            if (__any(taken && t > filled)) fill();
             if (taken) {
-              if (++t == DISTINCT_ROUNDS) {
-                live = taken = false;
-              } else {
-                numbers(t);
-                take();
-                taken = (final >> cand) & 1;
-              }
+              cand = (uint32_t)(next >> (6 * (t - 1))) & 63u;
+              taken = (final >> cand) & 1;
             }
           }
         }
