@@ -4,6 +4,8 @@
 // 29 microseconds around an empty kernel, this one 9 (MI355X, ROCm 7.2: 11 for launch and stream synchronisation, 4 for the events, 3
 // for the memset, 11 for the copy; against 6 for a launch that is polled for, 3 for the second launch).
 #pragma once
+#include <cstddef>
+
 #include "sky_common.h"
 
 struct sky_graph;
@@ -11,11 +13,16 @@ struct sky_graph;
 namespace sky {
 
 // Device words of a call.  All zero between calls: the end kernel clears what it has read.
+// Edges sampled so far, in parts: a word serves its atomics one after another, 5 to 6 ns each, so that 3,900 wavefronts that add to one, each
+// at its end, took 23 us of a walk of 104.  A cache line each, and as many as a wavefront has lanes to add them up, for CALL_MANY wavefronts
+// and more; fewer have the first (64 parts cost the end 0.6 us).  (One word / parts, us: 250,007 PPR walkers on the scale-24 graph with the index 104 /
+// 81, without 127 / 107, 1 M with 277 / 183, 1 M x 5 273 / 160, 200,000 x 40, scale 20, with the index 146 / 126, 100,000 x 60, scale 18, 126 / 120.)
+constexpr uint32_t CALL_PARTS = 64, CALL_PART_WORDS = 16, CALL_MANY = 512;
 struct CallDevice {
-  unsigned long long start;    // wall clock of the first kernel
-  unsigned long long sampled;  // edges sampled so far
+  unsigned long long start;  // wall clock of the first kernel
   unsigned long long entries, arrived, refused;  // sample_check_kernel; the last is left as it is
-  unsigned long long pad[3];
+  unsigned long long pad[12];
+  unsigned long long part[CALL_PARTS * CALL_PART_WORDS];
 };
 constexpr int CALL_ANSWERS = 10;
 // Pinned host words of a call, written by the end kernel: each carries the number of the call in its upper 16 bits, so that the
@@ -28,7 +35,7 @@ struct CallHost {
   unsigned long long pad[2];
 };
 constexpr int CALL_VALUE_BITS = 48;  // 2^48 edges fill the GPU's memory a thousand times over; 2^48 ticks of 10 ns are a month
-static_assert(sizeof(CallDevice) == 64 && sizeof(CallHost) == 128, "cache lines of their own");
+static_assert(sizeof(CallDevice) % 128 == 0 && offsetof(CallDevice, part) == 128 && sizeof(CallHost) == 128, "cache lines of their own");
 // Where a call reports.  A graph has one for the calls that begin and end within one entry point; a call that stays open
 // between entry points (a sampling session) has its own, because other calls on the graph begin and end meanwhile.
 struct CallWords {
@@ -37,6 +44,7 @@ struct CallWords {
   unsigned long long seq = 0, asked = 0;  // numbers of the last end and of the last question
   uint32_t forks = 0;                     // and of the last fork
   int khz = 0;
+  uint32_t parts = 0;  // words that the call's kernels add sampled edges to: none, one or CALL_PARTS
   bool dirty = false;  // a call has begun and not ended well: its device words may not be zero
 };
 
@@ -44,19 +52,24 @@ struct CallWords {
 __device__ __forceinline__ void call_stamp(CallDevice* call) {
   if (call && blockIdx.x == 0 && threadIdx.x == 0) call->start = wall_clock64();
 }
+// Adds to the edges sampled; `who`: the number of the workgroup or wavefront, parts: the call's (CallWords).
+__device__ __forceinline__ void call_sampled(CallDevice* call, uint32_t who, uint32_t parts, unsigned long long n) {
+  if (n) atomicAdd(&call->part[(who & (parts - 1u)) * CALL_PART_WORDS], n);
+}
 // Last statement of the call's last kernel, by one thread that has seen every other thread's contribution.  The host may go on
 // before the device words are zero again; who uses them next is a kernel behind this one on the device's null stream, whichever graph
 // it belongs to.
 __device__ __forceinline__ void call_report(CallDevice* call, CallHost* host, unsigned long long seq,
-                                            unsigned long long sampled) {
-  const unsigned long long start = call->start, ticks = start ? wall_clock64() - start : 0;  // 0: the call had nothing to launch
+                                            unsigned long long start, unsigned long long sampled) {
+  const unsigned long long ticks = start ? wall_clock64() - start : 0;  // 0: the call had nothing to launch
   constexpr unsigned long long VALUE = (1ull << CALL_VALUE_BITS) - 1;
   __hip_atomic_store(&host->sampled, (sampled & VALUE) | seq << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(&host->ticks, (ticks & VALUE) | seq << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   call->start = 0;
-  call->sampled = 0;
 }
 
+// How many words `waves` wavefronts that each add once should have.
+inline uint32_t call_parts(uint64_t waves) { return waves >= CALL_MANY ? CALL_PARTS : 1u; }
 // The device words of `w` (taken on first use), cleared; a call that ended in an error may have left something in them.
 int call_begin(sky_graph* g, CallWords* w, CallDevice** call);
 // Enqueues the end kernel behind what the call has put on the graph's stream, waits for it and hands out the results.

@@ -10,11 +10,23 @@ namespace sky {
 
 // One workgroup: adds up `counts` if there are any, reports.
 __global__ __launch_bounds__(1024) void call_end_kernel(CallDevice* call, CallHost* host, unsigned long long seq,
-                                                        const uint32_t* __restrict__ counts, uint32_t n) {
+                                                        const uint32_t* __restrict__ counts, uint32_t n, uint32_t parts) {
   __shared__ unsigned long long s_w[16];
-  unsigned long long t = 0;
+  const unsigned long long start = call->start;  // on its way meanwhile
+  unsigned long long t = 0, x = 0;
+  if (threadIdx.x < parts) {
+    unsigned long long* const part = &call->part[threadIdx.x * CALL_PART_WORDS];
+    x = *part;
+    if (x) *part = 0;
+  }
   if (n) {
-    for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) t += counts[i];
+    for (uint32_t i = threadIdx.x; i < n; i += 4 * blockDim.x) {
+      uint32_t c[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) c[k] = i + k * blockDim.x < n ? counts[i + k * blockDim.x] : 0u;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) t += c[k];
+    }
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
     if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = t;
@@ -22,8 +34,11 @@ __global__ __launch_bounds__(1024) void call_end_kernel(CallDevice* call, CallHo
     t = 0;
     for (uint32_t w = 0; w < blockDim.x / 64; ++w) t += s_w[w];
   }
-  if (threadIdx.x == 0) call_report(call, host, seq, call->sampled + t);
+  if (threadIdx.x >= 64) return;
+  if (parts > 1) x = shfl_u64(group_scan_u64<64>(x), 63);
+  if (threadIdx.x == 0) call_report(call, host, seq, start, t + x);
 }
+static_assert(CALL_PARTS == 64, "by the first wavefront");
 
 __global__ __launch_bounds__(256) void sum_counts_kernel(const uint32_t* __restrict__ x, uint64_t n, CallDevice* call) {
   __shared__ unsigned long long s_w[4];
@@ -33,10 +48,7 @@ __global__ __launch_bounds__(256) void sum_counts_kernel(const uint32_t* __restr
   for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
   if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = t;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned long long b = s_w[0] + s_w[1] + s_w[2] + s_w[3];
-    if (b) atomicAdd(&call->sampled, b);
-  }
+  if (threadIdx.x == 0) call_sampled(call, blockIdx.x, CALL_PARTS, s_w[0] + s_w[1] + s_w[2] + s_w[3]);
 }
 
 // The call words of all graphs and sessions: chunks of 64, per device, handed out one to an owner for its lifetime.  A chunk none of
@@ -235,10 +247,12 @@ int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, con
     hipLaunchKernelGGL(sum_counts_kernel, dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 1024)), dim3(256), 0, st, counts,
                        n, w->dev);
     n = 0;
+    w->parts = CALL_PARTS;
   }
   const unsigned long long seq = ++w->seq;
   hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, st, w->dev, w->host, seq, counts,
-                     (uint32_t)n);
+                     (uint32_t)n, w->parts);
+  w->parts = 0;
   SKY_HIP(hipGetLastError());
   static_assert(offsetof(CallHost, ticks) == offsetof(CallHost, sampled) + 8, "taken together");
   unsigned long long words[2];

@@ -136,7 +136,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
     const WalkEntry* __restrict__ index, const uint32_t* __restrict__ seeds, const uint32_t* __restrict__ live,
     const uint32_t* __restrict__ n_live_dev, uint32_t n_live, uint32_t V, uint32_t len, uint32_t s_begin,
     uint32_t s_end, float stop_prob, uint64_t seed, uint32_t* __restrict__ paths, uint32_t* __restrict__ lengths,
-    uint32_t* __restrict__ next_live, uint32_t* __restrict__ n_next, CallDevice* __restrict__ call,
+    uint32_t* __restrict__ next_live, uint32_t* __restrict__ n_next, CallDevice* __restrict__ call, uint32_t parts,
     unsigned long long* __restrict__ block_partials) {
   if (s_begin == 0) call_stamp(call);
   __shared__ unsigned long long s_part[WALK_BLOCK / 64];
@@ -246,8 +246,8 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
       for (int w = 0; w < WALK_BLOCK / 64; ++w) b += s_part[w];
       block_partials[blockIdx.x] = b;
     }
-  } else if ((threadIdx.x & 63) == 0 && tot) {
-    atomicAdd(&call->sampled, tot);
+  } else if ((threadIdx.x & 63) == 0) {
+    call_sampled(call, t / 64, parts, tot);
   }
 }
 
@@ -268,11 +268,11 @@ static void launch_walk(sky_graph* g, const uint32_t* seeds, const uint32_t* liv
   if (walk_reads_once(g))
     hipLaunchKernelGGL((walk_offline_kernel<INDEXED, true>), grid, block, 0, g->stream, g->xadj, g->adjncy, g->table,
                        INDEXED ? g->walk_index : nullptr, seeds, live, n_live_dev, n_live, g->V, len, s_begin, s_end, stop_prob,
-                       seed, paths, lengths, next_live, n_next, call, partials);
+                       seed, paths, lengths, next_live, n_next, call, g->call.parts, partials);
   else
     hipLaunchKernelGGL((walk_offline_kernel<INDEXED, false>), grid, block, 0, g->stream, g->xadj, g->adjncy, g->table,
                        INDEXED ? g->walk_index : nullptr, seeds, live, n_live_dev, n_live, g->V, len, s_begin, s_end, stop_prob,
-                       seed, paths, lengths, next_live, n_next, call, partials);
+                       seed, paths, lengths, next_live, n_next, call, g->call.parts, partials);
 }
 
 // Few walkers get a wavefront each.  Beyond ALONE_SCALAR the vector cache takes part (4,096 walkers x 80 steps on the scale-16 graph
@@ -315,6 +315,7 @@ int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, 
     else vec ? go(walk_alone_kernel<false, true>) : go(walk_alone_kernel<false, false>);
     return call_end(g, sampled, seconds, lengths, N);
   }
+  g->call.parts = call_parts((N + 63ull) / 64);
   if (N && !segmented) {
     run(seeds, (const uint32_t*)nullptr, (const uint32_t*)nullptr, N, len, 0u, len, stop_prob, seed, paths, lengths,
         (uint32_t*)nullptr, (uint32_t*)nullptr, call, (unsigned long long*)nullptr);
@@ -538,7 +539,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
     const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
     const AliasEntry* __restrict__ table, const uint32_t* __restrict__ seeds, uint32_t walker0, uint32_t N, uint32_t V, uint32_t len,
     float fp, float fq, float fmax, float stop_prob, uint64_t seed, bool once, uint32_t* __restrict__ paths,
-    uint32_t* __restrict__ lengths, CallDevice* __restrict__ call) {
+    uint32_t* __restrict__ lengths, CallDevice* __restrict__ call, uint32_t parts) {
   // One trial a turn: the numbers of the next one and of the next step's first are kept, which takes two lanes.  Four: those of the turn.
   static_assert(TR == 1 ? G >= 2 : TR == N2V_TRIALS && G >= TR, "a lane for every number that is kept");
   // Numbers kept of a step, a lane each, of the last one fewer.
@@ -658,7 +659,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
   unsigned long long t = first ? s : 0u;
 #pragma unroll
   for (int m = 32; m >= 1; m >>= 1) t += shfl_xor_u64(t, m);
-  if ((threadIdx.x & 63) == 0 && t) atomicAdd(&call->sampled, t);
+  if ((threadIdx.x & 63) == 0) call_sampled(call, blockIdx.x * (WALK_BLOCK / 64) + threadIdx.x / 64, parts, t);
 }
 
 int walk_node2vec_reject(sky_graph* g, float p, float q, const uint32_t* seeds, uint32_t N, uint32_t len,
@@ -679,12 +680,13 @@ int walk_node2vec_reject(sky_graph* g, float p, float q, const uint32_t* seeds, 
   SKY_TRY(call_begin(g, &call));
   auto run = [&](auto lanes, auto trials) {
     constexpr int G = decltype(lanes)::value;
+    g->call.parts = call_parts((uint64_t)N * G / 64);
     const uint64_t most = 0x80000000ull / G;  // walkers of one launch: below 2^32 threads
     for (uint64_t f = 0; f < N; f += most) {
       const uint64_t threads = std::min<uint64_t>(most, N - f) * G;
       hipLaunchKernelGGL((walk_n2v_reject_group_kernel<G, decltype(trials)::value>), dim3((uint32_t)((threads + WALK_BLOCK - 1) / WALK_BLOCK)),
                          dim3(WALK_BLOCK), 0, st, g->xadj, g->adjncy, g->table, seeds, (uint32_t)f, N, g->V, len, fp, fq, fmax,
-                         stop_prob, seed, walk_reads_once(g), paths, lengths, call);
+                         stop_prob, seed, walk_reads_once(g), paths, lengths, call, g->call.parts);
     }
   };
   using One = std::integral_constant<int, 1>;

@@ -610,3 +610,25 @@ def test_short_walks_from_well_connected_vertices_build_their_rows(orc, length, 
     print({k: "%.1f us" % (v * 1e6) for k, v in took.items()})
     assert took["hub"] < 3 * took["any"]
     g.free()
+
+
+@pytest.mark.parametrize("walkers", [32704, 32705, 32768, 32769, 100001])
+def test_sampled_edges_counted_in_one_word_and_in_many(orc, walkers):
+    # 511 and 512 wavefronts of a walker a lane, which add to one word and to 64, more of them in the rejection walk, counts behind a
+    # kernel of their own: one call after another on the same words, each of which starts from zero
+    from skywalker_amd import capi
+    xadj, adjncy = orc.rmat_csr(12, 8, 77)
+    w = orc.gen_weights(orc.W_UNIFORM, 77, len(adjncy), 1.0, 100.0)
+    seeds = orc.gen_seeds(3, 1 << 12, walkers)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_full_build", 0)
+    runs = [lambda: g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 2, 0.0, 5)]
+    for _ in range(2):
+        runs += [lambda: g.walk_offline(seeds, 6, 0.15, 5), lambda: g.walk_online(capi.BIAS_NODE2VEC_REJECT, 2.0, 0.5, seeds, 4, 0.0, 5),
+                 lambda: g.walk_online(capi.BIAS_NODE2VEC_REJECT, 0.25, 1.0, seeds[:700], 4, 0.0, 5), lambda: g.walk_offline(seeds[:100], 6, 0.0, 5)]
+    for k, run in enumerate(runs):
+        if k == 1:
+            g.build_tables()
+        _, lengths, sampled, _ = run()
+        assert sampled == int(lengths.to_host().sum()) > 0, k
+    g.free()
