@@ -137,10 +137,11 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
     const uint32_t* __restrict__ n_live_dev, uint32_t n_live, uint32_t V, uint32_t len, uint32_t s_begin,
     uint32_t s_end, float stop_prob, uint64_t seed, uint32_t* __restrict__ paths, uint32_t* __restrict__ lengths,
     uint32_t* __restrict__ next_live, uint32_t* __restrict__ n_next, CallDevice* __restrict__ call, uint32_t parts,
-    unsigned long long* __restrict__ block_partials) {
+    unsigned long long* __restrict__ block_partials, uint32_t per) {
   if (s_begin == 0) call_stamp(call);
   __shared__ unsigned long long s_part[WALK_BLOCK / 64];
-  const uint32_t t = blockIdx.x * WALK_BLOCK + threadIdx.x;
+  const uint32_t wave = blockIdx.x * (WALK_BLOCK / 64) + (threadIdx.x >> 6);
+  const uint32_t t = (threadIdx.x & 63) < per ? wave * per + (threadIdx.x & 63) : 0xFFFFFFFFu;
   if (n_live_dev) n_live = min(n_live, *n_live_dev);  // the list's length is only known on the device
   uint32_t steps = 0;
   bool walking = false;
@@ -247,7 +248,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_offline_kernel(
       block_partials[blockIdx.x] = b;
     }
   } else if ((threadIdx.x & 63) == 0) {
-    call_sampled(call, t / 64, parts, tot);
+    call_sampled(call, wave, parts, tot);
   }
 }
 
@@ -263,16 +264,17 @@ template <bool INDEXED>
 static void launch_walk(sky_graph* g, const uint32_t* seeds, const uint32_t* live, const uint32_t* n_live_dev,
                         uint32_t n_live, uint32_t len, uint32_t s_begin, uint32_t s_end, float stop_prob, uint64_t seed,
                         uint32_t* paths, uint32_t* lengths, uint32_t* next_live, uint32_t* n_next,
-                        CallDevice* call, unsigned long long* partials) {
-  const dim3 grid((n_live + WALK_BLOCK - 1) / WALK_BLOCK), block(WALK_BLOCK);
+                        CallDevice* call, unsigned long long* partials, uint32_t per = 64) {
+  const uint32_t walkers = WALK_BLOCK / 64 * per;  // of a workgroup
+  const dim3 grid((n_live + walkers - 1) / walkers), block(WALK_BLOCK);
   if (walk_reads_once(g))
     hipLaunchKernelGGL((walk_offline_kernel<INDEXED, true>), grid, block, 0, g->stream, g->xadj, g->adjncy, g->table,
                        INDEXED ? g->walk_index : nullptr, seeds, live, n_live_dev, n_live, g->V, len, s_begin, s_end, stop_prob,
-                       seed, paths, lengths, next_live, n_next, call, g->call.parts, partials);
+                       seed, paths, lengths, next_live, n_next, call, g->call.parts, partials, per);
   else
     hipLaunchKernelGGL((walk_offline_kernel<INDEXED, false>), grid, block, 0, g->stream, g->xadj, g->adjncy, g->table,
                        INDEXED ? g->walk_index : nullptr, seeds, live, n_live_dev, n_live, g->V, len, s_begin, s_end, stop_prob,
-                       seed, paths, lengths, next_live, n_next, call, g->call.parts, partials);
+                       seed, paths, lengths, next_live, n_next, call, g->call.parts, partials, per);
 }
 
 // Few walkers get a wavefront each.  Beyond ALONE_SCALAR the vector cache takes part (4,096 walkers x 80 steps on the scale-16 graph
@@ -286,6 +288,14 @@ constexpr uint32_t ALONE_SCALAR = 2048;
 static uint32_t alone_walkers(const sky_graph* g, uint32_t len) {
   if (g->has_walk_index || len < 16) return ALONE_SCALAR;
   return len >= 24 && (uint64_t)g->E * sizeof(AliasEntry) > (4u << 20) ? 8192u : 4096u;
+}
+// Walkers of a wavefront beyond that: 16 while three such wavefronts to a SIMD hold them all, because each waits in every step for the
+// slowest of its gathers.  Not on tables that L2 holds, where it does not wait long.  (64 / 16, us: 10,000 PPR walkers on the scale-24 graph
+// with the index 33.9 / 30.7, 30,000 45 / 42.7, 50,000 without 57.5 / 54, 10,000 on the scale-22 graph 44.6 / 38, 12,000 x 80, scale 20,
+// 124 / 112, 20,000 x 80 on the scale-25 graph with 30 edges a vertex 162 / 152; 60,000 x 40, scale 20, 87 / 88, 130,000 with the index 59.5 / 60.7;
+// 30,000 x 60, scale 18, 78.7 / 80.2, 50,000 x 50 on the scale-14 graph 42.5 / 48.4.  32: in between.)
+static uint32_t lane_walkers(const sky_graph* g, uint32_t N) {
+  return N <= 3u * 1024u * 16u && (uint64_t)g->E * sizeof(AliasEntry) > (32u << 20) ? 16u : 64u;
 }
 int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, float stop_prob, uint64_t seed,
                  uint32_t* paths, uint32_t* lengths, uint64_t* sampled, double* seconds) {
@@ -315,10 +325,11 @@ int walk_offline(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32_t len, 
     else vec ? go(walk_alone_kernel<false, true>) : go(walk_alone_kernel<false, false>);
     return call_end(g, sampled, seconds, lengths, N);
   }
-  g->call.parts = call_parts((N + 63ull) / 64);
+  const uint32_t per = segmented ? 64u : lane_walkers(g, N);
+  g->call.parts = call_parts((N + per - 1ull) / per);
   if (N && !segmented) {
     run(seeds, (const uint32_t*)nullptr, (const uint32_t*)nullptr, N, len, 0u, len, stop_prob, seed, paths, lengths,
-        (uint32_t*)nullptr, (uint32_t*)nullptr, call, (unsigned long long*)nullptr);
+        (uint32_t*)nullptr, (uint32_t*)nullptr, call, (unsigned long long*)nullptr, per);
   } else if (N) {
     for (uint32_t k = 0; k < nseg; ++k) {
       const uint32_t s0 = k * every, s1 = std::min(len, s0 + every);

@@ -632,3 +632,25 @@ def test_sampled_edges_counted_in_one_word_and_in_many(orc, walkers):
         _, lengths, sampled, _ = run()
         assert sampled == int(lengths.to_host().sum()) > 0, k
     g.free()
+
+
+@pytest.mark.parametrize("index", [False, True])
+@pytest.mark.parametrize("walkers", [8193, 8207, 8208, 49152, 49153])
+def test_walks_of_sixteen_walkers_a_wavefront(orc, walkers, index):
+    # tables of more than 32 MB: partly filled wavefronts and workgroups, the most walkers that go sixteen to a wavefront and one more;
+    # walkers that end at vertices without edges, at the stop test, alone in their wavefronts, and at a start vertex that does not exist
+    from skywalker_amd import capi
+    xadj, adjncy = orc.rmat_csr(17, 34, 5)
+    w = orc.gen_weights(orc.W_UNIFORM, 5, len(adjncy), 1.0, 100.0)
+    seeds = orc.gen_seeds(3, 1 << 17, walkers)
+    seeds[-1] = 1 << 17
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.build_tables()
+    if index:
+        g.build_walk_index()
+    prob, alias, _ = g.tables()
+    for stop in (0.15, 0.0):
+        paths, lengths, sampled, _ = g.walk_offline(seeds, 24, stop, 9)
+        want = orc.walk_offline(xadj, adjncy, prob, alias, seeds, 24, stop, 9)
+        assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host((walkers, 25)), want[0]) and sampled == want[2]
+    g.free()
