@@ -38,6 +38,7 @@ struct FrontierLists {
   RowRef* list = nullptr;
   uint32_t start[CLS_COUNT] = {0}, cap[CLS_COUNT] = {0};
   int tiled_from = 0;
+  bool few = false;  // at most SMALL_FRONTIER rows
 };
 // A frontier's bitmap: the bit of vertex v.  A word serves its atomics one after another, and a graph's busiest vertices tend to
 // have neighbouring ids (R-MAT: one draw in a hundred lands on 32 of 4 M); an odd factor, modulo the number of bits, a power of

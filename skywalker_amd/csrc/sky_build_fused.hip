@@ -24,8 +24,8 @@
 // From 60 M entries on the tails no longer count: scale 22 with 31 649 / 655, scale 24 with 6 530 / 530.  On one graph again and again, with
 // the long rows in front of the sweep scale 23 with 10 483 instead of 430; those on a third stream scale 20 with 6 69 instead of 82, with 16 110
 // instead of 104, scale 16 with 16 45 instead of 42; rows of up to 107 entries alone, one launch in order, 128 / 138.)  The
-// workgroups of a frontier's launches stay until all units are done and leave no room beside them: those follow one another.  (The second
-// hop of 40,000 seeds on the scale-22 graph with 32 edges a vertex takes 10 to 90 us longer beside one another.)
+// workgroups of a large frontier's launches stay until all units are done and leave no room beside them: those follow one another.  (The
+// second hop of 40,000 seeds on the scale-22 graph with 32 edges a vertex takes 10 to 90 us longer beside one another.)
 #include <algorithm>
 #include <cstddef>
 #include <type_traits>
@@ -967,7 +967,8 @@ int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call) { retur
 int frontier_lists(sky_graph* g, const BuildPlan& p, uint32_t n_upper, sky_graph::PoolBuf* buf, FrontierLists* f) {
   // A workgroup needs 125 us to stream a row of 65,000 entries, which is as long as everything else that the build of a
   // small frontier does; the rows of a large one keep all workgroups streaming, and that is cheaper by the entry.
-  f->tiled_from = n_upper <= SMALL_FRONTIER ? p.t_first : p.t_all;
+  f->few = n_upper <= SMALL_FRONTIER;
+  f->tiled_from = f->few ? p.t_first : p.t_all;
   uint64_t at = 0;
   for (int c = 0; c < CLS_COUNT; ++c) {
     f->start[c] = (uint32_t)at;
@@ -994,12 +995,17 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
   base.bit_mask = frontier_mask(g->V);
   base.built = built;
   Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
+  Launch sum(base, 64), totals(base, 128), scan(base, 512), emit(base, 256);
+  // The passes over tiles wait for one another, and of a frontier of few rows they are a good part: the rows go out beside them, the longest
+  // first.  (In the same four launches / beside, us: 40,000 seeds x 20 on the scale-22 graph with 30 edges a vertex 125 / 115, 300 x 25 x 10 with
+  // 32 231 / 225, 2,000 x 10 x 10, scale 21 with 40, 338 / 329, 40,000 x 25 x 10, scale 22 with 32, 676 / 669; the rest within 1 %.)
+  const bool apart = f.few && n_tiles;
   auto add = [&](Launch& l, Section k, uint32_t per, int cls, int ncls = 1) {
     uint32_t upper = 0;
     for (int c = 0; c < ncls; ++c) upper += f.cap[cls + c];
     l.add_dev(k, upper, per, f.start[cls], cls, ncls, ncls > 1 ? f.start[cls + 1] - f.start[cls] : 0u);
   };
-  wave.add(SEC_SUM, n_tiles, 1, 0);
+  (apart ? sum : wave).add(SEC_SUM, n_tiles, 1, 0);
   add(wave, SEC_W2, 1, CLS_LDS_W2);
   add(wave, SEC_W6, 1, CLS_LDS_W6);
   add(wave, SEC_W1, 1, CLS_LDS_W1);
@@ -1011,10 +1017,10 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
   add(wave, SEC_G4, 64 / SHAPE_G4.lanes, CLS_G4);
   add(wave, SEC_G2, 64 / SHAPE_G2.lanes, CLS_G2);
   add(wave, SEC_TINY, 64, CLS_TINY);
-  pair.add(SEC_TOTALS, n_tiles, 2, 0);
+  (apart ? totals : pair).add(SEC_TOTALS, n_tiles, 2, 0);
   add(pair, SEC_P8, 1, CLS_MW2);
   add(pair, SEC_P6, 1, CLS_MW2_6);
-  wide.add(SEC_SCAN, n_trows, 1, 0);
+  (apart ? scan : wide).add(SEC_SCAN, n_trows, 1, 0);
   if (f.tiled_from > CLS_STREAM) add(wide, SEC_STREAM, 1, CLS_STREAM);
   if (f.tiled_from > CLS_STREAM_LAST) add(wide, SEC_STREAM, 1, CLS_STREAM_LAST);
   add(wide, SEC_STREAM, 1, CLS_HOLD);
@@ -1030,13 +1036,27 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
     add(wide, SEC_B8, 1, CLS_MW2 + 5, 2);
     add(wide, SEC_B6, 1, CLS_MW2 + 4);
   }
-  block.add(SEC_EMIT, n_tiles, 1, 0);
+  (apart ? emit : block).add(SEC_EMIT, n_tiles, 1, 0);
   if (longer) add(block, SEC_M14, 1, CLS_MW2 + 4, 2);
   add(block, SEC_M10, 1, CLS_MW2 + 3);
   add(block, SEC_M8, 1, CLS_MW2 + 2);
   add(block, SEC_M6, 1, CLS_MW2 + 1);
-  for (const Launch* l : {&wave, &pair, &wide, &block}) SKY_TRY(enqueue<true>(p, *l, longer, g->stream));
-  return SKY_OK;
+  if (!apart) {
+    for (const Launch* l : {&wave, &pair, &wide, &block}) SKY_TRY(enqueue<true>(p, *l, longer, g->stream));
+    return SKY_OK;
+  }
+  Beside side;
+  SKY_TRY(beside_begin(g, &side, &sum.a.fork));
+  SKY_TRY(enqueue<true>(p, sum, longer, g->stream));
+  auto others = [&]() -> int {
+    if (side.stream[0]) SKY_TRY(beside_fork(&side, 0));
+    for (const Launch* l : {&wide, &block, &pair, &wave}) SKY_TRY(enqueue<true>(p, *l, longer, side.stream[0] ? side.stream[0] : g->stream));
+    for (const Launch* l : {&totals, &scan, &emit}) SKY_TRY(enqueue<true>(p, *l, false, g->stream));
+    return beside_join(&side);
+  };
+  const int rc = others();
+  if (rc != SKY_OK) beside_drop(&side);
+  return rc;
 }
 
 }  // namespace sky
