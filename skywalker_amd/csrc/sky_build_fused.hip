@@ -817,11 +817,13 @@ bool streams_by_queue(const sky_graph* g, int tiled_from, bool longer) {
 }
 
 // One launch, if it has anything to do.  Device-sized ones know a bound of their units only: as many workgroups as the GPU holds at a time
-// stride over what there is.
+// stride over what there is; of the pairs and of 256 threads, whose units differ most, three and two times as many, of which the last go where
+// there is room first.  (Once / so many times, us: 40,000 seeds 25 x 10 on the scale-22 graph with 32 edges a vertex 671 / 666, 5,000 x 15 x 10 x 5
+// 537 / 530, 300 x 25 x 10 236 / 223, 40,000 x 25 x 10, scale 20, 298 / 293.  Twice as many of 64 or 512 threads: 2 to 7 us more.)
 template <bool DEV>
 int enqueue(const BuildPlan& p, const Launch& l, bool longer, hipStream_t st) {
   if (!l.units) return SKY_OK;
-  const uint32_t resident = l.threads == 64 ? 5120 : l.threads == 128 ? 2560 : l.threads == 256 ? 1024 : 512;
+  const uint32_t resident = l.threads == 64 ? 5120 : l.threads == 128 ? 3 * 2560 : l.threads == 256 ? 2 * 1024 : 512;
   const dim3 grid((uint32_t)(DEV ? std::min<uint64_t>(l.units, resident) : l.units));
   if (l.threads == 64) hipLaunchKernelGGL((fused_wave_kernel<DEV>), grid, dim3(64), 0, st, l.a);
   else if (l.threads == 128) hipLaunchKernelGGL((fused_pair_kernel<DEV>), grid, dim3(128), 0, st, l.a);
