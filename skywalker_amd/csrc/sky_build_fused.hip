@@ -179,6 +179,9 @@ __device__ __forceinline__ void each_wanted(uint32_t n, uint32_t first, uint32_t
     for (unsigned long long m = __ballot(u < n && wanted(u)); m; m &= m - 1ull) work(u0 + ((uint32_t)__ffsll((long long)m) - 1u) * stride);
   }
 }
+// The first unit from n on for the workgroup that also has units blockIdx.x, blockIdx.x + gridDim.x, ... of the n in front: what follows
+// few tiles goes to workgroups without (476 seeds 5 x 3 on the scale-22 graph with 5 edges a vertex 88 us where the first ones have both).
+__device__ __forceinline__ uint32_t unit_behind(uint32_t n) { return n + (blockIdx.x + gridDim.x - n % gridDim.x) % gridDim.x; }
 // Whether the tile belongs to a row that the frontier asks for; its first tile says so to the passes behind.
 __device__ __forceinline__ bool tile_asked(const FusedArgs& a, uint32_t tile) {
   const TileGeom tg = a.geom[tile];
@@ -336,7 +339,7 @@ __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
     each_wanted(tiles, blockIdx.x, gridDim.x, [&](uint32_t t) { return tile_asked(a, a.tile0 + t); },
                 [&](uint32_t t) { tile_sum_wave(a, a.tile0 + t); });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = tiles + blockIdx.x;; u += gridDim.x) {
+  for (uint32_t u = unit_behind(tiles);; u += gridDim.x) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -383,7 +386,7 @@ __global__ __launch_bounds__(128, 5) void fused_pair_kernel(FusedArgs a) {
                 [&](uint32_t t) { return t < a.sec[0].stride && tile_active(a, a.tile0 + t); },
                 [&](uint32_t t) { tile_totals_wave(a, a.tile0 + t); });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = pairs + blockIdx.x;; u += gridDim.x) {
+  for (uint32_t u = unit_behind(pairs);; u += gridDim.x) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -427,7 +430,7 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
                   __syncthreads();
                 });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = scans + blockIdx.x;;) {
+  for (uint32_t u = a.next ? scans + blockIdx.x : unit_behind(scans);;) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -499,7 +502,7 @@ __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
                   __syncthreads();
                 });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = tiles + blockIdx.x;; u += gridDim.x) {
+  for (uint32_t u = unit_behind(tiles);; u += gridDim.x) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -659,6 +662,13 @@ constexpr uint32_t MID_ALONE = 1u << 24;
 // Rows of 5118..8189 entries from which they are a launch of their own (10,000 rows of 6,500 streamed 478 us, held 402; 20,000
 // 885 and 745): fewer save less than a launch costs.
 constexpr uint32_t HOLD_ALONE = 2048;
+
+// Entries of a graph from which a build of its longer rows alone, which has no sweep, is worth a fork (in order / beside, us: walks without tables of
+// 10,000 x 8 on the scale-22 graph 195 / 188, of 836 x 10 on the scale-16 graph with 47 edges a vertex 74 / 79).
+constexpr uint32_t PART_BESIDE = 1u << 24;
+
+// Tiles of a graph's plan from which a frontier of few rows has launches of their own for them (build_frontier).
+constexpr uint32_t TILES_APART = 8192;
 
 // Frontiers of at most this many rows make the rows of 8190..65533 entries tile by tile.
 constexpr uint32_t SMALL_FRONTIER = 65536;
@@ -845,20 +855,21 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   FusedArgs base = common_args(g, p, p.t_all);
   const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
   base.list = p.rows;
-  // Vertices of a wavefront: enough wavefronts for every SIMD, but 128 to 256 rather than fewer where four wavefronts a SIMD remain: the
-  // rows of a few vertices fill no batch of their class.  The last wavefronts of a sweep are what is left of it behind the launches beside
-  // it, so no more than that either where it makes 12,288 wavefronts.  (64 where there were fewer than 4,096 wavefronts of 128, 256 up to
-  // 2 M vertices, an 8,192th above / now, us: 3 M entries in 478,000 rows 44 / 36, scale 20 with 6 edges a vertex 83 / 78, scale 22 with 3
-  // 115 / 110, scale 23 with 4 232 / 219, 19 M entries in 4.8 M rows of up to 107, one launch, 133 / 130; scale 22 with 4 127 / 129, with 10
-  // 242 / 245; most others within 1 %.)
-  base.split = g->V <= SPLIT_SWEEP;
-  const uint32_t least = g->V > 1u << 20 ? 256u : std::min(192u, std::max(g->V / 4096u, std::min(128u, g->V / 2048u)));
-  base.per_wave = base.split ? 64u : std::max(64u, std::min(SMALL_RANGE, std::max(g->V / 12288u, least) / 64u * 64u));
-  const uint32_t ranges = (g->V + base.per_wave - 1) / base.per_wave, sweeps = base.split ? 4 * ranges : ranges;
   auto rows = [&](int c) { return class_min_degree(c) >= min_degree ? g->bin_counts[c] : 0u; };
   uint32_t past_wave = 0;  // rows of more than 509 entries: what a second launch would be for
   for (int c = CLS_COUNT - 1; c > CLS_LDS_W2; --c)
     if (class_min_degree(c) >= 510) past_wave += rows(c);
+  // Vertices of a wavefront: enough wavefronts for every SIMD, but 128 to 256 rather than fewer where four wavefronts a SIMD remain: the
+  // rows of a few vertices fill no batch of their class.  The last wavefronts of a sweep beside other launches are what is left of it behind
+  // them: there a 12,288th of the vertices is the limit instead of an 8,192th.  (64 where there were fewer than 4,096 wavefronts of 128, 256 up
+  // to 2 M vertices, an 8,192th above / now, us: 3 M entries in 478,000 rows 44 / 36, scale 20 with 6 edges a vertex 83 / 78, scale 22 with 3
+  // 115 / 110, scale 23 with 4 232 / 219; scale 22 with 4 127 / 129, with 10 242 / 245; most others within 1 %.  29 M entries in rows of up to
+  // 339, one launch, an 8,192th / a 12,288th 176 / 181.)
+  base.split = g->V <= SPLIT_SWEEP;
+  const uint32_t least = g->V > 1u << 20 ? 256u : std::min(192u, std::max(g->V / 4096u, std::min(128u, g->V / 2048u)));
+  const uint32_t range = std::max(g->V / (past_wave ? 12288u : 8192u), least) / 64u * 64u;
+  base.per_wave = base.split ? 64u : std::max(64u, std::min(SMALL_RANGE, range));
+  const uint32_t ranges = (g->V + base.per_wave - 1) / base.per_wave, sweeps = base.split ? 4 * ranges : ranges;
   if (past_wave && g->max_degree <= ALL_LONGEST) {
     Launch all(base, 512);
     auto waves = [&](Section k, int c, uint32_t per) { all.add(k, rows(c), per * ALL_WAVES, p.start[c]); };
@@ -939,7 +950,8 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   Beside side;
   if (first) {
     first->a.call = call;
-    if (rest.units + wide.units + alone.units && first != &rest && first != &wide) SKY_TRY(beside_begin(g, &side, &first->a.fork));
+    const bool worth = min_degree == 0 || g->E >= PART_BESIDE;
+    if (worth && rest.units + wide.units + alone.units && first != &rest && first != &wide) SKY_TRY(beside_begin(g, &side, &first->a.fork));
     SKY_TRY(enqueue<false>(p, *first, longer, g->stream));
   }
   auto others = [&]() -> int {
@@ -998,10 +1010,12 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
   base.built = built;
   Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
   Launch sum(base, 64), totals(base, 128), scan(base, 512), emit(base, 256);
-  // The passes over tiles wait for one another, and of a frontier of few rows they are a good part: the rows go out beside them, the longest
-  // first.  (In the same four launches / beside, us: 40,000 seeds x 20 on the scale-22 graph with 30 edges a vertex 125 / 115, 300 x 25 x 10 with
-  // 32 231 / 225, 2,000 x 10 x 10, scale 21 with 40, 338 / 329, 40,000 x 25 x 10, scale 22 with 32, 676 / 669; the rest within 1 %.)
-  const bool apart = f.few && n_tiles;
+  // The passes over tiles wait for one another, and where they look at many tiles for a frontier of few rows they are a good part: the rows then
+  // go out beside them, the longest first.  (In the same four launches / beside, us: 40,000 seeds x 20 on the scale-22 graph with 30 edges a
+  // vertex, 26,000 tiles, 125 / 115, 300 x 25 x 10 with 32 231 / 225, 40,000 x 25 x 10 676 / 669, 2,000 x 10 x 10 on the scale-21 graph with 40, 13,000
+  // tiles, 338 / 329; with few tiles it costs more launches: 28,208 x 10 x 10 on the scale-19 graph with 5 140 / 149, 1,165 x 25 x 10, scale 16,
+  // 125 / 139, 476 x 5 x 3 on the scale-22 graph with 5 75 / 79.)
+  const bool apart = f.few && n_tiles >= TILES_APART;
   auto add = [&](Launch& l, Section k, uint32_t per, int cls, int ncls = 1) {
     uint32_t upper = 0;
     for (int c = 0; c < ncls; ++c) upper += f.cap[cls + c];

@@ -21,7 +21,8 @@ constexpr uint32_t CALL_PARTS = 64, CALL_PART_WORDS = 16, CALL_MANY = 512;
 struct CallDevice {
   unsigned long long start;  // wall clock of the first kernel
   unsigned long long entries, arrived, refused;  // sample_check_kernel; the last is left as it is
-  unsigned long long pad[12];
+  uint32_t joined, pad0;     // side streams of a fork that have nothing left (Beside)
+  unsigned long long pad[11];
   unsigned long long part[CALL_PARTS * CALL_PART_WORDS];
 };
 constexpr int CALL_ANSWERS = 10;
@@ -31,8 +32,8 @@ constexpr int CALL_ANSWERS = 10;
 struct CallHost {
   unsigned long long sampled, ticks;
   unsigned long long answer[CALL_ANSWERS];  // in the course of a call, with a number of their own (call_ask)
-  uint32_t begun, done[3];                  // what streams wait for (Beside)
-  unsigned long long pad[2];
+  uint32_t begun, done;                     // what streams wait for (Beside)
+  unsigned long long pad[3];
 };
 constexpr int CALL_VALUE_BITS = 48;  // 2^48 edges fill the GPU's memory a thousand times over; 2^48 ticks of 10 ns are a month
 static_assert(sizeof(CallDevice) % 128 == 0 && offsetof(CallDevice, part) == 128 && sizeof(CallHost) == 128, "cache lines of their own");
@@ -83,16 +84,18 @@ __device__ __forceinline__ void call_answer(CallHost* host, unsigned long long n
 }
 int call_answered(sky_graph* g, CallWords* w, unsigned long long* values, int n);
 // Kernels beside those of the graph's stream, on streams that all graphs of a device share.  These and the graph's stream wait for one
-// another by words in pinned memory that a kernel writes and the waiting queue's command processor reads: a kernel on the graph's stream
-// notes that it runs (fork_mark), so that everything in front of it has ended, and a small last one on each of the others that everything
-// in front of it has.  2 us each way, where events and stream waits take 9 (two kernels of 40 us side by side 55 us in all, with
-// events 68, one after the other 89).  Who waits is enqueued behind the kernel that writes, so that every wait ends also where other
-// threads' calls lie between, and where streams share a hardware queue.
+// another by words in pinned memory: a kernel on the graph's stream notes that it runs (fork_mark), so that everything in front of it has
+// ended, and of small last ones on the others the one that finds all of them there that everything in front of these has.  Who waits, by a stream operation (one
+// thread of the runtime's that reads the word until the number is there), is always enqueued behind the kernel that writes, so that
+// every wait ends: also where other threads' calls lie between, where streams share a hardware queue, and where there is only one.  2 us
+// each way, where events and stream waits take 9 (two kernels of 40 us side by side 55 us in all, with events 68, one after
+// the other 89).
 constexpr int SIDE_STREAMS = 3;
 struct Beside {
   hipStream_t main = nullptr;
   hipStream_t stream[SIDE_STREAMS] = {nullptr, nullptr, nullptr};  // null: no fork
   bool used[SIDE_STREAMS] = {false, false, false};
+  CallDevice* dev = nullptr;
   CallHost* host = nullptr;
   uint32_t number = 0;
 };
@@ -103,7 +106,7 @@ struct ForkMark {
 __device__ __forceinline__ void fork_mark(const ForkMark& f) {
   if (f.word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(f.word, f.number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-// A fork, and the mark for the next kernel on the graph's stream.  b->stream stays null on a device whose queues know no such wait, and where
+// A fork, and the mark for the next kernel on the graph's stream.  b->stream stays null on a device without such waits, and where
 // another device than the graph's is current.
 int beside_begin(sky_graph* g, Beside* b, ForkMark* mark);
 // With that kernel on its way: side stream k waits for its mark, if it does not already.

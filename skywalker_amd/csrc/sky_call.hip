@@ -147,11 +147,13 @@ struct SideStreams {
   hipStream_t stream[SIDE_STREAMS] = {nullptr, nullptr, nullptr};
   bool tried = false;
 } g_side[MAX_DEVICES];  // of every device, which keeps them until the process ends
-static_assert(sizeof(CallHost::done) / sizeof(CallHost::done[0]) == SIDE_STREAMS, "a word for each");
 }  // namespace
 
-__global__ void beside_done_kernel(uint32_t* word, uint32_t number) {
-  __hip_atomic_store(word, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+// The last kernel of each of the n side streams of a fork.  (A word for each, and a wait for each on the graph's stream: 4.5 us apiece.)
+__global__ void beside_done_kernel(CallDevice* dev, CallHost* host, uint32_t n, uint32_t number) {
+  if (__hip_atomic_fetch_add(&dev->joined, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u != n) return;
+  __hip_atomic_store(&dev->joined, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(&host->done, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
@@ -174,6 +176,7 @@ int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
   if (!side.stream[0]) return SKY_OK;
   for (int k = 0; k < SIDE_STREAMS; ++k) b->stream[k] = side.stream[k];
   b->main = g->stream;
+  b->dev = g->call.dev;
   b->host = g->call.host;
   b->number = ++g->call.forks;
   *mark = ForkMark{&b->host->begun, b->number};
@@ -186,18 +189,24 @@ int beside_fork(Beside* b, int k) {
   return SKY_OK;
 }
 int beside_join(Beside* b) {
-  for (int k = 0; k < SIDE_STREAMS; ++k) {
-    if (!b->used[k]) continue;
-    hipLaunchKernelGGL(beside_done_kernel, dim3(1), dim3(1), 0, b->stream[k], &b->host->done[k], b->number);
-    SKY_HIP(hipGetLastError());
-    SKY_HIP(hipStreamWaitValue32(b->main, &b->host->done[k], b->number, hipStreamWaitValueEq, 0xFFFFFFFFu));
-    b->used[k] = false;
-  }
+  uint32_t n = 0;
+  for (bool u : b->used) n += u;
+  if (!n) return SKY_OK;
+  for (int k = 0; k < SIDE_STREAMS; ++k)
+    if (b->used[k]) hipLaunchKernelGGL(beside_done_kernel, dim3(1), dim3(1), 0, b->stream[k], b->dev, b->host, n, b->number);
+  SKY_HIP(hipGetLastError());
+  SKY_HIP(hipStreamWaitValue32(b->main, &b->host->done, b->number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+  for (bool& u : b->used) u = false;
   return SKY_OK;
 }
 void beside_drop(Beside* b) {
+  bool any = false;
   for (int k = 0; k < SIDE_STREAMS; ++k)
-    if (b->used[k]) (void)hipStreamSynchronize(b->stream[k]);
+    if (b->used[k]) {
+      any = true;
+      (void)hipStreamSynchronize(b->stream[k]);
+    }
+  if (any) (void)hipMemset(&b->dev->joined, 0, sizeof(b->dev->joined));
   for (bool& u : b->used) u = false;
 }
 
