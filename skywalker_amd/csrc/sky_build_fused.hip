@@ -664,7 +664,7 @@ constexpr uint32_t MID_ALONE = 1u << 24;
 constexpr uint32_t HOLD_ALONE = 2048;
 
 // Entries of a graph from which a build of its longer rows alone, which has no sweep, is worth a fork (in order / beside, us: walks without tables of
-// 10,000 x 8 on the scale-22 graph 195 / 188, of 836 x 10 on the scale-16 graph with 47 edges a vertex 74 / 79).
+// 10,000 x 8 on the scale-22 graph 195 / 188, of 836 x 10 on the scale-16 graph with 47 edges a vertex 75 / 79).
 constexpr uint32_t PART_BESIDE = 1u << 24;
 
 // Tiles of a graph's plan from which a frontier of few rows has launches of their own for them (build_frontier).
@@ -904,17 +904,18 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
     }
   }
   Launch pair(base, 128), scan(base, 512), block(base, 256), rest(base, 64), wide(base, 512), alone(base, 512);
-  Launch& mid = min_degree == 0 && g->E >= MID_ALONE ? alone : wide;
+  const bool worth = min_degree == 0 || g->E >= PART_BESIDE;  // a fork; without, the long rows follow the scans in their launch
+  Launch &longs = worth ? wide : scan, &mid = min_degree == 0 && g->E >= MID_ALONE ? alone : longs;
   pair.add(SEC_TOTALS, n_tiles, 2, 0);
   pair.add(SEC_P8, rows(CLS_MW2), 1, p.start[CLS_MW2]);
   pair.add(SEC_P6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
   scan.add(SEC_SCAN, n_trows, 1, 0);
-  if (p.t_all > CLS_STREAM) wide.add(SEC_STREAM, rows(CLS_STREAM), 1, p.start[CLS_STREAM]);
-  if (p.t_all > CLS_STREAM_LAST) wide.add(SEC_STREAM, rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM_LAST]);
+  if (p.t_all > CLS_STREAM) longs.add(SEC_STREAM, rows(CLS_STREAM), 1, p.start[CLS_STREAM]);
+  if (p.t_all > CLS_STREAM_LAST) longs.add(SEC_STREAM, rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM_LAST]);
   // Rows of 5118..8189 entries: streamed beside the others, where hold_row would spill, or, where they are enough for a launch,
   // HOLD_ALONE, by build_hold_kernel.
   const bool hold_alone = min_degree == 0 && rows(CLS_HOLD) >= HOLD_ALONE;  // behind the sweep, which notes when the call began
-  if (!hold_alone) wide.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);
+  if (!hold_alone) longs.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);
   // two classes whose lists lie back to back; min_degree may leave out the first
   auto add_two = [&](Launch& l, Section k, int c) { l.add(k, rows(c) + rows(c + 1), 1, p.start[rows(c) ? c : c + 1]); };
   add_two(mid, SEC_B10, CLS_MW2 + 7);
@@ -950,7 +951,6 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   Beside side;
   if (first) {
     first->a.call = call;
-    const bool worth = min_degree == 0 || g->E >= PART_BESIDE;
     if (worth && rest.units + wide.units + alone.units && first != &rest && first != &wide) SKY_TRY(beside_begin(g, &side, &first->a.fork));
     SKY_TRY(enqueue<false>(p, *first, longer, g->stream));
   }
