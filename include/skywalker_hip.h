@@ -257,10 +257,10 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      them by degree class like all other rows; -1 takes the former for builds of at least 2^25 rows or of all rows of a
  *      graph of more than 2^27 entries, and in the four launches that make all of a build of up to 2^27 entries.  0 or 1
  *      gives such a build its class kernels back.  Same tables.
- *      "build_streams" (default 1): builds of up to 2^27 entries without per-kernel timing go out in four launches;
- *      larger ones of up to 1 G entries (and smaller ones whose other knobs ask for class kernels) send the kernels of
- *      their degree classes out over the graph's stream and three side streams (small builds are bound by one
- *      kernel waiting for the one before); 0 keeps every class kernel on the graph's stream.  Same tables.
+ *      "build_streams" (default 1): builds of up to 2^27 entries without per-kernel timing go out in a few launches
+ *      beside one another; larger ones (and smaller ones of 2 M entries and more whose other knobs ask for class kernels)
+ *      send the kernels of their degree classes out over the graph's stream and three side streams, which the graphs of a
+ *      device share; 0 keeps every class kernel on the graph's stream.  Same tables.
  *      "build_profile" (default 0): 1 records a HIP event after every kernel of sky_alias_build_all for
  *      sky_last_build_profile (about 3 microseconds each; a small graph pays 20 % of its build for them).
  *      "online_full_build" (default -1): how sky_walk_online serves a static bias on a graph without tables:
