@@ -179,9 +179,11 @@ __device__ __forceinline__ void each_wanted(uint32_t n, uint32_t first, uint32_t
     for (unsigned long long m = __ballot(u < n && wanted(u)); m; m &= m - 1ull) work(u0 + ((uint32_t)__ffsll((long long)m) - 1u) * stride);
   }
 }
-// The first unit from n on for the workgroup that also has units blockIdx.x, blockIdx.x + gridDim.x, ... of the n in front: what follows
-// few tiles goes to workgroups without (476 seeds 5 x 3 on the scale-22 graph with 5 edges a vertex 88 us where the first ones have both).
-__device__ __forceinline__ uint32_t unit_behind(uint32_t n) { return n + (blockIdx.x + gridDim.x - n % gridDim.x) % gridDim.x; }
+// The first unit from n on for a workgroup of a device-sized launch, which has units of the n in front too; one of the others has one unit.
+template <bool DEV>
+__device__ __forceinline__ uint32_t unit_behind(uint32_t n) {
+  return DEV ? first_behind(n, blockIdx.x, gridDim.x) : blockIdx.x;
+}
 // Whether the tile belongs to a row that the frontier asks for; its first tile says so to the passes behind.
 __device__ __forceinline__ bool tile_asked(const FusedArgs& a, uint32_t tile) {
   const TileGeom tg = a.geom[tile];
@@ -339,7 +341,7 @@ __global__ __launch_bounds__(64, 5) void fused_wave_kernel(FusedArgs a) {
     each_wanted(tiles, blockIdx.x, gridDim.x, [&](uint32_t t) { return tile_asked(a, a.tile0 + t); },
                 [&](uint32_t t) { tile_sum_wave(a, a.tile0 + t); });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = unit_behind(tiles);; u += gridDim.x) {
+  for (uint32_t u = unit_behind<DEV>(tiles);; u += gridDim.x) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -386,7 +388,7 @@ __global__ __launch_bounds__(128, 5) void fused_pair_kernel(FusedArgs a) {
                 [&](uint32_t t) { return t < a.sec[0].stride && tile_active(a, a.tile0 + t); },
                 [&](uint32_t t) { tile_totals_wave(a, a.tile0 + t); });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = unit_behind(pairs);; u += gridDim.x) {
+  for (uint32_t u = unit_behind<DEV>(pairs);; u += gridDim.x) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -430,7 +432,7 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
                   __syncthreads();
                 });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = a.next ? scans + blockIdx.x : unit_behind(scans);;) {
+  for (uint32_t u = a.next ? scans + blockIdx.x : unit_behind<DEV>(scans);;) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;
@@ -502,7 +504,7 @@ __global__ __launch_bounds__(256, 4) void fused_block_kernel(FusedArgs a) {
                   __syncthreads();
                 });
   const UnitFinder<DEV> units(a);
-  for (uint32_t u = unit_behind(tiles);; u += gridDim.x) {
+  for (uint32_t u = unit_behind<DEV>(tiles);; u += gridDim.x) {
     SectionRef s;
     uint32_t unit = 0, rows = 0;
     if (!units.find(a, u, s, unit, rows)) return;

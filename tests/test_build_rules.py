@@ -64,3 +64,22 @@ def test_limit_of_the_streamed_rows(narrow_rows):
 ])
 def test_narrow_rows_of_some_builds(narrow_rows, limit, last, stream, wide, longest, want):
     assert narrow_rows([(limit, last, stream, wide, longest)])[0] == want
+
+
+def test_units_behind_others_go_once_to_a_workgroup_each(tmp_path):
+    # every unit from n on to exactly one workgroup, which has it after its own of the n in front and strides on by the grid; the first of
+    # them to the workgroup whose turn it is
+    (tmp_path / "behind.cpp").write_text("""
+#include <cstdio>
+#include "sky_build_rules.h"
+int main() {
+  for (unsigned grid : {1u, 2u, 3u, 7u, 64u, 512u, 2048u, 5120u})
+    for (unsigned n : {0u, 1u, 2u, grid - 1u, grid, grid + 1, 3 * grid - 1, 3 * grid, 3 * grid + 5, 4194304u})
+      for (unsigned block = 0; block < grid; ++block) {
+        const unsigned u = sky::first_behind(n, block, grid);
+        if (u < n || u >= n + grid || u % grid != block) return std::printf("%u %u %u: %u\\n", n, block, grid, u), 1;
+      }
+}
+""")
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", CSRC, str(tmp_path / "behind.cpp"), "-o", str(tmp_path / "behind")], check=True)
+    subprocess.run([str(tmp_path / "behind")], check=True)
