@@ -7,6 +7,7 @@
 #include <cstddef>
 
 #include "sky_common.h"
+#include "sky_sides.h"
 
 struct sky_graph;
 
@@ -83,14 +84,13 @@ __device__ __forceinline__ void call_answer(CallHost* host, unsigned long long n
   __hip_atomic_store(&host->answer[word], value | number << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 int call_answered(sky_graph* g, CallWords* w, unsigned long long* values, int n);
-// Kernels beside those of the graph's stream, on streams that all graphs of a device share.  These and the graph's stream wait for one
+// Kernels beside those of the graph's stream, on streams that all graphs of a device share and the last of them takes with it (sky_sides.h).  These and the graph's stream wait for one
 // another by words in pinned memory: a kernel on the graph's stream notes that it runs (fork_mark), so that everything in front of it has
 // ended, and of small last ones on the others the one that finds all of them there that everything in front of these has.  Who waits, by a stream operation (one
 // thread of the runtime's that reads the word until the number is there), is always enqueued behind the kernel that writes, so that
 // every wait ends: also where other threads' calls lie between, where streams share a hardware queue, and where there is only one.  2 us
 // each way, where events and stream waits take 9 (two kernels of 40 us side by side 55 us in all, with events 68, one after
 // the other 89).
-constexpr int SIDE_STREAMS = 3;
 struct Beside {
   hipStream_t main = nullptr;
   hipStream_t stream[SIDE_STREAMS] = {nullptr, nullptr, nullptr};  // null: no fork
@@ -115,6 +115,8 @@ int beside_fork(Beside* b, int k);
 int beside_join(Beside* b);
 // Instead of a join, after an error: the host waits for them.
 void beside_drop(Beside* b);
+// A graph that is about to be freed, with nothing of it on the way, gives back its share of the streams.
+void beside_release(sky_graph* g);
 // With the graph's own words.
 int call_begin(sky_graph* g, CallDevice** call);
 int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);

@@ -143,10 +143,15 @@ void call_cancel(sky_graph* g) { g->call.dirty = false; }
 // ---------------------------------------------------------------- beside the graph's stream
 namespace {
 constexpr int MAX_DEVICES = 64;
-struct SideStreams {
-  hipStream_t stream[SIDE_STREAMS] = {nullptr, nullptr, nullptr};
-  bool tried = false;
-} g_side[MAX_DEVICES];  // of every device, which keeps them until the process ends
+struct SideRuntime {
+  using Stream = hipStream_t;
+  int create(Stream* s) {
+    SKY_HIP(hipStreamCreateWithFlags(s, hipStreamNonBlocking));
+    return SKY_OK;
+  }
+  void destroy(Stream s) { (void)hipStreamDestroy(s); }
+};
+SidePool<SideRuntime> g_side[MAX_DEVICES];
 }  // namespace
 
 // The last kernel of each of the n side streams of a fork.  (A word for each, and a wait for each on the graph's stream: 4.5 us apiece.)
@@ -163,18 +168,13 @@ int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
   SKY_HIP(hipGetDevice(&current));
   if (g->device != current || current < 0 || current >= MAX_DEVICES) return SKY_OK;  // the graph's stream is the current device's
   if (!g->call.host) SKY_TRY(take_words(g->device, &g->call));
+  int can = 0;
+  SKY_HIP(hipDeviceGetAttribute(&can, hipDeviceAttributeCanUseStreamWaitValue, g->device));
+  if (!can) return SKY_OK;
   std::lock_guard<std::mutex> lock(g_mutex);
-  SideStreams& side = g_side[g->device];
-  if (!side.tried) {
-    int can = 0;
-    SKY_HIP(hipDeviceGetAttribute(&can, hipDeviceAttributeCanUseStreamWaitValue, g->device));
-    if (can)
-      for (hipStream_t& s : side.stream)
-        if (!s) SKY_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-    side.tried = true;
-  }
-  if (!side.stream[0]) return SKY_OK;
-  for (int k = 0; k < SIDE_STREAMS; ++k) b->stream[k] = side.stream[k];
+  SideRuntime runtime;
+  SKY_TRY(g_side[g->device].take(runtime, &g->sides));
+  for (int k = 0; k < SIDE_STREAMS; ++k) b->stream[k] = g_side[g->device].stream[k];
   b->main = g->stream;
   b->dev = g->call.dev;
   b->host = g->call.host;
@@ -208,6 +208,13 @@ void beside_drop(Beside* b) {
     }
   if (any) (void)hipMemset(&b->dev->joined, 0, sizeof(b->dev->joined));
   for (bool& u : b->used) u = false;
+}
+
+void beside_release(sky_graph* g) {
+  if (!g->sides.held) return;
+  std::lock_guard<std::mutex> lock(g_mutex);
+  SideRuntime runtime;
+  g_side[g->device].give(runtime, &g->sides);
 }
 
 // ---------------------------------------------------------------- the end

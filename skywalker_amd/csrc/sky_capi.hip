@@ -241,6 +241,7 @@ int sky_graph_free(sky_graph* g) {
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   pool_release(g);
+  beside_release(g);  // the frees have waited for whatever the graph had on its way
   call_release(&g->call);
   g->plan.reset();
   free_build_scratch(g);

@@ -64,6 +64,7 @@ struct sky_graph {
   std::vector<ProfileEntry> build_profile;
 
   sky::CallWords call;  // how a call on this graph reports its end (sky_call.h)
+  sky::SideHold sides;  // its share of the device's side streams
 
   // Device buffers that calls on this graph reuse instead of allocating each time (they only grow).
   enum PoolSlot { POOL_WALK_LIST = 0, POOL_WALK_COUNTS, POOL_BITMAP, POOL_LIST, POOL_TOTALS, POOL_FRONT, POOL_SEGMENTS, POOL_SLOTS };
