@@ -145,11 +145,19 @@ namespace {
 constexpr int MAX_DEVICES = 64;
 struct SideRuntime {
   using Stream = hipStream_t;
-  int create(Stream* s) {
-    SKY_HIP(hipStreamCreateWithFlags(s, hipStreamNonBlocking));
-    return SKY_OK;
+  int device;
+  bool can() const {
+    int yes = 0;
+    return worked(hipDeviceGetAttribute(&yes, hipDeviceAttributeCanUseStreamWaitValue, device)) && yes;
   }
-  void destroy(Stream s) { (void)hipStreamDestroy(s); }
+  bool create(Stream* s) const { return worked(hipStreamCreateWithFlags(s, hipStreamNonBlocking)); }
+  void destroy(Stream s) const { (void)hipStreamDestroy(s); }
+
+ private:
+  static bool worked(hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();  // not an error of the call, which does without
+    return e == hipSuccess;
+  }
 };
 SidePool<SideRuntime> g_side[MAX_DEVICES];
 }  // namespace
@@ -168,12 +176,9 @@ int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
   SKY_HIP(hipGetDevice(&current));
   if (g->device != current || current < 0 || current >= MAX_DEVICES) return SKY_OK;  // the graph's stream is the current device's
   if (!g->call.host) SKY_TRY(take_words(g->device, &g->call));
-  int can = 0;
-  SKY_HIP(hipDeviceGetAttribute(&can, hipDeviceAttributeCanUseStreamWaitValue, g->device));
-  if (!can) return SKY_OK;
   std::lock_guard<std::mutex> lock(g_mutex);
-  SideRuntime runtime;
-  SKY_TRY(g_side[g->device].take(runtime, &g->sides));
+  SideRuntime runtime{g->device};
+  if (!g_side[g->device].take(runtime, &g->sides)) return SKY_OK;
   for (int k = 0; k < SIDE_STREAMS; ++k) b->stream[k] = g_side[g->device].stream[k];
   b->main = g->stream;
   b->dev = g->call.dev;
@@ -213,7 +218,7 @@ void beside_drop(Beside* b) {
 void beside_release(sky_graph* g) {
   if (!g->sides.held) return;
   std::lock_guard<std::mutex> lock(g_mutex);
-  SideRuntime runtime;
+  SideRuntime runtime{g->device};
   g_side[g->device].give(runtime, &g->sides);
 }
 

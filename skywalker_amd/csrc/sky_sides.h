@@ -9,28 +9,31 @@ constexpr int SIDE_STREAMS = 3;
 
 // What a graph has of them.
 struct SideHold {
-  bool held = false;  // they stay as long as it does
+  bool held = false;     // they stay as long as it does
+  bool refused = false;  // it asked for some that could not be made
 };
 
 // The side streams of one device: shared by the graphs that have asked for them, and destroyed when the last of these is freed.  Calls
-// are the caller's to serialise.  Runtime: int create(Stream*), 0 or an error, and destroy(Stream).
+// are the caller's to serialise.  Runtime: can(), whether the device has what they wait with; create(Stream*); destroy(Stream).
 template <class Runtime>
 struct SidePool {
   using Stream = typename Runtime::Stream;
   Stream stream[SIDE_STREAMS] = {};
   int holders = 0;
 
-  int take(Runtime& rt, SideHold* h) {
+  // Whether the graph has them.  Where they cannot be made its kernels go out in order, then and later.
+  bool take(Runtime& rt, SideHold* h) {
+    if (h->refused) return false;
     for (Stream& s : stream) {
-      const int rc = s ? 0 : rt.create(&s);
-      if (rc == 0) continue;
+      if (s || (rt.can() && rt.create(&s))) continue;
       s = Stream{};
+      h->refused = true;
       if (!holders) clear(rt);
-      return rc;
+      return false;
     }
     if (!h->held) ++holders;
     h->held = true;
-    return 0;
+    return true;
   }
   // The graph is about to be freed.
   void give(Runtime& rt, SideHold* h) {

@@ -15,11 +15,16 @@ struct Runtime {
   using Stream = int*;
   std::set<int*> live;
   int made = 0, fail_from = 1000;  // streams made so far; number of the first that cannot be made
-  int create(Stream* s) {
-    if (made >= fail_from) return 7;
+  bool able = true;
+  bool can() const { return able; }
+  bool create(Stream* s) {
+    if (made >= fail_from) {
+      *s = (int*)8;  // whatever a failing call leaves behind
+      return false;
+    }
     ++made;
     live.insert(*s = new int);
-    return 0;
+    return true;
   }
   void destroy(Stream s) {
     assert(live.erase(s) == 1);
@@ -47,7 +52,7 @@ def test_streams_are_shared_and_go_with_the_last_graph_that_has_them(run):
     run("""
   for (int round = 0; round < 3; ++round) {
     SideHold a, b, never;
-    assert(pool.take(rt, &a) == 0 && pool.take(rt, &a) == 0 && pool.take(rt, &b) == 0);
+    assert(pool.take(rt, &a) && pool.take(rt, &a) && pool.take(rt, &b));
     assert(rt.live.size() == SIDE_STREAMS && rt.made == SIDE_STREAMS * (round + 1));
     pool.give(rt, &never);
     pool.give(rt, &a);
@@ -59,14 +64,20 @@ def test_streams_are_shared_and_go_with_the_last_graph_that_has_them(run):
 """)
 
 
-def test_streams_made_before_one_that_fails_go_back_unless_another_graph_has_them(run):
+@pytest.mark.parametrize("able,fail_from", [(0, 1000), (1, 0), (1, 1), (1, 2)])
+def test_a_graph_does_without_streams_that_cannot_be_made(run, able, fail_from):
+    # those that were made before the one that failed go back; the graph does not ask again, others do
     run("""
   SideHold a, b;
-  rt.fail_from = 2;
-  assert(pool.take(rt, &a) == 7 && !a.held && rt.live.empty());
-  rt.fail_from = 1000;
-  assert(pool.take(rt, &a) == 0 && pool.take(rt, &b) == 0);
+  rt.able = %d, rt.fail_from = %d;
+  assert(!pool.take(rt, &a) && !a.held && rt.live.empty() && pool.holders == 0);
+  rt.able = true, rt.fail_from = 1000;
+  const int made = rt.made;
+  assert(!pool.take(rt, &a) && rt.made == made);
+  assert(pool.take(rt, &b) && rt.live.size() == SIDE_STREAMS);
+  pool.give(rt, &a);
+  assert(rt.live.size() == SIDE_STREAMS && pool.take(rt, &a));
   pool.give(rt, &b);
   pool.give(rt, &a);
   assert(rt.live.empty());
-""")
+""" % (able, fail_from))
