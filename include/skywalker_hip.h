@@ -257,10 +257,13 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      them by degree class like all other rows; -1 takes the former for builds of at least 2^25 rows or of all rows of a
  *      graph of more than 2^27 entries, and in the four launches that make all of a build of up to 2^27 entries.  0 or 1
  *      gives such a build its class kernels back.  Same tables.
- *      "build_streams" (default 1): builds of up to 2^27 entries without per-kernel timing go out in a few launches
- *      beside one another; larger ones (and smaller ones of 2 M entries and more whose other knobs ask for class kernels)
- *      send the kernels of their degree classes out over the graph's stream and three side streams, which the graphs of a
- *      device share; 0 keeps every class kernel on the graph's stream.  Same tables.
+ *      "build_streams" (default 1): kernels of a build that do not depend on one another go out beside one another, on the graph's
+ *      stream and up to three side streams, which the graphs of a device share and the last of them takes with it: the launches of a build of
+ *      up to 2^27 entries, the longer rows alone that an online walk makes on a graph of 2^24 entries and more, the rows of a frontier of up to
+ *      65,536 beside the passes over 8,192 tiles and more, and the kernels of the degree classes of larger builds (and of smaller ones of
+ *      2 M entries and more whose other knobs ask for class kernels).  What follows waits for a word in pinned memory, by a kernel of
+ *      the runtime's.  0 keeps every kernel of every build on the graph's stream, for tools that let one kernel run at a time, and makes all
+ *      rows of a graph by class kernels.  Same tables.
  *      "build_profile" (default 0): 1 records a HIP event after every kernel of sky_alias_build_all for
  *      sky_last_build_profile (about 3 microseconds each; a small graph pays 20 % of its build for them).
  *      "online_full_build" (default -1): how sky_walk_online serves a static bias on a graph without tables:

@@ -868,11 +868,15 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   // 115 / 110, scale 23 with 4 232 / 219; scale 22 with 4 127 / 129, with 10 242 / 245; most others within 1 %.  29 M entries in rows of up to
   // 339, one launch, an 8,192th / a 12,288th 176 / 181.)
   base.split = g->V <= SPLIT_SWEEP;
-  const uint32_t least = g->V > 1u << 20 ? 256u : std::min(192u, std::max(g->V / 4096u, std::min(128u, g->V / 2048u)));
-  const uint32_t range = std::max(g->V / (past_wave ? 12288u : 8192u), least) / 64u * 64u;
-  base.per_wave = base.split ? 64u : std::max(64u, std::min(SMALL_RANGE, range));
-  const uint32_t ranges = (g->V + base.per_wave - 1) / base.per_wave, sweeps = base.split ? 4 * ranges : ranges;
+  auto sweep = [&](bool beside) -> uint32_t {  // its wavefronts
+    const uint32_t least = g->V > 1u << 20 ? 256u : std::min(192u, std::max(g->V / 4096u, std::min(128u, g->V / 2048u)));
+    const uint32_t range = std::max(g->V / (beside ? 12288u : 8192u), least) / 64u * 64u;
+    base.per_wave = base.split ? 64u : std::max(64u, std::min(SMALL_RANGE, range));
+    const uint32_t ranges = (g->V + base.per_wave - 1) / base.per_wave;
+    return base.split ? 4 * ranges : ranges;
+  };
   if (past_wave && g->max_degree <= ALL_LONGEST) {
+    const uint32_t sweeps = sweep(true);
     Launch all(base, 512);
     auto waves = [&](Section k, int c, uint32_t per) { all.add(k, rows(c), per * ALL_WAVES, p.start[c]); };
     all.add(SEC_STREAM, rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM_LAST]);
@@ -905,9 +909,18 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
       return SKY_OK;
     }
   }
+  uint32_t past_block = p.t_all > CLS_STREAM ? rows(CLS_STREAM) : 0u;  // rows of 2558 entries and more that are not made tile by tile
+  if (p.t_all > CLS_STREAM_LAST) past_block += rows(CLS_STREAM_LAST);
+  past_block += rows(CLS_HOLD);
+  for (int c = CLS_MW2 + 4; c <= CLS_MW2 + MERGE_MAX_NW - 2; ++c) past_block += rows(c);
+  Beside side;
+  ForkMark mark{nullptr, 0};
+  if (min_degree == 0 ? past_wave : g->E >= PART_BESIDE && past_block) SKY_TRY(beside_begin(g, &side, &mark));
+  // Without a fork four launches follow one another: the sweep rides along in the first, the long rows behind the scans.
+  const bool fork = side.stream[0] != nullptr;
+  const uint32_t sweeps = sweep(fork);
   Launch pair(base, 128), scan(base, 512), block(base, 256), rest(base, 64), wide(base, 512), alone(base, 512);
-  const bool worth = min_degree == 0 || g->E >= PART_BESIDE;  // a fork; without, the long rows follow the scans in their launch
-  Launch &longs = worth ? wide : scan, &mid = min_degree == 0 && g->E >= MID_ALONE ? alone : longs;
+  Launch &longs = fork ? wide : scan, &mid = fork && min_degree == 0 && g->E >= MID_ALONE ? alone : longs;
   pair.add(SEC_TOTALS, n_tiles, 2, 0);
   pair.add(SEC_P8, rows(CLS_MW2), 1, p.start[CLS_MW2]);
   pair.add(SEC_P6, rows(CLS_MW2_6), 1, p.start[CLS_MW2_6]);
@@ -934,7 +947,7 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   block.add(SEC_M8, rows(CLS_MW2 + 2), 1, p.start[CLS_MW2 + 2]);
   block.add(SEC_M6, rows(CLS_MW2 + 1), 1, p.start[CLS_MW2 + 1]);
   // Rows of up to 509 entries alone are one launch; beside others the sweep goes to the side.
-  const bool sides = pair.units + scan.units + block.units + wide.units + alone.units > 0;
+  const bool sides = fork && pair.units + scan.units + block.units + wide.units + alone.units > 0;
   Launch wave(base, 64);
   wave.add(SEC_SUM, n_tiles, 1, 0);
   wave.add(SEC_W2, rows(CLS_LDS_W2), 1, p.start[CLS_LDS_W2]);
@@ -950,10 +963,10 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   Launch* first = nullptr;
   for (Launch* l : order)
     if (l->units && !first) first = l;
-  Beside side;
   if (first) {
     first->a.call = call;
-    if (worth && rest.units + wide.units + alone.units && first != &rest && first != &wide) SKY_TRY(beside_begin(g, &side, &first->a.fork));
+    if (rest.units + wide.units + alone.units && first != &rest && first != &wide) first->a.fork = mark;
+    else side = Beside{};
     SKY_TRY(enqueue<false>(p, *first, longer, g->stream));
   }
   auto others = [&]() -> int {
@@ -1017,7 +1030,11 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
   // vertex, 26,000 tiles, 125 / 115, 300 x 25 x 10 with 32 231 / 225, 40,000 x 25 x 10 676 / 669, 2,000 x 10 x 10 on the scale-21 graph with 40, 13,000
   // tiles, 338 / 329; with few tiles it costs more launches: 28,208 x 10 x 10 on the scale-19 graph with 5 140 / 149, 1,165 x 25 x 10, scale 16,
   // 125 / 139, 476 x 5 x 3 on the scale-22 graph with 5 75 / 79.)
-  const bool apart = f.few && n_tiles >= TILES_APART;
+  Beside side;
+  ForkMark mark{nullptr, 0};
+  if (f.few && n_tiles >= TILES_APART) SKY_TRY(beside_begin(g, &side, &mark));
+  const bool apart = side.stream[0] != nullptr;
+  sum.a.fork = mark;
   auto add = [&](Launch& l, Section k, uint32_t per, int cls, int ncls = 1) {
     uint32_t upper = 0;
     for (int c = 0; c < ncls; ++c) upper += f.cap[cls + c];
@@ -1063,12 +1080,10 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
     for (const Launch* l : {&wave, &pair, &wide, &block}) SKY_TRY(enqueue<true>(p, *l, longer, g->stream));
     return SKY_OK;
   }
-  Beside side;
-  SKY_TRY(beside_begin(g, &side, &sum.a.fork));
   SKY_TRY(enqueue<true>(p, sum, longer, g->stream));
   auto others = [&]() -> int {
-    if (side.stream[0]) SKY_TRY(beside_fork(&side, 0));
-    for (const Launch* l : {&wide, &block, &pair, &wave}) SKY_TRY(enqueue<true>(p, *l, longer, side.stream[0] ? side.stream[0] : g->stream));
+    SKY_TRY(beside_fork(&side, 0));
+    for (const Launch* l : {&wide, &block, &pair, &wave}) SKY_TRY(enqueue<true>(p, *l, longer, side.stream[0]));
     for (const Launch* l : {&totals, &scan, &emit}) SKY_TRY(enqueue<true>(p, *l, false, g->stream));
     return beside_join(&side);
   };

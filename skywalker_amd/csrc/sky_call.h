@@ -106,8 +106,8 @@ struct ForkMark {
 __device__ __forceinline__ void fork_mark(const ForkMark& f) {
   if (f.word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(f.word, f.number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-// A fork, and the mark for the next kernel on the graph's stream.  b->stream stays null where the streams cannot be made, on a
-// device without such waits, and where another device than the graph's is current.
+// A fork, and the mark for the next kernel on the graph's stream.  b->stream stays null where the knob build_streams is 0, on a
+// device without such waits, where the streams cannot be made, and where another device than the graph's is current.
 int beside_begin(sky_graph* g, Beside* b, ForkMark* mark);
 // With that kernel on its way: side stream k waits for its mark, if it does not already.
 int beside_fork(Beside* b, int k);

@@ -142,7 +142,6 @@ void call_cancel(sky_graph* g) { g->call.dirty = false; }
 
 // ---------------------------------------------------------------- beside the graph's stream
 namespace {
-constexpr int MAX_DEVICES = 64;
 struct SideRuntime {
   using Stream = hipStream_t;
   int device;
@@ -159,7 +158,7 @@ struct SideRuntime {
     return e == hipSuccess;
   }
 };
-SidePool<SideRuntime> g_side[MAX_DEVICES];
+SidePool<SideRuntime> g_side[SIDE_DEVICES];
 }  // namespace
 
 // The last kernel of each of the n side streams of a fork.  (A word for each, and a wait for each on the graph's stream: 4.5 us apiece.)
@@ -174,11 +173,12 @@ int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
   *mark = ForkMark{nullptr, 0};
   int current = -1;
   SKY_HIP(hipGetDevice(&current));
-  if (g->device != current || current < 0 || current >= MAX_DEVICES) return SKY_OK;  // the graph's stream is the current device's
+  const SideAsk ask{option(g, OPT_BUILD_STREAMS), g->device, current};
+  if (!ask.allowed()) return SKY_OK;
   if (!g->call.host) SKY_TRY(take_words(g->device, &g->call));
   std::lock_guard<std::mutex> lock(g_mutex);
   SideRuntime runtime{g->device};
-  if (!g_side[g->device].take(runtime, &g->sides)) return SKY_OK;
+  if (!g_side[g->device].take(runtime, &g->sides, ask)) return SKY_OK;
   for (int k = 0; k < SIDE_STREAMS; ++k) b->stream[k] = g_side[g->device].stream[k];
   b->main = g->stream;
   b->dev = g->call.dev;

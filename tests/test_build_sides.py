@@ -34,6 +34,7 @@ struct Runtime {
 int main() {
   Runtime rt;
   SidePool<Runtime> pool;
+  const SideAsk yes{1, 0, 0};
   %s
 }
 """
@@ -52,7 +53,7 @@ def test_streams_are_shared_and_go_with_the_last_graph_that_has_them(run):
     run("""
   for (int round = 0; round < 3; ++round) {
     SideHold a, b, never;
-    assert(pool.take(rt, &a) && pool.take(rt, &a) && pool.take(rt, &b));
+    assert(pool.take(rt, &a, yes) && pool.take(rt, &a, yes) && pool.take(rt, &b, yes));
     assert(rt.live.size() == SIDE_STREAMS && rt.made == SIDE_STREAMS * (round + 1));
     pool.give(rt, &never);
     pool.give(rt, &a);
@@ -70,14 +71,30 @@ def test_a_graph_does_without_streams_that_cannot_be_made(run, able, fail_from):
     run("""
   SideHold a, b;
   rt.able = %d, rt.fail_from = %d;
-  assert(!pool.take(rt, &a) && !a.held && rt.live.empty() && pool.holders == 0);
+  assert(!pool.take(rt, &a, yes) && !a.held && rt.live.empty() && pool.holders == 0);
   rt.able = true, rt.fail_from = 1000;
   const int made = rt.made;
-  assert(!pool.take(rt, &a) && rt.made == made);
-  assert(pool.take(rt, &b) && rt.live.size() == SIDE_STREAMS);
+  assert(!pool.take(rt, &a, yes) && rt.made == made);
+  assert(pool.take(rt, &b, yes) && rt.live.size() == SIDE_STREAMS);
   pool.give(rt, &a);
-  assert(rt.live.size() == SIDE_STREAMS && pool.take(rt, &a));
+  assert(rt.live.size() == SIDE_STREAMS && pool.take(rt, &a, yes));
   pool.give(rt, &b);
   pool.give(rt, &a);
   assert(rt.live.empty());
 """ % (able, fail_from))
+
+
+@pytest.mark.parametrize("ask", ["0, 0, 0", "1, 0, 1", "1, 1, 0", "1, 0, -1", "1, -1, -1", "1, 64, 64"])
+def test_no_fork_with_the_knob_off_or_another_device_current(run, ask):
+    # nor where the streams are there, for this graph too; nothing is made, nothing held
+    run("""
+  const SideAsk no{%s};
+  SideHold a, b;
+  assert(!pool.take(rt, &a, no) && rt.made == 0 && !a.held);
+  assert(pool.take(rt, &a, yes) && !pool.take(rt, &a, no) && a.held);
+  assert(!pool.take(rt, &b, no) && !b.held && pool.holders == 1);
+  assert(pool.take(rt, &b, yes) && pool.holders == 2);
+  pool.give(rt, &a);
+  pool.give(rt, &b);
+  assert(rt.live.empty());
+""" % ask)

@@ -687,3 +687,62 @@ def test_vertices_that_a_workgroup_of_the_collection_meets_again(orc, kind):
         d, sl, sampled, _ = g.sample_online(seeds, fan, 76)
         assert np.array_equal(sl.to_host((n, slen)), want[1]) and np.array_equal(d.to_host((n, lps)), want[0]) and sampled == want[2]
         g.free()
+
+
+@pytest.fixture(scope="module")
+def many_tiles():
+    # 1,200 rows of 9 to 13 tiles each: 14,500 tiles, more than a launch of one workgroup a row holds rows at a time, and enough for launches of
+    # their own beside the rows of a frontier
+    rng = np.random.default_rng(93)
+    degs = np.concatenate([rng.integers(8190, 12500, 1200), rng.integers(33, 5000, 300), np.full(20000, 3)])
+    rng.shuffle(degs)
+    xadj, adjncy, w = graph_from_degrees(degs, rng, "lognormal2")
+    long_rows = np.flatnonzero(degs >= 8190).astype(np.uint32)
+    adjncy[rng.random(len(adjncy)) < 0.5] = rng.choice(long_rows, 1)[0]  # a row that is met at the next hop too
+    return xadj, adjncy, w, long_rows, np.flatnonzero(degs < 8190).astype(np.uint32)
+
+
+@pytest.mark.parametrize("streams", [1, 0])
+@pytest.mark.parametrize("asked", ["one", "tenth", "all", "none"])
+def test_frontiers_beside_the_passes_over_many_tiles(orc, many_tiles, asked, streams):
+    # two hops, so that a build follows the build before on the same words; the third call finds what the first two left
+    from skywalker_amd import capi
+    xadj, adjncy, w, long_rows, others = many_tiles
+    rng = np.random.default_rng(94)
+    mine = {"one": long_rows[600:601], "tenth": long_rows[::10], "all": long_rows, "none": long_rows[:0]}[asked]
+    seeds = np.concatenate([mine, rng.permutation(others)[:2000].astype(np.uint32)])
+    fan = [1, 7, 3]
+    lps, slen = capi.sample_layout(fan)
+    want = orc.sample_online(xadj, adjncy, w, seeds, fan, 77)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_direct", 0)
+    g.set_option("build_streams", streams)
+    for _ in range(3):
+        d, sl, sampled, _ = g.sample_online(seeds, fan, 77)
+        assert np.array_equal(sl.to_host((len(seeds), slen)), want[1]) and np.array_equal(d.to_host((len(seeds), lps)), want[0])
+        assert sampled == want[2]
+    g.free()
+
+
+@pytest.mark.parametrize("streams", [1, 0])
+def test_sessions_beside_the_passes_over_many_tiles(orc, many_tiles, streams):
+    # weights of the caller's, other ones in the graph
+    import ctypes as C
+    from skywalker_amd import capi
+    xadj, adjncy, w, long_rows, others = many_tiles
+    seeds = np.concatenate([long_rows[::3], others[:500]])
+    fan = [1, 5, 2]
+    lps, slen = capi.sample_layout(fan)
+    want = orc.sample_online(xadj, adjncy, w, seeds, fan, 78)
+    g = capi.Graph.upload(xadj, adjncy, w[::-1].copy())
+    g.set_option("build_streams", streams)
+    w_d = capi.DeviceArray.from_host(w)
+    for _ in range(2):
+        s = open_session(capi, g, seeds, fan, 78)
+        for hop in range(2):
+            session_frontier(capi, s[0], hop)
+            capi._ck(capi.lib().sky_sample_session_hop(s[0], C.c_uint32(hop), w_d.ptr))
+        sampled, _ = session_end(capi, s[0])
+        assert np.array_equal(s[4].to_host((len(seeds), slen)), want[1]) and np.array_equal(s[3].to_host((len(seeds), lps)), want[0])
+        assert sampled == want[2]
+    g.free()

@@ -654,3 +654,34 @@ def test_walks_of_sixteen_walkers_a_wavefront(orc, walkers, index):
         want = orc.walk_offline(xadj, adjncy, prob, alias, seeds, 24, stop, 9)
         assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host((walkers, 25)), want[0]) and sampled == want[2]
     g.free()
+
+
+@pytest.mark.parametrize("streams", [1, 0])
+@pytest.mark.parametrize("E", [(1 << 24) - 1, 1 << 24])
+def test_online_walks_that_build_the_longer_rows(orc, E, streams):
+    # the largest graph whose longer rows are built in order and the smallest where they go out beside one another: rows of two wavefronts and
+    # more, merged and held ones, streamed ones, ones by tiles; the third walk finds what the first two left
+    from skywalker_amd import capi
+    rng = np.random.default_rng(67)
+    degs = list(rng.integers(510, 2558, 900)) + list(rng.integers(2558, 5118, 500)) + list(rng.integers(5118, 8190, 200)) + \
+        list(rng.integers(8190, 24577, 250)) + list(rng.integers(24577, 65534, 12)) + [70001, 600001] + list(rng.integers(33, 510, 3000))
+    left = E - sum(degs)
+    degs += [31] * (left // 31) + [left % 31]
+    rng.shuffle(degs)
+    xadj = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    V = len(degs)
+    adjncy = rng.integers(0, V, E, dtype=np.uint32)
+    long_rows = np.flatnonzero(np.array(degs) >= 510)
+    some = rng.random(E) < 0.5
+    adjncy[some] = rng.choice(long_rows, int(some.sum()))
+    w = rng.lognormal(0, 2, E).astype(np.float32)
+    seeds = rng.integers(0, V, 6000).astype(np.uint32)
+    prob, alias, _ = orc.alias_build(xadj, w)
+    want = orc.walk_offline(xadj, adjncy, prob, alias, seeds, 12, 0.0, 5)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_full_build", 0)
+    g.set_option("build_streams", streams)
+    for _ in range(3):
+        paths, lengths, sampled, _ = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 12, 0.0, 5)
+        assert np.array_equal(lengths.to_host(), want[1]) and np.array_equal(paths.to_host(want[0].shape), want[0]) and sampled == want[2]
+    g.free()
