@@ -64,10 +64,10 @@ int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call);
 // for all frontiers of a call.
 int frontier_lists(sky_graph* g, const BuildPlan& p, uint32_t n_upper, sky_graph::PoolBuf* buf, FrontierLists* f);
 // Builds the rows in the segments (counts: their lengths, on the device, and behind them a word that is 0 the first time; `again`: not
-// the first time with these counts) and those of the tiled classes whose bit is set
-// and whose word in `built` (one per row of the plan that has geometry, the call's own, 0 at first) is not: it then is.
-// Nothing waits for the device.
-int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uint32_t* counts, bool again, const uint32_t* bitmap, uint32_t* built);
+// the first time with these counts) and those of the tiled classes whose bit is set, unless another hop has: `built`, a word for each row of the
+// plan that has geometry, the call's own, 0 at first, then holds the hop's number + 1.  Nothing waits for the device.
+int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uint32_t* counts, bool again, const uint32_t* bitmap,
+                   uint32_t* built, uint32_t hop);
 
 // Appends the vertices of the calling workgroup's lanes whose `fresh` is set to their classes' segments: one global atomic
 // per class that occurs.  All threads of the workgroup call it; s_cnt and s_base hold CLS_COUNT words of LDS each.

@@ -79,7 +79,8 @@ struct FusedArgs {
   uint4* ranges;
   const uint32_t* bitmap;  // frontier: bit set for every vertex whose row has been asked for (null: every row is built)
   uint32_t bit_mask;       // of the bitmap (frontier_bit)
-  uint32_t* built;         // frontier: by row of trows, set once a build of the same call has made it
+  uint32_t* built;         // frontier: by row of trows, the hop (from 1 on) whose build in the same call has made it
+  uint32_t hop;            // this one
   uint32_t* next;          // frontier: units of the wide launch that are taken, 0 at first (null: every grid-th for each workgroup)
   uint32_t tile0, trow0;  // first tile and row of those this build makes tile by tile
   bool ledgers_done;
@@ -189,7 +190,8 @@ __device__ __forceinline__ bool tile_asked(const FusedArgs& a, uint32_t tile) {
   const TileGeom tg = a.geom[tile];
   if (tg.span == 0) return false;  // there are fewer tiles than their bound
   const uint32_t b = frontier_bit(a.trows[tg.row].v, a.bit_mask);
-  const bool active = ((a.bitmap[b >> 5] >> (b & 31)) & 1u) && !a.built[tg.row];
+  const uint32_t made = a.built[tg.row];
+  const bool active = ((a.bitmap[b >> 5] >> (b & 31)) & 1u) && (made == 0 || made == a.hop);  // a hop may be built once more
   if (tg.T == 0) a.trows[tg.row].active = active ? 1u : 0u;
   return active;
 }
@@ -428,7 +430,7 @@ __global__ __launch_bounds__(512, 4) void fused_wide_kernel(FusedArgs a) {
     each_wanted(scans, blockIdx.x, gridDim.x, [&](uint32_t r) { return a.trows[a.trow0 + r].active != 0; },
                 [&](uint32_t r) {
                   scan(a.trow0 + r);
-                  if (threadIdx.x == 0) a.built[a.trow0 + r] = 1;
+                  if (threadIdx.x == 0) a.built[a.trow0 + r] = a.hop;
                   __syncthreads();
                 });
   const UnitFinder<DEV> units(a);
@@ -1014,7 +1016,7 @@ int frontier_lists(sky_graph* g, const BuildPlan& p, uint32_t n_upper, sky_graph
 __global__ void clear_taken_kernel(uint32_t* taken) { *taken = 0; }
 
 int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uint32_t* counts, bool again, const uint32_t* bitmap,
-                   uint32_t* built) {
+                   uint32_t* built, uint32_t hop) {
   g->has_walk_index = false;
   FusedArgs base = common_args(g, p, f.tiled_from);
   const uint32_t n_tiles = p.n_tiles - base.tile0, n_trows = p.n_trows - base.trow0;
@@ -1023,6 +1025,7 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
   base.bitmap = bitmap;
   base.bit_mask = frontier_mask(g->V);
   base.built = built;
+  base.hop = hop + 1;
   Launch wave(base, 64), pair(base, 128), wide(base, 512), block(base, 256);
   Launch sum(base, 64), totals(base, 128), scan(base, 512), emit(base, 256);
   // The passes over tiles wait for one another, and where they look at many tiles for a frontier of few rows they are a good part: the rows then

@@ -725,8 +725,8 @@ struct SampleSession {
   CallWords own_words;  // of a session whose steps are calls of their own
   uint32_t *bitmap = nullptr, *list = nullptr, *d_count = nullptr;
   // Counters of the frontiers, a hop's own each, cleared when the call begins: the length of its list, then FRONTIER_WORDS
-  // with the rows of every degree class (dev_sized).  Behind them a word for every row that can be made tile by tile, set when
-  // this call has built it: kept with the graph's rows instead, another call's build between two hops of a session made the
+  // with the rows of every degree class (dev_sized).  Behind them a word for every row that can be made tile by tile, for the hop
+  // of this call that has built it: kept with the graph's rows instead, another call's build between two hops of a session made the
   // session build the row again, from weights that its caller had not supplied.
   uint32_t *list_counts = nullptr, *front_counts = nullptr, *built = nullptr;
   FrontierLists front;
@@ -904,7 +904,7 @@ struct SampleSession {
     if (!online || !N || !frontier_upper) return SKY_OK;
     float* const own = g->adjwgt;
     if (weights) g->adjwgt = const_cast<float*>(weights);  // the build only reads it
-    const int rc = dev_sized ? build_frontier(g, *plan, front, front_counts + h * FRONTIER_WORDS, made[h], bitmap, built)
+    const int rc = dev_sized ? build_frontier(g, *plan, front, front_counts + h * FRONTIER_WORDS, made[h], bitmap, built, h)
                              : build_rows(g, list, frontier_count, nullptr);
     made[h] = 1;
     g->adjwgt = own;
