@@ -258,7 +258,7 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      graph of more than 2^27 entries, and in the four launches that make all of a build of up to 2^27 entries.  0 or 1
  *      gives such a build its class kernels back.  Same tables.
  *      "build_streams" (default 1): kernels of a build that do not depend on one another go out beside one another, on the graph's
- *      stream and up to three side streams, which the graphs of a device share and the last of them takes with it: the launches of a build of
+ *      stream and up to three side streams, which the graphs of a device share, from the second such call of a graph on or once they are there: the launches of a build of
  *      up to 2^27 entries, the longer rows alone that an online walk makes on a graph of 2^24 entries and more, the rows of a frontier of up to
  *      65,536 beside the passes over 8,192 tiles and more, and the kernels of the degree classes of larger builds (and of smaller ones of
  *      2 M entries and more whose other knobs ask for class kernels).  What follows waits for a word in pinned memory, by a kernel of

@@ -787,7 +787,8 @@ int build_rows(sky_graph* g, const uint32_t* src, uint32_t n, EventTimer* tm, Ca
   RowRef* vlist = planned ? g->plan->rows : sc.vlist;
   // clears the counters of the binning pass and, unless the plan's first kernel has, notes when the call began
   ForkMark fork{nullptr, 0};
-  if (!tm && n > 0) SKY_TRY(beside_begin(g, &fan.b, &fork));
+  if (!tm && n > 0 && (small_in_place || std::min<uint64_t>(g->E, (uint64_t)n * g->max_degree) >= FAN_MIN_EDGES))
+    SKY_TRY(beside_begin(g, &fan.b, &fork, SIDE_STREAMS));
   hipLaunchKernelGGL(build_begin_kernel, dim3(1), dim3(128), 0, st, sc.counters, (uint32_t)(COUNTER_BYTES / 4), call, fork);
   SKY_HIP(hipGetLastError());
   if (n > 0) {

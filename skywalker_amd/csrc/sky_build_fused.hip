@@ -917,7 +917,8 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   for (int c = CLS_MW2 + 4; c <= CLS_MW2 + MERGE_MAX_NW - 2; ++c) past_block += rows(c);
   Beside side;
   ForkMark mark{nullptr, 0};
-  if (min_degree == 0 ? past_wave : g->E >= PART_BESIDE && past_block) SKY_TRY(beside_begin(g, &side, &mark));
+  const bool two = min_degree == 0 && g->E >= MID_ALONE && past_block;
+  if (min_degree == 0 ? past_wave : g->E >= PART_BESIDE && past_block) SKY_TRY(beside_begin(g, &side, &mark, two ? 2 : 1));
   // Without a fork four launches follow one another: the sweep rides along in the first, the long rows behind the scans.
   const bool fork = side.stream[0] != nullptr;
   const uint32_t sweeps = sweep(fork);
@@ -1035,7 +1036,7 @@ int build_frontier(sky_graph* g, const BuildPlan& p, const FrontierLists& f, uin
   // 125 / 139, 476 x 5 x 3 on the scale-22 graph with 5 75 / 79.)
   Beside side;
   ForkMark mark{nullptr, 0};
-  if (f.few && n_tiles >= TILES_APART) SKY_TRY(beside_begin(g, &side, &mark));
+  if (f.few && n_tiles >= TILES_APART) SKY_TRY(beside_begin(g, &side, &mark, 1));
   const bool apart = side.stream[0] != nullptr;
   sum.a.fork = mark;
   auto add = [&](Launch& l, Section k, uint32_t per, int cls, int ncls = 1) {

@@ -84,7 +84,7 @@ __device__ __forceinline__ void call_answer(CallHost* host, unsigned long long n
   __hip_atomic_store(&host->answer[word], value | number << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 int call_answered(sky_graph* g, CallWords* w, unsigned long long* values, int n);
-// Kernels beside those of the graph's stream, on streams that all graphs of a device share and the last of them takes with it (sky_sides.h).  These and the graph's stream wait for one
+// Kernels beside those of the graph's stream, on streams that all graphs of a device share (sky_sides.h).  These and the graph's stream wait for one
 // another by words in pinned memory: a kernel on the graph's stream notes that it runs (fork_mark), so that everything in front of it has
 // ended, and of small last ones on the others the one that finds all of them there that everything in front of these has.  Who waits, by a stream operation (one
 // thread of the runtime's that reads the word until the number is there), is always enqueued behind the kernel that writes, so that
@@ -106,9 +106,10 @@ struct ForkMark {
 __device__ __forceinline__ void fork_mark(const ForkMark& f) {
   if (f.word && blockIdx.x == 0 && threadIdx.x == 0) __hip_atomic_store(f.word, f.number, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
-// A fork, and the mark for the next kernel on the graph's stream.  b->stream stays null where the knob build_streams is 0, on a
-// device without such waits, where the streams cannot be made, and where another device than the graph's is current.
-int beside_begin(sky_graph* g, Beside* b, ForkMark* mark);
+// A fork over so many side streams, and the mark for the next kernel on the graph's stream.  b->stream stays null where the knob
+// build_streams is 0, in the first call of a graph that asks unless the streams are there, on a device without such waits, where the
+// streams cannot be made, and where another device than the graph's is current.
+int beside_begin(sky_graph* g, Beside* b, ForkMark* mark, int streams);
 // With that kernel on its way: side stream k waits for its mark, if it does not already.
 int beside_fork(Beside* b, int k);
 // The graph's stream waits for what the side streams of the fork hold.

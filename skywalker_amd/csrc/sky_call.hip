@@ -133,6 +133,7 @@ int call_begin(sky_graph* g, CallWords* w, CallDevice** call) {
   if (!w->host) SKY_TRY(take_words(g->device, w));
   if (w->dirty) SKY_HIP(hipMemsetAsync(w->dev, 0, sizeof(CallDevice), g->stream));
   w->dirty = true;  // until it has ended well
+  ++g->calls;
   *call = w->dev;
   return SKY_OK;
 }
@@ -168,18 +169,18 @@ __global__ void beside_done_kernel(CallDevice* dev, CallHost* host, uint32_t n, 
   __hip_atomic_store(&host->done, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-int beside_begin(sky_graph* g, Beside* b, ForkMark* mark) {
+int beside_begin(sky_graph* g, Beside* b, ForkMark* mark, int streams) {
   *b = Beside{};
   *mark = ForkMark{nullptr, 0};
   int current = -1;
   SKY_HIP(hipGetDevice(&current));
-  const SideAsk ask{option(g, OPT_BUILD_STREAMS), g->device, current};
+  const SideAsk ask{option(g, OPT_BUILD_STREAMS), g->device, current, g->calls, streams};
   if (!ask.allowed()) return SKY_OK;
   if (!g->call.host) SKY_TRY(take_words(g->device, &g->call));
   std::lock_guard<std::mutex> lock(g_mutex);
   SideRuntime runtime{g->device};
   if (!g_side[g->device].take(runtime, &g->sides, ask)) return SKY_OK;
-  for (int k = 0; k < SIDE_STREAMS; ++k) b->stream[k] = g_side[g->device].stream[k];
+  for (int k = 0; k < streams; ++k) b->stream[k] = g_side[g->device].stream[k];
   b->main = g->stream;
   b->dev = g->call.dev;
   b->host = g->call.host;
@@ -216,7 +217,7 @@ void beside_drop(Beside* b) {
 }
 
 void beside_release(sky_graph* g) {
-  if (!g->sides.held) return;
+  if (g->device < 0 || g->device >= SIDE_DEVICES) return;
   std::lock_guard<std::mutex> lock(g_mutex);
   SideRuntime runtime{g->device};
   g_side[g->device].give(runtime, &g->sides);

@@ -64,6 +64,7 @@ struct sky_graph {
   std::vector<ProfileEntry> build_profile;
 
   sky::CallWords call;  // how a call on this graph reports its end (sky_call.h)
+  unsigned long long calls = 0;  // begun so far, sessions and their steps among them
   sky::SideHold sides;  // its share of the device's side streams
 
   // Device buffers that calls on this graph reuse instead of allocating each time (they only grow).

@@ -6,36 +6,50 @@
 namespace sky {
 
 constexpr int SIDE_STREAMS = 3;
+constexpr int SIDE_IDLE = 16;
 
 // What a graph has of them.
 struct SideHold {
-  bool held = false;     // they stay as long as it does
-  bool refused = false;  // it asked for some that could not be made
+  bool held = false;             // they stay as long as it does
+  bool refused = false;          // it asked for some that could not be made
+  unsigned long long first = 0;  // its first call that asked for some
 };
 constexpr int SIDE_DEVICES = 64;
 // What a call asks with.
 struct SideAsk {
   long long knob;       // build_streams
   int device, current;  // the graph's and the one that is current, whose null stream the graph's kernels go to
+  unsigned long long call;  // which of the graph's calls, from 1 on
+  int streams = SIDE_STREAMS;
   bool allowed() const { return knob != 0 && device == current && device >= 0 && device < SIDE_DEVICES; }
 };
 
-// The side streams of one device: shared by the graphs that have asked for them, and destroyed when the last of these is freed.  Calls
-// are the caller's to serialise.  Runtime: can(), whether the device has what they wait with; create(Stream*); destroy(Stream).
+// The side streams of one device, shared by the graphs that have asked for them.
+// One to three of them take 0.05 to 0.5 ms to make where the process has had as many before, 3.5 ms each where it has not, and 0.7 to 1.2 ms to
+// destroy, most of it in the next allocations and frees; a call gains 5 to 100 us by them (MI355X, ROCm 7.2).  So a graph's first call
+// that asks finds those that are there and makes none (a graph that is built once never has that back, one whose rows are built again is built
+// many times), and they outlast the graphs that had them until SIDE_IDLE graphs in a row have been freed that did without: a program
+// that takes one graph after another makes them once.  (The first build of a graph of 17 M entries with its lists and the tables' allocation, no
+// other graph there, us: in order 400, on streams that are there 380, on streams of its own 600, of which a process's first 12,000; the
+// graph after one that has taken its streams with it also 0.5 ms later to upload.)
+// Calls are the caller's to serialise.  Runtime: can(), whether the device has what they wait with; create(Stream*); destroy(Stream).
 template <class Runtime>
 struct SidePool {
   using Stream = typename Runtime::Stream;
   Stream stream[SIDE_STREAMS] = {};
-  int holders = 0;
+  int holders = 0, without = 0;  // graphs freed since the last holder
 
   // Whether the graph has them for the present call; without, its kernels go out in order, after some that could not be made for good.
   bool take(Runtime& rt, SideHold* h, const SideAsk& ask) {
     if (!ask.allowed() || h->refused) return false;
-    for (Stream& s : stream) {
-      if (s || (rt.can() && rt.create(&s))) continue;
+    if (!h->first) h->first = ask.call;
+    for (int k = 0; k < ask.streams; ++k) {
+      Stream& s = stream[k];
+      if (s) continue;
+      if (h->first == ask.call) return false;
+      if (rt.can() && rt.create(&s)) continue;
       s = Stream{};
-      h->refused = true;
-      if (!holders) clear(rt);
+      h->refused = true;  // those made before it are for graphs that need fewer
       return false;
     }
     if (!h->held) ++holders;
@@ -44,7 +58,12 @@ struct SidePool {
   }
   // The graph is about to be freed.
   void give(Runtime& rt, SideHold* h) {
-    if (h->held && --holders == 0) clear(rt);
+    if (h->held) {
+      --holders;
+      without = 0;
+    } else if (holders == 0 && ++without >= SIDE_IDLE) {
+      clear(rt);
+    }
     *h = SideHold{};
   }
 

@@ -11,6 +11,9 @@ MAIN = """
 #include <set>
 #include "sky_sides.h"
 using namespace sky;
+struct Asked : SideHold {
+  Asked() { first = 1; }  // a graph that asked in its first call
+};
 struct Runtime {
   using Stream = int*;
   std::set<int*> live;
@@ -34,7 +37,8 @@ struct Runtime {
 int main() {
   Runtime rt;
   SidePool<Runtime> pool;
-  const SideAsk yes{1, 0, 0};
+  const SideAsk yes{1, 0, 0, 2}, first{1, 0, 0, 1};
+  (void)first;
   %s
 }
 """
@@ -49,37 +53,51 @@ def run(tmp_path):
     return go
 
 
-def test_streams_are_shared_and_go_with_the_last_graph_that_has_them(run):
+def test_streams_are_shared_and_go_when_graphs_do_without(run):
+    # graph after graph, one at a time or several, on the streams of the first; after SIDE_IDLE freed in a row without, they are made again
     run("""
-  for (int round = 0; round < 3; ++round) {
-    SideHold a, b, never;
-    assert(pool.take(rt, &a, yes) && pool.take(rt, &a, yes) && pool.take(rt, &b, yes));
-    assert(rt.live.size() == SIDE_STREAMS && rt.made == SIDE_STREAMS * (round + 1));
-    pool.give(rt, &never);
-    pool.give(rt, &a);
-    pool.give(rt, &a);
-    assert(rt.live.size() == SIDE_STREAMS && !a.held && b.held);
-    pool.give(rt, &b);
-    assert(rt.live.empty() && pool.holders == 0);
+  for (int round = 1; round <= 3; ++round) {
+    for (int k = 0; k < 40; ++k) {
+      Asked a, b;
+      SideHold never;
+      assert(pool.take(rt, &a, yes) && pool.take(rt, &a, yes) && pool.take(rt, &b, yes) && pool.holders == 2);
+      pool.give(rt, &a);
+      pool.give(rt, &b);
+      assert(!a.held && !a.first && pool.holders == 0 && rt.made == SIDE_STREAMS * round);
+      pool.give(rt, &never);
+    }
+    Asked c;
+    assert(pool.take(rt, &c, yes));
+    SideHold never;
+    for (int k = 0; k < 2 * SIDE_IDLE; ++k) pool.give(rt, &never);
+    assert(rt.live.size() == SIDE_STREAMS);  // whatever others do, not while a graph has them
+    pool.give(rt, &c);
+    for (int k = 0; k < SIDE_IDLE; ++k) {
+      assert(rt.live.size() == SIDE_STREAMS);
+      pool.give(rt, &never);
+    }
+    assert(rt.live.empty() && rt.made == SIDE_STREAMS * round);
   }
 """)
 
 
 @pytest.mark.parametrize("able,fail_from", [(0, 1000), (1, 0), (1, 1), (1, 2)])
 def test_a_graph_does_without_streams_that_cannot_be_made(run, able, fail_from):
-    # those that were made before the one that failed go back; the graph does not ask again, others do
+    # the graph does not ask again, others do
     run("""
-  SideHold a, b;
+  Asked a, b;
   rt.able = %d, rt.fail_from = %d;
-  assert(!pool.take(rt, &a, yes) && !a.held && rt.live.empty() && pool.holders == 0);
+  assert(!pool.take(rt, &a, yes) && !a.held && pool.holders == 0);
   rt.able = true, rt.fail_from = 1000;
   const int made = rt.made;
   assert(!pool.take(rt, &a, yes) && rt.made == made);
   assert(pool.take(rt, &b, yes) && rt.live.size() == SIDE_STREAMS);
   pool.give(rt, &a);
+  a.first = 1;
   assert(rt.live.size() == SIDE_STREAMS && pool.take(rt, &a, yes));
   pool.give(rt, &b);
   pool.give(rt, &a);
+  for (int k = 0; k < SIDE_IDLE; ++k) pool.give(rt, &b);
   assert(rt.live.empty());
 """ % (able, fail_from))
 
@@ -88,13 +106,40 @@ def test_a_graph_does_without_streams_that_cannot_be_made(run, able, fail_from):
 def test_no_fork_with_the_knob_off_or_another_device_current(run, ask):
     # nor where the streams are there, for this graph too; nothing is made, nothing held
     run("""
-  const SideAsk no{%s};
-  SideHold a, b;
+  const SideAsk no{%s, 2};
+  Asked a, b;
   assert(!pool.take(rt, &a, no) && rt.made == 0 && !a.held);
   assert(pool.take(rt, &a, yes) && !pool.take(rt, &a, no) && a.held);
   assert(!pool.take(rt, &b, no) && !b.held && pool.holders == 1);
-  assert(pool.take(rt, &b, yes) && pool.holders == 2);
-  pool.give(rt, &a);
-  pool.give(rt, &b);
-  assert(rt.live.empty());
+  assert(pool.take(rt, &b, yes) && pool.holders == 2 && rt.made == SIDE_STREAMS);
 """ % ask)
+
+
+def test_a_graphs_first_call_makes_no_streams(run):
+    # however often it asks; it takes those that another graph has, as many as there are
+    run("""
+  SideHold a, b, c, d;
+  SideAsk one = yes, later{1, 0, 0, 7};
+  one.streams = 1;
+  for (int k = 0; k < 3; ++k) assert(!pool.take(rt, &a, first) && !a.held && !a.refused);
+  assert(rt.made == 0 && pool.take(rt, &a, one) && rt.made == 1 && pool.take(rt, &a, one) && rt.made == 1);
+  SideAsk b1 = first;
+  b1.streams = 1;
+  assert(pool.take(rt, &b, b1) && b.held && rt.made == 1 && !pool.take(rt, &b, first) && rt.made == 1);
+  assert(pool.take(rt, &b, yes) && rt.made == SIDE_STREAMS && pool.holders == 2);
+  assert(pool.take(rt, &c, later) && rt.made == SIDE_STREAMS);
+  pool.give(rt, &a), pool.give(rt, &b), pool.give(rt, &c);
+  for (int k = 0; k < SIDE_IDLE; ++k) pool.give(rt, &d);
+  assert(rt.live.empty() && !pool.take(rt, &d, later) && rt.live.empty());
+""")
+
+
+def test_a_graph_that_holds_one_stream_keeps_it_where_another_cannot_be_made(run):
+    run("""
+  Asked a, b;
+  SideAsk one = yes;
+  one.streams = 1;
+  rt.fail_from = 2;
+  assert(pool.take(rt, &a, one) && !pool.take(rt, &a, yes) && a.held && a.refused && !pool.take(rt, &a, one));
+  assert(pool.take(rt, &b, one) && rt.live.size() == 2 && pool.holders == 2);
+""")
