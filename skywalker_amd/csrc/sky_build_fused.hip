@@ -21,7 +21,7 @@
 // of 2558 and more, go out beside the rest (Beside, sky_call.h), so that the tails of four launches no longer follow one another.
 // (In order / beside, us, three graphs in turn: scale 16 with 16 edges a vertex 46 / 42, scale 20 with 16 131 / 120, with 6 96 / 82, with 3
 // 69 / 54, scale 23 with 4 253 / 233, with 10 437 / 433, 3 M entries in rows of up to 20,000 70 / 58, 40 M in rows of up to 300,007 331 / 319.
-// From 60 M entries on the tails no longer count: scale 22 with 31 649 / 655, scale 24 with 6 530 / 530.  On one graph again and again, with
+// Where the launches that follow one another fill the GPU the tails no longer count: BESIDE_MERGED.  On one graph again and again, with
 // the long rows in front of the sweep scale 23 with 10 483 instead of 430; those on a third stream scale 20 with 6 69 instead of 82, with 16 110
 // instead of 104, scale 16 with 16 45 instead of 42; rows of up to 107 entries alone, one launch in order, 128 / 138.)  The
 // workgroups of a large frontier's launches stay until all units are done and leave no room beside them: those follow one another.  (The
@@ -670,6 +670,19 @@ constexpr uint32_t HOLD_ALONE = 2048;
 // Entries of a graph from which a build of its longer rows alone, which has no sweep, is worth a fork (in order / beside, us: walks without tables of
 // 10,000 x 8 on the scale-22 graph 195 / 188, of 836 x 10 on the scale-16 graph with 47 edges a vertex 75 / 79).
 constexpr uint32_t PART_BESIDE = 1u << 24;
+// Entries to build from which it is not any more: the launches then fill the GPU one after another, and share caches and LDS beside one
+// another.  (In order / beside, us, entries to build: walks of 10,000 x 8 on the scale-22 graph with 16 edges a vertex, 12.8 M, 183 / 176,
+// scale 23 with 10, 13.6 M, 175 / 169, with 12, 16.3 M, 235 / 234, with 16, 21.7 M, 279 / 282, scale 22 with 24, 19 M, 271 / 273, with 32, 25 M, 353 / 352;
+// 2,000 x 8 on the scale-24 graph with 16, 13.4 M, 266 / 220; 30,000 x 12 on scale 23 with 16, 43 M, 434 / 443, with 20, 54 M, 547 / 563, 40,000 x 16, scale
+// 22 with 24, 56 M, 524 / 531.)
+constexpr uint64_t PART_MOST = 16000000;
+
+// Entries in rows of 510..2557, which the launches of the tile passes take, from which a whole build goes out in order for the same reason.
+// (In order / beside, us, their number: scale 23 with 8 edges a vertex, 10.7 M, 371 / 364, with 10, 14.8 M, 433 / 419, scale 24 with 6, 14.7 M, 525 / 516,
+// 80 M entries in rows of up to 300,007, 9.2 M, 598 / 576, scale 22 with 16, 17 M, 364 / 348; scale 21 with 45, 18.9 M, 499 / 504, 110 M in rows of up
+// to 3,000, 22.8 M, 606 / 607, scale 22 with 31, 25.7 M, 651 / 659, scale 24 with 7, 27.8 M, 626 / 629, scale 22 with 18, 27.9 M, 425 / 435, with 22, 34 M, 491 /
+// 500, scale 23 with 14, 41 M, 612 / 619.)
+constexpr uint64_t BESIDE_MERGED = 18000000;
 
 // Tiles of a graph's plan from which a frontier of few rows has launches of their own for them (build_frontier).
 constexpr uint32_t TILES_APART = 8192;
@@ -915,10 +928,16 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   if (p.t_all > CLS_STREAM_LAST) past_block += rows(CLS_STREAM_LAST);
   past_block += rows(CLS_HOLD);
   for (int c = CLS_MW2 + 4; c <= CLS_MW2 + MERGE_MAX_NW - 2; ++c) past_block += rows(c);
+  auto entries = [&](uint32_t from, uint32_t to) {  // in rows of so many
+    uint64_t n = 0;
+    for (int c = CLS_TINY; c < CLS_COUNT; ++c)
+      if (class_min_degree(c) >= from && class_min_degree(c) < to) n += g->bin_edges[c];
+    return n;
+  };
   Beside side;
   ForkMark mark{nullptr, 0};
   const bool two = min_degree == 0 && g->E >= MID_ALONE && past_block;
-  if (min_degree == 0 ? past_wave : g->E >= PART_BESIDE && past_block) SKY_TRY(beside_begin(g, &side, &mark, two ? 2 : 1));
+  if (min_degree == 0 ? past_wave && entries(510, 2558) < BESIDE_MERGED : g->E >= PART_BESIDE && past_block && entries(min_degree, 0xFFFFFFFFu) < PART_MOST) SKY_TRY(beside_begin(g, &side, &mark, two ? 2 : 1));
   // Without a fork four launches follow one another: the sweep rides along in the first, the long rows behind the scans.
   const bool fork = side.stream[0] != nullptr;
   const uint32_t sweeps = sweep(fork);
