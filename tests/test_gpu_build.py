@@ -864,9 +864,9 @@ def test_rows_of_8190_to_24576_entries_streamed_and_longer_ones_by_tiles(orc, se
 @pytest.mark.parametrize("by_class", [False, True])
 @pytest.mark.parametrize("longest", [600, 13000, 30000, 70001])
 def test_builds_over_several_streams_one_after_another_and_from_two_threads(orc, longest, by_class):
-    # the sweep and the long rows beside the other launches, a tile path among these for the longest, or the class kernels on four
-    # streams: two weight arrays in turn, so that what an earlier build left shows, written just before each build and read just after
-    # it; two graphs, a thread each
+    # the sweep and the long rows beside the other launches, a tile path among these for the longest (rows of up to 600 entries are
+    # one launch), or the class kernels on four streams: two weight arrays in turn, so that what an earlier build left shows, written
+    # just before each build and read just after it; two graphs, a thread each
     import threading
     from helpers import weights
     from skywalker_amd import capi
@@ -906,12 +906,14 @@ def test_builds_over_several_streams_one_after_another_and_from_two_threads(orc,
 
 
 @pytest.mark.parametrize("E", [(1 << 24) - 1, 1 << 24])
-def test_rows_of_2558_to_5117_entries_in_a_launch_of_their_own(orc, E):
-    # the smallest build that gives them one and the largest that does not; the edges of their classes
+@pytest.mark.parametrize("longer", [False, True])
+def test_rows_of_2558_to_5117_entries_in_a_launch_of_their_own(orc, E, longer):
+    # the smallest build that gives them one and the largest that does not; the edges of their classes; enough rows of 2558..3581 entries that
+    # these go out with the launch of 256 threads.  A row of more than 12288 entries keeps the build out of the one launch of small ones.
     from skywalker_amd import capi
     rng = np.random.default_rng(61)
     degs = list(rng.integers(2558, 5118, 300)) + [2557, 2558, 3069, 3070, 3581, 3582, 4093, 4094, 4605, 4606, 5117, 5118] * 2 + \
-        list(rng.integers(1, 300, 20000)) + list(rng.integers(8190, 9000, 20))
+        list(rng.integers(1, 300, 20000)) + list(rng.integers(8190, 9000, 20)) + [13000] + list(rng.integers(2558, 3582, 1500 if longer else 0))
     left = E - sum(degs)
     degs += [31] * (left // 31) + [left % 31]
     rng.shuffle(degs)
@@ -919,8 +921,9 @@ def test_rows_of_2558_to_5117_entries_in_a_launch_of_their_own(orc, E):
     adjncy = np.zeros(E, np.uint32)
     w = rng.lognormal(0, 2, E).astype(np.float32)
     g = capi.Graph.upload(xadj, adjncy, w)
-    for _ in range(2):
-        g.build_tables()
+    # a graph's first build goes out in order where there are no side streams yet; from other weights, so that rows the second leaves out show
+    g.build_tables_from_weights(capi.DeviceArray.from_host(np.concatenate([w[::-1], np.zeros(4, np.float32)])))
+    g.build_tables()
     prob, alias, valid = g.tables()
     g.free()
     oprob, oalias, ovalid = orc.alias_build(xadj, w)

@@ -645,7 +645,7 @@ def test_a_vertex_that_starts_every_sample_is_not_swept_for_each_of_them():
 
 @pytest.mark.parametrize("asked", ["one", "tenth", "all", "none"])
 def test_frontiers_that_ask_for_some_of_many_rows_made_by_tiles(orc, asked):
-    # 500 rows of 9 to 13 tiles each, five tiles to a workgroup of the launch with the fewest, of which the frontier wants some
+    # 500 rows of 9 to 13 tiles each, of which the frontier wants some; fewer than the 8,192 tiles from which the rows go out beside the passes
     from skywalker_amd import capi
     rng = np.random.default_rng(91)
     degs = np.concatenate([rng.integers(8190, 12500, 500), np.full(20000, 3)])
