@@ -235,7 +235,7 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      entry (the tile-parallel path from 4094 entries on).  Both give the same table.
  *      "stream_min_edges" (default 4000000): rows of 8190..524287 entries have a kernel of their own (one workgroup
  *      streams a row); when a build holds no more than this many entries in such rows, too few to fill the GPU
- *      with one workgroup each, they go to the tile-parallel path instead.  Builds that go out in four launches take
+ *      with one workgroup each, they go to the tile-parallel path instead.  Builds that go out in few launches take
  *      that path also above the limit, for all of these rows or for those of more than 24576 entries, where the longest such row would
  *      outlast everything else, and at the default, and no other value, stream those of up to 24576 entries below it where
  *      that takes less.  Tests set 0: always by one workgroup.
@@ -255,11 +255,12 @@ int sky_philox_selftest(const uint32_t* ctr_host, const uint32_t* key_host, uint
  *      "small_in_place" (default -1): 1 builds the rows of at most 32 entries in one kernel that walks the vertices
  *      in order and needs no row lists (it runs beside the kernels of the long rows); 0 builds
  *      them by degree class like all other rows; -1 takes the former for builds of at least 2^25 rows or of all rows of a
- *      graph of more than 2^27 entries, and in the four launches that make all of a build of up to 2^27 entries.  0 or 1
+ *      graph of more than 2^27 entries, and in the few launches that make all of a build of up to 2^27 entries.  0 or 1
  *      gives such a build its class kernels back.  Same tables.
  *      "build_streams" (default 1): kernels of a build that do not depend on one another go out beside one another, on the graph's
  *      stream and up to three side streams, which the graphs of a device share, from the second such call of a graph on or once they are there: the launches of a build of
- *      up to 2^27 entries, the longer rows alone that an online walk makes on a graph of 2^24 entries and more, the rows of a frontier of up to
+ *      up to 2^27 entries (of which less than 18 M in rows of 510..2557), up to 16 M entries in the longer rows alone that an online walk makes on a graph of
+ *      2^24 entries and more, the rows of a frontier of up to
  *      65,536 beside the passes over 8,192 tiles and more, and the kernels of the degree classes of larger builds (and of smaller ones of
  *      2 M entries and more whose other knobs ask for class kernels).  What follows waits for a word in pinned memory, by a kernel of
  *      the runtime's.  0 keeps every kernel of every build on the graph's stream, for tools that let one kernel run at a time, and makes all

@@ -22,7 +22,7 @@
 // Dispatch is by degree class (sky_graph.h): one lane per vertex (deg <= 2), 2 to 32 lanes per vertex with the prefix
 // arrays in a per-wave LDS strip (deg <= 192), 64 to 512 threads per vertex that pair by a merge in LDS (deg <= 5117),
 // 512 threads that hold or stream the row (sky_build_stream.hip), and the tile-parallel path of sky_build_tiled.hip for
-// longer rows.  Builds of up to FUSED_MAX_ENTRIES send the same row builders out in four launches (sky_build_fused.hip).
+// longer rows.  Builds of up to FUSED_MAX_ENTRIES send the same row builders out in few launches (sky_build_fused.hip).
 #include <algorithm>
 #include <vector>
 
@@ -647,7 +647,8 @@ void pool_release(sky_graph* g) {
 // (With events for the waits, and one stream for the classes of builds of 1 G entries and more / now, us: scale 26 with 8 edges a vertex
 // 2,435 / 2,368, with 28 8,013 / 8,010, means of ten processes a side, of which those of the latter differ by 200; scale 23 with 40
 // 1,535 / 1,495, scale 22 with 50 965 / 937, scale 24 with 16 1,235 / 1,230.  The streaming kernel in front of the merge kernels, the
-// short rows behind them, or two streams instead of four: the same or up to 5 % slower.)
+// short rows behind them, or two streams instead of four: the same or up to 5 % slower.  Smaller builds, which come here by other
+// knobs, in order / over four streams: 2.1 M entries in rows of up to 5,000 178 / 146, 4 M of up to 50,000 247 / 190, scale 20 with 6 207 / 177.)
 constexpr uint64_t FAN_MIN_EDGES = 2000000;
 struct StreamFan {
   Beside b;
@@ -741,17 +742,19 @@ int prepare_build_scratch(sky_graph* g, uint32_t max_rows) {
   return SKY_OK;
 }
 
-// Largest build that goes out in the four launches of sky_build_fused.hip.  Above, a class fills the GPU by itself, and short
-// rows beside the others in a kernel of their own are worth more than fewer launches.  (Four launches / by class, us:
-// scale 20 with 120 edges a vertex 799 / 829, scale 23 with 10 585 / 608, scale 24 with 7 868 / 877, scale 22 with 20
-// 588 / 564; scale 22 with 36 911 / 846, scale 24 with 9 1071 / 1045, with 16 1631 / 1534, scale 23 with 31 1433 / 1438.)
+// Largest build that goes out in the few launches of sky_build_fused.hip.  Above, a class fills the GPU by itself, and short
+// rows beside the others in a kernel of their own are worth more than fewer launches.  (In few launches / by class, us, one after
+// another and, in brackets, with the device waited for in between, which takes 35 us more where all side streams have had work: scale 22 with
+// 16 edges a vertex 352 / 409, with 18 425 / 460, with 22 493 / 467 (507 / 522), with 31 652 / 647 (665 / 707), scale 20 with 120 763 / 749 (775 / 826), scale 21
+// with 60 698 / 689 (710 / 749), scale 23 with 10 420 / 422, with 14 613 / 587 (627 / 641), scale 24 with 5 453 / 438 (486 / 491), with 7 626 / 696, 100 M
+// entries in rows of up to 50,000 594 / 612, 110 M of up to 3,000 607 / 574 (621 / 613).)
 constexpr uint64_t FUSED_MAX_ENTRIES = 1ull << 27;
 
 // Whether a build leaves its rows of at most 32 entries to small_rows_kernel, which builds them where they lie,
 // without lists.  Taken alone it is slower than the class kernels of these rows (1.39 against 1.12 ms on the
 // scale-26 graph), but it depends on no list: on a side stream it runs beside the kernels of the long rows (it waits on
 // memory, they on the vector ALU).  A build of all vertices then needs no binning either: the lists of the longer rows
-// are in the graph's plan.  Every build of all vertices that is too large for four launches gains by that (R-MAT
+// are in the graph's plan.  Every build of all vertices that is too large for few launches gains by that (R-MAT
 // lognormal, by class / in place, us: scale 24 with 16 edges a vertex 1613 / 1535, with 56 5172 / 4888, scale 23 with 40
 // 2069 / 1928, scale 22 with 66 1772 / 1668); a list of vertices has to be binned, and takes it from 2^25 rows on.
 static bool small_rows_in_place(const sky_graph* g, const uint32_t* src, uint32_t n) {

@@ -1,4 +1,4 @@
-// Builds in four launches (sky_build_fused.hip): what a graph keeps for them, and the rows of a frontier.
+// Builds in few launches (sky_build_fused.hip): what a graph keeps for them, and the rows of a frontier.
 #pragma once
 #include "sky_graph.h"
 

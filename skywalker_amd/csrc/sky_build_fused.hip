@@ -656,7 +656,7 @@ static_assert(ALL_LONGEST <= 24576, "none is of class CLS_STREAM");
 // scale 16 with 8 25.5 / 26, scale 17 with 4 19.7 / 20.5, scale 18 with 3 25.7 / 28, scale 20 with 16 137 / 171).
 constexpr uint32_t SPLIT_SWEEP = 1u << 15;
 
-// Whole builds of at least so many entries send out the rows of 2558..5117 entries (3582.. beside block_takes_longer) in a launch of
+// Whole builds of at least so many entries that go out beside one another send out the rows of 2558..5117 entries in a launch of
 // their own, beside the others on a third stream, which costs smaller ones more (in the launch of the longer rows / by
 // themselves, us: scale 16 with 16 edges a vertex 43 / 46, scale 20 with 6 82 / 86, 10 M entries in rows of up to 50,000 100 / 103, of
 // up to 7,000 87 / 87, scale 20 with 16 119 / 119, with 30 193 / 187, scale 22 with 16 357 / 348, scale 23 with 10 432 / 421, 40 M entries in rows of
@@ -820,10 +820,12 @@ FusedArgs common_args(sky_graph* g, const BuildPlan& p, int tiled_from) {
   return a;
 }
 
-// Whether the rows of 2558..3581 entries (CLS_MW2 + 4 and + 5) go out with the launch of 256 threads, 14 slots each, rather than beside
-// the streamed rows, whose LDS leaves two workgroups of 512 to a CU (23 M entries in such rows of the scale-22 graph with 32 edges a
-// vertex: 120 us there, 94 here; its build 725 -> 700).  With their LDS a CU holds four workgroups of that launch instead of five,
-// which costs tiles more (16 M entries in tiles 543 -> 570 us).
+// Whether the rows of 2558..3581 entries (CLS_MW2 + 4 and + 5) go out with the launch of 256 threads, 14 slots each, rather than in
+// that of the streamed rows, whose LDS leaves two workgroups of 512 to a CU (in the streamed rows' launch / here, us: scale 22 with 31 edges a vertex
+// 674 / 652, scale 21 with 45 510 / 499, 110 M entries in rows of up to 3,000 617 / 607, 40,000 seeds 25 x 10 on the scale-22 graph with 32 714 / 671).
+// With their LDS a CU holds four workgroups of that launch instead of five, which costs tiles more (16 M entries in tiles 543 -> 570 us),
+// and where they have a launch of their own (MID_ALONE) there is nothing to be had by it (there / here: scale 22 with 10 238 / 245, with 11
+// 263 / 269).
 constexpr double LONGER_ENTRIES = 4e6, LONGER_PER_TILED = 2;
 bool block_takes_longer(const sky_graph* g, int tiled_from) {
   double tiled = 0;
@@ -956,7 +958,7 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   // two classes whose lists lie back to back; min_degree may leave out the first
   auto add_two = [&](Launch& l, Section k, int c) { l.add(k, rows(c) + rows(c + 1), 1, p.start[rows(c) ? c : c + 1]); };
   add_two(mid, SEC_B10, CLS_MW2 + 7);
-  const bool longer = block_takes_longer(g, p.t_all);
+  const bool longer = &mid != &alone && block_takes_longer(g, p.t_all);
   if (longer) {
     mid.add(SEC_B8, rows(CLS_MW2 + 6), 1, p.start[CLS_MW2 + 6]);
   } else {
