@@ -5,12 +5,13 @@
 // the GPU for a millisecond; a build of 17 M entries spent 220 us on 27 launches of 5 to 25 us each, 2.4 us apart on
 // the host and each with a tail of its own, and spreading them over four streams costs 30 us for the fork and the
 // join by events alone.  Here one launch takes all classes whose rows need the same number of threads, and the passes of the
-// rows that are built tile by tile, which depend on one another, ride along in the same four launches:
+// rows that are built tile by tile, which depend on one another, ride along in the same launches:
 //
 //   fused_wave_kernel    64 threads    rows of up to 509 entries         tile sums
 //   fused_pair_kernel    128 threads   rows of 510..1021                 row sums -> ledger, tile totals
 //   fused_wide_kernel    512 threads   rows of 2558 and more             scan over a row's tiles
 //   fused_block_kernel   256 threads   rows of 1022..2557                entries of the tiles
+//   fused_mid_kernel     512 threads   rows of 2558..5117, where a fork (below) gives them a launch of their own
 //
 // A launch whose classes are empty is left out.  A small build with rows for more than the first of them, and none for tiles, goes
 // out in one launch of 512 threads instead (fused_all_kernel).  Every row builder is the one the class kernels call, so the
@@ -878,8 +879,8 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   uint32_t past_wave = 0;  // rows of more than 509 entries: what a second launch would be for
   for (int c = CLS_COUNT - 1; c > CLS_LDS_W2; --c)
     if (class_min_degree(c) >= 510) past_wave += rows(c);
-  // Vertices of a wavefront: enough wavefronts for every SIMD, but 128 to 256 rather than fewer where four wavefronts a SIMD remain: the
-  // rows of a few vertices fill no batch of their class.  The last wavefronts of a sweep beside other launches are what is left of it behind
+  // Vertices of a wavefront: enough wavefronts for every SIMD, but 128 rather than fewer where two wavefronts a SIMD remain, and up to 256 where
+  // four do: the rows of a few vertices fill no batch of their class.  The last wavefronts of a sweep beside other launches are what is left of it behind
   // them: there a 12,288th of the vertices is the limit instead of an 8,192th.  (64 where there were fewer than 4,096 wavefronts of 128, 256 up
   // to 2 M vertices, an 8,192th above / now, us: 3 M entries in 478,000 rows 44 / 36, scale 20 with 6 edges a vertex 83 / 78, scale 22 with 3
   // 115 / 110, scale 23 with 4 232 / 219; scale 22 with 4 127 / 129, with 10 242 / 245; most others within 1 %.  29 M entries in rows of up to
@@ -953,7 +954,7 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
   if (p.t_all > CLS_STREAM_LAST) longs.add(SEC_STREAM, rows(CLS_STREAM_LAST), 1, p.start[CLS_STREAM_LAST]);
   // Rows of 5118..8189 entries: streamed beside the others, where hold_row would spill, or, where they are enough for a launch,
   // HOLD_ALONE, by build_hold_kernel.
-  const bool hold_alone = min_degree == 0 && rows(CLS_HOLD) >= HOLD_ALONE;  // behind the sweep, which notes when the call began
+  const bool hold_alone = min_degree == 0 && rows(CLS_HOLD) >= HOLD_ALONE;  // last on the graph's stream; `first` stamps the call
   if (!hold_alone) longs.add(SEC_STREAM, rows(CLS_HOLD), 1, p.start[CLS_HOLD]);
   // two classes whose lists lie back to back; min_degree may leave out the first
   auto add_two = [&](Launch& l, Section k, int c) { l.add(k, rows(c) + rows(c + 1), 1, p.start[rows(c) ? c : c + 1]); };
