@@ -314,6 +314,7 @@ __device__ __forceinline__ uint32_t wave_lower_bound(const uint32_t* __restrict_
 template <uint32_t WIN>
 struct N2vRow {
   static constexpr int U = 1;
+  static constexpr bool WAVE = false;
   static constexpr int HELD = 16;
   const float* w;
   const uint32_t* nbr;
@@ -508,6 +509,7 @@ constexpr uint32_t MAP_KEEP = 4096;          // slots of a row whose weights are
 constexpr uint32_t MAP_FEW = 768;
 struct N2vMapRow {
   static constexpr int U = 2;
+  static constexpr bool WAVE = true;
   static constexpr int HELD = 16;
   const float* w;
   const uint32_t* nbr;
@@ -560,6 +562,13 @@ struct N2vMapRow {
       }
       if (!again && d <= keep && at < end) reinterpret_cast<float4*>(kept)[at >> 2] = make_float4(x[j][0], x[j][1], x[j][2], x[j][3]);
     }
+  }
+  __device__ __forceinline__ void load(uint32_t k, float (&x)[4]) const {
+    const uint32_t at = min(k, (d - 1) & ~3u);
+    const float4u a = *reinterpret_cast<const float4u*>(w + at);
+    const uint4u b = *reinterpret_cast<const uint4u*>(nbr + at);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[t] = weigh(a[t], k + t < d ? b[t] : 0u, k + t < d);
   }
   __device__ __forceinline__ void again(uint32_t k, float (&x)[4]) const {
     x[0] = x[1] = x[2] = x[3] = 0.0f;

@@ -264,7 +264,10 @@ __device__ __forceinline__ uint32_t draw_entry(Row& row, const uint32_t d, const
 // the thread of col the key, and the thread whose prefixes it falls between the slot.  Three barriers and some 3,000 cycles, where the
 // sweep over chunks and the chain on one wavefront behind it take 9,000 (counted in the table-per-step walk, rows of 800 entries on
 // average).  The amounts of four quads held in registers would make them 147, three wavefronts to a SIMD: they are computed again.
-template <bool SAT, int Q, int T, class Row>
+// Not for rows whose surpluses may wrap (a second form that saturates cost a walker of one wavefront 9 registers, which is the sixth wavefront to
+// a SIMD: 20,000 walkers x 4 without tables, scale 16, 78.5 -> 76.2 us).
+constexpr uint32_t HELD_MOST = 4095;
+template <int Q, int T, class Row>
 __device__ __forceinline__ uint32_t draw_held(Row& row, const uint32_t d, const Ledger& L, const uint32_t col, const Entry& ec,
                                               const float u, DrawLds<T>& lds) {
   constexpr int NW = T / 64, S = 4 * Q;
@@ -297,10 +300,10 @@ __device__ __forceinline__ uint32_t draw_held(Row& row, const uint32_t d, const 
   each(false, [&](int k, bool h, uint64_t x) {
     heavy |= (h ? 1u : 0u) << k;
     sd += h ? 0 : x;
-    su = add_sat<SAT>(su, h ? x : 0);
+    su += h ? x : 0;
   });
-  const uint64_t id = group_scan_u64<64>(sd), iu = group_scan_sat_u64<64, SAT>(su);
-  uint64_t bd = id - sd, bu = before_own<SAT>(iu, su);  // before the thread's slots
+  const uint64_t id = group_scan_u64<64>(sd), iu = group_scan_u64<64>(su);
+  uint64_t bd = id - sd, bu = iu - su;  // before the thread's slots
   uint64_t tu = 0;                                      // surpluses of the row
   if (lane == 63) {
     lds.d[wave] = id;
@@ -310,16 +313,16 @@ __device__ __forceinline__ uint32_t draw_held(Row& row, const uint32_t d, const 
 #pragma unroll
   for (int i = 0; i < NW; ++i) {
     const uint64_t x = lds.d[i], y = lds.u[i];
-    tu = add_sat<SAT>(tu, y);
+    tu += y;
     if (i < (int)wave) {
       bd += x;
-      bu = add_sat<SAT>(bu, y);
+      bu += y;
     }
   }
   if (tid == owner) {  // deficits before a light col, surpluses up to and with a heavy col
     uint64_t key = ec.heavy ? bu : bd;
     each(true, [&](int k, bool h, uint64_t x) {
-      key = add_sat<SAT>(key, ec.heavy ? (h && k <= (int)own ? x : 0) : (!h && k < (int)own ? x : 0));
+      key += ec.heavy ? (h && k <= (int)own ? x : 0) : (!h && k < (int)own ? x : 0);
     });
     lds.key = key;
     lds.result = col;
@@ -337,10 +340,10 @@ __device__ __forceinline__ uint32_t draw_held(Row& row, const uint32_t d, const 
   if (!ec.heavy) {
     // first heavy whose surplus prefix exceeds the key; the last heavy if there is none; col itself without any heavy
     if (key < tu) {
-      if (bu <= key && key < add_sat<SAT>(bu, su)) {
+      if (bu <= key && key < bu + su) {
         uint32_t at = S;
         each(true, [&](int k, bool h, uint64_t x) {
-          if (h) bu = add_sat<SAT>(bu, x);
+          if (h) bu += x;
           at = at == S && bu > key ? k : at;
         });
         lds.result = min(k0 + at, d - 1);  // a bias operator may answer differently each time
@@ -447,13 +450,124 @@ __device__ __forceinline__ bool row_ledger(Row& row, const uint32_t d, const uin
   return true;
 }
 
+// The draw from a row of at most WAVE_MOST entries by one wavefront, four consecutive slots a lane: no barrier, no LDS, no sweep twice.  The
+// other wavefronts of the workgroup wait for it and leave the SIMDs to the walkers beside.  In the table-per-step walk a step from a row of 256
+// entries and fewer, half of all, takes 8,300 cycles instead of 11,000 (2,000 x 40 on the scale-18 graph 549 -> 518 us, on the scale-17 graph 449
+// -> 410, 200 x 40 there 254 -> 217).  With eight slots a lane a row of 300 takes as long as by the workgroup, with sixteen a row of 950 takes
+// longer (518 / 520 / 803 us).
+// All lanes call it together.
+constexpr uint32_t WAVE_MOST = 256;
+__device__ __forceinline__ uint64_t lane_u64(uint64_t v, int lane) {
+  return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane) << 32 |
+         (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+}
+template <class Row>
+__device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const uint32_t rx, const float u) {
+  const uint32_t lane = threadIdx.x & 63, k0 = 4 * lane;
+  float w[4];
+  row.load(k0, w);
+  double fsum = 0.0;
+  uint32_t most = 0;  // the complement of the least (weight bits - 1): what lanes without a source add to a scan, 0, changes nothing
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    fsum += (double)w[k];
+    most = max(most, 0u - __float_as_uint(w[k]));
+  }
+  auto scan = [&](auto step) {
+    step(std::integral_constant<int, DPP_ROW_SHR1>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, DPP_ROW_SHR2>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, DPP_ROW_SHR4>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, DPP_ROW_SHR8>{}, std::integral_constant<int, 0xF>{});
+    step(std::integral_constant<int, DPP_ROW_BCAST15>{}, std::integral_constant<int, 0xA>{});
+    step(std::integral_constant<int, DPP_ROW_BCAST31>{}, std::integral_constant<int, 0xC>{});
+  };
+  scan([&](auto ctrl, auto rows) {
+    constexpr int C = decltype(ctrl)::value, R = decltype(rows)::value;
+    fsum += __longlong_as_double((long long)dpp0_u64<C, R>((uint64_t)__double_as_longlong(fsum)));
+    most = max(most, dpp0<C, R>(most));
+  });
+  fsum = __longlong_as_double((long long)lane_u64((uint64_t)__double_as_longlong(fsum), 63));
+  most = (uint32_t)__builtin_amdgcn_readlane((int)most, 63);
+  Ledger L;
+  if (plain_sum_is_exact(fsum, ~most)) {
+    if (fsum == 0.0) return NONE_SLOT;
+    L = make_ledger_small(d, fsum);
+  } else {
+    u128 sum{0, 0};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) sum = add128(sum, weight_fixed(w[k]));
+    sum = group_sum_u128<64>(sum);
+    if ((sum.lo | sum.hi) == 0) return NONE_SLOT;
+    L = make_ledger(d, sum);
+  }
+  const uint32_t col = __umulhi(rx, d), j = col & 3u;
+  const float wc = j == 0 ? w[0] : j == 1 ? w[1] : j == 2 ? w[2] : w[3];
+  const Entry ec = classify_fast((double)__uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(wc), (int)(col >> 2))), true, L);
+  const bool heavy = __builtin_amdgcn_readfirstlane(ec.heavy ? 1 : 0);
+  if (!heavy && u < (float)ec.p) return col;  // the light keeps the draw: its alias is never read
+  uint64_t a[4];
+  uint32_t h = 0;  // bit k: slot k0 + k is heavy
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const Entry e = classify_fast((double)w[k], k0 + k < d, L);
+    a[k] = e.amount;
+    h |= (e.heavy ? 1u : 0u) << k;
+  }
+  // deficits before a light col, surpluses up to and with a heavy col
+  uint64_t key = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) key += ((h >> k) & 1) == (heavy ? 1u : 0u) && (heavy ? k0 + k <= col : k0 + k < col) ? a[k] : 0;
+  key = lane_u64(group_scan_u64<64>(key), 63);
+  // first slot of a kind whose inclusive prefix exceeds `past`, and that prefix; NONE_SLOT if there is none
+  uint64_t at = 0;
+  auto above = [&](uint32_t kind, uint64_t past) -> uint32_t {
+    uint64_t run[4], t = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      t += ((h >> k) & 1) == kind ? a[k] : 0;
+      run[k] = t;
+    }
+    const uint64_t inc = group_scan_u64<64>(t), before = inc - t;
+    const unsigned long long m = __ballot(inc > past);
+    if (!m) return NONE_SLOT;
+    const int l = __ffsll((long long)m) - 1;
+    uint32_t k = 3;
+    uint64_t x = inc;
+#pragma unroll
+    for (int i = 2; i >= 0; --i)
+      if (before + run[i] > past) {
+        k = i;
+        x = before + run[i];
+      }
+    at = lane_u64(x, l);
+    return 4u * l + (uint32_t)__builtin_amdgcn_readlane((int)k, l);
+  };
+  if (!heavy) {
+    // first heavy whose surplus prefix exceeds the key; the last heavy if there is none; col itself without any heavy
+    const uint32_t s = above(1, key);
+    if (s != NONE_SLOT) return s;
+    const unsigned long long m = __ballot(h != 0);
+    if (!m) return col;
+    const int l = 63 - __clzll((long long)m);
+    return 4u * l + 31u - (uint32_t)__clz(__builtin_amdgcn_readlane((int)h, l));
+  }
+  // next heavy after col (none: col is the last heavy and keeps the draw), then the first light l with SL(l) >= key:
+  // prob = (one + key - SL(l)) / one
+  const uint32_t after = k0 > col ? h : k0 + 3 <= col ? 0u : h & ~((2u << j) - 1u);
+  const unsigned long long m = __ballot(after != 0);
+  if (!m || above(0, key - 1) == NONE_SLOT) return col;
+  const int l = __ffsll((long long)m) - 1;
+  return u < residual_prob(L.one + key - at, L) ? col : 4u * l + (uint32_t)__ffs(__builtin_amdgcn_readlane((int)after, l)) - 1u;
+}
+
 // Row-local slot that (walker, step) with random numbers r draws from the row of d >= 1 entries, or NONE_SLOT when
 // their weights sum to zero.  Called by every thread of a workgroup of T.  `row`:
 //   row.first(k, w)   clamped weights of slots k .. k + 3 (k a multiple of 4; zeros past the row).  A wavefront goes
 //                     through its part of the row in slot order, once, all lanes together (k advances by 4 per lane)
 //   row.again(k, w)   the same, afterwards, for any slots and by any wavefront
 //   Row::U            how many times 256 slots are in flight at once; if that is more than one, instead of first():
-//   Row::HELD         0, 4 or 16: rows of up to so many slots a thread by draw_held
+//   Row::WAVE         rows of up to WAVE_MOST entries by draw_wave, from row.load(k, w): the same before any other
+//   Row::HELD         0, 4 or 16: rows of up to so many slots a thread (4,095 at most) by draw_held
 //   row.many(k, end, again, w)  slots k + 256 j .. k + 256 j + 3 for j < U, zeros from slot `end` on, in both sweeps
 template <int T, class Row>
 __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const u32x4& r, DrawLds<T>& lds) {
@@ -464,6 +578,17 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
   const uint32_t nc = (uint32_t)(((uint64_t)d + csz - 1) / csz), cpw = (nc + NW - 1) / NW;
   const uint32_t c0 = wave * cpw, c1 = min(nc, c0 + cpw);
   __syncthreads();  // the draw before has been read by everyone
+  if constexpr (Row::WAVE) {
+    if (d <= WAVE_MOST) {
+      static_assert(NW > 1, "a wavefront alone goes on as it is");
+      if (wave == (blockIdx.x & (NW - 1))) {  // not always on the same SIMD
+        const uint32_t cand = draw_wave(row, d, r.x, u24(r.y));
+        if ((threadIdx.x & 63) == 0) lds.result = cand;
+      }
+      __syncthreads();
+      return lds.result;
+    }
+  }
   const uint32_t k0 = c0 < nc ? c0 * csz : d, k1 = c0 < nc ? (c1 == nc ? d : c1 * csz) : d;  // this wavefront's slots
 
   Ledger L;
@@ -483,19 +608,19 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
     return surpluses_may_wrap(L.scale) ? draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds)
                                        : draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
   }
-  if (surpluses_may_wrap(L.scale)) {
-    if (d <= 4 * T) return draw_held<true, 1, T>(row, d, L, col, ec, u, lds);
-    if constexpr (Row::HELD == 16) if (d <= 16 * T) return draw_held<true, 4, T>(row, d, L, col, ec, u, lds);
-    return draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
+  if (d <= std::min(4u * T, HELD_MOST)) return draw_held<1, T>(row, d, L, col, ec, u, lds);
+  if constexpr (Row::HELD == 16) {
+    constexpr uint32_t Q = T >= 512 ? 2 : 4;
+    if (d <= std::min(4 * Q * T, HELD_MOST)) return draw_held<Q, T>(row, d, L, col, ec, u, lds);
   }
-  if (d <= 4 * T) return draw_held<false, 1, T>(row, d, L, col, ec, u, lds);
-  if constexpr (Row::HELD == 16) if (d <= 16 * T) return draw_held<false, 4, T>(row, d, L, col, ec, u, lds);
+  if (surpluses_may_wrap(L.scale)) return draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
   return draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
 }
 
 // The graph's own weights of a row (the weight array has 16 spare bytes, so four slots can be read from any).
 struct PlainRow {
   static constexpr int U = 4;
+  static constexpr bool WAVE = false;  // most of its walkers are a wavefront anyway (with it 10,000 x 8, scale 22, 187 -> 194 us)
   static constexpr int HELD = 4;
   const float* w;
   uint32_t d;
@@ -526,6 +651,7 @@ constexpr uint32_t FN_CACHE = 4096;
 template <class Fn>
 struct FunctionRow {
   static constexpr int U = 1;
+  static constexpr bool WAVE = false;
   static constexpr int HELD = 0;  // the operator is called where it is linked in: node2vec's, 8,000 walkers x 20, scale 16, 5.5 ms, 6.0 with
   Fn fn;
   uint32_t d;

@@ -528,6 +528,31 @@ def test_node2vec_table_with_a_bit_per_vertex(orc, V, walkers, p, q):
     assert sampled == want[2]
 
 
+@pytest.mark.parametrize("kind", ["uniform", "equal", "sparse", "tiny"])
+@pytest.mark.parametrize("walkers", [300, 1000])
+def test_node2vec_table_rows_of_one_wavefront(orc, walkers, kind):
+    # rows around the 256 entries that one wavefront draws from by itself, and around the 4,095 whose surpluses fit 64 bits whatever the
+    # weights; weights that sum up exactly in doubles or not, none lighter than the others, most of no weight, all next to none
+    from skywalker_amd import capi
+    rng = np.random.default_rng(53)
+    degs = list(range(1, 9)) * 4 + [63, 64, 65, 127, 128, 129] * 6 + list(range(250, 262)) * 12 + [4094, 4095, 4096, 4097] * 3
+    rng.shuffle(degs)
+    n = len(degs)
+    xadj = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    adjncy = np.concatenate([np.sort(rng.integers(0, n, k)) for k in degs]).astype(np.uint32)
+    w = weights(len(adjncy), rng, {"tiny": "sparse"}.get(kind, kind))
+    if kind == "tiny":
+        w *= np.float32(1e-19)
+    seeds = rng.integers(0, n, walkers).astype(np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    paths, lengths, sampled, _ = g.walk_online(capi.BIAS_NODE2VEC, 2.0, 0.5, seeds, 10, 0.0, 41)
+    got = paths.to_host((walkers, 11)), lengths.to_host()
+    g.free()
+    want = orc.walk_online(xadj, adjncy, w, 1, 2.0, 0.5, seeds, 10, 0.0, 41)
+    assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
+    assert sampled == want[2]
+
+
 @pytest.mark.parametrize("longest,walkers", [(70001, 256), (70001, 257), (70001, 8193), (40001, 512), (40001, 513), (40001, 16385),
                                              (12289, 1024), (12289, 1025), (12289, 8193)])
 def test_online_static_draws_by_workgroups_of_every_size(longest, walkers):
