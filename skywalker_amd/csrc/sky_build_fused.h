@@ -56,7 +56,7 @@ bool fused_possible(const sky_graph* g);
 // The graph's plan, made if there is none or a knob has changed.  *first as in bin_all_rows: making the plan is part of the
 // call that needs it, and of its time.
 int ensure_plan(sky_graph* g, CallDevice** first);
-// All rows; needs the plan and vertices.
+// All rows; needs the plan and vertices, and the end of the call behind it.
 int build_all_fused(sky_graph* g, CallDevice* call);
 // The rows of at least min_degree entries alone (a class boundary of 33 or more); needs the plan.  `call` is stamped (null: another kernel was).
 int build_rows_from(sky_graph* g, uint32_t min_degree, CallDevice* call);

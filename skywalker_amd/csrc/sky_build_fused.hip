@@ -1008,6 +1008,7 @@ static int build_host_sized(sky_graph* g, uint32_t min_degree, CallDevice* call)
     for (Launch* l : {&wave, &pair, &scan, &block})
       if (l != first) SKY_TRY(enqueue<false>(p, *l, longer, g->stream));
     if (hold_alone) SKY_TRY(build_rows_hold(g, p.rows + p.start[CLS_HOLD], rows(CLS_HOLD)));
+    if (min_degree == 0) side.last = &g->call;  // build_all_fused: nothing but the call's end follows
     return beside_join(&side);
   };
   const int rc = others();

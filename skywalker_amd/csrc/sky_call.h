@@ -46,6 +46,7 @@ struct CallWords {
   unsigned long long seq = 0, asked = 0;  // numbers of the last end and of the last question
   uint32_t forks = 0;                     // and of the last fork
   int khz = 0;
+  uint32_t awaited = 0;  // side streams that the end kernel waits for
   uint32_t parts = 0;  // words that the call's kernels add sampled edges to: none, one or CALL_PARTS
   bool dirty = false;  // a call has begun and not ended well: its device words may not be zero
 };
@@ -87,7 +88,7 @@ int call_answered(sky_graph* g, CallWords* w, unsigned long long* values, int n)
 // Kernels beside those of the graph's stream, on streams that all graphs of a device share (sky_sides.h).  These and the graph's stream wait for one
 // another by words in pinned memory: a kernel on the graph's stream notes that it runs (fork_mark), so that everything in front of it has
 // ended, and of small last ones on the others the one that finds all of them there that everything in front of these has.  Who waits, by a stream operation (one
-// thread of the runtime's that reads the word until the number is there), is always enqueued behind the kernel that writes.  The runtime
+// thread of the runtime's that reads the word until the number is there) or in the call's end kernel (beside_join), is always enqueued behind the kernel that writes.  The runtime
 // gives a hardware queue what is enqueued in the order of the calls, so that every wait ends: also where other threads' calls lie
 // between, where streams share a hardware queue, and where there is only one.  Who waits for the whole device after a call, which does
 // not need it, waits 8 to 10 us longer for every side stream that has had work.  2 us
@@ -100,6 +101,7 @@ struct Beside {
   CallDevice* dev = nullptr;
   CallHost* host = nullptr;
   uint32_t number = 0;
+  CallWords* last = nullptr;  // of the call that ends with the join: its end kernel waits, not the graph's stream
 };
 struct ForkMark {
   uint32_t* word;  // null: none
@@ -114,7 +116,10 @@ __device__ __forceinline__ void fork_mark(const ForkMark& f) {
 int beside_begin(sky_graph* g, Beside* b, ForkMark* mark, int streams);
 // With that kernel on its way: side stream k waits for its mark, if it does not already.
 int beside_fork(Beside* b, int k);
-// The graph's stream waits for what the side streams of the fork hold.
+// The graph's stream waits for what the side streams of the fork hold, or, where nothing but the call's end follows, the end kernel does: it is
+// there anyway, and a stream's wait takes 4.5 us and 3 more until the next kernel runs.  (A stream's wait / the end kernel's, us: scale 16 with 16
+// edges a vertex 45 / 42.5, scale 18 with 10 60 / 56.5, scale 20 with 6 78.4 / 73.5, with 16 120 / 118.3, 3 M entries in rows of up to 20,000
+// 57.4 / 55.1, 40 M of up to 300,007 312 / 309.5, scale 23 with 8 373 / 369.)
 int beside_join(Beside* b);
 // Instead of a join, after an error: the host waits for them.
 void beside_drop(Beside* b);

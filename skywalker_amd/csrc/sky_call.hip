@@ -40,6 +40,20 @@ __global__ __launch_bounds__(1024) void call_end_kernel(CallDevice* call, CallHo
 }
 static_assert(CALL_PARTS == 64, "by the first wavefront");
 
+// The end of a call that has work on `awaited` side streams, and samples no edges.  The last kernels of these were enqueued before this one, so
+// that they run to their end whichever queue each is in.  If they do not, the host finds that out: nothing is reported to it.
+__global__ __launch_bounds__(64) void call_end_beside_kernel(CallDevice* call, CallHost* host, unsigned long long seq, uint32_t awaited,
+                                                             unsigned long long patience) {
+  if (threadIdx.x) return;
+  const unsigned long long start = call->start, since = wall_clock64();
+  while (__hip_atomic_load(&call->joined, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != awaited) {
+    if (wall_clock64() - since > patience) return;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  call->joined = 0;
+  call_report(call, host, seq, start, 0);
+}
+
 __global__ __launch_bounds__(256) void sum_counts_kernel(const uint32_t* __restrict__ x, uint64_t n, CallDevice* call) {
   __shared__ unsigned long long s_w[4];
   unsigned long long t = 0;
@@ -132,6 +146,7 @@ void call_release(CallWords* w) {
 int call_begin(sky_graph* g, CallWords* w, CallDevice** call) {
   if (!w->host) SKY_TRY(take_words(g->device, w));
   if (w->dirty) SKY_HIP(hipMemsetAsync(w->dev, 0, sizeof(CallDevice), g->stream));
+  w->awaited = 0;
   w->dirty = true;  // until it has ended well
   ++g->calls;
   *call = w->dev;
@@ -162,7 +177,8 @@ struct SideRuntime {
 SidePool<SideRuntime> g_side[SIDE_DEVICES];
 }  // namespace
 
-// The last kernel of each of the n side streams of a fork.  (A word for each, and a wait for each on the graph's stream: 4.5 us apiece.)
+// The last kernel of each of the n side streams of a fork (n = 0: the call's end kernel counts them).  (A word for each, and a wait for each on
+// the graph's stream: 4.5 us apiece.)
 __global__ void beside_done_kernel(CallDevice* dev, CallHost* host, uint32_t n, uint32_t number) {
   if (__hip_atomic_fetch_add(&dev->joined, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u != n) return;
   __hip_atomic_store(&dev->joined, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -199,9 +215,10 @@ int beside_join(Beside* b) {
   for (bool u : b->used) n += u;
   if (!n) return SKY_OK;
   for (int k = 0; k < SIDE_STREAMS; ++k)
-    if (b->used[k]) hipLaunchKernelGGL(beside_done_kernel, dim3(1), dim3(1), 0, b->stream[k], b->dev, b->host, n, b->number);
+    if (b->used[k]) hipLaunchKernelGGL(beside_done_kernel, dim3(1), dim3(1), 0, b->stream[k], b->dev, b->host, b->last ? 0u : n, b->number);
   SKY_HIP(hipGetLastError());
-  SKY_HIP(hipStreamWaitValue32(b->main, &b->host->done, b->number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+  if (b->last) b->last->awaited = n;
+  else SKY_HIP(hipStreamWaitValue32(b->main, &b->host->done, b->number, hipStreamWaitValueEq, 0xFFFFFFFFu));
   for (bool& u : b->used) u = false;
   return SKY_OK;
 }
@@ -229,6 +246,8 @@ constexpr uint64_t END_COUNTS = 32768;
 // The host polls this long before it hands the wait to the runtime: a call that takes longer does not notice the
 // five microseconds, and one whose kernels fault ends with the runtime's error instead of polling for ever.
 constexpr auto POLL_FOR = std::chrono::microseconds(3000);
+
+constexpr unsigned long long END_PATIENCE = 60;  // seconds that an end kernel waits for side streams; a build takes 0.02
 
 // Waits until n host words from `from` on carry the number `seq`, and takes their values.
 static int take_values(hipStream_t st, const unsigned long long* from, int n, unsigned long long seq, unsigned long long* values) {
@@ -272,10 +291,16 @@ int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, con
     w->parts = CALL_PARTS;
   }
   const unsigned long long seq = ++w->seq;
-  hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, st, w->dev, w->host, seq, counts,
-                     (uint32_t)n, w->parts);
-  w->parts = 0;
-  SKY_HIP(hipGetLastError());
+  if (w->awaited)
+    hipLaunchKernelGGL(call_end_beside_kernel, dim3(1), dim3(64), 0, st, w->dev, w->host, seq, w->awaited,
+                       (unsigned long long)w->khz * 1000 * END_PATIENCE);
+  else
+    hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, st, w->dev, w->host, seq, counts, (uint32_t)n, w->parts);
+  const bool awaited = w->awaited != 0;
+  w->parts = w->awaited = 0;
+  const hipError_t launched = hipGetLastError();
+  if (launched != hipSuccess && awaited) (void)hipDeviceSynchronize();  // the next call clears the words that the side streams write
+  SKY_HIP(launched);
   static_assert(offsetof(CallHost, ticks) == offsetof(CallHost, sampled) + 8, "taken together");
   unsigned long long words[2];
   SKY_TRY(take_values(st, &w->host->sampled, 2, seq, words));
