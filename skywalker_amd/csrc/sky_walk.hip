@@ -492,9 +492,16 @@ int walk_offline_noalloc(sky_graph* g, const uint32_t* seeds, uint32_t N, uint32
 // instructions than everything else in a trial, are computed for several trials of several steps at once, one lane each, and
 // all search the previous row together, G probes per round.  Most trials need no search at all: whether the candidate is
 // kept depends on its being a neighbour of the previous vertex only when the drawn number lies between the two cases'
-// limits.  The bounds of the candidate's own row are requested before the search, for the step after.  Leaving the first
-// probe until it is known to be needed, or reading the next step's entry during the search as if the candidate were
-// kept, was slower.
+// limits.  The bounds of the candidate's own row are requested before the search, for the step after.  The first probe, a line of memory for
+// every lane where the previous row is long, goes out with the table's entry, but only for a drawn number between the limits: lines are what
+// bounds large graphs (40,000 x 80 on the scale-24 graph read 10.6 M of them, 32 G a second of the 50 that random reads reach; us, for every step /
+// for such numbers: 40,000 x 80 345 / 325, 1,000 x 80 with q = 1/2 there 143 / 117, 50,000 x 40, scale 20, 175 / 168, 8,000 x 30, scale 22,
+// p = q = 2, 138 / 130, 150,000 x 30, scale 22, 286 / 275, 10,000 x 50, scale 21, p = 1/2, q = 1, 152 / 137; in turns of four trials one of which
+// nearly always asks 273 / 297, so there it stays with the move; behind the entry's load instead of in front of it 324 / 368: what waits for the
+// entry then waits for a probe too).  Leaving it until it is known to be needed or reading the next step's entry during the search as if the
+// candidate were kept was slower, and doing the whole search beside the next step's loads and taking a refused step back gains on the largest
+// graphs what it costs elsewhere several times (40,000 x 80 on the scale-24 graph 324 / 312, but 50,000 x 40, scale 20, 167 / 187, 500 x 60, scale 14,
+// 68 / 99, 8,000 x 30, scale 22, q = 2, 129 / 231).
 //
 // A turn of the loop is TR trials of every walker of the wavefront, whichever step each of them is in: where a turn was a step,
 // every walker waited in each for the one with the most trials.
@@ -592,6 +599,9 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
         const int from = base + (int)lane_of(s, t);
         if (t == 0 && ((stop_prob > 0.0f && u24(of(mine.z, from)) < stop_prob) || deg == 0)) break;
         const uint32_t rx = of(mine.x, from + (int)my), ry = of(mine.y, from + (int)my), rw = of(mine.w, from + (int)my);
+        const float need = u24(rw) * fmax;
+        // The previous row can only be asked about a candidate drawn with such a number: its first probe is on its way then, beside the entry.
+        if (TR == 1) x0 = group_first_probe<G>(adjncy + prev_off, need >= lo && need < hi ? prev_deg : 0u);  // no row before the first step
         const uint32_t col = __umulhi(rx, deg);
         const AliasEntry e = once ? load_entry_once(table + off + col) : table[off + col];
         // The numbers of what may come next, while the entry is on its way: all walkers of the wavefront together.
@@ -609,7 +619,6 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
         uint32_t next = adjncy[off + (TR > 1 && ends ? col : cand)];
         x = *reinterpret_cast<const bounds2u*>(xadj + next);
         bool keep = s == 0 || t + my >= 65536u, ask = false;
-        const float need = u24(rw) * fmax;
         if (!keep) {
           if (next == prev) keep = need < fp;
           else if (need < lo) keep = true;
@@ -652,7 +661,7 @@ __global__ __launch_bounds__(WALK_BLOCK) void walk_n2v_reject_group_kernel(
           prev = v;
           prev_off = off;
           prev_deg = deg;
-          x0 = group_first_probe<G>(adjncy + off, deg);  // in flight during the loads of the step
+          if (TR > 1 && lo < hi) x0 = group_first_probe<G>(adjncy + off, deg);  // some trial of four asks; in flight during the loads of the step
           v = next;
           off = x.x;
           deg = x.y - x.x;
