@@ -23,8 +23,14 @@ int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, 
 // ---------------------------------------------------------------- static bias
 // A walker per workgroup of T threads, for the whole walk.  Rows of table_from entries and more have tables; from the
 // others the draw is evaluated directly.
+// A step is a chain: bounds, weights, draw, neighbour.  Most rows met are short (half of all cycles went to rows below 64 entries, 9,000 to 12,000
+// a draw by the forms for long rows), so up to 64 entries have a slot a lane (draw_wave) and their neighbours loaded beside the weights,
+// and up to 256 four slots a lane: 20,000 walkers x 4 on the scale-16 graph 79.1 -> 68.7 us, 9,000 x 10 on the scale-20 graph 124 -> 112.5,
+// 10,000 x 8 on the scale-22 graph 187.9 -> 183.7, most of it the build of the long rows.
+// Six wavefronts to a SIMD, 80 registers, is what 64 and 128 threads come to without spills (5,000 x 10 on the scale-18 graph by 128 threads
+// 92.5 us before, 83.3 with the short rows apart, 78.7 with 80 registers for 87); 256 threads would spill and gain nothing.
 template <int T>
-__global__ __launch_bounds__(T) void walk_direct_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
+__global__ __launch_bounds__(T, T <= 128 ? 6 : 1) void walk_direct_kernel(const uint32_t* __restrict__ xadj, const uint32_t* __restrict__ adjncy,
                                                         const float* __restrict__ wgt, const AliasEntry* __restrict__ table,
                                                         uint32_t table_from, const uint32_t* __restrict__ seeds, uint32_t first,
                                                         uint32_t V, uint32_t len, float stop_prob, uint64_t seed,
@@ -49,6 +55,14 @@ __global__ __launch_bounds__(T) void walk_direct_kernel(const uint32_t* __restri
       const AliasEntry e = table[off + col];
       cand = u24(r.y) < e.prob ? col : e.alias;
       static_assert(NONE_SLOT == SKY_INVALID, "a row without weight ends the walk either way");
+    } else if (d <= 64) {
+      const uint32_t next = adjncy[off + min(threadIdx.x & 63, d - 1)];
+      PlainRow row{wgt + off, d};
+      cand = draw_wave<1>(row, d, r.x, u24(r.y));
+      if (cand == NONE_SLOT) break;
+      v = (uint32_t)__builtin_amdgcn_readlane((int)next, (int)cand);
+      if (threadIdx.x == 0) path[s + 1] = v;
+      continue;
     } else {
       PlainRow row{wgt + off, d};
       cand = draw_slot<T>(row, d, r, lds);
@@ -314,7 +328,7 @@ __device__ __forceinline__ uint32_t wave_lower_bound(const uint32_t* __restrict_
 template <uint32_t WIN>
 struct N2vRow {
   static constexpr int U = 1;
-  static constexpr bool WAVE = false;
+  static constexpr WaveRows WAVE = WAVE_NONE;
   static constexpr int HELD = 16;
   const float* w;
   const uint32_t* nbr;
@@ -509,7 +523,7 @@ constexpr uint32_t MAP_KEEP = 4096;          // slots of a row whose weights are
 constexpr uint32_t MAP_FEW = 768;
 struct N2vMapRow {
   static constexpr int U = 2;
-  static constexpr bool WAVE = true;
+  static constexpr WaveRows WAVE = WAVE_ONE;
   static constexpr int HELD = 16;
   const float* w;
   const uint32_t* nbr;

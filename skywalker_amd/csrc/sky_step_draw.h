@@ -450,26 +450,29 @@ __device__ __forceinline__ bool row_ledger(Row& row, const uint32_t d, const uin
   return true;
 }
 
-// The draw from a row of at most WAVE_MOST entries by one wavefront, four consecutive slots a lane: no barrier, no LDS, no sweep twice.  The
-// other wavefronts of the workgroup wait for it and leave the SIMDs to the walkers beside.  In the table-per-step walk a step from a row of 256
-// entries and fewer, half of all, takes 8,300 cycles instead of 11,000 (2,000 x 40 on the scale-18 graph 549 -> 518 us, on the scale-17 graph 449
-// -> 410, 200 x 40 there 254 -> 217).  With eight slots a lane a row of 300 takes as long as by the workgroup, with sixteen a row of 950 takes
-// longer (518 / 520 / 803 us).
+// The draw from a row of at most 64 S entries by one wavefront, S consecutive slots a lane: no barrier, no LDS, no sweep twice.  S is 4 for rows
+// of up to WAVE_MOST entries, and 1 for those of up to 64 where the caller takes the trouble.
+// In the table-per-step walk one wavefront of the workgroup draws for all (WAVE_ONE: its weights come from windows in LDS); the others wait for it
+// and leave the SIMDs to the walkers beside.  A step from a row of 256 entries and fewer, half of all, takes 8,300 cycles instead of 11,000 (2,000 x
+// 40 on the scale-18 graph 549 -> 518 us, on the scale-17 graph 449 -> 410, 200 x 40 there 254 -> 217).  With eight slots a lane a row of 300
+// takes as long as by the workgroup, with sixteen a row of 950 takes longer (518 / 520 / 803 us).
+// In the walk without tables every wavefront of the workgroup draws for itself, all the same slot, and no barrier is met (WAVE_EACH).
 // All lanes call it together.
 constexpr uint32_t WAVE_MOST = 256;
+enum WaveRows { WAVE_NONE, WAVE_ONE, WAVE_EACH };
 __device__ __forceinline__ uint64_t lane_u64(uint64_t v, int lane) {
   return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane) << 32 |
          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
 }
-template <class Row>
+template <int S = 4, class Row>
 __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const uint32_t rx, const float u) {
-  const uint32_t lane = threadIdx.x & 63, k0 = 4 * lane;
-  float w[4];
+  const uint32_t lane = threadIdx.x & 63, k0 = S * lane;
+  float w[S];
   row.load(k0, w);
   double fsum = 0.0;
   uint32_t most = 0;  // the complement of the least (weight bits - 1): what lanes without a source add to a scan, 0, changes nothing
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < S; ++k) {
     fsum += (double)w[k];
     most = max(most, 0u - __float_as_uint(w[k]));
   }
@@ -495,20 +498,22 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
   } else {
     u128 sum{0, 0};
 #pragma unroll
-    for (int k = 0; k < 4; ++k) sum = add128(sum, weight_fixed(w[k]));
+    for (int k = 0; k < S; ++k) sum = add128(sum, weight_fixed(w[k]));
     sum = group_sum_u128<64>(sum);
     if ((sum.lo | sum.hi) == 0) return NONE_SLOT;
     L = make_ledger(d, sum);
   }
-  const uint32_t col = __umulhi(rx, d), j = col & 3u;
-  const float wc = j == 0 ? w[0] : j == 1 ? w[1] : j == 2 ? w[2] : w[3];
-  const Entry ec = classify_fast((double)__uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(wc), (int)(col >> 2))), true, L);
+  const uint32_t col = __umulhi(rx, d), j = col % S;
+  float wc = w[0];
+#pragma unroll
+  for (int k = 1; k < S; ++k) wc = j == (uint32_t)k ? w[k] : wc;
+  const Entry ec = classify_fast((double)__uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(wc), (int)(col / S))), true, L);
   const bool heavy = __builtin_amdgcn_readfirstlane(ec.heavy ? 1 : 0);
   if (!heavy && u < (float)ec.p) return col;  // the light keeps the draw: its alias is never read
-  uint64_t a[4];
+  uint64_t a[S];
   uint32_t h = 0;  // bit k: slot k0 + k is heavy
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
+  for (int k = 0; k < S; ++k) {
     const Entry e = classify_fast((double)w[k], k0 + k < d, L);
     a[k] = e.amount;
     h |= (e.heavy ? 1u : 0u) << k;
@@ -516,14 +521,14 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
   // deficits before a light col, surpluses up to and with a heavy col
   uint64_t key = 0;
 #pragma unroll
-  for (int k = 0; k < 4; ++k) key += ((h >> k) & 1) == (heavy ? 1u : 0u) && (heavy ? k0 + k <= col : k0 + k < col) ? a[k] : 0;
+  for (int k = 0; k < S; ++k) key += ((h >> k) & 1) == (heavy ? 1u : 0u) && (heavy ? k0 + k <= col : k0 + k < col) ? a[k] : 0;
   key = lane_u64(group_scan_u64<64>(key), 63);
   // first slot of a kind whose inclusive prefix exceeds `past`, and that prefix; NONE_SLOT if there is none
   uint64_t at = 0;
   auto above = [&](uint32_t kind, uint64_t past) -> uint32_t {
-    uint64_t run[4], t = 0;
+    uint64_t run[S], t = 0;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < S; ++k) {
       t += ((h >> k) & 1) == kind ? a[k] : 0;
       run[k] = t;
     }
@@ -531,16 +536,16 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
     const unsigned long long m = __ballot(inc > past);
     if (!m) return NONE_SLOT;
     const int l = __ffsll((long long)m) - 1;
-    uint32_t k = 3;
+    uint32_t k = S - 1;
     uint64_t x = inc;
 #pragma unroll
-    for (int i = 2; i >= 0; --i)
+    for (int i = S - 2; i >= 0; --i)
       if (before + run[i] > past) {
         k = i;
         x = before + run[i];
       }
     at = lane_u64(x, l);
-    return 4u * l + (uint32_t)__builtin_amdgcn_readlane((int)k, l);
+    return S * (uint32_t)l + (uint32_t)__builtin_amdgcn_readlane((int)k, l);
   };
   if (!heavy) {
     // first heavy whose surplus prefix exceeds the key; the last heavy if there is none; col itself without any heavy
@@ -549,15 +554,15 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
     const unsigned long long m = __ballot(h != 0);
     if (!m) return col;
     const int l = 63 - __clzll((long long)m);
-    return 4u * l + 31u - (uint32_t)__clz(__builtin_amdgcn_readlane((int)h, l));
+    return S * (uint32_t)l + 31u - (uint32_t)__clz(__builtin_amdgcn_readlane((int)h, l));
   }
   // next heavy after col (none: col is the last heavy and keeps the draw), then the first light l with SL(l) >= key:
   // prob = (one + key - SL(l)) / one
-  const uint32_t after = k0 > col ? h : k0 + 3 <= col ? 0u : h & ~((2u << j) - 1u);
+  const uint32_t after = k0 > col ? h : k0 + S - 1 <= col ? 0u : h & ~((2u << j) - 1u);
   const unsigned long long m = __ballot(after != 0);
   if (!m || above(0, key - 1) == NONE_SLOT) return col;
   const int l = __ffsll((long long)m) - 1;
-  return u < residual_prob(L.one + key - at, L) ? col : 4u * l + (uint32_t)__ffs(__builtin_amdgcn_readlane((int)after, l)) - 1u;
+  return u < residual_prob(L.one + key - at, L) ? col : S * (uint32_t)l + (uint32_t)__ffs(__builtin_amdgcn_readlane((int)after, l)) - 1u;
 }
 
 // Row-local slot that (walker, step) with random numbers r draws from the row of d >= 1 entries, or NONE_SLOT when
@@ -566,19 +571,22 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
 //                     through its part of the row in slot order, once, all lanes together (k advances by 4 per lane)
 //   row.again(k, w)   the same, afterwards, for any slots and by any wavefront
 //   Row::U            how many times 256 slots are in flight at once; if that is more than one, instead of first():
-//   Row::WAVE         rows of up to WAVE_MOST entries by draw_wave, from row.load(k, w): the same before any other
+//   Row::WAVE         whether rows of up to WAVE_MOST entries go to draw_wave, from row.load(k, w): as first(), before any other call
 //   Row::HELD         0, 4 or 16: rows of up to so many slots a thread (4,095 at most) by draw_held
 //   row.many(k, end, again, w)  slots k + 256 j .. k + 256 j + 3 for j < U, zeros from slot `end` on, in both sweeps
 template <int T, class Row>
 __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const u32x4& r, DrawLds<T>& lds) {
   constexpr int NW = T / 64;
   const uint32_t wave = threadIdx.x >> 6;
+  if constexpr (Row::WAVE == WAVE_EACH) {
+    if (d <= WAVE_MOST) return draw_wave<4>(row, d, r.x, u24(r.y));
+  }
   uint32_t csz = DRAW_CHUNK;
   while ((uint64_t)csz * DRAW_CHUNKS < d) csz *= 2;
   const uint32_t nc = (uint32_t)(((uint64_t)d + csz - 1) / csz), cpw = (nc + NW - 1) / NW;
   const uint32_t c0 = wave * cpw, c1 = min(nc, c0 + cpw);
   __syncthreads();  // the draw before has been read by everyone
-  if constexpr (Row::WAVE) {
+  if constexpr (Row::WAVE == WAVE_ONE) {
     if (d <= WAVE_MOST) {
       static_assert(NW > 1, "a wavefront alone goes on as it is");
       if (wave == (blockIdx.x & (NW - 1))) {  // not always on the same SIMD
@@ -608,7 +616,9 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
     return surpluses_may_wrap(L.scale) ? draw_entry<true, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds)
                                        : draw_entry<false, T>(row, d, L, col, ec, u, csz, nc, k0, k1, lds);
   }
-  if (d <= std::min(4u * T, HELD_MOST)) return draw_held<1, T>(row, d, L, col, ec, u, lds);
+  if constexpr (Row::WAVE == WAVE_NONE || 4 * T > WAVE_MOST) {
+    if (d <= std::min(4u * T, HELD_MOST)) return draw_held<1, T>(row, d, L, col, ec, u, lds);
+  }
   if constexpr (Row::HELD == 16) {
     constexpr uint32_t Q = T >= 512 ? 2 : 4;
     if (d <= std::min(4 * Q * T, HELD_MOST)) return draw_held<Q, T>(row, d, L, col, ec, u, lds);
@@ -620,10 +630,12 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
 // The graph's own weights of a row (the weight array has 16 spare bytes, so four slots can be read from any).
 struct PlainRow {
   static constexpr int U = 4;
-  static constexpr bool WAVE = false;  // most of its walkers are a wavefront anyway (with it 10,000 x 8, scale 22, 187 -> 194 us)
+  static constexpr WaveRows WAVE = WAVE_EACH;
   static constexpr int HELD = 4;
   const float* w;
   uint32_t d;
+  __device__ __forceinline__ void load(uint32_t k, float (&x)[4]) const { again(k, x); }
+  __device__ __forceinline__ void load(uint32_t k, float (&x)[1]) const { x[0] = masked_weight(w[min(k, d - 1)], k < d); }
   // Branches that a wavefront takes as one: all loads are on their way before the first is waited for.
   __device__ __forceinline__ void many(uint32_t k, uint32_t end, bool, float (&x)[U][4]) const {
     const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)k);
@@ -651,7 +663,7 @@ constexpr uint32_t FN_CACHE = 4096;
 template <class Fn>
 struct FunctionRow {
   static constexpr int U = 1;
-  static constexpr bool WAVE = false;
+  static constexpr WaveRows WAVE = WAVE_NONE;
   static constexpr int HELD = 0;  // the operator is called where it is linked in: node2vec's, 8,000 walkers x 20, scale 16, 5.5 ms, 6.0 with
   Fn fn;
   uint32_t d;

@@ -553,6 +553,32 @@ def test_node2vec_table_rows_of_one_wavefront(orc, walkers, kind):
     assert sampled == want[2]
 
 
+@pytest.mark.parametrize("kind", ["uniform", "lognormal", "equal", "sparse", "tiny"])
+@pytest.mark.parametrize("walkers", [900, 3000, 9000])
+def test_online_static_draws_from_short_rows(orc, walkers, kind):
+    # walkers of four wavefronts, two and one; rows around the 64 entries that have a slot a lane and the 256 that have four
+    from skywalker_amd import capi
+    rng = np.random.default_rng(59)
+    degs = list(range(1, 9)) * 4 + [31, 32, 33, 62, 63, 64, 65, 66, 127, 128, 129] * 6 + list(range(252, 260)) * 6 + [300, 1023, 1025] * 2
+    rng.shuffle(degs)
+    n = len(degs)
+    xadj = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
+    adjncy = np.concatenate([np.sort(rng.integers(0, n, k)) for k in degs]).astype(np.uint32)
+    w = weights(len(adjncy), rng, {"tiny": "sparse"}.get(kind, kind))
+    if kind == "tiny":
+        w *= np.float32(1e-19)
+    seeds = rng.integers(0, n, walkers).astype(np.uint32)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_full_build", 0)
+    g.set_option("online_direct", 1)
+    paths, lengths, sampled, _ = g.walk_online(capi.BIAS_STATIC, 1.0, 1.0, seeds, 12, 0.02, 43)
+    got = paths.to_host((walkers, 13)), lengths.to_host()
+    g.free()
+    want = orc.walk_online(xadj, adjncy, w, 0, 1.0, 1.0, seeds, 12, 0.02, 43)
+    assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
+    assert sampled == want[2]
+
+
 @pytest.mark.parametrize("longest,walkers", [(70001, 256), (70001, 257), (70001, 8193), (40001, 512), (40001, 513), (40001, 16385),
                                              (12289, 1024), (12289, 1025), (12289, 8193)])
 def test_online_static_draws_by_workgroups_of_every_size(longest, walkers):
