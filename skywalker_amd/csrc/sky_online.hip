@@ -25,8 +25,8 @@ int walk_online_node2vec(sky_graph* g, float p, float q, const uint32_t* seeds, 
 // others the draw is evaluated directly.
 // A step is a chain: bounds, weights, draw, neighbour.  Most rows met are short (half of all cycles went to rows below 64 entries, 9,000 to 12,000
 // a draw by the forms for long rows), so up to 64 entries have a slot a lane (draw_wave) and their neighbours loaded beside the weights,
-// and up to 256 four slots a lane: 20,000 walkers x 4 on the scale-16 graph 79.1 -> 68.7 us, 9,000 x 10 on the scale-20 graph 124 -> 112.5,
-// 10,000 x 8 on the scale-22 graph 187.9 -> 183.7, most of it the build of the long rows.
+// and up to 256 (512 where a walker is a wavefront) four (eight) slots a lane: 20,000 walkers x 4 on the scale-16 graph 79.1 -> 68.7 us, 9,000 x 10 on the scale-20 graph 124 -> 112.5,
+// 10,000 x 8 on the scale-22 graph 187.9 -> 180.3, most of it the build of the long rows.
 // Six wavefronts to a SIMD, 80 registers, is what 64 and 128 threads come to without spills (5,000 x 10 on the scale-18 graph by 128 threads
 // 92.5 us before, 83.3 with the short rows apart, 78.7 with 80 registers for 87); 256 threads would spill and gain nothing.
 template <int T>

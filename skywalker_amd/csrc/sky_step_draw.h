@@ -451,12 +451,15 @@ __device__ __forceinline__ bool row_ledger(Row& row, const uint32_t d, const uin
 }
 
 // The draw from a row of at most 64 S entries by one wavefront, S consecutive slots a lane: no barrier, no LDS, no sweep twice.  S is 4 for rows
-// of up to WAVE_MOST entries, and 1 for those of up to 64 where the caller takes the trouble.
+// of up to WAVE_MOST entries, and 1 for those of up to 64 in the walk without tables.
 // In the table-per-step walk one wavefront of the workgroup draws for all (WAVE_ONE: its weights come from windows in LDS); the others wait for it
 // and leave the SIMDs to the walkers beside.  A step from a row of 256 entries and fewer, half of all, takes 8,300 cycles instead of 11,000 (2,000 x
 // 40 on the scale-18 graph 549 -> 518 us, on the scale-17 graph 449 -> 410, 200 x 40 there 254 -> 217).  With eight slots a lane a row of 300
 // takes as long as by the workgroup, with sixteen a row of 950 takes longer (518 / 520 / 803 us).
-// In the walk without tables every wavefront of the workgroup draws for itself, all the same slot, and no barrier is met (WAVE_EACH).
+// In the walk without tables every wavefront of the workgroup draws for itself, all the same slot, and no barrier is met (WAVE_EACH).  A workgroup
+// of one wavefront has eight slots a lane for rows of 257 to 512 entries too (10,000 x 8 on the scale-22 graph 183.9 -> 180.3 us, while the 80
+// registers of six wavefronts to a SIMD suffice: with what the compiler keeps of the sum for the amounts it spills, 181.5).  Sixteen for rows
+// of up to 1,024 spill (217, and 183.5 with the slots in four strips and the amounts computed again).
 // All lanes call it together.
 constexpr uint32_t WAVE_MOST = 256;
 enum WaveRows { WAVE_NONE, WAVE_ONE, WAVE_EACH };
@@ -498,10 +501,17 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
   } else {
     u128 sum{0, 0};
 #pragma unroll
-    for (int k = 0; k < S; ++k) sum = add128(sum, weight_fixed(w[k]));
+    for (int k = 0; k < S; ++k) {
+      sum = add128(sum, weight_fixed(w[k]));
+      if (S > 4 && k + 1 < S) asm volatile("" : "+v"(w[k + 1]), "+v"(sum.lo));  // one after another
+    }
     sum = group_sum_u128<64>(sum);
     if ((sum.lo | sum.hi) == 0) return NONE_SLOT;
     L = make_ledger(d, sum);
+  }
+  if (S > 4) {  // the doubles of the sum are not kept for the amounts
+#pragma unroll
+    for (int k = 0; k < S; ++k) asm volatile("" : "+v"(w[k]));
   }
   const uint32_t col = __umulhi(rx, d), j = col % S;
   float wc = w[0];
@@ -571,7 +581,8 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
 //                     through its part of the row in slot order, once, all lanes together (k advances by 4 per lane)
 //   row.again(k, w)   the same, afterwards, for any slots and by any wavefront
 //   Row::U            how many times 256 slots are in flight at once; if that is more than one, instead of first():
-//   Row::WAVE         whether rows of up to WAVE_MOST entries go to draw_wave, from row.load(k, w): as first(), before any other call
+//   Row::WAVE         whether rows of up to WAVE_MOST entries (twice that for WAVE_EACH and T = 64) go to draw_wave, from row.load(k, w): as
+//                     first(), before any other call
 //   Row::HELD         0, 4 or 16: rows of up to so many slots a thread (4,095 at most) by draw_held
 //   row.many(k, end, again, w)  slots k + 256 j .. k + 256 j + 3 for j < U, zeros from slot `end` on, in both sweeps
 template <int T, class Row>
@@ -580,6 +591,9 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
   const uint32_t wave = threadIdx.x >> 6;
   if constexpr (Row::WAVE == WAVE_EACH) {
     if (d <= WAVE_MOST) return draw_wave<4>(row, d, r.x, u24(r.y));
+    if constexpr (NW == 1) {
+      if (d <= 2 * WAVE_MOST) return draw_wave<8>(row, d, r.x, u24(r.y));
+    }
   }
   uint32_t csz = DRAW_CHUNK;
   while ((uint64_t)csz * DRAW_CHUNKS < d) csz *= 2;
@@ -635,6 +649,16 @@ struct PlainRow {
   const float* w;
   uint32_t d;
   __device__ __forceinline__ void load(uint32_t k, float (&x)[4]) const { again(k, x); }
+  __device__ __forceinline__ void load(uint32_t k, float (&x)[8]) const {
+    float a[4], b[4];
+    again(k, a);
+    again(k + 4, b);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      x[t] = a[t];
+      x[4 + t] = b[t];
+    }
+  }
   __device__ __forceinline__ void load(uint32_t k, float (&x)[1]) const { x[0] = masked_weight(w[min(k, d - 1)], k < d); }
   // Branches that a wavefront takes as one: all loads are on their way before the first is waited for.
   __device__ __forceinline__ void many(uint32_t k, uint32_t end, bool, float (&x)[U][4]) const {

@@ -556,10 +556,11 @@ def test_node2vec_table_rows_of_one_wavefront(orc, walkers, kind):
 @pytest.mark.parametrize("kind", ["uniform", "lognormal", "equal", "sparse", "tiny"])
 @pytest.mark.parametrize("walkers", [900, 3000, 9000])
 def test_online_static_draws_from_short_rows(orc, walkers, kind):
-    # walkers of four wavefronts, two and one; rows around the 64 entries that have a slot a lane and the 256 that have four
+    # walkers of four wavefronts, two and one; rows around the 64 entries that have a slot a lane, the 256 that have four and
+    # the 512 that have eight where a walker is one wavefront
     from skywalker_amd import capi
     rng = np.random.default_rng(59)
-    degs = list(range(1, 9)) * 4 + [31, 32, 33, 62, 63, 64, 65, 66, 127, 128, 129] * 6 + list(range(252, 260)) * 6 + [300, 1023, 1025] * 2
+    degs = list(range(1, 9)) * 4 + [31, 32, 33, 62, 63, 64, 65, 66, 127, 128, 129] * 6 + list(range(252, 260)) * 6 + [300, 509, 510, 511, 512, 513, 1025] * 2
     rng.shuffle(degs)
     n = len(degs)
     xadj = np.concatenate([[0], np.cumsum(degs)]).astype(np.uint32)
