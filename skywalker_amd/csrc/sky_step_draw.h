@@ -467,11 +467,9 @@ __device__ __forceinline__ uint64_t lane_u64(uint64_t v, int lane) {
   return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane) << 32 |
          (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
 }
-template <int S = 4, class Row>
-__device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const uint32_t rx, const float u) {
-  const uint32_t lane = threadIdx.x & 63, k0 = S * lane;
-  float w[S];
-  row.load(k0, w);
+// Ledger of a row of d >= 1 entries that the lanes of one wavefront hold, S each, zeros past the row; false when the weights sum to zero.
+template <int S>
+__device__ __forceinline__ bool wave_ledger(float (&w)[S], const uint32_t d, Ledger& L) {
   double fsum = 0.0;
   uint32_t most = 0;  // the complement of the least (weight bits - 1): what lanes without a source add to a scan, 0, changes nothing
 #pragma unroll
@@ -494,9 +492,8 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
   });
   fsum = __longlong_as_double((long long)lane_u64((uint64_t)__double_as_longlong(fsum), 63));
   most = (uint32_t)__builtin_amdgcn_readlane((int)most, 63);
-  Ledger L;
   if (plain_sum_is_exact(fsum, ~most)) {
-    if (fsum == 0.0) return NONE_SLOT;
+    if (fsum == 0.0) return false;
     L = make_ledger_small(d, fsum);
   } else {
     u128 sum{0, 0};
@@ -506,9 +503,18 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
       if (S > 4 && k + 1 < S) asm volatile("" : "+v"(w[k + 1]), "+v"(sum.lo));  // one after another
     }
     sum = group_sum_u128<64>(sum);
-    if ((sum.lo | sum.hi) == 0) return NONE_SLOT;
+    if ((sum.lo | sum.hi) == 0) return false;
     L = make_ledger(d, sum);
   }
+  return true;
+}
+template <int S = 4, class Row>
+__device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const uint32_t rx, const float u) {
+  const uint32_t lane = threadIdx.x & 63, k0 = S * lane;
+  float w[S];
+  row.load(k0, w);
+  Ledger L;
+  if (!wave_ledger(w, d, L)) return NONE_SLOT;
   if (S > 4) {  // the doubles of the sum are not kept for the amounts
 #pragma unroll
     for (int k = 0; k < S; ++k) asm volatile("" : "+v"(w[k]));

@@ -102,6 +102,28 @@ def test_distinct_children_of_rows_held_in_lds(orc, fanout, weights):
     g.free()
 
 
+@pytest.mark.parametrize("weights", ["lognormal", "equal", "sparse", "tiny"])
+@pytest.mark.parametrize("fanout", [[1, 3], [1, 20, 2], [1, 63], [1, 70]])
+def test_online_children_of_short_rows_from_the_weights(orc, fanout, weights):
+    # rows around the 64 entries that have a slot a lane, longer than the fan-out and not; more draws than lanes; weights that sum up exactly
+    # in doubles or not, most of none, all next to none
+    from skywalker_amd import capi
+    rng = np.random.default_rng(71)
+    degs = [0, 1, 2, 3, 4, 5, 19, 20, 21, 22, 31, 32, 33, 62, 63, 64, 65, 66, 69, 70, 71, 130]
+    xadj, adjncy, w = graph_from_degrees(degs * 12, rng, {"tiny": "sparse"}.get(weights, weights))
+    if weights == "tiny":
+        w = w * np.float32(1e-19)
+    seeds = rng.integers(0, len(xadj), 700).astype(np.uint32)
+    lps, slen = capi.sample_layout(fanout)
+    want = orc.sample_online(xadj, adjncy, w, seeds, fanout, 31)
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_direct", 1)
+    data, sl, sampled, _ = g.sample_online(seeds, fanout, 31)
+    assert np.array_equal(sl.to_host((700, slen)), want[1]) and np.array_equal(data.to_host((700, lps)), want[0])
+    assert sampled == want[2]
+    g.free()
+
+
 def test_online_sampling_with_short_rows_built_in_vertex_order(orc):
     # option small_in_place = 1 on a list of frontier vertices (by default only builds of 2^25 rows and more use it)
     from skywalker_amd import capi
