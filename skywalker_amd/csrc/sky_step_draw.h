@@ -2,7 +2,7 @@
 // the threads of a workgroup evaluate that entry alone, from the same prefix-sum definition the offline build uses:
 //   pass 1  exact sum of the row's weights -> ledger, class of entry col
 //           (a light col whose own share accepts the draw needs nothing more)
-// in rows of up to 16 slots a thread
+// in rows of up to 256 entries all of it by one wavefront, in registers (draw_wave); in rows of up to 16 slots a thread
 //   scan    of deficits and surpluses over the workgroup, whose prefixes each thread has for its own slots (draw_held)
 // and in longer ones
 //   pass 2  deficits and surpluses of every chunk of the row; their prefixes over the chunks
