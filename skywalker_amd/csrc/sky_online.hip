@@ -577,6 +577,10 @@ struct N2vMapRow {
       if (!again && d <= keep && at < end) reinterpret_cast<float4*>(kept)[at >> 2] = make_float4(x[j][0], x[j][1], x[j][2], x[j][3]);
     }
   }
+  __device__ __forceinline__ void load(uint32_t k, float (&x)[1]) const {
+    const uint32_t at = min(k, d - 1);
+    x[0] = weigh(w[at], nbr[at], k < d);
+  }
   __device__ __forceinline__ void load(uint32_t k, float (&x)[4]) const {
     const uint32_t at = min(k, (d - 1) & ~3u);
     const float4u a = *reinterpret_cast<const float4u*>(w + at);

@@ -451,7 +451,8 @@ __device__ __forceinline__ bool row_ledger(Row& row, const uint32_t d, const uin
 }
 
 // The draw from a row of at most 64 S entries by one wavefront, S consecutive slots a lane: no barrier, no LDS, no sweep twice.  S is 4 for rows
-// of up to WAVE_MOST entries, and 1 for those of up to 64 in the walk without tables.
+// of up to WAVE_MOST entries, and 1 for those of up to 64 (table-per-step walks: 2,000 x 40 on the scale-18 graph 525 -> 507 us, on the scale-17
+// graph 412 -> 392, 1,500 x 20 on the scale-14 graph with 5 edges a vertex 88 -> 80).
 // In the table-per-step walk one wavefront of the workgroup draws for all (WAVE_ONE: its weights come from windows in LDS); the others wait for it
 // and leave the SIMDs to the walkers beside.  A step from a row of 256 entries and fewer, half of all, takes 8,300 cycles instead of 11,000 (2,000 x
 // 40 on the scale-18 graph 549 -> 518 us, on the scale-17 graph 449 -> 410, 200 x 40 there 254 -> 217).  With eight slots a lane a row of 300
@@ -610,7 +611,7 @@ __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const 
     if (d <= WAVE_MOST) {
       static_assert(NW > 1, "a wavefront alone goes on as it is");
       if (wave == (blockIdx.x & (NW - 1))) {  // not always on the same SIMD
-        const uint32_t cand = draw_wave(row, d, r.x, u24(r.y));
+        const uint32_t cand = d <= 64 ? draw_wave<1>(row, d, r.x, u24(r.y)) : draw_wave<4>(row, d, r.x, u24(r.y));
         if ((threadIdx.x & 63) == 0) lds.result = cand;
       }
       __syncthreads();
