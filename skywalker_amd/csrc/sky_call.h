@@ -46,7 +46,8 @@ struct CallWords {
   unsigned long long seq = 0, asked = 0;  // numbers of the last end and of the last question
   uint32_t forks = 0;                     // and of the last fork
   int khz = 0;
-  uint32_t awaited = 0;  // side streams that the end kernel waits for
+  int sides = 0;  // side streams over which the call ends beside the graph's, and these
+  hipStream_t side[SIDE_STREAMS] = {nullptr, nullptr, nullptr};
   uint32_t parts = 0;  // words that the call's kernels add sampled edges to: none, one or CALL_PARTS
   bool dirty = false;  // a call has begun and not ended well: its device words may not be zero
 };
@@ -59,16 +60,12 @@ __device__ __forceinline__ void call_stamp(CallDevice* call) {
 __device__ __forceinline__ void call_sampled(CallDevice* call, uint32_t who, uint32_t parts, unsigned long long n) {
   if (n) atomicAdd(&call->part[(who & (parts - 1u)) * CALL_PART_WORDS], n);
 }
-// Last statement of the call's last kernel, by one thread that has seen every other thread's contribution.  The host may go on
-// before the device words are zero again; who uses them next is a kernel behind this one on the device's null stream, whichever graph
-// it belongs to.
-__device__ __forceinline__ void call_report(CallDevice* call, CallHost* host, unsigned long long seq,
-                                            unsigned long long start, unsigned long long sampled) {
+// By one thread of the call's last kernel, which has seen every other thread's contribution.
+__device__ __forceinline__ void call_report(CallHost* host, unsigned long long seq, unsigned long long start, unsigned long long sampled) {
   const unsigned long long ticks = start ? wall_clock64() - start : 0;  // 0: the call had nothing to launch
   constexpr unsigned long long VALUE = (1ull << CALL_VALUE_BITS) - 1;
   __hip_atomic_store(&host->sampled, (sampled & VALUE) | seq << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(&host->ticks, (ticks & VALUE) | seq << CALL_VALUE_BITS, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-  call->start = 0;
 }
 
 // How many words `waves` wavefronts that each add once should have.
@@ -76,7 +73,8 @@ inline uint32_t call_parts(uint64_t waves) { return waves >= CALL_MANY ? CALL_PA
 // The device words of `w` (taken on first use), cleared; a call that ended in an error may have left something in them.
 int call_begin(sky_graph* g, CallWords* w, CallDevice** call);
 // Enqueues the end kernel behind what the call has put on the graph's stream, waits for it and hands out the results.
-// Outputs may be null.  `counts` (n of them, device, may be null) are added to the sampled edges.
+// Outputs may be null.  `counts` (n of them, device, may be null) are added to the sampled edges; a call that ends over side streams has none.  After
+// an error nothing of the call is left on its side streams.
 int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts = nullptr, uint64_t n = 0);
 // The host's questions in the course of a call: a kernel answers question number call_ask(w) by call_answer, word by word, and
 // call_answered waits for the first n.
@@ -88,7 +86,7 @@ int call_answered(sky_graph* g, CallWords* w, unsigned long long* values, int n)
 // Kernels beside those of the graph's stream, on streams that all graphs of a device share (sky_sides.h).  These and the graph's stream wait for one
 // another by words in pinned memory: a kernel on the graph's stream notes that it runs (fork_mark), so that everything in front of it has
 // ended, and of small last ones on the others the one that finds all of them there that everything in front of these has.  Who waits, by a stream operation (one
-// thread of the runtime's that reads the word until the number is there) or in the call's end kernel (beside_join), is always enqueued behind the kernel that writes.  The runtime
+// thread of the runtime's that reads the word until the number is there), is always enqueued behind the kernel that writes.  The runtime
 // gives a hardware queue what is enqueued in the order of the calls, so that every wait ends: also where other threads' calls lie
 // between, where streams share a hardware queue, and where there is only one.  Who waits for the whole device after a call, which does
 // not need it, waits 8 to 10 us longer for every side stream that has had work.  2 us
@@ -101,7 +99,7 @@ struct Beside {
   CallDevice* dev = nullptr;
   CallHost* host = nullptr;
   uint32_t number = 0;
-  CallWords* last = nullptr;  // of the call that ends with the join: its end kernel waits, not the graph's stream
+  CallWords* last = nullptr;  // of the call that ends with the join: the graph's stream waits for nothing
 };
 struct ForkMark {
   uint32_t* word;  // null: none
@@ -116,10 +114,11 @@ __device__ __forceinline__ void fork_mark(const ForkMark& f) {
 int beside_begin(sky_graph* g, Beside* b, ForkMark* mark, int streams);
 // With that kernel on its way: side stream k waits for its mark, if it does not already.
 int beside_fork(Beside* b, int k);
-// The graph's stream waits for what the side streams of the fork hold, or, where nothing but the call's end follows, the end kernel does: it is
-// there anyway, and a stream's wait takes 4.5 us and 3 more until the next kernel runs.  (A stream's wait / the end kernel's, us: scale 16 with 16
-// edges a vertex 45 / 42.5, scale 18 with 10 60 / 56.5, scale 20 with 6 78.4 / 73.5, with 16 120 / 118.3, 3 M entries in rows of up to 20,000
-// 57.4 / 55.1, 40 M of up to 300,007 312 / 309.5, scale 23 with 8 373 / 369.)
+// The graph's stream waits for what the side streams of the fork hold.  Where nothing but the call's end follows no stream waits: the last kernels of all
+// of them report the call together (side_arrive), while a stream's wait takes 4.5 us and 3 more until the next kernel runs.  (A stream's wait / so, us:
+// scale 16 with 16 edges a vertex 47.0 / 45.0, scale 18 with 10 61.0 / 58.1, scale 20 with 6 78.9 / 75.5, with 16 120.6 / 118.5, 3 M entries in rows
+// of up to 20,000 57.5 / 55.4, 40 M of up to 300,007 311.7 / 309.3, scale 23 with 8 371.8 / 369.6.  An end kernel that waits for the words
+// of the others took 0.5 to 1.5 us less, but wants kernels of two queues to run at once, and to give up where they do not.)
 int beside_join(Beside* b);
 // Instead of a join, after an error: the host waits for them.
 void beside_drop(Beside* b);

@@ -36,23 +36,33 @@ __global__ __launch_bounds__(1024) void call_end_kernel(CallDevice* call, CallHo
   }
   if (threadIdx.x >= 64) return;
   if (parts > 1) x = shfl_u64(group_scan_u64<64>(x), 63);
-  if (threadIdx.x == 0) call_report(call, host, seq, start, t + x);
+  // The host may go on before the device words are zero again; who uses them next is a kernel behind this one on the device's null
+  // stream, whichever graph it belongs to.
+  if (threadIdx.x == 0) {
+    call_report(host, seq, start, t + x);
+    call->start = 0;
+  }
 }
 static_assert(CALL_PARTS == 64, "by the first wavefront");
 
-// The end of a call that has work on `awaited` side streams, and samples no edges.  The last kernels of these were enqueued before this one, so
-// that they run to their end whichever queue each is in.  If they do not, the host finds that out: nothing is reported to it.
-__global__ __launch_bounds__(64) void call_end_beside_kernel(CallDevice* call, CallHost* host, unsigned long long seq, uint32_t awaited,
-                                                             unsigned long long patience) {
-  if (threadIdx.x) return;
-  const unsigned long long start = call->start, since = wall_clock64();
-  while (__hip_atomic_load(&call->joined, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != awaited) {
-    if (wall_clock64() - since > patience) return;
-    __builtin_amdgcn_s_sleep(1);
+// The end of a call over several streams, which samples no edges: the last kernel of each.
+struct SideEnd {
+  CallDevice* call;
+  CallHost* host;
+  unsigned long long seq;
+  __device__ uint32_t arrive() const { return __hip_atomic_fetch_add(&call->joined, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u; }
+  __device__ unsigned long long clear() const {
+    const unsigned long long start = __hip_atomic_load(&call->start, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&call->start, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&call->joined, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return start;
   }
-  call->joined = 0;
-  call_report(call, host, seq, start, 0);
-}
+  __device__ void report(unsigned long long start) const {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+    call_report(host, seq, start, 0);
+  }
+};
+__global__ void call_end_sides_kernel(CallDevice* call, CallHost* host, unsigned long long seq, uint32_t of) { side_arrive(SideEnd{call, host, seq}, of); }
 
 __global__ __launch_bounds__(256) void sum_counts_kernel(const uint32_t* __restrict__ x, uint64_t n, CallDevice* call) {
   __shared__ unsigned long long s_w[4];
@@ -146,8 +156,8 @@ void call_release(CallWords* w) {
 int call_begin(sky_graph* g, CallWords* w, CallDevice** call) {
   if (!w->host) SKY_TRY(take_words(g->device, w));
   if (w->dirty) SKY_HIP(hipMemsetAsync(w->dev, 0, sizeof(CallDevice), g->stream));
-  w->awaited = 0;
   w->dirty = true;  // until it has ended well
+  w->parts = 0;
   ++g->calls;
   *call = w->dev;
   return SKY_OK;
@@ -177,8 +187,7 @@ struct SideRuntime {
 SidePool<SideRuntime> g_side[SIDE_DEVICES];
 }  // namespace
 
-// The last kernel of each of the n side streams of a fork (n = 0: the call's end kernel counts them).  (A word for each, and a wait for each on
-// the graph's stream: 4.5 us apiece.)
+// The last kernel of each of the n side streams of a fork.  (A word for each, and a wait for each on the graph's stream: 4.5 us apiece.)
 __global__ void beside_done_kernel(CallDevice* dev, CallHost* host, uint32_t n, uint32_t number) {
   if (__hip_atomic_fetch_add(&dev->joined, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) + 1u != n) return;
   __hip_atomic_store(&dev->joined, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -215,10 +224,14 @@ int beside_join(Beside* b) {
   for (bool u : b->used) n += u;
   if (!n) return SKY_OK;
   for (int k = 0; k < SIDE_STREAMS; ++k)
-    if (b->used[k]) hipLaunchKernelGGL(beside_done_kernel, dim3(1), dim3(1), 0, b->stream[k], b->dev, b->host, b->last ? 0u : n, b->number);
+    if (b->used[k]) {
+      if (b->last) hipLaunchKernelGGL(call_end_sides_kernel, dim3(1), dim3(1), 0, b->stream[k], b->dev, b->host, b->last->seq + 1, n + 1);
+      else hipLaunchKernelGGL(beside_done_kernel, dim3(1), dim3(1), 0, b->stream[k], b->dev, b->host, n, b->number);
+    }
   SKY_HIP(hipGetLastError());
-  if (b->last) b->last->awaited = n;
-  else SKY_HIP(hipStreamWaitValue32(b->main, &b->host->done, b->number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+  if (!b->last) SKY_HIP(hipStreamWaitValue32(b->main, &b->host->done, b->number, hipStreamWaitValueEq, 0xFFFFFFFFu));
+  for (int k = 0; k < SIDE_STREAMS; ++k)
+    if (b->last && b->used[k]) b->last->side[b->last->sides++] = b->stream[k];
   for (bool& u : b->used) u = false;
   return SKY_OK;
 }
@@ -247,10 +260,9 @@ constexpr uint64_t END_COUNTS = 32768;
 // five microseconds, and one whose kernels fault ends with the runtime's error instead of polling for ever.
 constexpr auto POLL_FOR = std::chrono::microseconds(3000);
 
-constexpr unsigned long long END_PATIENCE = 60;  // seconds that an end kernel waits for side streams; a build takes 0.02
-
-// Waits until n host words from `from` on carry the number `seq`, and takes their values.
-static int take_values(hipStream_t st, const unsigned long long* from, int n, unsigned long long seq, unsigned long long* values) {
+// Waits until n host words from `from` on carry the number `seq`, and takes their values.  They are written from the graph's stream or one of `sides`.
+static int take_values(sky_graph* g, const unsigned long long* from, int n, unsigned long long seq, unsigned long long* values, const hipStream_t* sides = nullptr,
+                       int n_sides = 0) {
   constexpr unsigned long long VALUE = (1ull << CALL_VALUE_BITS) - 1;
   auto there = [&] {
     unsigned long long other = 0;
@@ -272,18 +284,20 @@ static int take_values(hipStream_t st, const unsigned long long* from, int n, un
     } while (!done && std::chrono::steady_clock::now() - t0 < POLL_FOR);
   }
   if (!done) {
-    SKY_HIP(hipStreamSynchronize(st));
+    const int waited = side_wait(1 + n_sides, [&](int k) { return (int)hipStreamSynchronize(k ? sides[k - 1] : g->stream); });
+    SKY_HIP((hipError_t)waited);
     if (!there()) return fail(SKY_ERR_HIP, "the call's end was not reported");
   }
   return SKY_OK;
 }
 
 int call_answered(sky_graph* g, CallWords* w, unsigned long long* values, int n) {
-  return take_values(g->stream, w->host->answer, n, w->asked, values);
+  return take_values(g, w->host->answer, n, w->asked, values);
 }
 
-int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
+static int end_call(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
   hipStream_t st = g->stream;
+  if (w->sides && (n || w->parts)) return fail(SKY_ERR_ARG, "a call that samples edges does not end over side streams");
   if (n > END_COUNTS) {
     hipLaunchKernelGGL(sum_counts_kernel, dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 1024)), dim3(256), 0, st, counts,
                        n, w->dev);
@@ -291,23 +305,24 @@ int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, con
     w->parts = CALL_PARTS;
   }
   const unsigned long long seq = ++w->seq;
-  if (w->awaited)
-    hipLaunchKernelGGL(call_end_beside_kernel, dim3(1), dim3(64), 0, st, w->dev, w->host, seq, w->awaited,
-                       (unsigned long long)w->khz * 1000 * END_PATIENCE);
+  if (w->sides) hipLaunchKernelGGL(call_end_sides_kernel, dim3(1), dim3(1), 0, st, w->dev, w->host, seq, (uint32_t)w->sides + 1);
   else
     hipLaunchKernelGGL(call_end_kernel, dim3(1), dim3(n > 64 ? 1024 : 64), 0, st, w->dev, w->host, seq, counts, (uint32_t)n, w->parts);
-  const bool awaited = w->awaited != 0;
-  w->parts = w->awaited = 0;
-  const hipError_t launched = hipGetLastError();
-  if (launched != hipSuccess && awaited) (void)hipDeviceSynchronize();  // the next call clears the words that the side streams write
-  SKY_HIP(launched);
+  w->parts = 0;
+  SKY_HIP(hipGetLastError());
   static_assert(offsetof(CallHost, ticks) == offsetof(CallHost, sampled) + 8, "taken together");
   unsigned long long words[2];
-  SKY_TRY(take_values(st, &w->host->sampled, 2, seq, words));
+  SKY_TRY(take_values(g, &w->host->sampled, 2, seq, words, w->side, w->sides));
   w->dirty = false;
   if (sampled) *sampled = words[0];
   if (seconds) *seconds = (double)words[1] / ((double)w->khz * 1e3);
   return SKY_OK;
+}
+int call_end(sky_graph* g, CallWords* w, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
+  const int rc = end_call(g, w, sampled, seconds, counts, n);
+  if (rc != SKY_OK) (void)side_wait(w->sides, [&](int k) { return (int)hipStreamSynchronize(w->side[k]); });  // the next call clears the words that these write
+  w->sides = 0;
+  return rc;
 }
 int call_end(sky_graph* g, uint64_t* sampled, double* seconds, const uint32_t* counts, uint64_t n) {
   return call_end(g, &g->call, sampled, seconds, counts, n);

@@ -1,5 +1,5 @@
-// Which graphs have side streams (sky_call.h, Beside), and how long these are there.  Host code without a kernel: tests compile it for the CPU
-// with a runtime of their own.
+// Which graphs have side streams (sky_call.h, Beside), how long these are there, and how a call over several streams ends.  Tests compile it for
+// the CPU with a runtime of their own.
 #pragma once
 #include <cstdint>
 
@@ -75,5 +75,25 @@ struct SidePool {
     }
   }
 };
+
+// The last kernels of the streams of a call that ends over `of` of them, one each.  The one that finds all the others there reports, whatever the order
+// they run in: none waits for another, so that they may also run one at a time.  What the next call uses is cleared before the report, behind which
+// its kernels may follow on any of the streams.
+template <class Words>
+constexpr bool side_arrive(Words words, uint32_t of) {
+  if (words.arrive() != of) return false;
+  words.report(words.clear());
+  return true;
+}
+// The host's wait for n streams: for all of them, also after an error.  The first error, or 0.
+template <class Wait>
+int side_wait(int n, Wait wait) {
+  int first = 0;
+  for (int k = 0; k < n; ++k) {
+    const int rc = wait(k);
+    if (!first) first = rc;
+  }
+  return first;
+}
 
 }  // namespace sky

@@ -1,4 +1,4 @@
-"""Which graphs have side streams for their builds and how long these are there, compiled for the host with a runtime that counts (CPU only)."""
+"""Which graphs have side streams for their builds, how long these are there and how a call over several streams ends, compiled for the host with a runtime that counts (CPU only)."""
 import os
 import subprocess
 
@@ -7,8 +7,10 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "skywalker_amd", "csrc")
 MAIN = """
 #undef NDEBUG
+#include <algorithm>
 #include <cassert>
 #include <set>
+#include <vector>
 #include "sky_sides.h"
 using namespace sky;
 struct Asked : SideHold {
@@ -38,7 +40,7 @@ int main() {
   Runtime rt;
   SidePool<Runtime> pool;
   const SideAsk yes{1, 0, 0, 2}, first{1, 0, 0, 1};
-  (void)first;
+  (void)yes, (void)first;
   %s
 }
 """
@@ -143,3 +145,51 @@ def test_a_graph_that_holds_one_stream_keeps_it_where_another_cannot_be_made(run
   assert(pool.take(rt, &a, one) && !pool.take(rt, &a, yes) && a.held && a.refused && !pool.take(rt, &a, one));
   assert(pool.take(rt, &b, one) && rt.live.size() == 2 && pool.holders == 2);
 """)
+
+
+@pytest.mark.parametrize("sides", [1, 2, 3])
+def test_a_call_over_several_streams_ends_with_whichever_kernel_is_last(run, sides):
+    # the last kernels of the streams one at a time, in every order: each runs to its end, the last of them reports, once, with the words cleared
+    # before it does; call after call
+    run("""
+  static uint32_t joined, reports;
+  static unsigned long long start;
+  struct Words {
+    uint32_t arrive() { return ++joined; }
+    unsigned long long clear() {
+      const unsigned long long s = start;
+      joined = 0, start = 0;
+      return s;
+    }
+    void report(unsigned long long s) {
+      assert(s == 77 && joined == 0 && start == 0);
+      ++reports;
+    }
+  };
+  const uint32_t of = %d + 1;
+  std::vector<int> order(of);
+  for (uint32_t k = 0; k < of; ++k) order[k] = k;  // 0: the graph's stream
+  uint32_t calls = 0;
+  do {
+    start = 77;
+    for (uint32_t k = 0; k < of; ++k) {
+      assert(reports == calls);
+      assert(side_arrive(Words{}, of) == (k + 1 == of));
+    }
+    assert(reports == ++calls && joined == 0);
+  } while (std::next_permutation(order.begin(), order.end()));
+""" % sides)
+
+
+@pytest.mark.parametrize("failing", [-1, 0, 1, 2])
+def test_every_stream_of_a_call_is_waited_for_also_after_an_error(run, failing):
+    run("""
+  const int failing = %d;
+  std::vector<int> waited;
+  const int rc = side_wait(4, [&](int k) {
+    waited.push_back(k);
+    return k == failing ? 700 : k == 3 && failing >= 0 ? 701 : 0;
+  });
+  assert(rc == (failing >= 0 ? 700 : 0) && waited == (std::vector<int>{0, 1, 2, 3}));
+  assert(side_wait(0, [&](int) { return 1; }) == 0);
+""" % failing)
