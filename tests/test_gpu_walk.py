@@ -531,8 +531,8 @@ def test_node2vec_table_with_a_bit_per_vertex(orc, V, walkers, p, q):
 @pytest.mark.parametrize("kind", ["uniform", "equal", "sparse", "tiny"])
 @pytest.mark.parametrize("walkers", [300, 1000])
 def test_node2vec_table_rows_of_one_wavefront(orc, walkers, kind):
-    # rows around the 256 entries that one wavefront draws from by itself, and around the 4,095 whose surpluses fit 64 bits whatever the
-    # weights; weights that sum up exactly in doubles or not, none lighter than the others, most of no weight, all next to none
+    # rows around the 256 entries that one wavefront draws from by itself, and around the 4,095 up to which the workgroup holds them; weights that
+    # sum up exactly in doubles or not, none lighter than the others, most of no weight, all next to none
     from skywalker_amd import capi
     rng = np.random.default_rng(53)
     degs = list(range(1, 9)) * 4 + [63, 64, 65, 127, 128, 129] * 6 + list(range(250, 262)) * 12 + [4094, 4095, 4096, 4097] * 3
@@ -551,6 +551,45 @@ def test_node2vec_table_rows_of_one_wavefront(orc, walkers, kind):
     want = orc.walk_online(xadj, adjncy, w, 1, 2.0, 0.5, seeds, 10, 0.0, 41)
     assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0])
     assert sampled == want[2]
+
+
+def nearly_vanishing_row(d, lights):
+    """One weight counts in the row's sum, of d; `lights` weigh next to nothing, the others a hair less than what counts: d - 1 shares each."""
+    u = 2.0 ** -64
+    w = np.full(d, u * (1 - 2.0 ** -24))
+    w[d // 3] = u
+    w[np.random.default_rng(d).permutation(np.delete(np.arange(d), d // 3))[:lights]] = u * 2.0 ** -30
+    return w.astype(np.float32)
+
+
+@pytest.mark.parametrize("walkers", [300, 1000, 3000, 9000])
+def test_draws_from_rows_whose_surpluses_come_close_to_64_bits(orc, walkers):
+    # the longest rows that are held, by a wavefront or a workgroup, have sums just below 2^64; longer ones pass it, some by next to nothing, so that
+    # what wraps is below the deficits of most lights; walkers of 512, 256, 128 and 64 threads
+    from skywalker_amd import capi
+    near = [(d, 3) for d in (63, 64, 65, 255, 256, 257, 511, 512, 513, 1024, 1025, 2048, 2049, 4094, 4095, 4096, 4097)]
+    past = [(4227, 257), (4361, 513), (7080, 4710), (7941, 5828)]
+    rows = [nearly_vanishing_row(d, k) for d, k in near + past]
+    for w, (d, k) in zip(rows, near + past):
+        surplus = np.maximum(w.astype(np.float64) * 2.0 ** 64 * d - 1, 0).sum()  # the weights' sum is 1; 2^24 of these pass 64 bits
+        if (d, k) in past:
+            assert 0 < surplus - 2 ** 24 < k / 4
+        else:
+            assert surplus < 2 ** 24 and (d < 4094 or surplus > 0.998 * 2 ** 24)
+    w = np.concatenate(rows + [np.ones(32 * 20000, np.float32)])
+    lens = np.concatenate([[len(r) for r in rows], np.full(20000, 32)])
+    xadj = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    adjncy = np.arange(len(w), dtype=np.uint32) - np.repeat(xadj[:-1], lens)  # a vertex of its own for every slot of a row
+    seeds = np.arange(walkers, dtype=np.uint32) % len(rows)
+    seeds[walkers // 2:] = len(near) + seeds[walkers // 2:] % len(past)
+    oprob, oalias, _ = orc.alias_build(xadj, w)
+    want = orc.walk_offline(xadj, adjncy, oprob, oalias, seeds, 1, 0.0, 5)[0].ravel()
+    g = capi.Graph.upload(xadj, adjncy, w)
+    g.set_option("online_full_build", 0)
+    g.set_option("online_direct", 1)  # no row is built
+    for bias in (capi.BIAS_STATIC, capi.BIAS_NODE2VEC):
+        assert np.array_equal(g.walk_online(bias, 2.0, 0.5, seeds, 1, 0.0, 5)[0].to_host(), want), bias
+    g.free()
 
 
 @pytest.mark.parametrize("kind", ["uniform", "lognormal", "equal", "sparse", "tiny"])
