@@ -210,25 +210,23 @@ __device__ __forceinline__ uint32_t direct_children(const SampleArgs& a, const H
     lds.u[tid] = group_scan_u64<64>(e.heavy ? e.amount : 0);
     sync();
     const uint64_t total_u = lds.u[63], total_d = lds.d[63];
-    for (uint32_t first = 0; first < g.k; first += 64) {  // all lanes together: they have the row
-      const uint32_t i = first + tid;
-      const u32x4 r = philox(a.seed, (uint32_t)si, s * g.k + i, g.h, DOM_SAMPLE);
-      const uint32_t col = __umulhi(r.x, d);
-      const float u = u24(r.y);
-      const bool heavy = heavies >> col & 1, kept = u < __shfl(p, (int)col, 64);
-      uint32_t cand = col;
-      if (!heavy && !kept) {
-        // first heavy whose surplus prefix exceeds the deficits before col; the last heavy if there is none; col itself without any heavy
-        if (total_u) cand = first_greater(lds.u, 0, 64, min(col ? lds.d[col - 1] : 0, total_u - 1));
-      } else if (heavy) {
-        // the first light l with SL(l) >= the key, and the next heavy: prob = (one + key - SL(l)) / one
-        const uint64_t key = lds.u[col];
-        if (key < total_u && key <= total_d && !(u < residual_prob(L.one + key - lds.d[first_greater(lds.d, 0, 64, key - 1)], L)))
-          cand = col + (uint32_t)__ffsll((long long)(heavies >> (col + 1)));
-      }
-      const uint32_t child = (uint32_t)__shfl((int)next, (int)cand, 64);
-      if (i < g.k) out[i] = child;
+    // fewer draws than entries, so one a lane; all lanes together: they have the row
+    const u32x4 r = philox(a.seed, (uint32_t)si, s * g.k + tid, g.h, DOM_SAMPLE);
+    const uint32_t col = __umulhi(r.x, d);
+    const float u = u24(r.y);
+    const bool heavy = heavies >> col & 1, kept = u < __shfl(p, (int)col, 64);
+    uint32_t cand = col;
+    if (!heavy && !kept) {
+      // first heavy whose surplus prefix exceeds the deficits before col; the last heavy if there is none; col itself without any heavy
+      if (total_u) cand = first_greater(lds.u, 0, 64, min(col ? lds.d[col - 1] : 0, total_u - 1));
+    } else if (heavy) {
+      // the first light l with SL(l) >= the key, and the next heavy: prob = (one + key - SL(l)) / one
+      const uint64_t key = lds.u[col];
+      if (key < total_u && key <= total_d && !(u < residual_prob(L.one + key - lds.d[first_greater(lds.d, 0, 64, key - 1)], L)))
+        cand = col + (uint32_t)__ffsll((long long)(heavies >> (col + 1)));
     }
+    const uint32_t child = (uint32_t)__shfl((int)next, (int)cand, 64);
+    if (tid < g.k) out[tid] = child;
     return g.k;
   }
   uint32_t csz = DRAW_CHUNK;

@@ -105,8 +105,8 @@ def test_distinct_children_of_rows_held_in_lds(orc, fanout, weights):
 @pytest.mark.parametrize("weights", ["lognormal", "equal", "sparse", "tiny"])
 @pytest.mark.parametrize("fanout", [[1, 3], [1, 20, 2], [1, 63], [1, 70]])
 def test_online_children_of_short_rows_from_the_weights(orc, fanout, weights):
-    # rows around the 64 entries that have a slot a lane, longer than the fan-out and not; more draws than lanes; weights that sum up exactly
-    # in doubles or not, most of none, all next to none
+    # rows around the 64 entries that have a slot a lane, longer than the fan-out and not (those are taken whole); a draw for all lanes but one, and
+    # fan-outs that only longer rows draw for; weights that sum up exactly in doubles or not, most of none, all next to none
     from skywalker_amd import capi
     rng = np.random.default_rng(71)
     degs = [0, 1, 2, 3, 4, 5, 19, 20, 21, 22, 31, 32, 33, 62, 63, 64, 65, 66, 69, 70, 71, 130]
