@@ -79,7 +79,9 @@ __global__ __launch_bounds__(T, T <= 128 ? 6 : 1) void walk_direct_kernel(const 
 // 300,000: 207 walkers x 3 233 / 137 / 86 / 69 / 69; 5,000 x 2 1137 / 604 / 328 / 226; 7,000 x 2 1410 / 774 / 413 / 303 / 307.  Of 50,000
 // to 65,000: 352 x 8 269 / 158 / 102 / 84 / 89; 8,500 x 1 91 / 61 / 46 / 66; 20,000 x 2 233 / 190 / 195 / 288.  Of 25,000: 1,000 x 6
 // 155 / 135 / 122 / 133 / 180; 3,000 x 10 471 / 348 / 274 / 333.  Of 5,000 to 8,000: 100 x 10 80 / 65 / 57 / 59 / 73; 1,000 x 12 135 / 119 / 119 / 142;
-// 3,800 x 8 172 / 156 / 168 / 211; 7,000 x 10 237 / 221 / 252 / 371.)
+// 3,800 x 8 172 / 156 / 168 / 211; 7,000 x 10 237 / 221 / 252 / 371.  These are of draws before rows of up to 512 entries had draw_wave.  With it, over 36
+// walks drawn from graphs of 1 M to 235 M entries, the number taken is 1.5 % slower than the best of the five in the mean and 13 % at most:
+// 9,738 x 8, scale 23, 174 / 153 / 167, and 11 x 8 on the scale-22 graph with 18 edges a vertex 34 by 512 threads and 39 by 1024.)
 static uint32_t walker_threads(uint32_t N, uint32_t longest) {
   if (longest > 65533) return N <= 256 ? 1024 : N <= 8192 ? 512 : 256;
   if (longest > 16384) return N <= 512 ? 512 : N <= 16384 ? 256 : 128;
@@ -92,8 +94,10 @@ static uint32_t walker_threads(uint32_t N, uint32_t longest) {
 // times, and its table pays from some length on.  But a walk also lasts as long as the walker that meets the longest row without
 // a table, ROW_NS an entry with 512 threads, inversely more with fewer and down to ROW_LEAST_NS with more.  What every choice would
 // take is added up, from no tables over those of the longest class alone to those of every class from 33 entries on, and the least is taken.
-// The figures were fitted to 36 walks on graphs of 1 M to 260 M entries with ten choices each: what is taken is 2 % slower than the best
-// of the ten in the mean, 25 % at most.  (Tables where N * len * d / E * 2.5 ps exceeds 8 ps, as before, and now, us: 5,000 walkers x 2 on the
+// The figures were fitted, before rows of up to 512 entries were drawn from by draw_wave, to 36 walks on graphs of 1 M to 260 M entries with ten
+// choices each: what was taken was 2 % slower than the best of the ten in the mean, 25 % at most.  With draw_wave, over 36 other walks with
+// eleven choices each: 4 % in the mean, 19 % at most (343 x 13 on the scale-18 graph with 32 edges a vertex, 103 us without tables, 87 with those of
+// rows from 382 entries on), so they are left as they are.  (Tables where N * len * d / E * 2.5 ps exceeds 8 ps, as before, and now, us: 5,000 walkers x 2 on the
 // scale-24 graph 1301 / 169, 4,000 x 2 on the scale-22 graph with 40 edges a vertex 640 / 186, 500 x 8 with 30 288 / 192, 8,500 x 1 on the
 // scale-23 graph 180 / 46, 20,000 x 12 there 415 / 375.)
 constexpr double BUILD_PS = 7.5, DRAW_PS = 2.4, BUILD_US = 31.0, ROW_NS = 0.39, ROW_LEAST_NS = 0.25, STEP_US = 2.4;

@@ -2,7 +2,8 @@
 // the threads of a workgroup evaluate that entry alone, from the same prefix-sum definition the offline build uses:
 //   pass 1  exact sum of the row's weights -> ledger, class of entry col
 //           (a light col whose own share accepts the draw needs nothing more)
-// in rows of up to 256 entries all of it by one wavefront, in registers (draw_wave); in rows of up to 16 slots a thread
+// in rows of up to 256 entries all of it by one wavefront, in registers (draw_wave), where the row type says so (Row::WAVE); in rows of up to 4 or
+// 16 slots a thread (Row::HELD) and 4,095 entries
 //   scan    of deficits and surpluses over the workgroup, whose prefixes each thread has for its own slots (draw_held)
 // and in longer ones
 //   pass 2  deficits and surpluses of every chunk of the row; their prefixes over the chunks
@@ -264,8 +265,11 @@ __device__ __forceinline__ uint32_t draw_entry(Row& row, const uint32_t d, const
 // the thread of col the key, and the thread whose prefixes it falls between the slot.  Three barriers and some 3,000 cycles, where the
 // sweep over chunks and the chain on one wavefront behind it take 9,000 (counted in the table-per-step walk, rows of 800 entries on
 // average).  The amounts of four quads held in registers would make them 147, three wavefronts to a SIMD: they are computed again.
-// Not for rows whose surpluses may wrap (a second form that saturates cost a walker of one wavefront 9 registers, which is the sixth wavefront to
-// a SIMD: 20,000 walkers x 4 without tables, scale 16, 78.5 -> 76.2 us).
+// Up to HELD_MOST entries, whose surpluses add up to less than 2^64 whatever the weights (d times d, in shares of 2^40): a second form that saturates
+// cost a walker of one wavefront 9 registers, which is the sixth wavefront to a SIMD (20,000 walkers x 4 without tables, scale 16, 78.5 -> 76.2 us).
+// Longer rows have nothing to gain by it: where all rows have 4,097..8,191 entries, 200 walkers x 40 of 512 threads take 668 us with four quads a
+// thread and 501 with the two sweeps (700 x 20 672 / 517; with windows 891 / 777 and, 500 x 20, 568 / 500), 1,500 x 20 of 256 threads through
+// rows of 4,096 698 / 553.  Rows of 2,049..4,095 with two quads a thread of 512 instead of four: 200 x 40 365 -> 280, with windows 568 -> 478.
 constexpr uint32_t HELD_MOST = 4095;
 template <int Q, int T, class Row>
 __device__ __forceinline__ uint32_t draw_held(Row& row, const uint32_t d, const Ledger& L, const uint32_t col, const Entry& ec,
@@ -453,14 +457,15 @@ __device__ __forceinline__ bool row_ledger(Row& row, const uint32_t d, const uin
 // The draw from a row of at most 64 S entries by one wavefront, S consecutive slots a lane: no barrier, no LDS, no sweep twice.  S is 4 for rows
 // of up to WAVE_MOST entries, and 1 for those of up to 64 (table-per-step walks: 2,000 x 40 on the scale-18 graph 525 -> 507 us, on the scale-17
 // graph 412 -> 392, 1,500 x 20 on the scale-14 graph with 5 edges a vertex 88 -> 80).
-// In the table-per-step walk one wavefront of the workgroup draws for all (WAVE_ONE: its weights come from windows in LDS); the others wait for it
-// and leave the SIMDs to the walkers beside.  A step from a row of 256 entries and fewer, half of all, takes 8,300 cycles instead of 11,000 (2,000 x
+// In the table-per-step walk with a bit a vertex one wavefront of the workgroup draws for all (WAVE_ONE), from weights that it has tested bits for; the
+// others wait for it and leave the SIMDs to the walkers beside.  A step from a row of 256 entries and fewer, half of all, takes 8,300 cycles instead of 11,000 (2,000 x
 // 40 on the scale-18 graph 549 -> 518 us, on the scale-17 graph 449 -> 410, 200 x 40 there 254 -> 217).  With eight slots a lane a row of 300
 // takes as long as by the workgroup, with sixteen a row of 950 takes longer (518 / 520 / 803 us).
 // In the walk without tables every wavefront of the workgroup draws for itself, all the same slot, and no barrier is met (WAVE_EACH).  A workgroup
 // of one wavefront has eight slots a lane for rows of 257 to 512 entries too (10,000 x 8 on the scale-22 graph 183.9 -> 180.3 us, while the 80
 // registers of six wavefronts to a SIMD suffice: with what the compiler keeps of the sum for the amounts it spills, 181.5).  Sixteen for rows
 // of up to 1,024 spill (217, and 183.5 with the slots in four strips and the amounts computed again).
+// Not for rows whose weights only come in slot order, as a window in LDS moves along (N2vRow), or from an operator (FunctionRow): WAVE_NONE, untried.
 // All lanes call it together.
 constexpr uint32_t WAVE_MOST = 256;
 enum WaveRows { WAVE_NONE, WAVE_ONE, WAVE_EACH };
@@ -588,10 +593,10 @@ __device__ __forceinline__ uint32_t draw_wave(Row& row, const uint32_t d, const 
 //                     through its part of the row in slot order, once, all lanes together (k advances by 4 per lane)
 //   row.again(k, w)   the same, afterwards, for any slots and by any wavefront
 //   Row::U            how many times 256 slots are in flight at once; if that is more than one, instead of first():
-//   Row::WAVE         whether rows of up to WAVE_MOST entries (twice that for WAVE_EACH and T = 64) go to draw_wave, from row.load(k, w): as
-//                     first(), before any other call
-//   Row::HELD         0, 4 or 16: rows of up to so many slots a thread (4,095 at most) by draw_held
 //   row.many(k, end, again, w)  slots k + 256 j .. k + 256 j + 3 for j < U, zeros from slot `end` on, in both sweeps
+//   Row::WAVE         whether rows of up to WAVE_MOST entries (twice that for WAVE_EACH and T = 64) go to draw_wave, and then instead of all these:
+//   row.load(k, w)    clamped weights of slots k, k + 1, .. of one lane (zeros past the row), as many as w holds: 1, 4 or 8
+//   Row::HELD         0, 4 or 16: rows of up to so many slots a thread (HELD_MOST entries at most, 8 slots a thread of 512) by draw_held
 template <int T, class Row>
 __device__ __forceinline__ uint32_t draw_slot(Row& row, const uint32_t d, const u32x4& r, DrawLds<T>& lds) {
   constexpr int NW = T / 64;
